@@ -2,7 +2,6 @@
 // (flat and paged scatter), decode.  General kernels (any float dtype, head_dim 64/128/256,
 // 2/3/4-bit); the MFMA fast path for fp16 / head_dim 128 lives in akv_encode_mfma.hip.
 #include "akv_common.h"
-#include "akv_frag.h"
 
 // ----------------------------------------------------------------------------------
 // host state
@@ -132,9 +131,7 @@ int akv_prepare_decode_mfma(const float* rotation, int d, void* prep, hipStream_
 int akv_decode_mfma_try(const akv_gen_args& a, bool blocks, int d, int bits, int out_dtype, const void* rot_prep,
                         hipStream_t stream);
 
-int akv_prepare_frags(const float* rotation, int d, void* prep, hipStream_t stream);
-
-extern "C" size_t akv_rotation_prepared_bytes(int d) { return akv_prep_bytes(d); }
+extern "C" size_t akv_rotation_prepared_bytes(int d) { return akv_prep_floats(d) * sizeof(float); }
 
 extern "C" int akv_rotation_prepare(const float* rotation, int d, void* prep, size_t prep_bytes,
                                     void* stream) {
@@ -145,10 +142,8 @@ extern "C" int akv_rotation_prepare(const float* rotation, int d, void* prep, si
   dim3 grid(d / 32, d / 32);
   akv_prepare_rotation_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(rotation, (float*)prep, d);
   AKV_LAUNCH_CHECK("akv_prepare_rotation_kernel");
-  int rc = akv_prepare_frags(rotation, d, prep, (hipStream_t)stream);
-  if (rc) return rc;
   if (d == 128) {
-    rc = akv_prepare_rotation_mfma(rotation, d, prep, (hipStream_t)stream);
+    int rc = akv_prepare_rotation_mfma(rotation, d, prep, (hipStream_t)stream);
     if (rc) return rc;
     return akv_prepare_decode_mfma(rotation, d, prep, (hipStream_t)stream);
   }
@@ -269,7 +264,7 @@ extern "C" int akv_unpack_lookup(const uint8_t* packed, int64_t n, int d, int64_
 }
 
 // ----------------------------------------------------------------------------------
-// general encode / decode (head_dim 512, rows the other kernels' loads and stores do not fit): one workgroup of 4 wavefronts, each wavefront rotates VPW vectors
+// general encode / decode: one workgroup of 4 wavefronts, each wavefront rotates VPW vectors
 // at a time with lanes owning D/64 output coordinates; the matrix (Pi^T for encode, Pi for
 // decode) is staged in LDS as [k][out].
 // ----------------------------------------------------------------------------------
@@ -555,25 +550,6 @@ static int akv_encode_dispatch(int d, int bits, int dt, const akv_gen_args& a, v
 // MFMA fast path (akv_encode_mfma.hip); returns AKV_ERR_UNSUPPORTED when it does not apply.
 int akv_encode_mfma_try(const akv_gen_args& a, bool paged, int x_dtype, int d, int bits,
                         const void* rot_prep, hipStream_t stream);
-int akv_encode_rows_try(const akv_gen_args& a, bool paged, int x_dtype, int d, int bits, const void* rot_prep, hipStream_t stream);
-
-// The matrix-core encode kernels.  At head_dim 128 the kernel whose workgroups hold the matrix in LDS issues fewer vector
-// instructions per row but fills 64 KB before its first product: it is the better one for very many 16-bit rows.  Where
-// the line lies was measured with K and V rows scattered into a 4-bit cache (us, that kernel : the other one, bfloat16 /
-// float16 / float32): 8,192 vectors 10.0 : 7.9 / 9.2 : 5.6 / 10.9 : 8.3; 131,072 vectors 18.9 : 17.2 / 17.6 : 16.7 / 24.4 :
-// 22.7; 262,144 vectors 30.0 : 28.0 / 27.3 : 26.5 / 41.5 : 38.3; 1,048,576 vectors 107 : 110 / 98 : 103 / 171 : 162.
-// The smallest 16-bit calls take that kernel's split form, whose chain from the first load to the last store is shorter
-// (its rows are the operand as they are loaded, a wavefront searches four values): a serving step of 16 sequences is
-// 0.5 us faster with it, at 4,096 vectors the two are level.
-static int akv_encode_fast_try(const akv_gen_args& a, bool paged, int x_dtype, int d, int bits, const void* rot_prep, hipStream_t stream) {
-  const int64_t n_total = (paged && a.x2) ? 2 * a.n : a.n;
-  const bool split = d == 128 && x_dtype != AKV_F32 && n_total <= AKV_ENCODE_SPLIT_MAX;
-  if (!split && (d != 128 || x_dtype == AKV_F32 || n_total <= 262144)) {
-    const int rc = akv_encode_rows_try(a, paged, x_dtype, d, bits, rot_prep, stream);
-    if (rc != AKV_ERR_UNSUPPORTED) return rc;
-  }
-  return akv_encode_mfma_try(a, paged, x_dtype, d, bits, rot_prep, stream);
-}
 
 static int akv_check_codec_args(const char* fn, int d, int bits) {
   if (!(d == 64 || d == 128 || d == 256 || d == 512))
@@ -599,7 +575,7 @@ extern "C" int akv_encode(const void* x, int x_dtype, int64_t n, int d, int64_t 
   a.table = boundaries;
   a.packed = out_packed; a.ps0 = packed_stride;
   a.norms = out_norms;
-  rc = akv_encode_fast_try(a, false, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
+  rc = akv_encode_mfma_try(a, false, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
   if (rc != AKV_ERR_UNSUPPORTED) return rc;
   return akv_encode_dispatch<false>(d, bits, x_dtype, a, stream);
 }
@@ -627,7 +603,7 @@ extern "C" int akv_encode_paged_kv(const void* k, const void* v, int x_dtype, in
   a.packed = k_packed; a.ps0 = ps_blk; a.ps1 = ps_pos; a.ps2 = ps_head;
   a.norms = k_norms; a.ns0 = ns_blk; a.ns1 = ns_pos; a.ns2 = ns_head;
   a.x2 = v; a.packed2 = v_packed; a.norms2 = v_norms;
-  rc = akv_encode_fast_try(a, true, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
+  rc = akv_encode_mfma_try(a, true, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
   if (rc != AKV_ERR_UNSUPPORTED) return rc;
   // layouts the matrix-core kernel does not take: one launch per tensor
   akv_gen_args b = a;
@@ -659,7 +635,7 @@ extern "C" int akv_encode_paged(const void* x, int x_dtype, int64_t num_tokens, 
   a.table = boundaries;
   a.packed = out_packed; a.ps0 = ps_blk; a.ps1 = ps_pos; a.ps2 = ps_head;
   a.norms = out_norms; a.ns0 = ns_blk; a.ns1 = ns_pos; a.ns2 = ns_head;
-  rc = akv_encode_fast_try(a, true, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
+  rc = akv_encode_mfma_try(a, true, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
   if (rc != AKV_ERR_UNSUPPORTED) return rc;
   return akv_encode_dispatch<true>(d, bits, x_dtype, a, stream);
 }

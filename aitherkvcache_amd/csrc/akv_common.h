@@ -81,10 +81,6 @@ void akv_profile_stamp(hipStream_t s, hipEvent_t begin);
 static inline size_t akv_prep_floats(int d) { return (size_t)4 * d * d + 1024; }
 #define AKV_PREP_DECODE_OFFSET(d) ((size_t)2 * (d) * (d) * 4 + 65536 + 256)
 
-// 16-bit vectors of head_dim 128 up to which the encode kernel that shares a step of 16 vectors among eight wavefronts is
-// used (akv_codec.hip draws the line)
-#define AKV_ENCODE_SPLIT_MAX 2048
-
 // Arguments of the encode / decode kernels (flat and paged forms share one struct).
 struct akv_gen_args {
   // encode input

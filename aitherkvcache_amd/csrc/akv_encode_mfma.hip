@@ -1,6 +1,5 @@
 // MFMA encode (norm -> rotate -> codebook search -> pack -> store) for float16, bfloat16 and float32
-// input at head_dim 128: calls of very many vectors and, in its split form, of very few (akv_encode_rows.hip takes what
-// lies between and the other head sizes; the line is drawn and its reasons given in akv_codec.hip).
+// input at head_dim 128.
 //
 // The rotation is the only heavy arithmetic of the encode path (128 x 128 multiply-adds per
 // vector), so it runs on the matrix cores; everything else is arranged so that the matrix-core
@@ -134,7 +133,7 @@ __device__ __forceinline__ uint32_t em_cell(float y) {
 }
 
 // MT: M-tiles (16 vectors each) per wavefront step -- MT, or 1 for float32 input
-// SPLIT (calls of up to AKV_ENCODE_SPLIT_MAX vectors, e.g. one serving step): a workgroup is eight wavefronts that share ONE
+// SPLIT (calls of a few thousand vectors, e.g. one serving step): a workgroup is eight wavefronts that share ONE
 // step of 16 vectors, wavefront w computes N-tile w with its eighth of the B operand straight from memory in
 // registers -- no 64 KB fill, no cell table, one barrier; the codes meet in LDS and 256 threads pack and store
 // them.  Same products, same reciprocal, same comparison against the boundaries: the same codes.
@@ -318,11 +317,9 @@ __global__ __launch_bounds__(EM_THREADS) void akv_encode_mfma_kernel(akv_gen_arg
         dst_n[lane] = dn;
       }
     }
-    // squared norms: the lane's 32 elements as two sums of sixteen, added at the end (the order of akv_encode_rows.hip:
-    // the kernels that share head_dim 128 by the size of the call store the same norms)
-    float ss[MT], ss2[MT];
+    float ss[MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) { ss[mt] = 0.f; ss2[mt] = 0.f; }
+    for (int mt = 0; mt < MT; ++mt) ss[mt] = 0.f;
     uint32_t unscale[MT];     // float bits of the power of two taken out of each M-tile's rows
     bool nonfinite[MT];       // bfloat16 only: the row holds an infinity or a NaN
     if constexpr (XDT == AKV_F16) {
@@ -335,10 +332,7 @@ __global__ __launch_bounds__(EM_THREADS) void akv_encode_mfma_kernel(akv_gen_arg
           union { em_half8 h; em_half2 h2[4]; } cv;
           cv.h = A[mt][ks];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            float& sq = ks < 2 ? ss[mt] : ss2[mt];
-            sq = __builtin_amdgcn_fdot2(cv.h2[q], cv.h2[q], sq, false);
-          }
+          for (int q = 0; q < 4; ++q) ss[mt] = __builtin_amdgcn_fdot2(cv.h2[q], cv.h2[q], ss[mt], false);
         }
       }
     } else if constexpr (XDT == AKV_F32) {
@@ -357,8 +351,7 @@ __global__ __launch_bounds__(EM_THREADS) void akv_encode_mfma_kernel(akv_gen_arg
           for (int q = 0; q < 4; ++q) {
             mx = max(mx, w[q] & 0x7fffffffu);
             const float v = __uint_as_float(w[q]);
-            float& sq = pc < 4 ? ss[mt] : ss2[mt];
-            sq = fmaf(v, v, sq);
+            ss[mt] = fmaf(v, v, ss[mt]);
           }
         }
         {   // largest magnitude of the row over its four lanes
@@ -409,9 +402,8 @@ __global__ __launch_bounds__(EM_THREADS) void akv_encode_mfma_kernel(akv_gen_arg
             mm.u = cv.w[q] & 0x7fff7fffu;
             mx2 = __builtin_elementwise_max(mx2, mm.v);
             const float lo = __uint_as_float(cv.w[q] << 16), hi = __uint_as_float(cv.w[q] & 0xffff0000u);
-            float& sq = ks < 2 ? ss[mt] : ss2[mt];
-            sq = fmaf(lo, lo, sq);
-            sq = fmaf(hi, hi, sq);
+            ss[mt] = fmaf(lo, lo, ss[mt]);
+            ss[mt] = fmaf(hi, hi, ss[mt]);
           }
         }
         uint32_t mx = max((uint32_t)mx2[0], (uint32_t)mx2[1]);
@@ -443,8 +435,6 @@ __global__ __launch_bounds__(EM_THREADS) void akv_encode_mfma_kernel(akv_gen_arg
     }
     // lane l < ROWS finishes vector l = 16 mt + row: transpose-reduce the partial sums over the
     // four lanes of a row
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) ss[mt] += ss2[mt];
     bool any_nan;       // some vector of the step holds a NaN or an infinity (the same in every lane)
     {
       const bool g1 = (g & 1) != 0;
@@ -723,11 +713,17 @@ int akv_encode_mfma_try(const akv_gen_args& a, bool paged, int x_dtype, int d, i
   const uint4* bop = (const uint4*)((const float*)rot_prep + (size_t)2 * d * d);
   const int64_t n_total = (paged && a.x2) ? 2 * a.n : a.n;
   const int cus = akv_cached_cu_count();
-  // A 16-bit call that leaves every CU at most one step of 16 vectors shares each step among eight wavefronts.
-  const bool split = x_dtype != AKV_F32 && n_total <= AKV_ENCODE_SPLIT_MAX;
-  const int rows_per_step = (x_dtype == AKV_F32 || split) ? 16 : EM_ROWS;
+  // A call too small to give every CU a step of 32 vectors (one serving step: 4,096 vectors) runs the form with 16
+  // vectors per wavefront step: twice the workgroups, half the chain of products and searches that its one busy
+  // wavefront per workgroup walks through alone.
+  const bool narrow = paged && x_dtype != AKV_F32 && (n_total + EM_ROWS - 1) / EM_ROWS < cus;
+  // ... and one (paged or flat) that leaves a workgroup at most two steps of 16 vectors shares each step among
+  // eight wavefronts
+  const bool split = x_dtype != AKV_F32 && (n_total + 15) / 16 <= 2 * (int64_t)cus && !getenv("AKV_ENCODE_NO_SPLIT");
+  const int rows_per_step = (x_dtype == AKV_F32 || narrow || split) ? 16 : EM_ROWS;
   const int64_t steps = (n_total + rows_per_step - 1) / rows_per_step;
-  // steps are dealt round-robin over workgroups first, so that every CU gets as many as the next
+  // steps are dealt round-robin over workgroups first, so a small call (one serving step) spreads
+  // over as many CUs as it has steps instead of filling the wavefronts of a few
   const int grid = (int)(steps < cus ? steps : cus);
 #define EM_LAUNCH_MT(BB, PG, DT, DR, MM)                                                              \
   do {                                                                                               \
@@ -742,7 +738,8 @@ int akv_encode_mfma_try(const akv_gen_args& a, bool paged, int x_dtype, int d, i
 #define EM_LAUNCH(BB, PG, DT, DR)                                                                     \
   do {                                                                                               \
     if (split && em_launch_split<BB, PG, DT, DR>(grid, stream, a, bop)) break;                       \
-    EM_LAUNCH_MT(BB, PG, DT, DR, (DT == AKV_F32 ? 1 : EM_MT));                                        \
+    if (DT == AKV_F32 || (PG && narrow)) EM_LAUNCH_MT(BB, PG, DT, DR, 1);                             \
+    else EM_LAUNCH_MT(BB, PG, DT, DR, (DT == AKV_F32 ? 1 : EM_MT));                                   \
   } while (0)
 #define EM_LAUNCH_DT(BB, PG, DR) do { if (x_dtype == AKV_F16) EM_LAUNCH(BB, PG, AKV_F16, DR); else if (x_dtype == AKV_BF16) EM_LAUNCH(BB, PG, AKV_BF16, DR); else EM_LAUNCH(BB, PG, AKV_F32, DR); } while (0)
   // flat rows whose byte offsets stay below 2^31 take the variant with 32-bit lane offsets
