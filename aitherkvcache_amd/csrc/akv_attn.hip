@@ -218,49 +218,49 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
       }
     }
   } else {
-  // inverse rotation: thread t owns coordinates (t % 128) * JP .. of heads 2 * (t / 128) and + 1
-  constexpr int JT = 128;                 // threads along the coordinate axis
-  constexpr int JP = D / JT > 0 ? D / JT : 1;   // coordinates per thread (D=256 -> 2)
-  const int jt = threadIdx.x % JT, pr = threadIdx.x / JT;
-  if (jt * JP < D) {
-    float o[2][JP];
+  // Inverse rotation: thread (share, jt) owns coordinates jt * JP .. of all four heads for the share's part of the sum;
+  // the shares are added up in LDS.  KB rows of the matrix are requested before the first is used, at an offset that is
+  // opaque inside the item loop: one entry at a time the rotation was a chain of trips to the L2 cache (head_dim 256,
+  // 24 sequences of 16 heads: 62 us for the kernel, now 13.5), and entries held across items, which the compiler made
+  // of the invariant loads, lived in scratch memory (head_dim 64, 48 sequences of 32 heads: 36 us, now 5).
+  constexpr int JT = D < 128 ? D : 128, JP = D / JT, SHARES = 256 / JT, KS = D / SHARES, KB = D == 64 ? 16 : D == 512 ? 16 : 32;
+  __shared__ __align__(16) float o_lds[SHARES][4][D];
+  const int jt = threadIdx.x % JT, share = threadIdx.x / JT;
+  float o[4][JP];
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+  for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int i = 0; i < JP; ++i) o[q][i] = 0.f;
-    // Entries of KB rows are requested before the first is used, and the matrix pointer is opaque inside the item loop:
-    // one entry at a time the rotation was a chain of trips to the L2 cache (head_dim 256, 24 sequences of 16 heads: 62 us for the kernel, now 16),
-    // and entries held across items, which the compiler made of the invariant loads, lived in scratch memory
-    // (head_dim 64, 48 sequences of 32 heads: 36 us, now 19).
-    constexpr int KB = 32 / JP;
-    const float* Pp = Pi;
-    asm volatile("" : "+s"(Pp));
-    for (int k0 = 0; k0 < D; k0 += KB) {
-      float pv[KB][JP];
+    for (int i = 0; i < JP; ++i) o[q][i] = 0.f;
+  uint32_t base = (uint32_t)(share * KS * D + jt * JP);
+  asm volatile("" : "+v"(base));
+#pragma unroll 1
+  for (int k0 = 0; k0 < KS; k0 += KB) {
+    float pv[KB][JP];
 #pragma unroll
-      for (int k = 0; k < KB; ++k)
+    for (int k = 0; k < KB; ++k)
 #pragma unroll
-        for (int i = 0; i < JP; ++i) pv[k][i] = Pp[(size_t)(k0 + k) * D + jt * JP + i];
-      __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < JP; ++i) pv[k][i] = Pi[base + (uint32_t)((k0 + k) * D + i)];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 0; k < KB; ++k) {
-        const float a0v = a_lds[2 * pr][k0 + k], a1v = a_lds[2 * pr + 1][k0 + k];
+    for (int k = 0; k < KB; ++k)
 #pragma unroll
-        for (int i = 0; i < JP; ++i) {
-          o[0][i] = fmaf(a0v, pv[k][i], o[0][i]);
-          o[1][i] = fmaf(a1v, pv[k][i], o[1][i]);
-        }
+      for (int q = 0; q < 4; ++q) {
+        const float av = a_lds[q][share * KS + k0 + k];
+#pragma unroll
+        for (int i = 0; i < JP; ++i) o[q][i] = fmaf(av, pv[k][i], o[q][i]);
       }
-    }
+  }
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int hq = hg * 4 + 2 * pr + q;
-      if (hq < QH) {
+  for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int i = 0; i < JP; ++i)
-          akv_elem<ODT>::store(out, s * os_seq + hq * os_head + jt * JP + i, o[q][i] + poison);
-      }
-    }
+    for (int i = 0; i < JP; ++i) o_lds[share][q][jt * JP + i] = o[q][i];
+  __syncthreads();
+  for (int e = threadIdx.x; e < 4 * D; e += 256) {
+    const int q = e / D, j = e % D;
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < SHARES; ++i) v += o_lds[i][q][j];
+    if (hg * 4 + q < QH) akv_elem<ODT>::store(out, s * os_seq + (hg * 4 + q) * os_head + j, v + poison);
   }
   }
   __syncthreads();       // the merged vectors are read until here; the next item overwrites them
@@ -437,6 +437,11 @@ extern "C" size_t akv_paged_attn_workspace_bytes(int num_seqs, int num_q_heads, 
          akv_attn_mfma_extra_bytes(num_seqs, num_q_heads);
 }
 
+// the same for head_dim 64 and 256, and few kv heads at head_dim 128 (akv_attn_wave.hip)
+bool akv_attn_wave_applicable(const akv_attn_args& a, int d, int bits);
+int akv_attn_wave_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* PiT, const akv_attn_args& a,
+                      int d, int bits, const akv_attn_ws& ws, void* extra_ws, int grid, hipStream_t stream);
+
 static void* akv_static_scratch_of_current_device();   // null before the first akv_paged_attn_static call there
 
 extern "C" int akv_paged_attn_status(const void* workspace, int* flags, void* stream_) {
@@ -549,7 +554,11 @@ static int akv_paged_attn_impl(
   int rc;
   int Gused = G;
   const int32_t* seqw = nullptr;      // set by the matrix-core path, whose prologue cuts the block axis itself
-  if (akv_attn_mfma_applicable(a, d, bits)) {
+  if (akv_attn_wave_applicable(a, d, bits)) {
+    seqw = ws.seqw;
+    Gused = G / AKV_ATTN_WG_PER_CU;
+    rc = akv_attn_wave_run(query, q_dtype, qs_seq, qs_head, PiT, a, d, bits, ws, (char*)workspace + ws.bytes, Gused, stream);
+  } else if (akv_attn_mfma_applicable(a, d, bits)) {
     seqw = ws.seqw;
     Gused = G / AKV_ATTN_WG_PER_CU;   // one 8-wavefront workgroup per CU (64 KiB table, up to 256 VGPRs)
     rc = akv_attn_mfma_run(query, q_dtype, qs_seq, qs_head, PiT, a, bits, ws, (char*)workspace + ws.bytes, Gused, stream);

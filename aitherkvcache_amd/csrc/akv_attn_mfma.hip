@@ -1137,15 +1137,15 @@ extern "C" int akv_debug_set_handoff_spin_limit(int polls) {
 }
 
 // query heads per kv head -> number of groups of at most eight the kv head is presented as (0: none fits)
-static int akv_attn_mfma_head_groups(int gqa) {
+int akv_attn_mfma_head_groups(int gqa) {
   for (int hg = (gqa + 7) / 8; hg <= gqa && hg <= 8; ++hg)
     if (gqa % hg == 0) return hg;
   return 0;
 }
 
-bool akv_attn_mfma_applicable(const akv_attn_args& a, int d, int bits) {
+bool akv_attn_mfma_takes(const akv_attn_args& a, int bits) {
   if (mfma_disabled()) return false;
-  if (d != 128 || bits < 2 || bits > 4 || (a.block_size != 16 && a.block_size != 32)) return false;
+  if (bits < 2 || bits > 4 || (a.block_size != 16 && a.block_size != 32)) return false;
   if (akv_attn_mfma_head_groups(a.QH / a.KVH) == 0) return false;
   if (a.num_blocks >= ((int64_t)1 << 31)) return false;                       // block ids travel as 32-bit lanes
   // K rows are read 16 / 12 / 8 bytes per lane, V rows by dword / dword / halfword.  Multi-dword
@@ -1159,11 +1159,12 @@ bool akv_attn_mfma_applicable(const akv_attn_args& a, int d, int bits) {
   for (int i = 0; i < 12; ++i)
     if (strides[i] < 0 || strides[i] >= ((int64_t)1 << 27)) return false;   // 32-bit in-block offsets
   // the largest in-block offset a lane forms (head, then position of the second tile, then the row) fits 32 bits
-  const int64_t kmax = (int64_t)a.KVH * a.kps_head + 32 * a.kps_pos + 64, vmax = (int64_t)a.KVH * a.vps_head + 32 * a.vps_pos + 64;
+  const int64_t kmax = (int64_t)a.KVH * a.kps_head + 32 * a.kps_pos + 128, vmax = (int64_t)a.KVH * a.vps_head + 32 * a.vps_pos + 128;
   const int64_t nmax = (int64_t)a.KVH * (a.kns_head > a.vns_head ? a.kns_head : a.vns_head) + 32 * (a.kns_pos > a.vns_pos ? a.kns_pos : a.vns_pos);
   if (kmax >= ((int64_t)1 << 32) || vmax >= ((int64_t)1 << 32) || nmax >= ((int64_t)1 << 32)) return false;
   return true;
 }
+bool akv_attn_mfma_applicable(const akv_attn_args& a, int d, int bits) { return d == 128 && akv_attn_mfma_takes(a, bits); }
 
 int akv_attn_mfma_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* PiT,
                       const akv_attn_args& a_in, int bits, const akv_attn_ws& ws, void* extra_ws, int grid, hipStream_t stream) {

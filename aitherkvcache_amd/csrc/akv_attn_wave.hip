@@ -1,0 +1,614 @@
+// MFMA paged decode attention in which every wavefront works on its own: 4- and 2-bit caches at head_dim 64 and 256,
+// and at head_dim 128 where few kv heads are at hand, block_size 16 or 32.
+//
+// A workgroup owns a range of the global block axis (akv_attn_partition).  Its W wavefronts are laid out as
+// (kv head slot) x (R shares of the tokens): wavefront (hs, r) takes chunks r, r + R, ... of 32 tokens of a segment for
+// kv head hs, scores AND values, with no barrier until the segment ends; then the R partial results of a head are
+// merged through LDS.  With at least W kv heads R is 1 and nothing is merged.  (The kernel in akv_attn_mfma.hip splits
+// scores and values between the wavefronts of a fixed set of eight kv heads: one kv head -- a rank of a sharded
+// model -- leaves seven eighths of it idle.)
+//
+//   scores   S^T[token, col] = sum_d Khat[token, d] Qop[d, col]         v_mfma_f32_16x16x32_f16
+//            A: lane (n = l % 16, g = l / 16) owns quarter g of token n's code row; an LDS table turns a byte (two codes)
+//            into (hi pair, lo pair), two look-ups side by side are the operand.  B: the rotated query, every pair
+//            twice (it faces hi and lo); columns 0..7 the float16 rounding, columns 8..15 the remainder.
+//   softmax  on the accumulator as it lies: lane (col, g) holds tokens 4 g .. 4 g + 3 of both tiles.
+//   values   O^T[coord, col] += sum_token Vhat[token, coord] W[token, col].  The tokens a lane weighs are the tokens
+//            whose look-ups it makes, so the weights are the operand without crossing a lane.  A byte is the same
+//            coordinate of two tokens; columns 0..7 carry the float16 rounding of the weights, 8..15 the remainder.
+//
+// Precision: codebook, queries and weights are split into two float16 terms each (rounded to nearest: 2^-23 of the
+// value), products are exact, sums float32; only the product of two remainders (2^-24) is left out.  The codebook and
+// every query row are scaled by powers of two, and the weights are kept below 2^15 rather than 1, so that no remainder
+// is a float16 subnormal that matters.
+//
+// One table serves keys and values: 256 entries x 8 bytes x 32 copies (a lane reads copy lane % 32: no bank conflicts).
+// 2-bit codes are looked up as nibbles: two masks and a shift spread a byte of four codes, no second table.
+//
+// What bounds it: the look-ups, 64 eight-byte LDS reads per kv head, 16 tokens and 256 coordinates, and the vector
+// instructions around them.
+#include <type_traits>
+
+#include "akv_attn_common.h"
+
+typedef _Float16 aw_half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 aw_half2 __attribute__((ext_vector_type(2)));
+typedef float aw_float2 __attribute__((ext_vector_type(2)));
+typedef float aw_float4 __attribute__((ext_vector_type(4)));
+typedef uint32_t aw_u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t aw_u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) const aw_u32x2 aw_lds_cu64;
+typedef __attribute__((address_space(3))) aw_u32x4 aw_lds_u128;
+typedef __attribute__((address_space(3))) float aw_lds_f32;
+typedef __attribute__((address_space(3))) aw_float2 aw_lds_f64;
+typedef __attribute__((address_space(3))) aw_float4 aw_lds_f128;
+
+#define AW_FRAME 15.f          // weights stay below 2^AW_FRAME
+// Value norms count as at least 2^-AW_TINY in the running maximum: the plain exponentials, summed for the denominator, then
+// stay below 2^(AW_TINY + AW_FRAME), and a million of them in float32.  A vector of that norm still has 2^15 times the
+// smallest float16 the weights need, so only norms below some 2^-110 lose digits (a zero vector weighs nothing).
+#define AW_TINY 90
+#define AW_WIN 32              // chunks of a wavefront served by one window of 64 block ids
+
+template <int D, int BITS> struct aw_cfg {
+  static constexpr int W = D == 64 ? 16 : 8;            // wavefronts: what their registers admit on a CU
+  static constexpr int CPL = D / 16;                    // coordinates per lane of a value tile = M-tiles
+  static constexpr int KS = D / 16;                     // MFMA steps of a score tile (four coordinates a lane each)
+  static constexpr int KDW = D * BITS / 128;            // dwords of a quarter of a code row
+  static constexpr int VB = CPL * BITS / 8;             // bytes of a lane's codes of one token
+  static constexpr int VDW = VB >= 4 ? VB / 4 : 1;
+};
+// LDS: table | per wavefront: 32 key norms, 32 value norms, 32 exponents of those | per wavefront: (max, sum) of eight
+// heads | per wavefront: accumulators of its heads (merging only)
+#define AW_NORM 65536u
+#define AW_NORM_WAVE 384u
+template <int W> constexpr uint32_t aw_ml_off() { return AW_NORM + W * AW_NORM_WAVE; }
+template <int W> constexpr uint32_t aw_acc_off() { return aw_ml_off<W>() + W * 64u; }
+
+struct aw_extra {
+  const uint2* qop;        // [S][KVH][D / 16][64 lanes] four float16 (workspace)
+  const float* fac;        // [S][QH] power of two taken out of a query row, times scale * log2 e
+  const int32_t* wgdesc;   // [G][AKV_WGREC]
+  int hp;                  // kv head slots of a workgroup (a power of two)
+};
+
+// ----------------------------------------------------------------------------------
+// prologue: block 0 cuts the block axis; the others take query heads blockIdx.x - 1, + gridDim.x - 1, ...: rotate, write
+// in operand order.  A thread holds AW_PRO_K entries of one column of Pi^T in registers, requested in one go before
+// anything else and kept for all heads of its workgroup (a trip to the L2 cache per entry, as in a plain loop over the
+// matrix, was 20 us at head_dim 256); D / AW_PRO_K threads share an output coordinate.
+// ----------------------------------------------------------------------------------
+#define AW_PRO_K(D) ((D) == 64 ? 16 : 64)
+template <int D> constexpr int aw_pro_threads() { return D * (D / AW_PRO_K(D)); }      // 256, 256, 1024
+template <int D, int QDT>
+__global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_attn_wave_prologue_kernel(
+    const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const float* __restrict__ PiT, int S, int QH, int KVH,
+    const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix, uint2* __restrict__ qop,
+    float* __restrict__ fac, uint32_t* __restrict__ status, float qscale, int bits, int32_t* __restrict__ wgdesc,
+    int32_t* __restrict__ seqw, int G) {
+  constexpr int K = AW_PRO_K(D), SHARES = D / K;
+  __shared__ __align__(16) float q_lds[2][D];          // [parity of the head]
+  __shared__ float sum_lds[SHARES][D];
+  __shared__ float max_lds[2][4];
+  __shared__ int32_t scratch[257];
+  const int tid = threadIdx.x;
+  if (blockIdx.x == 0) {
+    if (tid == 0) status[0] = 0u;
+    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq);
+    return;
+  }
+  const int t = tid % D, share = tid / D, gqa = QH / KVH;
+  float m[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) m[j] = PiT[(size_t)(share * K + j) * D + t];
+  int par = 0;
+  for (int item = (int)blockIdx.x - 1; item < S * QH; item += (int)gridDim.x - 1, par ^= 1) {
+    const int s = item / QH, hq = item % QH, h = hq / gqa, q = hq % gqa;
+    if (tid < D) q_lds[par][tid] = akv_elem<QDT>::load(query, s * qs_seq + hq * qs_head + tid);
+    __syncthreads();
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < K; j += 4) {
+      const float4 x = *(const float4*)&q_lds[par][share * K + j];
+      acc = fmaf(m[j], x.x, acc);
+      acc = fmaf(m[j + 1], x.y, acc);
+      acc = fmaf(m[j + 2], x.z, acc);
+      acc = fmaf(m[j + 3], x.w, acc);
+    }
+    sum_lds[share][t] = acc;
+    __syncthreads();
+    float y = 0.f;
+    if (tid < D) {
+#pragma unroll
+      for (int i = 0; i < SHARES; ++i) y += sum_lds[i][tid];
+      const float mx = akv_wave_max(fabsf(y));
+      if ((tid & 63) == 0) max_lds[par][tid >> 6] = mx;
+    }
+    __syncthreads();
+    if (tid < D) {
+      float mx = 0.f;
+#pragma unroll
+      for (int i = 0; i < D / 64; ++i) mx = fmaxf(mx, max_lds[par][i]);
+      const uint32_t ex = akv_row_exponent(mx);
+      if (tid == 0) fac[(size_t)s * QH + hq] = akv_row_unscale(ex) * qscale;
+      // coordinate tid = quarter g, step n, place e of the step's four (2-bit codes are looked up as (0, 2) and (1, 3))
+      const float x = y * akv_row_scale(ex);
+      const __half hi = __float2half_rn(x);
+      const int g = tid / (D / 4), n = tid % (D / 4) / 4, c4 = tid & 3;
+      const int e = bits == 2 ? ((c4 & 1) << 1) + (c4 >> 1) : c4;
+      __half* dst = (__half*)(qop + (size_t)(s * KVH + h) * (D / 16 * 64) + n * 64 + 16 * g + q) + e;
+      dst[0] = hi;
+      dst[8 * 4] = __float2half_rn(x - __half2float(hi));
+      // (columns of no query head hold zeros)
+      if (q == 0)
+        for (int z = gqa; z < 8; ++z) { dst[z * 4] = __float2half_rn(0.f); dst[(8 + z) * 4] = __float2half_rn(0.f); }
+    }
+  }
+}
+
+// ----------------------------------------------------------------------------------
+// main kernel
+// ----------------------------------------------------------------------------------
+// address of a table entry: byte k of `word` * 256 + the lane's copy, one byte permute
+template <int K> __device__ __forceinline__ aw_u32x2 aw_look(uint32_t lanebits, uint32_t word) {
+  return *(aw_lds_cu64*)(uintptr_t)__builtin_amdgcn_perm(word, lanebits, 0x0c020400u + (K << 8));
+}
+__device__ __forceinline__ aw_half8 aw_operand(aw_u32x2 a, aw_u32x2 b) {
+  union { uint32_t u[4]; aw_half8 h; } x;
+  x.u[0] = a.x; x.u[1] = a.y; x.u[2] = b.x; x.u[3] = b.y;
+  return x.h;
+}
+// value of the lane eight columns away in the row of sixteen, added
+__device__ __forceinline__ float aw_add_cols(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128 /*row_ror:8*/, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float aw_rows_sum(float v) {
+  auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+// (keeps the widening of a 32-bit lane offset next to its load: scalar base + 32-bit lane offset)
+__device__ __forceinline__ uint32_t aw_here(uint32_t v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+__device__ __forceinline__ void aw_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the words whose bytes are table indices of lane coordinates: pairs (ta, tb) of tokens, words `wa`, `wb` of codes
+template <int BITS, int N> struct aw_pairs { uint32_t w[BITS == 4 ? 2 : 4]; };
+template <int BITS, int N>
+__device__ __forceinline__ void aw_pair(aw_pairs<BITS, N>& p, uint32_t wa, uint32_t wb) {
+  if constexpr (BITS == 4) {
+    p.w[0] = (wa & 0xF0F0F0F0u) | ((wb >> 4) & 0x0F0F0F0Fu);      // the even one of a byte's two codes
+    p.w[1] = ((wa << 4) & 0xF0F0F0F0u) | (wb & 0x0F0F0F0Fu);
+  } else {
+    p.w[0] = ((wa >> 2) & 0x30303030u) | ((wb >> 6) & 0x03030303u);   // code 0 of a byte's four, ...
+    p.w[1] = (wa & 0x30303030u) | ((wb >> 4) & 0x03030303u);
+    p.w[2] = ((wa << 2) & 0x30303030u) | ((wb >> 2) & 0x03030303u);
+    p.w[3] = ((wa << 4) & 0x30303030u) | (wb & 0x03030303u);
+  }
+}
+
+template <int D, int BITS>
+__global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(akv_attn_args a, aw_extra x) {
+  typedef aw_cfg<D, BITS> cfg;
+  constexpr int W = cfg::W, CPL = cfg::CPL, KS = cfg::KS, KDW = cfg::KDW, VB = cfg::VB, VDW = cfg::VDW;
+  constexpr int CPB = 8 / BITS;                            // codes of a byte
+  // The dynamic LDS block is the kernel's only LDS object: its offsets are LDS addresses.
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const uint32_t copy = (uint32_t)(lane & 31) * 8u;
+
+  // ---- table; the scale brings the largest level to [2^9, 2^10)
+  float inv_cs;
+  {
+    float mx = 0.f;
+    for (int v = 0; v < (1 << BITS); ++v) mx = fmaxf(mx, fabsf(a.centroids[v]));
+    const uint32_t ex = min(max((__float_as_uint(mx) >> 23) & 0xffu, 12u), 250u);
+    const float cs = __uint_as_float((254u - ex) << 23) * 512.f;
+    inv_cs = __uint_as_float(ex << 23) * (1.f / 512.f);
+    constexpr int TPE = W * 64 / 256;                      // threads of an entry
+    const int e = threadIdx.x / TPE, part = threadIdx.x % TPE;
+    const float c0 = a.centroids[(e >> 4) & ((1 << BITS) - 1)] * cs, c1 = a.centroids[e & ((1 << BITS) - 1)] * cs;
+    const __half h0 = __float2half_rn(c0), h1 = __float2half_rn(c1);
+    const __half l0 = __float2half_rn(c0 - __half2float(h0)), l1 = __float2half_rn(c1 - __half2float(h1));
+    const uint32_t hi = (uint32_t)__half_as_ushort(h0) | ((uint32_t)__half_as_ushort(h1) << 16);
+    const uint32_t lo = (uint32_t)__half_as_ushort(l0) | ((uint32_t)__half_as_ushort(l1) << 16);
+#pragma unroll
+    for (int i = 0; i < 16 / TPE; ++i) *(aw_lds_u128*)(uintptr_t)(uint32_t)(e * 256 + (part * (16 / TPE) + i) * 16) = (aw_u32x4){hi, lo, hi, lo};
+  }
+  __syncthreads();
+
+  const bool bs32 = a.block_size == 32;
+  const int bs = bs32 ? 32 : 16;
+  const int gqa = a.QH / a.KVH;
+  const int hp = x.hp, R = W / hp;
+  const int hs = wave % hp, r = wave / hp;
+  const int held = akv_prefix_hold(a.prefix, a.S);
+  const int32_t* rec = x.wgdesc + (size_t)blockIdx.x * AKV_WGREC;
+  const int g0 = rec[AKV_WGREC_G0], g1 = rec[AKV_WGREC_G1], s_first = rec[AKV_WGREC_SEQ];
+
+  const uint32_t nbase = AW_NORM + (uint32_t)wave * AW_NORM_WAVE;
+  const uint32_t nread = nbase + (uint32_t)g * 16u;
+
+  int gcur = g0;
+  while (gcur < g1) {
+    int s, sb0, sb1;
+    int64_t ctx;
+    if (gcur == g0 && s_first >= 0) {
+      s = s_first;
+      sb0 = rec[AKV_WGREC_SB0];
+      sb1 = rec[AKV_WGREC_SB1];
+      ctx = rec[AKV_WGREC_CTX];
+    } else {
+      s = akv_find_seq_held(a.prefix, a.S, held, gcur, sb0, sb1);
+      ctx = akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq);
+    }
+    const int blk_lo = gcur - sb0;
+    const int blk_hi = min(g1, sb1) - sb0;
+    const int t_end = (int)min((int64_t)blk_hi * bs, ctx);
+    gcur = sb0 + blk_hi;
+    const int nblk = blk_hi - blk_lo;
+    const int nchunks = bs32 ? nblk : (nblk + 1) >> 1;
+    const int mine = r < nchunks ? (nchunks - r + R - 1) / R : 0;     // chunks r, r + R, ...
+
+    for (int hbase = 0; hbase < a.KVH; hbase += hp) {
+      const int h = hbase + hs;
+      const bool active = h < a.KVH;
+      const int hd = a.hgroup > 1 ? h / a.hgroup : h;                 // the head whose rows are read
+      float m_run = -INFINITY, l_run = 0.f;
+      aw_float4 o[CPL];
+#pragma unroll
+      for (int n = 0; n < CPL; ++n) o[n] = (aw_float4){0.f, 0.f, 0.f, 0.f};
+
+      if (active && mine > 0) {
+        // ---- block ids of the wavefront's chunks from win_k on: lane 2 i + j block j of chunk win_k + i (blocks of 32: lane i)
+        int pbwin = 0, win_k = 0;
+        auto load_window = [&](int k0) {
+          const int k = k0 + (bs32 ? lane : lane >> 1);
+          const int c = r + k * R;
+          const int bi = blk_lo + (int)min((int64_t)(nblk - 1), bs32 ? (int64_t)c : 2 * (int64_t)c + (lane & 1));
+          pbwin = (int)akv_clamp_block(akv_load_index(a.block_tables, a.bt_itype, s * a.bt_stride + bi), a.num_blocks);
+          win_k = k0;
+        };
+        const uint32_t koff = (uint32_t)(hd * a.kps_head + col * a.kps_pos + KDW * 4 * g);
+        const uint32_t voff = (uint32_t)(hd * a.vps_head + 4 * g * a.vps_pos + VB * col);
+        const uint32_t ktile1 = bs32 ? 16u * (uint32_t)a.kps_pos : 0u, vtile1 = bs32 ? 16u * (uint32_t)a.vps_pos : 0u;
+        const int ntok = lane & 31, npos = bs32 ? ntok : ntok & 15;
+        const float* nptr = lane >= 32 ? a.vn : a.kn;
+        const uint32_t nblk_stride = (uint32_t)(lane >= 32 ? a.vns_blk : a.kns_blk);
+        const uint32_t noff = (uint32_t)(lane >= 32 ? hd * a.vns_head + npos * a.vns_pos : hd * a.kns_head + npos * a.kns_pos);
+
+        // Codes and norms sit in one set of registers: the next chunk's keys are requested when this one's are scored, its
+        // values when these are weighed (a second set made the compiler spill at head_dim 256 and move registers elsewhere).
+        uint32_t kr[2][KDW], vr[8][VDW];
+        float nrm;
+        auto blocks = [&](int k, uint32_t& pb0, uint32_t& pb1) {
+          const int w = bs32 ? k - win_k : 2 * (k - win_k);
+          pb0 = (uint32_t)__builtin_amdgcn_readlane(pbwin, w);
+          pb1 = bs32 ? pb0 : (uint32_t)__builtin_amdgcn_readlane(pbwin, w + 1);
+        };
+        auto load_keys = [&](int k) {
+          uint32_t pb[2];
+          blocks(k, pb[0], pb[1]);
+          nrm = nptr[(uint64_t)(ntok >= 16 ? pb[1] : pb[0]) * nblk_stride + noff];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const unsigned char* p = a.kp + (uint64_t)pb[j] * (uint32_t)a.kps_blk + (j ? ktile1 : 0u) + aw_here(koff);
+            if constexpr (KDW == 1) {
+              kr[j][0] = *(const uint32_t*)p;
+            } else if constexpr (KDW == 2) {
+              const uint2 t = *(const uint2*)p;
+              kr[j][0] = t.x; kr[j][1] = t.y;
+            } else {
+#pragma unroll
+              for (int i = 0; i < KDW / 4; ++i) {
+                const uint4 t = *(const uint4*)(p + 16 * i);
+                kr[j][4 * i] = t.x; kr[j][4 * i + 1] = t.y; kr[j][4 * i + 2] = t.z; kr[j][4 * i + 3] = t.w;
+              }
+            }
+          }
+        };
+        auto load_values = [&](int k) {
+          uint32_t pb[2];
+          blocks(k, pb[0], pb[1]);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const unsigned char* vb = a.vp + (uint64_t)pb[j] * (uint32_t)a.vps_blk + (j ? vtile1 : 0u);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const unsigned char* p = vb + (uint32_t)(i * (int)a.vps_pos) + aw_here(voff);
+              if constexpr (VB == 1) vr[4 * j + i][0] = *p;
+              else if constexpr (VB == 2) vr[4 * j + i][0] = *(const uint16_t*)p;
+              else if constexpr (VB == 4) vr[4 * j + i][0] = *(const uint32_t*)p;
+              else {
+                const uint2 t = *(const uint2*)p;
+                vr[4 * j + i][0] = t.x; vr[4 * j + i][VDW - 1] = t.y;
+              }
+            }
+          }
+        };
+
+        load_window(0);
+        load_keys(0);
+        load_values(0);
+        uint2 qd[KS];
+        {
+          const uint2* qp = x.qop + (size_t)(s * a.KVH + h) * (KS * 64) + lane;
+#pragma unroll
+          for (int st = 0; st < KS; ++st) qd[st] = qp[st * 64];
+        }
+        const float fac = x.fac[(size_t)s * a.QH + h * gqa + min(col & 7, gqa - 1)] * inv_cs;
+
+        for (int k = 0; k < mine; ++k) {
+          const int c = r + k * R;
+          // ---- norms: lanes 0..31 hold the key norms, 32..63 the value norms; the exponent of a value norm bounds it
+          // from above by a power of two
+          *(aw_lds_f32*)(uintptr_t)(nbase + (uint32_t)lane * 4u) = nrm;
+          if (lane >= 32) {
+            const int e = (int)((__float_as_uint(nrm) >> 23) & 0xffu) - 126;
+            *(aw_lds_f32*)(uintptr_t)(nbase + 256u + (uint32_t)ntok * 4u) = (float)max(e, -AW_TINY);
+          }
+          aw_wave_sync();
+
+          // ---- scores
+          aw_float4 acc[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            acc[j] = (aw_float4){0.f, 0.f, 0.f, 0.f};
+            auto step = [&](int st, aw_u32x2 lo, aw_u32x2 hi) {
+              const aw_u32x2 q0 = {qd[st].x, qd[st].x}, q1 = {qd[st].y, qd[st].y};
+              acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(lo, hi), aw_operand(q0, q1), acc[j], 0, 0, 0);
+            };
+#pragma unroll
+            for (int i = 0; i < KDW; ++i) {
+              const uint32_t w = kr[j][i];
+              if constexpr (BITS == 4) {
+                step(2 * i, aw_look<0>(copy, w), aw_look<1>(copy, w));
+                step(2 * i + 1, aw_look<2>(copy, w), aw_look<3>(copy, w));
+              } else {
+                const uint32_t even = (w >> 2) & 0x33333333u, odd = w & 0x33333333u;
+                step(4 * i, aw_look<0>(copy, even), aw_look<0>(copy, odd));
+                step(4 * i + 1, aw_look<1>(copy, even), aw_look<1>(copy, odd));
+                step(4 * i + 2, aw_look<2>(copy, even), aw_look<2>(copy, odd));
+                step(4 * i + 3, aw_look<3>(copy, even), aw_look<3>(copy, odd));
+              }
+            }
+          }
+
+          __builtin_amdgcn_sched_barrier(0);
+          if (k + 1 - win_k >= AW_WIN) load_window(k + 1);
+          load_keys(min(k + 1, mine - 1));      // (past the end: the last chunk once more)
+          __builtin_amdgcn_sched_barrier(0);
+
+          // ---- running softmax in the log2 domain over t = score + exponent of the value norm
+          float sv[8], vn[8], tv[8], mx = -INFINITY;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const aw_float4 kn4 = *(aw_lds_f128*)(uintptr_t)(nread + 64u * j);
+            const aw_float4 vn4 = *(aw_lds_f128*)(uintptr_t)(nread + 128u + 64u * j);
+            const aw_float4 ve4 = *(aw_lds_f128*)(uintptr_t)(nread + 256u + 64u * j);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              sv[4 * j + i] = aw_add_cols(acc[j][i]) * (kn4[i] * fac);
+              vn[4 * j + i] = vn4[i];
+              tv[4 * j + i] = sv[4 * j + i] + ve4[i];
+            }
+          }
+          if (c == nchunks - 1) {        // only the last chunk of a segment holds tokens past its end
+            // (such a row may hold anything, NaN norms included.  The empty statement keeps this a branch: as selects the
+            // comparisons cost every chunk 24 instructions.)
+            asm volatile("");
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                if (blk_lo * bs + 32 * c + 16 * j + 4 * g + i >= t_end) { sv[4 * j + i] = -INFINITY; vn[4 * j + i] = 0.f; tv[4 * j + i] = -INFINITY; }
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) mx = fmaxf(mx, tv[i]);
+          aw_wave_sync();      // the norms have been read: the next chunk overwrites them
+          mx = akv_rows_max(mx);
+          const float m_new = fmaxf(m_run, mx - AW_FRAME);
+          const float resc = __builtin_amdgcn_exp2f(m_run - m_new);      // 0 on the first chunk
+          m_run = m_new;
+          float psum = 0.f;
+          aw_half8 wop[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            uint32_t pr[2];
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+              const float p0 = __builtin_amdgcn_exp2f(sv[4 * j + 2 * p] - m_new), p1 = __builtin_amdgcn_exp2f(sv[4 * j + 2 * p + 1] - m_new);
+              psum += p0 + p1;
+              const aw_float2 w2 = {p0 * vn[4 * j + 2 * p], p1 * vn[4 * j + 2 * p + 1]};
+              const aw_half2 h2 = __builtin_convertvector(w2, aw_half2);
+              const aw_half2 l2 = __builtin_convertvector(w2 - __builtin_convertvector(h2, aw_float2), aw_half2);
+              union { aw_half2 h; uint32_t u; } hu, lu;
+              hu.h = h2;
+              lu.h = l2;
+              pr[p] = col < 8 ? hu.u : lu.u;
+            }
+            wop[j] = aw_operand((aw_u32x2){pr[0], pr[0]}, (aw_u32x2){pr[1], pr[1]});
+          }
+          l_run = l_run * resc + psum;
+          if (__builtin_amdgcn_ballot_w64(resc != 1.f) != 0) {
+#pragma unroll
+            for (int n = 0; n < CPL; ++n)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) o[n][i] *= resc;
+          }
+
+          // ---- values
+          if constexpr (VB >= 4) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int d = 0; d < VDW; ++d) {
+                aw_pairs<BITS, 0> p01, p23;
+                aw_pair(p01, vr[4 * j][d], vr[4 * j + 1][d]);
+                aw_pair(p23, vr[4 * j + 2][d], vr[4 * j + 3][d]);
+                auto byte = [&](auto kc) __attribute__((always_inline)) {
+                  constexpr int K = decltype(kc)::value;
+#pragma unroll
+                  for (int q = 0; q < CPB; ++q) {
+                    const int n = (4 * d + K) * CPB + q;
+                    o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<K>(copy, p01.w[q]), aw_look<K>(copy, p23.w[q])), wop[j], o[n], 0, 0, 0);
+                  }
+                };
+                byte(std::integral_constant<int, 0>{}); byte(std::integral_constant<int, 1>{});
+                byte(std::integral_constant<int, 2>{}); byte(std::integral_constant<int, 3>{});
+              }
+          } else if constexpr (VB == 2) {
+            // two bytes per token: both token pairs of a tile side by side in one word
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              aw_pairs<BITS, 0> p;
+              aw_pair(p, vr[4 * j][0] | (vr[4 * j + 2][0] << 16), vr[4 * j + 1][0] | (vr[4 * j + 3][0] << 16));
+#pragma unroll
+              for (int q = 0; q < CPB; ++q) {
+                o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<0>(copy, p.w[q]), aw_look<2>(copy, p.w[q])), wop[j], o[q], 0, 0, 0);
+                o[CPB + q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<1>(copy, p.w[q]), aw_look<3>(copy, p.w[q])), wop[j], o[CPB + q], 0, 0, 0);
+              }
+            }
+          } else {
+            // one byte per token: the pairs of both tiles side by side
+            aw_pairs<BITS, 0> p;
+            auto join = [&](int t) { return vr[t][0] | (vr[t + 2][0] << 8) | (vr[t + 4][0] << 16) | (vr[t + 6][0] << 24); };
+            aw_pair(p, join(0), join(1));
+#pragma unroll
+            for (int q = 0; q < CPB; ++q) {
+              o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<0>(copy, p.w[q]), aw_look<1>(copy, p.w[q])), wop[0], o[q], 0, 0, 0);
+              o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<2>(copy, p.w[q]), aw_look<3>(copy, p.w[q])), wop[1], o[q], 0, 0, 0);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          load_values(min(k + 1, mine - 1));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        l_run = aw_rows_sum(l_run);
+      }
+
+      // ---- partial result: lane (col < gqa, g) holds coordinates CPL (4 g + i) + n of query head col
+      const size_t slot = (size_t)(blockIdx.x + s) * a.QH + h * gqa;
+      float M = m_run, wgt = inv_cs, L = l_run;
+      if (R > 1) {
+        if (lane < 8) *(aw_lds_f64*)(uintptr_t)(aw_ml_off<W>() + (uint32_t)wave * 64u + (uint32_t)lane * 8u) = (aw_float2){m_run, l_run};
+        __syncthreads();
+        L = 0.f;
+        for (int rr = 0; rr < R; ++rr) {
+          const aw_float2 ml = *(aw_lds_f64*)(uintptr_t)(aw_ml_off<W>() + (uint32_t)(rr * hp + hs) * 64u + (uint32_t)(col & 7) * 8u);
+          M = fmaxf(M, ml.x);
+        }
+        for (int rr = 0; rr < R; ++rr) {
+          const aw_float2 ml = *(aw_lds_f64*)(uintptr_t)(aw_ml_off<W>() + (uint32_t)(rr * hp + hs) * 64u + (uint32_t)(col & 7) * 8u);
+          L += ml.x > -INFINITY ? __builtin_amdgcn_exp2f(ml.x - M) * ml.y : ml.y;      // (-inf: no token, or sums that are NaN)
+        }
+        wgt = m_run > -INFINITY ? __builtin_amdgcn_exp2f(m_run - M) * inv_cs : inv_cs;
+      }
+#pragma unroll
+      for (int n = 0; n < CPL; ++n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[n][i] = aw_add_cols(o[n][i]) * wgt;
+      if (R == 1) {
+        if (active && col < gqa) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int n = 0; n < CPL; n += 4)
+              *(float4*)(a.part_acc + (slot + col) * D + CPL * (4 * g + i) + n) = make_float4(o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]);
+        }
+      } else {
+        const uint32_t wave_bytes = (uint32_t)gqa * D * 4u;
+        if (active && col < gqa) {
+          const uint32_t at = aw_acc_off<W>() + (uint32_t)wave * wave_bytes + (uint32_t)(col * D + CPL * 4 * g) * 4u;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int n = 0; n < CPL; n += 4)
+              *(aw_lds_f128*)(uintptr_t)(at + (uint32_t)(CPL * i + n) * 4u) = (aw_float4){o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]};
+        }
+        __syncthreads();
+        if (active) {
+          // (no barrier after these reads: the next segment's accumulators are written behind its first barrier)
+          for (int idx = r * 64 + lane; idx < gqa * D / 4; idx += R * 64) {
+            aw_float4 sum = {0.f, 0.f, 0.f, 0.f};
+            for (int rr = 0; rr < R; ++rr) sum += *(aw_lds_f128*)(uintptr_t)(aw_acc_off<W>() + (uint32_t)(rr * hp + hs) * wave_bytes + (uint32_t)idx * 16u);
+            *(float4*)(a.part_acc + slot * D + 4 * (size_t)idx) = make_float4(sum.x, sum.y, sum.z, sum.w);
+          }
+        }
+      }
+      if (active && r == 0 && lane < gqa) {
+        a.part_ml[(slot + lane) * 2] = M * 0.6931471805599453f;     // back to the natural-log domain
+        a.part_ml[(slot + lane) * 2 + 1] = L;
+      }
+    }
+  }
+}
+
+// ----------------------------------------------------------------------------------
+// host side
+// ----------------------------------------------------------------------------------
+bool akv_attn_mfma_takes(const akv_attn_args& a, int bits);       // the conditions both matrix-core kernels share
+int akv_attn_mfma_head_groups(int gqa);
+
+// At head_dim 128 the kernel of akv_attn_mfma.hip has eight head slots: it is left with whole slots idle below five
+// (groups of) kv heads, and takes over from there.
+bool akv_attn_wave_applicable(const akv_attn_args& a, int d, int bits) {
+  if (!(d == 64 || d == 128 || d == 256) || (bits != 4 && bits != 2) || !akv_attn_mfma_takes(a, bits)) return false;
+  return d != 128 || a.KVH * akv_attn_mfma_head_groups(a.QH / a.KVH) <= 4;
+}
+
+template <int D, int BITS>
+static int aw_launch(const akv_attn_args& a, const aw_extra& x_in, int grid, hipStream_t stream) {
+  constexpr int W = aw_cfg<D, BITS>::W;
+  aw_extra x = x_in;
+  x.hp = 1;
+  while (x.hp < a.KVH && x.hp < W) x.hp *= 2;
+  const int gqa = a.QH / a.KVH;
+  constexpr int most = (int)aw_acc_off<W>() + W * 8 * D * 4;
+  static_assert(most <= 160 * 1024, "LDS of a CU");
+  const int lds = (int)aw_acc_off<W>() + (x.hp < W ? W * gqa * D * 4 : 0);
+  static bool configured = false;
+  if (!configured) {
+    AKV_HIP(hipFuncSetAttribute((const void*)akv_attn_wave_kernel<D, BITS>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
+    configured = true;
+  }
+  AKV_LAUNCH_TIMED((akv_attn_wave_kernel<D, BITS>), grid, W * 64, lds, stream, a, x);
+  AKV_LAUNCH_CHECK("akv_attn_wave_kernel");
+  return AKV_OK;
+}
+
+int akv_attn_wave_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* PiT, const akv_attn_args& a_in,
+                      int d, int bits, const akv_attn_ws& ws, void* extra_ws, int grid, hipStream_t stream) {
+  akv_attn_args a = a_in;
+  a.hgroup = akv_attn_mfma_head_groups(a.QH / a.KVH);
+  a.KVH *= a.hgroup;                        // from here on: groups of at most eight query heads
+  aw_extra x;
+  x.qop = (const uint2*)extra_ws;           // 32 d bytes per group: at most what the other kernel's operand takes (d <= 256)
+  x.fac = ws.qrot;
+  x.wgdesc = ws.wgdesc;
+  x.hp = 0;
+  const float qscale = a.scale * 1.4426950408889634f;   // scores come out in the log2 domain
+  // rotation blocks: one per query head, up to what the CUs hold at once (then they loop: the matrix is read once per block)
+  const int cus = akv_cached_cu_count();
+  auto pgrid = [&](int dd) {
+    const int64_t most = (int64_t)(cus > 0 ? cus : 256) * (dd == 256 ? 1 : 4) / (dd == 256 ? 2 : 1), items = (int64_t)a.S * a.QH;
+    return (int)(items < most ? items : most) + 1;
+  };
+#define AW_PRO(DD, DT) akv_attn_wave_prologue_kernel<DD, DT><<<pgrid(DD), aw_pro_threads<DD>(), 0, stream>>>(query, qs_seq, qs_head, PiT, a.S, a.QH, a.KVH, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint2*)extra_ws, ws.qrot, ws.status, qscale, bits, ws.wgdesc, ws.seqw, grid)
+#define AW_PRO_D(DD) do { if (q_dtype == AKV_F16) AW_PRO(DD, AKV_F16); else if (q_dtype == AKV_BF16) AW_PRO(DD, AKV_BF16); else AW_PRO(DD, AKV_F32); } while (0)
+  if (d == 64) AW_PRO_D(64); else if (d == 128) AW_PRO_D(128); else AW_PRO_D(256);
+#undef AW_PRO_D
+#undef AW_PRO
+  AKV_LAUNCH_CHECK("akv_attn_wave_prologue_kernel");
+  if (d == 64) return bits == 4 ? aw_launch<64, 4>(a, x, grid, stream) : aw_launch<64, 2>(a, x, grid, stream);
+  if (d == 128) return bits == 4 ? aw_launch<128, 4>(a, x, grid, stream) : aw_launch<128, 2>(a, x, grid, stream);
+  return bits == 4 ? aw_launch<256, 4>(a, x, grid, stream) : aw_launch<256, 2>(a, x, grid, stream);
+}

@@ -1,0 +1,117 @@
+"""Paged attention kernel whose wavefronts work on their own (head_dim 64 and 256; head_dim 128 with at most four kv heads),
+at the edges of its tiles, chunks, head slots and block-id windows, against float64."""
+import numpy as np
+import pytest
+import torch
+
+import aitherkvcache_amd as akv
+from oracle import tq_oracle as O
+from tests.util import kv_like
+
+pytestmark = pytest.mark.gpu
+
+# float32 outputs: the rounding of a few float32 sums and exponentials, 2 ** -23 each; scores of some tens carry it into
+# their exponentials.  Measured up to 8e-7.
+REL = 5e-6
+
+
+def make(dev, d, bits, kvh, blocks, bs, seed, pad=4):
+    rng = np.random.default_rng(seed)
+    tq = akv.TurboQuant(head_dim=d, bits=bits, device=str(dev), dtype=torch.float32)
+    rows = [torch.full((blocks, bs, kvh, tq._packed_dim + pad), 0x5A, dtype=torch.uint8, device=dev) for _ in range(2)]
+    norms = [torch.zeros(blocks, bs, kvh, device=dev) for _ in range(2)]
+    slots = torch.arange(blocks * bs, device=dev)
+    for r, n in zip(rows, norms):
+        x = torch.from_numpy(kv_like(rng, (blocks * bs, kvh, d)).astype(np.float32)).to(dev)
+        akv.fused_kv_update(x, slots, r[..., :tq._packed_dim], n, tq.rotation, tq.boundaries_inner, bits, bs)
+    return rng, tq, rows, norms
+
+
+def dequantised(tq, rows, norms, d, bits):
+    c, _, _ = O.get_codebook(d, bits)
+    codes = O._UNPACK[bits](rows[..., :tq._packed_dim].cpu().numpy(), d)
+    return torch.from_numpy(np.asarray(c, dtype=np.float64)[codes] * norms.double().cpu().numpy()[..., None])
+
+
+def attend(q, K, V, R, counts=None):
+    """q [heads, d], K and V [tokens, kv heads, d] in the rotated frame, each token `counts` times; float64."""
+    heads, kvh = q.shape[0], K.shape[1]
+    out = torch.zeros_like(q)
+    for h in range(heads):
+        s = K[:, h // (heads // kvh)] @ (R @ q[h]) / q.shape[1] ** 0.5
+        p = torch.exp(s - s.max()) * (1.0 if counts is None else counts)
+        out[h] = R.T @ (p @ V[:, h // (heads // kvh)] / p.sum())
+    return out
+
+
+HEADS = [(8, 1, 16), (16, 2, 32), (9, 3, 16), (28, 4, 16), (24, 2, 32), (5, 5, 32), (40, 8, 16), (18, 18, 16)]
+
+
+@pytest.mark.parametrize("d,bits,qh,kvh,bs", [(d, bits, *h) for d in (64, 128, 256) for bits in (4, 2) for h in HEADS if d != 128 or h[1] <= 4])
+def test_edges_vs_float64(dev, d, bits, qh, kvh, bs):
+    """Contexts at the edges of blocks, tiles and chunks, empty sequences; one to eight heads a kv head, groups of them beyond
+    eight, head slots left over, more heads than slots."""
+    ctx = np.array([1, 0, 15, 16, 17, 31, 32, 33, 64, 65, 257, 1000, 0, 3], dtype=np.int32)
+    need = -(-ctx // bs)
+    blocks = int(need.sum()) + 2
+    rng, tq, rows, norms = make(dev, d, bits, kvh, blocks, bs, d + bits + qh)
+    tables = np.full((len(ctx), int(need.max())), 10 ** 6, dtype=np.int32)
+    order, at = rng.permutation(blocks), 0
+    for i, n in enumerate(need):
+        tables[i, :n] = order[at:at + n]
+        at += int(n)
+    q = torch.from_numpy(rng.standard_normal((len(ctx), qh, d)).astype(np.float32)).to(dev)
+    P = tq._packed_dim
+    print(f"[attn wave] d={d} bits={bits} qh={qh} kvh={kvh} bs={bs}", flush=True)
+    out = akv.TQPagedAttention(tq, qh).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.from_numpy(tables).to(dev),
+                                               torch.from_numpy(ctx).to(dev), block_size=bs).double().cpu()
+    K, V = (dequantised(tq, r, n, d, bits) for r, n in zip(rows, norms))
+    R = tq.rotation.double().cpu()
+    for i, n in enumerate(ctx):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        t = torch.from_numpy(tables[i, :need[i]].astype(np.int64))
+        k, v = (x[t].reshape(-1, kvh, d)[:n] for x in (K, V))
+        ref = attend(q[i].double().cpu(), k, v, R)
+        assert (out[i] - ref).norm() <= REL * ref.norm(), (i, n)
+
+
+@pytest.mark.parametrize("d,qh,kvh,bs", [(256, 16, 8, 16), (256, 4, 1, 32), (64, 16, 16, 32)])
+def test_more_chunks_than_a_window_of_block_ids(dev, d, qh, kvh, bs):
+    """A context so long that a wavefront goes through several windows of block ids: its blocks repeat a few, which the
+    reference counts."""
+    rng, tq, rows, norms = make(dev, d, 4, kvh, 8, bs, 7)
+    shares = 8 // kvh if kvh < 8 else 1
+    n = 32 * 256 * 70 * shares - 5                       # 70 chunks a wavefront, or one less
+    table = rng.integers(0, 8, size=-(-n // bs)).astype(np.int32)
+    q = torch.from_numpy(rng.standard_normal((1, qh, d)).astype(np.float32)).to(dev)
+    P = tq._packed_dim
+    out = akv.TQPagedAttention(tq, qh).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.from_numpy(table[None]).to(dev),
+                                               torch.tensor([n], dtype=torch.int32, device=dev), block_size=bs).double().cpu()
+    counts = np.zeros((8, bs))
+    np.add.at(counts, table[:-1], 1.0)
+    counts[table[-1], :n - (len(table) - 1) * bs] += 1.0
+    K, V = (dequantised(tq, r, x, d, 4).reshape(-1, kvh, d) for r, x in zip(rows, norms))
+    ref = attend(q[0].double().cpu(), K, V, tq.rotation.double().cpu(), torch.from_numpy(counts.reshape(-1)))
+    # sums of 2^19 and more float32 terms in runs of some thousand: their rounding walks to a few times that of the test above
+    assert (out[0] - ref).norm() <= 4 * REL * ref.norm()
+
+
+@pytest.mark.parametrize("d,bits", [(64, 4), (256, 2), (128, 4)])
+@pytest.mark.parametrize("scale_v,scale_q", [(1e30, 1.0), (1e-30, 1.0), (1.0, 1e-20), (1.0, 1e20)])
+def test_norms_and_queries_far_outside_float16(dev, d, bits, scale_v, scale_q):
+    """Value norms and queries float16 cannot hold (keys scaled against the queries), and NaN rows past the context."""
+    rng, tq, rows, norms = make(dev, d, bits, 2, 8, 16, 3)
+    n = 100
+    norms[0] /= scale_q
+    norms[1] *= scale_v
+    norms[0].view(-1, 2)[n:] = float("nan")
+    norms[1].view(-1, 2)[n:] = float("nan")
+    q = torch.from_numpy(rng.standard_normal((1, 8, d)).astype(np.float32)).to(dev) * scale_q
+    P = tq._packed_dim
+    out = akv.TQPagedAttention(tq, 8).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.arange(8, dtype=torch.int32, device=dev)[None],
+                                              torch.tensor([n], dtype=torch.int32, device=dev), block_size=16).double().cpu()
+    K, V = (dequantised(tq, r, x, d, bits).reshape(-1, 2, d)[:n] for r, x in zip(rows, norms))
+    ref = attend(q[0].double().cpu(), K, V, tq.rotation.double().cpu())
+    assert (out[0] - ref).norm() <= REL * ref.norm()
