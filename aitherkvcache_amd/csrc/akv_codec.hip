@@ -550,6 +550,12 @@ static int akv_encode_dispatch(int d, int bits, int dt, const akv_gen_args& a, v
 // MFMA fast path (akv_encode_mfma.hip); returns AKV_ERR_UNSUPPORTED when it does not apply.
 int akv_encode_mfma_try(const akv_gen_args& a, bool paged, int x_dtype, int d, int bits,
                         const void* rot_prep, hipStream_t stream);
+// the same at head_dim 64 and 256 (akv_encode_wide.hip)
+int akv_encode_wide_try(const akv_gen_args& a, bool paged, int x_dtype, int d, int bits, const void* rot_prep, hipStream_t stream);
+static int akv_encode_matrix_try(const akv_gen_args& a, bool paged, int x_dtype, int d, int bits, const void* rot_prep, hipStream_t stream) {
+  if (d == 128) return akv_encode_mfma_try(a, paged, x_dtype, d, bits, rot_prep, stream);
+  return akv_encode_wide_try(a, paged, x_dtype, d, bits, rot_prep, stream);
+}
 
 static int akv_check_codec_args(const char* fn, int d, int bits) {
   if (!(d == 64 || d == 128 || d == 256 || d == 512))
@@ -575,7 +581,7 @@ extern "C" int akv_encode(const void* x, int x_dtype, int64_t n, int d, int64_t 
   a.table = boundaries;
   a.packed = out_packed; a.ps0 = packed_stride;
   a.norms = out_norms;
-  rc = akv_encode_mfma_try(a, false, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
+  rc = akv_encode_matrix_try(a, false, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
   if (rc != AKV_ERR_UNSUPPORTED) return rc;
   return akv_encode_dispatch<false>(d, bits, x_dtype, a, stream);
 }
@@ -603,7 +609,7 @@ extern "C" int akv_encode_paged_kv(const void* k, const void* v, int x_dtype, in
   a.packed = k_packed; a.ps0 = ps_blk; a.ps1 = ps_pos; a.ps2 = ps_head;
   a.norms = k_norms; a.ns0 = ns_blk; a.ns1 = ns_pos; a.ns2 = ns_head;
   a.x2 = v; a.packed2 = v_packed; a.norms2 = v_norms;
-  rc = akv_encode_mfma_try(a, true, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
+  rc = akv_encode_matrix_try(a, true, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
   if (rc != AKV_ERR_UNSUPPORTED) return rc;
   // layouts the matrix-core kernel does not take: one launch per tensor
   akv_gen_args b = a;
@@ -635,7 +641,7 @@ extern "C" int akv_encode_paged(const void* x, int x_dtype, int64_t num_tokens, 
   a.table = boundaries;
   a.packed = out_packed; a.ps0 = ps_blk; a.ps1 = ps_pos; a.ps2 = ps_head;
   a.norms = out_norms; a.ns0 = ns_blk; a.ns1 = ns_pos; a.ns2 = ns_head;
-  rc = akv_encode_mfma_try(a, true, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
+  rc = akv_encode_matrix_try(a, true, x_dtype, d, bits, rot_prep, (hipStream_t)stream);
   if (rc != AKV_ERR_UNSUPPORTED) return rc;
   return akv_encode_dispatch<true>(d, bits, x_dtype, a, stream);
 }

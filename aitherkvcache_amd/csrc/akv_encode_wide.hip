@@ -1,0 +1,278 @@
+// MFMA encode (norm -> rotate -> codebook search -> pack -> store) at head_dim 64 and 256 for float16, bfloat16 and float32
+// input, flat rows or scattered through a slot mapping (K and V of a step in one launch).
+//
+//   Y[row, j] = sum_i X[row, i] Pi[j, i]              v_mfma_f32_16x16x32_f16
+//
+// Wavefront w of a workgroup owns output coordinates 16 w .. 16 w + 15 and keeps its 16 x D slice of Pi in registers,
+// split into two float16 terms from the float32 matrix at its start.  A workgroup takes 16 MT rows at a time: its threads
+// load them (four neighbouring elements each), reduce the squared norms over the lanes of a row and leave the rows in LDS;
+// every wavefront multiplies all of them by its slice and searches the codebook; the codes meet in LDS and are packed by
+// the byte.  Two barriers a step, the next rows requested before the first.
+//
+// Precision: float16 rows are exact in the operand.  bfloat16 and float32 rows are scaled by the power of two that
+// brings the largest element to [2^10, 2^11): bfloat16 is then exact (down to 2^-34 of the largest element), float32 is
+// split into two terms like the matrix (2^-23 of the element, the product of two remainders left out).  The general
+// kernel's chain of float32 sums is no closer to 64 bits.
+//
+// What bounds it: a decode step (192 to 768 rows) is one step per workgroup, a chain of trips to memory: matrix and rows,
+// slots, stores.  Large calls are bound by the search, two vector instructions per boundary and value.
+#include "akv_common.h"
+
+typedef _Float16 ew_half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 ew_half4 __attribute__((ext_vector_type(4)));
+typedef float ew_float4 __attribute__((ext_vector_type(4)));
+
+#define EW_PI_SCALE 1024.f
+#define EW_PI_EXP 10
+
+template <int D, int MT, int XDT> struct ew_cfg {
+  static constexpr int WAVES = D / 16, THREADS = WAVES * 64, ROWS = 16 * MT;
+  static constexpr int TPR = D / 4;                        // threads of a row while loading
+  static constexpr int KS = D / 32;
+  static constexpr int PITCH = D + 8;                      // float16 per row in LDS (16 bytes more: eight rows meet all banks)
+  static constexpr int NA = XDT == AKV_F32 ? 2 : 1;        // float16 terms of a row
+};
+
+// four elements of a row as they lie in memory
+template <int XDT> struct ew_piece { typedef uint2 type; };
+template <> struct ew_piece<AKV_F32> { typedef uint4 type; };
+template <int XDT> __device__ __forceinline__ void ew_floats(const typename ew_piece<XDT>::type& r, float (&x)[4]) {
+  if constexpr (XDT == AKV_F32) {
+    x[0] = __uint_as_float(r.x); x[1] = __uint_as_float(r.y); x[2] = __uint_as_float(r.z); x[3] = __uint_as_float(r.w);
+  } else if constexpr (XDT == AKV_BF16) {
+    x[0] = __uint_as_float(r.x << 16); x[1] = __uint_as_float(r.x & 0xffff0000u);
+    x[2] = __uint_as_float(r.y << 16); x[3] = __uint_as_float(r.y & 0xffff0000u);
+  } else {
+    union { uint2 u; ew_half4 h; } cv;
+    cv.u = r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = (float)cv.h[i];
+  }
+}
+
+template <int D, int BITS, int XDT, bool PAGED, int MT>
+__global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kernel(akv_gen_args a, const float* __restrict__ Pi) {
+  typedef ew_cfg<D, MT, XDT> cfg;
+  typedef typename ew_piece<XDT>::type piece_t;
+  constexpr int ROWS = cfg::ROWS, TPR = cfg::TPR, KS = cfg::KS, PITCH = cfg::PITCH, NA = cfg::NA, THREADS = cfg::THREADS;
+  constexpr int NB = (1 << BITS) - 1;
+  constexpr int XB = XDT == AKV_F32 ? 4 : 2;
+  __shared__ __align__(16) _Float16 rows[NA][ROWS][PITCH];
+  __shared__ __align__(16) uint8_t codes[ROWS][D + 16];
+  __shared__ float4 info[ROWS];                            // reciprocal of the norm, exponent to put back, norm, not finite
+  __shared__ int64_t dst[2][ROWS];                         // [parity of the step] address of the packed row, 0 = skip
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int col = lane & 15, g = lane >> 4;
+  const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n;
+  const int64_t steps = (n_total + ROWS - 1) / ROWS;
+
+  // ---- rows: thread (row, part) of piece i
+  piece_t R[MT];
+  auto fetch = [&](int64_t step) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int u = tid + i * THREADS;
+      int64_t n = step * ROWS + u / TPR;
+      if (n >= n_total) n = n_total - 1;                   // past the end: loaded, not stored
+      const bool second = PAGED && n >= a.n;
+      if (second) n -= a.n;
+      int64_t off;
+      if constexpr (PAGED) {
+        const uint32_t tok = (uint32_t)n / (uint32_t)a.heads, head = (uint32_t)n - tok * (uint32_t)a.heads;
+        off = (int64_t)tok * a.xs0 + (int64_t)head * a.xs1;
+      } else {
+        off = n * a.xs0;
+      }
+      R[i] = *(const piece_t*)((const char*)(second ? a.x2 : a.x) + XB * (off + 4 * (u % TPR)));
+    }
+  };
+  fetch(blockIdx.x);
+
+  // ---- the wavefront's slice of Pi: lane (col, g) holds row 16 wave + col, elements 32 ks + 8 g + e
+  ew_half8 Bh[KS], Bl[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const float4* p = (const float4*)(Pi + (size_t)(16 * wave + col) * D + 32 * ks + 8 * g);
+    const float4 p0 = p[0], p1 = p[1];
+    const float v[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float s = v[e] * EW_PI_SCALE;
+      const _Float16 h = (_Float16)s;
+      Bh[ks][e] = h;
+      Bl[ks][e] = (_Float16)(s - (float)h);
+    }
+  }
+  float bnd[NB];
+#pragma unroll
+  for (int k = 0; k < NB; ++k) bnd[k] = a.table[k];
+
+  int par = 0;
+  for (int64_t step = blockIdx.x; step < steps; step += gridDim.x, par ^= 1) {
+    // ---- norm, conversion, rows into LDS
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int u = tid + i * THREADS, row = u / TPR, part = u % TPR;
+      float x[4];
+      ew_floats<XDT>(R[i], x);
+      float ss = 0.f, mx = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ss = fmaf(x[e], x[e], ss);
+        mx = fmaxf(mx, fabsf(x[e]));
+      }
+      ss += akv_lane_xor<1>(ss); ss += akv_lane_xor<2>(ss); ss += akv_lane_xor<4>(ss); ss += akv_lane_xor<8>(ss);
+      mx = fmaxf(mx, akv_lane_xor<1>(mx)); mx = fmaxf(mx, akv_lane_xor<2>(mx));
+      mx = fmaxf(mx, akv_lane_xor<4>(mx)); mx = fmaxf(mx, akv_lane_xor<8>(mx));
+      if constexpr (TPR == 64) {
+        ss += akv_lane_xor<16>(ss); ss += akv_lane_xor<32>(ss);
+        mx = fmaxf(mx, akv_lane_xor<16>(mx)); mx = fmaxf(mx, akv_lane_xor<32>(mx));
+      }
+      // a row with a NaN (its sum is NaN) or an infinity rotates to NaN everywhere; a finite row whose squares overflow
+      // has norm inf and rotates to zero
+      const bool bad = ss != ss || !(mx < INFINITY);
+      int put_back = -EW_PI_EXP;
+      union { ew_half4 h; uint2 u; } hi, lo;
+      if constexpr (XDT == AKV_F16) {
+        hi.u = R[i];
+      } else {
+        const int ef = bad ? 127 : (int)(__float_as_uint(mx) >> 23);
+        const int sef = min(254, 264 - ef);
+        const float sc = __uint_as_float((uint32_t)sef << 23);         // 2^(sef - 127)
+        put_back += 127 - sef;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float s = x[e] * sc;
+          hi.h[e] = (_Float16)s;
+          lo.h[e] = (_Float16)(s - (float)hi.h[e]);
+        }
+      }
+      *(uint2*)&rows[0][row][4 * part] = hi.u;
+      if constexpr (NA == 2) *(uint2*)&rows[NA - 1][row][4 * part] = lo.u;
+      if (part == 0) {
+        const float nrm = sqrtf(ss);
+        info[row] = make_float4(1.f / (nrm + 1e-10f), __int_as_float(put_back), nrm, bad ? 1.f : 0.f);
+      }
+    }
+    // ---- thread r resolves row r of the step
+    float* norm_at = nullptr;
+    if (tid < ROWS) {
+      int64_t n = step * ROWS + tid, dp = 0;
+      if (n < n_total) {
+        const bool second = PAGED && n >= a.n;
+        if (second) n -= a.n;
+        uint8_t* pb = second ? a.packed2 : a.packed;
+        float* nb = second ? a.norms2 : a.norms;
+        if constexpr (PAGED) {
+          const uint32_t tok = (uint32_t)n / (uint32_t)a.heads, head = (uint32_t)n - tok * (uint32_t)a.heads;
+          const int64_t slot = akv_load_index(a.slots, a.slot_itype, tok);
+          if (slot >= 0) {
+            const int64_t blk = slot / a.block_size, pos = slot - blk * a.block_size;
+            if (blk < a.max_blocks) {
+              dp = (int64_t)(uintptr_t)(pb + blk * a.ps0 + pos * a.ps1 + (int64_t)head * a.ps2);
+              norm_at = nb + blk * a.ns0 + pos * a.ns1 + (int64_t)head * a.ns2;
+            }
+          }
+        } else {
+          dp = (int64_t)(uintptr_t)(pb + n * a.ps0);
+          norm_at = nb + n;
+        }
+      }
+      dst[par][tid] = dp;
+    }
+    if (step + gridDim.x < steps) fetch(step + gridDim.x);
+    __syncthreads();
+    if (norm_at != nullptr) *norm_at = info[tid].z;
+
+    // ---- rotate and search: lane (col, g) ends up with rows 16 mt + 4 g + i of coordinate 16 wave + col
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      ew_float4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const ew_half8 x = *(const ew_half8*)&rows[0][16 * mt + col][32 * ks + 8 * g];
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, Bh[ks], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, Bl[ks], acc, 0, 0, 0);
+        if constexpr (NA == 2) {
+          const ew_half8 xl = *(const ew_half8*)&rows[NA - 1][16 * mt + col][32 * ks + 8 * g];
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, Bh[ks], acc, 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 f = info[16 * mt + 4 * g + i];
+        const float y = ldexpf(acc[i] * f.x, __float_as_int(f.y));
+        uint32_t c = 0;
+#pragma unroll
+        for (int k = 0; k < NB; ++k) c += bnd[k] < y ? 1u : 0u;
+        if (f.w != 0.f || y != y) c = NB;                  // NaN lies past every boundary
+        codes[16 * mt + 4 * g + i][16 * wave + col] = (uint8_t)c;
+      }
+    }
+    __syncthreads();
+
+    // ---- pack and store: eight codes are BITS bytes
+    for (int u = tid; u < ROWS * (D / 8); u += THREADS) {
+      const int row = u / (D / 8), part = u % (D / 8);
+      const int64_t dp = dst[par][row];
+      if (dp == 0) continue;
+      const uint2 c = *(const uint2*)&codes[row][8 * part];
+      uint8_t* p = (uint8_t*)(uintptr_t)dp + BITS * part;
+      // first code in the top bits
+      auto four = [](uint32_t v) { return ((v & 0xffu) << (3 * BITS)) | (((v >> 8) & 0xffu) << (2 * BITS)) | (((v >> 16) & 0xffu) << BITS) | (v >> 24); };
+      const uint32_t w = (four(c.x) << (4 * BITS)) | four(c.y);
+      if constexpr (BITS == 4) {
+        *(uint32_t*)p = __builtin_bswap32(w);
+      } else if constexpr (BITS == 2) {
+        *(uint16_t*)p = (uint16_t)((w >> 8) | (w << 8));
+      } else {
+        p[0] = (uint8_t)(w >> 16);
+        p[1] = (uint8_t)(w >> 8);
+        p[2] = (uint8_t)w;
+      }
+    }
+    // (the rows of the next step go where this one's were: read before the second barrier.  Its codes are written behind
+    // its first barrier, its destinations to the other parity.)
+  }
+}
+
+template <int D, int BITS, int XDT, bool PAGED, int MT>
+static int ew_launch(const akv_gen_args& a, const float* Pi, hipStream_t stream) {
+  typedef ew_cfg<D, MT, XDT> cfg;
+  const int cus = akv_cached_cu_count();
+  const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n, steps = (n_total + cfg::ROWS - 1) / cfg::ROWS;
+  const int64_t most = (int64_t)(cus > 0 ? cus : 256) * (D == 256 ? 1 : 4);
+  AKV_LAUNCH_TIMED((akv_encode_wide_kernel<D, BITS, XDT, PAGED, MT>), (int)(steps < most ? steps : most), cfg::THREADS, 0, stream, a, Pi);
+  AKV_LAUNCH_CHECK("akv_encode_wide_kernel");
+  return AKV_OK;
+}
+// More rows a step once every workgroup has several steps: a barrier is then shared by more products
+template <int D, int BITS, int XDT, bool PAGED>
+static int ew_launch_rows(const akv_gen_args& a, const float* Pi, hipStream_t stream) {
+  const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n;
+  return n_total > 16384 ? ew_launch<D, BITS, XDT, PAGED, D == 256 ? 2 : 4>(a, Pi, stream) : ew_launch<D, BITS, XDT, PAGED, 1>(a, Pi, stream);
+}
+template <int D, int BITS>
+static int ew_launch_dt(int x_dtype, bool paged, const akv_gen_args& a, const float* Pi, hipStream_t stream) {
+  if (x_dtype == AKV_F16) return paged ? ew_launch_rows<D, BITS, AKV_F16, true>(a, Pi, stream) : ew_launch_rows<D, BITS, AKV_F16, false>(a, Pi, stream);
+  if (x_dtype == AKV_BF16) return paged ? ew_launch_rows<D, BITS, AKV_BF16, true>(a, Pi, stream) : ew_launch_rows<D, BITS, AKV_BF16, false>(a, Pi, stream);
+  return paged ? ew_launch_rows<D, BITS, AKV_F32, true>(a, Pi, stream) : ew_launch_rows<D, BITS, AKV_F32, false>(a, Pi, stream);
+}
+
+// AKV_ERR_UNSUPPORTED: a shape or an alignment the general kernel takes
+int akv_encode_wide_try(const akv_gen_args& a, bool paged, int x_dtype, int d, int bits, const void* rot_prep, hipStream_t stream) {
+  static const bool disabled = [] { const char* e = getenv("AKV_DISABLE_MFMA"); return e && e[0] == '1'; }();
+  if ((d != 64 && d != 256) || disabled) return AKV_ERR_UNSUPPORTED;
+  if (paged && a.n >= ((int64_t)1 << 31)) return AKV_ERR_UNSUPPORTED;         // rows are divided by the heads in 32 bits
+  // rows are read four elements at a time and written four (4-bit) or two (2-bit) bytes at a time
+  const uintptr_t xa = x_dtype == AKV_F32 ? 15 : 7, pa = bits == 4 ? 3 : bits == 2 ? 1 : 0;
+  const uintptr_t xb = x_dtype == AKV_F32 ? 4 : 2;
+  if ((((uintptr_t)a.x | (uintptr_t)a.x2 | (uintptr_t)a.xs0 * xb | (uintptr_t)(paged ? a.xs1 : 0) * xb) & xa) != 0) return AKV_ERR_UNSUPPORTED;
+  if ((((uintptr_t)a.packed | (uintptr_t)a.packed2 | (uintptr_t)a.ps0 | (uintptr_t)(paged ? a.ps1 | a.ps2 : 0)) & pa) != 0) return AKV_ERR_UNSUPPORTED;
+  const float* Pi = (const float*)rot_prep;
+#define EW_CASE(DD, BB) if (d == DD && bits == BB) return ew_launch_dt<DD, BB>(x_dtype, paged, a, Pi, stream)
+  EW_CASE(64, 2); EW_CASE(64, 3); EW_CASE(64, 4);
+  EW_CASE(256, 2); EW_CASE(256, 3); EW_CASE(256, 4);
+#undef EW_CASE
+  return AKV_ERR_UNSUPPORTED;
+}
