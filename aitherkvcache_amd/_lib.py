@@ -45,6 +45,8 @@ SIGNATURES = {
     "akv_decode": (_i, [_p, _i64, _p, _i64, _i, _p, _p, _i, _p, _i, _i64, _p]),
     "akv_decode_blocks": (_i, [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i, _i64, _i64,
                                _i, _i, _i, _p, _p, _i, _p, _i, _i64, _i64, _i64, _p]),
+    "akv_decode_blocks_kv": (_i, [_p, _p, _i64, _i64, _i64, _p, _p, _i64, _i64, _i64, _p, _i, _i64, _i64,
+                                  _i, _i, _i, _p, _p, _i, _p, _p, _i, _i64, _i64, _i64, _p]),
     "akv_paged_attn_workspace_bytes": (_sz, [_i, _i, _i]),
     "akv_paged_attn": (_i, [_p, _i, _i64, _i64,
                             _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,

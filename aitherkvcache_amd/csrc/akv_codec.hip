@@ -693,28 +693,61 @@ extern "C" int akv_decode(const uint8_t* packed, int64_t packed_stride, const fl
 // Decode of whole cache blocks in place of the reference's gather + decode + scatter
 // (aither_kvcache/vllm/backend.py:1040-1091): every block id in `block_ids` that lies in
 // [0, num_blocks) is decoded from the packed cache into the block of the same index of `out`.
+static int akv_decode_blocks_impl(const char* fn, akv_gen_args& a, const void* block_ids, int ids_itype, int64_t num_ids,
+                                  int64_t num_blocks, int block_size, int num_kv_heads, int d, const void* rot_prep,
+                                  const float* centroids, int bits, int out_dtype, void* stream) {
+  AKV_REQUIRE(num_ids >= 0 && num_blocks >= 0 && block_size > 0 && num_kv_heads > 0, "%s: bad sizes", fn);
+  AKV_REQUIRE(akv_valid_dtype(out_dtype) && akv_valid_itype(ids_itype), "%s: bad dtype", fn);
+  int rc = akv_check_codec_args(fn, d, bits);
+  if (rc) return rc;
+  if (num_ids == 0 || num_blocks == 0) return AKV_OK;
+  AKV_REQUIRE(a.packed && a.norms && block_ids && rot_prep && centroids && a.out, "%s: null pointer", fn);
+  a.n = num_ids * block_size * num_kv_heads;
+  a.heads = num_kv_heads; a.block_size = block_size; a.max_blocks = num_blocks;
+  a.slots = block_ids; a.slot_itype = ids_itype;
+  a.mat = (const float*)rot_prep;
+  a.table = centroids;
+  rc = akv_decode_mfma_try(a, true, d, bits, out_dtype, rot_prep, (hipStream_t)stream);
+  if (rc != AKV_ERR_UNSUPPORTED) return rc;
+  // shapes the matrix-core kernel does not take: tensor by tensor
+  akv_gen_args b = a;
+  b.packed2 = nullptr; b.norms2 = nullptr; b.out2 = nullptr;
+  for (int second = 0; second < (a.packed2 != nullptr ? 2 : 1); ++second) {
+    if (second) { b.packed = a.packed2; b.norms = a.norms2; b.out = a.out2; }
+    rc = a.packed2 != nullptr ? akv_decode_mfma_try(b, true, d, bits, out_dtype, rot_prep, (hipStream_t)stream) : AKV_ERR_UNSUPPORTED;
+    if (rc == AKV_ERR_UNSUPPORTED) rc = akv_decode_dispatch<true>(d, bits, out_dtype, b, stream);
+    if (rc) return rc;
+  }
+  return AKV_OK;
+}
+
 extern "C" int akv_decode_blocks(const uint8_t* packed, int64_t ps_blk, int64_t ps_pos, int64_t ps_head,
                                  const float* norms, int64_t ns_blk, int64_t ns_pos, int64_t ns_head,
                                  const void* block_ids, int ids_itype, int64_t num_ids, int64_t num_blocks,
                                  int block_size, int num_kv_heads, int d, const void* rot_prep,
                                  const float* centroids, int bits, void* out, int out_dtype, int64_t os_blk,
                                  int64_t os_pos, int64_t os_head, void* stream) {
-  AKV_REQUIRE(num_ids >= 0 && num_blocks >= 0 && block_size > 0 && num_kv_heads > 0, "akv_decode_blocks: bad sizes");
-  AKV_REQUIRE(akv_valid_dtype(out_dtype) && akv_valid_itype(ids_itype), "akv_decode_blocks: bad dtype");
-  int rc = akv_check_codec_args("akv_decode_blocks", d, bits);
-  if (rc) return rc;
-  if (num_ids == 0 || num_blocks == 0) return AKV_OK;
-  AKV_REQUIRE(packed && norms && block_ids && rot_prep && centroids && out, "akv_decode_blocks: null pointer");
   akv_gen_args a = {};
-  a.n = num_ids * block_size * num_kv_heads;
-  a.heads = num_kv_heads; a.block_size = block_size; a.max_blocks = num_blocks;
-  a.slots = block_ids; a.slot_itype = ids_itype;
-  a.mat = (const float*)rot_prep;
-  a.table = centroids;
   a.packed = const_cast<uint8_t*>(packed); a.ps0 = ps_blk; a.ps1 = ps_pos; a.ps2 = ps_head;
   a.norms = const_cast<float*>(norms); a.ns0 = ns_blk; a.ns1 = ns_pos; a.ns2 = ns_head;
   a.out = out; a.os0 = os_blk; a.os1 = os_pos; a.os2 = os_head;
-  rc = akv_decode_mfma_try(a, true, d, bits, out_dtype, rot_prep, (hipStream_t)stream);
-  if (rc != AKV_ERR_UNSUPPORTED) return rc;
-  return akv_decode_dispatch<true>(d, bits, out_dtype, a, stream);
+  return akv_decode_blocks_impl("akv_decode_blocks", a, block_ids, ids_itype, num_ids, num_blocks, block_size, num_kv_heads, d,
+                                rot_prep, centroids, bits, out_dtype, stream);
+}
+
+// K and V of the listed blocks, same shapes and strides, in one launch
+extern "C" int akv_decode_blocks_kv(const uint8_t* k_packed, const uint8_t* v_packed, int64_t ps_blk, int64_t ps_pos,
+                                    int64_t ps_head, const float* k_norms, const float* v_norms, int64_t ns_blk,
+                                    int64_t ns_pos, int64_t ns_head, const void* block_ids, int ids_itype, int64_t num_ids,
+                                    int64_t num_blocks, int block_size, int num_kv_heads, int d, const void* rot_prep,
+                                    const float* centroids, int bits, void* k_out, void* v_out, int out_dtype,
+                                    int64_t os_blk, int64_t os_pos, int64_t os_head, void* stream) {
+  AKV_REQUIRE(num_ids <= 0 || num_blocks <= 0 || (v_packed && v_norms && v_out), "akv_decode_blocks_kv: null pointer");
+  akv_gen_args a = {};
+  a.packed = const_cast<uint8_t*>(k_packed); a.ps0 = ps_blk; a.ps1 = ps_pos; a.ps2 = ps_head;
+  a.norms = const_cast<float*>(k_norms); a.ns0 = ns_blk; a.ns1 = ns_pos; a.ns2 = ns_head;
+  a.out = k_out; a.os0 = os_blk; a.os1 = os_pos; a.os2 = os_head;
+  a.packed2 = const_cast<uint8_t*>(v_packed); a.norms2 = const_cast<float*>(v_norms); a.out2 = v_out;
+  return akv_decode_blocks_impl("akv_decode_blocks_kv", a, block_ids, ids_itype, num_ids, num_blocks, block_size, num_kv_heads,
+                                d, rot_prep, centroids, bits, out_dtype, stream);
 }

@@ -107,6 +107,7 @@ struct akv_gen_args {
   // decode output
   void* out;
   int64_t os0, os1, os2;  // flat: os0 = row stride; block-wise decode: blk, pos, head strides (elements)
+  void* out2;             // block-wise decode of a second tensor (packed2, norms2) in the same launch
 };
 
 // ----------------------------------------------------------------------------------

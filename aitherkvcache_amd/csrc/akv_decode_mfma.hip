@@ -1,60 +1,52 @@
-// MFMA decode (unpack -> centroid lookup -> inverse rotation -> x norm -> cast) for the 4-, 3- and
-// 2-bit codecs at head_dim 128: TurboQuant.decode, aither_kvcache/quantizer.py:168-197.
+// MFMA decode (unpack -> centroid lookup -> inverse rotation -> x norm -> cast) for the 4-, 3- and 2-bit codecs at
+// head_dim 64, 128 and 256: TurboQuant.decode, aither_kvcache/quantizer.py:168-197.
 //
-//   X[v, i] = n_v * sum_j c[code[v, j]] * Pi[j, i]              v_mfma_f32_16x16x32_f16
-//     A = centroids of the codes: lane (row = l%16, g = l/16) loads bytes [16g, 16g+16) of the
-//         vector's packed row (one 16-byte load) = coordinates j = 32g .. 32g+31; k-step ks takes
-//         dword ks of them.  A code BYTE (two codes) indexes a table in LDS whose entry is the
-//         float16 pair (c[a], c[b]); the table has a hi and a lo half (c = hi + lo to ~22 bits)
-//         and every entry is replicated 32 times (address = byte * 256 + (lane & 31) * 4, built
-//         by one byte permute) so lookups never conflict on a bank.
-//     B = Pi split into two float16 terms (hi + lo, scaled by 64).  Three MFMAs per tile:
-//         c_hi Pi_hi + c_lo Pi_hi + c_hi Pi_lo.  N-tile nt, column col is output element
-//         i = 8 col + nt, so that over the eight N-tiles a lane collects eight consecutive
-//         elements of a row: one 16-byte store, sixteen lanes write the 256-byte row.
-//     k-steps are the outer loop (A operands of one k-step live in registers, all 8 x 2
-//     accumulator tiles stay resident).
+//   X^T[i, v] = n_v * sum_j Pi[j, i] c[code[v, j]]              v_mfma_f32_16x16x32_f16
+//     A = Pi^T: a wavefront keeps the C x D slice of its C output coordinates in registers, two float16 terms (hi + lo,
+//         scaled by 64), split from the float32 matrix at its start.  D / C wavefronts share a row.
+//     B = centroids of the codes: lane (v = l % 16, g = l / 16) loads quarter g of the packed row of vector v.  A code
+//         BYTE (two codes) indexes a table in LDS whose 8-byte entry is the float16 pair (c[a], c[b]) and the pair of
+//         remainders (c = hi + lo to ~22 bits); every entry is replicated 32 times (address = byte * 256 + (lane & 31) * 8,
+//         built by one byte permute), so look-ups do not conflict on a bank.
+//     Three products per tile: Pi_hi c_hi + Pi_hi c_lo + Pi_lo c_hi.
+//   The rows of an A tile are permuted so that the four lanes of a vector write 64 neighbouring bytes per store; a lane
+//   needs one norm and one address per vector.
 //
-// 3-bit and 2-bit rows are spread to one code per nibble in registers (akv_nibble.h) and then take the
-// same table and products; the coordinate order that the spreading leaves is matched by the order in
-// which the rows of the B operand are copied into LDS.
+// 3-bit and 2-bit rows are spread to one code per nibble in registers (akv_nibble.h) and take the same table; the
+// coordinate order that the spreading leaves is matched when the matrix is loaded.
 //
-// A wavefront decodes 32 vectors per step; a workgroup is eight independent wavefronts plus the
-// B operand (64 KB) and the byte table (64 KB).
+// What bounds it: the stores (head_dim 128: 64 + 4 bytes in, 256 out per vector) and close behind them the products.  With
+// the matrix in LDS (64 KB read per 32 rows, three barriers of set-up, 32 address words per step in LDS) the same decode
+// at head_dim 128 took 40 us for 21k tokens x 8 heads of one tensor; head_dim 64 and 256 went through the vector kernel.
+// No barrier after the set-up: the wavefronts of a row only share cache lines.
 #include "akv_common.h"
 #include "akv_nibble.h"
 
 typedef _Float16 dm_half8 __attribute__((ext_vector_type(8)));
 typedef float dm_float4 __attribute__((ext_vector_type(4)));
+typedef uint32_t dm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t dm_u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) const dm_u32x2 dm_lds_cu64;
 typedef __attribute__((address_space(3))) dm_u32x4 dm_lds_u128;
-typedef __attribute__((address_space(3))) const uint32_t dm_lds_cu32;
 
 #define DM_WAVES 8
 #define DM_THREADS (DM_WAVES * 64)
-#define DM_ROWS 32
+#define DM_MT 2
+#define DM_ROWS (16 * DM_MT)
 #define DM_PSCALE 64.f
-#define DM_LUT_OFF 0                 // 256 entries x 256 B: [hi pair x 32 copies][lo pair x 32 copies]
-#define DM_B_OFF 65536               // [hi/lo][8 nt][4 ks][64 lanes] x 16 B
-#define DM_ROW_OFF 131072            // per wavefront: DM_ROWS x {packed offset, norm offset, output offset} (block-wise decode)
-#define DM_LDS_BYTES (131072 + DM_WAVES * DM_ROWS * 24)
-#define DM_SEL(k) (0x0c0c0400u + ((uint32_t)(k) << 8))
+#define DM_LDS_BYTES 65536           // 256 entries x 32 copies x {hi pair, lo pair}
 
-// the lane's quarter of a packed row: 16 / 12 / 8 bytes
-template <int BITS>
-__device__ __forceinline__ uint4 dm_load_quarter(const uint8_t* row, int g) {
-  if constexpr (BITS == 4) {
-    return *(const uint4*)(row + 16 * g);
-  } else if constexpr (BITS == 3) {
-    const uint32_t* p = (const uint32_t*)(row + 12 * g);
-    return make_uint4(p[0], p[1], p[2], 0u);
-  } else {
-    const uint2 t = *(const uint2*)(row + 8 * g);
-    return make_uint4(t.x, t.y, 0u, 0u);
-  }
-}
+template <int D, int BITS> struct dm_cfg {
+  static constexpr int C = D == 256 ? 32 : 64;              // output coordinates of a wavefront (its matrix slice: 64 to 128 registers)
+  static constexpr int CW = D / C;                          // wavefronts of a row
+  static constexpr int RG = DM_WAVES / CW;                  // row groups of a workgroup
+  static constexpr int NT = C / 16, KS = D / 32;
+  static constexpr int QB = D * BITS / 32;                  // bytes of a quarter row
+  static constexpr int RAW = BITS == 3 && D == 64 ? 2 : QB / 4;   // dwords a lane loads of it
+};
 
-// B operand of the decode kernel, stored after the encode operand in the prepared-rotation buffer
+// Operand of the inverse rotation in the attention kernels (head_dim 128), stored after the encode operand in the
+// prepared-rotation buffer
 __global__ __launch_bounds__(256) void akv_dm_prepare_kernel(const float* __restrict__ Pi, uint4* __restrict__ bop) {
   const int t = blockIdx.x * 256 + threadIdx.x;      // (nt, ks, lane): 2048 threads
   const int lane = t & 63, ks = (t >> 6) & 3, nt = t >> 8;
@@ -86,182 +78,243 @@ int akv_prepare_decode_mfma(const float* rotation, int d, void* prep, hipStream_
   return AKV_OK;
 }
 
-// BLOCKS = false: n contiguous rows (TurboQuant.decode).  BLOCKS = true: the rows are the
-// (position, head) entries of the cache blocks listed in a.slots; every listed block that exists is
-// decoded into the block of the same index of the output buffer (the batch decompress of
-// aither_kvcache/vllm/backend.py:1040-1091 without its gather / unique / scatter passes).
-template <bool BLOCKS, int BITS, int ODT>
-__global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_args a, const uint4* __restrict__ bop) {
-  extern __shared__ __align__(16) unsigned char lds[];
+// quarter g of a packed row.  (3-bit, head_dim 64: six bytes, read as the two dwords of the row that hold them)
+template <int D, int BITS>
+__device__ __forceinline__ void dm_load_quarter(const uint8_t* row, int g, uint32_t (&w)[dm_cfg<D, BITS>::RAW]) {
+  constexpr int RAW = dm_cfg<D, BITS>::RAW, QB = dm_cfg<D, BITS>::QB;
+  const uint32_t* p = (const uint32_t*)(row + (QB % 4 ? (QB * g & ~3) : QB * g));
+  if constexpr (RAW == 1) {
+    w[0] = p[0];
+  } else if constexpr (RAW == 2) {
+    const uint2 t = *(const uint2*)p;
+    w[0] = t.x; w[1] = t.y;
+  } else if constexpr (RAW % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < RAW; i += 4) {
+      const uint4 t = *(const uint4*)(p + i);
+      w[i] = t.x; w[i + 1] = t.y; w[i + 2] = t.z; w[i + 3] = t.w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < RAW; ++i) w[i] = p[i];
+  }
+}
+// one code per nibble: dword st, byte b, nibble lo holds coordinate mf_kcoord<BITS>(st, b, lo) of the quarter
+template <int D, int BITS>
+__device__ __forceinline__ void dm_spread(const uint32_t (&w)[dm_cfg<D, BITS>::RAW], int g, uint32_t (&kw)[dm_cfg<D, BITS>::KS]) {
+  constexpr int KS = dm_cfg<D, BITS>::KS;
+  if constexpr (BITS == 4) {
+#pragma unroll
+    for (int i = 0; i < KS; ++i) kw[i] = w[i];
+  } else if constexpr (BITS == 2) {
+#pragma unroll
+    for (int i = 0; i < KS / 2; ++i) { kw[2 * i] = w[i] & 0x33333333u; kw[2 * i + 1] = (w[i] >> 2) & 0x33333333u; }
+  } else if constexpr (D == 64) {
+    // bytes 2 (g % 2) .. + 5 of the eight
+    const uint32_t lo = (g & 1) ? (w[0] >> 16) | (w[1] << 16) : w[0], hi = (g & 1) ? w[1] >> 16 : w[1];
+    kw[0] = mf_spread3(__builtin_amdgcn_perm(lo, lo, 0x0c000102u));
+    kw[1] = mf_spread3(__builtin_amdgcn_perm(hi, lo, 0x0c030405u));
+  } else {
+#pragma unroll
+    for (int i = 0; i < KS / 4; ++i) {
+      const uint32_t part[4] = {w[3 * i], w[3 * i + 1], w[3 * i + 2], 0u};
+      uint32_t out[4];
+      mf_spread_row<3>(part, out);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) kw[4 * i + q] = out[q];
+    }
+  }
+}
+
+// n / d and the remainder for n < 2^31; r = floor((2^32 - 1) / d): the estimate is at most one too small
+__device__ __forceinline__ uint32_t dm_div(uint32_t n, uint32_t d, uint32_t r, uint32_t& rem) {
+  uint32_t q = __umulhi(n, r);
+  rem = n - q * d;
+  if (rem >= d) { ++q; rem -= d; }
+  return q;
+}
+
+// BLOCKS = false: n contiguous rows (TurboQuant.decode).  BLOCKS = true: the rows are the (position, head) entries of the
+// cache blocks listed in a.slots; every listed block that exists is decoded into the block of the same index of the
+// output buffer (the batch decompress of aither_kvcache/vllm/backend.py:1040-1091 without its gather / unique / scatter
+// passes).  An entry equal to the one before it is not decoded again: the padding of a block table is such a run.
+// With a.packed2 the rows of a second tensor (V) follow those of the first.
+template <int D, int BITS, int ODT, bool BLOCKS>
+__global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_args a, const float* __restrict__ PiT) {
+  typedef dm_cfg<D, BITS> cfg;
+  constexpr int C = cfg::C, CW = cfg::CW, RG = cfg::RG, NT = cfg::NT, KS = cfg::KS, RAW = cfg::RAW;
+  typedef typename akv_elem<ODT>::type out_t;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
-  {
-    if constexpr (BITS == 4) {
-      uint4* b_lds = (uint4*)(lds + DM_B_OFF);
-      for (int i = threadIdx.x; i < 65536 / 16; i += DM_THREADS) b_lds[i] = bop[i];
-    } else {
-      // element e of k-step ks of a lane faces the coordinate that the spread code stream holds there
-      const uint16_t* src = (const uint16_t*)bop;
-      uint16_t* b_lds = (uint16_t*)(lds + DM_B_OFF);
-      for (int i = threadIdx.x; i < 65536 / 2; i += DM_THREADS) {
-        const int e = i & 7, ln = (i >> 3) & 63, ks = (i >> 9) & 3, rest = i >> 11;   // rest = (hi | lo, nt)
-        const int c = mf_kcoord<BITS>(ks, e >> 1, e & 1);
-        b_lds[i] = src[((rest * 4 + (c >> 3)) * 64 + ln) * 8 + (c & 7)];
-      }
-    }
-    // byte table: entry (hi nibble, lo nibble) -> (c[hi nibble], c[lo nibble]): the code of the
-    // even coordinate is the high nibble (packing.py:13-23) and goes to the low half of the pair
-    uint32_t* lut = (uint32_t*)(lds + DM_LUT_OFF);
-    for (int i = threadIdx.x; i < 256 * 64; i += DM_THREADS) {
-      const int e = i >> 6, half = (i >> 5) & 1;
-      constexpr int LM = (1 << BITS) - 1;      // nibble values above the top level do not occur
-      const float c0 = a.table[(e >> 4) & LM], c1 = a.table[e & 15 & LM];
-      const __half h0 = __float2half_rn(c0), h1 = __float2half_rn(c1);
-      uint32_t w;
-      if (half == 0) {
-        w = (uint32_t)__half_as_ushort(h0) | ((uint32_t)__half_as_ushort(h1) << 16);
-      } else {
-        const __half l0 = __float2half_rn(c0 - __half2float(h0)), l1 = __float2half_rn(c1 - __half2float(h1));
-        w = (uint32_t)__half_as_ushort(l0) | ((uint32_t)__half_as_ushort(l1) << 16);
-      }
-      lut[i] = w;
-    }
-    __syncthreads();
-  }
-  const uint32_t lane4 = (uint32_t)(lane & 31) * 4u;
-  const uint32_t b_addr = DM_B_OFF + (uint32_t)lane * 16u;
+  const int cw = wave % CW, rg = wave / CW;
+  const uint32_t n_one = (uint32_t)a.n, n_total = BLOCKS && a.packed2 ? 2u * n_one : n_one;
+  const uint32_t steps = (n_total + DM_ROWS - 1) / DM_ROWS, stride = gridDim.x * RG;
+  const uint32_t per_blk = BLOCKS ? (uint32_t)a.block_size * (uint32_t)a.heads : 1u, heads = BLOCKS ? (uint32_t)a.heads : 1u;
+  const uint32_t per_r = 0xffffffffu / per_blk, heads_r = 0xffffffffu / heads;
 
-  const int64_t steps = (a.n + DM_ROWS - 1) / DM_ROWS;
-  const int64_t stride = (int64_t)gridDim.x * DM_WAVES;
-  for (int64_t step = (int64_t)wave * gridDim.x + blockIdx.x; step < steps; step += stride) {
-    const int64_t base = step * DM_ROWS;
-    // ---- packed rows and norms
-    uint4 pk[2];
-    float4 nr[2];
-    int64_t* row_p = (int64_t*)(lds + DM_ROW_OFF + wave * DM_ROWS * 24);   // packed byte offset, or -1
-    int64_t* row_n = row_p + DM_ROWS;                                      // norm element offset
-    int64_t* row_o = row_n + DM_ROWS;                                      // output element offset
+  // ---- rows: block ids two steps ahead, codes and norms one step ahead
+  int64_t id[DM_MT], before[DM_MT];
+  uint32_t raw[DM_MT][RAW];
+  float nrm[DM_MT];
+  out_t* dst[DM_MT];                          // null: nothing to write
+  auto fetch_ids = [&](uint32_t step) {
     if constexpr (BLOCKS) {
-      if (lane < DM_ROWS) {   // lane l resolves row base + l = (listed block, position, head)
-        const int64_t n = base + lane;
-        int64_t po = -1, no = 0, oo = 0;
-        if (n < a.n) {
-          const int64_t per_blk = (int64_t)a.block_size * a.heads;
-          const int64_t li = n / per_blk, rem = n - li * per_blk;
-          const int64_t pos = rem / a.heads, head = rem - pos * a.heads;
-          const int64_t blk = akv_load_index(a.slots, a.slot_itype, li);
-          if (blk >= 0 && blk < a.max_blocks) {
-            po = blk * a.ps0 + pos * a.ps1 + head * a.ps2;
-            no = blk * a.ns0 + pos * a.ns1 + head * a.ns2;
-            oo = blk * a.os0 + pos * a.os1 + head * a.os2;
-          }
-        }
-        row_p[lane] = po; row_n[lane] = no; row_o[lane] = oo;
+#pragma unroll
+      for (int mt = 0; mt < DM_MT; ++mt) {
+        uint32_t n = min(step * DM_ROWS + 16 * mt + col, n_total - 1), rem;
+        if (n >= n_one) n -= n_one;
+        const uint32_t li = dm_div(n, per_blk, per_r, rem);
+        id[mt] = akv_load_index(a.slots, a.slot_itype, li);
+        before[mt] = li > 0 ? akv_load_index(a.slots, a.slot_itype, li - 1) : -1;
       }
     }
+  };
+  auto fetch_rows = [&](uint32_t step) {
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      float nv[4];
+    for (int mt = 0; mt < DM_MT; ++mt) {
+      const uint32_t at = step * DM_ROWS + 16 * mt + col;
+      uint32_t n = min(at, n_total - 1);
+      const bool second = BLOCKS && n >= n_one;
+      if (second) n -= n_one;
+      int64_t po, no, oo;
+      bool live = at < n_total;
       if constexpr (BLOCKS) {
-        const int64_t po = row_p[16 * mt + (lane & 15)];
-        pk[mt] = po >= 0 ? dm_load_quarter<BITS>(a.packed + po, g) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 16 * mt + 4 * g + i;
-          nv[i] = row_p[r] >= 0 ? a.norms[row_n[r]] : 0.f;
-        }
+        uint32_t rem, head;
+        dm_div(n, per_blk, per_r, rem);
+        const uint32_t pos = dm_div(rem, heads, heads_r, head);
+        live = live && id[mt] >= 0 && id[mt] < a.max_blocks && id[mt] != before[mt];
+        const int64_t blk = live ? id[mt] : 0;          // (a row of block 0 is read and dropped)
+        po = blk * a.ps0 + pos * a.ps1 + head * a.ps2;
+        no = blk * a.ns0 + pos * a.ns1 + head * a.ns2;
+        oo = blk * a.os0 + pos * a.os1 + head * a.os2;
       } else {
-        const int64_t n = base + 16 * mt + (lane & 15);
-        pk[mt] = n < a.n ? dm_load_quarter<BITS>(a.packed + n * a.ps0, g) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int64_t r = base + 16 * mt + 4 * g + i;
-          nv[i] = r < a.n ? a.norms[r] : 0.f;
-        }
+        po = n * a.ps0; no = n; oo = n * a.os0;
       }
-      nr[mt] = make_float4(nv[0], nv[1], nv[2], nv[3]);
+      dm_load_quarter<D, BITS>((second ? a.packed2 : a.packed) + po, g, raw[mt]);
+      nrm[mt] = (second ? a.norms2 : a.norms)[no];
+      dst[mt] = live ? (out_t*)(second ? a.out2 : a.out) + oo : nullptr;
     }
-    uint32_t kw[2][4];      // one code per nibble
+  };
+  uint32_t step = (uint32_t)rg * gridDim.x + blockIdx.x;
+  fetch_ids(step);
+
+  // ---- table; the scale brings the largest level to [2^9, 2^10): no remainder that matters is a float16 subnormal
+  float inv_cs;
+  {
+    constexpr int LM = (1 << BITS) - 1;                // nibble values above the top level do not occur
+    const int e = threadIdx.x >> 1, half = threadIdx.x & 1;
+    const float r0 = a.table[(e >> 4) & LM], r1 = a.table[e & LM];
+    float mx = 0.f;
+    for (int v = 0; v <= LM; ++v) mx = fmaxf(mx, fabsf(a.table[v]));
+    const uint32_t ex = min(max((__float_as_uint(mx) >> 23) & 0xffu, 12u), 250u);
+    const float cs = __uint_as_float((254u - ex) << 23) * 512.f;
+    inv_cs = __uint_as_float(ex << 23) * (1.f / 512.f / DM_PSCALE);
+    // the code of the even coordinate is the high nibble (packing.py:13-23) and goes to the low half of the pair
+    const float c0 = r0 * cs, c1 = r1 * cs;
+    const __half h0 = __float2half_rn(c0), h1 = __float2half_rn(c1);
+    const __half l0 = __float2half_rn(c0 - __half2float(h0)), l1 = __float2half_rn(c1 - __half2float(h1));
+    const uint32_t hi = (uint32_t)__half_as_ushort(h0) | ((uint32_t)__half_as_ushort(h1) << 16);
+    const uint32_t lo = (uint32_t)__half_as_ushort(l0) | ((uint32_t)__half_as_ushort(l1) << 16);
+    // (the dynamic LDS block is the kernel's only LDS object: its offsets are LDS addresses)
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const uint32_t raw[4] = {pk[mt].x, pk[mt].y, pk[mt].z, pk[mt].w};
-      mf_spread_row<BITS>(raw, kw[mt]);
-    }
-    dm_float4 acc[2][8];
+    for (int i = 0; i < 8; ++i) *(dm_lds_u128*)(uintptr_t)(uint32_t)(e * 256 + half * 128 + i * 16) = (dm_u32x4){hi, lo, hi, lo};
+  }
+
+  // ---- matrix slice: row m of tile nt is output coordinate `mine` below (see the stores); lane (m, g) holds the contracted
+  // coordinates that quarter g of a row brings at k-step ks
+  dm_half8 Ah[NT][KS], Al[NT][KS];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+  for (int nt = 0; nt < NT; ++nt) {
+    const int m4 = col >> 2, mi = col & 3;
+    const int mine = C * cw + (ODT == AKV_F32 ? 16 * nt + 4 * m4 + mi : 32 * (nt >> 1) + 8 * m4 + 4 * (nt & 1) + mi);
+    const float4* p = (const float4*)(PiT + (size_t)mine * D + (D / 4) * g);
 #pragma unroll
-      for (int nt = 0; nt < 8; ++nt) acc[mt][nt] = (dm_float4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      // A operands of this k-step: four byte lookups (hi and lo) per M-tile
-      dm_half8 ah[2], al[2];
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        const uint32_t w = kw[mt][ks];
-        union { uint32_t u[4]; dm_half8 h; } ch, cl;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const uint32_t addr = __builtin_amdgcn_perm(w, lane4, DM_SEL(b));
-          ch.u[b] = *(dm_lds_cu32*)(uintptr_t)addr;
-          cl.u[b] = *(dm_lds_cu32*)(uintptr_t)(addr + 128u);
-        }
-        ah[mt] = ch.h;
-        al[mt] = cl.h;
-      }
-#pragma unroll
-      for (int nt = 0; nt < 8; ++nt) {
-        union { dm_u32x4 u; dm_half8 h; } bh, bl;
-        bh.u = *(dm_lds_u128*)(uintptr_t)(b_addr + (uint32_t)((nt * 4 + ks) * 1024));
-        bl.u = *(dm_lds_u128*)(uintptr_t)(b_addr + 32768u + (uint32_t)((nt * 4 + ks) * 1024));
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mt], bh.h, acc[mt][nt], 0, 0, 0);
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mt], bh.h, acc[mt][nt], 0, 0, 0);
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mt], bl.h, acc[mt][nt], 0, 0, 0);
-        }
-        // (the loops are unrolled because the accumulators are register arrays; without a fence
-        // the scheduler hoists every B read of the step and spills)
-        if (nt & 1) __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    // ---- x norm, to float16, one 16-byte store per row: lane (col, g) holds elements 8 col + nt
-    //      of rows 4g + i
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const float nv[4] = {nr[mt].x, nr[mt].y, nr[mt].z, nr[mt].w};
+    for (int k2 = 0; k2 < KS / 2; ++k2) {               // two k-steps: 16 neighbouring coordinates
+      float v[16];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        typedef typename akv_elem<ODT>::type out_t;
-        out_t* orow;
-        if constexpr (BLOCKS) {
-          const int r = 16 * mt + 4 * g + i;
-          if (row_p[r] < 0) continue;
-          orow = (out_t*)a.out + row_o[r];
-        } else {
-          const int64_t r = base + 16 * mt + 4 * g + i;
-          if (r >= a.n) continue;
-          orow = (out_t*)a.out + r * a.os0;
-        }
-        // the reference multiplies the float32 rotated vector by the norm and then casts
-        float v[8];
+        const float4 t = p[4 * k2 + i];
+        v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+      }
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) v[nt] = __fmul_rn(acc[mt][nt][i] * (1.f / DM_PSCALE), nv[i]);
-        if constexpr (ODT == AKV_F32) {
-          *(float4*)(orow + 8 * col) = make_float4(v[0], v[1], v[2], v[3]);
-          *(float4*)(orow + 8 * col + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        } else {
+      for (int k1 = 0; k1 < 2; ++k1)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float s = v[mf_kcoord<BITS>(k1, e >> 1, e & 1)] * DM_PSCALE;
+          const _Float16 h = (_Float16)s;
+          Ah[nt][2 * k2 + k1][e] = h;
+          Al[nt][2 * k2 + k1][e] = (_Float16)(s - (float)h);
+        }
+    }
+  }
+  __syncthreads();
+  const uint32_t copy = (uint32_t)(lane & 31) * 8u;
+
+  if (step >= steps) return;
+  fetch_rows(step);
+  fetch_ids(min(step + stride, steps - 1));
+  for (; step < steps; step += stride) {
+    uint32_t kw[DM_MT][KS];
+    float nv[DM_MT];
+    out_t* orow[DM_MT];
+#pragma unroll
+    for (int mt = 0; mt < DM_MT; ++mt) {
+      dm_spread<D, BITS>(raw[mt], g, kw[mt]);
+      nv[mt] = nrm[mt];
+      orow[mt] = dst[mt];
+    }
+    fetch_rows(min(step + stride, steps - 1));          // (past the end: the last step once more)
+    fetch_ids(min(step + 2 * stride, steps - 1));
+    if (__builtin_amdgcn_ballot_w64(orow[0] != nullptr || orow[DM_MT - 1] != nullptr) == 0) continue;
+    dm_float4 acc[DM_MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < DM_MT; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = (dm_float4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+      for (int mt = 0; mt < DM_MT; ++mt) {
+        union { uint32_t u[4]; dm_half8 h; } ch, cl;
+        const uint32_t w = kw[mt][ks];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const dm_u32x2 t = *(dm_lds_cu64*)(uintptr_t)__builtin_amdgcn_perm(w, copy, 0x0c020400u + ((uint32_t)b << 8));
+          ch.u[b] = t.x;
+          cl.u[b] = t.y;
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[nt][ks], ch.h, acc[mt][nt], 0, 0, 0);
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[nt][ks], cl.h, acc[mt][nt], 0, 0, 0);
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[nt][ks], ch.h, acc[mt][nt], 0, 0, 0);
+        }
+      }
+    }
+    // ---- x norm, cast (the reference multiplies the float32 rotated vector by the norm and then casts): lane (v, g)
+    // holds rows 4 g + i of every tile
+#pragma unroll
+    for (int mt = 0; mt < DM_MT; ++mt) {
+      if (orow[mt] == nullptr) continue;
+      if constexpr (ODT == AKV_F32) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          const dm_float4 y = acc[mt][nt] * inv_cs;
+          *(float4*)(orow[mt] + C * cw + 16 * nt + 4 * g) = make_float4(y.x * nv[mt], y.y * nv[mt], y.z * nv[mt], y.w * nv[mt]);
+        }
+      } else {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt += 2) {
           uint32_t w[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            if constexpr (ODT == AKV_F16) {
-              w[q] = (uint32_t)__half_as_ushort(__float2half_rn(v[2 * q])) | ((uint32_t)__half_as_ushort(__float2half_rn(v[2 * q + 1])) << 16);
-            } else {
-              w[q] = (uint32_t)akv_float_to_bf16_bits(v[2 * q]) | ((uint32_t)akv_float_to_bf16_bits(v[2 * q + 1]) << 16);
-            }
+            const float v0 = __fmul_rn(acc[mt][nt + (q >> 1)][2 * (q & 1)] * inv_cs, nv[mt]);
+            const float v1 = __fmul_rn(acc[mt][nt + (q >> 1)][2 * (q & 1) + 1] * inv_cs, nv[mt]);
+            if constexpr (ODT == AKV_F16) w[q] = (uint32_t)__half_as_ushort(__float2half_rn(v0)) | ((uint32_t)__half_as_ushort(__float2half_rn(v1)) << 16);
+            else w[q] = (uint32_t)akv_float_to_bf16_bits(v0) | ((uint32_t)akv_float_to_bf16_bits(v1) << 16);
           }
-          *(uint4*)(orow + 8 * col) = make_uint4(w[0], w[1], w[2], w[3]);
+          *(uint4*)(orow[mt] + C * cw + 16 * nt + 8 * g) = make_uint4(w[0], w[1], w[2], w[3]);
         }
       }
     }
@@ -269,45 +322,42 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
 }
 
 static bool dm_disabled() {
-  static int v = -1;
-  if (v < 0) {
-    const char* e = getenv("AKV_DISABLE_MFMA");
-    v = (e && e[0] == '1') ? 1 : 0;
-  }
-  return v == 1;
+  static const bool off = [] { const char* e = getenv("AKV_DISABLE_MFMA"); return e && e[0] == '1'; }();
+  return off;
+}
+
+template <int D, int BITS, int ODT, bool BLOCKS>
+static int dm_launch(const akv_gen_args& a, const float* PiT, hipStream_t stream) {
+  const int64_t n_total = BLOCKS && a.packed2 ? 2 * a.n : a.n, steps = (n_total + DM_ROWS - 1) / DM_ROWS;
+  const int cus = akv_cached_cu_count() > 0 ? akv_cached_cu_count() : 256;
+  AKV_LAUNCH_TIMED((akv_decode_mfma_kernel<D, BITS, ODT, BLOCKS>), (int)(steps < cus ? steps : cus), DM_THREADS, DM_LDS_BYTES, stream, a, PiT);
+  AKV_LAUNCH_CHECK("akv_decode_mfma_kernel");
+  return AKV_OK;
+}
+template <int D, int BITS>
+static int dm_launch_dt(bool blocks, int out_dtype, const akv_gen_args& a, const float* PiT, hipStream_t stream) {
+  if (out_dtype == AKV_F16) return blocks ? dm_launch<D, BITS, AKV_F16, true>(a, PiT, stream) : dm_launch<D, BITS, AKV_F16, false>(a, PiT, stream);
+  if (out_dtype == AKV_BF16) return blocks ? dm_launch<D, BITS, AKV_BF16, true>(a, PiT, stream) : dm_launch<D, BITS, AKV_BF16, false>(a, PiT, stream);
+  return blocks ? dm_launch<D, BITS, AKV_F32, true>(a, PiT, stream) : dm_launch<D, BITS, AKV_F32, false>(a, PiT, stream);
 }
 
 // returns AKV_ERR_UNSUPPORTED when the fast path does not apply (the caller then uses the general kernel)
 int akv_decode_mfma_try(const akv_gen_args& a, bool blocks, int d, int bits, int out_dtype, const void* rot_prep,
                         hipStream_t stream) {
-  if (dm_disabled() || d != 128 || bits < 2 || bits > 4) return AKV_ERR_UNSUPPORTED;
-  const uintptr_t palign = 3;      // a lane reads 16 / 12 / 8 bytes of a row: multi-dword loads need dword alignment only
-  if ((((uintptr_t)a.packed | (uintptr_t)a.ps0) & palign) || ((uintptr_t)a.out & 15)) return AKV_ERR_UNSUPPORTED;
-  if (a.os0 & 7) return AKV_ERR_UNSUPPORTED;      // rows of the output are written 8 elements (16 or 32 bytes) per lane
+  if (dm_disabled() || !(d == 64 || d == 128 || d == 256)) return AKV_ERR_UNSUPPORTED;
+  const uintptr_t palign = 3;      // multi-dword loads need dword alignment only
+  if (((uintptr_t)a.packed | (uintptr_t)a.packed2 | (uintptr_t)a.ps0) & palign) return AKV_ERR_UNSUPPORTED;
+  if (((uintptr_t)a.out | (uintptr_t)a.out2) & 15) return AKV_ERR_UNSUPPORTED;
+  if (a.os0 & 7) return AKV_ERR_UNSUPPORTED;      // the output is written 16 bytes (8 or 4 elements) per lane
   if (blocks && (((uintptr_t)a.ps1 | (uintptr_t)a.ps2) & palign || ((a.os1 | a.os2) & 7))) return AKV_ERR_UNSUPPORTED;
-  const uint4* bop = (const uint4*)((const char*)rot_prep + AKV_PREP_DECODE_OFFSET(d));
-  const int64_t steps = (a.n + DM_ROWS - 1) / DM_ROWS;
-  const int grid = (int)(steps < akv_cached_cu_count() ? steps : akv_cached_cu_count());
-#define DM_GO(BL, BB, OD)                                                                                      \
-  do {                                                                                                       \
-    static bool configured = false;                                                                          \
-    if (!configured) {                                                                                       \
-      AKV_HIP(hipFuncSetAttribute((const void*)akv_decode_mfma_kernel<BL, BB, OD>,                           \
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, DM_LDS_BYTES));                \
-      configured = true;                                                                                     \
-    }                                                                                                        \
-    AKV_LAUNCH_TIMED((akv_decode_mfma_kernel<BL, BB, OD>), grid, DM_THREADS, DM_LDS_BYTES, stream, a, bop);  \
-  } while (0)
-#define DM_GO_DT(BL, BB)                                                                                       \
-  do {                                                                                                       \
-    if (out_dtype == AKV_F16) DM_GO(BL, BB, AKV_F16);                                                        \
-    else if (out_dtype == AKV_BF16) DM_GO(BL, BB, AKV_BF16);                                                 \
-    else DM_GO(BL, BB, AKV_F32);                                                                             \
-  } while (0)
-  if (blocks) { if (bits == 4) DM_GO_DT(true, 4); else if (bits == 3) DM_GO_DT(true, 3); else DM_GO_DT(true, 2); }
-  else { if (bits == 4) DM_GO_DT(false, 4); else if (bits == 3) DM_GO_DT(false, 3); else DM_GO_DT(false, 2); }
-#undef DM_GO_DT
-#undef DM_GO
-  AKV_LAUNCH_CHECK("akv_decode_mfma_kernel");
-  return AKV_OK;
+  // rows are counted in 32 bits, with room for two strides past the end
+  if ((a.packed2 ? 2 : 1) * a.n >= ((int64_t)1 << 31) - ((int64_t)1 << 22)) return AKV_ERR_UNSUPPORTED;
+  if (blocks && (int64_t)a.block_size * a.heads >= ((int64_t)1 << 31)) return AKV_ERR_UNSUPPORTED;
+  const float* PiT = (const float*)rot_prep + (size_t)d * d;
+#define DM_CASE(DD, BB) if (d == DD && bits == BB) return dm_launch_dt<DD, BB>(blocks, out_dtype, a, PiT, stream)
+  DM_CASE(64, 2); DM_CASE(64, 3); DM_CASE(64, 4);
+  DM_CASE(128, 2); DM_CASE(128, 3); DM_CASE(128, 4);
+  DM_CASE(256, 2); DM_CASE(256, 3); DM_CASE(256, 4);
+#undef DM_CASE
+  return AKV_ERR_UNSUPPORTED;
 }

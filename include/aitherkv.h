@@ -161,6 +161,16 @@ int akv_decode_blocks(const uint8_t* packed, int64_t ps_blk, int64_t ps_pos, int
                       void* out, int out_dtype, int64_t os_blk, int64_t os_pos, int64_t os_head,
                       void* stream);
 
+/* akv_decode_blocks of K and V in one launch: two caches of the same shape and strides, two output buffers of the same
+ * shape and strides, which must not overlap. */
+int akv_decode_blocks_kv(const uint8_t* k_packed, const uint8_t* v_packed, int64_t ps_blk, int64_t ps_pos, int64_t ps_head,
+                         const float* k_norms, const float* v_norms, int64_t ns_blk, int64_t ns_pos, int64_t ns_head,
+                         const void* block_ids, int ids_itype, int64_t num_ids, int64_t num_blocks,
+                         int block_size, int num_kv_heads, int d,
+                         const void* rot_prep, const float* centroids, int bits,
+                         void* k_out, void* v_out, int out_dtype, int64_t os_blk, int64_t os_pos, int64_t os_head,
+                         void* stream);
+
 /* ---------------------------------------------------------------------------------
  * TQPagedAttention.forward -- aither_kvcache/fused_attention.py:594-748, with the result
  * of TQPagedAttentionRef.forward (:91-185).  The query pre-rotation (:659) and the output

@@ -1,0 +1,75 @@
+"""The matrix-core decode kernel at the edges of a step and of the grid, against the oracle's codes in float64."""
+import numpy as np
+import pytest
+import torch
+
+import aitherkvcache_amd as akv
+from aitherkvcache_amd.vllm.decompress import batch_decompress_active_blocks, decode_blocks
+from oracle import tq_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# Against 64 bits: the two-term operands and float32 sums stay below 2^-20 of a row's length (three products of 2^-22 and
+# the float32 rounding of at most 256 terms), the cast adds half a unit of the output type (2^-11, 2^-8) of the element.
+UNIT = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def check(got, packed, norms, tq, dtype):
+    d = tq.head_dim
+    c = tq.centroids.cpu().numpy().astype(np.float64)
+    y = c[O._UNPACK[tq.bits](packed.reshape(-1, packed.shape[-1])[:, :tq._packed_dim], d).astype(np.int64)]
+    ref = (y @ tq.rotation.cpu().numpy().astype(np.float64)) * norms.reshape(-1, 1).astype(np.float64)
+    err = np.abs(got.reshape(-1, d).astype(np.float64) - ref)
+    bound = np.abs(ref) * UNIT[dtype] * 1.01 + np.linalg.norm(ref, axis=-1, keepdims=True) * 2.0 ** -20 + (2.0 ** -25 if dtype == torch.float16 else 0)
+    assert np.all(err <= bound), float(np.max(err - bound))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("d,bits", [(d, b) for d in (64, 128, 256) for b in (4, 3, 2)])
+def test_flat_rows(dev, d, bits, dtype):
+    tq = akv.TurboQuant(head_dim=d, bits=bits, device=str(dev), dtype=dtype)
+    rng = np.random.default_rng(d + bits)
+    for n in (1, 15, 16, 33, 700) + ((70001,) if bits == 4 else ()):       # (the last: more steps than row groups)
+        packed = rng.integers(0, 256, (n, tq._packed_dim), dtype=np.uint8)
+        norms = rng.lognormal(0, 1, n).astype(np.float32)
+        print(f"[decode] d={d} bits={bits} {dtype} n={n}", flush=True)
+        out = tq.decode(torch.from_numpy(packed).to(dev), torch.from_numpy(norms).to(dev))
+        assert out.dtype == dtype
+        k = slice(None) if n < 1000 else slice(n - 500, n)
+        check(out[k].float().cpu().numpy(), packed[k], norms[k], tq, dtype)
+
+
+@pytest.mark.parametrize("d,bits,heads,bs,dtype", [(64, 4, 3, 16, torch.bfloat16), (64, 3, 1, 32, torch.float16), (128, 4, 8, 16, torch.float32),
+                                                   (128, 2, 5, 7, torch.float16), (256, 3, 2, 16, torch.bfloat16), (256, 4, 1, 1, torch.float16)])
+def test_listed_blocks(dev, d, bits, heads, bs, dtype):
+    """Padding, repeated and out-of-range ids; rows behind reserved bytes; K and V in one launch, from one tensor and from
+    tensors whose layouts differ; outputs that share storage; blocks that are not listed keep what they held."""
+    tq = akv.TurboQuant(head_dim=d, bits=bits, device=str(dev), dtype=dtype)
+    rng = np.random.default_rng(heads)
+    P, blocks = tq._packed_dim, 37
+    both = torch.from_numpy(rng.integers(0, 256, (blocks, 2, bs, heads, P + 4), dtype=np.uint8)).to(dev)
+    norms = [torch.from_numpy(rng.lognormal(0, 1, (blocks, bs, heads)).astype(np.float32)).to(dev) for _ in range(2)]
+    table = np.array([[5, 9, 9, 9, 0, 0, 0, -1, -1], [30, 2, 36, 37, 99, 2, 5, 0, 0], [-5, -1, 17, 17, 3, 4, 17, 17, 35]], dtype=np.int64)
+    listed = sorted({int(b) for b in table.ravel() if 0 <= b < 36})        # (36 lies outside the declared blocks)
+    rest = [b for b in range(blocks) if b not in listed]
+
+    def caches(form):
+        k, v = both[:, 0], both[:, 1]
+        return (k, v) if form != "differ" else (k, v.contiguous())
+
+    for form in ("same", "differ", "shared"):
+        for ids in (torch.from_numpy(table).to(dev), torch.from_numpy(table.astype(np.int32)).to(dev)):
+            k, v = caches(form)
+            if form == "shared":
+                pair = torch.full((blocks, bs, heads, 2, d), 7.0, dtype=dtype, device=dev)
+                outs = [pair[..., 0, :], pair[..., 1, :]]
+            else:
+                outs = [torch.full((blocks, bs, heads, d), 7.0, dtype=dtype, device=dev) for _ in range(2)]
+            print(f"[decode blocks] d={d} bits={bits} {form} {ids.dtype}", flush=True)
+            batch_decompress_active_blocks(k, v, outs[0], outs[1], tq, P, ids, 36, norms[0], norms[1])
+            for o, rows, n in zip(outs, (k, v), norms):
+                check(o[listed].float().cpu().numpy(), rows[listed].cpu().numpy(), n[listed].cpu().numpy(), tq, dtype)
+                assert bool((o[rest] == 7.0).all())
+                one = torch.full((blocks, bs, heads, d), 7.0, dtype=dtype, device=dev)
+                decode_blocks(rows, n, one, tq, ids, 36)
+                assert torch.equal(one, o)
