@@ -205,9 +205,14 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
   const int col = lane & 15, g = lane >> 4;
   const uint32_t copy = (uint32_t)(lane & 31) * 8u;
 
+  // (requested before the table is built, not behind its barrier)
+  const int held = akv_prefix_hold(a.prefix, a.S);
+  const int32_t* rec = x.wgdesc + (size_t)blockIdx.x * AKV_WGREC;
+  const int g0 = rec[AKV_WGREC_G0], g1 = rec[AKV_WGREC_G1], s_first = rec[AKV_WGREC_SEQ];
+
   // ---- table; the scale brings the largest level to [2^9, 2^10)
-  float inv_cs;
-  {
+  float inv_cs = 0.f;
+  if (g0 < g1) {
     float mx = 0.f;
     for (int v = 0; v < (1 << BITS); ++v) mx = fmaxf(mx, fabsf(a.centroids[v]));
     const uint32_t ex = min(max((__float_as_uint(mx) >> 23) & 0xffu, 12u), 250u);
@@ -230,10 +235,6 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
   const int gqa = a.QH / a.KVH;
   const int hp = x.hp, R = W / hp;
   const int hs = wave % hp, r = wave / hp;
-  const int held = akv_prefix_hold(a.prefix, a.S);
-  const int32_t* rec = x.wgdesc + (size_t)blockIdx.x * AKV_WGREC;
-  const int g0 = rec[AKV_WGREC_G0], g1 = rec[AKV_WGREC_G1], s_first = rec[AKV_WGREC_SEQ];
-
   const uint32_t nbase = AW_NORM + (uint32_t)wave * AW_NORM_WAVE;
   const uint32_t nread = nbase + (uint32_t)g * 16u;
 
@@ -558,11 +559,16 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
 bool akv_attn_mfma_takes(const akv_attn_args& a, int bits);       // the conditions both matrix-core kernels share
 int akv_attn_mfma_head_groups(int gqa);
 
-// At head_dim 128 the kernel of akv_attn_mfma.hip has eight head slots: it is left with whole slots idle below five
-// (groups of) kv heads, and takes over from there.
+// At head_dim 128 the kernel of akv_attn_mfma.hip has eight head slots, most of them idle where a rank keeps one or two (groups
+// of) kv heads; it starts some 5 us sooner.  Measured, main kernels, this against that one: one head, 418k tokens 31 against
+// 43 us, 2.7k tokens 11 against 6; two heads, 583k tokens 12 % faster as a step, 366k tokens 44 against 46 us and a prologue
+// 4 us longer; four heads, 36k tokens 21 against 17.  The host knows the width of the tables, not the contexts.
+#define AW_FEW_TOKENS 262144
 bool akv_attn_wave_applicable(const akv_attn_args& a, int d, int bits) {
   if (!(d == 64 || d == 128 || d == 256) || (bits != 4 && bits != 2) || !akv_attn_mfma_takes(a, bits)) return false;
-  return d != 128 || a.KVH * akv_attn_mfma_head_groups(a.QH / a.KVH) <= 4;
+  if (d != 128) return true;
+  const int heads = a.KVH * akv_attn_mfma_head_groups(a.QH / a.KVH);
+  return heads <= 2 && (int64_t)a.S * a.max_blocks_per_seq * a.block_size >= (int64_t)heads * AW_FEW_TOKENS;
 }
 
 template <int D, int BITS>
