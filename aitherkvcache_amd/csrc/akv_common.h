@@ -110,6 +110,14 @@ struct akv_gen_args {
   void* out2;             // block-wise decode of a second tensor (packed2, norms2) in the same launch
 };
 
+// n / d and the remainder for n < 2^31, d > 0; r = floor((2^32 - 1) / d): the estimate is at most one too small
+__device__ __forceinline__ uint32_t akv_div32(uint32_t n, uint32_t d, uint32_t r, uint32_t& rem) {
+  uint32_t q = __umulhi(n, r);
+  rem = n - q * d;
+  if (rem >= d) { ++q; rem -= d; }
+  return q;
+}
+
 // ----------------------------------------------------------------------------------
 // device: element loads / stores
 // ----------------------------------------------------------------------------------

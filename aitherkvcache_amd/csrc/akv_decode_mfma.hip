@@ -15,15 +15,20 @@
 // 3-bit and 2-bit rows are spread to one code per nibble in registers (akv_nibble.h) and take the same table; the
 // coordinate order that the spreading leaves is matched when the matrix is loaded.
 //
-// What bounds it: the stores (head_dim 128: 64 + 4 bytes in, 256 out per vector) and close behind them the products.  With
-// the matrix in LDS (64 KB read per 32 rows, three barriers of set-up, 32 address words per step in LDS) the same decode
-// at head_dim 128 took 40 us for 21k tokens x 8 heads of one tensor; head_dim 64 and 256 went through the vector kernel.
+// What bounds it: the loop, 24 products of 16 cycles and some 430 vector instructions per 16 rows of head_dim 128 and
+// wavefront at two wavefronts a SIMD, and the trips to memory around it; it moves 2.0 TB/s.  17k tokens x 8 heads at
+// head_dim 128, K and V: 45 us (two launches with the matrix in LDS, 64 KB read per 32 rows and three barriers of set-up:
+// 72 us; with block ids widened to 64 bits where they are loaded, a wait per load: 53 us).  6,290 tokens x 8 heads at
+// head_dim 256 784 us on the vector kernel, 56 here; 20,936 tokens x 16 heads at head_dim 64, 3 bits, 385 and 36 us.
 // No barrier after the set-up: the wavefronts of a row only share cache lines.
 #include "akv_common.h"
 #include "akv_nibble.h"
 
 typedef _Float16 dm_half8 __attribute__((ext_vector_type(8)));
 typedef float dm_float4 __attribute__((ext_vector_type(4)));
+typedef float dm_float2 __attribute__((ext_vector_type(2)));
+typedef _Float16 dm_half2 __attribute__((ext_vector_type(2)));
+typedef __bf16 dm_bf162 __attribute__((ext_vector_type(2)));
 typedef uint32_t dm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t dm_u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const dm_u32x2 dm_lds_cu64;
@@ -126,14 +131,6 @@ __device__ __forceinline__ void dm_spread(const uint32_t (&w)[dm_cfg<D, BITS>::R
   }
 }
 
-// n / d and the remainder for n < 2^31; r = floor((2^32 - 1) / d): the estimate is at most one too small
-__device__ __forceinline__ uint32_t dm_div(uint32_t n, uint32_t d, uint32_t r, uint32_t& rem) {
-  uint32_t q = __umulhi(n, r);
-  rem = n - q * d;
-  if (rem >= d) { ++q; rem -= d; }
-  return q;
-}
-
 // BLOCKS = false: n contiguous rows (TurboQuant.decode).  BLOCKS = true: the rows are the (position, head) entries of the
 // cache blocks listed in a.slots; every listed block that exists is decoded into the block of the same index of the
 // output buffer (the batch decompress of aither_kvcache/vllm/backend.py:1040-1091 without its gather / unique / scatter
@@ -151,45 +148,50 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
   const uint32_t n_one = (uint32_t)a.n, n_total = BLOCKS && a.packed2 ? 2u * n_one : n_one;
   const uint32_t steps = (n_total + DM_ROWS - 1) / DM_ROWS, stride = gridDim.x * RG;
   const uint32_t per_blk = BLOCKS ? (uint32_t)a.block_size * (uint32_t)a.heads : 1u, heads = BLOCKS ? (uint32_t)a.heads : 1u;
+  const uint32_t most_blocks = (uint32_t)a.max_blocks;
   const uint32_t per_r = 0xffffffffu / per_blk, heads_r = 0xffffffffu / heads;
 
   // ---- rows: block ids two steps ahead, codes and norms one step ahead
-  int64_t id[DM_MT], before[DM_MT];
+  uint32_t id[DM_MT][2], before[DM_MT][2];    // of a block and of the one listed before it: low and high word, or the same word twice
+  uint32_t place[DM_MT];                      // position and head inside the block
   uint32_t raw[DM_MT][RAW];
   float nrm[DM_MT];
   out_t* dst[DM_MT];                          // null: nothing to write
+  const uint32_t* ids = (const uint32_t*)a.slots;
+  const uint32_t wide = a.slot_itype == AKV_I64 ? 1u : 0u;
   auto fetch_ids = [&](uint32_t step) {
     if constexpr (BLOCKS) {
 #pragma unroll
       for (int mt = 0; mt < DM_MT; ++mt) {
-        uint32_t n = min(step * DM_ROWS + 16 * mt + col, n_total - 1), rem;
+        uint32_t n = min(step * DM_ROWS + 16 * mt + col, n_total - 1);
         if (n >= n_one) n -= n_one;
-        const uint32_t li = dm_div(n, per_blk, per_r, rem);
-        id[mt] = akv_load_index(a.slots, a.slot_itype, li);
-        before[mt] = li > 0 ? akv_load_index(a.slots, a.slot_itype, li - 1) : -1;
+        const uint32_t li = akv_div32(n, per_blk, per_r, place[mt]);
+        // (words as they lie: widened to 64 bits here, each of the loads was waited for on its own)
+        const uint32_t at = li << wide, prev = (li - min(li, 1u)) << wide;
+        id[mt][0] = ids[at]; id[mt][1] = ids[at + wide];
+        before[mt][0] = ids[prev]; before[mt][1] = ids[prev + wide];
       }
     }
   };
   auto fetch_rows = [&](uint32_t step) {
 #pragma unroll
     for (int mt = 0; mt < DM_MT; ++mt) {
-      const uint32_t at = step * DM_ROWS + 16 * mt + col;
-      uint32_t n = min(at, n_total - 1);
+      const uint32_t at = step * DM_ROWS + 16 * mt + col, n = min(at, n_total - 1);
       const bool second = BLOCKS && n >= n_one;
-      if (second) n -= n_one;
-      int64_t po, no, oo;
+      uint64_t po, no, oo;
       bool live = at < n_total;
       if constexpr (BLOCKS) {
-        uint32_t rem, head;
-        dm_div(n, per_blk, per_r, rem);
-        const uint32_t pos = dm_div(rem, heads, heads_r, head);
-        live = live && id[mt] >= 0 && id[mt] < a.max_blocks && id[mt] != before[mt];
-        const int64_t blk = live ? id[mt] : 0;          // (a row of block 0 is read and dropped)
-        po = blk * a.ps0 + pos * a.ps1 + head * a.ps2;
-        no = blk * a.ns0 + pos * a.ns1 + head * a.ns2;
-        oo = blk * a.os0 + pos * a.os1 + head * a.os2;
+        uint32_t head;
+        const uint32_t pos = akv_div32(place[mt], heads, heads_r, head);
+        const bool first = n - (second ? n_one : 0u) < per_blk;
+        live = live && (wide ? id[mt][1] == 0u : (int32_t)id[mt][0] >= 0) && id[mt][0] < most_blocks;
+        live = live && (first || id[mt][0] != before[mt][0] || id[mt][1] != before[mt][1]);
+        const uint32_t blk = live ? id[mt][0] : 0u;                 // (a row of block 0 is read and dropped)
+        po = (uint64_t)blk * (uint32_t)a.ps0 + (__umul24(pos, (uint32_t)a.ps1) + __umul24(head, (uint32_t)a.ps2));
+        no = (uint64_t)blk * (uint32_t)a.ns0 + (__umul24(pos, (uint32_t)a.ns1) + __umul24(head, (uint32_t)a.ns2));
+        oo = (uint64_t)blk * (uint32_t)a.os0 + (__umul24(pos, (uint32_t)a.os1) + __umul24(head, (uint32_t)a.os2));
       } else {
-        po = n * a.ps0; no = n; oo = n * a.os0;
+        po = (uint64_t)n * (uint32_t)a.ps0; no = n; oo = (uint64_t)n * (uint32_t)a.os0;
       }
       dm_load_quarter<D, BITS>((second ? a.packed2 : a.packed) + po, g, raw[mt]);
       nrm[mt] = (second ? a.norms2 : a.norms)[no];
@@ -252,56 +254,72 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
   const uint32_t copy = (uint32_t)(lane & 31) * 8u;
 
   if (step >= steps) return;
-  fetch_rows(step);
-  fetch_ids(min(step + stride, steps - 1));
-  for (; step < steps; step += stride) {
-    uint32_t kw[DM_MT][KS];
-    float nv[DM_MT];
-    out_t* orow[DM_MT];
+  uint32_t kw[DM_MT][KS];
+  float nv[DM_MT];
+  out_t* orow[DM_MT];
+  auto take = [&]() {
 #pragma unroll
     for (int mt = 0; mt < DM_MT; ++mt) {
       dm_spread<D, BITS>(raw[mt], g, kw[mt]);
       nv[mt] = nrm[mt];
       orow[mt] = dst[mt];
     }
-    fetch_rows(min(step + stride, steps - 1));          // (past the end: the last step once more)
-    fetch_ids(min(step + 2 * stride, steps - 1));
-    if (__builtin_amdgcn_ballot_w64(orow[0] != nullptr || orow[DM_MT - 1] != nullptr) == 0) continue;
+  };
+  auto ahead = [&](uint32_t k) { return min(step + k * stride, steps - 1); };      // (past the end: the last step once more)
+  fetch_rows(step);
+  fetch_ids(ahead(1));
+  take();
+  fetch_rows(ahead(1));
+  fetch_ids(ahead(2));
+  for (; step < steps; step += stride) {
     dm_float4 acc[DM_MT][NT];
+    if (__builtin_amdgcn_ballot_w64(orow[0] != nullptr || orow[DM_MT - 1] != nullptr) != 0) {
 #pragma unroll
-    for (int mt = 0; mt < DM_MT; ++mt)
+      for (int mt = 0; mt < DM_MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = (dm_float4){0.f, 0.f, 0.f, 0.f};
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = (dm_float4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
+      for (int ks = 0; ks < KS; ++ks) {
+        union { uint32_t u[4]; dm_half8 h; } ch[DM_MT], cl[DM_MT];
 #pragma unroll
-      for (int mt = 0; mt < DM_MT; ++mt) {
-        union { uint32_t u[4]; dm_half8 h; } ch, cl;
-        const uint32_t w = kw[mt][ks];
+        for (int mt = 0; mt < DM_MT; ++mt)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const dm_u32x2 t = *(dm_lds_cu64*)(uintptr_t)__builtin_amdgcn_perm(w, copy, 0x0c020400u + ((uint32_t)b << 8));
-          ch.u[b] = t.x;
-          cl.u[b] = t.y;
-        }
+          for (int b = 0; b < 4; ++b) {
+            const dm_u32x2 t = *(dm_lds_cu64*)(uintptr_t)__builtin_amdgcn_perm(kw[mt][ks], copy, 0x0c020400u + ((uint32_t)b << 8));
+            ch[mt].u[b] = t.x;
+            cl[mt].u[b] = t.y;
+          }
+        // (term by term: products in a row do not wait for each other's sum)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[nt][ks], ch.h, acc[mt][nt], 0, 0, 0);
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah[nt][ks], cl.h, acc[mt][nt], 0, 0, 0);
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al[nt][ks], ch.h, acc[mt][nt], 0, 0, 0);
-        }
+        for (int term = 0; term < 3; ++term)
+#pragma unroll
+          for (int mt = 0; mt < DM_MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+              acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(term == 2 ? Al[nt][ks] : Ah[nt][ks], term == 1 ? cl[mt].h : ch[mt].h, acc[mt][nt], 0, 0, 0);
       }
     }
+    // The next rows are taken, and those after them requested, before this step's stores: loads and stores complete in one
+    // order, and the stores depend on a condition, so a wait behind them is a wait for the stores themselves.
+    __builtin_amdgcn_sched_barrier(0);
+    out_t* now[DM_MT];
+    float nvn[DM_MT];
+#pragma unroll
+    for (int mt = 0; mt < DM_MT; ++mt) { now[mt] = orow[mt]; nvn[mt] = nv[mt]; }
+    take();
+    fetch_rows(ahead(2));
+    fetch_ids(ahead(3));
+    __builtin_amdgcn_sched_barrier(0);
     // ---- x norm, cast (the reference multiplies the float32 rotated vector by the norm and then casts): lane (v, g)
     // holds rows 4 g + i of every tile
 #pragma unroll
     for (int mt = 0; mt < DM_MT; ++mt) {
-      if (orow[mt] == nullptr) continue;
+      if (now[mt] == nullptr) continue;
       if constexpr (ODT == AKV_F32) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           const dm_float4 y = acc[mt][nt] * inv_cs;
-          *(float4*)(orow[mt] + C * cw + 16 * nt + 4 * g) = make_float4(y.x * nv[mt], y.y * nv[mt], y.z * nv[mt], y.w * nv[mt]);
+          *(float4*)(now[mt] + C * cw + 16 * nt + 4 * g) = make_float4(y.x * nvn[mt], y.y * nvn[mt], y.z * nvn[mt], y.w * nvn[mt]);
         }
       } else {
 #pragma unroll
@@ -309,12 +327,12 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
           uint32_t w[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const float v0 = __fmul_rn(acc[mt][nt + (q >> 1)][2 * (q & 1)] * inv_cs, nv[mt]);
-            const float v1 = __fmul_rn(acc[mt][nt + (q >> 1)][2 * (q & 1) + 1] * inv_cs, nv[mt]);
-            if constexpr (ODT == AKV_F16) w[q] = (uint32_t)__half_as_ushort(__float2half_rn(v0)) | ((uint32_t)__half_as_ushort(__float2half_rn(v1)) << 16);
-            else w[q] = (uint32_t)akv_float_to_bf16_bits(v0) | ((uint32_t)akv_float_to_bf16_bits(v1) << 16);
+            const dm_float2 v = {acc[mt][nt + (q >> 1)][2 * (q & 1)] * inv_cs * nvn[mt], acc[mt][nt + (q >> 1)][2 * (q & 1) + 1] * inv_cs * nvn[mt]};
+            // (one conversion instruction per pair, to nearest even; element by element the bfloat16 one was six and a branch)
+            if constexpr (ODT == AKV_F16) w[q] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, dm_half2));
+            else w[q] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, dm_bf162));
           }
-          *(uint4*)(orow[mt] + C * cw + 16 * nt + 8 * g) = make_uint4(w[0], w[1], w[2], w[3]);
+          *(uint4*)(now[mt] + C * cw + 16 * nt + 8 * g) = make_uint4(w[0], w[1], w[2], w[3]);
         }
       }
     }
@@ -352,7 +370,16 @@ int akv_decode_mfma_try(const akv_gen_args& a, bool blocks, int d, int bits, int
   if (blocks && (((uintptr_t)a.ps1 | (uintptr_t)a.ps2) & palign || ((a.os1 | a.os2) & 7))) return AKV_ERR_UNSUPPORTED;
   // rows are counted in 32 bits, with room for two strides past the end
   if ((a.packed2 ? 2 : 1) * a.n >= ((int64_t)1 << 31) - ((int64_t)1 << 22)) return AKV_ERR_UNSUPPORTED;
-  if (blocks && (int64_t)a.block_size * a.heads >= ((int64_t)1 << 31)) return AKV_ERR_UNSUPPORTED;
+  // strides: of a block (or flat row) 32 bits, inside a block 24 bits and the sum of both products in 32
+  const int64_t outer[3] = {a.ps0, blocks ? a.ns0 : 0, a.os0};
+  for (int i = 0; i < 3; ++i)
+    if (outer[i] < 0 || outer[i] >= ((int64_t)1 << 32)) return AKV_ERR_UNSUPPORTED;
+  if (blocks) {      // (listed blocks, at most 2^31 of them, are indexed by 32-bit words)
+    const int64_t in1[3] = {a.ps1, a.ns1, a.os1}, in2[3] = {a.ps2, a.ns2, a.os2}, most = (int64_t)1 << 24;
+    if (a.block_size >= most || a.heads >= most || (int64_t)a.block_size * a.heads >= ((int64_t)1 << 31) || a.max_blocks >= ((int64_t)1 << 32)) return AKV_ERR_UNSUPPORTED;
+    for (int i = 0; i < 3; ++i)
+      if (in1[i] < 0 || in2[i] < 0 || in1[i] >= most || in2[i] >= most || a.block_size * in1[i] + a.heads * in2[i] >= ((int64_t)1 << 32)) return AKV_ERR_UNSUPPORTED;
+  }
   const float* PiT = (const float*)rot_prep + (size_t)d * d;
 #define DM_CASE(DD, BB) if (d == DD && bits == BB) return dm_launch_dt<DD, BB>(blocks, out_dtype, a, PiT, stream)
   DM_CASE(64, 2); DM_CASE(64, 3); DM_CASE(64, 4);
