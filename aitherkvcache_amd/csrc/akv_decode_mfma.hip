@@ -16,10 +16,11 @@
 // coordinate order that the spreading leaves is matched when the matrix is loaded.
 //
 // What bounds it: the loop, 24 products of 16 cycles and some 430 vector instructions per 16 rows of head_dim 128 and
-// wavefront at two wavefronts a SIMD, and the trips to memory around it; it moves 2.0 TB/s.  17k tokens x 8 heads at
-// head_dim 128, K and V: 45 us (two launches with the matrix in LDS, 64 KB read per 32 rows and three barriers of set-up:
-// 72 us; with block ids widened to 64 bits where they are loaded, a wait per load: 53 us).  6,290 tokens x 8 heads at
-// head_dim 256 784 us on the vector kernel, 56 here; 20,936 tokens x 16 heads at head_dim 64, 3 bits, 385 and 36 us.
+// wavefront at two wavefronts a SIMD, and the trips to memory around it; it moves 2.1 TB/s.  17k tokens x 8 heads at
+// head_dim 128, K and V: 42 us (two launches with the matrix in LDS, 64 KB read per 32 rows and three barriers of set-up:
+// 72 to 75 us; with block ids widened to 64 bits where they are loaded, a wait per load: 53 us; with the matrix read as the
+// lanes need it, 64 cache lines per load: 45 us).  6,290 tokens x 8 heads at head_dim 256 784 us on the vector kernel, 53
+// here; 20,936 tokens x 16 heads at head_dim 64, 3 bits, 385 and 34 us.
 // No barrier after the set-up: the wavefronts of a row only share cache lines.
 #include "akv_common.h"
 #include "akv_nibble.h"
@@ -33,6 +34,7 @@ typedef uint32_t dm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t dm_u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const dm_u32x2 dm_lds_cu64;
 typedef __attribute__((address_space(3))) dm_u32x4 dm_lds_u128;
+typedef __attribute__((address_space(3))) dm_float4 dm_lds_f128;
 
 #define DM_WAVES 8
 #define DM_THREADS (DM_WAVES * 64)
@@ -131,6 +133,12 @@ __device__ __forceinline__ void dm_spread(const uint32_t (&w)[dm_cfg<D, BITS>::R
   }
 }
 
+__device__ __forceinline__ void dm_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // BLOCKS = false: n contiguous rows (TurboQuant.decode).  BLOCKS = true: the rows are the (position, head) entries of the
 // cache blocks listed in a.slots; every listed block that exists is decoded into the block of the same index of the
 // output buffer (the batch decompress of aither_kvcache/vllm/backend.py:1040-1091 without its gather / unique / scatter
@@ -201,6 +209,59 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
   uint32_t step = (uint32_t)rg * gridDim.x + blockIdx.x;
   fetch_ids(step);
 
+  // ---- matrix slice: row m of tile nt is output coordinate `mine` below (see the stores); lane (m, g) holds the contracted
+  // coordinates that quarter g of a row brings at k-step ks.  A wavefront takes a piece of a tile (16 rows x 4 quarters x F
+  // coordinates) through 8 KB of LDS of its own: read as the lanes need it, every load instruction touched 64 cache lines.
+  dm_half8 Ah[NT][KS], Al[NT][KS];
+  {
+    constexpr int F = D == 64 ? 16 : 32, Q = F / 4, PK = D / 4 / F, PIECES = NT * PK;     // PK pieces per tile
+    auto coordinate = [&](int nt, int m) {
+      return C * cw + (ODT == AKV_F32 ? 16 * nt + m : 32 * (nt >> 1) + 8 * (m >> 2) + 4 * (nt & 1) + (m & 3));
+    };
+    float4 part[Q];
+    auto request = [&](int piece) {
+      const int nt = piece / PK, pk = piece % PK;
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        const int seg = (i * 64 + lane) / Q, q = lane % Q;             // segment 16 g + m: F neighbouring floats
+        part[i] = *(const float4*)(PiT + (size_t)coordinate(nt, seg & 15) * D + (D / 4) * (seg >> 4) + F * pk + 4 * q);
+      }
+    };
+    const uint32_t stage = (uint32_t)wave * (64 * F * 4);
+    request(0);
+#pragma unroll
+    for (int piece = 0; piece < PIECES; ++piece) {
+      const int nt = piece / PK, pk = piece % PK;
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        const int seg = (i * 64 + lane) / Q, q = lane % Q;
+        *(dm_lds_f128*)(uintptr_t)(stage + (uint32_t)(seg * F * 4 + 16 * (q ^ (seg & (Q - 1))))) = (dm_float4){part[i].x, part[i].y, part[i].z, part[i].w};
+      }
+      if (piece + 1 < PIECES) request(piece + 1);
+      dm_wave_sync();
+#pragma unroll
+      for (int k2 = 0; k2 < F / 16; ++k2) {                           // two k-steps: 16 neighbouring coordinates
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const dm_float4 x = *(dm_lds_f128*)(uintptr_t)(stage + (uint32_t)(lane * F * 4 + 16 * ((4 * k2 + i) ^ (lane & (Q - 1)))));
+          v[4 * i] = x.x; v[4 * i + 1] = x.y; v[4 * i + 2] = x.z; v[4 * i + 3] = x.w;
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < 2; ++k1)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float s = v[mf_kcoord<BITS>(k1, e >> 1, e & 1)] * DM_PSCALE;
+            const _Float16 h = (_Float16)s;
+            Ah[nt][(F / 8) * pk + 2 * k2 + k1][e] = h;
+            Al[nt][(F / 8) * pk + 2 * k2 + k1][e] = (_Float16)(s - (float)h);
+          }
+      }
+      dm_wave_sync();
+    }
+  }
+  __syncthreads();          // the table takes the same LDS
+
   // ---- table; the scale brings the largest level to [2^9, 2^10): no remainder that matters is a float16 subnormal
   float inv_cs;
   {
@@ -223,33 +284,6 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
     for (int i = 0; i < 8; ++i) *(dm_lds_u128*)(uintptr_t)(uint32_t)(e * 256 + half * 128 + i * 16) = (dm_u32x4){hi, lo, hi, lo};
   }
 
-  // ---- matrix slice: row m of tile nt is output coordinate `mine` below (see the stores); lane (m, g) holds the contracted
-  // coordinates that quarter g of a row brings at k-step ks
-  dm_half8 Ah[NT][KS], Al[NT][KS];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int m4 = col >> 2, mi = col & 3;
-    const int mine = C * cw + (ODT == AKV_F32 ? 16 * nt + 4 * m4 + mi : 32 * (nt >> 1) + 8 * m4 + 4 * (nt & 1) + mi);
-    const float4* p = (const float4*)(PiT + (size_t)mine * D + (D / 4) * g);
-#pragma unroll
-    for (int k2 = 0; k2 < KS / 2; ++k2) {               // two k-steps: 16 neighbouring coordinates
-      float v[16];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 t = p[4 * k2 + i];
-        v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
-      }
-#pragma unroll
-      for (int k1 = 0; k1 < 2; ++k1)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float s = v[mf_kcoord<BITS>(k1, e >> 1, e & 1)] * DM_PSCALE;
-          const _Float16 h = (_Float16)s;
-          Ah[nt][2 * k2 + k1][e] = h;
-          Al[nt][2 * k2 + k1][e] = (_Float16)(s - (float)h);
-        }
-    }
-  }
   __syncthreads();
   const uint32_t copy = (uint32_t)(lane & 31) * 8u;
 
