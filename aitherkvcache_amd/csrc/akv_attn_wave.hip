@@ -384,8 +384,9 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           }
 
           __builtin_amdgcn_sched_barrier(0);
-          if (k + 1 - win_k >= AW_WIN) load_window(k + 1);
-          load_keys(min(k + 1, mine - 1));      // (past the end: the last chunk once more)
+          // (past the end: the last chunk once more, out of the window it is in)
+          if (k + 1 < mine && k + 1 - win_k >= AW_WIN) load_window(k + 1);
+          load_keys(min(k + 1, mine - 1));
           __builtin_amdgcn_sched_barrier(0);
 
           // ---- running softmax in the log2 domain over t = score + exponent of the value norm

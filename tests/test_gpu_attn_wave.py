@@ -86,13 +86,14 @@ def test_edges_vs_float64(dev, d, bits, qh, kvh, bs):
         assert (out[i] - ref).norm() <= REL * ref.norm(), (i, n)
 
 
-@pytest.mark.parametrize("d,qh,kvh,bs", [(256, 16, 8, 16), (256, 4, 1, 32), (64, 16, 16, 32)])
-def test_more_chunks_than_a_window_of_block_ids(dev, d, qh, kvh, bs):
-    """A context so long that a wavefront goes through several windows of block ids: its blocks repeat a few, which the
-    reference counts."""
+@pytest.mark.parametrize("d,qh,kvh,bs,chunks", [(256, 16, 8, 16, 70), (256, 4, 1, 32, 70), (64, 16, 16, 32, 70),
+                                                (256, 8, 8, 16, 32), (256, 8, 8, 32, 64), (64, 16, 16, 16, 64), (64, 16, 16, 32, 32)])
+def test_more_chunks_than_a_window_of_block_ids(dev, d, qh, kvh, bs, chunks):
+    """A context so long that a wavefront goes through several windows of block ids, of 32 chunks each: `chunks` a wavefront, or
+    one less; at 32 and 64 the last chunk is the last of a window.  Its blocks repeat a few, which the reference counts."""
     rng, tq, rows, norms = make(dev, d, 4, kvh, 8, bs, 7)
     shares = 8 // kvh if kvh < 8 else 1
-    n = 32 * 256 * 70 * shares - 5                       # 70 chunks a wavefront, or one less
+    n = 32 * 256 * chunks * shares - (5 if chunks == 70 else 0)
     table = rng.integers(0, 8, size=-(-n // bs)).astype(np.int32)
     q = torch.from_numpy(rng.standard_normal((1, qh, d)).astype(np.float32)).to(dev)
     P = tq._packed_dim
