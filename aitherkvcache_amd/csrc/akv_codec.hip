@@ -128,6 +128,7 @@ __global__ void akv_prepare_rotation_kernel(const float* __restrict__ R, float* 
 
 int akv_prepare_rotation_mfma(const float* rotation, int d, void* prep, hipStream_t stream);
 int akv_prepare_decode_mfma(const float* rotation, int d, void* prep, hipStream_t stream);
+int akv_prepare_decode_slices(const float* rotation, int d, void* prep, hipStream_t stream);
 int akv_decode_mfma_try(const akv_gen_args& a, bool blocks, int d, int bits, int out_dtype, const void* rot_prep,
                         hipStream_t stream);
 
@@ -145,9 +146,10 @@ extern "C" int akv_rotation_prepare(const float* rotation, int d, void* prep, si
   if (d == 128) {
     int rc = akv_prepare_rotation_mfma(rotation, d, prep, (hipStream_t)stream);
     if (rc) return rc;
-    return akv_prepare_decode_mfma(rotation, d, prep, (hipStream_t)stream);
+    rc = akv_prepare_decode_mfma(rotation, d, prep, (hipStream_t)stream);
+    if (rc) return rc;
   }
-  return AKV_OK;
+  return akv_prepare_decode_slices(rotation, d, prep, (hipStream_t)stream);
 }
 
 // ----------------------------------------------------------------------------------

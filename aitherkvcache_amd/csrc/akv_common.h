@@ -77,9 +77,14 @@ void akv_profile_stamp(hipStream_t s, hipEvent_t begin);
 //   [0, d*d)        Pi     row-major  (y_i = sum_j Pi[i][j] x_j)
 //   [d*d, 2*d*d)    Pi^T   row-major
 //   [2*d*d, ...)    d = 128 only: float16 hi/lo operand tiles of the MFMA encode kernel (64 KB),
-//                   a flag word (256 B reserved), the same for the MFMA decode kernel (64 KB)
-static inline size_t akv_prep_floats(int d) { return (size_t)4 * d * d + 1024; }
+//                   a flag word (256 B reserved), the same for the rotations of the attention kernels (64 KB)
+//   then            d = 64, 128, 256: float16 hi/lo slices of Pi^T, the operand of the MFMA decode kernel (4 d*d bytes)
 #define AKV_PREP_DECODE_OFFSET(d) ((size_t)2 * (d) * (d) * 4 + 65536 + 256)
+#define AKV_PREP_SLICES_OFFSET(d) ((size_t)2 * (d) * (d) * 4 + ((d) == 128 ? 2 * 65536 + 256 : 0))
+static inline size_t akv_prep_floats(int d) {
+  const size_t reserved = (size_t)4 * d * d + 1024, used = AKV_PREP_SLICES_OFFSET(d) / 4 + (d == 512 ? 0 : (size_t)d * d);
+  return reserved > used ? reserved : used;
+}
 
 // Arguments of the encode / decode kernels (flat and paged forms share one struct).
 struct akv_gen_args {

@@ -3,24 +3,27 @@
 //
 //   X^T[i, v] = n_v * sum_j Pi[j, i] c[code[v, j]]              v_mfma_f32_16x16x32_f16
 //     A = Pi^T: a wavefront keeps the C x D slice of its C output coordinates in registers, two float16 terms (hi + lo,
-//         scaled by 64), split from the float32 matrix at its start.  D / C wavefronts share a row.
+//         scaled by 64), in the order its lanes take them from the prepared-rotation buffer (akv_dm_slices_kernel).  D / C
+//         wavefronts share a row.
 //     B = centroids of the codes: lane (v = l % 16, g = l / 16) loads quarter g of the packed row of vector v.  A code
 //         BYTE (two codes) indexes a table in LDS whose 8-byte entry is the float16 pair (c[a], c[b]) and the pair of
 //         remainders (c = hi + lo to ~22 bits); every entry is replicated 32 times (address = byte * 256 + (lane & 31) * 8,
 //         built by one byte permute), so look-ups do not conflict on a bank.
 //     Three products per tile: Pi_hi c_hi + Pi_hi c_lo + Pi_lo c_hi.
-//   The rows of an A tile are permuted so that the four lanes of a vector write 64 neighbouring bytes per store; a lane
-//   needs one norm and one address per vector.
+//   The rows of an A tile are permuted so that a lane ends up with eight neighbouring coordinates of ONE row from two tiles:
+//   it needs one norm and one address per vector, and the four lanes of a vector write 64 neighbouring bytes per store.
 //
 // 3-bit and 2-bit rows are spread to one code per nibble in registers (akv_nibble.h) and take the same table; the
 // coordinate order that the spreading leaves is matched when the matrix is loaded.
 //
-// What bounds it: the loop, 24 products of 16 cycles and some 430 vector instructions per 16 rows of head_dim 128 and
-// wavefront at two wavefronts a SIMD, and the trips to memory around it; it moves 2.1 TB/s.  17k tokens x 8 heads at
-// head_dim 128, K and V: 42 us (two launches with the matrix in LDS, 64 KB read per 32 rows and three barriers of set-up:
-// 72 to 75 us; with block ids widened to 64 bits where they are loaded, a wait per load: 53 us; with the matrix read as the
-// lanes need it, 64 cache lines per load: 45 us).  6,290 tokens x 8 heads at head_dim 256 784 us on the vector kernel, 53
-// here; 20,936 tokens x 16 heads at head_dim 64, 3 bits, 385 and 34 us.
+// What bounds it: the loop, 48 products of 16 cycles and some 430 vector instructions of four per 16 rows of head_dim 128
+// and wavefront at two wavefronts a SIMD, and the trips to memory around it.
+// Flat rows at head_dim 128 (us; the matrix in LDS, 64 KB read per 32 rows | split from the float32 matrix in every launch |
+// as it is now): 4-bit to float16, 65,536 rows 14.2 | 16.0 | 12.4, 2^20 rows 110 | 111 | 106; 3-bit 2^20 113 | 116 | 110;
+// 4-bit to float32 2^20 156 | 181 | 124.
+// K and V of 17k tokens x 8 heads at head_dim 128: 72 to 75 us as two launches with the matrix in LDS, 42 with the slice split
+// in the launch (53 with block ids widened to 64 bits where they are loaded, a wait per load).  6,290 tokens x 8 heads at
+// head_dim 256 784 us on the vector kernel, 53; 20,936 tokens x 16 heads at head_dim 64, 3 bits, 385 and 34 us.
 // No barrier after the set-up: the wavefronts of a row only share cache lines.
 #include "akv_common.h"
 #include "akv_nibble.h"
@@ -34,7 +37,6 @@ typedef uint32_t dm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t dm_u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const dm_u32x2 dm_lds_cu64;
 typedef __attribute__((address_space(3))) dm_u32x4 dm_lds_u128;
-typedef __attribute__((address_space(3))) dm_float4 dm_lds_f128;
 
 #define DM_WAVES 8
 #define DM_THREADS (DM_WAVES * 64)
@@ -82,6 +84,34 @@ int akv_prepare_decode_mfma(const float* rotation, int d, void* prep, hipStream_
   uint4* bop = (uint4*)((char*)prep + AKV_PREP_DECODE_OFFSET(d));
   akv_dm_prepare_kernel<<<8, 256, 0, stream>>>(rotation, bop);
   AKV_LAUNCH_CHECK("akv_dm_prepare_kernel");
+  return AKV_OK;
+}
+
+// Operand of the decode kernel: Pi^T in tiles of 16 output coordinates, [hi | lo][tile][piece][lane] x 16 bytes.  Lane (m, g)
+// of piece h holds contracted coordinates (D / 4) g + 8 h + 0 .. 7 of the tile's row m, output coordinate dm_coordinate.
+__host__ __device__ constexpr int dm_coordinate(int tile, int m) {
+  return 32 * (tile >> 1) + 8 * (m >> 2) + 4 * (tile & 1) + (m & 3);   // a lane's rows 4 g + i of two tiles are eight neighbours
+}
+__global__ __launch_bounds__(256) void akv_dm_slices_kernel(const float* __restrict__ Pi, int d, uint4* __restrict__ slices) {
+  const int pieces = d / 32, n = d * d / 8, t = blockIdx.x * 256 + threadIdx.x;      // (tile, piece, lane)
+  if (t >= n) return;
+  const int lane = t & 63, h = (t >> 6) % pieces, tile = (t >> 6) / pieces;
+  const int i = dm_coordinate(tile, lane & 15), k0 = (d / 4) * (lane >> 4) + 8 * h;
+  uint32_t hi[4] = {0u, 0u, 0u, 0u}, lo[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float v = Pi[(size_t)(k0 + e) * d + i] * DM_PSCALE;
+    const __half hh = __float2half_rn(v);
+    hi[e >> 1] |= (uint32_t)__half_as_ushort(hh) << (16 * (e & 1));
+    lo[e >> 1] |= (uint32_t)__half_as_ushort(__float2half_rn(v - __half2float(hh))) << (16 * (e & 1));
+  }
+  slices[t] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+  slices[n + t] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+}
+int akv_prepare_decode_slices(const float* rotation, int d, void* prep, hipStream_t stream) {
+  if (!(d == 64 || d == 128 || d == 256)) return AKV_OK;
+  akv_dm_slices_kernel<<<(d * d / 8 + 255) / 256, 256, 0, stream>>>(rotation, d, (uint4*)((char*)prep + AKV_PREP_SLICES_OFFSET(d)));
+  AKV_LAUNCH_CHECK("akv_dm_slices_kernel");
   return AKV_OK;
 }
 
@@ -133,19 +163,13 @@ __device__ __forceinline__ void dm_spread(const uint32_t (&w)[dm_cfg<D, BITS>::R
   }
 }
 
-__device__ __forceinline__ void dm_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // BLOCKS = false: n contiguous rows (TurboQuant.decode).  BLOCKS = true: the rows are the (position, head) entries of the
 // cache blocks listed in a.slots; every listed block that exists is decoded into the block of the same index of the
 // output buffer (the batch decompress of aither_kvcache/vllm/backend.py:1040-1091 without its gather / unique / scatter
 // passes).  An entry equal to the one before it is not decoded again: the padding of a block table is such a run.
 // With a.packed2 the rows of a second tensor (V) follow those of the first.
 template <int D, int BITS, int ODT, bool BLOCKS>
-__global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_args a, const float* __restrict__ PiT) {
+__global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_args a, const uint4* __restrict__ slices) {
   typedef dm_cfg<D, BITS> cfg;
   constexpr int C = cfg::C, CW = cfg::CW, RG = cfg::RG, NT = cfg::NT, KS = cfg::KS, RAW = cfg::RAW;
   typedef typename akv_elem<ODT>::type out_t;
@@ -187,8 +211,9 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
       const uint32_t at = step * DM_ROWS + 16 * mt + col, n = min(at, n_total - 1);
       const bool second = BLOCKS && n >= n_one;
       uint64_t po, no, oo;
-      bool live = at < n_total;
+      bool live = true;          // (flat: a row past the end is the last one, stored once more)
       if constexpr (BLOCKS) {
+        live = at < n_total;
         uint32_t head;
         const uint32_t pos = akv_div32(place[mt], heads, heads_r, head);
         const bool first = n - (second ? n_one : 0u) < per_blk;
@@ -209,58 +234,31 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
   uint32_t step = (uint32_t)rg * gridDim.x + blockIdx.x;
   fetch_ids(step);
 
-  // ---- matrix slice: row m of tile nt is output coordinate `mine` below (see the stores); lane (m, g) holds the contracted
-  // coordinates that quarter g of a row brings at k-step ks.  A wavefront takes a piece of a tile (16 rows x 4 quarters x F
-  // coordinates) through 8 KB of LDS of its own: read as the lanes need it, every load instruction touched 64 cache lines.
+  // ---- matrix slice, as prepared; float32 rows are stored four neighbouring coordinates a lane and tile, so there row m of
+  // tile nt is coordinate 16 nt + m, wherever the operand has it
   dm_half8 Ah[NT][KS], Al[NT][KS];
   {
-    constexpr int F = D == 64 ? 16 : 32, Q = F / 4, PK = D / 4 / F, PIECES = NT * PK;     // PK pieces per tile
-    auto coordinate = [&](int nt, int m) {
-      return C * cw + (ODT == AKV_F32 ? 16 * nt + m : 32 * (nt >> 1) + 8 * (m >> 2) + 4 * (nt & 1) + (m & 3));
-    };
-    float4 part[Q];
-    auto request = [&](int piece) {
-      const int nt = piece / PK, pk = piece % PK;
+    const uint4* hi = slices + (size_t)(C / 16 * cw) * (KS * 64);
+    const uint4* lo = hi + (D / 16) * (KS * 64);
 #pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        const int seg = (i * 64 + lane) / Q, q = lane % Q;             // segment 16 g + m: F neighbouring floats
-        part[i] = *(const float4*)(PiT + (size_t)coordinate(nt, seg & 15) * D + (D / 4) * (seg >> 4) + F * pk + 4 * q);
-      }
-    };
-    const uint32_t stage = (uint32_t)wave * (64 * F * 4);
-    request(0);
+    for (int nt = 0; nt < NT; ++nt) {
+      const int at = ODT == AKV_F32 ? (2 * (nt >> 1) + ((col >> 2) & 1)) * (KS * 64) + 16 * g + 4 * (2 * (nt & 1) + (col >> 3)) + (col & 3)
+                                    : nt * (KS * 64) + lane;
 #pragma unroll
-    for (int piece = 0; piece < PIECES; ++piece) {
-      const int nt = piece / PK, pk = piece % PK;
-#pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        const int seg = (i * 64 + lane) / Q, q = lane % Q;
-        *(dm_lds_f128*)(uintptr_t)(stage + (uint32_t)(seg * F * 4 + 16 * (q ^ (seg & (Q - 1))))) = (dm_float4){part[i].x, part[i].y, part[i].z, part[i].w};
-      }
-      if (piece + 1 < PIECES) request(piece + 1);
-      dm_wave_sync();
-#pragma unroll
-      for (int k2 = 0; k2 < F / 16; ++k2) {                           // two k-steps: 16 neighbouring coordinates
-        float v[16];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const dm_float4 x = *(dm_lds_f128*)(uintptr_t)(stage + (uint32_t)(lane * F * 4 + 16 * ((4 * k2 + i) ^ (lane & (Q - 1)))));
-          v[4 * i] = x.x; v[4 * i + 1] = x.y; v[4 * i + 2] = x.z; v[4 * i + 3] = x.w;
-        }
+      for (int ks = 0; ks < KS; ks += 2) {            // 16 neighbouring coordinates, in the order a row's codes are spread
+        union { uint4 u[2]; _Float16 h[16]; } ph, pl;
+        ph.u[0] = hi[at + ks * 64]; ph.u[1] = hi[at + (ks + 1) * 64];
+        pl.u[0] = lo[at + ks * 64]; pl.u[1] = lo[at + (ks + 1) * 64];
 #pragma unroll
         for (int k1 = 0; k1 < 2; ++k1)
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float s = v[mf_kcoord<BITS>(k1, e >> 1, e & 1)] * DM_PSCALE;
-            const _Float16 h = (_Float16)s;
-            Ah[nt][(F / 8) * pk + 2 * k2 + k1][e] = h;
-            Al[nt][(F / 8) * pk + 2 * k2 + k1][e] = (_Float16)(s - (float)h);
+            Ah[nt][ks + k1][e] = ph.h[mf_kcoord<BITS>(k1, e >> 1, e & 1)];
+            Al[nt][ks + k1][e] = pl.h[mf_kcoord<BITS>(k1, e >> 1, e & 1)];
           }
       }
-      dm_wave_sync();
     }
   }
-  __syncthreads();          // the table takes the same LDS
 
   // ---- table; the scale brings the largest level to [2^9, 2^10): no remainder that matters is a float16 subnormal
   float inv_cs;
@@ -305,9 +303,14 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
   take();
   fetch_rows(ahead(1));
   fetch_ids(ahead(2));
+  // (the slice is waited for here: left to its first use, in the loop, the wait would be for the stores of the step before too)
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(Ah[nt][ks]), "+v"(Al[nt][ks]));
   for (; step < steps; step += stride) {
     dm_float4 acc[DM_MT][NT];
-    if (__builtin_amdgcn_ballot_w64(orow[0] != nullptr || orow[DM_MT - 1] != nullptr) != 0) {
+    if (!BLOCKS || __builtin_amdgcn_ballot_w64(orow[0] != nullptr || orow[DM_MT - 1] != nullptr) != 0) {
 #pragma unroll
       for (int mt = 0; mt < DM_MT; ++mt)
 #pragma unroll
@@ -348,8 +351,31 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
     // holds rows 4 g + i of every tile
 #pragma unroll
     for (int mt = 0; mt < DM_MT; ++mt) {
-      if (now[mt] == nullptr) continue;
-      if constexpr (ODT == AKV_F32) {
+      if (BLOCKS && now[mt] == nullptr) continue;
+      if constexpr (ODT == AKV_F32 && !BLOCKS) {
+        // Neighbouring lanes exchange half of what they hold: eight lanes then write 128 bytes of one row, a whole cache line
+        // that need not stay in the L2 cache.  (2^20 rows of 128: 124 us; 139 without the hint, 177 as 64-byte pieces, 158 so
+        // with the hint.  A block-wise row may have nothing to write beside one that has: there the pieces stay.)
+        const bool odd = col & 1;
+        const uint64_t mine = (uint64_t)(uintptr_t)now[mt];
+        const uint64_t theirs = (uint64_t)akv_dpp_u32<0xB1>((uint32_t)mine) | ((uint64_t)akv_dpp_u32<0xB1>((uint32_t)(mine >> 32)) << 32);
+        float* const r0 = (float*)(uintptr_t)(odd ? theirs : mine) + C * cw + 4 * g + (odd ? 16 : 0);      // the even lane's row, then the odd one's
+        float* const r1 = (float*)(uintptr_t)(odd ? mine : theirs) + C * cw + 4 * g + (odd ? 16 : 0);
+#pragma unroll
+        for (int nt = 0; nt < NT; nt += 2) {
+          const dm_float4 y0 = acc[mt][nt] * inv_cs * nvn[mt], y1 = acc[mt][nt + 1] * inv_cs * nvn[mt];
+          dm_float4 w0, w1;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float give = odd ? y0[i] : y1[i];
+            const float got = __uint_as_float(akv_dpp_u32<0xB1>(__float_as_uint(give)));
+            w0[i] = odd ? got : y0[i];
+            w1[i] = odd ? y1[i] : got;
+          }
+          __builtin_nontemporal_store(w0, (dm_float4*)(r0 + 16 * nt));
+          __builtin_nontemporal_store(w1, (dm_float4*)(r1 + 16 * nt));
+        }
+      } else if constexpr (ODT == AKV_F32) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
           const dm_float4 y = acc[mt][nt] * inv_cs;
@@ -379,18 +405,18 @@ static bool dm_disabled() {
 }
 
 template <int D, int BITS, int ODT, bool BLOCKS>
-static int dm_launch(const akv_gen_args& a, const float* PiT, hipStream_t stream) {
+static int dm_launch(const akv_gen_args& a, const uint4* slices, hipStream_t stream) {
   const int64_t n_total = BLOCKS && a.packed2 ? 2 * a.n : a.n, steps = (n_total + DM_ROWS - 1) / DM_ROWS;
   const int cus = akv_cached_cu_count() > 0 ? akv_cached_cu_count() : 256;
-  AKV_LAUNCH_TIMED((akv_decode_mfma_kernel<D, BITS, ODT, BLOCKS>), (int)(steps < cus ? steps : cus), DM_THREADS, DM_LDS_BYTES, stream, a, PiT);
+  AKV_LAUNCH_TIMED((akv_decode_mfma_kernel<D, BITS, ODT, BLOCKS>), (int)(steps < cus ? steps : cus), DM_THREADS, DM_LDS_BYTES, stream, a, slices);
   AKV_LAUNCH_CHECK("akv_decode_mfma_kernel");
   return AKV_OK;
 }
 template <int D, int BITS>
-static int dm_launch_dt(bool blocks, int out_dtype, const akv_gen_args& a, const float* PiT, hipStream_t stream) {
-  if (out_dtype == AKV_F16) return blocks ? dm_launch<D, BITS, AKV_F16, true>(a, PiT, stream) : dm_launch<D, BITS, AKV_F16, false>(a, PiT, stream);
-  if (out_dtype == AKV_BF16) return blocks ? dm_launch<D, BITS, AKV_BF16, true>(a, PiT, stream) : dm_launch<D, BITS, AKV_BF16, false>(a, PiT, stream);
-  return blocks ? dm_launch<D, BITS, AKV_F32, true>(a, PiT, stream) : dm_launch<D, BITS, AKV_F32, false>(a, PiT, stream);
+static int dm_launch_dt(bool blocks, int out_dtype, const akv_gen_args& a, const uint4* slices, hipStream_t stream) {
+  if (out_dtype == AKV_F16) return blocks ? dm_launch<D, BITS, AKV_F16, true>(a, slices, stream) : dm_launch<D, BITS, AKV_F16, false>(a, slices, stream);
+  if (out_dtype == AKV_BF16) return blocks ? dm_launch<D, BITS, AKV_BF16, true>(a, slices, stream) : dm_launch<D, BITS, AKV_BF16, false>(a, slices, stream);
+  return blocks ? dm_launch<D, BITS, AKV_F32, true>(a, slices, stream) : dm_launch<D, BITS, AKV_F32, false>(a, slices, stream);
 }
 
 // returns AKV_ERR_UNSUPPORTED when the fast path does not apply (the caller then uses the general kernel)
@@ -414,8 +440,8 @@ int akv_decode_mfma_try(const akv_gen_args& a, bool blocks, int d, int bits, int
     for (int i = 0; i < 3; ++i)
       if (in1[i] < 0 || in2[i] < 0 || in1[i] >= most || in2[i] >= most || a.block_size * in1[i] + a.heads * in2[i] >= ((int64_t)1 << 32)) return AKV_ERR_UNSUPPORTED;
   }
-  const float* PiT = (const float*)rot_prep + (size_t)d * d;
-#define DM_CASE(DD, BB) if (d == DD && bits == BB) return dm_launch_dt<DD, BB>(blocks, out_dtype, a, PiT, stream)
+  const uint4* slices = (const uint4*)((const char*)rot_prep + AKV_PREP_SLICES_OFFSET(d));
+#define DM_CASE(DD, BB) if (d == DD && bits == BB) return dm_launch_dt<DD, BB>(blocks, out_dtype, a, slices, stream)
   DM_CASE(64, 2); DM_CASE(64, 3); DM_CASE(64, 4);
   DM_CASE(128, 2); DM_CASE(128, 3); DM_CASE(128, 4);
   DM_CASE(256, 2); DM_CASE(256, 3); DM_CASE(256, 4);
