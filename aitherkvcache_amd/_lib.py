@@ -128,6 +128,7 @@ def lib() -> C.CDLL:
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
+        handle.akv_last_error()       # the thread's thread-local block of the library, touched: see akv_touch_thread
         _lib = handle
     return _lib
 

@@ -4,7 +4,10 @@ tensors (reference: tests/test_core.py:246-425, tests/test_hybrid_hooks.py:411-4
 tests/test_triattention.py:62-86)."""
 import ctypes
 import os
+import platform
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -66,6 +69,26 @@ def test_library_loads_and_reports_version():
     assert L.akv_hybrid25_encode(ptr, 0, 3, 128, ptr, ptr, 43, None) == _lib.AKV_ERR_INVALID
     assert L.akv_hybrid25_decode(ptr, 40, 3, ptr, ptr, 128, None) == _lib.AKV_ERR_INVALID
     assert L.akv_hybrid25_decode(None, 44, 0, None, None, 128, None) == _lib.AKV_OK
+
+
+def test_loading_brings_the_thread_up_to_date():
+    """A library with thread-local storage leaves every thread behind that has not touched it, and the HIP runtime's own
+    thread-local accesses slow until then (1 us a launch): lib() touches it.  Read from where x86-64 glibc keeps it: the
+    second word of the thread's control block points to the generation its table of blocks is of."""
+    if platform.machine() != "x86_64" or platform.libc_ver()[0] != "glibc":
+        pytest.skip("the layout of the control block is x86-64 glibc's")
+    code = """
+import ctypes as C, torch
+from aitherkvcache_amd import _lib
+this = C.CDLL(None).pthread_self
+this.restype = C.c_void_p
+generation = lambda: C.c_size_t.from_address(C.c_void_p.from_address(this() + 8).value).value
+lib = _lib.lib()
+loaded = generation()
+lib.akv_last_error()
+assert generation() == loaded, (loaded, generation())
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 
 
 # ---- TurboQuant surface -------------------------------------------------------------------
