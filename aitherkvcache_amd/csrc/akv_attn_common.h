@@ -124,7 +124,7 @@ __device__ __forceinline__ int64_t akv_seq_tokens(const void* context_lens, int 
   return ctx < cap ? ctx : cap;
 }
 
-// One workgroup (256 threads) writes prefix[0..S].
+// One workgroup (256 threads or more: those past 255 hold nothing) writes prefix[0..S].
 __device__ __forceinline__ void akv_block_prefix_scan(const void* context_lens, int cl_itype, int S,
                                                       int block_size, int64_t max_blocks_per_seq,
                                                       int32_t* prefix, int32_t* scratch /*[>= 4] LDS*/) {
@@ -155,7 +155,7 @@ __device__ __forceinline__ void akv_block_prefix_scan(const void* context_lens, 
 
 // ----------------------------------------------------------------------------------
 // Block prefix of the batch and partition of the global block axis among the G workgroups of the matrix-core
-// kernel, written by one workgroup of 256 threads.
+// kernel, written by one workgroup of 256 threads or more.
 //
 // A workgroup whose range crosses a sequence boundary starts twice (query operand, block ids, first rows, a
 // partial chunk at both ends): measured, such workgroups finish 5 us after the others and ARE the tail of
@@ -166,11 +166,15 @@ __device__ __forceinline__ void akv_block_prefix_scan(const void* context_lens, 
 // Otherwise the axis is cut into G equal ranges as before.  Either way workgroups and sequences both advance
 // monotonically along the axis, so slot = workgroup + sequence stays unique, and seqw[s] = (first, last
 // workgroup that meets sequence s), which the reduce kernel reads instead of dividing by the range length.
-// `cb` = blocks per chunk of the main kernel (2 for blocks of 16 tokens, 1 for blocks of 32).
+// `cb` = blocks per chunk of the main kernel (2 for blocks of 16 tokens, 1 for blocks of 32).  `shares` > 1: so many wavefronts
+// of a workgroup go through its chunks side by side and merge their results at the end of every segment.  Whole workgroups then
+// pay for more sequences too (a second segment costs what one more round of chunks does): up to half the workgroups, while the
+// longest range is at most a round longer than an equal one (one kv head, 48 sequences: of 700 tokens 21.3 -> 17.7 us, of 1k to
+// 16k the step 41.2 -> 36.6).
 // ----------------------------------------------------------------------------------
 __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G, int cb, int32_t* wgdesc, int32_t* seqw,
                                                    int32_t* lds /*[>= 257]*/, const void* context_lens, int cl_itype,
-                                                   int block_size, int64_t max_blocks_per_seq) {
+                                                   int block_size, int64_t max_blocks_per_seq, int shares = 1) {
   const int tid = threadIdx.x, lane = tid & 63;
   int32_t* p_wfirst = lds;              // [65] first workgroup of each sequence; [64] = workgroups in use
   int32_t* p_pref = lds + 65;           // [65] block prefix; [64] = total
@@ -215,15 +219,20 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
     const int c = (n + cb - 1) / cb;                             // chunks of the lane's sequence
     const int sumc = akv_wave_sum(c);
     const int nz = __popcll(__ballot(c > 0));
-    const int aligned = (nz >= 1 && nz * 8 <= G) ? 1 : 0;
-    if (aligned) {
-      int lo = (sumc + G - 1) / G, hi = (sumc + (G - nz) - 1) / (G - nz);      // hi is always feasible
-      if (lo < 1) lo = 1;
+    int aligned = (nz >= 1 && nz * 8 <= G) ? 1 : 0;
+    int lo = (sumc + G - 1) / G;
+    if (lo < 1) lo = 1;
+    if (aligned || (shares > 1 && nz >= 1 && 2 * nz <= G)) {
+      const int equal = lo;
+      int hi = (sumc + (G - nz) - 1) / (G - nz);      // always feasible
       while (lo < hi) {
         const int mid = (lo + hi) >> 1;
         const int tot = akv_wave_sum((c + mid - 1) / mid);
         if (tot <= G) hi = mid; else lo = mid + 1;
       }
+      if ((lo + shares - 1) / shares <= (equal + shares - 1) / shares + 1) aligned = 1;
+    }
+    if (aligned) {
       const int k = (c + lo - 1) / lo;
       const int kinc = akv_wave_inclusive_scan(k);
       p_wfirst[lane] = kinc - k;

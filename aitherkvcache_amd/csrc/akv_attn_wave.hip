@@ -1,10 +1,11 @@
 // MFMA paged decode attention in which every wavefront works on its own: 4- and 2-bit caches at head_dim 64 and 256,
-// and at head_dim 128 where few kv heads are at hand, block_size 16 or 32.
+// and at head_dim 128 with one or two kv heads (akv_attn_wave_applicable), block_size 16 or 32.
 //
 // A workgroup owns a range of the global block axis (akv_attn_partition).  Its W wavefronts are laid out as
 // (kv head slot) x (R shares of the tokens): wavefront (hs, r) takes chunks r, r + R, ... of 32 tokens of a segment for
 // kv head hs, scores AND values, with no barrier until the segment ends; then the R partial results of a head are
-// merged through LDS.  With at least W kv heads R is 1 and nothing is merged.  (The kernel in akv_attn_mfma.hip splits
+// merged through LDS.  The slots are a power of two: from W / 2 + 1 kv heads on R is 1 and nothing is merged, and where only one
+// share of a segment has tokens neither.  (The kernel in akv_attn_mfma.hip splits
 // scores and values between the wavefronts of a fixed set of eight kv heads: one kv head -- a rank of a sharded
 // model -- leaves seven eighths of it idle.)
 //
@@ -85,7 +86,7 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_attn_wave_prologu
     const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const float* __restrict__ PiT, int S, int QH, int KVH,
     const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix, uint2* __restrict__ qop,
     float* __restrict__ fac, uint32_t* __restrict__ status, float qscale, int bits, int32_t* __restrict__ wgdesc,
-    int32_t* __restrict__ seqw, int G) {
+    int32_t* __restrict__ seqw, int G, int shares) {
   constexpr int K = AW_PRO_K(D), SHARES = D / K;
   __shared__ __align__(16) float q_lds[2][D];          // [parity of the head]
   __shared__ float sum_lds[SHARES][D];
@@ -94,7 +95,7 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_attn_wave_prologu
   const int tid = threadIdx.x;
   if (blockIdx.x == 0) {
     if (tid == 0) status[0] = 0u;
-    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq);
+    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares);
     return;
   }
   const int t = tid % D, share = tid / D, gqa = QH / KVH;
@@ -146,6 +147,100 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_attn_wave_prologu
   }
 }
 
+// The same at head_dim 128, where the prepared rotation holds the matrix as an operand of the matrix cores (entries x 64: see
+// akv_attn_common.h): a workgroup takes 16 rows, the eight of two items (sequence, kv head) each, rows past the group's heads
+// zero.  200 sequences of eight query heads: 8.6 us with the kernel above, whose workgroups read the 64 KB matrix for one or two
+// rows each, 6.6 here; for few rows that one is shorter (16 sequences: 4.1 against 6.6).
+template <int QDT>
+__global__ __launch_bounds__(256) void akv_attn_wave_prologue128_kernel(
+    const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const uint4* __restrict__ bop, int S, int QH, int KVH,
+    const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix, uint2* __restrict__ qop,
+    float* __restrict__ fac, uint32_t* __restrict__ status, float qscale, int bits, int32_t* __restrict__ wgdesc,
+    int32_t* __restrict__ seqw, int G, int shares) {
+  __shared__ __align__(16) float q_lds[16][132];
+  __shared__ __align__(16) float y_lds[16][132];
+  __shared__ int32_t scratch[257];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (blockIdx.x == 0) {
+    if (tid == 0) status[0] = 0u;
+    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares);
+    return;
+  }
+  // wavefront w owns the operand's N-tiles 2 w and 2 w + 1: lane (col, g) = output coordinate 8 col + N-tile
+  const int col = lane & 15, g = lane >> 4, gqa = QH / KVH, nq = S * KVH;
+  akv_half8 bh[2][4], bl[2][4];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const int idx = ((2 * wave + t) * 4 + ks) * 64 + lane;
+      bh[t][ks] = akv_as_half8(bop[idx]);
+      bl[t][ks] = akv_as_half8(bop[2048 + idx]);
+    }
+  for (int pair = (int)blockIdx.x - 1; 2 * pair < nq; pair += (int)gridDim.x - 1) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = 2 * i + (tid >> 7), j = tid & 127, item = 2 * pair + (row >> 3), q = row & 7;
+      const int s = item / KVH, h = item % KVH;
+      q_lds[row][j] = item < nq && q < gqa ? akv_elem<QDT>::load(query, s * qs_seq + (h * gqa + q) * qs_head + j) : 0.f;
+    }
+    __syncthreads();
+    float v[4][8];
+    float m = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const float4 x0 = *(const float4*)&q_lds[col][32 * g + 8 * ks], x1 = *(const float4*)&q_lds[col][32 * g + 8 * ks + 4];
+      v[ks][0] = x0.x; v[ks][1] = x0.y; v[ks][2] = x0.z; v[ks][3] = x0.w;
+      v[ks][4] = x1.x; v[ks][5] = x1.y; v[ks][6] = x1.z; v[ks][7] = x1.w;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(v[ks][e]));
+    }
+    const uint32_t ex = akv_row_exponent(akv_rows_max(m));
+    const float sc = akv_row_scale(ex), usc = akv_row_unscale(ex) * (1.f / 64.f);      // of row `col`
+    akv_float4v acc[2];
+    acc[0] = (akv_float4v){0.f, 0.f, 0.f, 0.f};
+    acc[1] = (akv_float4v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      akv_half8 hi, lo;
+      akv_split8(v[ks], sc, hi, lo);
+      acc[0] = akv_mfma3(hi, lo, bh[0][ks], bl[0][ks], acc[0]);
+      acc[1] = akv_mfma3(hi, lo, bh[1][ks], bl[1][ks], acc[1]);
+    }
+    // lane (col, g) holds rows 4 g + i at coordinates 8 col + 2 wave and + 1
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float u = __shfl(usc, 4 * g + i);
+      *(float2*)&y_lds[4 * g + i][8 * col + 2 * wave] = make_float2(acc[0][i] * u, acc[1][i] * u);
+    }
+    __syncthreads();
+    // wavefront w writes rows 4 w .. 4 w + 3: lane l % 32 = quarter and step, four coordinates; lanes 0..31 the rounding,
+    // 32..63 the remainder (2-bit codes are looked up as (0, 2) and (1, 3))
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 4 * wave + i, item = 2 * pair + (row >> 3), q = row & 7;
+      const float4 y = *(const float4*)&y_lds[row][4 * (lane & 31)];
+      const float mx = akv_wave_max(fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
+      const uint32_t ey = akv_row_exponent(mx);
+      const float s1 = akv_row_scale(ey);
+      float c[4] = {y.x * s1, y.y * s1, y.z * s1, y.w * s1};
+      if (bits == 2) { const float t = c[1]; c[1] = c[2]; c[2] = t; }
+      uint32_t w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const __half hi = __float2half_rn(c[e]);
+        w[e] = __half_as_ushort(lane < 32 ? hi : __float2half_rn(c[e] - __half2float(hi)));
+      }
+      if (item < nq) {
+        qop[(size_t)item * (8 * 64) + (lane & 7) * 64 + 16 * ((lane >> 3) & 3) + (lane >> 5) * 8 + q] = make_uint2(w[0] | (w[1] << 16), w[2] | (w[3] << 16));
+        if (lane == 0 && q < gqa) fac[(size_t)(item / KVH) * QH + (item % KVH) * gqa + q] = akv_row_unscale(ey) * qscale;
+      }
+    }
+    // (the next rows are written behind this loop's first barrier's readers: q_lds is read before the second barrier, and
+    // y_lds is written behind the next first one)
+  }
+}
+
 // ----------------------------------------------------------------------------------
 // main kernel
 // ----------------------------------------------------------------------------------
@@ -179,6 +274,9 @@ __device__ __forceinline__ void aw_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// workgroup barrier that orders LDS traffic only (what has been requested from memory keeps flying)
+__device__ __forceinline__ void aw_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // the words whose bytes are table indices of lane coordinates: pairs (ta, tb) of tokens, words `wa`, `wb` of codes
 template <int BITS, int N> struct aw_pairs { uint32_t w[BITS == 4 ? 2 : 4]; };
 template <int BITS, int N>
@@ -205,30 +303,44 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
   const int col = lane & 15, g = lane >> 4;
   const uint32_t copy = (uint32_t)(lane & 31) * 8u;
 
-  // (requested before the table is built, not behind its barrier)
-  const int held = akv_prefix_hold(a.prefix, a.S);
+  // (one argument of every cache line, requested together: left to the compiler the lines are fetched one after another, each
+  // where the first of its arguments is needed)
+  asm volatile("" ::"s"(a.kp), "s"(a.vp), "s"(a.block_tables), "s"(a.num_blocks), "s"(x.wgdesc));
   const int32_t* rec = x.wgdesc + (size_t)blockIdx.x * AKV_WGREC;
   const int g0 = rec[AKV_WGREC_G0], g1 = rec[AKV_WGREC_G1], s_first = rec[AKV_WGREC_SEQ];
+  const int sb0_first = rec[AKV_WGREC_SB0], sb1_first = rec[AKV_WGREC_SB1], ctx_first = rec[AKV_WGREC_CTX];
 
-  // ---- table; the scale brings the largest level to [2^9, 2^10)
-  float inv_cs = 0.f;
-  if (g0 < g1) {
-    float mx = 0.f;
-    for (int v = 0; v < (1 << BITS); ++v) mx = fmaxf(mx, fabsf(a.centroids[v]));
-    const uint32_t ex = min(max((__float_as_uint(mx) >> 23) & 0xffu, 12u), 250u);
-    const float cs = __uint_as_float((254u - ex) << 23) * 512.f;
-    inv_cs = __uint_as_float(ex << 23) * (1.f / 512.f);
-    constexpr int TPE = W * 64 / 256;                      // threads of an entry
-    const int e = threadIdx.x / TPE, part = threadIdx.x % TPE;
-    const float c0 = a.centroids[(e >> 4) & ((1 << BITS) - 1)] * cs, c1 = a.centroids[e & ((1 << BITS) - 1)] * cs;
+  // ---- table; the scale brings the largest level to [2^9, 2^10).  At head_dim 128 it is written once every wavefront has
+  // requested its first block ids, rows and queries, so that the fill and the barrier behind it run beside those trips to
+  // memory; at 64 and 256 there are no registers left to hold its words until then (they would be spilled).
+  constexpr int TPE = W * 64 / 256;                        // threads of an entry
+  const float r0 = a.centroids[(threadIdx.x / TPE >> 4) & ((1 << BITS) - 1)], r1 = a.centroids[threadIdx.x / TPE & ((1 << BITS) - 1)];
+  // block prefix of the batch, lane i: entry i * pstep, the first step of the search for a segment's sequence
+  const int pstep = a.S <= 63 ? 1 : (a.S + 64) / 64;
+  int pwin = a.prefix[min(lane * pstep, a.S)], pwin0 = pstep == 1 ? 0 : -1;
+  float mx_c = 0.f;
+  for (int v = 0; v < (1 << BITS); ++v) mx_c = fmaxf(mx_c, fabsf(a.centroids[v]));
+  asm volatile("" : "+v"(mx_c) : "s"(g0), "s"(sb0_first));      // (the record and the codebook in one wait)
+  if (g0 >= g1) return;
+  const uint32_t ex_c = min(max((__float_as_uint(mx_c) >> 23) & 0xffu, 12u), 250u);
+  const float inv_cs = __uint_as_float(ex_c << 23) * (1.f / 512.f);
+  bool filled = false;
+  auto fill_once = [&]() {
+    if (filled) return;
+    filled = true;
+    const float cs = __uint_as_float((254u - ex_c) << 23) * 512.f;
+    const float c0 = r0 * cs, c1 = r1 * cs;
     const __half h0 = __float2half_rn(c0), h1 = __float2half_rn(c1);
     const __half l0 = __float2half_rn(c0 - __half2float(h0)), l1 = __float2half_rn(c1 - __half2float(h1));
     const uint32_t hi = (uint32_t)__half_as_ushort(h0) | ((uint32_t)__half_as_ushort(h1) << 16);
     const uint32_t lo = (uint32_t)__half_as_ushort(l0) | ((uint32_t)__half_as_ushort(l1) << 16);
+    // (each thread starts a piece further than its neighbour: all in step they would write to the same banks, 2,500 cycles)
+    const uint32_t e = threadIdx.x / TPE, at = e * 256u + threadIdx.x % TPE * (256u / TPE);
 #pragma unroll
-    for (int i = 0; i < 16 / TPE; ++i) *(aw_lds_u128*)(uintptr_t)(uint32_t)(e * 256 + (part * (16 / TPE) + i) * 16) = (aw_u32x4){hi, lo, hi, lo};
-  }
-  __syncthreads();
+    for (uint32_t i = 0; i < 16 / TPE; ++i) *(aw_lds_u128*)(uintptr_t)(at + (i + e) % (16u / TPE) * 16u) = (aw_u32x4){hi, lo, hi, lo};
+    aw_lds_barrier();
+  };
+  if constexpr (D != 128) fill_once();
 
   const bool bs32 = a.block_size == 32;
   const int bs = bs32 ? 32 : 16;
@@ -244,11 +356,28 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
     int64_t ctx;
     if (gcur == g0 && s_first >= 0) {
       s = s_first;
-      sb0 = rec[AKV_WGREC_SB0];
-      sb1 = rec[AKV_WGREC_SB1];
-      ctx = rec[AKV_WGREC_CTX];
+      sb0 = sb0_first;
+      sb1 = sb1_first;
+      ctx = ctx_first;
     } else {
-      s = akv_find_seq_held(a.prefix, a.S, held, gcur, sb0, sb1);
+      // the last s with prefix[s] <= gcur (below prefix[S]).  From 64 sequences on pwin first says in which stretch, then holds
+      // the 64 entries from pwin0 on, which mostly serve the next segments too.  (A binary search was eight dependent loads for
+      // 200 sequences, again in every segment.)
+      int below = __popcll(__ballot(pwin <= gcur));
+      if (pwin0 < 0) {
+        pwin0 = (below - 1) * pstep;
+        below = 64;
+      } else if (below == 64) {
+        pwin0 += 63;
+      }
+      while (below == 64) {
+        pwin = a.prefix[min(pwin0 + lane, a.S)];
+        below = __popcll(__ballot(pwin <= gcur));
+        if (below == 64) pwin0 += 63;
+      }
+      s = pwin0 + below - 1;
+      sb0 = __builtin_amdgcn_readlane(pwin, below - 1);
+      sb1 = __builtin_amdgcn_readlane(pwin, below);
       ctx = akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq);
     }
     const int blk_lo = gcur - sb0;
@@ -346,6 +475,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           for (int st = 0; st < KS; ++st) qd[st] = qp[st * 64];
         }
         const float fac = x.fac[(size_t)s * a.QH + h * gqa + min(col & 7, gqa - 1)] * inv_cs;
+        fill_once();
 
         for (int k = 0; k < mine; ++k) {
           const int c = r + k * R;
@@ -495,22 +625,38 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           __builtin_amdgcn_sched_barrier(0);
         }
         l_run = aw_rows_sum(l_run);
+      } else {
+        fill_once();
       }
 
       // ---- partial result: lane (col < gqa, g) holds coordinates CPL (4 g + i) + n of query head col
       const size_t slot = (size_t)(blockIdx.x + s) * a.QH + h * gqa;
       float M = m_run, wgt = inv_cs, L = l_run;
-      if (R > 1) {
+      const int shares = min(R, nchunks);      // wavefronts of the head that hold a result
+      if (shares > 1) {
         if (lane < 8) *(aw_lds_f64*)(uintptr_t)(aw_ml_off<W>() + (uint32_t)wave * 64u + (uint32_t)lane * 8u) = (aw_float2){m_run, l_run};
-        __syncthreads();
+        aw_lds_barrier();
+        // (AT requested at a time, at 128 and 256 all there can be; past the last share that one again, for nothing)
+        constexpr int AT = D == 64 ? 4 : W;
+        const int rounds = D == 64 ? shares : 1;
+        auto of_share = [&](int rr) { return *(aw_lds_f64*)(uintptr_t)(aw_ml_off<W>() + (uint32_t)(min(rr, shares - 1) * hp + hs) * 64u + (uint32_t)(col & 7) * 8u); };
         L = 0.f;
-        for (int rr = 0; rr < R; ++rr) {
-          const aw_float2 ml = *(aw_lds_f64*)(uintptr_t)(aw_ml_off<W>() + (uint32_t)(rr * hp + hs) * 64u + (uint32_t)(col & 7) * 8u);
-          M = fmaxf(M, ml.x);
+        for (int r0 = 0; r0 < rounds; r0 += AT) {
+          aw_float2 ml[AT];
+#pragma unroll
+          for (int i = 0; i < AT; ++i) ml[i] = of_share(r0 + i);
+#pragma unroll
+          for (int i = 0; i < AT; ++i) M = fmaxf(M, ml[i].x);
         }
-        for (int rr = 0; rr < R; ++rr) {
-          const aw_float2 ml = *(aw_lds_f64*)(uintptr_t)(aw_ml_off<W>() + (uint32_t)(rr * hp + hs) * 64u + (uint32_t)(col & 7) * 8u);
-          L += ml.x > -INFINITY ? __builtin_amdgcn_exp2f(ml.x - M) * ml.y : ml.y;      // (-inf: no token, or sums that are NaN)
+        for (int r0 = 0; r0 < rounds; r0 += AT) {
+          aw_float2 ml[AT];
+#pragma unroll
+          for (int i = 0; i < AT; ++i) ml[i] = of_share(r0 + i);
+#pragma unroll
+          for (int i = 0; i < AT; ++i) {
+            const float part = ml[i].x > -INFINITY ? __builtin_amdgcn_exp2f(ml[i].x - M) * ml[i].y : ml[i].y;      // (-inf: no token, or sums that are NaN)
+            L += r0 + i < shares ? part : 0.f;
+          }
         }
         wgt = m_run > -INFINITY ? __builtin_amdgcn_exp2f(m_run - M) * inv_cs : inv_cs;
       }
@@ -518,8 +664,8 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
       for (int n = 0; n < CPL; ++n)
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[n][i] = aw_add_cols(o[n][i]) * wgt;
-      if (R == 1) {
-        if (active && col < gqa) {
+      if (shares <= 1) {
+        if (active && r == 0 && col < gqa) {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -528,7 +674,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
         }
       } else {
         const uint32_t wave_bytes = (uint32_t)gqa * D * 4u;
-        if (active && col < gqa) {
+        if (active && r < shares && col < gqa) {
           const uint32_t at = aw_acc_off<W>() + (uint32_t)wave * wave_bytes + (uint32_t)(col * D + CPL * 4 * g) * 4u;
 #pragma unroll
           for (int i = 0; i < 4; ++i)
@@ -536,12 +682,13 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
             for (int n = 0; n < CPL; n += 4)
               *(aw_lds_f128*)(uintptr_t)(at + (uint32_t)(CPL * i + n) * 4u) = (aw_float4){o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]};
         }
-        __syncthreads();
+        aw_lds_barrier();
         if (active) {
           // (no barrier after these reads: the next segment's accumulators are written behind its first barrier)
           for (int idx = r * 64 + lane; idx < gqa * D / 4; idx += R * 64) {
             aw_float4 sum = {0.f, 0.f, 0.f, 0.f};
-            for (int rr = 0; rr < R; ++rr) sum += *(aw_lds_f128*)(uintptr_t)(aw_acc_off<W>() + (uint32_t)(rr * hp + hs) * wave_bytes + (uint32_t)idx * 16u);
+#pragma unroll 4
+            for (int rr = 0; rr < shares; ++rr) sum += *(aw_lds_f128*)(uintptr_t)(aw_acc_off<W>() + (uint32_t)(rr * hp + hs) * wave_bytes + (uint32_t)idx * 16u);
             *(float4*)(a.part_acc + slot * D + 4 * (size_t)idx) = make_float4(sum.x, sum.y, sum.z, sum.w);
           }
         }
@@ -561,23 +708,35 @@ bool akv_attn_mfma_takes(const akv_attn_args& a, int bits);       // the conditi
 int akv_attn_mfma_head_groups(int gqa);
 
 // At head_dim 128 the kernel of akv_attn_mfma.hip has eight head slots, most of them idle where a rank keeps one or two (groups
-// of) kv heads; it starts some 5 us sooner.  Measured, main kernels, this against that one: one head, 418k tokens 31 against
-// 43 us, 2.7k tokens 11 against 6; two heads, 583k tokens 12 % faster as a step, 366k tokens 44 against 46 us and a prologue
-// 4 us longer; four heads, 36k tokens 21 against 17.  The host knows the width of the tables, not the contexts.
-#define AW_FEW_TOKENS 262144
+// of) kv heads.  The rule takes nothing that the width of the tables changes: a serving engine's are as wide as its longest
+// context may become, whatever the contexts are.  Measured, prologue, main kernel and reduce in a graph (us, this | that), eight
+// query heads a group:
+//   one group     1 context of 700 14.7 | 14.7, of 2,700 19.7 | 20.0; 16 of 170 14.9 | 15.4; 48 of 700 17.7 | 20.1,
+//                 of 8,192 30.1 | 48.9; 64 of 100 15.9 | 18.6; 200 of 300 25.6 | 25.8; 256 of 1,000 29.5 | 39.3
+//                 (slower only near 100 of 300: 23.0 | 21.8)
+//   two groups    1 of 700 15.0 | 15.5; 32 of 700 18.5 | 18.4; 48 of 8,192 43.1 | 51.7; 64 of 100 18.0 | 20.4, of 700
+//                 21.8 | 20.8, of 3,000 32.2 | 33.0; but 200 of 300 33.0 | 31.6
+// Two groups lose once sequences no longer get whole workgroups (more than 64: akv_attn_partition): four wavefronts then merge
+// a few chunks at every change of the sequence.
 bool akv_attn_wave_applicable(const akv_attn_args& a, int d, int bits) {
   if (!(d == 64 || d == 128 || d == 256) || (bits != 4 && bits != 2) || !akv_attn_mfma_takes(a, bits)) return false;
   if (d != 128) return true;
   const int heads = a.KVH * akv_attn_mfma_head_groups(a.QH / a.KVH);
-  return heads <= 2 && (int64_t)a.S * a.max_blocks_per_seq * a.block_size >= (int64_t)heads * AW_FEW_TOKENS;
+  return heads == 1 || (heads == 2 && a.S <= 64);
+}
+
+// kv head slots of a workgroup of w wavefronts
+static int aw_slots(int kv_heads, int w) {
+  int hp = 1;
+  while (hp < kv_heads && hp < w) hp *= 2;
+  return hp;
 }
 
 template <int D, int BITS>
 static int aw_launch(const akv_attn_args& a, const aw_extra& x_in, int grid, hipStream_t stream) {
   constexpr int W = aw_cfg<D, BITS>::W;
   aw_extra x = x_in;
-  x.hp = 1;
-  while (x.hp < a.KVH && x.hp < W) x.hp *= 2;
+  x.hp = aw_slots(a.KVH, W);
   const int gqa = a.QH / a.KVH;
   constexpr int most = (int)aw_acc_off<W>() + W * 8 * D * 4;
   static_assert(most <= 160 * 1024, "LDS of a CU");
@@ -603,15 +762,28 @@ int akv_attn_wave_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs
   x.wgdesc = ws.wgdesc;
   x.hp = 0;
   const float qscale = a.scale * 1.4426950408889634f;   // scores come out in the log2 domain
+  const int slots = aw_slots(a.KVH, d == 64 ? 16 : 8), shares = (d == 64 ? 16 : 8) / slots;
   // rotation blocks: one per query head, up to what the CUs hold at once (then they loop: the matrix is read once per block)
   const int cus = akv_cached_cu_count();
   auto pgrid = [&](int dd) {
     const int64_t most = (int64_t)(cus > 0 ? cus : 256) * (dd == 256 ? 1 : 4) / (dd == 256 ? 2 : 1), items = (int64_t)a.S * a.QH;
     return (int)(items < most ? items : most) + 1;
   };
-#define AW_PRO(DD, DT) akv_attn_wave_prologue_kernel<DD, DT><<<pgrid(DD), aw_pro_threads<DD>(), 0, stream>>>(query, qs_seq, qs_head, PiT, a.S, a.QH, a.KVH, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint2*)extra_ws, ws.qrot, ws.status, qscale, bits, ws.wgdesc, ws.seqw, grid)
+#define AW_PRO(DD, DT) akv_attn_wave_prologue_kernel<DD, DT><<<pgrid(DD), aw_pro_threads<DD>(), 0, stream>>>(query, qs_seq, qs_head, PiT, a.S, a.QH, a.KVH, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint2*)extra_ws, ws.qrot, ws.status, qscale, bits, ws.wgdesc, ws.seqw, grid, shares)
 #define AW_PRO_D(DD) do { if (q_dtype == AKV_F16) AW_PRO(DD, AKV_F16); else if (q_dtype == AKV_BF16) AW_PRO(DD, AKV_BF16); else AW_PRO(DD, AKV_F32); } while (0)
-  if (d == 64) AW_PRO_D(64); else if (d == 128) AW_PRO_D(128); else AW_PRO_D(256);
+  // (16 rows a workgroup; its registers admit three on a CU)
+  const int64_t pairs = ((int64_t)a.S * a.KVH + 1) / 2, most128 = (int64_t)(cus > 0 ? cus : 256) * 3;
+  const int grid128 = (int)(pairs < most128 ? pairs : most128) + 1;
+#define AW_PRO128(DT) akv_attn_wave_prologue128_kernel<DT><<<grid128, 256, 0, stream>>>(query, qs_seq, qs_head, (const uint4*)(PiT + 128 * 128), a.S, a.QH, a.KVH, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint2*)extra_ws, ws.qrot, ws.status, qscale, bits, ws.wgdesc, ws.seqw, grid, shares)
+  // (a row a workgroup while three on a CU hold them all: 512 rows 4.8 | 6.0 us, 1,024 rows 7.3 | 6.5)
+  const bool plain128 = (int64_t)a.S * a.QH <= most128;
+  if (d == 64) AW_PRO_D(64);
+  else if (d == 256) AW_PRO_D(256);
+  else if (plain128) AW_PRO_D(128);
+  else if (q_dtype == AKV_F16) AW_PRO128(AKV_F16);
+  else if (q_dtype == AKV_BF16) AW_PRO128(AKV_BF16);
+  else AW_PRO128(AKV_F32);
+#undef AW_PRO128
 #undef AW_PRO_D
 #undef AW_PRO
   AKV_LAUNCH_CHECK("akv_attn_wave_prologue_kernel");

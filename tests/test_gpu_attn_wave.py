@@ -1,4 +1,4 @@
-"""Paged attention kernel whose wavefronts work on their own (head_dim 64 and 256; head_dim 128 with one or two kv heads and wide tables),
+"""Paged attention kernel whose wavefronts work on their own (head_dim 64 and 256; head_dim 128 with one kv head, or two and few sequences),
 at the edges of its tiles, chunks, head slots and block-id windows, against float64."""
 import numpy as np
 import pytest
@@ -44,15 +44,6 @@ def attend(q, K, V, R, counts=None):
     return out
 
 
-def wide(tables, d):
-    """At head_dim 128 the kernel is chosen from 262,144 tokens per kv head on, counted by the width of the tables."""
-    if d != 128:
-        return tables
-    out = np.full((len(tables), 2 * 262144 // 16 // len(tables) + 1), 10 ** 6, dtype=np.int32)
-    out[:, :tables.shape[1]] = tables
-    return out
-
-
 HEADS = [(8, 1, 16), (16, 2, 32), (9, 3, 16), (28, 4, 16), (24, 2, 32), (5, 5, 32), (40, 8, 16), (18, 18, 16)]
 
 
@@ -72,7 +63,7 @@ def test_edges_vs_float64(dev, d, bits, qh, kvh, bs):
     q = torch.from_numpy(rng.standard_normal((len(ctx), qh, d)).astype(np.float32)).to(dev)
     P = tq._packed_dim
     print(f"[attn wave] d={d} bits={bits} qh={qh} kvh={kvh} bs={bs}", flush=True)
-    out = akv.TQPagedAttention(tq, qh).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.from_numpy(wide(tables, d)).to(dev),
+    out = akv.TQPagedAttention(tq, qh).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.from_numpy(tables).to(dev),
                                                torch.from_numpy(ctx).to(dev), block_size=bs).double().cpu()
     K, V = (dequantised(tq, r, n, d, bits) for r, n in zip(rows, norms))
     R = tq.rotation.double().cpu()
@@ -120,8 +111,57 @@ def test_norms_and_queries_far_outside_float16(dev, d, bits, scale_v, scale_q):
     norms[1].view(-1, 2)[n:] = float("nan")
     q = torch.from_numpy(rng.standard_normal((1, 8, d)).astype(np.float32)).to(dev) * scale_q
     P = tq._packed_dim
-    out = akv.TQPagedAttention(tq, 8).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.from_numpy(wide(np.arange(8, dtype=np.int32)[None], d)).to(dev),
+    out = akv.TQPagedAttention(tq, 8).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.arange(8, dtype=torch.int32, device=dev)[None],
                                               torch.tensor([n], dtype=torch.int32, device=dev), block_size=16).double().cpu()
     K, V = (dequantised(tq, r, x, d, bits).reshape(-1, 2, d)[:n] for r, x in zip(rows, norms))
     ref = attend(q[0].double().cpu(), K, V, tq.rotation.double().cpu())
     assert (out[0] - ref).norm() <= REL * ref.norm()
+
+
+@pytest.mark.parametrize("d,bits,qh,kvh,bs", [(64, 4, 16, 2, 16), (256, 4, 8, 4, 16), (256, 2, 4, 1, 32), (128, 4, 8, 1, 16), (128, 2, 5, 1, 32)])
+@pytest.mark.parametrize("seqs", [63, 64, 65, 127, 300, 4300])
+def test_many_sequences(dev, d, bits, qh, kvh, bs, seqs):
+    """The axis cut into equal ranges, sequences searched in the prefix by one step (up to 63), two, and more (from 4,033 on),
+    runs of empty ones among them; 64-bit tables and lengths, bfloat16 queries of strided heads."""
+    ctx = np.random.default_rng(seqs).integers(0, 90, size=seqs)
+    ctx[seqs // 3:seqs // 3 + seqs // 6] = 0
+    ctx[0], ctx[-1] = 33, 0
+    need = -(-ctx // bs)
+    rng, tq, rows, norms = make(dev, d, bits, kvh, 40, bs, seqs + d)
+    tables = np.full((seqs, int(need.max())), -1, dtype=np.int64)
+    for i, n in enumerate(need):
+        tables[i, :n] = rng.integers(0, 40, size=n)
+    q = torch.from_numpy(rng.standard_normal((seqs, 2 * qh, d)).astype(np.float32)).to(dev).bfloat16()[:, ::2]
+    P = tq._packed_dim
+    print(f"[attn wave] many sequences: d={d} bits={bits} qh={qh} kvh={kvh} bs={bs} seqs={seqs}", flush=True)
+    out = akv.TQPagedAttention(tq, qh).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.from_numpy(tables).to(dev),
+                                               torch.from_numpy(ctx).to(dev), block_size=bs).double().cpu()
+    K, V = (dequantised(tq, r, n, d, bits) for r, n in zip(rows, norms))
+    R = tq.rotation.double().cpu()
+    qc = q.double().cpu()
+    for i in range(0, seqs, max(1, seqs // 100)):
+        n = int(ctx[i])
+        if n == 0:
+            assert not out[i].any(), i
+            continue
+        t = torch.from_numpy(tables[i, :need[i]])
+        k, v = (x[t].reshape(-1, kvh, d)[:n] for x in (K, V))
+        ref = attend(qc[i], k, v, R)
+        assert (out[i] - ref).norm() <= 2.0 ** -8 * ref.norm(), (i, n)      # (bfloat16 outputs: half a unit in the last place each)
+
+
+@pytest.mark.parametrize("qh,kvh,seqs", [(8, 1, 1), (8, 1, 16), (4, 1, 70), (16, 2, 3), (16, 1, 32), (16, 2, 40), (32, 8, 4)])
+@pytest.mark.parametrize("bits", [4, 3, 2])
+def test_padding_of_the_tables_changes_nothing(dev, qh, kvh, seqs, bits):
+    """A serving engine's block tables are as wide as its longest context may become: the kernel, and every bit of the result,
+    are those of tables cut to the contexts."""
+    rng, tq, rows, norms = make(dev, 128, bits, kvh, 30, 16, seqs)
+    ctx = rng.integers(1, 400, size=seqs).astype(np.int32)
+    tables = rng.integers(0, 30, size=(seqs, 25)).astype(np.int32)
+    padded = np.zeros((seqs, 2 * 262144 // 16 // seqs + 25), dtype=np.int32)
+    padded[:, :25] = tables
+    q = torch.from_numpy(rng.standard_normal((seqs, qh, 128)).astype(np.float32)).to(dev)
+    P = tq._packed_dim
+    out = [akv.TQPagedAttention(tq, qh).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.from_numpy(t).to(dev),
+                                                torch.from_numpy(ctx).to(dev), block_size=16) for t in (tables, padded)]
+    assert torch.equal(*out)
