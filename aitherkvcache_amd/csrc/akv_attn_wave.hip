@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "akv_attn_common.h"
+#include "akv_device_once.h"
 
 typedef _Float16 aw_half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 aw_half2 __attribute__((ext_vector_type(2)));
@@ -741,11 +742,14 @@ static int aw_launch(const akv_attn_args& a, const aw_extra& x_in, int grid, hip
   constexpr int most = (int)aw_acc_off<W>() + W * 8 * D * 4;
   static_assert(most <= 160 * 1024, "LDS of a CU");
   const int lds = (int)aw_acc_off<W>() + (x.hp < W ? W * gqa * D * 4 : 0);
-  static bool configured = false;
-  if (!configured) {
+  static akv_device_once allowed;
+  int dev = -1;
+  AKV_HIP(hipGetDevice(&dev));
+  const int rc = allowed(dev, []() -> int {
     AKV_HIP(hipFuncSetAttribute((const void*)akv_attn_wave_kernel<D, BITS>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
-    configured = true;
-  }
+    return AKV_OK;
+  });
+  if (rc) return rc;
   AKV_LAUNCH_TIMED((akv_attn_wave_kernel<D, BITS>), grid, W * 64, lds, stream, a, x);
   AKV_LAUNCH_CHECK("akv_attn_wave_kernel");
   return AKV_OK;

@@ -6,6 +6,7 @@ import ctypes
 import os
 import platform
 import re
+import shutil
 import subprocess
 import sys
 
@@ -89,6 +90,40 @@ lib.akv_last_error()
 assert generation() == loaded, (loaded, generation())
 """
     subprocess.run([sys.executable, "-c", code], check=True, timeout=300, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
+def test_every_device_is_told_once(tmp_path):
+    """akv_device_once: each device of a process is told what a kernel may use, once, and again after a failure."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(_lib.__file__)), "csrc")
+    (tmp_path / "once.cpp").write_text("""
+#include "akv_device_once.h"
+#include <stdio.h>
+int main() {
+  static akv_device_once once;
+  int calls = 0, rc = 0;
+  auto tell = [&] { ++calls; return rc; };
+  const int devices[] = {0, 0, 1, 0, 1, 63, 63, 64, 64};
+  for (int d : devices) once(d, tell);
+  rc = 7;
+  const int failed = once(2, tell);
+  rc = 0;
+  once(2, tell);
+  once(2, tell);
+  printf("%d %d", calls, failed);
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-I", csrc, str(tmp_path / "once.cpp"), "-o", str(tmp_path / "once")], check=True, timeout=120)
+    out = subprocess.run([str(tmp_path / "once")], check=True, timeout=60, capture_output=True, text=True).stdout
+    assert out == "7 7"      # devices 0, 1, 63, 64 twice; device 2 twice, the first call failing
+
+
+def test_the_kernel_of_independent_wavefronts_is_allowed_its_lds_per_device():
+    """No flag of the whole process stands before the call that allows a kernel its dynamic LDS."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(_lib.__file__)), "csrc", "akv_attn_wave.hip")
+    with open(csrc) as f:
+        source = f.read()
+    assert "static bool" not in source and "akv_device_once" in source
 
 
 # ---- TurboQuant surface -------------------------------------------------------------------
