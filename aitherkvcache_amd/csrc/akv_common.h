@@ -85,11 +85,19 @@ void akv_profile_stamp(hipStream_t s, hipEvent_t begin);
 //   [d*d, 2*d*d)    Pi^T   row-major
 //   [2*d*d, ...)    d = 128 only: float16 hi/lo operand tiles of the MFMA encode kernel (64 KB),
 //                   a flag word (256 B reserved), the same for the rotations of the attention kernels (64 KB)
-//   then            d = 64, 128, 256: float16 hi/lo slices of Pi^T, the operand of the MFMA decode kernel (4 d*d bytes)
+//   then            d = 64, 128, 256: float16 hi/lo slices of Pi^T, the operand of the MFMA decode kernel (4 d*d bytes),
+//                   and an akv_prep_scale
 #define AKV_PREP_DECODE_OFFSET(d) ((size_t)2 * (d) * (d) * 4 + 65536 + 256)
 #define AKV_PREP_SLICES_OFFSET(d) ((size_t)2 * (d) * (d) * 4 + ((d) == 128 ? 2 * 65536 + 256 : 0))
+#define AKV_PREP_SCALE_OFFSET(d) (AKV_PREP_SLICES_OFFSET(d) + ((d) == 512 ? 0 : (size_t)4 * (d) * (d)))
+// Power of two the kernels that take the matrix as two float16 terms bring it into their range with: 1 for the entries of a
+// rotation; others scale it by its largest entry.
+struct akv_prep_scale {
+  float down, up;      // 2^-k, 2^k
+  int k;
+};
 static inline size_t akv_prep_floats(int d) {
-  const size_t reserved = (size_t)4 * d * d + 1024, used = AKV_PREP_SLICES_OFFSET(d) / 4 + (d == 512 ? 0 : (size_t)d * d);
+  const size_t reserved = (size_t)4 * d * d + 1024, used = (AKV_PREP_SCALE_OFFSET(d) + sizeof(akv_prep_scale) + 3) / 4;
   return reserved > used ? reserved : used;
 }
 

@@ -92,7 +92,7 @@ int akv_prepare_decode_mfma(const float* rotation, int d, void* prep, hipStream_
 __host__ __device__ constexpr int dm_coordinate(int tile, int m) {
   return 32 * (tile >> 1) + 8 * (m >> 2) + 4 * (tile & 1) + (m & 3);   // a lane's rows 4 g + i of two tiles are eight neighbours
 }
-__global__ __launch_bounds__(256) void akv_dm_slices_kernel(const float* __restrict__ Pi, int d, uint4* __restrict__ slices) {
+__global__ __launch_bounds__(256) void akv_dm_slices_kernel(const float* __restrict__ Pi, int d, const akv_prep_scale* __restrict__ scale, uint4* __restrict__ slices) {
   const int pieces = d / 32, n = d * d / 8, t = blockIdx.x * 256 + threadIdx.x;      // (tile, piece, lane)
   if (t >= n) return;
   const int lane = t & 63, h = (t >> 6) % pieces, tile = (t >> 6) / pieces;
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void akv_dm_slices_kernel(const float* __restr
   uint32_t hi[4] = {0u, 0u, 0u, 0u}, lo[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float v = Pi[(size_t)(k0 + e) * d + i] * DM_PSCALE;
+    const float v = Pi[(size_t)(k0 + e) * d + i] * scale->down * DM_PSCALE;
     const __half hh = __float2half_rn(v);
     hi[e >> 1] |= (uint32_t)__half_as_ushort(hh) << (16 * (e & 1));
     lo[e >> 1] |= (uint32_t)__half_as_ushort(__float2half_rn(v - __half2float(hh))) << (16 * (e & 1));
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void akv_dm_slices_kernel(const float* __restr
 }
 int akv_prepare_decode_slices(const float* rotation, int d, void* prep, hipStream_t stream) {
   if (!(d == 64 || d == 128 || d == 256)) return AKV_OK;
-  akv_dm_slices_kernel<<<(d * d / 8 + 255) / 256, 256, 0, stream>>>(rotation, d, (uint4*)((char*)prep + AKV_PREP_SLICES_OFFSET(d)));
+  akv_dm_slices_kernel<<<(d * d / 8 + 255) / 256, 256, 0, stream>>>(rotation, d, (const akv_prep_scale*)((char*)prep + AKV_PREP_SCALE_OFFSET(d)), (uint4*)((char*)prep + AKV_PREP_SLICES_OFFSET(d)));
   AKV_LAUNCH_CHECK("akv_dm_slices_kernel");
   return AKV_OK;
 }
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
     for (int v = 0; v <= LM; ++v) mx = fmaxf(mx, fabsf(a.table[v]));
     const uint32_t ex = min(max((__float_as_uint(mx) >> 23) & 0xffu, 12u), 250u);
     const float cs = __uint_as_float((254u - ex) << 23) * 512.f;
-    inv_cs = __uint_as_float(ex << 23) * (1.f / 512.f / DM_PSCALE);
+    inv_cs = __uint_as_float(ex << 23) * (1.f / 512.f / DM_PSCALE) * ((const akv_prep_scale*)((const char*)slices + (size_t)4 * D * D))->up;
     // the code of the even coordinate is the high nibble (packing.py:13-23) and goes to the low half of the pair
     const float c0 = r0 * cs, c1 = r1 * cs;
     const __half h0 = __float2half_rn(c0), h1 = __float2half_rn(c1);

@@ -10,7 +10,7 @@
 // the byte.  Two barriers a step, the next rows requested before the first.
 //
 // Precision: float16 rows are exact in the operand.  bfloat16 and float32 rows are scaled by the power of two that
-// brings the largest element to [2^10, 2^11): bfloat16 is then exact (down to 2^-34 of the largest element), float32 is
+// brings the largest element to [2^10, 2^11): bfloat16 is then exact (down to 2^-27 of the largest element), float32 is
 // split into two terms like the matrix (2^-23 of the element, the product of two remainders left out).  The general
 // kernel's chain of float32 sums is no closer to 64 bits.
 //
@@ -51,7 +51,7 @@ template <int XDT> __device__ __forceinline__ void ew_floats(const typename ew_p
 }
 
 template <int D, int BITS, int XDT, bool PAGED, int MT>
-__global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kernel(akv_gen_args a, const float* __restrict__ Pi) {
+__global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kernel(akv_gen_args a, const float* __restrict__ Pi, const akv_prep_scale* __restrict__ scale) {
   typedef ew_cfg<D, MT, XDT> cfg;
   typedef typename ew_piece<XDT>::type piece_t;
   constexpr int ROWS = cfg::ROWS, TPR = cfg::TPR, KS = cfg::KS, PITCH = cfg::PITCH, NA = cfg::NA, THREADS = cfg::THREADS;
@@ -88,6 +88,8 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kerne
   };
   fetch(blockIdx.x);
 
+  const float pi_scale = EW_PI_SCALE * scale->down;
+  const int pi_exp = scale->k - EW_PI_EXP;
   // ---- the wavefront's slice of Pi: lane (col, g) holds row 16 wave + col, elements 32 ks + 8 g + e
   ew_half8 Bh[KS], Bl[KS];
 #pragma unroll
@@ -97,7 +99,7 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kerne
     const float v[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float s = v[e] * EW_PI_SCALE;
+      const float s = v[e] * pi_scale;
       const _Float16 h = (_Float16)s;
       Bh[ks][e] = h;
       Bl[ks][e] = (_Float16)(s - (float)h);
@@ -131,7 +133,7 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kerne
       // a row with a NaN (its sum is NaN) or an infinity rotates to NaN everywhere; a finite row whose squares overflow
       // has norm inf and rotates to zero
       const bool bad = ss != ss || !(mx < INFINITY);
-      int put_back = -EW_PI_EXP;
+      int put_back = pi_exp;
       union { ew_half4 h; uint2 u; } hi, lo;
       if constexpr (XDT == AKV_F16) {
         hi.u = R[i];
@@ -238,11 +240,12 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kerne
 
 template <int D, int BITS, int XDT, bool PAGED, int MT>
 static int ew_launch(const akv_gen_args& a, const float* Pi, hipStream_t stream) {
+  const akv_prep_scale* scale = (const akv_prep_scale*)((const char*)Pi + AKV_PREP_SCALE_OFFSET(D));
   typedef ew_cfg<D, MT, XDT> cfg;
   const int cus = akv_cached_cu_count();
   const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n, steps = (n_total + cfg::ROWS - 1) / cfg::ROWS;
   const int64_t most = (int64_t)(cus > 0 ? cus : 256) * (D == 256 ? 1 : 4);
-  AKV_LAUNCH_TIMED((akv_encode_wide_kernel<D, BITS, XDT, PAGED, MT>), (int)(steps < most ? steps : most), cfg::THREADS, 0, stream, a, Pi);
+  AKV_LAUNCH_TIMED((akv_encode_wide_kernel<D, BITS, XDT, PAGED, MT>), (int)(steps < most ? steps : most), cfg::THREADS, 0, stream, a, Pi, scale);
   AKV_LAUNCH_CHECK("akv_encode_wide_kernel");
   return AKV_OK;
 }

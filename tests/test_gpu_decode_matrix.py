@@ -73,3 +73,15 @@ def test_listed_blocks(dev, d, bits, heads, bs, dtype):
                 one = torch.full((blocks, bs, heads, d), 7.0, dtype=dtype, device=dev)
                 decode_blocks(rows, n, one, tq, ids, 36)
                 assert torch.equal(one, o)
+
+
+@pytest.mark.parametrize("factor", [3000.0, 1e-4, 2.0 ** 100])
+@pytest.mark.parametrize("d,bits", [(64, 4), (64, 3), (128, 4), (256, 4), (256, 2)])
+def test_matrices_that_are_no_rotation(dev, d, bits, factor):
+    """An assigned matrix may have entries far outside what two float16 terms hold: it is scaled by its largest."""
+    tq = akv.TurboQuant(head_dim=d, bits=bits, device=str(dev), dtype=torch.float32)
+    tq.rotation = tq.rotation * factor
+    rng = np.random.default_rng(bits)
+    packed, norms = rng.integers(0, 256, (100, tq._packed_dim), dtype=np.uint8), rng.lognormal(0, 1, 100).astype(np.float32)
+    out = tq.decode(torch.from_numpy(packed).to(dev), torch.from_numpy(norms).to(dev))
+    check(out.cpu().numpy(), packed, norms, tq, torch.float32)

@@ -100,3 +100,21 @@ def test_rows_of_any_magnitude(dev, d, dtype, scale):
     assert np.all(codes[big] == np.searchsorted(b, 0.0))
     got = norms.double().cpu().numpy()
     assert np.array_equal(np.isinf(got), big) and np.allclose(got[~big], n32[~big], rtol=1e-6, atol=0 if scale > 1e-20 else 1e-22)
+
+
+@pytest.mark.parametrize("factor", [3000.0, 1e-4, 2.0 ** 100])
+@pytest.mark.parametrize("d,bits,dtype", [(64, 4, torch.float16), (64, 3, torch.float32), (256, 4, torch.bfloat16), (256, 2, torch.float32)])
+def test_matrices_that_are_no_rotation(dev, d, bits, dtype, factor):
+    """A matrix given with the call may have entries far outside what two float16 terms hold: it is scaled by its largest."""
+    rng = np.random.default_rng(d)
+    tq = akv.TurboQuant(head_dim=d, bits=bits, device=str(dev))
+    R, b = tq.rotation * factor, tq.boundaries_inner * factor
+    x = torch.from_numpy(kv_like(rng, (500, 2, d)).astype(np.float32)).to(dev).to(dtype)
+    packed, norms = torch.zeros(32, 16, 2, tq._packed_dim, dtype=torch.uint8, device=dev), torch.zeros(32, 16, 2, device=dev)
+    akv.fused_kv_update(x, torch.arange(500, device=dev), packed, norms, R, b, bits, 16)
+    x64 = x.double().cpu().numpy().reshape(-1, d)
+    y = x64 / np.linalg.norm(x64, axis=-1, keepdims=True) @ R.double().cpu().numpy().T
+    ref = np.searchsorted(b.double().cpu().numpy(), y)
+    got = O._UNPACK[bits](packed.cpu().numpy().reshape(-1, tq._packed_dim)[:1000], d)
+    assert np.count_nonzero(got != ref) <= max(3, ref.size * 2e-5)      # (values that lie on a boundary to within float32)
+    assert np.allclose(norms.cpu().numpy().reshape(-1)[:1000], np.linalg.norm(x64, axis=-1), rtol=1e-6)
