@@ -723,21 +723,29 @@ static int akv_decode_blocks_impl(const char* fn, akv_gen_args& a, const void* b
   if (rc) return rc;
   if (num_ids == 0 || num_blocks == 0) return AKV_OK;
   AKV_REQUIRE(a.packed && a.norms && block_ids && rot_prep && centroids && a.out, "%s: null pointer", fn);
-  a.n = num_ids * block_size * num_kv_heads;
   a.heads = num_kv_heads; a.block_size = block_size; a.max_blocks = num_blocks;
-  a.slots = block_ids; a.slot_itype = ids_itype;
+  a.slot_itype = ids_itype;
   a.mat = (const float*)rot_prep;
   a.table = centroids;
-  rc = akv_decode_mfma_try(a, true, d, bits, out_dtype, rot_prep, (hipStream_t)stream);
-  if (rc != AKV_ERR_UNSUPPORTED) return rc;
-  // shapes the matrix-core kernel does not take: tensor by tensor
-  akv_gen_args b = a;
-  b.packed2 = nullptr; b.norms2 = nullptr; b.out2 = nullptr;
-  for (int second = 0; second < (a.packed2 != nullptr ? 2 : 1); ++second) {
-    if (second) { b.packed = a.packed2; b.norms = a.norms2; b.out = a.out2; }
-    rc = a.packed2 != nullptr ? akv_decode_mfma_try(b, true, d, bits, out_dtype, rot_prep, (hipStream_t)stream) : AKV_ERR_UNSUPPORTED;
-    if (rc == AKV_ERR_UNSUPPORTED) rc = akv_decode_dispatch<true>(d, bits, out_dtype, b, stream);
-    if (rc) return rc;
+  // (the matrix-core kernel counts the rows of a launch, K's and V's, in 32 bits: a longer list, such as a table of a very long
+  // model's width, goes in pieces)
+  const int64_t per_id = (int64_t)block_size * num_kv_heads, most = per_id < ((int64_t)1 << 29) ? ((int64_t)1 << 29) / per_id : 1;
+  for (int64_t first = 0; first < num_ids; first += most) {
+    const int64_t ids = num_ids - first < most ? num_ids - first : most;
+    a.slots = (const char*)block_ids + first * (ids_itype == AKV_I64 ? 8 : 4);
+    a.n = ids * per_id;
+    rc = akv_decode_mfma_try(a, true, d, bits, out_dtype, rot_prep, (hipStream_t)stream);
+    if (rc == AKV_OK) continue;
+    if (rc != AKV_ERR_UNSUPPORTED) return rc;
+    // shapes the matrix-core kernel does not take: tensor by tensor
+    akv_gen_args b = a;
+    b.packed2 = nullptr; b.norms2 = nullptr; b.out2 = nullptr;
+    for (int second = 0; second < (a.packed2 != nullptr ? 2 : 1); ++second) {
+      if (second) { b.packed = a.packed2; b.norms = a.norms2; b.out = a.out2; }
+      rc = a.packed2 != nullptr ? akv_decode_mfma_try(b, true, d, bits, out_dtype, rot_prep, (hipStream_t)stream) : AKV_ERR_UNSUPPORTED;
+      if (rc == AKV_ERR_UNSUPPORTED) rc = akv_decode_dispatch<true>(d, bits, out_dtype, b, stream);
+      if (rc) return rc;
+    }
   }
   return AKV_OK;
 }

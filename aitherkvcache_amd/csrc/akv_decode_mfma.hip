@@ -167,8 +167,9 @@ __device__ __forceinline__ void dm_spread(const uint32_t (&w)[dm_cfg<D, BITS>::R
 // cache blocks listed in a.slots; every listed block that exists is decoded into the block of the same index of the
 // output buffer (the batch decompress of aither_kvcache/vllm/backend.py:1040-1091 without its gather / unique / scatter
 // passes).  An entry equal to the one before it is not decoded again: the padding of a block table is such a run.
-// With a.packed2 the rows of a second tensor (V) follow those of the first.
-template <int D, int BITS, int ODT, bool BLOCKS>
+// With a.packed2 the rows of a second tensor (V) follow those of the first.  WIDE: strides of a block beyond 32 bits or inside a
+// block beyond 24 (a cache whose heads or blocks lie further apart than its rows), all offsets in 64.
+template <int D, int BITS, int ODT, bool BLOCKS, bool WIDE>
 __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_args a, const uint4* __restrict__ slices) {
   typedef dm_cfg<D, BITS> cfg;
   constexpr int C = cfg::C, CW = cfg::CW, RG = cfg::RG, NT = cfg::NT, KS = cfg::KS, RAW = cfg::RAW;
@@ -220,9 +221,15 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
         live = live && (wide ? id[mt][1] == 0u : (int32_t)id[mt][0] >= 0) && id[mt][0] < most_blocks;
         live = live && (first || id[mt][0] != before[mt][0] || id[mt][1] != before[mt][1]);
         const uint32_t blk = live ? id[mt][0] : 0u;                 // (a row of block 0 is read and dropped)
-        po = (uint64_t)blk * (uint32_t)a.ps0 + (__umul24(pos, (uint32_t)a.ps1) + __umul24(head, (uint32_t)a.ps2));
-        no = (uint64_t)blk * (uint32_t)a.ns0 + (__umul24(pos, (uint32_t)a.ns1) + __umul24(head, (uint32_t)a.ns2));
-        oo = (uint64_t)blk * (uint32_t)a.os0 + (__umul24(pos, (uint32_t)a.os1) + __umul24(head, (uint32_t)a.os2));
+        if constexpr (WIDE) {
+          po = (uint64_t)blk * (uint64_t)a.ps0 + (uint64_t)pos * (uint64_t)a.ps1 + (uint64_t)head * (uint64_t)a.ps2;
+          no = (uint64_t)blk * (uint64_t)a.ns0 + (uint64_t)pos * (uint64_t)a.ns1 + (uint64_t)head * (uint64_t)a.ns2;
+          oo = (uint64_t)blk * (uint64_t)a.os0 + (uint64_t)pos * (uint64_t)a.os1 + (uint64_t)head * (uint64_t)a.os2;
+        } else {
+          po = (uint64_t)blk * (uint32_t)a.ps0 + (__umul24(pos, (uint32_t)a.ps1) + __umul24(head, (uint32_t)a.ps2));
+          no = (uint64_t)blk * (uint32_t)a.ns0 + (__umul24(pos, (uint32_t)a.ns1) + __umul24(head, (uint32_t)a.ns2));
+          oo = (uint64_t)blk * (uint32_t)a.os0 + (__umul24(pos, (uint32_t)a.os1) + __umul24(head, (uint32_t)a.os2));
+        }
       } else {
         po = (uint64_t)n * (uint32_t)a.ps0; no = n; oo = (uint64_t)n * (uint32_t)a.os0;
       }
@@ -404,19 +411,19 @@ static bool dm_disabled() {
   return off;
 }
 
-template <int D, int BITS, int ODT, bool BLOCKS>
+template <int D, int BITS, int ODT, bool BLOCKS, bool WIDE>
 static int dm_launch(const akv_gen_args& a, const uint4* slices, hipStream_t stream) {
   const int64_t n_total = BLOCKS && a.packed2 ? 2 * a.n : a.n, steps = (n_total + DM_ROWS - 1) / DM_ROWS;
   const int cus = akv_cached_cu_count() > 0 ? akv_cached_cu_count() : 256;
-  AKV_LAUNCH_TIMED((akv_decode_mfma_kernel<D, BITS, ODT, BLOCKS>), (int)(steps < cus ? steps : cus), DM_THREADS, DM_LDS_BYTES, stream, a, slices);
+  AKV_LAUNCH_TIMED((akv_decode_mfma_kernel<D, BITS, ODT, BLOCKS, WIDE>), (int)(steps < cus ? steps : cus), DM_THREADS, DM_LDS_BYTES, stream, a, slices);
   AKV_LAUNCH_CHECK("akv_decode_mfma_kernel");
   return AKV_OK;
 }
-template <int D, int BITS>
-static int dm_launch_dt(bool blocks, int out_dtype, const akv_gen_args& a, const uint4* slices, hipStream_t stream) {
-  if (out_dtype == AKV_F16) return blocks ? dm_launch<D, BITS, AKV_F16, true>(a, slices, stream) : dm_launch<D, BITS, AKV_F16, false>(a, slices, stream);
-  if (out_dtype == AKV_BF16) return blocks ? dm_launch<D, BITS, AKV_BF16, true>(a, slices, stream) : dm_launch<D, BITS, AKV_BF16, false>(a, slices, stream);
-  return blocks ? dm_launch<D, BITS, AKV_F32, true>(a, slices, stream) : dm_launch<D, BITS, AKV_F32, false>(a, slices, stream);
+template <int D, int BITS, bool BLOCKS, bool WIDE>
+static int dm_launch_dt(int out_dtype, const akv_gen_args& a, const uint4* slices, hipStream_t stream) {
+  if (out_dtype == AKV_F16) return dm_launch<D, BITS, AKV_F16, BLOCKS, WIDE>(a, slices, stream);
+  if (out_dtype == AKV_BF16) return dm_launch<D, BITS, AKV_BF16, BLOCKS, WIDE>(a, slices, stream);
+  return dm_launch<D, BITS, AKV_F32, BLOCKS, WIDE>(a, slices, stream);
 }
 
 // returns AKV_ERR_UNSUPPORTED when the fast path does not apply (the caller then uses the general kernel)
@@ -430,18 +437,29 @@ int akv_decode_mfma_try(const akv_gen_args& a, bool blocks, int d, int bits, int
   if (blocks && (((uintptr_t)a.ps1 | (uintptr_t)a.ps2) & palign || ((a.os1 | a.os2) & 7))) return AKV_ERR_UNSUPPORTED;
   // rows are counted in 32 bits, with room for two strides past the end
   if ((a.packed2 ? 2 : 1) * a.n >= ((int64_t)1 << 31) - ((int64_t)1 << 22)) return AKV_ERR_UNSUPPORTED;
-  // strides: of a block (or flat row) 32 bits, inside a block 24 bits and the sum of both products in 32
+  // strides: of a block (or flat row) 32 bits, inside a block 24 bits and the sum of both products in 32; others in 64
+  bool wide = false;
   const int64_t outer[3] = {a.ps0, blocks ? a.ns0 : 0, a.os0};
-  for (int i = 0; i < 3; ++i)
-    if (outer[i] < 0 || outer[i] >= ((int64_t)1 << 32)) return AKV_ERR_UNSUPPORTED;
+  for (int i = 0; i < 3; ++i) {
+    if (outer[i] < 0) return AKV_ERR_UNSUPPORTED;
+    wide = wide || outer[i] >= ((int64_t)1 << 32);
+  }
   if (blocks) {      // (listed blocks, at most 2^31 of them, are indexed by 32-bit words)
     const int64_t in1[3] = {a.ps1, a.ns1, a.os1}, in2[3] = {a.ps2, a.ns2, a.os2}, most = (int64_t)1 << 24;
-    if (a.block_size >= most || a.heads >= most || (int64_t)a.block_size * a.heads >= ((int64_t)1 << 31) || a.max_blocks >= ((int64_t)1 << 32)) return AKV_ERR_UNSUPPORTED;
-    for (int i = 0; i < 3; ++i)
-      if (in1[i] < 0 || in2[i] < 0 || in1[i] >= most || in2[i] >= most || a.block_size * in1[i] + a.heads * in2[i] >= ((int64_t)1 << 32)) return AKV_ERR_UNSUPPORTED;
+    if ((int64_t)a.block_size * a.heads >= ((int64_t)1 << 31) || a.max_blocks >= ((int64_t)1 << 32)) return AKV_ERR_UNSUPPORTED;
+    wide = wide || a.block_size >= most || a.heads >= most;
+    for (int i = 0; i < 3; ++i) {
+      if (in1[i] < 0 || in2[i] < 0) return AKV_ERR_UNSUPPORTED;
+      wide = wide || in1[i] >= most || in2[i] >= most || a.block_size * in1[i] + a.heads * in2[i] >= ((int64_t)1 << 32);
+    }
   }
+  if (wide && !blocks) return AKV_ERR_UNSUPPORTED;
   const uint4* slices = (const uint4*)((const char*)rot_prep + AKV_PREP_SLICES_OFFSET(d));
-#define DM_CASE(DD, BB) if (d == DD && bits == BB) return dm_launch_dt<DD, BB>(blocks, out_dtype, a, slices, stream)
+#define DM_CASE(DD, BB)                                                                        \
+  if (d == DD && bits == BB)                                                                   \
+    return !blocks ? dm_launch_dt<DD, BB, false, false>(out_dtype, a, slices, stream)          \
+           : wide  ? dm_launch_dt<DD, BB, true, true>(out_dtype, a, slices, stream)            \
+                   : dm_launch_dt<DD, BB, true, false>(out_dtype, a, slices, stream)
   DM_CASE(64, 2); DM_CASE(64, 3); DM_CASE(64, 4);
   DM_CASE(128, 2); DM_CASE(128, 3); DM_CASE(128, 4);
   DM_CASE(256, 2); DM_CASE(256, 3); DM_CASE(256, 4);

@@ -85,3 +85,55 @@ def test_matrices_that_are_no_rotation(dev, d, bits, factor):
     packed, norms = rng.integers(0, 256, (100, tq._packed_dim), dtype=np.uint8), rng.lognormal(0, 1, 100).astype(np.float32)
     out = tq.decode(torch.from_numpy(packed).to(dev), torch.from_numpy(norms).to(dev))
     check(out.cpu().numpy(), packed, norms, tq, torch.float32)
+
+
+@pytest.mark.parametrize("d,bits", [(64, 4), (128, 4), (128, 3), (256, 2)])
+@pytest.mark.parametrize("far", ["heads of the cache", "heads of the output", "positions of the norms"])
+def test_strides_beyond_24_bits(dev, d, bits, far):
+    """Heads or positions that lie further apart than 2^24 elements take the same kernel, to the same bits."""
+    tq = akv.TurboQuant(head_dim=d, bits=bits, device=str(dev), dtype=torch.float32)
+    rng = np.random.default_rng(d)
+    P, blocks, bs, heads = tq._packed_dim, 5, 4, 2
+    rows = torch.from_numpy(rng.integers(0, 256, (blocks, bs, heads, P), dtype=np.uint8)).to(dev)
+    norms = torch.from_numpy(rng.lognormal(0, 1, (blocks, bs, heads)).astype(np.float32)).to(dev)
+    ids = torch.tensor([3, 0, 0, 4, 7, -1], device=dev)
+    want = torch.zeros(blocks, bs, heads, d, device=dev)
+    decode_blocks(rows, norms, want, tq, ids, blocks)
+
+    def spread(t, dim):                       # the same values, `dim` 2^24 elements (and a few rows) apart
+        step = (1 << 24) + 64 * t.shape[-1]
+        shape = [n for i, n in enumerate(t.shape) if i != dim]
+        inner = torch.zeros(shape).stride()
+        strides = list(inner[:dim]) + [step] + list(inner[dim:])
+        out = torch.zeros(step * t.shape[dim], dtype=t.dtype, device=dev).as_strided(t.shape, strides)
+        out.copy_(t)
+        return out
+    got = torch.zeros_like(want)
+    if far == "heads of the cache":
+        rows = spread(rows, 2)
+    elif far == "heads of the output":
+        got = spread(got, 2)
+    else:
+        norms = spread(norms, 1)
+    decode_blocks(rows, norms, got, tq, ids, blocks)
+    assert torch.equal(got, want)
+
+
+def test_more_rows_than_32_bits_count(dev):
+    """A list so long that the rows of K and V pass 2^31 is decoded in pieces, by the same kernel: most of it padding."""
+    tq = akv.TurboQuant(head_dim=64, bits=4, device=str(dev), dtype=torch.float32)
+    rng = np.random.default_rng(0)
+    blocks, bs, heads = 12, 32, 8
+    rows = [torch.from_numpy(rng.integers(0, 256, (blocks, bs, heads, tq._packed_dim), dtype=np.uint8)).to(dev) for _ in range(2)]
+    norms = [torch.from_numpy(rng.lognormal(0, 1, (blocks, bs, heads)).astype(np.float32)).to(dev) for _ in range(2)]
+    short = torch.tensor([3, 1, 11, 5, 6, 2, 9], dtype=torch.int32, device=dev)
+    ids = torch.full(((1 << 22) + 10,), -1, dtype=torch.int32, device=dev)
+    piece = (1 << 29) // (bs * heads)
+    for at, i in zip((0, piece - 1, piece, piece + 1, 2 * piece, len(ids) - 2, len(ids) - 1), short.tolist()):
+        ids[at] = i
+    outs = []
+    for listed in (short, ids):
+        o = [torch.zeros(blocks, bs, heads, 64, device=dev) for _ in range(2)]
+        batch_decompress_active_blocks(*rows, *o, tq, tq._packed_dim, listed, blocks, *norms)
+        outs.append(o)
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
