@@ -137,3 +137,23 @@ def test_more_rows_than_32_bits_count(dev):
         batch_decompress_active_blocks(*rows, *o, tq, tq._packed_dim, listed, blocks, *norms)
         outs.append(o)
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("d,bits,form", [(512, 4, "head_dim"), (512, 3, "head_dim")] + [(d, b, f) for d, b in ((64, 4), (128, 3), (256, 2)) for f in ("odd rows", "odd output of V")])
+def test_keys_and_values_the_matrix_kernel_does_not_take_together(dev, d, bits, form):
+    """Equal layouts of K and V that one launch cannot take: head_dim 512, rows of an odd pitch (the vector kernel for both), an
+    output of V that lies 4 bytes off (the matrix kernel for K, the vector kernel for V)."""
+    tq = akv.TurboQuant(head_dim=d, bits=bits, device=str(dev), dtype=torch.float32)
+    rng = np.random.default_rng(d + bits)
+    P, blocks, bs, heads = tq._packed_dim, 9, 16, 3
+    pad = 1 if form == "odd rows" else 4
+    both = torch.from_numpy(rng.integers(0, 256, (2, blocks, bs, heads, P + pad), dtype=np.uint8)).to(dev)
+    norms = torch.from_numpy(rng.lognormal(0, 1, (2, blocks, bs, heads)).astype(np.float32)).to(dev)
+    off = 1 if form == "odd output of V" else 0
+    outs = [torch.full((blocks * bs * heads * d + 4,), 7.0, device=dev)[o:o + blocks * bs * heads * d].view(blocks, bs, heads, d) for o in (0, off)]
+    listed, rest = [1, 2, 7, 8], [0, 3, 4, 5, 6]
+    ids = torch.tensor([[7, 1, -1], [8, 2, 30]], device=dev)
+    batch_decompress_active_blocks(both[0], both[1], outs[0], outs[1], tq, P, ids, blocks, norms[0], norms[1])
+    for o, rows, n in zip(outs, both, norms):
+        check(o[listed].cpu().numpy(), rows[listed].cpu().numpy(), n[listed].cpu().numpy(), tq, torch.float32)
+        assert bool((o[rest] == 7.0).all())
