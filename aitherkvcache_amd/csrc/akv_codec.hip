@@ -126,16 +126,20 @@ __global__ void akv_prepare_rotation_kernel(const float* __restrict__ R, float* 
   for (int r = ty; r < 32; r += 8) RT[(size_t)(bx + r) * d + by + tx] = tile[tx][r];
 }
 
-// one workgroup: the largest entry's exponent, 0 while it is that of a rotation (or of no number)
-__global__ __launch_bounds__(256) void akv_prepare_scale_kernel(const float* __restrict__ R, int n, akv_prep_scale* __restrict__ out) {
-  __shared__ float part[4];
+// one workgroup: the largest entry's exponent, 0 while it is that of a rotation (or of no number); n a multiple of 4,096
+__global__ __launch_bounds__(1024) void akv_prepare_scale_kernel(const float4* __restrict__ R, int n, akv_prep_scale* __restrict__ out) {
+  __shared__ float part[16];
   float m = 0.f;
-  for (int i = threadIdx.x; i < n; i += 256) m = fmaxf(m, fabsf(R[i]));
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n / 4; i += 1024) {
+    const float4 v = R[i];
+    m = fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+  }
   m = akv_wave_max(m);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x != 0) return;
-  m = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+  for (int i = 0; i < 16; ++i) m = fmaxf(m, part[i]);
   int k = 0;
   if (m > 0.f && m < INFINITY && !(m >= 0x1p-7f && m < 2.f)) k = min(max(ilogbf(m) + 1, -120), 120);
   out->down = ldexpf(1.f, -k);
@@ -160,8 +164,10 @@ extern "C" int akv_rotation_prepare(const float* rotation, int d, void* prep, si
   dim3 grid(d / 32, d / 32);
   akv_prepare_rotation_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(rotation, (float*)prep, d);
   AKV_LAUNCH_CHECK("akv_prepare_rotation_kernel");
-  akv_prepare_scale_kernel<<<1, 256, 0, (hipStream_t)stream>>>(rotation, d * d, (akv_prep_scale*)((char*)prep + AKV_PREP_SCALE_OFFSET(d)));
-  AKV_LAUNCH_CHECK("akv_prepare_scale_kernel");
+  if (d != 512) {      // (no kernel of head_dim 512 takes the matrix as float16 terms)
+    akv_prepare_scale_kernel<<<1, 1024, 0, (hipStream_t)stream>>>((const float4*)prep, d * d, (akv_prep_scale*)((char*)prep + AKV_PREP_SCALE_OFFSET(d)));
+    AKV_LAUNCH_CHECK("akv_prepare_scale_kernel");
+  }
   if (d == 128) {
     int rc = akv_prepare_rotation_mfma(rotation, d, prep, (hipStream_t)stream);
     if (rc) return rc;
