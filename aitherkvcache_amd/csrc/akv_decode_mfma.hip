@@ -19,11 +19,11 @@
 // What bounds it: the loop, 48 products of 16 cycles and some 430 vector instructions of four per 16 rows of head_dim 128
 // and wavefront at two wavefronts a SIMD, and the trips to memory around it.
 // Flat rows at head_dim 128 (us; the matrix in LDS, 64 KB read per 32 rows | split from the float32 matrix in every launch |
-// as it is now): 4-bit to float16, 65,536 rows 14.2 | 16.0 | 12.4, 2^20 rows 110 | 111 | 106; 3-bit 2^20 113 | 116 | 110;
-// 4-bit to float32 2^20 156 | 181 | 124.
+// as it is now): 4-bit to float16, 4,096 rows 10.2 | 9.5 | 5.9, 65,536 rows 14.6 | 16.9 | 13.1, 2^20 rows 110 | 110 | 105; 3-bit
+// 2^20 115 | 115 | 109; 4-bit to float32 2^20 156 | 183 | 126.  2^20 rows at head_dim 64, 3 bits: 511 on the vector kernel, 35.
 // K and V of 17k tokens x 8 heads at head_dim 128: 72 to 75 us as two launches with the matrix in LDS, 42 with the slice split
-// in the launch (53 with block ids widened to 64 bits where they are loaded, a wait per load).  6,290 tokens x 8 heads at
-// head_dim 256 784 us on the vector kernel, 53; 20,936 tokens x 16 heads at head_dim 64, 3 bits, 385 and 34 us.
+// in the launch (53 with block ids widened to 64 bits where they are loaded, a wait per load), 40 as it is now.  6,290 tokens x
+// 8 heads at head_dim 256 784 us on the vector kernel, 53; 20,936 tokens x 16 heads at head_dim 64, 3 bits, 385 and 34 us.
 // No barrier after the set-up: the wavefronts of a row only share cache lines.
 #include "akv_common.h"
 #include "akv_nibble.h"
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(Ah[nt][ks]), "+v"(Al[nt][ks]));
-  for (; step < steps; step += stride) {
+  auto one_step = [&]() __attribute__((always_inline)) {
     dm_float4 acc[DM_MT][NT];
     if (!BLOCKS || __builtin_amdgcn_ballot_w64(orow[0] != nullptr || orow[DM_MT - 1] != nullptr) != 0) {
 #pragma unroll
@@ -403,7 +403,14 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
         }
       }
     }
+  };
+  // (flat: the first step stands before the loop, so that the stores of the step before are outstanding on every way into it; else
+  // the wait for a step's rows, which are older, is one for those stores too)
+  if constexpr (!BLOCKS) {
+    one_step();
+    step += stride;
   }
+  for (; step < steps; step += stride) one_step();
 }
 
 static bool dm_disabled() {
