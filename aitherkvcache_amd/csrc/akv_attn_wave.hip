@@ -5,9 +5,8 @@
 // (kv head slot) x (R shares of the tokens): wavefront (hs, r) takes chunks r, r + R, ... of 32 tokens of a segment for
 // kv head hs, scores AND values, with no barrier until the segment ends; then the R partial results of a head are
 // merged through LDS.  The slots are a power of two: from W / 2 + 1 kv heads on R is 1 and nothing is merged, and where only one
-// share of a segment has tokens neither.  (The kernel in akv_attn_mfma.hip splits
-// scores and values between the wavefronts of a fixed set of eight kv heads: one kv head -- a rank of a sharded
-// model -- leaves seven eighths of it idle.)
+// share of a segment has tokens neither.  (The kernel in akv_attn_mfma.hip splits scores and values between the wavefronts of
+// a fixed set of eight kv heads: one kv head -- a rank of a sharded model -- leaves seven eighths of it idle.)
 //
 //   scores   S^T[token, col] = sum_d Khat[token, d] Qop[d, col]         v_mfma_f32_16x16x32_f16
 //            A: lane (n = l % 16, g = l / 16) owns quarter g of token n's code row; an LDS table turns a byte (two codes)
@@ -26,8 +25,9 @@
 // One table serves keys and values: 256 entries x 8 bytes x 32 copies (a lane reads copy lane % 32: no bank conflicts).
 // 2-bit codes are looked up as nibbles: two masks and a shift spread a byte of four codes, no second table.
 //
-// What bounds it: the look-ups, 64 eight-byte LDS reads per kv head, 16 tokens and 256 coordinates, and the vector
-// instructions around them.
+// What bounds it: the chain of trips to LDS and memory a wavefront walks, at two to four wavefronts a SIMD.  No unit is full
+// (profiles/attn_wave_sq_counters.txt, share of the kernel's cycles): vector unit
+// 49, 43 and 36 % at head_dim 64, 128 and 256, matrix cores 12 to 16, LDS 19 to 24.
 #include <type_traits>
 
 #include "akv_attn_common.h"
@@ -48,7 +48,8 @@ typedef __attribute__((address_space(3))) aw_float4 aw_lds_f128;
 #define AW_FRAME 15.f          // weights stay below 2^AW_FRAME
 // Value norms count as at least 2^-AW_TINY in the running maximum: the plain exponentials, summed for the denominator, then
 // stay below 2^(AW_TINY + AW_FRAME), and a million of them in float32.  A vector of that norm still has 2^15 times the
-// smallest float16 the weights need, so only norms below some 2^-110 lose digits (a zero vector weighs nothing).
+// smallest float16 the weights need, so only norms below some 2^-110 lose digits (a zero vector weighs nothing).  The encoders
+// write none: a norm is the root of a float32 sum of squares, 0 or at least 2^-75.
 #define AW_TINY 90
 #define AW_WIN 32              // chunks of a wavefront served by one window of 64 block ids
 
@@ -417,7 +418,8 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
         const uint32_t noff = (uint32_t)(lane >= 32 ? hd * a.vns_head + npos * a.vns_pos : hd * a.kns_head + npos * a.kns_pos);
 
         // Codes and norms sit in one set of registers: the next chunk's keys are requested when this one's are scored, its
-        // values when these are weighed (a second set made the compiler spill at head_dim 256 and move registers elsewhere).
+        // values when these are weighed (a second set made the compiler spill in the loop at head_dim 256 and move registers
+        // elsewhere; as it is the 4-bit kernels of 64 and 256 keep six registers in scratch memory, outside the loop).
         uint32_t kr[2][KDW], vr[8][VDW];
         float nrm;
         auto blocks = [&](int k, uint32_t& pb0, uint32_t& pb1) {
