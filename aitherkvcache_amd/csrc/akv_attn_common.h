@@ -385,3 +385,43 @@ __device__ __forceinline__ akv_float4v akv_mfma3(akv_half8 hi, akv_half8 lo, akv
   return acc;
 }
 
+// Row shifts that write ONE bank (four neighbouring lanes) of every row of sixteen; the other lanes keep `old`.
+// akv_to_bank<K>: lane 4K + c of a row receives `src` of lane c.
+template <int K>
+__device__ __forceinline__ float akv_to_bank(float old, float src) {
+  static_assert(K >= 1 && K <= 3, "bank 0 holds its own values");
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(src), 0x110 + 4 * K /*row_shr:4K*/, 0xf, 1 << K, false));
+}
+// akv_dpp_bank<CTRL, K>: lanes of bank K receive `src` through the row operation CTRL, the others keep `old`;
+// akv_dpp_banks<CTRL, MASK>: the same for a set of banks
+template <int CTRL, int K>
+__device__ __forceinline__ float akv_dpp_bank(float old, float src) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(src), CTRL, 0xf, 1 << K, false));
+}
+template <int CTRL, int MASK>
+__device__ __forceinline__ float akv_dpp_banks(float old, float src) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(src), CTRL, 0xf, MASK, false));
+}
+template <int CTRL, int MASK>
+__device__ __forceinline__ uint32_t akv_dpp_banks_u(uint32_t old, uint32_t src) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, CTRL, 0xf, MASK, false);
+}
+// akv_pair_from_bank<Q>: lanes 0..3 of a row receive `hi` of lanes 4Q + c, lanes 8..11 receive `lo` of lanes 4Q + c,
+// every other lane zero (quad_perm 0,1,2,3 is the shift by nothing)
+template <int Q>
+__device__ __forceinline__ uint32_t akv_pair_from_bank(uint32_t hi, uint32_t lo) {
+  constexpr int hi_ctrl = Q == 0 ? 0xE4 : 0x100 + 4 * Q;                                            // row_shl:4Q
+  constexpr int lo_ctrl = Q == 2 ? 0xE4 : (Q < 2 ? 0x110 + (8 - 4 * Q) : 0x100 + (4 * Q - 8));      // row_shr:8-4Q / row_shl:4Q-8
+  int w = __builtin_amdgcn_update_dpp(0, (int)hi, hi_ctrl, 0xf, 0x1, false);
+  w = __builtin_amdgcn_update_dpp(w, (int)lo, lo_ctrl, 0xf, 0x4, false);
+  return (uint32_t)w;
+}
+// sum / maximum over the four banks of a row (every lane gets the result of the lanes c, c + 4, c + 8, c + 12)
+__device__ __forceinline__ float akv_banks_max(float v) {
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124 /*row_ror:4*/, 0xf, 0xf, false)));
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128 /*row_ror:8*/, 0xf, 0xf, false)));
+}
+__device__ __forceinline__ float akv_banks_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124 /*row_ror:4*/, 0xf, 0xf, false));
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128 /*row_ror:8*/, 0xf, 0xf, false));
+}

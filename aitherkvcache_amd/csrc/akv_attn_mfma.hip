@@ -368,47 +368,6 @@ __device__ __forceinline__ float mf_rows_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// Row shifts that write ONE bank (four neighbouring lanes) of every row of sixteen; the other lanes keep `old`.
-// mf_to_bank<K>: lane 4K + c of a row receives `src` of lane c.
-template <int K>
-__device__ __forceinline__ float mf_to_bank(float old, float src) {
-  static_assert(K >= 1 && K <= 3, "bank 0 holds its own values");
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(src), 0x110 + 4 * K /*row_shr:4K*/, 0xf, 1 << K, false));
-}
-// mf_dpp_bank<CTRL, K>: lanes of bank K receive `src` through the row operation CTRL, the others keep `old`;
-// mf_dpp_banks<CTRL, MASK>: the same for a set of banks
-template <int CTRL, int K>
-__device__ __forceinline__ float mf_dpp_bank(float old, float src) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(src), CTRL, 0xf, 1 << K, false));
-}
-template <int CTRL, int MASK>
-__device__ __forceinline__ float mf_dpp_banks(float old, float src) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(src), CTRL, 0xf, MASK, false));
-}
-template <int CTRL, int MASK>
-__device__ __forceinline__ uint32_t mf_dpp_banks_u(uint32_t old, uint32_t src) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, CTRL, 0xf, MASK, false);
-}
-// mf_pair_from_bank<Q>: lanes 0..3 of a row receive `hi` of lanes 4Q + c, lanes 8..11 receive `lo` of lanes 4Q + c,
-// every other lane zero (quad_perm 0,1,2,3 is the shift by nothing)
-template <int Q>
-__device__ __forceinline__ uint32_t mf_pair_from_bank(uint32_t hi, uint32_t lo) {
-  constexpr int hi_ctrl = Q == 0 ? 0xE4 : 0x100 + 4 * Q;                                            // row_shl:4Q
-  constexpr int lo_ctrl = Q == 2 ? 0xE4 : (Q < 2 ? 0x110 + (8 - 4 * Q) : 0x100 + (4 * Q - 8));      // row_shr:8-4Q / row_shl:4Q-8
-  int w = __builtin_amdgcn_update_dpp(0, (int)hi, hi_ctrl, 0xf, 0x1, false);
-  w = __builtin_amdgcn_update_dpp(w, (int)lo, lo_ctrl, 0xf, 0x4, false);
-  return (uint32_t)w;
-}
-// sum / maximum over the four banks of a row (every lane gets the result of the lanes c, c + 4, c + 8, c + 12)
-__device__ __forceinline__ float mf_banks_max(float v) {
-  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124 /*row_ror:4*/, 0xf, 0xf, false)));
-  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128 /*row_ror:8*/, 0xf, 0xf, false)));
-}
-__device__ __forceinline__ float mf_banks_sum(float v) {
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124 /*row_ror:4*/, 0xf, 0xf, false));
-  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128 /*row_ror:8*/, 0xf, 0xf, false));
-}
-
 // Pairwise hand-off between the score and the value wavefront of a head slot (tq35 kernel; the kernel
 // for the uniform formats orders its chunks with workgroup barriers instead): two counters in LDS,
 // `ready` (chunks whose weights are written) and `done` (chunks whose weights have been read), both
@@ -753,8 +712,8 @@ __device__ __forceinline__ void mf_role_main(const akv_attn_args& a, const akv_m
               // other lane by one row shift of eight that writes half of the row.
 #pragma unroll
               for (int jj = 0; jj < 4; ++jj) {
-                const float hi = mf_dpp_banks<0x118 /*row_shr:8*/, 0xc>(acc[0][jj], acc[1][jj]);
-                const float lo = mf_dpp_banks<0x108 /*row_shl:8*/, 0x3>(acc[1][jj], acc[0][jj]);
+                const float hi = akv_dpp_banks<0x118 /*row_shr:8*/, 0xc>(acc[0][jj], acc[1][jj]);
+                const float lo = akv_dpp_banks<0x108 /*row_shl:8*/, 0x3>(acc[1][jj], acc[0][jj]);
                 sv[jj] = hi + lo;
               }
             } else if constexpr (PACK == 4) {
@@ -768,13 +727,13 @@ __device__ __forceinline__ void mf_role_main(const akv_attn_args& a, const akv_m
 #pragma unroll
               for (int jj = 0; jj < 2; ++jj) {
                 float hi = acc[0][jj];                                              // bank 0: its own values 0, 1
-                hi = mf_dpp_bank<0x114 /*row_shr:4*/, 1>(hi, acc[0][2 + jj]);
-                hi = mf_dpp_bank<0x118 /*row_shr:8*/, 2>(hi, acc[1][jj]);
-                hi = mf_dpp_bank<0x11c /*row_shr:12*/, 3>(hi, acc[1][2 + jj]);
+                hi = akv_dpp_bank<0x114 /*row_shr:4*/, 1>(hi, acc[0][2 + jj]);
+                hi = akv_dpp_bank<0x118 /*row_shr:8*/, 2>(hi, acc[1][jj]);
+                hi = akv_dpp_bank<0x11c /*row_shr:12*/, 3>(hi, acc[1][2 + jj]);
                 float lo = acc[1][jj];                                              // bank 2: its own values 4, 5
-                lo = mf_dpp_bank<0x108 /*row_shl:8*/, 0>(lo, acc[0][jj]);
-                lo = mf_dpp_bank<0x104 /*row_shl:4*/, 1>(lo, acc[0][2 + jj]);
-                lo = mf_dpp_bank<0x114 /*row_shr:4*/, 3>(lo, acc[1][2 + jj]);
+                lo = akv_dpp_bank<0x108 /*row_shl:8*/, 0>(lo, acc[0][jj]);
+                lo = akv_dpp_bank<0x104 /*row_shl:4*/, 1>(lo, acc[0][2 + jj]);
+                lo = akv_dpp_bank<0x114 /*row_shr:4*/, 3>(lo, acc[1][2 + jj]);
                 sv[jj] = hi + lo;
               }
             }
@@ -855,8 +814,8 @@ __device__ __forceinline__ void mf_role_main(const akv_attn_args& a, const akv_m
             // operand dword qq = token pair q(qq) = pair q % 2 of tile q / 2: columns 0..7 take its hi form, columns
             // 8..15 its lo form, each from the lane of the pair's tile (its own, or the one eight lanes away)
             // (2-bit: the value side's operand takes the tokens as 4g, 4g+1 of both tiles, then 4g+2, 4g+3 of both)
-            auto tile0 = [&](int pp) { return mf_dpp_banks_u<0x118 /*row_shr:8*/, 0xc>(hb[pp], lb[pp]); };
-            auto tile1 = [&](int pp) { return mf_dpp_banks_u<0x108 /*row_shl:8*/, 0x3>(lb[pp], hb[pp]); };
+            auto tile0 = [&](int pp) { return akv_dpp_banks_u<0x118 /*row_shr:8*/, 0xc>(hb[pp], lb[pp]); };
+            auto tile1 = [&](int pp) { return akv_dpp_banks_u<0x108 /*row_shl:8*/, 0x3>(lb[pp], hb[pp]); };
             if constexpr (BITS == 2) {
               cv.w[0] = tile0(0); cv.w[1] = tile1(0); cv.w[2] = tile0(1); cv.w[3] = tile1(1);
             } else {
@@ -867,7 +826,7 @@ __device__ __forceinline__ void mf_role_main(const akv_attn_args& a, const akv_m
             // every lane of a row knows the running maximum of its head c; the sum is kept per lane (its own
             // pair's share) and added up over the banks when the segment ends
             float mx = fmaxf(tv[0], tv[1]);
-            mx = mf_rows_max(mf_banks_max(mx));
+            mx = mf_rows_max(akv_banks_max(mx));
             const float m_new = fmaxf(m_run, mx);
             const float resc = __builtin_amdgcn_exp2f(m_run - m_new);   // 0 on the first chunk
             m_run = m_new;
@@ -883,10 +842,10 @@ __device__ __forceinline__ void mf_role_main(const akv_attn_args& a, const akv_m
             // operand dword qq of a lane = token pair q(qq): columns 0..3 take the hi pair from bank q of their row,
             // columns 8..11 the lo pair; the other columns belong to no query head and hold zeros
             // (2-bit: the value side's operand takes the tokens as 4g, 4g+1 of both tiles, then 4g+2, 4g+3 of both)
-            cv.w[0] = mf_pair_from_bank<0>(hb.u, lb.u);
-            cv.w[1] = mf_pair_from_bank<BITS == 2 ? 2 : 1>(hb.u, lb.u);
-            cv.w[2] = mf_pair_from_bank<BITS == 2 ? 1 : 2>(hb.u, lb.u);
-            cv.w[3] = mf_pair_from_bank<3>(hb.u, lb.u);
+            cv.w[0] = akv_pair_from_bank<0>(hb.u, lb.u);
+            cv.w[1] = akv_pair_from_bank<BITS == 2 ? 2 : 1>(hb.u, lb.u);
+            cv.w[2] = akv_pair_from_bank<BITS == 2 ? 1 : 2>(hb.u, lb.u);
+            cv.w[3] = akv_pair_from_bank<3>(hb.u, lb.u);
             resc_out = resc;
           }
           // the buffer was last read for chunk c - 2, two barriers ago
@@ -923,7 +882,7 @@ __device__ __forceinline__ void mf_role_main(const akv_attn_args& a, const akv_m
         float lsum = l_run;
         lsum = mf_rows_sum(lsum);
         // every lane of a row summed its own share
-        if constexpr (PACK == 4) lsum = mf_banks_sum(lsum);
+        if constexpr (PACK == 4) lsum = akv_banks_sum(lsum);
         else lsum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(lsum), 0x128 /*row_ror:8*/, 0xf, 0xf, false));
         if (active && col < gqa && g == 0) {
           const size_t slot = (size_t)(blockIdx.x + s) * a.QH + (h * gqa + col);
@@ -1570,7 +1529,7 @@ __device__ __forceinline__ void hm_role_main(const akv_hyb_mfma_args& a, const i
           float ps[2];
 #pragma unroll
           for (int jj = 0; jj < 2; ++jj)
-            ps[jj] = mf_to_bank<3>(mf_to_bank<2>(mf_to_bank<1>(sv[jj], sv[2 + jj]), sv[4 + jj]), sv[6 + jj]);
+            ps[jj] = akv_to_bank<3>(akv_to_bank<2>(akv_to_bank<1>(sv[jj], sv[2 + jj]), sv[4 + jj]), sv[6 + jj]);
           // value-side factors of the lane's token pair (tile kb / 2, tokens 4g + 2 (kb % 2) + {0, 1})
           union { mf_u32x2 u; float f[2]; } vn0, vr0, vn1, vr1;
           {
@@ -1587,7 +1546,7 @@ __device__ __forceinline__ void hm_role_main(const akv_hyb_mfma_args& a, const i
             for (int jj = 0; jj < 2; ++jj)
               if (!(tile_ok && tok0 + jj < t_end)) { ps[jj] = -INFINITY; vn0.f[jj] = 0.f; vr0.f[jj] = 0.f; vn1.f[jj] = 0.f; vr1.f[jj] = 0.f; }
           }
-          const float mx = mf_rows_max(mf_banks_max(fmaxf(ps[0], ps[1])));
+          const float mx = mf_rows_max(akv_banks_max(fmaxf(ps[0], ps[1])));
           const float m_new = fmaxf(m_run, mx);
           const float resc = __builtin_amdgcn_exp2f(m_run - m_new);
           m_run = m_new;
@@ -1639,7 +1598,7 @@ __device__ __forceinline__ void hm_role_main(const akv_hyb_mfma_args& a, const i
         __builtin_amdgcn_s_waitcnt(MF_WAIT_VM0);
         T += (uint32_t)nchunks;
         float lsum = l_run;
-        lsum = mf_banks_sum(mf_rows_sum(lsum));
+        lsum = akv_banks_sum(mf_rows_sum(lsum));
         if (col < 4 && g == 0) {
           const size_t slot = (size_t)(blockIdx.x + s) * a.QH + (h * 4 + col);
           a.part_ml[slot * 2] = m_run * 0.6931471805599453f;

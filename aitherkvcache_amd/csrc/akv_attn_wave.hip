@@ -294,11 +294,13 @@ __device__ __forceinline__ void aw_pair(aw_pairs<BITS, N>& p, uint32_t wa, uint3
   }
 }
 
-template <int D, int BITS>
+// PACK: lanes of a row that share the eight tokens of a query head from the scores to the weights (below)
+template <int D, int BITS, int PACK>
 __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(akv_attn_args a, aw_extra x) {
   typedef aw_cfg<D, BITS> cfg;
   constexpr int W = cfg::W, CPL = cfg::CPL, KS = cfg::KS, KDW = cfg::KDW, VB = cfg::VB, VDW = cfg::VDW;
-  constexpr int CPB = 8 / BITS;                            // codes of a byte
+  constexpr int CPB = BITS == 2 ? 4 : 2;                   // codes of a byte
+  constexpr int NV = 8 / PACK;                             // tokens of a lane in the softmax
   // The dynamic LDS block is the kernel's only LDS object: its offsets are LDS addresses.
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -350,7 +352,8 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
   const int hp = x.hp, R = W / hp;
   const int hs = wave % hp, r = wave / hp;
   const uint32_t nbase = AW_NORM + (uint32_t)wave * AW_NORM_WAVE;
-  const uint32_t nread = nbase + (uint32_t)g * 16u;
+  const int kb = PACK == 4 ? (lane >> 2) & 3 : (lane >> 3) & 1;     // which NV of a head's eight tokens
+  const uint32_t nread = nbase + (uint32_t)g * 16u + (PACK == 4 ? 64u * (uint32_t)(kb >> 1) + 8u * (uint32_t)(kb & 1) : 64u * (uint32_t)kb);
 
   int gcur = g0;
   while (gcur < g1) {
@@ -419,7 +422,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
 
         // Codes and norms sit in one set of registers: the next chunk's keys are requested when this one's are scored, its
         // values when these are weighed (a second set made the compiler spill in the loop at head_dim 256 and move registers
-        // elsewhere; as it is the 4-bit kernels of 64 and 256 keep six registers in scratch memory, outside the loop).
+        // elsewhere).
         uint32_t kr[2][KDW], vr[8][VDW];
         float nrm;
         auto blocks = [&](int k, uint32_t& pb0, uint32_t& pb1) {
@@ -477,7 +480,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
 #pragma unroll
           for (int st = 0; st < KS; ++st) qd[st] = qp[st * 64];
         }
-        const float fac = x.fac[(size_t)s * a.QH + h * gqa + min(col & 7, gqa - 1)] * inv_cs;
+        const float fac = x.fac[(size_t)s * a.QH + h * gqa + min(col & (PACK == 4 ? 3 : 7), gqa - 1)] * inv_cs;
         fill_once();
 
         for (int k = 0; k < mine; ++k) {
@@ -522,57 +525,102 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           load_keys(min(k + 1, mine - 1));
           __builtin_amdgcn_sched_barrier(0);
 
-          // ---- running softmax in the log2 domain over t = score + exponent of the value norm
-          float sv[8], vn[8], tv[8], mx = -INFINITY;
+          // ---- running softmax in the log2 domain over t = score + exponent of the value norm, on a PACKED copy of the scores:
+          // the accumulator holds eight tokens per lane, sums of the queries' roundings in columns 0..7 and of their remainders
+          // in 8..15.  PACK = 4 (at most four query heads): lane 4 k + c of a row takes the token pair k of head c, the first
+          // term from lane c, the second from lane 8 + c; PACK = 2: lane c takes tile 0, lane 8 + c tile 1 of head c.  Every lane
+          // on all eight tokens of its column, as the accumulator lies, were 16 exponentials a lane (a quarter of the rate of
+          // other vector instructions) in place of 4 or 8.  A decode step, 32 query heads on 8 of 64, 48 sequences of 512 to 8,192
+          // tokens: 64.9 -> 60.1 us; 16 on 4 of 256, 24 sequences: 64.4 -> 63.0; 8 on 1 of 128, 48 of 1,024 to 16,384: 36.9 -> 35.9.
+          float sv[NV], vn[NV], tv[NV];
+          if constexpr (PACK == 4) {
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const aw_float4 kn4 = *(aw_lds_f128*)(uintptr_t)(nread + 64u * j);
-            const aw_float4 vn4 = *(aw_lds_f128*)(uintptr_t)(nread + 128u + 64u * j);
-            const aw_float4 ve4 = *(aw_lds_f128*)(uintptr_t)(nread + 256u + 64u * j);
+            for (int jj = 0; jj < 2; ++jj) {
+              float hi = acc[0][jj];
+              hi = akv_dpp_bank<0x114 /*row_shr:4*/, 1>(hi, acc[0][2 + jj]);
+              hi = akv_dpp_bank<0x118 /*row_shr:8*/, 2>(hi, acc[1][jj]);
+              hi = akv_dpp_bank<0x11c /*row_shr:12*/, 3>(hi, acc[1][2 + jj]);
+              float lo = acc[1][jj];
+              lo = akv_dpp_bank<0x108 /*row_shl:8*/, 0>(lo, acc[0][jj]);
+              lo = akv_dpp_bank<0x104 /*row_shl:4*/, 1>(lo, acc[0][2 + jj]);
+              lo = akv_dpp_bank<0x114 /*row_shr:4*/, 3>(lo, acc[1][2 + jj]);
+              sv[jj] = hi + lo;
+            }
+            const aw_float2 kn2 = *(aw_lds_f64*)(uintptr_t)nread, vn2 = *(aw_lds_f64*)(uintptr_t)(nread + 128u);
+            const aw_float2 ve2 = *(aw_lds_f64*)(uintptr_t)(nread + 256u);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              sv[4 * j + i] = aw_add_cols(acc[j][i]) * (kn4[i] * fac);
-              vn[4 * j + i] = vn4[i];
-              tv[4 * j + i] = sv[4 * j + i] + ve4[i];
+            for (int jj = 0; jj < 2; ++jj) {
+              sv[jj] *= kn2[jj] * fac;
+              vn[jj] = vn2[jj];
+              tv[jj] = sv[jj] + ve2[jj];
+            }
+          } else {
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+              sv[jj] = akv_dpp_banks<0x118 /*row_shr:8*/, 0xc>(acc[0][jj], acc[1][jj]) + akv_dpp_banks<0x108 /*row_shl:8*/, 0x3>(acc[1][jj], acc[0][jj]);
+            const aw_float4 kn4 = *(aw_lds_f128*)(uintptr_t)nread, vn4 = *(aw_lds_f128*)(uintptr_t)(nread + 128u);
+            const aw_float4 ve4 = *(aw_lds_f128*)(uintptr_t)(nread + 256u);
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj) {
+              sv[jj] *= kn4[jj] * fac;
+              vn[jj] = vn4[jj];
+              tv[jj] = sv[jj] + ve4[jj];
             }
           }
           if (c == nchunks - 1) {        // only the last chunk of a segment holds tokens past its end
             // (such a row may hold anything, NaN norms included.  The empty statement keeps this a branch: as selects the
-            // comparisons cost every chunk 24 instructions.)
+            // comparisons cost every chunk instructions.)
             asm volatile("");
+            const int tok0 = blk_lo * bs + 32 * c + 4 * g + (PACK == 4 ? 16 * (kb >> 1) + 2 * (kb & 1) : 16 * kb);
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (blk_lo * bs + 32 * c + 16 * j + 4 * g + i >= t_end) { sv[4 * j + i] = -INFINITY; vn[4 * j + i] = 0.f; tv[4 * j + i] = -INFINITY; }
+            for (int jj = 0; jj < NV; ++jj)
+              if (tok0 + jj >= t_end) { sv[jj] = -INFINITY; vn[jj] = 0.f; tv[jj] = -INFINITY; }
           }
-#pragma unroll
-          for (int i = 0; i < 8; ++i) mx = fmaxf(mx, tv[i]);
+          float mx = fmaxf(tv[0], tv[1]);
+          if constexpr (PACK == 2) {
+            mx = fmaxf(mx, fmaxf(tv[2], tv[3]));
+            mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0x128 /*row_ror:8*/, 0xf, 0xf, false)));
+          } else {
+            mx = akv_banks_max(mx);
+          }
           aw_wave_sync();      // the norms have been read: the next chunk overwrites them
           mx = akv_rows_max(mx);
           const float m_new = fmaxf(m_run, mx - AW_FRAME);
           const float resc = __builtin_amdgcn_exp2f(m_run - m_new);      // 0 on the first chunk
           m_run = m_new;
           float psum = 0.f;
-          aw_half8 wop[2];
+          uint32_t wh[NV / 2], wl[NV / 2];       // the lane's token pairs as float16 rounding and remainder
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            uint32_t pr[2];
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-              const float p0 = __builtin_amdgcn_exp2f(sv[4 * j + 2 * p] - m_new), p1 = __builtin_amdgcn_exp2f(sv[4 * j + 2 * p + 1] - m_new);
-              psum += p0 + p1;
-              const aw_float2 w2 = {p0 * vn[4 * j + 2 * p], p1 * vn[4 * j + 2 * p + 1]};
-              const aw_half2 h2 = __builtin_convertvector(w2, aw_half2);
-              const aw_half2 l2 = __builtin_convertvector(w2 - __builtin_convertvector(h2, aw_float2), aw_half2);
-              union { aw_half2 h; uint32_t u; } hu, lu;
-              hu.h = h2;
-              lu.h = l2;
-              pr[p] = col < 8 ? hu.u : lu.u;
-            }
-            wop[j] = aw_operand((aw_u32x2){pr[0], pr[0]}, (aw_u32x2){pr[1], pr[1]});
+          for (int p = 0; p < NV / 2; ++p) {
+            const float p0 = __builtin_amdgcn_exp2f(sv[2 * p] - m_new), p1 = __builtin_amdgcn_exp2f(sv[2 * p + 1] - m_new);
+            psum += p0 + p1;
+            const aw_float2 w2 = {p0 * vn[2 * p], p1 * vn[2 * p + 1]};
+            const aw_half2 h2 = __builtin_convertvector(w2, aw_half2);
+            const aw_half2 l2 = __builtin_convertvector(w2 - __builtin_convertvector(h2, aw_float2), aw_half2);
+            union { aw_half2 h; uint32_t u; } hu, lu;
+            hu.h = h2;
+            lu.h = l2;
+            wh[p] = hu.u;
+            wl[p] = lu.u;
           }
           l_run = l_run * resc + psum;
+          // back to the operand's columns: roundings in 0..7, remainders in 8..15, zeros where there is no query head
+          aw_half8 wop[2];
+          if constexpr (PACK == 4) {
+            const uint32_t w0 = akv_pair_from_bank<0>(wh[0], wl[0]), w1 = akv_pair_from_bank<1>(wh[0], wl[0]);
+            const uint32_t w2 = akv_pair_from_bank<2>(wh[0], wl[0]), w3 = akv_pair_from_bank<3>(wh[0], wl[0]);
+            wop[0] = aw_operand((aw_u32x2){w0, w0}, (aw_u32x2){w1, w1});
+            wop[1] = aw_operand((aw_u32x2){w2, w2}, (aw_u32x2){w3, w3});
+          } else {
+            uint32_t w0[2], w1[2];
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+              w0[p] = akv_dpp_banks_u<0x118 /*row_shr:8*/, 0xc>(wh[p], wl[p]);
+              w1[p] = akv_dpp_banks_u<0x108 /*row_shl:8*/, 0x3>(wl[p], wh[p]);
+            }
+            wop[0] = aw_operand((aw_u32x2){w0[0], w0[0]}, (aw_u32x2){w0[1], w0[1]});
+            wop[1] = aw_operand((aw_u32x2){w1[0], w1[0]}, (aw_u32x2){w1[1], w1[1]});
+          }
           if (__builtin_amdgcn_ballot_w64(resc != 1.f) != 0) {
 #pragma unroll
             for (int n = 0; n < CPL; ++n)
@@ -627,7 +675,9 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           load_values(min(k + 1, mine - 1));
           __builtin_amdgcn_sched_barrier(0);
         }
-        l_run = aw_rows_sum(l_run);
+        l_run = aw_rows_sum(l_run);      // (every lane of a row had its own tokens)
+        if constexpr (PACK == 4) l_run = akv_banks_sum(l_run);
+        else l_run = aw_add_cols(l_run);
       } else {
         fill_once();
       }
@@ -735,8 +785,8 @@ static int aw_slots(int kv_heads, int w) {
   return hp;
 }
 
-template <int D, int BITS>
-static int aw_launch(const akv_attn_args& a, const aw_extra& x_in, int grid, hipStream_t stream) {
+template <int D, int BITS, int PACK>
+static int aw_launch_as(const akv_attn_args& a, const aw_extra& x_in, int grid, hipStream_t stream) {
   constexpr int W = aw_cfg<D, BITS>::W;
   aw_extra x = x_in;
   x.hp = aw_slots(a.KVH, W);
@@ -748,13 +798,20 @@ static int aw_launch(const akv_attn_args& a, const aw_extra& x_in, int grid, hip
   int dev = -1;
   AKV_HIP(hipGetDevice(&dev));
   const int rc = allowed(dev, []() -> int {
-    AKV_HIP(hipFuncSetAttribute((const void*)akv_attn_wave_kernel<D, BITS>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
+    AKV_HIP(hipFuncSetAttribute((const void*)akv_attn_wave_kernel<D, BITS, PACK>, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return AKV_OK;
   });
   if (rc) return rc;
-  AKV_LAUNCH_TIMED((akv_attn_wave_kernel<D, BITS>), grid, W * 64, lds, stream, a, x);
+  AKV_LAUNCH_TIMED((akv_attn_wave_kernel<D, BITS, PACK>), grid, W * 64, lds, stream, a, x);
   AKV_LAUNCH_CHECK("akv_attn_wave_kernel");
   return AKV_OK;
+}
+
+template <int D>
+static int aw_launch(const akv_attn_args& a, const aw_extra& x, int bits, int grid, hipStream_t stream) {
+  const bool four = a.QH / a.KVH <= 4;
+  if (bits == 4) return four ? aw_launch_as<D, 4, 4>(a, x, grid, stream) : aw_launch_as<D, 4, 2>(a, x, grid, stream);
+  return four ? aw_launch_as<D, 2, 4>(a, x, grid, stream) : aw_launch_as<D, 2, 2>(a, x, grid, stream);
 }
 
 int akv_attn_wave_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* PiT, const akv_attn_args& a_in,
@@ -793,7 +850,7 @@ int akv_attn_wave_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs
 #undef AW_PRO_D
 #undef AW_PRO
   AKV_LAUNCH_CHECK("akv_attn_wave_prologue_kernel");
-  if (d == 64) return bits == 4 ? aw_launch<64, 4>(a, x, grid, stream) : aw_launch<64, 2>(a, x, grid, stream);
-  if (d == 128) return bits == 4 ? aw_launch<128, 4>(a, x, grid, stream) : aw_launch<128, 2>(a, x, grid, stream);
-  return bits == 4 ? aw_launch<256, 4>(a, x, grid, stream) : aw_launch<256, 2>(a, x, grid, stream);
+  if (d == 64) return aw_launch<64>(a, x, bits, grid, stream);
+  if (d == 128) return aw_launch<128>(a, x, bits, grid, stream);
+  return aw_launch<256>(a, x, bits, grid, stream);
 }
