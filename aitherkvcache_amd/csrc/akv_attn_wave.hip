@@ -1,4 +1,4 @@
-// MFMA paged decode attention in which every wavefront works on its own: 4- and 2-bit caches at head_dim 64 and 256,
+// MFMA paged decode attention in which every wavefront works on its own: 4-, 3- and 2-bit caches at head_dim 64 and 256,
 // and at head_dim 128 with one or two kv heads (akv_attn_wave_applicable), block_size 16 or 32.
 //
 // A workgroup owns a range of the global block axis (akv_attn_partition).  Its W wavefronts are laid out as
@@ -23,7 +23,12 @@
 // is a float16 subnormal that matters.
 //
 // One table serves keys and values: 256 entries x 8 bytes x 32 copies (a lane reads copy lane % 32: no bank conflicts).
-// 2-bit codes are looked up as nibbles: two masks and a shift spread a byte of four codes, no second table.
+// 2-bit codes are looked up as nibbles: two masks and a shift spread a byte of four codes, no second table.  3-bit codes are
+// looked up in pairs, six bits as they lie: a group of eight codes is 24 bits, big-endian, spread to a byte a field by six
+// instructions (one permute among them, which also takes the group out of unaligned bytes); the table then has 64 entries.
+// 3 bits, decode step, this | the vector kernel that served 64 and 256 and the eight-slot kernel at 128: 32 heads on 8 of 64,
+// 48 sequences of 512 to 8,192 tokens 56.3 | 113.2 us; 16 on 4 of 256, 24 sequences 66.7 | 141.5; 8 on 1 of 128, 48 of 1,024
+// to 16,384 39.3 | 62.2; 8 on 2 of 128 52.6 | 62.3.
 //
 // What bounds it: the chain of trips to LDS and memory a wavefront walks, at two to four wavefronts a SIMD.  No unit is full
 // (profiles/attn_wave_sq_counters.txt, share of the kernel's cycles): vector unit
@@ -57,9 +62,9 @@ template <int D, int BITS> struct aw_cfg {
   static constexpr int W = D == 64 ? 16 : 8;            // wavefronts: what their registers admit on a CU
   static constexpr int CPL = D / 16;                    // coordinates per lane of a value tile = M-tiles
   static constexpr int KS = D / 16;                     // MFMA steps of a score tile (four coordinates a lane each)
-  static constexpr int KDW = D * BITS / 128;            // dwords of a quarter of a code row
-  static constexpr int VB = CPL * BITS / 8;             // bytes of a lane's codes of one token
-  static constexpr int VDW = VB >= 4 ? VB / 4 : 1;
+  static constexpr int KDW = BITS == 3 && D == 64 ? 2 : D * BITS / 128;   // dwords read for a quarter of a code row
+  static constexpr int VB = CPL * (BITS == 3 ? 4 : BITS) / 8;             // bytes of a lane's codes of one token (3 bits: spread to nibbles' room)
+  static constexpr int VDW = BITS == 3 ? 2 : VB >= 4 ? VB / 4 : 1;        // dwords (3 bits: the eight bytes around them)
 };
 // LDS: table | per wavefront: 32 key norms, 32 value norms, 32 exponents of those | per wavefront: (max, sum) of eight
 // heads | per wavefront: accumulators of its heads (merging only)
@@ -279,11 +284,20 @@ __device__ __forceinline__ void aw_wave_sync() {
 // workgroup barrier that orders LDS traffic only (what has been requested from memory keeps flying)
 __device__ __forceinline__ void aw_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// the words whose bytes are table indices of lane coordinates: pairs (ta, tb) of tokens, words `wa`, `wb` of codes
-template <int BITS, int N> struct aw_pairs { uint32_t w[BITS == 4 ? 2 : 4]; };
+// 3-bit codes: a group of eight is a big-endian word of 24 bits.  Its four fields of two codes each, one per byte (the first
+// field in byte 3); and the same for two half groups of twelve bits in the halves of a word (first field in byte 1 and 3).
+__device__ __forceinline__ uint32_t aw_spread12(uint32_t x) { return ((x << 2) & 0x3F003F00u) | (x & 0x003F003Fu); }
+__device__ __forceinline__ uint32_t aw_spread24(uint32_t x) { return aw_spread12((x & 0xFFFu) | ((x << 4) & ~0xFFFu)); }
+
+// the words whose bytes are table indices of lane coordinates: pairs (ta, tb) of tokens, words `wa`, `wb` of codes (3 bits: of
+// fields)
+template <int BITS, int N> struct aw_pairs { uint32_t w[BITS == 2 ? 4 : 2]; };
 template <int BITS, int N>
 __device__ __forceinline__ void aw_pair(aw_pairs<BITS, N>& p, uint32_t wa, uint32_t wb) {
-  if constexpr (BITS == 4) {
+  if constexpr (BITS == 3) {
+    p.w[0] = (wa & 0x38383838u) | ((wb >> 3) & 0x07070707u);
+    p.w[1] = ((wa << 3) & 0x38383838u) | (wb & 0x07070707u);
+  } else if constexpr (BITS == 4) {
     p.w[0] = (wa & 0xF0F0F0F0u) | ((wb >> 4) & 0x0F0F0F0Fu);      // the even one of a byte's two codes
     p.w[1] = ((wa << 4) & 0xF0F0F0F0u) | (wb & 0x0F0F0F0Fu);
   } else {
@@ -318,7 +332,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
   // requested its first block ids, rows and queries, so that the fill and the barrier behind it run beside those trips to
   // memory; at 64 and 256 there are no registers left to hold its words until then (they would be spilled).
   constexpr int TPE = W * 64 / 256;                        // threads of an entry
-  const float r0 = a.centroids[(threadIdx.x / TPE >> 4) & ((1 << BITS) - 1)], r1 = a.centroids[threadIdx.x / TPE & ((1 << BITS) - 1)];
+  const float r0 = a.centroids[(threadIdx.x / TPE >> (BITS == 3 ? 3 : 4)) & ((1 << BITS) - 1)], r1 = a.centroids[threadIdx.x / TPE & ((1 << BITS) - 1)];
   // block prefix of the batch, lane i: entry i * pstep, the first step of the search for a segment's sequence
   const int pstep = a.S <= 63 ? 1 : (a.S + 64) / 64;
   int pwin = a.prefix[min(lane * pstep, a.S)], pwin0 = pstep == 1 ? 0 : -1;
@@ -412,8 +426,15 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           pbwin = (int)akv_clamp_block(akv_load_index(a.block_tables, a.bt_itype, s * a.bt_stride + bi), a.num_blocks);
           win_k = k0;
         };
-        const uint32_t koff = (uint32_t)(hd * a.kps_head + col * a.kps_pos + KDW * 4 * g);
-        const uint32_t voff = (uint32_t)(hd * a.vps_head + 4 * g * a.vps_pos + VB * col);
+        // 3 bits: a lane reads whole dwords around its codes; the selectors gather a group's three bytes, first byte on top
+        // (at head_dim 64 a lane of values has half a group: the two bytes with its twelve bits)
+        constexpr int GB = D == 64 ? 3 : 3 * D / 128;                   // bytes from one (pair of) lane's groups to the next's
+        const int vfirst = GB * (D == 64 ? col >> 1 : col), vdw = BITS != 3 ? 0 : min(vfirst >> 2, 3 * D / 32 - 2);
+        const uint32_t o3k = D == 64 ? 2u * (g & 1) : 0u, o3v = (uint32_t)(vfirst - 4 * vdw) + (D == 64 ? (uint32_t)(col & 1) : 0u);
+        const uint32_t ksel3 = 0x0c000102u + 0x010101u * o3k;
+        const uint32_t vsel3 = D == 64 ? 0x0c0c0001u + 0x0101u * o3v : 0x0c000102u + 0x010101u * o3v;
+        const uint32_t koff = (uint32_t)(hd * a.kps_head + col * a.kps_pos + (BITS == 3 ? (3 * D / 32 * g) & ~3 : KDW * 4 * g));
+        const uint32_t voff = (uint32_t)(hd * a.vps_head + 4 * g * a.vps_pos + (BITS == 3 ? 4 * vdw : VB * col));
         const uint32_t ktile1 = bs32 ? 16u * (uint32_t)a.kps_pos : 0u, vtile1 = bs32 ? 16u * (uint32_t)a.vps_pos : 0u;
         const int ntok = lane & 31, npos = bs32 ? ntok : ntok & 15;
         const float* nptr = lane >= 32 ? a.vn : a.kn;
@@ -439,9 +460,14 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
             const unsigned char* p = a.kp + (uint64_t)pb[j] * (uint32_t)a.kps_blk + (j ? ktile1 : 0u) + aw_here(koff);
             if constexpr (KDW == 1) {
               kr[j][0] = *(const uint32_t*)p;
-            } else if constexpr (KDW == 2) {
-              const uint2 t = *(const uint2*)p;
-              kr[j][0] = t.x; kr[j][1] = t.y;
+            } else if constexpr (KDW == 2 || KDW == 3 || KDW == 6) {
+              const uint2 t = *(const uint2*)(p + (KDW - 2) * 4);
+              kr[j][KDW - 2] = t.x; kr[j][KDW - 1] = t.y;
+              if constexpr (KDW == 3) kr[j][0] = *(const uint32_t*)p;
+              if constexpr (KDW == 6) {
+                const uint4 f = *(const uint4*)p;
+                kr[j][0] = f.x; kr[j][1] = f.y; kr[j][2] = f.z; kr[j][3] = f.w;
+              }
             } else {
 #pragma unroll
               for (int i = 0; i < KDW / 4; ++i) {
@@ -460,7 +486,10 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               const unsigned char* p = vb + (uint32_t)(i * (int)a.vps_pos) + aw_here(voff);
-              if constexpr (VB == 1) vr[4 * j + i][0] = *p;
+              if constexpr (BITS == 3) {
+                const uint2 t = *(const uint2*)p;
+                vr[4 * j + i][0] = t.x; vr[4 * j + i][VDW - 1] = t.y;
+              } else if constexpr (VB == 1) vr[4 * j + i][0] = *p;
               else if constexpr (VB == 2) vr[4 * j + i][0] = *(const uint16_t*)p;
               else if constexpr (VB == 4) vr[4 * j + i][0] = *(const uint32_t*)p;
               else {
@@ -503,6 +532,17 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
               const aw_u32x2 q0 = {qd[st].x, qd[st].x}, q1 = {qd[st].y, qd[st].y};
               acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(lo, hi), aw_operand(q0, q1), acc[j], 0, 0, 0);
             };
+            if constexpr (BITS == 3) {
+#pragma unroll
+              for (int i = 0; i < D / 32; ++i) {
+                // (four groups in three dwords; at head_dim 64 two in eight bytes)
+                const int b = D == 64 ? 3 * i : 3 * (i & 3), at = D == 64 ? 0 : 3 * (i >> 2) + b / 4;
+                const uint32_t up = kr[j][min(at + 1, KDW - 1)], sel = D == 64 ? ksel3 + 0x030303u * i : 0x0c000102u + 0x010101u * (b % 4);
+                const uint32_t w = aw_spread24(__builtin_amdgcn_perm(up, kr[j][at], sel));
+                step(2 * i, aw_look<3>(copy, w), aw_look<2>(copy, w));
+                step(2 * i + 1, aw_look<1>(copy, w), aw_look<0>(copy, w));
+              }
+            } else
 #pragma unroll
             for (int i = 0; i < KDW; ++i) {
               const uint32_t w = kr[j][i];
@@ -633,15 +673,18 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-              for (int d = 0; d < VDW; ++d) {
+              for (int d = 0; d < VB / 4; ++d) {
                 aw_pairs<BITS, 0> p01, p23;
-                aw_pair(p01, vr[4 * j][d], vr[4 * j + 1][d]);
-                aw_pair(p23, vr[4 * j + 2][d], vr[4 * j + 3][d]);
+                auto word = [&](int i) __attribute__((always_inline)) {
+                  return BITS == 3 ? aw_spread24(__builtin_amdgcn_perm(vr[4 * j + i][VDW - 1], vr[4 * j + i][0], vsel3 + 0x030303u * d)) : vr[4 * j + i][d];
+                };
+                aw_pair(p01, word(0), word(1));
+                aw_pair(p23, word(2), word(3));
                 auto byte = [&](auto kc) __attribute__((always_inline)) {
                   constexpr int K = decltype(kc)::value;
 #pragma unroll
                   for (int q = 0; q < CPB; ++q) {
-                    const int n = (4 * d + K) * CPB + q;
+                    const int n = (4 * d + (BITS == 3 ? 3 - K : K)) * CPB + q;
                     o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<K>(copy, p01.w[q]), aw_look<K>(copy, p23.w[q])), wop[j], o[n], 0, 0, 0);
                   }
                 };
@@ -653,7 +696,20 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
               aw_pairs<BITS, 0> p;
-              aw_pair(p, vr[4 * j][0] | (vr[4 * j + 2][0] << 16), vr[4 * j + 1][0] | (vr[4 * j + 3][0] << 16));
+              auto word = [&](int i) __attribute__((always_inline)) {
+                if constexpr (BITS != 3) return vr[4 * j + i][0] | (vr[4 * j + i + 2][0] << 16);
+                const uint32_t x = __builtin_amdgcn_perm(vr[4 * j + i][VDW - 1], vr[4 * j + i][0], vsel3) |
+                                   __builtin_amdgcn_perm(vr[4 * j + i + 2][VDW - 1], vr[4 * j + i + 2][0], (vsel3 << 16) | 0x0c0cu);
+                return aw_spread12(x >> (col & 1 ? 0 : 4));
+              };
+              aw_pair(p, word(0), word(1));
+              if constexpr (BITS == 3) {         // (the first field is the upper byte of a half)
+#pragma unroll
+                for (int q = 0; q < CPB; ++q) {
+                  o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<1>(copy, p.w[q]), aw_look<3>(copy, p.w[q])), wop[j], o[q], 0, 0, 0);
+                  o[CPB + q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<0>(copy, p.w[q]), aw_look<2>(copy, p.w[q])), wop[j], o[CPB + q], 0, 0, 0);
+                }
+              } else
 #pragma unroll
               for (int q = 0; q < CPB; ++q) {
                 o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<0>(copy, p.w[q]), aw_look<2>(copy, p.w[q])), wop[j], o[q], 0, 0, 0);
@@ -772,7 +828,7 @@ int akv_attn_mfma_head_groups(int gqa);
 // Two groups lose once sequences no longer get whole workgroups (more than 64: akv_attn_partition): four wavefronts then merge
 // a few chunks at every change of the sequence.
 bool akv_attn_wave_applicable(const akv_attn_args& a, int d, int bits) {
-  if (!(d == 64 || d == 128 || d == 256) || (bits != 4 && bits != 2) || !akv_attn_mfma_takes(a, bits)) return false;
+  if (!(d == 64 || d == 128 || d == 256) || bits < 2 || bits > 4 || !akv_attn_mfma_takes(a, bits)) return false;
   if (d != 128) return true;
   const int heads = a.KVH * akv_attn_mfma_head_groups(a.QH / a.KVH);
   return heads == 1 || (heads == 2 && a.S <= 64);
@@ -811,6 +867,7 @@ template <int D>
 static int aw_launch(const akv_attn_args& a, const aw_extra& x, int bits, int grid, hipStream_t stream) {
   const bool four = a.QH / a.KVH <= 4;
   if (bits == 4) return four ? aw_launch_as<D, 4, 4>(a, x, grid, stream) : aw_launch_as<D, 4, 2>(a, x, grid, stream);
+  if (bits == 3) return four ? aw_launch_as<D, 3, 4>(a, x, grid, stream) : aw_launch_as<D, 3, 2>(a, x, grid, stream);
   return four ? aw_launch_as<D, 2, 4>(a, x, grid, stream) : aw_launch_as<D, 2, 2>(a, x, grid, stream);
 }
 

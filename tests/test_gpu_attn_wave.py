@@ -77,6 +77,12 @@ def test_edges_vs_float64(dev, d, bits, qh, kvh, bs):
         assert (out[i] - ref).norm() <= REL * ref.norm(), (i, n)
 
 
+@pytest.mark.parametrize("d,qh,kvh,bs", [(d, *h) for d in (64, 128, 256) for h in HEADS if d != 128 or (h[0] <= 16 and h[1] <= 2)])
+def test_edges_of_3bit_rows_vs_float64(dev, d, qh, kvh, bs):
+    """The same with 3-bit rows: groups of 24 bits, at head_dim 64 half of one a lane, none on a dword of its own."""
+    test_edges_vs_float64(dev, d, 3, qh, kvh, bs)
+
+
 @pytest.mark.parametrize("d,qh,kvh,bs,chunks", [(256, 16, 8, 16, 70), (256, 4, 1, 32, 70), (64, 16, 16, 32, 70),
                                                 (256, 8, 8, 16, 32), (256, 8, 8, 32, 64), (64, 16, 16, 16, 64), (64, 16, 16, 32, 32)])
 def test_more_chunks_than_a_window_of_block_ids(dev, d, qh, kvh, bs, chunks):
