@@ -44,7 +44,7 @@
 // never conflict on a bank.
 //
 // The 3-bit and 2-bit caches index tables of their own shape with the packed bits as they lie in memory (no
-// spreading to nibbles; the tq35 kernel below, whose parts mix code widths, does spread):
+// spreading to nibbles):
 //   3-bit  a group of eight codes is a big-endian 24-bit word (one byte permute); an index is a 6-bit FIELD of it.
 //          K: field = two neighbouring codes of a token, 64 entries of 8 bytes.  V: the codes at odd and at even
 //          positions of two neighbouring tokens are merged into two words of four fields (three operations
@@ -72,7 +72,6 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 // entry e of table A at e*256:          [(hi pair, lo pair) for K x 32 copies]
 // entry e of table B at 65536 + e*256:  [fp16(alpha c) pairs for V x 32 copies][128 bytes of exchange buffer]
 #define MF_TABB 65536u
-#define MF_XBUF 4096u                // distance of the two exchange buffers of a head slot
 // exchange units of the kernel for the uniform formats: stride and start (4- and 3-bit: the spare halves of table B
 // entries; 2-bit: 128-byte units after the tables)
 #define MF_XSTRIDE(bits) ((bits) == 2 ? 128u : 256u)
@@ -95,7 +94,6 @@ struct akv_mfma_extra {
   const uint4* qop;      // [S][KVH][8 k-steps][64 lanes] half8 as uint4 (workspace)
   const int32_t* wgdesc; // [G][AKV_WGREC] record of every workgroup (workspace)
   uint32_t* status;      // status words of the call (workspace header)
-  int spin_limit;        // polls a hand-off wait makes before it gives up
 };
 
 // ----------------------------------------------------------------------------------
@@ -333,10 +331,6 @@ __device__ __forceinline__ half8 mf_pack(uint32_t a, uint32_t b, uint32_t c, uin
 __device__ __forceinline__ float mf_from_hi_cols(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x108 /*row_shl:8*/, 0xf, 0xf, true));
 }
-// lane c receives the value of lane c - 8 of its row (zero for c < 8)
-__device__ __forceinline__ float mf_from_lo_cols(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118 /*row_shr:8*/, 0xf, 0xf, true));
-}
 
 // block id x block stride on the scalar unit (a 64-bit product of 64-bit operands would go through
 // the vector unit and drag the whole address into vector registers); strides are below 2^31
@@ -366,29 +360,6 @@ __device__ __forceinline__ float mf_rows_sum(float v) {
   v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
   auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
-// Pairwise hand-off between the score and the value wavefront of a head slot (tq35 kernel; the kernel
-// for the uniform formats orders its chunks with workgroup barriers instead): two counters in LDS,
-// `ready` (chunks whose weights are written) and `done` (chunks whose weights have been read), both
-// counted from the start of the kernel.  LDS operations of a wavefront are executed in order, so a
-// counter written after the data is seen after the data.  Waiting polls the counter with a short
-// sleep; the wait is bounded, so every wavefront finishes whatever happens.  A wait that gives up
-// leaves a mark in the status word of the call (an ordinary vector store): the kernel goes on with
-// whatever the buffer holds, the reduce kernel turns every output of the call into NaN, and the host
-// can read the word back (akv_paged_attn_status).
-#define MF_SPIN_LIMIT (1 << 16)
-__device__ __forceinline__ void mf_wait_ge(uint32_t addr, uint32_t need, uint32_t* status, int limit) {
-  for (int spin = 0; spin < limit; ++spin) {
-    uint32_t v;
-    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(addr) : "memory");
-    if ((int32_t)((uint32_t)__builtin_amdgcn_readfirstlane((int)v) - need) >= 0) return;
-    __builtin_amdgcn_s_sleep(2);
-  }
-  if ((threadIdx.x & 63) == 0) *(volatile uint32_t*)status = AKV_STATUS_HANDOFF_TIMEOUT;
-}
-__device__ __forceinline__ void mf_publish(uint32_t addr, uint32_t value) {
-  asm volatile("ds_write_b32 %0, %1" : : "v"(addr), "v"(value) : "memory");
 }
 
 // workgroup barrier that orders LDS traffic only (outstanding global loads keep flying)
@@ -1073,7 +1044,7 @@ __global__ __launch_bounds__(MF_THREADS) void akv_attn_mfma_kernel(akv_attn_args
 // ----------------------------------------------------------------------------------
 // host side
 // ----------------------------------------------------------------------------------
-static bool mfma_disabled() {
+bool akv_attn_mfma_disabled() {
   static int v = -1;
   if (v < 0) {
     const char* e = getenv("AKV_DISABLE_MFMA");
@@ -1087,14 +1058,6 @@ size_t akv_attn_mfma_extra_bytes(int S, int KVH) {
   return akv_align256((size_t)S * KVH * 8 * 64 * 16);
 }
 
-// polls a hand-off wait makes before it gives up (akv_debug_set_handoff_spin_limit)
-static int g_spin_limit = MF_SPIN_LIMIT;
-int akv_attn_spin_limit() { return g_spin_limit; }
-extern "C" int akv_debug_set_handoff_spin_limit(int polls) {
-  g_spin_limit = polls < 0 ? MF_SPIN_LIMIT : polls;
-  return AKV_OK;
-}
-
 // query heads per kv head -> number of groups of at most eight the kv head is presented as (0: none fits)
 int akv_attn_mfma_head_groups(int gqa) {
   for (int hg = (gqa + 7) / 8; hg <= gqa && hg <= 8; ++hg)
@@ -1103,7 +1066,7 @@ int akv_attn_mfma_head_groups(int gqa) {
 }
 
 bool akv_attn_mfma_takes(const akv_attn_args& a, int bits) {
-  if (mfma_disabled()) return false;
+  if (akv_attn_mfma_disabled()) return false;
   if (bits < 2 || bits > 4 || (a.block_size != 16 && a.block_size != 32)) return false;
   if (akv_attn_mfma_head_groups(a.QH / a.KVH) == 0) return false;
   if (a.num_blocks >= ((int64_t)1 << 31)) return false;                       // block ids travel as 32-bit lanes
@@ -1136,7 +1099,6 @@ int akv_attn_mfma_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs
   x.qop = (const uint4*)extra_ws;
   x.wgdesc = ws.wgdesc;
   x.status = ws.status;
-  x.spin_limit = g_spin_limit;
   const float qscale = a.scale * 1.4426950408889634f;   // scores come out in the log2 domain
   // rotation blocks: one per (sequence, kv head) up to six per CU (what its registers admit at once), then they loop
   const int cus = akv_cached_cu_count();
@@ -1166,648 +1128,5 @@ int akv_attn_mfma_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs
   else MF_RUN(2, MF_LDS_BYTES_2BIT);
 #undef MF_RUN
   AKV_LAUNCH_CHECK("akv_attn_mfma_kernel");
-  return AKV_OK;
-}
-
-// ==================================================================================
-// tq35 rows on the same machinery
-// ==================================================================================
-// A tq35 row is four parts per token: A0 (64 codes of 3 bits), B0 (64 sign bits), A1 (64 codes of
-// 2 bits), B1 (64 sign bits), plus two fp16 factors per group inside the row.  Spread to one code
-// per nibble they are 256 "virtual coordinates" over ONE table of sixteen levels -- 0..7 the 3-bit
-// codebook, 8..11 the 2-bit codebook, 12 / 13 the signs -1 / +1 -- so the byte-pair tables and
-// both products of the kernel above serve unchanged:
-//
-//   scores   four accumulators per 16-token tile, one per part (lane group g supplies nibble dwords
-//            2g and 2g+1 of the part, four MFMAs per part), combined per token as
-//            n0 (A0 + r0 B0) + n1 (A1 + r1 B1); the query operand holds the four transformed copies of
-//            the query (aither_kvcache/hybrid_quantizer.py:600-640) in the coordinate order the
-//            spreading leaves.
-//   values   an M-tile mixes two parts so that a lane owns a dword-aligned piece of the row.  Pass C:
-//            rows 0-7 the eight 3-byte groups of A0, rows 8-15 the eight halfwords of A1; pass S: rows
-//            0-7 the sign bytes of B0, rows 8-15 those of B1.  The weight operand of a pass carries both
-//            of its parts' weights (p n0 and p n1, or p n0 r0 and p n1 r1): columns 4t + q hold the fp16
-//            part of set t for query head q of the group of four, columns 8 + 4t + q the remainder, and
-//            a lane keeps the results whose rows belong to its column's set.  The V table holds
-//            fp16(alpha c) with one alpha per codebook; pass S builds its operand straight from the sign
-//            bits (fp16 -1 and +1 differ in one bit), no table; 1 / alpha and kappa = sqrt(pi/2)/64 are
-//            applied to the finished sums (on the score side kappa rides in the query copies).
-//
-// One workgroup = 8 wavefronts: 4 score + 4 value (two passes of 8 accumulator tiles need twice the
-// registers of the uniform formats), four groups of four query heads at a time.
-#include "akv_hybrid_layout.h"
-
-#define HM_HEADS 4
-#define HM_THREADS 512
-#define HM_NORMX ((uint32_t)MF_LDS_BYTES)    // float32 factors of a chunk: [parity][head slot][K | V][tile][field][16 tokens]
-#define HM_WBUF2 (HM_NORMX + 2u * HM_HEADS * 1024u)   // weight operand of the second value pass
-#define HM_LDS_BYTES (MF_LDS_BYTES + 4 * HM_HEADS * 1024)
-#define HM_BITS_TAG 35
-
-// level v of the merged table; the sign levels carry `sign_mag`
-__device__ __forceinline__ float hm_level(const float* __restrict__ table, int v, float sign_mag) {
-  return v < 12 ? table[HYB_CEN0 + v] : v == 12 ? -sign_mag : v == 13 ? sign_mag : 0.f;
-}
-
-// coordinate (0..63 inside its part) of nibble (byte b, lo = low nibble) of nibble dword D of part X
-// (0 = A0, 1 = B0, 2 = A1, 3 = B1)
-__host__ __device__ constexpr int hm_coord(int X, int D, int b, int lo) {
-  if (X == 0) return 8 * D + mf_kcoord<3>(0, b, lo);
-  if (X == 2) return 8 * D + (b == 0 ? 2 : b == 1 ? 0 : b == 2 ? 6 : 4) + lo;   // mf_spread2: bytes (c2,c3) (c0,c1) (c6,c7) (c4,c5)
-  return 8 * D + 6 - 2 * b + lo;                                                  // hm_spread1: nibble i <- bit i <- coordinate 7 - i
-}
-
-// value side, 2-bit lanes: code of M-tile n (byte n/2; odd n = low nibble) among the lane's eight; the
-// nibbles are [c3 c1 c7 c5 c2 c0 c6 c4] from bit 0 up
-__host__ __device__ constexpr int hm_vcoord2(int n) {
-  constexpr int nib[8] = {3, 1, 7, 5, 2, 0, 6, 4};
-  return nib[2 * (n >> 1) + ((n & 1) ? 0 : 1)];
-}
-
-// eight sign bits (coordinate k at bit 7 - k) -> nibbles 12 | bit, nibble i <- bit i
-__device__ __forceinline__ uint32_t hm_spread1(uint32_t b) {
-  uint32_t t = (b | (b << 12)) & 0x000F000Fu;
-  t = (t | (t << 6)) & 0x03030303u;
-  return ((t | (t << 3)) & 0x11111111u) | 0xCCCCCCCCu;
-}
-
-template <int QDT>
-__global__ __launch_bounds__(256) void akv_hyb_mfma_prologue_kernel(
-    const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const float* __restrict__ table,
-    float kappa, float qscale, int S, int QH, int KVH, const void* context_lens, int cl_itype,
-    int block_size, int64_t max_blocks_per_seq, int32_t* prefix, uint4* __restrict__ qop,
-    uint32_t* __restrict__ lut, uint32_t* __restrict__ status) {
-  __shared__ float qv[4][4][64];     // [query head of the group][part][coordinate]
-  __shared__ int32_t scratch[257];
-  __shared__ float best_err[256];
-  __shared__ float best_alpha[256];
-  const int tid = threadIdx.x;
-  const int nq = S * KVH;
-  if ((int)blockIdx.x == nq) {
-    if (tid == 0) status[0] = 0u;
-    akv_block_prefix_scan(context_lens, cl_itype, S, block_size, max_blocks_per_seq, prefix, scratch);
-    return;
-  }
-  if ((int)blockIdx.x == nq + 1) {
-    // tables of the merged sixteen levels, rebuilt only when the codebooks in the table change
-    __shared__ int stale;
-    __shared__ float alphas[2];
-    if (tid == 0) stale = (lut[MF_W_MARK] != MF_MARK + (uint32_t)HM_BITS_TAG) ? 1 : 0;
-    __syncthreads();
-    if (tid < 12 && __float_as_uint(table[HYB_CEN0 + tid]) != lut[MF_W_TAG + tid]) stale = 1;
-    __syncthreads();
-    if (!stale) return;
-    // V table: fp16(alpha0 c) for the 3-bit codebook, fp16(alpha1 c) for the 2-bit codebook, each alpha in
-    // [1,2) minimising the largest relative rounding error of its levels; the signs are exactly -1 / +1
-    // (kappa and 1 / alpha are applied to the sums at the end)
-    float c[12];
-    for (int v = 0; v < 12; ++v) c[v] = table[HYB_CEN0 + v];
-    for (int set = 0; set < 2; ++set) {
-      const int v0 = set ? 8 : 0, v1 = set ? 12 : 8;
-      float berr = 1e30f, balpha = 1.f;
-      for (int k = 0; k < MF_ALPHA_CANDIDATES / 256; ++k) {
-        const float al = 1.f + (float)(tid * (MF_ALPHA_CANDIDATES / 256) + k) / (float)MF_ALPHA_CANDIDATES;
-        float worst = 0.f;
-        for (int v = v0; v < v1; ++v) {
-          const float x = al * c[v];
-          const float r = __half2float(__float2half_rn(x));
-          const float e = x != 0.f ? fabsf(r - x) / fabsf(x) : 0.f;
-          worst = fmaxf(worst, e);
-        }
-        if (worst < berr) { berr = worst; balpha = al; }
-      }
-      __syncthreads();
-      best_err[tid] = berr;
-      best_alpha[tid] = balpha;
-      __syncthreads();
-      if (tid == 0) {
-        for (int t = 1; t < 256; ++t)
-          if (best_err[t] < best_err[0]) { best_err[0] = best_err[t]; best_alpha[0] = best_alpha[t]; }
-        lut[MF_W_ALPHA + set] = __float_as_uint(best_alpha[0]);
-        alphas[set] = best_alpha[0];
-      }
-    }
-    __syncthreads();
-    auto vlevel = [&](int v) { return v < 8 ? alphas[0] * c[v] : v < 12 ? alphas[1] * c[v] : v == 12 ? -1.f : v == 13 ? 1.f : 0.f; };
-    const float c0 = hm_level(table, tid >> 4, 1.f), c1 = hm_level(table, tid & 15, 1.f);
-    const __half k0 = __float2half_rn(c0), k1 = __float2half_rn(c1);
-    lut[MF_W_KHI + tid] = (unsigned)__half_as_ushort(k0) | ((unsigned)__half_as_ushort(k1) << 16);
-    const __half l0 = __float2half_rn(c0 - __half2float(k0)), l1 = __float2half_rn(c1 - __half2float(k1));
-    lut[MF_W_KLO + tid] = (unsigned)__half_as_ushort(l0) | ((unsigned)__half_as_ushort(l1) << 16);
-    const __half v0 = __float2half_rn(vlevel(tid >> 4)), v1 = __float2half_rn(vlevel(tid & 15));
-    lut[MF_W_VHI + tid] = (unsigned)__half_as_ushort(v0) | ((unsigned)__half_as_ushort(v1) << 16);
-    if (tid < 12) lut[MF_W_TAG + tid] = __float_as_uint(table[HYB_CEN0 + tid]);
-    __threadfence();
-    __syncthreads();
-    if (tid == 0) lut[MF_W_MARK] = MF_MARK + (uint32_t)HM_BITS_TAG;
-    return;
-  }
-  const int s = blockIdx.x / KVH, hv = blockIdx.x % KVH;
-  const int lane = tid & 63, w = tid >> 6;
-  {
-    const int64_t off = s * qs_seq + (int64_t)(hv * 4 + w) * qs_head;
-    const float q0 = akv_elem<QDT>::load(query, off + lane);
-    const float q1 = akv_elem<QDT>::load(query, off + 64 + lane);
-    qv[w][0][lane] = hyb_fwht64(q0 * table[HYB_HAD0 + lane], lane) * 0.125f * qscale;
-    qv[w][1][lane] = hyb_fwht64(q0 * table[HYB_QJL0 + lane], lane) * 0.125f * kappa * qscale;
-    qv[w][2][lane] = hyb_fwht64(q1 * table[HYB_HAD1 + lane], lane) * 0.125f * qscale;
-    qv[w][3][lane] = hyb_fwht64(q1 * table[HYB_QJL1 + lane], lane) * 0.125f * kappa * qscale;
-  }
-  __syncthreads();
-  // operand layout: [k-step n = 4 X + n4][lane (col, g)][e]: nibble dword 2g + n4/2 of part X, byte
-  // 2(n4 % 2) + e/4, nibble e % 2 (0 = high); elements 2,3 and 6,7 repeat 0,1 and 4,5 (they face the lo
-  // halves of the K table entries); columns [0,4) the fp16 rounding of the query copy, [8,12) its remainder
-  for (int n = w; n < 16; n += 4) {
-    const int X = n >> 2, n4 = n & 3;
-    const int col = lane & 15, g = lane >> 4;
-    unsigned short hbits[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int D = 2 * g + (n4 >> 1), b = 2 * (n4 & 1) + (e >> 2), lo = e & 1;
-      const int coord = hm_coord(X, D, b, lo);
-      float v = 0.f;
-      if (col < 4) {
-        v = __half2float(__float2half_rn(qv[col][X][coord]));
-      } else if (col >= 8 && col < 12) {
-        const float full = qv[col - 8][X][coord];
-        v = full - __half2float(__float2half_rn(full));
-      }
-      hbits[e] = __half_as_ushort(__float2half_rn(v));
-    }
-    uint4 o;
-    o.x = hbits[0] | (hbits[1] << 16); o.y = hbits[2] | (hbits[3] << 16);
-    o.z = hbits[4] | (hbits[5] << 16); o.w = hbits[6] | (hbits[7] << 16);
-    qop[((size_t)(s * KVH + hv) * 16 + n) * 64 + lane] = o;
-  }
-}
-
-struct hm_kraw {        // score wavefront, one 32-token chunk: the lane's pieces of token l%16 of both tiles
-  mf_u32x2 a0[2];       // 8 bytes holding 3-byte groups 2g, 2g+1 of A0
-  uint32_t b0[2];       // dword holding sign bytes 2g, 2g+1 of B0
-  uint32_t a1[2];       // halfwords 2g, 2g+1 of A1
-  uint32_t b1[2];
-  uint32_t n0, n1;      // lane < 32: the two factor dwords of token l's K row, else of token (l - 32)'s V row
-};
-struct hm_vraw {        // value wavefront: tokens 4g + i of both tiles
-  uint32_t c[8];        // pass C dword (A0 group col / A1 halfword col - 8)
-  uint32_t s[8];        // pass S dword (sign byte)
-};
-
-template <int ROLE>
-__device__ __forceinline__ void hm_role_main(const akv_hyb_mfma_args& a, const int hs) {
-  const int lane = threadIdx.x & 63;
-  const int col = lane & 15, g = lane >> 4;
-  const uint32_t lane4v = MF_TABB + (uint32_t)(lane & 31) * 4u;
-  const uint32_t lane4k = (uint32_t)(lane & 31) * 8u;
-  // exchange buffers as in the kernel above: weights (16 B per reader lane L) at entry 32 hs + L/8,
-  // rescale factors (4 B per lane) at entries 32 hs + 8, 9, flags at entry 32 hs + 12
-  auto pbx = [&](uint32_t L) { return MF_TABB + (32u * hs + (L >> 3)) * 256u + 128u + (L & 7u) * 16u; };
-  auto wsx = [&](uint32_t L) { return HM_WBUF2 + (uint32_t)hs * 1024u + L * 16u; };   // pass S weights: [parity][head slot][lane]
-  auto rsx = [&](uint32_t L) { return MF_TABB + (32u * hs + 8u + (L >> 5)) * 256u + 128u + (L & 31u) * 4u; };
-  const uint32_t fl_addr = MF_TABB + (32u * hs + 12u) * 256u + 128u;
-  uint32_t T = 0;
-
-  // blocks of 16 tokens: a chunk is two blocks; blocks of 32: one block, its second tile 16 positions further in
-  const bool bs32 = a.block_size == 32;
-  const int bs = bs32 ? 32 : 16;
-  const int G = gridDim.x;
-  const int total = a.prefix[a.S];
-  const int per = (total + G - 1) / G;
-  const int g0 = blockIdx.x * per;
-  const int g1 = min(total, g0 + per);
-
-  int gcur = g0;
-  while (gcur < g1) {
-    const int s = akv_find_seq(a.prefix, a.S, gcur);
-    const int sb0 = a.prefix[s], sb1 = a.prefix[s + 1];
-    const int blk_lo = gcur - sb0;
-    const int blk_hi = min(g1, sb1) - sb0;
-    const int64_t ctx = akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq);
-    const int t_end = (int)min((int64_t)blk_hi * bs, ctx);
-    gcur = sb0 + blk_hi;
-    const int nblk = blk_hi - blk_lo;
-    const int nchunks = bs32 ? nblk : (nblk + 1) >> 1;
-
-    for (int hbase = 0; hbase < a.KVH; hbase += HM_HEADS) {
-      const int h = hbase + hs;
-      if (h >= a.KVH || nchunks <= 0) continue;
-      const int hd = h / a.hgroup;      // the kv head whose rows are read
-
-      int pbwin = 0, win_c0 = 0;
-      auto load_window = [&](int c0) {
-        const int bi = min(blk_lo + (bs32 ? c0 : 2 * c0) + lane, blk_hi - 1);
-        pbwin = (int)akv_clamp_block(akv_load_index(a.block_tables, a.bt_itype, s * a.bt_stride + bi), a.num_blocks);
-        asm volatile("" : "+v"(pbwin));
-        win_c0 = c0;
-      };
-      auto chunk_blocks = [&](int c_in, uint32_t& p0, uint32_t& p1) {
-        const int c = min(c_in, nchunks - 1);
-        const int w0 = bs32 ? c - win_c0 : 2 * (c - win_c0);
-        const int w1 = (!bs32 && 2 * c + 1 < nblk) ? w0 + 1 : w0;
-        p0 = (uint32_t)__builtin_amdgcn_readlane(pbwin, w0);
-        p1 = (uint32_t)__builtin_amdgcn_readlane(pbwin, w1);
-      };
-      load_window(0);
-
-      if constexpr (ROLE == 0) {
-        // =========================== score wavefront ===========================
-        half8 qb[16];
-        {
-          const uint4* qp = a.qop + ((size_t)(s * a.KVH + h) * 16) * 64 + lane;
-#pragma unroll
-          for (int st = 0; st < 16; ++st) {
-            const uint4 u = qp[st * 64];
-            qb[st] = mf_pack(u.x, u.y, u.z, u.w);
-          }
-        }
-        float m_run = -INFINITY, l_run = 0.f;
-        const uint32_t krow = (uint32_t)(hd * a.kps_head + col * a.kps_pos);
-        const uint32_t offA0 = krow + (g == 0 ? 0u : g == 1 ? 4u : g == 2 ? 12u : 16u);
-        const uint32_t offB0 = krow + 24u + 4u * (uint32_t)(g >> 1);
-        const uint32_t offA1 = krow + 36u + 4u * (uint32_t)g;
-        const uint32_t offB1 = krow + 52u + 4u * (uint32_t)(g >> 1);
-        const uint32_t selA = (g & 1) ? 0x0c020304u : 0x0c000102u;    // big-endian 24-bit words of the two groups
-        const uint32_t selB = (g & 1) ? 0x0c050607u : 0x0c030405u;
-        const uint32_t hsh = 16u * (uint32_t)(g & 1);
-        const int ntok = lane & 31;
-        const bool nrm_is_v = lane >= 32;
-        const uint8_t* nrm_base = nrm_is_v ? a.vc : a.kc;
-        const uint32_t nrm_blk = (uint32_t)(nrm_is_v ? a.vps_blk : a.kps_blk);
-        const int npos = bs32 ? ntok : (ntok & 15);          // position of token ntok inside its block
-        const uint32_t nrm_off = (uint32_t)(nrm_is_v ? hd * a.vps_head + npos * a.vps_pos
-                                                     : hd * a.kps_head + npos * a.kps_pos);
-        const uint32_t ktile1 = bs32 ? 16u * (uint32_t)a.kps_pos : 0u;
-        // factor exchange: writer lane (kind = l/32, tile = (l/16)%2, token l%16) field f; reader lane (col, g)
-        // takes tokens 4g..4g+3 of a (kind, tile, field) with one 16-byte read
-        const uint32_t nw_addr = HM_NORMX + (uint32_t)hs * 1024u + (uint32_t)(lane >> 4) * 256u + (uint32_t)(lane & 15) * 4u;
-        const uint32_t nr_addr = HM_NORMX + (uint32_t)hs * 1024u + (uint32_t)g * 16u;
-        auto load_chunk = [&](hm_kraw& r, int c) {
-          uint32_t pb[2];
-          chunk_blocks(c, pb[0], pb[1]);
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const unsigned char* kb = a.kc + mf_umul(pb[j], (uint32_t)a.kps_blk) + (j ? ktile1 : 0u);
-            r.a0[j] = *(const mf_u32x2*)(kb + mf_here(offA0));
-            r.b0[j] = *(const uint32_t*)(kb + mf_here(offB0));
-            r.a1[j] = *(const uint32_t*)(kb + mf_here(offA1));
-            r.b1[j] = *(const uint32_t*)(kb + mf_here(offB1));
-          }
-          const unsigned char* nb = nrm_base + mf_umul(ntok >= 16 ? pb[1] : pb[0], nrm_blk) + mf_here(nrm_off);
-          r.n0 = *(const uint32_t*)(nb + 32);
-          r.n1 = *(const uint32_t*)(nb + 60);
-        };
-        auto half_lo = [](uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w & 0xffffu))); };
-        auto half_hi = [](uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w >> 16))); };
-        auto produce = [&](hm_kraw& r, int c, const uint32_t par) {
-          *(mf_lds_u32*)(uintptr_t)(nw_addr + 4096u * par) = __float_as_uint(half_lo(r.n0));
-          *(mf_lds_u32*)(uintptr_t)(nw_addr + 4096u * par + 64u) = __float_as_uint(half_hi(r.n0));
-          *(mf_lds_u32*)(uintptr_t)(nw_addr + 4096u * par + 128u) = __float_as_uint(half_lo(r.n1));
-          *(mf_lds_u32*)(uintptr_t)(nw_addr + 4096u * par + 192u) = __float_as_uint(half_hi(r.n1));
-          // nibble dwords: step n = 8 j + 2 X + Dl
-          uint32_t kw[16];
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            kw[8 * j + 0] = mf_spread3(__builtin_amdgcn_perm(r.a0[j].y, r.a0[j].x, selA));
-            kw[8 * j + 1] = mf_spread3(__builtin_amdgcn_perm(r.a0[j].y, r.a0[j].x, selB));
-            const uint32_t s0 = r.b0[j] >> hsh;
-            kw[8 * j + 2] = hm_spread1(s0 & 0xffu);
-            kw[8 * j + 3] = hm_spread1((s0 >> 8) & 0xffu);
-            kw[8 * j + 4] = mf_spread2(r.a1[j] & 0xffffu) | 0x88888888u;
-            kw[8 * j + 5] = mf_spread2(r.a1[j] >> 16) | 0x88888888u;
-            const uint32_t s1 = r.b1[j] >> hsh;
-            kw[8 * j + 6] = hm_spread1(s1 & 0xffu);
-            kw[8 * j + 7] = hm_spread1((s1 >> 8) & 0xffu);
-          }
-          mf_u32x2 w[3][4];
-          float4v acc[2][4];
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int X = 0; X < 4; ++X) acc[j][X] = (float4v){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int n = 0; n < 2; ++n)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) w[n][b] = mf_lut2(lane4k, kw[n], MF_SEL(b));
-#pragma unroll
-          for (int n = 0; n < 16; ++n) {
-            if (n + 2 < 16) {
-#pragma unroll
-              for (int b = 0; b < 4; ++b) w[(n + 2) % 3][b] = mf_lut2(lane4k, kw[n + 2], MF_SEL(b));
-            }
-            const int j = n >> 3, X = (n >> 1) & 3, st = 2 * (n & 7);
-            acc[j][X] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                mf_pack(w[n % 3][0].x, w[n % 3][0].y, w[n % 3][1].x, w[n % 3][1].y), qb[st], acc[j][X], 0, 0, 0);
-            acc[j][X] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                mf_pack(w[n % 3][2].x, w[n % 3][2].y, w[n % 3][3].x, w[n % 3][3].y), qb[st + 1], acc[j][X], 0, 0, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          load_chunk(r, c + 2);
-          __builtin_amdgcn_sched_barrier(0);
-          float sv[8];
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            union { mf_u32x4 u; float f[4]; } kn0, kr0, kn1, kr1;
-            const uint32_t base = nr_addr + 4096u * par + 256u * j;
-            kn0.u = *(mf_lds_u128*)(uintptr_t)(base);
-            kr0.u = *(mf_lds_u128*)(uintptr_t)(base + 64u);
-            kn1.u = *(mf_lds_u128*)(uintptr_t)(base + 128u);
-            kr1.u = *(mf_lds_u128*)(uintptr_t)(base + 192u);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float t0 = fmaf(kr0.f[i], acc[j][1][i], acc[j][0][i]);
-              const float t1 = fmaf(kr1.f[i], acc[j][3][i], acc[j][2][i]);
-              const float raw = fmaf(kn1.f[i], t1, kn0.f[i] * t0);
-              sv[4 * j + i] = raw + mf_from_hi_cols(raw);
-            }
-          }
-          // From here on the wavefront works on a PACKED copy of the scores: the group has four query heads, so only
-          // columns 0..3 of a row of sixteen lanes hold scores, eight per lane.  Lane 4k + c takes the token pair k
-          // (values 2k, 2k + 1) of head c: two exponentials, eight weight products and four float16 splits per lane
-          // and chunk in place of eight, thirty-two and sixteen; every lane then writes its own pair straight into
-          // the operand fragments of the value side.
-          const int kb = col >> 2, c4 = col & 3;
-          float ps[2];
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj)
-            ps[jj] = akv_to_bank<3>(akv_to_bank<2>(akv_to_bank<1>(sv[jj], sv[2 + jj]), sv[4 + jj]), sv[6 + jj]);
-          // value-side factors of the lane's token pair (tile kb / 2, tokens 4g + 2 (kb % 2) + {0, 1})
-          union { mf_u32x2 u; float f[2]; } vn0, vr0, vn1, vr1;
-          {
-            const uint32_t base = nr_addr + 4096u * par + 512u + 256u * (uint32_t)(kb >> 1) + 8u * (uint32_t)(kb & 1);
-            vn0.u = *(mf_lds_cu64*)(uintptr_t)(base);
-            vr0.u = *(mf_lds_cu64*)(uintptr_t)(base + 64u);
-            vn1.u = *(mf_lds_cu64*)(uintptr_t)(base + 128u);
-            vr1.u = *(mf_lds_cu64*)(uintptr_t)(base + 192u);
-          }
-          if (c == nchunks - 1) {     // only the last chunk of a segment can hold masked tokens (whose rows may hold anything)
-            const int tok0 = blk_lo * bs + 32 * c + 16 * (kb >> 1) + 4 * g + 2 * (kb & 1);
-            const bool tile_ok = (kb >> 1) == 0 || bs32 || 2 * c + 1 < nblk;
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-              if (!(tile_ok && tok0 + jj < t_end)) { ps[jj] = -INFINITY; vn0.f[jj] = 0.f; vr0.f[jj] = 0.f; vn1.f[jj] = 0.f; vr1.f[jj] = 0.f; }
-          }
-          const float mx = mf_rows_max(akv_banks_max(fmaxf(ps[0], ps[1])));
-          const float m_new = fmaxf(m_run, mx);
-          const float resc = __builtin_amdgcn_exp2f(m_run - m_new);
-          m_run = m_new;
-          float pw[4][2];
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj) {
-            const float p = __builtin_amdgcn_exp2f(ps[jj] - m_new);
-            pw[0][jj] = p * vn0.f[jj];
-            pw[1][jj] = pw[0][jj] * vr0.f[jj];
-            pw[2][jj] = p * vn1.f[jj];
-            pw[3][jj] = pw[2][jj] * vr1.f[jj];
-            ps[jj] = p;
-          }
-          l_run = l_run * resc + (ps[0] + ps[1]);       // the lane's own pair; summed over the banks when the segment ends
-          mf_wait_ge(fl_addr + 4u, c >= 2 ? T + (uint32_t)c - 1u : T, a.status, a.spin_limit);
-          // weight operand of pass P (0 = C: sets A0, A1; 1 = S: sets B0, B1): column 4 t + c holds the fp16 part of
-          // set t of query head c, column 8 + 4 t + c its remainder; column k of the tile is read by lane 16 g + k,
-          // whose sixteen bytes are the token pairs 0..3: this lane supplies dword kb of each
-#pragma unroll
-          for (int X = 0; X < 4; ++X) {
-            auto h2 = __builtin_amdgcn_cvt_pkrtz(pw[X][0], pw[X][1]);
-            auto l2 = __builtin_amdgcn_cvt_pkrtz(pw[X][0] - (float)h2[0], pw[X][1] - (float)h2[1]);
-            union { decltype(h2) h; uint32_t u; } hb, lb;
-            hb.h = h2;
-            lb.h = l2;
-            const uint32_t L = (uint32_t)(16 * g + 4 * (X >> 1) + c4);
-            const uint32_t base = ((X & 1) ? wsx(L) + 4096u * par : pbx(L) + MF_XBUF * par) + 4u * (uint32_t)kb;
-            const uint32_t base8 = ((X & 1) ? wsx(L + 8u) + 4096u * par : pbx(L + 8u) + MF_XBUF * par) + 4u * (uint32_t)kb;
-            *(mf_lds_u32*)(uintptr_t)base = hb.u;
-            *(mf_lds_u32*)(uintptr_t)base8 = lb.u;
-          }
-          *(mf_lds_u32*)(uintptr_t)(rsx((uint32_t)lane) + MF_XBUF * par) = __float_as_uint(resc);
-          mf_publish(fl_addr, T + (uint32_t)c + 1u);
-        };
-
-        hm_kraw ra, rb;
-        __builtin_amdgcn_sched_barrier(0);
-        load_chunk(ra, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        load_chunk(rb, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        int c = 0;
-        for (; c + 1 < nchunks; c += 2) {
-          if (c - win_c0 >= MF_WIN) load_window(c);
-          produce(ra, c, 0);
-          produce(rb, c + 1, 1);
-        }
-        if (c < nchunks) produce(ra, c, 0);
-        __builtin_amdgcn_s_waitcnt(MF_WAIT_VM0);
-        T += (uint32_t)nchunks;
-        float lsum = l_run;
-        lsum = akv_banks_sum(mf_rows_sum(lsum));
-        if (col < 4 && g == 0) {
-          const size_t slot = (size_t)(blockIdx.x + s) * a.QH + (h * 4 + col);
-          a.part_ml[slot * 2] = m_run * 0.6931471805599453f;
-          a.part_ml[slot * 2 + 1] = lsum;
-        }
-      } else {
-        // =========================== value wavefront ===========================
-        float4v oC[8], oS[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) { oC[j] = (float4v){0.f, 0.f, 0.f, 0.f}; oS[j] = (float4v){0.f, 0.f, 0.f, 0.f}; }
-        const int m = col;
-        const bool is3 = m < 8;
-        const uint32_t vrow = (uint32_t)(hd * a.vps_head + 4 * g * a.vps_pos);
-        const uint32_t offC = vrow + (is3 ? 4u * (uint32_t)((3 * m) >> 2) : 36u + 4u * (uint32_t)((m - 8) >> 1));
-        const uint32_t offS = vrow + (is3 ? 24u + 4u * (uint32_t)(m >> 2) : 52u + 4u * (uint32_t)((m - 8) >> 2));
-        // pass C pieces as one word: lanes [0,8) the big-endian 24-bit word of 3-byte group m (from the
-        // aligned dword holding its first byte and, where it runs over, the neighbour lane's dword), lanes
-        // [8,16) halfword m - 8 of A1
-        const uint32_t o3 = (uint32_t)(3 * m) & 3u;
-        const uint32_t selC = is3 ? (0x0c000000u | (o3 << 16) | ((o3 + 1u) << 8) | (o3 + 2u))
-                                  : ((m & 1) ? 0x0c0c0302u : 0x0c0c0100u);
-        // ... spread to one code per nibble by five (shift, mask) terms whose constants differ by lane class:
-        // mf_spread3 for the 3-bit lanes; for the 2-bit lanes (shift 0, mask 0x3333) and (shift 14, mask
-        // 0x33330000) do the whole job (nibbles [c3 c1 c7 c5 c2 c0 c6 c4] from bit 0 up) and the levels
-        // 8..11 of the merged table are selected by the constant 8 in every nibble
-        const uint32_t cm0 = is3 ? 0x7007u : 0x3333u, corc = is3 ? 0u : 0x88888888u;
-        const uint32_t cs1 = is3 ? 1u : 14u, cm1 = is3 ? 0x70070u : 0x33330000u;
-        const uint32_t cm2 = is3 ? 0x700700u : 0u, cm3 = is3 ? 0x07000000u : 0u, cm4 = is3 ? 0x70000000u : 0u;
-        const uint32_t selS = 0x0c000c00u | ((4u + (uint32_t)(m & 3)) << 16) | (uint32_t)(m & 3);
-        const uint32_t vtile1 = bs32 ? 16u * (uint32_t)a.vps_pos : 0u;
-        auto load_chunk = [&](hm_vraw& r, int c) {
-          uint32_t pb[2];
-          chunk_blocks(c, pb[0], pb[1]);
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const unsigned char* vb = a.vc + mf_umul(pb[j], (uint32_t)a.vps_blk) + (j ? vtile1 : 0u);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const unsigned char* vr = vb + (uint32_t)(i * (int)a.vps_pos);
-              r.c[4 * j + i] = *(const uint32_t*)(vr + mf_here(offC));
-              r.s[4 * j + i] = *(const uint32_t*)(vr + mf_here(offS));
-            }
-          }
-        };
-        // both constants of (x & mask) | pattern live in registers: as literals they would split the
-        // operation in two
-        uint32_t sgn_mask = 0x80008000u, one_pair = 0x3C003C00u;
-        asm volatile("" : "+v"(sgn_mask));
-        asm volatile("" : "+s"(one_pair));
-        struct hm_vx { uint32_t ce[4], co[4], sg[4]; };   // token pairs: bytes of (high | low) nibbles; sign bytes
-        auto transcode = [&](const hm_vraw& r, hm_vx& x) {
-          uint32_t xc[8];
-#pragma unroll
-          for (int t = 0; t < 8; ++t) {
-            const uint32_t wa = r.c[t];
-            const uint32_t na = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)wa, 0x101 /*row_shl:1*/, 0xf, 0xf, true);
-            const uint32_t w = __builtin_amdgcn_perm(na, wa, selC);
-            uint32_t v = (w & cm0) | corc;
-            v = ((w << cs1) & cm1) | v;
-            v = ((w << 2) & cm2) | v;
-            v = ((w << 15) & cm3) | v;
-            v = ((w << 7) & cm4) | v;
-            xc[t] = v;
-          }
-#pragma unroll
-          for (int p = 0; p < 4; ++p) {
-            x.ce[p] = (xc[2 * p] & 0xF0F0F0F0u) | ((xc[2 * p + 1] >> 4) & 0x0F0F0F0Fu);
-            x.co[p] = ((xc[2 * p] << 4) & 0xF0F0F0F0u) | (xc[2 * p + 1] & 0x0F0F0F0Fu);
-            // the lane's sign byte of token 2p in bits [0,8), of token 2p + 1 in bits [16,24)
-            x.sg[p] = __builtin_amdgcn_perm(r.s[2 * p + 1], r.s[2 * p], selS);
-          }
-        };
-        hm_vraw r;
-        load_chunk(r, 0);
-        for (int c = 0; c < nchunks; ++c) {
-          const uint32_t par = (uint32_t)(c & 1);
-          if (c - win_c0 >= MF_WIN) load_window(c);
-          hm_vx x;
-          transcode(r, x);
-          __builtin_amdgcn_sched_barrier(0);
-          load_chunk(r, c + 1);
-          __builtin_amdgcn_sched_barrier(0);
-          uint32_t wv[8][4];
-#pragma unroll
-          for (int n = 0; n < 8; ++n)
-#pragma unroll
-            for (int p = 0; p < 4; ++p) wv[n][p] = mf_lut(lane4v, (n & 1) ? x.co[p] : x.ce[p], MF_SEL(n >> 1));
-          mf_wait_ge(fl_addr, T + (uint32_t)c + 1u, a.status, a.spin_limit);
-          union { half8 h; mf_u32x4 u; } cv, cs;
-          cv.u = *(mf_lds_u128*)(uintptr_t)(pbx((uint32_t)lane) + MF_XBUF * par);
-          cs.u = *(mf_lds_u128*)(uintptr_t)(wsx((uint32_t)lane) + 4096u * par);
-          const float resc = __uint_as_float(*(mf_lds_cu32*)(uintptr_t)(rsx((uint32_t)(16 * g + (col & 3))) + MF_XBUF * par));
-          mf_publish(fl_addr + 4u, T + (uint32_t)c + 1u);
-          if (__builtin_amdgcn_ballot_w64(resc != 1.f) != 0) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-#pragma unroll
-              for (int i = 0; i < 4; ++i) { oC[j][i] *= resc; oS[j][i] *= resc; }
-          }
-#pragma unroll
-          for (int n = 0; n < 8; ++n)
-            oC[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(mf_pack(wv[n][0], wv[n][1], wv[n][2], wv[n][3]), cv.h, oC[n], 0, 0, 0);
-          // pass S needs no table: fp16 -1 and +1 differ in the sign bit only, so the operand of tile n
-          // (coordinate n of the byte = bit 7 - n) is that bit moved to bits 15 / 31 over the pattern of 1.0
-          // (a set bit reads as -1 here; the sign is turned back with kappa at the end)
-#pragma unroll
-          for (int n = 0; n < 8; ++n) {
-#pragma unroll
-            for (int p = 0; p < 4; ++p) wv[n][p] = ((x.sg[p] << (8 + n)) & sgn_mask) | one_pair;
-            oS[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(mf_pack(wv[n][0], wv[n][1], wv[n][2], wv[n][3]), cs.h, oS[n], 0, 0, 0);
-          }
-        }
-        __builtin_amdgcn_s_waitcnt(MF_WAIT_VM0);
-        T += (uint32_t)nchunks;
-        // columns k and k + 8 carry the two fp16 terms of one weight; lane (column 4 t + q, g) then holds
-        // rows 4g + i of every tile for set t of query head q, and rows [0,8) belong to set 0 (A0 in pass
-        // C, B0 in pass S), rows [8,16) to set 1 (A1, B1)
-        const int t = col >> 2, q = col & 3;
-        const float inv_alpha = 1.f / __uint_as_float(a.lut[MF_W_ALPHA + (t & 1)]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            oC[j][i] = (oC[j][i] + mf_from_hi_cols(oC[j][i])) * inv_alpha;
-            oS[j][i] = (oS[j][i] + mf_from_hi_cols(oS[j][i])) * -a.kappa;
-          }
-        if (col < 8 && (g >= 2) == (t == 1)) {
-          const size_t slot = (size_t)(blockIdx.x + s) * a.QH + (h * 4 + q);
-          float* dst = a.part_acc + slot * 256 + 128 * t + 32 * (g & 1);      // parts A_t | B_t, rows 4 (g & 1) + i
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float v[8], u[8];
-            if (t == 0) {
-#pragma unroll
-              for (int n = 0; n < 8; ++n) v[hm_coord(0, 0, n >> 1, n & 1)] = oC[n][i];
-            } else {
-#pragma unroll
-              for (int n = 0; n < 8; ++n) v[hm_vcoord2(n)] = oC[n][i];
-            }
-#pragma unroll
-            for (int n = 0; n < 8; ++n) u[n] = oS[n][i];
-            *(float4*)(dst + 8 * i) = make_float4(v[0], v[1], v[2], v[3]);
-            *(float4*)(dst + 8 * i + 4) = make_float4(v[4], v[5], v[6], v[7]);
-            *(float4*)(dst + 64 + 8 * i) = make_float4(u[0], u[1], u[2], u[3]);
-            *(float4*)(dst + 64 + 8 * i + 4) = make_float4(u[4], u[5], u[6], u[7]);
-          }
-        }
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(HM_THREADS) void akv_hyb_mfma_kernel(akv_hyb_mfma_args a) {
-  extern __shared__ __align__(16) unsigned char lds_raw[];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  {
-    // thread (entry e, half hf) writes 16 of the entry's 32 copies
-    const int e = threadIdx.x >> 1, hf = threadIdx.x & 1;
-    const uint32_t khi = a.lut[MF_W_KHI + e], klo = a.lut[MF_W_KLO + e], vhi = a.lut[MF_W_VHI + e];
-    uint4* ka = (uint4*)(lds_raw + e * 256 + hf * 128);
-    uint4* va = (uint4*)(lds_raw + MF_TABB + e * 256 + hf * 64);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ka[i] = make_uint4(khi, klo, khi, klo);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) va[i] = make_uint4(vhi, vhi, vhi, vhi);
-  }
-  if (threadIdx.x < HM_HEADS) *(uint2*)(lds_raw + MF_TABB + (32u * threadIdx.x + 12u) * 256u + 128u) = make_uint2(0u, 0u);
-  __syncthreads();
-  if ((wave >> 2) == 0) hm_role_main<0>(a, wave & 3);
-  else hm_role_main<1>(a, wave & 3);
-}
-
-size_t akv_hyb_mfma_extra_bytes(int S, int QH) {
-  return akv_align256((size_t)S * ((QH + 3) / 4) * 16 * 64 * 16);
-}
-
-// rows are dword-aligned (the caller checks); groups of four query heads; blocks of 16 or 32 tokens
-bool akv_hyb_mfma_applicable(int QH, int KVH, int block_size, const int64_t* strides6) {
-  if (mfma_disabled()) return false;
-  const int gqa = QH / KVH;
-  if (gqa % 4 != 0 || (block_size != 16 && block_size != 32)) return false;
-  for (int i = 0; i < 6; ++i)
-    if (strides6[i] < 0 || strides6[i] >= ((int64_t)1 << 27)) return false;
-  return true;
-}
-
-int akv_hyb_mfma_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float kappa,
-                     float scale, akv_hyb_mfma_args a, int block_size, int32_t* prefix, uint32_t* lut, void* extra_ws,
-                     int grid, hipStream_t stream) {
-  a.block_size = block_size;
-  a.hgroup = (a.QH / a.KVH) / 4;
-  a.KVH *= a.hgroup;
-  a.lut = lut;
-  a.qop = (const uint4*)extra_ws;
-  a.prefix = prefix;
-  a.spin_limit = g_spin_limit;
-  const float qscale = scale * 1.4426950408889634f;
-  a.kappa = kappa;
-  const int pgrid = a.S * a.KVH + 2;
-#define HM_PRO(DT) akv_hyb_mfma_prologue_kernel<DT><<<pgrid, 256, 0, stream>>>(query, qs_seq, qs_head, table, kappa, qscale, a.S, a.QH, a.KVH, a.context_lens, a.cl_itype, block_size, a.max_blocks_per_seq, prefix, (uint4*)a.qop, (uint32_t*)a.lut, a.status)
-  if (q_dtype == AKV_F16) HM_PRO(AKV_F16); else if (q_dtype == AKV_BF16) HM_PRO(AKV_BF16); else HM_PRO(AKV_F32);
-#undef HM_PRO
-  AKV_LAUNCH_CHECK("akv_hyb_mfma_prologue_kernel");
-  static bool configured = false;
-  if (!configured) {
-    AKV_HIP(hipFuncSetAttribute((const void*)akv_hyb_mfma_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, HM_LDS_BYTES));
-    configured = true;
-  }
-  AKV_LAUNCH_TIMED(akv_hyb_mfma_kernel, grid, HM_THREADS, HM_LDS_BYTES, stream, a);
-  AKV_LAUNCH_CHECK("akv_hyb_mfma_kernel");
   return AKV_OK;
 }

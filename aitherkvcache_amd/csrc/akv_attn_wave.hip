@@ -264,26 +264,11 @@ __device__ __forceinline__ aw_half8 aw_operand(aw_u32x2 a, aw_u32x2 b) {
 __device__ __forceinline__ float aw_add_cols(float v) {
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128 /*row_ror:8*/, 0xf, 0xf, false));
 }
-__device__ __forceinline__ float aw_rows_sum(float v) {
-  auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
 // (keeps the widening of a 32-bit lane offset next to its load: scalar base + 32-bit lane offset)
 __device__ __forceinline__ uint32_t aw_here(uint32_t v) {
   asm volatile("" : "+v"(v));
   return v;
 }
-__device__ __forceinline__ void aw_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// workgroup barrier that orders LDS traffic only (what has been requested from memory keeps flying)
-__device__ __forceinline__ void aw_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // 3-bit codes: a group of eight is a big-endian word of 24 bits.  Its four fields of two codes each, one per byte (the first
 // field in byte 3); and the same for two half groups of twelve bits in the halves of a word (first field in byte 1 and 3).
 __device__ __forceinline__ uint32_t aw_spread12(uint32_t x) { return ((x << 2) & 0x3F003F00u) | (x & 0x003F003Fu); }
@@ -356,7 +341,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
     const uint32_t e = threadIdx.x / TPE, at = e * 256u + threadIdx.x % TPE * (256u / TPE);
 #pragma unroll
     for (uint32_t i = 0; i < 16 / TPE; ++i) *(aw_lds_u128*)(uintptr_t)(at + (i + e) % (16u / TPE) * 16u) = (aw_u32x4){hi, lo, hi, lo};
-    aw_lds_barrier();
+    akv_lds_barrier();
   };
   if constexpr (D != 128) fill_once();
 
@@ -521,7 +506,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
             const int e = (int)((__float_as_uint(nrm) >> 23) & 0xffu) - 126;
             *(aw_lds_f32*)(uintptr_t)(nbase + 256u + (uint32_t)ntok * 4u) = (float)max(e, -AW_TINY);
           }
-          aw_wave_sync();
+          akv_wave_sync();
 
           // ---- scores
           aw_float4 acc[2];
@@ -623,7 +608,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           } else {
             mx = akv_banks_max(mx);
           }
-          aw_wave_sync();      // the norms have been read: the next chunk overwrites them
+          akv_wave_sync();      // the norms have been read: the next chunk overwrites them
           mx = akv_rows_max(mx);
           const float m_new = fmaxf(m_run, mx - AW_FRAME);
           const float resc = __builtin_amdgcn_exp2f(m_run - m_new);      // 0 on the first chunk
@@ -731,7 +716,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           load_values(min(k + 1, mine - 1));
           __builtin_amdgcn_sched_barrier(0);
         }
-        l_run = aw_rows_sum(l_run);      // (every lane of a row had its own tokens)
+        l_run = akv_rows_sum(l_run);      // (every lane of a row had its own tokens)
         if constexpr (PACK == 4) l_run = akv_banks_sum(l_run);
         else l_run = aw_add_cols(l_run);
       } else {
@@ -744,7 +729,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
       const int shares = min(R, nchunks);      // wavefronts of the head that hold a result
       if (shares > 1) {
         if (lane < 8) *(aw_lds_f64*)(uintptr_t)(aw_ml_off<W>() + (uint32_t)wave * 64u + (uint32_t)lane * 8u) = (aw_float2){m_run, l_run};
-        aw_lds_barrier();
+        akv_lds_barrier();
         // (AT requested at a time, at 128 and 256 all there can be; past the last share that one again, for nothing)
         constexpr int AT = D == 64 ? 4 : W;
         const int rounds = D == 64 ? shares : 1;
@@ -791,7 +776,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
             for (int n = 0; n < CPL; n += 4)
               *(aw_lds_f128*)(uintptr_t)(at + (uint32_t)(CPL * i + n) * 4u) = (aw_float4){o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]};
         }
-        aw_lds_barrier();
+        akv_lds_barrier();
         if (active) {
           // (no barrier after these reads: the next segment's accumulators are written behind its first barrier)
           for (int idx = r * 64 + lane; idx < gqa * D / 4; idx += R * 64) {

@@ -722,7 +722,7 @@ extern "C" int akv_hybrid_decode(const uint8_t* packed, int64_t packed_stride_by
 extern "C" size_t akv_hybrid_paged_attn_workspace_bytes(int num_seqs, int num_q_heads) {
   if (num_seqs < 0 || num_q_heads <= 0) return 0;
   return akv_attn_ws_layout(nullptr, num_seqs, num_q_heads, 256, akv_attn_grid()).bytes +
-         akv_hyb_mfma_extra_bytes(num_seqs, num_q_heads);
+         akv_attn_hyb_extra_bytes(num_seqs, num_q_heads);
 }
 
 template <int GQ>
@@ -765,29 +765,23 @@ extern "C" int akv_hybrid_paged_attn(
   const int G = akv_attn_grid();
   AKV_REQUIRE(workspace != nullptr && ((uintptr_t)workspace & 255) == 0, "akv_hybrid_paged_attn: workspace null or not 256-byte aligned");
   akv_attn_ws ws = akv_attn_ws_layout(workspace, num_seqs, num_q_heads, 256, G);
-  const size_t need = ws.bytes + akv_hyb_mfma_extra_bytes(num_seqs, num_q_heads);
+  const size_t need = ws.bytes + akv_attn_hyb_extra_bytes(num_seqs, num_q_heads);
   if (workspace_bytes < need)
     return akv_fail(AKV_ERR_WORKSPACE, "akv_hybrid_paged_attn: workspace %zu < %zu bytes", workspace_bytes, need);
 
   // groups of four query heads over blocks of 16 or 32 tokens: the matrix-core kernel
   const int64_t strides6[6] = {kps_blk, kps_pos, kps_head, vps_blk, vps_pos, vps_head};
-  const int rgrid = num_seqs * num_q_heads;
-  int Gused = G;
-  if (max_blocks_per_seq > 0 && akv_hyb_mfma_applicable(num_q_heads, num_kv_heads, block_size, strides6)) {
-    akv_hyb_mfma_args m;
+  if (max_blocks_per_seq > 0 && num_blocks < ((int64_t)1 << 31) && akv_attn_hyb_applicable(block_size, strides6)) {
+    akv_hyb_attn_args m;
     m.kc = k_cache; m.kps_blk = kps_blk; m.kps_pos = kps_pos; m.kps_head = kps_head;
     m.vc = v_cache; m.vps_blk = vps_blk; m.vps_pos = vps_pos; m.vps_head = vps_head;
     m.block_tables = block_tables; m.bt_itype = bt_itype; m.bt_stride = bt_stride;
     m.context_lens = context_lens; m.cl_itype = cl_itype;
-    m.S = num_seqs; m.QH = num_q_heads; m.KVH = num_kv_heads; m.hgroup = 1; m.block_size = block_size;
+    m.S = num_seqs; m.QH = num_q_heads; m.KVH = num_kv_heads; m.block_size = block_size;
     m.max_blocks_per_seq = max_blocks_per_seq; m.num_blocks = num_blocks;
-    m.prefix = ws.prefix; m.lut = nullptr; m.qop = nullptr; m.status = ws.status; m.spin_limit = 0;
-    m.part_acc = ws.part_acc; m.part_ml = ws.part_ml;
-    Gused = G / AKV_ATTN_WG_PER_CU;      // one workgroup per CU (its tables fill most of the LDS)
-    const int rc = akv_hyb_mfma_run(query, q_dtype, qs_seq, qs_head, hyb_table, kHybKappa, scale, m, block_size,
-                                    ws.prefix, ws.lut, (char*)workspace + ws.bytes, Gused, stream);
-    if (rc) return rc;
-  } else {
+    return akv_attn_hyb_run(query, q_dtype, qs_seq, qs_head, hyb_table, scale, m, ws, (char*)workspace + ws.bytes, out, out_dtype,
+                            os_seq, os_head, stream);
+  }
 
   const int nblocks_q = (num_seqs * num_q_heads + 3) / 4;
 #define HYB_PRO(DT) hyb_attn_prologue_kernel<DT><<<nblocks_q + 1, 256, 0, stream>>>(query, qs_seq, qs_head, hyb_table, kHybKappa, num_seqs, num_q_heads, context_lens, cl_itype, block_size, max_blocks_per_seq, ws.prefix, ws.qrot, nblocks_q, ws.status)
@@ -804,13 +798,13 @@ extern "C" int akv_hybrid_paged_attn(
   a.max_blocks_per_seq = max_blocks_per_seq; a.num_blocks = num_blocks; a.scale = scale; a.kappa = kHybKappa;
   a.prefix = ws.prefix; a.qt = ws.qrot; a.part_acc = ws.part_acc; a.part_ml = ws.part_ml;
   const int gqa = num_q_heads / num_kv_heads;
-  int rc = (gqa % 4 == 0) ? hyb_launch_attn<4>(a, G, stream) : hyb_launch_attn<1>(a, G, stream);
+  const int rgrid = num_seqs * num_q_heads;
+  const int rc = (gqa % 4 == 0) ? hyb_launch_attn<4>(a, G, stream) : hyb_launch_attn<1>(a, G, stream);
   if (rc) return rc;
-  }
   switch (out_dtype) {
-    case AKV_F16: hyb_attn_reduce_kernel<AKV_F16><<<rgrid, 64, 0, stream>>>(ws.prefix, ws.part_acc, ws.part_ml, hyb_table, num_seqs, num_q_heads, Gused, out, os_seq, os_head, ws.status); break;
-    case AKV_BF16: hyb_attn_reduce_kernel<AKV_BF16><<<rgrid, 64, 0, stream>>>(ws.prefix, ws.part_acc, ws.part_ml, hyb_table, num_seqs, num_q_heads, Gused, out, os_seq, os_head, ws.status); break;
-    default: hyb_attn_reduce_kernel<AKV_F32><<<rgrid, 64, 0, stream>>>(ws.prefix, ws.part_acc, ws.part_ml, hyb_table, num_seqs, num_q_heads, Gused, out, os_seq, os_head, ws.status); break;
+    case AKV_F16: hyb_attn_reduce_kernel<AKV_F16><<<rgrid, 64, 0, stream>>>(ws.prefix, ws.part_acc, ws.part_ml, hyb_table, num_seqs, num_q_heads, G, out, os_seq, os_head, ws.status); break;
+    case AKV_BF16: hyb_attn_reduce_kernel<AKV_BF16><<<rgrid, 64, 0, stream>>>(ws.prefix, ws.part_acc, ws.part_ml, hyb_table, num_seqs, num_q_heads, G, out, os_seq, os_head, ws.status); break;
+    default: hyb_attn_reduce_kernel<AKV_F32><<<rgrid, 64, 0, stream>>>(ws.prefix, ws.part_acc, ws.part_ml, hyb_table, num_seqs, num_q_heads, G, out, os_seq, os_head, ws.status); break;
   }
   AKV_LAUNCH_CHECK("hyb_attn_reduce_kernel");
   return AKV_OK;

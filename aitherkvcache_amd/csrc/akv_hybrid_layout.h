@@ -36,27 +36,19 @@ __device__ __forceinline__ float hyb_fwht64(float v, int lane) {
   return v;
 }
 
-// matrix-core attention on tq35 rows (akv_attn_mfma.hip)
-struct akv_hyb_mfma_args {
+// matrix-core attention on hybrid rows (akv_attn_hyb.hip)
+struct akv_attn_ws;
+struct akv_hyb_attn_args {
   const uint8_t* kc; int64_t kps_blk, kps_pos, kps_head;
   const uint8_t* vc; int64_t vps_blk, vps_pos, vps_head;
   const void* block_tables; int bt_itype; int64_t bt_stride;
   const void* context_lens; int cl_itype;
-  int S, QH, KVH, hgroup, block_size;      // KVH counts groups of four query heads; hgroup of them share a kv head's rows
+  int S, QH, KVH, block_size;
   int64_t max_blocks_per_seq;
   int64_t num_blocks;          // physical blocks in the cache; table entries are clamped into [0, num_blocks)
-  const int32_t* prefix;
-  uint32_t* status;            // status words of the call (workspace header)
-  int spin_limit;              // polls a hand-off wait makes before it gives up
-  const uint32_t* lut;         // table block, MF_W_*
-  const uint4* qop;            // [S][KVH][16 k-steps][64 lanes] half8
-  float* part_acc;             // [G + S][QH][256]: A0 | B0 | A1 | B1, natural coordinate order
-  float* part_ml;
-  float kappa;                 // sqrt(pi/2)/64, applied to the sign sums
 };
-
-size_t akv_hyb_mfma_extra_bytes(int S, int QH);
-bool akv_hyb_mfma_applicable(int QH, int KVH, int block_size, const int64_t* strides6);
-int akv_hyb_mfma_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float kappa,
-                     float scale, akv_hyb_mfma_args a, int block_size, int32_t* prefix, uint32_t* lut, void* extra_ws,
-                     int grid, hipStream_t stream);
+size_t akv_attn_hyb_extra_bytes(int S, int QH);
+bool akv_attn_hyb_applicable(int block_size, const int64_t* strides6);
+int akv_attn_hyb_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float scale,
+                     const akv_hyb_attn_args& in, const akv_attn_ws& ws, void* extra_ws, void* out, int out_dtype, int64_t os_seq,
+                     int64_t os_head, hipStream_t stream);

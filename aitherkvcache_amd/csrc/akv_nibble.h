@@ -6,8 +6,7 @@
 #include <hip/hip_runtime.h>
 
 // Code order after spreading.  Row side (K rows of attention, rows of decode): spread dword st (0..3)
-// of lane g, byte b, nibble `lo` (0 = high nibble) -> coordinate inside the lane's 32.  V side of
-// attention: M-tile n of the value product <-> coordinate inside the lane's 8.
+// of lane g, byte b, nibble `lo` (0 = high nibble) -> coordinate inside the lane's 32.
 template <int BITS>
 __host__ __device__ constexpr int mf_kcoord(int st, int b, int lo) {
   if (BITS == 4) return 8 * st + 2 * b + lo;
@@ -15,13 +14,6 @@ __host__ __device__ constexpr int mf_kcoord(int st, int b, int lo) {
   // 3-bit: bytes (c6,c7) (c3,c5) (c1,c2) (c0,c4) of each group of eight codes (see mf_spread3)
   constexpr int hi3[4] = {6, 3, 1, 0}, lo3[4] = {7, 5, 2, 4};
   return 8 * st + (lo ? lo3[b] : hi3[b]);
-}
-template <int BITS>
-__host__ __device__ constexpr int mf_vtile_of_coord(int k) {
-  if (BITS == 4) return k;
-  if (BITS == 2) { constexpr int inv[8] = {2, 3, 0, 1, 6, 7, 4, 5}; return inv[k]; }
-  constexpr int inv[8] = {6, 4, 5, 2, 7, 3, 0, 1};
-  return inv[k];
 }
 // eight 3-bit codes c0..c7 (c0 in bits 23:21 of w) -> nibbles [c7 c6 c5 c3 c2 c1 c4 c0] from bit 0 up
 __device__ __forceinline__ uint32_t mf_spread3(uint32_t w) {
@@ -32,14 +24,6 @@ __device__ __forceinline__ uint32_t mf_spread3(uint32_t w) {
   t = ((w << 7) & 0x70000000u) | t;
   return t;
 }
-// eight 2-bit codes in a halfword (byte 0 = c0..c3 from the top bits) -> bytes (c2,c3) (c0,c1) (c6,c7) (c4,c5)
-__device__ __forceinline__ uint32_t mf_spread2(uint32_t h) {
-  uint32_t t = (h | (h << 8)) & 0x00FF00FFu;
-  t = (t | (t << 4)) & 0x0F0F0F0Fu;
-  t = (t | (t << 2)) & 0x33333333u;
-  return t;
-}
-
 // the lane's quarter of a packed row (32 codes: 16 / 12 / 8 bytes in w[0..3] / w[0..2] / w[0..1]) as four
 // nibble dwords; dword st, byte b, nibble lo holds coordinate mf_kcoord<BITS>(st, b, lo) of the 32
 template <int BITS>

@@ -230,15 +230,13 @@ int akv_paged_attn_static(const void* query, int q_dtype, int64_t qs_seq, int64_
                           void* stream);
 
 /* Status of the most recent akv_paged_attn / akv_hybrid_paged_attn call that used `workspace`
- * (no counterpart in the reference).  Inside the main kernel pairs of wavefronts hand chunks to
- * each other through counters with BOUNDED waits, so that a kernel always finishes; a wait
- * that gives up marks the call, whose outputs are then all NaN.  This waits for `stream` and
- * copies the mark to *flags (host pointer): 0 = clean, bit 0 = a hand-off wait gave up.
+ * (no counterpart in the reference): 0 in *flags (host pointer) = clean, bit 0 = a bounded wait inside a kernel gave
+ * up; the outputs of such a call are all NaN.  This waits for `stream`.  (No kernel of this library waits inside any more.)
  * workspace == NULL asks about the most recent akv_paged_attn_static call on the current device
  * (0 when there has been none).
- * akv_debug_set_handoff_spin_limit changes the number of polls such a wait makes (negative =
- * the default, 65536); it exists so that a test can exercise the failure path from the host
- * (0 polls: every wait gives up at once, every kernel still runs to its end).  The akv_debug_* and
+ * akv_debug_set_handoff_spin_limit sets the number of polls such a wait makes (negative = the default).  It exists so that
+ * a test can exercise the failure path from the host: with 0 an akv_hybrid_paged_attn call on tq35 rows reports a failure,
+ * every kernel runs to its end.  The akv_debug_* and
  * akv_profile_* switches are process-global words read at each launch and are not synchronised: set them
  * from one thread while no call of another thread is being issued. */
 int akv_paged_attn_status(const void* workspace, int* flags, void* stream);

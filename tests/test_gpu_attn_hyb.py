@@ -1,0 +1,127 @@
+"""Hybrid paged attention whose wavefronts work on their own, at the edges of its tiles, chunks, head groups, alignments and
+block-id windows, against float64 over the decoded rows."""
+import numpy as np
+import pytest
+import torch
+
+import aitherkvcache_amd as akv
+from tests.util import kv_like
+
+pytestmark = pytest.mark.gpu
+
+# float32 outputs.  Head counts that are no multiple of four a kv head: the rounding of some float32 sums and exponentials, as
+# in the vector kernel (measured up to 2e-6).  Groups of four: float16 levels of values, 2.9e-5 of a level (measured 7e-5).
+EXACT, LEVELS = 6e-6, 2e-4
+
+
+def limit(qh, kvh):
+    return LEVELS if qh // kvh % 4 == 0 else EXACT
+
+
+def make(dev, mode, kvh, blocks, bs, pitch, seed, scale=(1.0, 1.0)):
+    rng = np.random.default_rng(seed)
+    h = akv.HybridTurboQuant(head_dim=128, mode=mode, device=str(dev))
+    h.calibrate_uniform(kvh)
+    rows = []
+    for i in range(2):
+        r = torch.full((blocks, bs, kvh, pitch), 0x5A, dtype=torch.uint8, device=dev)
+        x = torch.from_numpy((scale[i] * kv_like(rng, (blocks * bs, kvh, 128))).astype(np.float32)).to(dev)
+        akv.hybrid_encode_and_store(h, x, torch.arange(blocks * bs, device=dev), r, bs)
+        rows.append(r[..., :h.packed_dim])
+    return rng, h, rows
+
+
+def attend(q, K, V, counts=None):
+    """q [heads, d], K and V [tokens, kv heads, d], each token `counts` times; float64."""
+    heads, kvh = q.shape[0], K.shape[1]
+    out = torch.zeros_like(q)
+    for i in range(heads):
+        s = K[:, i // (heads // kvh)] @ q[i] / 128 ** 0.5
+        p = torch.exp(s - s.max()) * (1.0 if counts is None else counts)
+        out[i] = p @ V[:, i // (heads // kvh)] / p.sum()
+    return out
+
+
+@pytest.mark.parametrize("mode,pitch", [("tq35", 64), ("tq35", 68)])
+@pytest.mark.parametrize("qh,kvh,bs", [(4, 1, 16), (8, 1, 32), (8, 2, 16), (12, 3, 32), (20, 5, 16), (32, 8, 16), (3, 1, 16), (10, 2, 32), (21, 3, 16),
+                                       (7, 7, 32), (18, 2, 16)])
+def test_edges_vs_float64(dev, mode, pitch, qh, kvh, bs):
+    ctx = np.array([1, 0, 15, 16, 17, 31, 32, 33, 64, 65, 257, 1000, 0, 3], dtype=np.int32)
+    need = -(-ctx // bs)
+    blocks = int(need.sum()) + 2
+    rng, h, rows = make(dev, mode, kvh, blocks, bs, pitch, qh + bs)
+    tables = np.full((len(ctx), int(need.max())), 10 ** 6, dtype=np.int32)
+    order, at = rng.permutation(blocks), 0
+    for i, n in enumerate(need):
+        tables[i, :n] = order[at:at + n]
+        at += int(n)
+    K, V = (h.decode(r.contiguous()).double().cpu() for r in rows)
+    for i, n in enumerate(ctx):                        # rows that no context covers may hold anything: here float16 NaN factors
+        if n % bs:
+            for r in rows:
+                r[int(tables[i, need[i] - 1]), int(n) % bs:] = 0xFF
+    q = torch.from_numpy(rng.standard_normal((len(ctx), qh, 128)).astype(np.float32)).to(dev)
+    print(f"[attn hyb] {mode} pitch={pitch} qh={qh} kvh={kvh} bs={bs}", flush=True)
+    out = akv.HybridPagedAttention(h, qh).forward(q, rows[0], rows[1], torch.from_numpy(tables).to(dev), torch.from_numpy(ctx).to(dev),
+                                                  block_size=bs).double().cpu()
+    for i, n in enumerate(ctx):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        t = torch.from_numpy(tables[i, :need[i]].astype(np.int64))
+        k, v = (x[t].reshape(-1, kvh, 128)[:n] for x in (K, V))
+        ref = attend(q[i].double().cpu(), k, v)
+        assert (out[i] - ref).norm() <= limit(qh, kvh) * ref.norm(), (i, n, float((out[i] - ref).norm() / ref.norm()))
+
+
+@pytest.mark.parametrize("mode", ["tq35"])
+@pytest.mark.parametrize("qh,kvh,bs,chunks", [(16, 16, 16, 70), (48, 12, 32, 33), (4, 1, 16, 32)])
+def test_more_chunks_than_a_window_of_block_ids(dev, mode, qh, kvh, bs, chunks):
+    """A context so long that a wavefront goes through several windows of block ids, of 32 chunks each; its blocks repeat a few,
+    which the reference counts."""
+    rng, h, rows = make(dev, mode, kvh, 8, bs, h_pitch(mode), 7)
+    groups = kvh * (-(-(qh // kvh) // 4))
+    ranges, shares = (512, 4) if groups == 1 else (min(512, 768 // (-(-groups // 4))), 1)
+    n = 32 * chunks * ranges * shares - 5
+    table = rng.integers(0, 8, size=-(-n // bs)).astype(np.int32)
+    q = torch.from_numpy(rng.standard_normal((1, qh, 128)).astype(np.float32)).to(dev)
+    out = akv.HybridPagedAttention(h, qh).forward(q, rows[0], rows[1], torch.from_numpy(table[None]).to(dev),
+                                                  torch.tensor([n], dtype=torch.int32, device=dev), block_size=bs).double().cpu()
+    counts = np.zeros((8, bs))
+    np.add.at(counts, table[:-1], 1.0)
+    counts[table[-1], :n - (len(table) - 1) * bs] += 1.0
+    K, V = (h.decode(r.contiguous()).double().cpu().reshape(-1, kvh, 128) for r in rows)
+    ref = attend(q[0].double().cpu(), K, V, torch.from_numpy(counts.reshape(-1)))
+    # sums of 2^17 and more float32 terms: their rounding walks to a few times that of short contexts
+    assert (out[0] - ref).norm() <= max(limit(qh, kvh), 4 * EXACT) * ref.norm(), float((out[0] - ref).norm() / ref.norm())
+
+
+def h_pitch(mode):
+    return 64 if mode == "tq35" else 44
+
+
+@pytest.mark.parametrize("mode", ["tq35"])
+@pytest.mark.parametrize("qh,kvh", [(8, 2), (6, 2)])
+@pytest.mark.parametrize("scale_k,scale_v,scale_q", [(1.0, 3e2, 1.0), (1.0, 1e-3, 1.0), (1e-2, 1.0, 1e2), (1e2, 1.0, 1e-30), (1e-2, 1.0, 1e4)])
+def test_factors_and_queries_far_from_one(dev, mode, qh, kvh, scale_k, scale_v, scale_q):
+    """Value factors near both ends of float16, queries far outside it, scores of hundreds (one token takes all)."""
+    rng, h, rows = make(dev, mode, kvh, 8, 16, h_pitch(mode), 3, (scale_k, scale_v))
+    n = 100
+    q = torch.from_numpy((scale_q * rng.standard_normal((1, qh, 128))).astype(np.float32)).to(dev)
+    out = akv.HybridPagedAttention(h, qh).forward(q, rows[0], rows[1], torch.arange(8, dtype=torch.int32, device=dev)[None],
+                                                  torch.tensor([n], dtype=torch.int32, device=dev)).double().cpu()
+    K, V = (h.decode(r.contiguous()).double().cpu().reshape(-1, kvh, 128)[:n] for r in rows)
+    ref = attend(q[0].double().cpu(), K, V)
+    # scores of some hundreds carry 2^-22 of themselves into their exponentials
+    assert (out[0] - ref).norm() <= max(limit(qh, kvh), 5e-4 if scale_q == 1e4 else 0.0) * ref.norm(), float((out[0] - ref).norm() / ref.norm())
+
+
+def test_queries_that_are_no_numbers_stay_in_their_head(dev):
+    rng, h, rows = make(dev, "tq35", 2, 8, 16, 64, 5)
+    q = torch.from_numpy(rng.standard_normal((1, 8, 128)).astype(np.float32)).to(dev)
+    args = (rows[0], rows[1], torch.arange(8, dtype=torch.int32, device=dev)[None], torch.tensor([90], dtype=torch.int32, device=dev))
+    good = akv.HybridPagedAttention(h, 8).forward(q, *args)
+    q[0, 1, 5], q[0, 6, 127] = float("nan"), float("inf")
+    bad = akv.HybridPagedAttention(h, 8).forward(q, *args)
+    for i in range(8):
+        assert bool(torch.isnan(bad[0, i]).all()) if i in (1, 6) else torch.equal(bad[0, i], good[0, i])
