@@ -1,4 +1,4 @@
-// Paged decode attention on hybrid rows (tq35), on the matrix cores, every wavefront on its own.
+// Paged decode attention on hybrid rows (tq35 and tq25), on the matrix cores, every wavefront on its own.
 //
 // A row holds four parts: A0 and A1, codes of the two coordinate groups, and B0 and B1, the signs of their residuals; a decoded
 // group is n (Inv_had(c[code]) + r kappa Inv_qjl(sign)) with two float16 factors n, r per group (akv_hybrid_layout.h).  With
@@ -26,6 +26,8 @@
 // 64 sequences of 4,000 to 8,192 tokens, 32 heads on 8: 160 | 211 us; 256 of 64 to 512: 82 | 111; 64 of 300: 45 | 54; 4 of 300:
 // 29 | 38; 32 of 1,000 to 9,000 with 64 heads on 8: 130 | 188, 8 on 1: 42 | 61.  Head counts that are no multiple of four a kv
 // head (levels of float32's accuracy, see hw35) | the vector kernel: 28 on 4: 107 | 570; 16 on 16: 166 | 238.
+// tq25 rows | the vector kernel (tables of partial products in LDS): 64 of 4,000 to 8,192, 32 heads on 8: 160 | 335; 256 of 64 to
+// 512: 88 | 114; 32 of 1,000 to 9,000 with 8 heads on 1: 43 | 246, 28 on 4: 78 | 278, 16 on 16: 130 | 144; 4 of 300: the same.
 #include <type_traits>
 
 #include "akv_attn_common.h"
@@ -40,6 +42,8 @@ typedef int hw_int2 __attribute__((ext_vector_type(2)));
 typedef int hw_int4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const uint32_t hw_lds_cu32;
 typedef __attribute__((address_space(3))) const uint16_t hw_lds_cu16;
+typedef __attribute__((address_space(3))) const uint8_t hw_lds_cu8;
+typedef __attribute__((address_space(3))) const long hw_lds_l64;
 typedef __attribute__((address_space(3))) uint32_t hw_lds_u32;
 typedef __attribute__((address_space(3))) hw_int2 hw_lds_i64;
 typedef __attribute__((address_space(3))) float hw_lds_f32;
@@ -81,8 +85,10 @@ static_assert(HW_LDS <= 52 * 1024, "three workgroups a CU, whatever the granular
 #define HW_W_UNITP 31
 #define HW_W_TAG 768
 #define HW_W_MARK 784
-#define HW_MARK 0x48570023u
-constexpr float kHwKappa = (float)(1.2533141373155001 / 64.0);      // sqrt(pi/2) / 64
+#define HW_W_DELTA 33          // tq25: half the distance of the two levels of a 1-bit code, and their middle
+#define HW_W_MIDDLE 34
+#define HW_MARK 0x48570000u    // plus the format
+#define HW_VALUES 2048u        // of a chunk buffer: the value rows
 
 struct hw_args {
   const uint8_t* kc; int64_t kps_blk, kps_pos, kps_head;
@@ -123,6 +129,22 @@ template <int N> __device__ __forceinline__ void hw_request(const uint8_t* base,
 }
 __device__ __forceinline__ void hw_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// float16 levels of the codes of four tokens, low and high bytes: tokens 0 and 2, tokens 1 and 3
+__device__ __forceinline__ void hw_expand(uint32_t low, uint32_t high, uint32_t& e, uint32_t& o) {
+  e = __builtin_amdgcn_perm(high, low, 0x06020400u);
+  o = __builtin_amdgcn_perm(high, low, 0x07030501u);
+}
+// signs of four tokens, bit 7 - t of their bytes: 1.0 where it is clear, -1.0 where it is set
+__device__ __forceinline__ void hw_signs(uint32_t w, int t, uint32_t& e, uint32_t& o) {
+  e = hw_and_or(w << (8 + t), 0x80008000u, 0x3C003C00u);
+  o = hw_and_or(w << t, 0x80008000u, 0x3C003C00u);
+}
+// value of the lane four columns up in the row of sixteen, added (columns 0..3)
+__device__ __forceinline__ float hw_add_four(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104 /*row_shl:4*/, 0xf, 0xf, false));
+}
+__device__ __forceinline__ long hw_as_long(uint32_t a, uint32_t b) { return (long)((uint64_t)a | ((uint64_t)b << 32)); }
+
 // ----------------------------------------------------------------------------------
 // tq35 rows
 // ----------------------------------------------------------------------------------
@@ -135,6 +157,8 @@ __device__ __forceinline__ int hw35_kcoord(int part, int g, int r, int b) {
 
 // P: for float32's accuracy -- levels of keys in three digits, of values in two float16 terms
 template <bool P> struct hw35 {
+  static constexpr uint32_t MARK = HW_MARK + 35;
+  static constexpr float KAPPA = (float)(1.2533141373155001 / 64.0);         // sqrt(pi/2) / 64
   static constexpr int KD = P ? 3 : 2;       // digits of a level
   static constexpr int TILE = 1024;          // bytes of sixteen rows in LDS
   static constexpr int NT = 18;              // value tiles: A0 of bytes 0..15 (3), of 16..23 (3), A1 (4), B0 (4), B1 (4)
@@ -159,7 +183,7 @@ template <bool P> struct hw35 {
     b1 = buf + at(col, 52u + 2u * g);
     // lane 2 r + h of a row of sixteen supplies half h of a window of token r: tokens 4 g .. 4 g + 3 of tile 0, then of tile 1
     const uint32_t r = col >> 1, row = 4u * g + (r & 3u);
-    tr = buf + 2 * TILE + (r >> 2) * TILE + row * 64u + (col & 1u) * 8u + (g << 4);
+    tr = buf + HW_VALUES + (r >> 2) * TILE + row * 64u + (col & 1u) * 8u + (g << 4);
 #pragma unroll
     for (int i = 0; i < 2 * KD; ++i) ka0[i] = lut[(P ? HW_W_KP0 : HW_W_KA0) + i];
 #pragma unroll
@@ -197,6 +221,7 @@ template <bool P> struct hw35 {
       }
     }
   }
+  __device__ __forceinline__ void start(uint32_t) {}
   // the dword of factors of group `group` of row `row`
   static __device__ __forceinline__ uint32_t factors(uint32_t row, int group) { return at(row, group ? 60u : 32u); }
   static __device__ __forceinline__ uint32_t look8(uint32_t t0, uint32_t t1, uint32_t sel) { return __builtin_amdgcn_perm(t1, t0, sel); }
@@ -284,16 +309,6 @@ template <bool P> struct hw35 {
     }
   }
 
-  // float16 levels of the codes of four tokens: tokens 0 and 2, tokens 1 and 3
-  static __device__ __forceinline__ void expand(uint32_t low, uint32_t high, uint32_t& e, uint32_t& o) {
-    e = __builtin_amdgcn_perm(high, low, 0x06020400u);
-    o = __builtin_amdgcn_perm(high, low, 0x07030501u);
-  }
-  // signs of four tokens, bit 7 - t of their bytes: 1.0 where it is clear, -1.0 where it is set
-  static __device__ __forceinline__ void signs(uint32_t w, int t, uint32_t& e, uint32_t& o) {
-    e = hw_and_or(w << (8 + t), 0x80008000u, 0x3C003C00u);
-    o = hw_and_or(w << t, 0x80008000u, 0x3C003C00u);
-  }
   template <class W> __device__ __forceinline__ void values(uint32_t keys, W weights, hw_float4 (&o)[NT]) const {
     hw_int2 win[4];
 #pragma unroll
@@ -333,7 +348,7 @@ template <bool P> struct hw35 {
             uint32_t a[4];
             const uint32_t* lv = va0 + 4 * term;
 #pragma unroll
-            for (int d = 0; d < 2; ++d) expand(look8(lv[0], lv[1], sel[i][d]), look8(lv[2], lv[3], sel[i][d]), a[2 * d], a[2 * d + 1]);
+            for (int d = 0; d < 2; ++d) hw_expand(look8(lv[0], lv[1], sel[i][d]), look8(lv[2], lv[3], sel[i][d]), a[2 * d], a[2 * d + 1]);
             product(3 * part + i, w, a);
           }
       }
@@ -353,7 +368,7 @@ template <bool P> struct hw35 {
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
           const uint32_t c = (b1w[d] >> (6 - 2 * i)) & 0x03030303u;
-          expand(__builtin_amdgcn_perm(lv[0], lv[0], c), __builtin_amdgcn_perm(lv[1], lv[1], c), a[2 * d], a[2 * d + 1]);
+          hw_expand(__builtin_amdgcn_perm(lv[0], lv[0], c), __builtin_amdgcn_perm(lv[1], lv[1], c), a[2 * d], a[2 * d + 1]);
         }
         product(6 + i, wa1, a);
       }
@@ -372,7 +387,7 @@ template <bool P> struct hw35 {
       for (int i = 0; i < 4; ++i) {
         uint32_t a[4];
 #pragma unroll
-        for (int d = 0; d < 2; ++d) signs(w[d], i, a[2 * d], a[2 * d + 1]);
+        for (int d = 0; d < 2; ++d) hw_signs(w[d], i, a[2 * d], a[2 * d + 1]);
         product(10 + 4 * x + i, wb, a);
       }
     }
@@ -401,25 +416,263 @@ template <bool P> struct hw35 {
   }
   // constants of the factors: (n0, n0 r0, n1, n1 r1) times these on the score side
   static __device__ __forceinline__ hw_float4 kscale(const uint32_t* lut) {
-    const float sign = -kHwKappa / 64.f;
+    const float sign = -KAPPA / 64.f;
     const int u = P ? HW_W_UNITP : HW_W_UNIT;
     return (hw_float4){__uint_as_float(lut[u]), sign, __uint_as_float(lut[u + 1]), sign};
   }
-  // what the sums of a tile are multiplied by
-  static __device__ __forceinline__ float vscale(int tile, float ia0, float ia1) { return tile < 6 ? ia0 : tile < 10 ? ia1 : -kHwKappa; }
+  // row i of the lane's rows of the finished tiles
+  static __device__ __forceinline__ void finish(const uint32_t* lut, hw_float4 (&o)[NT], int i, float (&v)[NT]) {
+    const float ia0 = 1.f / __uint_as_float(lut[HW_W_ALPHA]), ia1 = 1.f / __uint_as_float(lut[HW_W_ALPHA + 1]);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) v[n] = hw_add_four(o[n][i]) * (n < 6 ? ia0 : n < 10 ? ia1 : -KAPPA);
+  }
+  // ---- transforms of queries and outputs: lane l holds four of the 256 sums' coordinates
+  static __device__ __forceinline__ int sum_of(int lane, int p) { return 64 * p + lane; }
+  // the sum faced by byte b of dword r of slot x of the query operand, lane group g
+  static __device__ __forceinline__ int faced(int x, int g, int r, int b) { return 64 * x + hw35_kcoord(x, g, r, b); }
+  static __device__ __forceinline__ int coord(int lane, int i) { return 64 * i + lane; }
+  static __device__ __forceinline__ void forward(float q0, float q1, int lane, const float* table, float (&y)[4]) {
+    y[0] = hyb_fwht64(q0 * table[HYB_HAD0 + lane], lane) * 0.125f;
+    y[1] = hyb_fwht64(q0 * table[HYB_QJL0 + lane], lane) * 0.125f;
+    y[2] = hyb_fwht64(q1 * table[HYB_HAD1 + lane], lane) * 0.125f;
+    y[3] = hyb_fwht64(q1 * table[HYB_QJL1 + lane], lane) * 0.125f;
+  }
+  static __device__ __forceinline__ void back(const float (&acc)[4], int lane, const float* table, float& o0, float& o1) {
+    o0 = (hyb_fwht64(acc[0], lane) * table[HYB_HAD0 + lane] + hyb_fwht64(acc[1], lane) * table[HYB_QJL0 + lane]) * 0.125f;
+    o1 = (hyb_fwht64(acc[2], lane) * table[HYB_HAD1 + lane] + hyb_fwht64(acc[3], lane) * table[HYB_QJL1 + lane]) * 0.125f;
+  }
+  static constexpr int TAGS = 12, TAG_AT = HYB_CEN0;        // the codebooks, which the tables are built from
+  static __device__ void tables(const float* table, uint32_t* lut);
+};
+
+// ----------------------------------------------------------------------------------
+// tq25 rows (44 bytes): A0 32 codes of 2 bits, B0 32 signs, two factors, A1 96 codes of 1 bit, B1 96 signs, two factors
+// ----------------------------------------------------------------------------------
+// In LDS a row is twelve dwords: A0 A0 B0 f0 | A1 A1 A1 f1 | B1 B1 B1 f1 (16 rows of 48 bytes meet sixteen different sets of banks).
+// A code of one bit is a sign around the middle of its two levels: c = middle - delta (+-1).  The sum of the query against the
+// middle is a constant of the head, and the sum of the weights comes out of the value product in a row nobody else has.
+struct hw25 {
+  static constexpr uint32_t MARK = HW_MARK + 25;
+  static constexpr int KD = 2;               // (only says how many wavefronts the registers admit)
+  static constexpr int TILE = 768;
+  static constexpr int NT = 20;              // value tiles: A0 (2), B0 (2), A1 (8), B1 (8)
+  static constexpr int SUM_B = 128;          // sums: A0 0..31, A1 32..127, B0 and B1 from 128 on in the same order
+  uint32_t half, byte;                       // lane (n, g) of a score tile: address of row n, plus 2 g, plus g
+  uint32_t tr;
+  uint32_t ka[3], va[4];
+  float delta;
+  uint32_t sh4, sh2, not15;
+  float middle;                              // what the middle of the 1-bit levels adds, for the lane's column
+
+  __device__ __forceinline__ hw25(const uint32_t* lut, int lane, uint32_t buf) {
+    const uint32_t col = lane & 15, g = lane >> 4;
+    half = buf + col * 48u + 2u * g;
+    byte = buf + col * 48u + g;
+    const uint32_t r = col >> 1, row = 4u * g + (r & 3u);
+    tr = buf + HW_VALUES + (r >> 2) * TILE + row * 48u + (col & 1u) * 8u;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) ka[i] = lut[HW_W_KP1 + i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) va[i] = lut[i < 2 ? HW_W_VA1 + i : HW_W_VP1 + i - 2];
+    delta = __uint_as_float(lut[HW_W_DELTA]);
+    middle = __uint_as_float(lut[HW_W_MIDDLE]) * -64.f;
+    sh4 = col >= 8 ? 4u : 0u;
+    sh2 = 2u * (col >> 2);
+    not15 = col == 15 ? 0u : ~0u;
+  }
+  template <int N> static __device__ __forceinline__ void request_tile(const uint8_t* base, int64_t pos, int lane, uint32_t lds) {
+    static_assert(N == 4, "rows of eleven dwords");
+#pragma unroll
+    for (uint32_t q = 0; q < 3; ++q) {
+      const uint32_t i = 64u * q + (uint32_t)lane, row = i / 12u, at = i % 12u, from = at < 7u ? at : at == 7u || at == 11u ? 10u : at - 1u;
+      hw_request<4>(base, row * (uint32_t)pos + from * 4u, lds + 256u * q);
+    }
+  }
+  // (the sum of the query integers over the 96 coordinates, column by column, against ones)
+  __device__ __forceinline__ void start(uint32_t query) {
+    const hw_int4 ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    const hw_int4 zero = {0, 0, 0, 0};
+    const hw_int4 a = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, *(hw_lds_i128*)(uintptr_t)(query + HW_Q_PART), zero, 0, 0, 0);
+    const hw_int4 b = __builtin_amdgcn_mfma_i32_16x16x32_i8(hw_as_long(0x01010101u, 0x01010101u), *(hw_lds_l64*)(uintptr_t)(query + 2 * HW_Q_PART), zero, 0, 0, 0);
+    middle_now = middle * (float)(a[0] + b[0]);
+  }
+  float middle_now;
+  static __device__ __forceinline__ uint32_t factors(uint32_t row, int group) { return row * 48u + (group ? 28u : 12u); }
+
+  __device__ __forceinline__ void scores(uint32_t keys, uint32_t fac, uint32_t query, float (&t)[8]) const {
+    auto q16 = [&](int slot) __attribute__((always_inline)) { return *(hw_lds_i128*)(uintptr_t)(query + HW_Q_PART * slot); };
+    auto q8 = [&](int slot, int up) __attribute__((always_inline)) { return *(hw_lds_l64*)(uintptr_t)(query + HW_Q_PART * slot + 8u * up); };
+    uint32_t a0[2], b0[2], h[2][2], e[2][2];      // two bytes of A0, one of B0; two and one of A1, B1
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      a0[j] = *(hw_lds_cu16*)(uintptr_t)(half + keys + TILE * j);
+      b0[j] = *(hw_lds_cu8*)(uintptr_t)(byte + keys + TILE * j + 8u);
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        h[j][x] = *(hw_lds_cu16*)(uintptr_t)(half + keys + TILE * j + 16u + 16u * x);
+        e[j][x] = *(hw_lds_cu8*)(uintptr_t)(byte + keys + TILE * j + 24u + 16u * x);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const hw_int4 zero = {0, 0, 0, 0};
+      auto eight = [&](uint32_t v) __attribute__((always_inline)) {      // a byte's signs: bits 7 - b in byte b, then 3 - b
+        uint32_t x = v | (v << 9);
+        x = x | (x << 18);
+        return hw_as_long(hw_and_or(x, 0x80808080u, 0x40404040u), hw_and_or(x << 4, 0x80808080u, 0x40404040u));
+      };
+      // (the two products of a part are added up here: the second one started from the first one's sums, which the compiler let
+      // overlap its own in part, and wrong sums came out)
+      hw_int4 c[3], sg[3], sh[2];
+      {
+        const uint32_t x = a0[j] | (a0[j] << 18), s0 = (x >> 6) & 0x03030303u, s1 = (x >> 2) & 0x03030303u;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+          c[d] = __builtin_amdgcn_mfma_i32_16x16x32_i8(hw_as_long(__builtin_amdgcn_perm(ka[d], ka[d], s0), __builtin_amdgcn_perm(ka[d], ka[d], s1)), q8(0, 0), zero, 0, 0, 0);
+      }
+      sg[2] = __builtin_amdgcn_mfma_i32_16x16x32_i8(eight(b0[j]), q8(0, 1), zero, 0, 0, 0);
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const uint32_t both = h[j][x] | (h[j][x] << 20);
+        hw_int4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = (int)hw_and_or(both << r, 0x80808080u, 0x40404040u);
+        sg[x] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v, q16(1 + 2 * x), zero, 0, 0, 0);
+        sh[x] = __builtin_amdgcn_mfma_i32_16x16x32_i8(eight(e[j][x]), q8(2, x), zero, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const hw_float4 f = *(hw_lds_f128*)(uintptr_t)(fac + 256u * j + 16u * i);
+        float x = fmaf((float)c[0][i], 65536.f, (float)((c[1][i] << 8) + c[2][i])) * f[0];
+        x = fmaf((float)sg[2][i], f[1], x);
+        x = fmaf(fmaf((float)(sg[0][i] + sh[0][i]), delta, middle_now), f[2], x);
+        t[4 * j + i] = fmaf((float)(sg[1][i] + sh[1][i]), f[3], x);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  template <class W> __device__ __forceinline__ void values(uint32_t keys, W weights, hw_float4 (&o)[NT]) const {
+    hw_int2 win[3];
+#pragma unroll
+    for (uint32_t p = 0; p < 3; ++p) win[p] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((hw_lds_i64*)(uintptr_t)(tr + keys + 16u * p));
+    auto product = [&](int tile, const hw_half8& w, uint32_t (&a)[4]) __attribute__((always_inline)) {
+      o[tile] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hw_operand(a[0], a[1], a[2], a[3]), w, o[tile], 0, 0, 0);
+    };
+    // ---- A0: bytes in lanes 0..7 (upper two codes), again in 8..15 (lower two)
+    {
+      const hw_half8 w = weights(0);
+      uint32_t c[2];
+#pragma unroll
+      for (int d = 0; d < 2; ++d) c[d] = (uint32_t)__builtin_amdgcn_update_dpp(win[0][d], win[0][d], 0x128 /*row_ror:8*/, 0xf, 0xc, false) << sh4;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int term = 0; term < 2; ++term) {
+          uint32_t a[4];
+#pragma unroll
+          for (int d = 0; d < 2; ++d) {
+            const uint32_t sel = (c[d] >> (6 - 2 * i)) & 0x03030303u;
+            hw_expand(__builtin_amdgcn_perm(va[2 * term], va[2 * term], sel), __builtin_amdgcn_perm(va[2 * term + 1], va[2 * term + 1], sel), a[2 * d], a[2 * d + 1]);
+          }
+          product(i, w, a);
+        }
+    }
+    // ---- B0: four bytes in lanes 8..11, again in every four lanes; bank k takes bits 7 - 2 k and 6 - 2 k
+    {
+      const hw_half8 w = weights(1);
+      uint32_t b[2];
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        int x = __builtin_amdgcn_update_dpp(win[0][d], win[0][d], 0x108 /*row_shl:8*/, 0xf, 0x1, false);
+        x = __builtin_amdgcn_update_dpp(x, win[0][d], 0x104 /*row_shl:4*/, 0xf, 0x2, false);
+        x = __builtin_amdgcn_update_dpp(x, win[0][d], 0x114 /*row_shr:4*/, 0xf, 0x8, false);
+        b[d] = (uint32_t)x << sh2;
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        uint32_t a[4];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) hw_signs(b[d], i, a[2 * d], a[2 * d + 1]);
+        product(2 + i, w, a);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- A1 and B1: twelve bytes in lanes 0..11, a bit a tile.  (Lane 15 of A1's: +1 for every token, the sum of the weights.)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const hw_half8 w = weights(2 + x);
+      uint32_t b[2];
+#pragma unroll
+      for (int d = 0; d < 2; ++d) b[d] = x == 0 ? (uint32_t)win[1][d] & not15 : (uint32_t)win[2][d];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        uint32_t a[4];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) hw_signs(b[d], i, a[2 * d], a[2 * d + 1]);
+        product(4 + 8 * x + i, w, a);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  template <class S> static __device__ __forceinline__ void places(int m, S store) {
+    // (rows 12..15 of A1 and B1 hold nothing: stored where A0 and B0 of the same lane belong, which come later)
+    const int a0 = m < 8 ? 4 * m : 4 * (m - 8) + 2, b0 = SUM_B + 8 * (m & 3) + 2 * (m >> 2);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      store(m < 12 ? 32 + 8 * m + t : a0, 4 + t);
+      store(m < 12 ? SUM_B + 32 + 8 * m + t : b0, 12 + t);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      store(a0 + t, t);
+      store(b0 + t, 2 + t);
+    }
+  }
+  static __device__ __forceinline__ hw_float4 kscale(const uint32_t* lut) {
+    return (hw_float4){__uint_as_float(lut[HW_W_UNITP + 1]), -kH25Kappa0 / 64.f, -1.f / 64.f, -kH25Kappa1 / 64.f};
+  }
+  static __device__ __forceinline__ void finish(const uint32_t* lut, hw_float4 (&o)[NT], int i, float (&v)[NT]) {
+    const float ia = 1.f / __uint_as_float(lut[HW_W_ALPHA + 1]), dl = __uint_as_float(lut[HW_W_DELTA]), md = __uint_as_float(lut[HW_W_MIDDLE]);
+    const float all = __shfl(hw_add_four(o[4][3]), 48 + (int)(threadIdx.x & 15)) * md;      // (row 15 of A1's tiles)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const float x = hw_add_four(o[n][i]);
+      v[n] = n < 2 ? x * ia : n < 4 ? x * -kH25Kappa0 : n < 12 ? fmaf(x, -dl, all) : x * -kH25Kappa1;
+    }
+  }
+  static __device__ __forceinline__ int sum_of(int lane, int p) { return (p & 1 ? SUM_B : 0) + coord(lane, p >> 1); }
+  static __device__ __forceinline__ int faced(int x, int g, int r, int b) {
+    const int eight = 8 * g + 4 * (r & 1) + b;       // of a byte a lane group
+    if (x == 0) return r < 2 ? 4 * (2 * g + (b & 1)) + 2 * r + (b >> 1) : SUM_B + eight;
+    if (x == 2) return (r < 2 ? 32 : SUM_B + 32) + 64 + eight;
+    return (x == 1 ? 32 : SUM_B + 32) + 8 * (2 * g + (b & 1)) + r + 4 * (b >> 1);
+  }
+  static __device__ __forceinline__ int coord(int lane, int i) {
+    const h25_roles r(lane);
+    return i == 0 ? r.ca : r.cb;
+  }
+  static __device__ __forceinline__ void forward(float qa, float qb, int lane, const float* table, float (&y)[4]) {
+    const h25_roles r(lane);
+    const float root_b = r.b0 ? kH25Root0 : kH25Root1;
+    y[0] = hyb_fwht64(qa * table[H25_HAD + r.ca], lane) / kH25Root1;
+    y[1] = hyb_fwht64(qa * table[H25_QJL + r.ca], lane) / kH25Root1;
+    y[2] = h25_fwht32(qb * table[H25_HAD + r.cb], lane) / root_b;
+    y[3] = h25_fwht32(qb * table[H25_QJL + r.cb], lane) / root_b;
+  }
+  static __device__ __forceinline__ void back(const float (&acc)[4], int lane, const float* table, float& o0, float& o1) {
+    const h25_roles r(lane);
+    const float inv_b = r.b0 ? 1.f / kH25Root0 : 1.f / kH25Root1;
+    o0 = (hyb_fwht64(acc[0], lane) * table[H25_HAD + r.ca] + hyb_fwht64(acc[1], lane) * table[H25_QJL + r.ca]) * (1.f / kH25Root1);
+    o1 = (h25_fwht32(acc[2], lane) * table[H25_HAD + r.cb] + h25_fwht32(acc[3], lane) * table[H25_QJL + r.cb]) * inv_b;
+  }
+  static constexpr int TAGS = 6, TAG_AT = H25_CEN0;
+  static __device__ void tables(const float* table, uint32_t* lut);
 };
 
 // ----------------------------------------------------------------------------------
 // main kernel
 // ----------------------------------------------------------------------------------
-// value of the lane four columns up in the row of sixteen, added (columns 0..3)
-__device__ __forceinline__ float hw_add_four(float v) {
-  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104 /*row_shl:4*/, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float hw_ror8(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128 /*row_ror:8*/, 0xf, 0xf, false));
-}
-
 // N: bytes of a request, 16 where rows allow it, else 4
 template <class F, int N>
 __global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_kernel(hw_args a) {
@@ -443,7 +696,7 @@ __global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_ke
   const int hd = h / a.hgroup, sub = h % a.hgroup;         // the head whose rows are read, which of its groups of query heads
   const int q0 = hd * a.gqa + 4 * sub, nq = min(4, a.gqa - 4 * sub);
   const uint32_t buf = (uint32_t)wave * HW_BUF;
-  const F f(a.lut, lane, buf);
+  F f(a.lut, lane, buf);
   const uint32_t fac_at = HW_FAC + (uint32_t)wave * HW_FAC_WAVE;
   const uint32_t fread = fac_at + (uint32_t)g * 64u;       // key factors of tokens 4 g of tile 0
   const int kb = (lane >> 2) & 3;                          // softmax: the lane has tokens kb % 2 and 2 + kb % 2 of tile kb / 2
@@ -453,7 +706,8 @@ __global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_ke
   const uint32_t vread = fac_at + 512u + vplace(tok);
   // factors: lanes 0..31 a key each, 32..63 a value each
   const hw_float4 ks = F::kscale(a.lut);
-  const uint32_t fsrc0 = buf + (uint32_t)(lane >> 4) * F::TILE + F::factors(col, 0), fsrc1 = buf + (uint32_t)(lane >> 4) * F::TILE + F::factors(col, 1);
+  const uint32_t fsrc = buf + (uint32_t)(lane >> 5) * HW_VALUES + (uint32_t)((lane >> 4) & 1) * F::TILE;
+  const uint32_t fsrc0 = fsrc + F::factors(col, 0), fsrc1 = fsrc + F::factors(col, 1);
   const uint32_t fwrite = fac_at + (lane < 32 ? (uint32_t)lane * 16u : 512u + vplace(lane & 31));
   // digits of a head's scores, columns 4 d + c: place 4 (d ^ g) + c of the lane group, so that groups meet different banks
   const uint32_t twrite = buf + (uint32_t)(g * 256 + (col ^ (4 * g)) * 16);
@@ -509,8 +763,8 @@ __global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_ke
         const uint32_t to = buf + (k & 1 ? HW_BUF / 2 : 0u);
         F::template request_tile<N>(kbase + (uint64_t)pb0 * (uint32_t)a.kps_blk, a.kps_pos, lane, to);
         F::template request_tile<N>(kbase + (uint64_t)pb1 * (uint32_t)a.kps_blk + (bs32 ? 16 * a.kps_pos : 0), a.kps_pos, lane, to + F::TILE);
-        F::template request_tile<N>(vbase + (uint64_t)pb0 * (uint32_t)a.vps_blk, a.vps_pos, lane, to + 2 * F::TILE);
-        F::template request_tile<N>(vbase + (uint64_t)pb1 * (uint32_t)a.vps_blk + (bs32 ? 16 * a.vps_pos : 0), a.vps_pos, lane, to + 3 * F::TILE);
+        F::template request_tile<N>(vbase + (uint64_t)pb0 * (uint32_t)a.vps_blk, a.vps_pos, lane, to + HW_VALUES);
+        F::template request_tile<N>(vbase + (uint64_t)pb1 * (uint32_t)a.vps_blk + (bs32 ? 16 * a.vps_pos : 0), a.vps_pos, lane, to + HW_VALUES + F::TILE);
       };
       load_window(0);
       request(0);
@@ -522,6 +776,8 @@ __global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_ke
           if (col < 12) *(hw_lds_i128*)(uintptr_t)(qat + HW_Q_PART * p) = hw_as_int4(u);
         }
       }
+      akv_wave_sync();
+      f.start(qat);
       const float qfac = a.fac[(size_t)s * a.QH + q0 + min(col & 3, nq - 1)];
 
       for (int k = 0; k < mine; ++k) {
@@ -641,12 +897,12 @@ __global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_ke
     if (active && r < shares) {
       int row = 4 * g;
       asm volatile("" : "+v"(row));      // (the places would be computed ahead of all segments, a register each)
-      const float ia0 = 1.f / __uint_as_float(a.lut[HW_W_ALPHA]), ia1 = 1.f / __uint_as_float(a.lut[HW_W_ALPHA + 1]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float v[NT];
+        F::finish(a.lut, o, i, v);
 #pragma unroll
-        for (int n = 0; n < NT; ++n) v[n] = hw_add_four(o[n][i]) * (F::vscale(n, ia0, ia1) * wgt);
+        for (int n = 0; n < NT; ++n) v[n] *= wgt;
         if (col < nq) F::places(row + i, [&](int at, int n) __attribute__((always_inline)) { *(hw_lds_f32*)(uintptr_t)(buf + (uint32_t)(col * 256 + at) * 4u) = v[n]; });
       }
     }
@@ -671,18 +927,135 @@ __global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_ke
 }
 
 // ----------------------------------------------------------------------------------
+// tables, built by a workgroup of 256 threads
+// ----------------------------------------------------------------------------------
+// byte `byte_of` of four levels, table[0..3], a word: of their integers in units of `unit` (kd digits, top first), or of the
+// float16 form of alpha times a level (low byte first), rounding or remainder
+__device__ __forceinline__ uint32_t hw_key_bytes(const float* table, float unit, int kd, int byte_of) {
+  uint32_t word = 0;
+  for (int v = 0; v < 4; ++v) {
+    const int n = (int)rintf(table[v] / unit), d0 = ((n + 128) & 255) - 128, n1 = (n - d0) >> 8;
+    const int d1 = kd == 3 ? ((n1 + 128) & 255) - 128 : n1, d2 = (n1 - d1) >> 8;
+    word |= ((uint32_t)(byte_of == kd - 1 ? d0 : byte_of == kd - 2 ? d1 : d2) & 255u) << (8 * v);
+  }
+  return word;
+}
+__device__ __forceinline__ uint32_t hw_value_bytes(const float* table, float alpha, bool remainder, int byte_of) {
+  uint32_t word = 0;
+  for (int v = 0; v < 4; ++v) {
+    const float x = alpha * table[v];
+    const __half hi = __float2half_rn(x);
+    const uint32_t bits = __half_as_ushort(remainder ? __float2half_rn(x - __half2float(hi)) : hi);
+    word |= (byte_of == 0 ? bits & 255u : bits >> 8) << (8 * v);
+  }
+  return word;
+}
+// largest magnitude of n levels, and the power of two that brings it to [2^9, 2^10)
+__device__ __forceinline__ float hw_top(const float* table, int n) {
+  float top = 0.f;
+  for (int v = 0; v < n; ++v) top = fmaxf(top, fabsf(table[v]));
+  return top;
+}
+__device__ __forceinline__ float hw_base(float top) {
+  return top > 0.f ? __uint_as_float((min(max(254u + 9u - ((__float_as_uint(top) >> 23) & 0xffu), 1u), 253u)) << 23) : 1.f;
+}
+
+template <bool P> __device__ void hw35<P>::tables(const float* table, uint32_t* lut) {
+  __shared__ float best_err[256], best[256];
+  __shared__ float chosen[4], fine[2];
+  const int tid = threadIdx.x;
+  // A free factor per set of levels makes them nearly exact: sets 0, 1 the unit of the 3- and 2-bit integers of two digits,
+  // sets 2, 3 alpha of fp16(alpha c), from HW_SEARCH candidates within a factor of two the one with the smallest largest error
+  // (relative to the largest level, and to each level).  16-bit integers then carry the levels to 1e-6, not 1.5e-5.  The
+  // largest alpha c lies in [2^9, 2^11), so that no remainder is a subnormal.
+#pragma unroll 1
+  for (int set = 0; set < 4; ++set) {
+    const int v0 = set & 1 ? 8 : 0, v1 = set & 1 ? 12 : 8;
+    float top = 0.f;
+    for (int v = v0; v < v1; ++v) top = fmaxf(top, fabsf(table[HYB_CEN0 + v]));
+    const float base = top > 0.f ? __uint_as_float((min(max(254u + 9u - ((__float_as_uint(top) >> 23) & 0xffu), 1u), 253u)) << 23) : 1.f;
+    float berr = INFINITY, bval = 1.f;
+#pragma unroll 1
+    for (int k = 0; k < HW_SEARCH / 256; ++k) {
+      const float al = 1.f + (float)(tid * (HW_SEARCH / 256) + k) / (float)HW_SEARCH;
+      const float inv = (float)HW_LEVELS * 0.5f * al / top;        // levels an integer, at most HW_LEVELS
+      float worst = 0.f;
+      for (int v = v0; v < v1; ++v) {
+        const float x = table[HYB_CEN0 + v] * (set < 2 ? inv : al * base);
+        const float e = set < 2 ? fabsf(rintf(x) - x) / al : x != 0.f ? fabsf(__half2float(__float2half_rn(x)) - x) / fabsf(x) : 0.f;
+        worst = fmaxf(worst, e);
+      }
+      if (worst < berr) { berr = worst; bval = al; }
+    }
+    __syncthreads();
+    best_err[tid] = berr;
+    best[tid] = bval;
+    __syncthreads();
+    if (tid == 0) {
+      int at = 0;
+      for (int t = 1; t < 256; ++t)
+        if (best_err[t] < best_err[at]) at = t;
+      chosen[set] = set < 2 ? (top > 0.f ? top / ((float)HW_LEVELS * 0.5f * best[at]) : 1.f) : best[at] * base;
+      if (set < 2) fine[set] = top > 0.f ? top * (1.f / HW_QMAX) : 1.f;
+    }
+    __syncthreads();
+  }
+  if (tid < 4) lut[HW_W_UNIT + tid] = __float_as_uint(chosen[tid]);      // (units, then alphas)
+  if (tid < 2) lut[HW_W_UNITP + tid] = __float_as_uint(fine[tid]);
+  if (tid < HW_W_UNITP && (tid < HW_W_UNIT || tid >= HW_W_KP0)) {
+    // thread = a word of the bytes of four levels: which set, which levels, which byte of what
+    const bool p = tid >= HW_W_KP0, vals = p ? tid >= HW_W_VP0 : tid >= HW_W_VA0;
+    const int i = tid - (p ? (vals ? HW_W_VP0 : HW_W_KP0) : (vals ? HW_W_VA0 : HW_W_KA0));
+    const int kd = vals ? 2 : p ? 3 : 2, set = i < 2 * kd ? 0 : 1;
+    const int v0 = set ? 8 : 4 * (i & 1), byte_of = set ? i - 2 * kd : i >> 1;       // keys: top digit first, values: low byte first
+    uint32_t word = 0;
+    for (int v = 0; v < 4; ++v) {
+      const float level = table[HYB_CEN0 + v0 + v];
+      uint32_t byte;
+      if (!vals) {
+        const int n = (int)rintf(level / (p ? fine[set] : chosen[set])), d0 = ((n + 128) & 255) - 128, n1 = (n - d0) >> 8;
+        const int d1 = p ? ((n1 + 128) & 255) - 128 : n1, d2 = (n1 - d1) >> 8;
+        byte = (uint32_t)(byte_of == kd - 1 ? d0 : byte_of == kd - 2 ? d1 : d2) & 255u;
+      } else {
+        const float x = chosen[2 + set] * level;
+        const __half hi = __float2half_rn(x);
+        const uint32_t bits = __half_as_ushort(p ? __float2half_rn(x - __half2float(hi)) : hi);
+        byte = byte_of == 0 ? bits & 255u : bits >> 8;
+      }
+      word |= byte << (8 * v);
+    }
+    lut[tid] = word;
+  }
+}
+
+__device__ void hw25::tables(const float* table, uint32_t* lut) {
+  const int tid = threadIdx.x;
+  const float* lv = table + H25_CEN0;
+  const float top = hw_top(lv, 4), alpha = hw_base(top), unit = top > 0.f ? top * (1.f / HW_QMAX) : 1.f;
+  const float c0 = table[H25_CEN1], c1 = table[H25_CEN1 + 1];
+  if (tid < 3) lut[HW_W_KP1 + tid] = hw_key_bytes(lv, unit, 3, tid);
+  if (tid < 2) lut[HW_W_VA1 + tid] = hw_value_bytes(lv, alpha, false, tid);
+  if (tid < 2) lut[HW_W_VP1 + tid] = hw_value_bytes(lv, alpha, true, tid);
+  if (tid == 0) {
+    lut[HW_W_UNITP + 1] = __float_as_uint(unit);
+    lut[HW_W_ALPHA + 1] = __float_as_uint(alpha);
+    lut[HW_W_DELTA] = __float_as_uint(0.5f * (c1 - c0));
+    lut[HW_W_MIDDLE] = __float_as_uint(0.5f * (c1 + c0));
+  }
+}
+
+// ----------------------------------------------------------------------------------
 // prologue: block 0 cuts the block axis, block 1 builds the tables (only when the codebooks are not the ones they were built
 // from), the others take a group of four query heads of a sequence: transform, scale, three signed bytes, operand order
 // ----------------------------------------------------------------------------------
-template <int QDT>
+template <class F, int QDT>
 __global__ __launch_bounds__(256) void akv_attn_hyb_prologue_kernel(
     const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const float* __restrict__ table, float qscale, int S, int QH,
     int KVH, int hgroup, int gqa, const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix,
     uint4* __restrict__ qop, float* __restrict__ fac, uint32_t* __restrict__ lut, uint32_t* __restrict__ status, uint32_t start_status,
     int32_t* __restrict__ wgdesc, int32_t* __restrict__ seqw, int G, int shares) {
-  __shared__ int8_t dig[3][4][4][64];     // [digit][query head][part][coordinate]
+  __shared__ int8_t dig[3][4][256];       // [digit][query head][sum]
   __shared__ int32_t scratch[257];
-  __shared__ float best_err[256], best[256];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (blockIdx.x == 0) {
     if (tid == 0) status[0] = start_status;
@@ -691,90 +1064,25 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_prologue_kernel(
   }
   if (blockIdx.x == 1) {
     __shared__ int stale;
-    __shared__ float chosen[4], fine[2];
-    if (tid == 0) stale = lut[HW_W_MARK] != HW_MARK ? 1 : 0;
+    if (tid == 0) stale = lut[HW_W_MARK] != F::MARK ? 1 : 0;
     __syncthreads();
-    if (tid < 12 && __float_as_uint(table[HYB_CEN0 + tid]) != lut[HW_W_TAG + tid]) stale = 1;
+    if (tid < F::TAGS && __float_as_uint(table[F::TAG_AT + tid]) != lut[HW_W_TAG + tid]) stale = 1;
     __syncthreads();
     if (!stale) return;
-    // A free factor per set of levels makes them nearly exact: sets 0, 1 the unit of the 3- and 2-bit integers of two digits,
-    // sets 2, 3 alpha of fp16(alpha c), from HW_SEARCH candidates within a factor of two the one with the smallest largest error
-    // (relative to the largest level, and to each level).  16-bit integers then carry the levels to 1e-6, not 1.5e-5.  The
-    // largest alpha c lies in [2^9, 2^11), so that no remainder is a subnormal.
-#pragma unroll 1
-    for (int set = 0; set < 4; ++set) {
-      const int v0 = set & 1 ? 8 : 0, v1 = set & 1 ? 12 : 8;
-      float top = 0.f;
-      for (int v = v0; v < v1; ++v) top = fmaxf(top, fabsf(table[HYB_CEN0 + v]));
-      const float base = top > 0.f ? __uint_as_float((min(max(254u + 9u - ((__float_as_uint(top) >> 23) & 0xffu), 1u), 253u)) << 23) : 1.f;
-      float berr = INFINITY, bval = 1.f;
-#pragma unroll 1
-      for (int k = 0; k < HW_SEARCH / 256; ++k) {
-        const float al = 1.f + (float)(tid * (HW_SEARCH / 256) + k) / (float)HW_SEARCH;
-        const float inv = (float)HW_LEVELS * 0.5f * al / top;        // levels an integer, at most HW_LEVELS
-        float worst = 0.f;
-        for (int v = v0; v < v1; ++v) {
-          const float x = table[HYB_CEN0 + v] * (set < 2 ? inv : al * base);
-          const float e = set < 2 ? fabsf(rintf(x) - x) / al : x != 0.f ? fabsf(__half2float(__float2half_rn(x)) - x) / fabsf(x) : 0.f;
-          worst = fmaxf(worst, e);
-        }
-        if (worst < berr) { berr = worst; bval = al; }
-      }
-      __syncthreads();
-      best_err[tid] = berr;
-      best[tid] = bval;
-      __syncthreads();
-      if (tid == 0) {
-        int at = 0;
-        for (int t = 1; t < 256; ++t)
-          if (best_err[t] < best_err[at]) at = t;
-        chosen[set] = set < 2 ? (top > 0.f ? top / ((float)HW_LEVELS * 0.5f * best[at]) : 1.f) : best[at] * base;
-        if (set < 2) fine[set] = top > 0.f ? top * (1.f / HW_QMAX) : 1.f;
-      }
-      __syncthreads();
-    }
-    if (tid < 4) lut[HW_W_UNIT + tid] = __float_as_uint(chosen[tid]);      // (units, then alphas)
-    if (tid < 2) lut[HW_W_UNITP + tid] = __float_as_uint(fine[tid]);
-    if (tid < HW_W_UNITP && (tid < HW_W_UNIT || tid >= HW_W_KP0)) {
-      // thread = a word of the bytes of four levels: which set, which levels, which byte of what
-      const bool p = tid >= HW_W_KP0, vals = p ? tid >= HW_W_VP0 : tid >= HW_W_VA0;
-      const int i = tid - (p ? (vals ? HW_W_VP0 : HW_W_KP0) : (vals ? HW_W_VA0 : HW_W_KA0));
-      const int kd = vals ? 2 : p ? 3 : 2, set = i < 2 * kd ? 0 : 1;
-      const int v0 = set ? 8 : 4 * (i & 1), byte_of = set ? i - 2 * kd : i >> 1;       // keys: top digit first, values: low byte first
-      uint32_t word = 0;
-      for (int v = 0; v < 4; ++v) {
-        const float level = table[HYB_CEN0 + v0 + v];
-        uint32_t byte;
-        if (!vals) {
-          const int n = (int)rintf(level / (p ? fine[set] : chosen[set])), d0 = ((n + 128) & 255) - 128, n1 = (n - d0) >> 8;
-          const int d1 = p ? ((n1 + 128) & 255) - 128 : n1, d2 = (n1 - d1) >> 8;
-          byte = (uint32_t)(byte_of == kd - 1 ? d0 : byte_of == kd - 2 ? d1 : d2) & 255u;
-        } else {
-          const float x = chosen[2 + set] * level;
-          const __half hi = __float2half_rn(x);
-          const uint32_t bits = __half_as_ushort(p ? __float2half_rn(x - __half2float(hi)) : hi);
-          byte = byte_of == 0 ? bits & 255u : bits >> 8;
-        }
-        word |= byte << (8 * v);
-      }
-      lut[tid] = word;
-    }
-    if (tid < 12) lut[HW_W_TAG + tid] = __float_as_uint(table[HYB_CEN0 + tid]);
+    F::tables(table, lut);
+    if (tid < F::TAGS) lut[HW_W_TAG + tid] = __float_as_uint(table[F::TAG_AT + tid]);
     __threadfence();
     __syncthreads();
-    if (tid == 0) lut[HW_W_MARK] = HW_MARK;
+    if (tid == 0) lut[HW_W_MARK] = F::MARK;
     return;
   }
   const int item = (int)blockIdx.x - 2, s = item / KVH, hv = item % KVH;
   const int q_first = hv / hgroup * gqa + hv % hgroup * 4, nq = min(4, gqa - hv % hgroup * 4);
   if (w < nq) {
     const int64_t off = s * qs_seq + (int64_t)(q_first + w) * qs_head;
-    const float q0 = akv_elem<QDT>::load(query, off + lane), q1 = akv_elem<QDT>::load(query, off + 64 + lane);
+    const float q0 = akv_elem<QDT>::load(query, off + F::coord(lane, 0)), q1 = akv_elem<QDT>::load(query, off + F::coord(lane, 1));
     float y[4];
-    y[0] = hyb_fwht64(q0 * table[HYB_HAD0 + lane], lane) * 0.125f;
-    y[1] = hyb_fwht64(q0 * table[HYB_QJL0 + lane], lane) * 0.125f;
-    y[2] = hyb_fwht64(q1 * table[HYB_HAD1 + lane], lane) * 0.125f;
-    y[3] = hyb_fwht64(q1 * table[HYB_QJL1 + lane], lane) * 0.125f;
+    F::forward(q0, q1, lane, table, y);
     const float top = akv_wave_max(fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3]))));
     const float nan = akv_wave_sum((q0 + q1) * 0.f);       // NaN when the query holds one, or an infinity
     // (a head of zeros, or one so small that the scale would overflow: integers of zero)
@@ -783,14 +1091,15 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_prologue_kernel(
     for (int p = 0; p < 4; ++p) {
       const int n = (int)rintf(fminf(fmaxf(y[p] * sc, -HW_QMAX), HW_QMAX));
       const int d0 = ((n + 128) & 255) - 128, n1 = (n - d0) >> 8, d1 = ((n1 + 128) & 255) - 128;
-      dig[0][w][p][lane] = (int8_t)((n1 - d1) >> 8);
-      dig[1][w][p][lane] = (int8_t)d1;
-      dig[2][w][p][lane] = (int8_t)d0;
+      const int at = F::sum_of(lane, p);
+      dig[0][w][at] = (int8_t)((n1 - d1) >> 8);
+      dig[1][w][at] = (int8_t)d1;
+      dig[2][w][at] = (int8_t)d0;
     }
     if (lane == 0) fac[(size_t)s * QH + q_first + w] = top * (1.f / HW_QMAX) * qscale + nan;
   }
   __syncthreads();
-  // thread = (part w, lane (column 4 d + head, lane group g)): sixteen coordinates of its head's digit d; columns of no digit or
+  // thread = (slot w, lane (column 4 d + head, lane group g)): sixteen coordinates of its head's digit d; columns of no digit or
   // head zero
   const int col = lane & 15, g = lane >> 4, d = col >> 2;
   uint32_t v[4];
@@ -798,7 +1107,7 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_prologue_kernel(
   for (int r = 0; r < 4; ++r) {
     v[r] = 0;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) v[r] |= d < 3 && (col & 3) < nq ? (uint32_t)(uint8_t)dig[d][col & 3][w][hw35_kcoord(w, g, r, b)] << (8 * b) : 0u;
+    for (int b = 0; b < 4; ++b) v[r] |= d < 3 && (col & 3) < nq ? (uint32_t)(uint8_t)dig[d][col & 3][F::faced(w, g, r, b)] << (8 * b) : 0u;
   }
   qop[((size_t)item * 4 + w) * 64 + lane] = make_uint4(v[0], v[1], v[2], v[3]);
 }
@@ -806,7 +1115,7 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_prologue_kernel(
 // ----------------------------------------------------------------------------------
 // reduce: a wavefront per query head of a sequence merges the partial results and transforms them back
 // ----------------------------------------------------------------------------------
-template <int ODT>
+template <class F, int ODT>
 __global__ __launch_bounds__(256) void akv_attn_hyb_reduce_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
                                                                   const float* __restrict__ table, int S, int QH, void* __restrict__ out,
                                                                   int64_t os_seq, int64_t os_head, const uint32_t* __restrict__ status,
@@ -819,14 +1128,16 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_reduce_kernel(const float* _
   const int64_t obase = s * os_seq + h * os_head;
   // (a call whose kernels reported a failure has produced garbage: every output says so)
   const float poison = status[0] != 0u ? __uint_as_float(0x7fc00000u) : 0.f;
-  const float had0 = table[HYB_HAD0 + lane], qjl0 = table[HYB_QJL0 + lane], had1 = table[HYB_HAD1 + lane], qjl1 = table[HYB_QJL1 + lane];
+  int at[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) at[i] = F::sum_of(lane, i);
   // the first PF partial sums are requested before their weights are known
   constexpr int PF = 8;
   float pre[PF][4];
 #pragma unroll
   for (int u = 0; u < PF; ++u)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) pre[u][i] = w_lo + u <= w_hi ? part_acc[((size_t)(w_lo + u + s) * QH + h) * 256 + i * 64 + lane] : 0.f;
+    for (int i = 0; i < 4; ++i) pre[u][i] = w_lo + u <= w_hi ? part_acc[((size_t)(w_lo + u + s) * QH + h) * 256 + at[i]] : 0.f;
   float M = -INFINITY;
   for (int w = w_lo + lane; w <= w_hi; w += 64) M = fmaxf(M, part_ml[((size_t)(w + s) * QH + h) * 2]);
   M = akv_wave_max(M);
@@ -851,16 +1162,18 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_reduce_kernel(const float* _
       for (int u = 0; u < PF; ++u) {
         const int w = w0 + u0 + PF + u;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pre[u][i] = w <= w_hi ? part_acc[((size_t)(w + s) * QH + h) * 256 + i * 64 + lane] : 0.f;
+        for (int i = 0; i < 4; ++i) pre[u][i] = w <= w_hi ? part_acc[((size_t)(w + s) * QH + h) * 256 + at[i]] : 0.f;
       }
     }
   }
   l = akv_wave_sum(l);
   const float inv = l > 0.f ? 1.f / l : l == 0.f ? 1.f : l;       // (NaN stays)
-  const float o0 = (hyb_fwht64(acc[0] * inv, lane) * had0 + hyb_fwht64(acc[1] * inv, lane) * qjl0) * 0.125f;
-  const float o1 = (hyb_fwht64(acc[2] * inv, lane) * had1 + hyb_fwht64(acc[3] * inv, lane) * qjl1) * 0.125f;
-  akv_elem<ODT>::store(out, obase + lane, o0 + poison);
-  akv_elem<ODT>::store(out, obase + 64 + lane, o1 + poison);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] *= inv;
+  float o0, o1;
+  F::back(acc, lane, table, o0, o1);
+  akv_elem<ODT>::store(out, obase + F::coord(lane, 0), o0 + poison);
+  akv_elem<ODT>::store(out, obase + F::coord(lane, 1), o1 + poison);
 }
 
 // ----------------------------------------------------------------------------------
@@ -902,7 +1215,28 @@ static int hw_launch(const hw_args& a, int grid, hipStream_t stream) {
   return AKV_OK;
 }
 
-int akv_attn_hyb_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float scale,
+// the three kernels of a call; `main` launches the middle one
+template <class F, class M>
+static int hw_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float scale, const hw_args& a,
+                  const akv_attn_ws& ws, void* out, int out_dtype, int64_t os_seq, int64_t os_head, hipStream_t stream, M main) {
+  const int G = hw_ranges(a.KVH, a.hp), shares = HW_W / a.hp;
+  const float qscale = scale * 1.4426950408889634f;      // scores come out in the log2 domain
+  const uint32_t start_status = g_spin_limit == 0 ? AKV_STATUS_HANDOFF_TIMEOUT : 0u;
+#define HW_PRO(DT) akv_attn_hyb_prologue_kernel<F, DT><<<a.S * a.KVH + 2, 256, 0, stream>>>(query, qs_seq, qs_head, table, qscale, a.S, a.QH, a.KVH, a.hgroup, a.gqa, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint4*)a.qop, ws.qrot, ws.lut, ws.status, start_status, ws.wgdesc, ws.seqw, G, shares)
+  if (q_dtype == AKV_F16) HW_PRO(AKV_F16); else if (q_dtype == AKV_BF16) HW_PRO(AKV_BF16); else HW_PRO(AKV_F32);
+#undef HW_PRO
+  AKV_LAUNCH_CHECK("akv_attn_hyb_prologue_kernel");
+  const int rc = main(G * a.hgroups);
+  if (rc) return rc;
+  const int rgrid = (a.S * a.QH + 3) / 4;
+#define HW_RED(DT) akv_attn_hyb_reduce_kernel<F, DT><<<rgrid, 256, 0, stream>>>(a.part_acc, a.part_ml, table, a.S, a.QH, out, os_seq, os_head, ws.status, ws.seqw)
+  if (out_dtype == AKV_F16) HW_RED(AKV_F16); else if (out_dtype == AKV_BF16) HW_RED(AKV_BF16); else HW_RED(AKV_F32);
+#undef HW_RED
+  AKV_LAUNCH_CHECK("akv_attn_hyb_reduce_kernel");
+  return AKV_OK;
+}
+
+int akv_attn_hyb_run(int format, const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float scale,
                      const akv_hyb_attn_args& in, const akv_attn_ws& ws, void* extra_ws, void* out, int out_dtype, int64_t os_seq,
                      int64_t os_head, hipStream_t stream) {
   hw_args a;
@@ -916,24 +1250,14 @@ int akv_attn_hyb_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_
   a.part_acc = ws.part_acc; a.part_ml = ws.part_ml;
   a.hp = a.KVH >= 3 ? 4 : a.KVH;
   a.hgroups = (a.KVH + a.hp - 1) / a.hp;
-  const int G = hw_ranges(a.KVH, a.hp), shares = HW_W / a.hp;
-  const float qscale = scale * 1.4426950408889634f;      // scores come out in the log2 domain
-  const uint32_t start_status = g_spin_limit == 0 ? AKV_STATUS_HANDOFF_TIMEOUT : 0u;
-#define HW_PRO(DT) akv_attn_hyb_prologue_kernel<DT><<<a.S * a.KVH + 2, 256, 0, stream>>>(query, qs_seq, qs_head, table, qscale, a.S, a.QH, a.KVH, a.hgroup, a.gqa, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint4*)extra_ws, ws.qrot, ws.lut, ws.status, start_status, ws.wgdesc, ws.seqw, G, shares)
-  if (q_dtype == AKV_F16) HW_PRO(AKV_F16); else if (q_dtype == AKV_BF16) HW_PRO(AKV_BF16); else HW_PRO(AKV_F32);
-#undef HW_PRO
-  AKV_LAUNCH_CHECK("akv_attn_hyb_prologue_kernel");
+  if (format == 25)
+    return hw_run<hw25>(query, q_dtype, qs_seq, qs_head, table, scale, a, ws, out, out_dtype, os_seq, os_head, stream,
+                        [&](int grid) { return hw_launch<hw25, 4>(a, grid, stream); });
   const uint64_t all = (uint64_t)(uintptr_t)a.kc | (uint64_t)(uintptr_t)a.vc | a.kps_blk | a.kps_pos | a.kps_head | a.vps_blk | a.vps_pos | a.vps_head;
   // groups of four query heads: the accuracy that the float16 levels of values leave; other counts: float32's, which they always had
   const bool wide = (all & 15) == 0, exact = a.gqa % 4 != 0;
-  const int grid = G * a.hgroups;
-  const int rc = exact ? (wide ? hw_launch<hw35<true>, 16>(a, grid, stream) : hw_launch<hw35<true>, 4>(a, grid, stream))
-                       : (wide ? hw_launch<hw35<false>, 16>(a, grid, stream) : hw_launch<hw35<false>, 4>(a, grid, stream));
-  if (rc) return rc;
-  const int rgrid = (a.S * a.QH + 3) / 4;
-#define HW_RED(DT) akv_attn_hyb_reduce_kernel<DT><<<rgrid, 256, 0, stream>>>(a.part_acc, a.part_ml, table, a.S, a.QH, out, os_seq, os_head, ws.status, ws.seqw)
-  if (out_dtype == AKV_F16) HW_RED(AKV_F16); else if (out_dtype == AKV_BF16) HW_RED(AKV_BF16); else HW_RED(AKV_F32);
-#undef HW_RED
-  AKV_LAUNCH_CHECK("akv_attn_hyb_reduce_kernel");
-  return AKV_OK;
+  return hw_run<hw35<false>>(query, q_dtype, qs_seq, qs_head, table, scale, a, ws, out, out_dtype, os_seq, os_head, stream, [&](int grid) {
+    return exact ? (wide ? hw_launch<hw35<true>, 16>(a, grid, stream) : hw_launch<hw35<true>, 4>(a, grid, stream))
+                 : (wide ? hw_launch<hw35<false>, 16>(a, grid, stream) : hw_launch<hw35<false>, 4>(a, grid, stream));
+  });
 }

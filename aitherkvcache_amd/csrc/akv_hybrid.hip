@@ -779,7 +779,7 @@ extern "C" int akv_hybrid_paged_attn(
     m.context_lens = context_lens; m.cl_itype = cl_itype;
     m.S = num_seqs; m.QH = num_q_heads; m.KVH = num_kv_heads; m.block_size = block_size;
     m.max_blocks_per_seq = max_blocks_per_seq; m.num_blocks = num_blocks;
-    return akv_attn_hyb_run(query, q_dtype, qs_seq, qs_head, hyb_table, scale, m, ws, (char*)workspace + ws.bytes, out, out_dtype,
+    return akv_attn_hyb_run(35, query, q_dtype, qs_seq, qs_head, hyb_table, scale, m, ws, (char*)workspace + ws.bytes, out, out_dtype,
                             os_seq, os_head, stream);
   }
 

@@ -23,31 +23,8 @@
 #include "akv_attn_common.h"
 #include "akv_hybrid_layout.h"
 
-#define H25_HAD 0          // [128] Hadamard signs in coordinate order (group 0's 32, then group 1's 96)
-#define H25_QJL 128        // [128] QJL signs likewise
-#define H25_CEN0 256       // 4 centroids
-#define H25_CEN1 260       // 2 centroids
-#define H25_BND0 262       // 3 boundaries
-#define H25_BND1 265       // 1 boundary
-#define H25_ROW 44
-
-// float32 values of sqrt(32), sqrt(96) and of sqrt(pi/2) / dim (hybrid_quantizer.py:232,540-541)
-constexpr float kH25Root0 = 5.656854249492381f;
-constexpr float kH25Root1 = 9.797958971132712f;
-constexpr float kH25Kappa0 = (float)(1.2533141373155001 / 32.0);
-constexpr float kH25Kappa1 = (float)(1.2533141373155001 / 96.0);
-
 __device__ __forceinline__ float h25_half_bits_to_float(uint32_t b) {
   return __half2float(__ushort_as_half((unsigned short)(b & 0xffffu)));
-}
-// 32-point Walsh-Hadamard transform inside each half of the wavefront
-__device__ __forceinline__ float h25_fwht32(float v, int lane) {
-  v = hyb_fwht_step<1>(v, lane);
-  v = hyb_fwht_step<2>(v, lane);
-  v = hyb_fwht_step<4>(v, lane);
-  v = hyb_fwht_step<8>(v, lane);
-  v = hyb_fwht_step<16>(v, lane);
-  return v;
 }
 // sum over the lanes of each half; every lane of a half receives its half's sum
 __device__ __forceinline__ float h25_half_sum(float v) {
@@ -61,15 +38,6 @@ __device__ __forceinline__ float h25_half_sum(float v) {
 __device__ __forceinline__ float h25_lane_value(float v, int src) {
   return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), src));
 }
-
-// the lane's two coordinates
-struct h25_roles {
-  int ca, cb;       // coordinate of the first value (group 1, 64-point block) and of the second
-  bool b0;          // the second value belongs to group 0
-  int ja, jb;       // position inside the group's code / sign streams
-  __device__ __forceinline__ explicit h25_roles(int lane)
-      : ca(32 + lane), cb(lane < 32 ? lane : 64 + lane), b0(lane < 32), ja(lane), jb(lane < 32 ? lane : 32 + lane) {}
-};
 
 // ----------------------------------------------------------------------------------
 // encode
@@ -652,6 +620,21 @@ extern "C" int akv_hybrid25_paged_attn(
   akv_attn_ws ws = akv_attn_ws_layout(workspace, num_seqs, num_q_heads, 256, G);
   if (workspace_bytes < ws.bytes)
     return akv_fail(AKV_ERR_WORKSPACE, "akv_hybrid25_paged_attn: workspace %zu < %zu bytes", workspace_bytes, ws.bytes);
+
+  // blocks of 16 or 32 tokens: the matrix-core kernel (a workspace without its part: the vector kernel, as ever)
+  const int64_t strides6[6] = {kps_blk, kps_pos, kps_head, vps_blk, vps_pos, vps_head};
+  if (max_blocks_per_seq > 0 && workspace_bytes >= ws.bytes + akv_attn_hyb_extra_bytes(num_seqs, num_q_heads) &&
+      akv_attn_hyb_applicable(block_size, strides6)) {
+    akv_hyb_attn_args m;
+    m.kc = k_cache; m.kps_blk = kps_blk; m.kps_pos = kps_pos; m.kps_head = kps_head;
+    m.vc = v_cache; m.vps_blk = vps_blk; m.vps_pos = vps_pos; m.vps_head = vps_head;
+    m.block_tables = block_tables; m.bt_itype = bt_itype; m.bt_stride = bt_stride;
+    m.context_lens = context_lens; m.cl_itype = cl_itype;
+    m.S = num_seqs; m.QH = num_q_heads; m.KVH = num_kv_heads; m.block_size = block_size;
+    m.max_blocks_per_seq = max_blocks_per_seq; m.num_blocks = num_blocks;
+    return akv_attn_hyb_run(25, query, q_dtype, qs_seq, qs_head, hyb_table, scale, m, ws, (char*)workspace + ws.bytes, out, out_dtype,
+                            os_seq, os_head, stream);
+  }
 
   const int nblocks_q = (num_seqs * num_q_heads + 3) / 4;
 #define H25_PRO(DT) h25_attn_prologue_kernel<DT><<<nblocks_q + 1, 256, 0, stream>>>(query, qs_seq, qs_head, hyb_table, num_seqs, num_q_heads, context_lens, cl_itype, block_size, max_blocks_per_seq, ws.prefix, ws.qrot, nblocks_q, ws.status)

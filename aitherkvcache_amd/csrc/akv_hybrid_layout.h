@@ -36,6 +36,38 @@ __device__ __forceinline__ float hyb_fwht64(float v, int lane) {
   return v;
 }
 
+// ---- tq25 (the row: akv_hybrid25.hip): tables, transforms
+#define H25_HAD 0          // [128] Hadamard signs in coordinate order (group 0's 32, then group 1's 96)
+#define H25_QJL 128        // [128] QJL signs likewise
+#define H25_CEN0 256       // 4 centroids
+#define H25_CEN1 260       // 2 centroids
+#define H25_BND0 262       // 3 boundaries
+#define H25_BND1 265       // 1 boundary
+#define H25_ROW 44
+
+// float32 values of sqrt(32), sqrt(96) and of sqrt(pi/2) / dim (hybrid_quantizer.py:232,540-541)
+constexpr float kH25Root0 = 5.656854249492381f;
+constexpr float kH25Root1 = 9.797958971132712f;
+constexpr float kH25Kappa0 = (float)(1.2533141373155001 / 32.0);
+constexpr float kH25Kappa1 = (float)(1.2533141373155001 / 96.0);
+// 32-point Walsh-Hadamard transform inside each half of the wavefront
+__device__ __forceinline__ float h25_fwht32(float v, int lane) {
+  v = hyb_fwht_step<1>(v, lane);
+  v = hyb_fwht_step<2>(v, lane);
+  v = hyb_fwht_step<4>(v, lane);
+  v = hyb_fwht_step<8>(v, lane);
+  v = hyb_fwht_step<16>(v, lane);
+  return v;
+}
+// the lane's two coordinates
+struct h25_roles {
+  int ca, cb;       // coordinate of the first value (group 1, 64-point block) and of the second
+  bool b0;          // the second value belongs to group 0
+  int ja, jb;       // position inside the group's code / sign streams
+  __device__ __forceinline__ explicit h25_roles(int lane)
+      : ca(32 + lane), cb(lane < 32 ? lane : 64 + lane), b0(lane < 32), ja(lane), jb(lane < 32 ? lane : 32 + lane) {}
+};
+
 // matrix-core attention on hybrid rows (akv_attn_hyb.hip)
 struct akv_attn_ws;
 struct akv_hyb_attn_args {
@@ -49,6 +81,7 @@ struct akv_hyb_attn_args {
 };
 size_t akv_attn_hyb_extra_bytes(int S, int QH);
 bool akv_attn_hyb_applicable(int block_size, const int64_t* strides6);
-int akv_attn_hyb_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float scale,
+// format: 35 or 25
+int akv_attn_hyb_run(int format, const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float scale,
                      const akv_hyb_attn_args& in, const akv_attn_ws& ws, void* extra_ws, void* out, int out_dtype, int64_t os_seq,
                      int64_t os_head, hipStream_t stream);
