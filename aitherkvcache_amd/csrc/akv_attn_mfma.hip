@@ -58,7 +58,7 @@
 //          order.  With 64 KB + 64 KB of tables the exchange buffers live in a third region (160 KB in all).
 // The order in which the coordinates reach the value product differs per format; it is undone for free by the order
 // in which the accumulators are written out (mf_vtile).  The query operand is in natural coordinate order for all.
-#include "akv_attn_common.h"
+#include "akv_attn_rows.h"
 #include "akv_nibble.h"
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -101,21 +101,18 @@ struct akv_mfma_extra {
 // ----------------------------------------------------------------------------------
 template <int QDT>
 __global__ __launch_bounds__(256) void akv_attn_mfma_prologue_kernel(
-    const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const uint4* __restrict__ bop,
-    const float* __restrict__ centroids, int S, int QH, int KVH, const void* context_lens,
+    const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const float* __restrict__ Pi, const akv_prep_scale* __restrict__ scale,
+    const float* __restrict__ centroids, int S, int QH, int KVH, int slots, const void* context_lens,
     int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix,
     uint4* __restrict__ qop, uint32_t* __restrict__ lut, uint32_t* __restrict__ status, float qscale, int bits, int nqb,
     int32_t* __restrict__ wgdesc, int32_t* __restrict__ seqw, int G) {
-  __shared__ __align__(16) float q_lds[8][132];   // [query head of the group][input coordinate], zero-padded heads
-  __shared__ float qr_lds[8][132];     // (rows 4 banks apart: the eight heads of a coordinate are read together)
+  __shared__ __align__(16) ar_rows<128> rows;
   __shared__ int32_t scratch[257];
   __shared__ float best_err[256];
   __shared__ float best_alpha[256];
   const int tid = threadIdx.x;
   // block 0: block prefix; block 1: tables (first, so that they start at once and do not wait for a free slot
-  // behind the rotation blocks); blocks [2, 2 + nqb): query rotation, (sequence, kv head) items blockIdx.x - 2,
-  // + nqb, ...
-  const int nq = S * KVH;
+  // behind the rotation blocks); blocks [2, 2 + nqb): query rotation
   if ((int)blockIdx.x == 0) {
     if (tid == 0) status[0] = 0u;
     akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size,
@@ -171,95 +168,12 @@ __global__ __launch_bounds__(256) void akv_attn_mfma_prologue_kernel(
     if (tid == 0) lut[MF_W_MARK] = MF_MARK + (uint32_t)bits;
     return;
   }
-  const int gqa = QH / KVH;
-  // q' = Pi q on the matrix cores: A = the queries of the kv head (row r = query head r % 8), B = the float16
-  // hi + lo operand of the encode kernel (lane (col, g): output coordinate 8 col + N-tile, input coordinates
-  // 32 g + 8 ks + e).  Wavefront w owns N-tiles 2w and 2w + 1; their operand registers are requested first and
-  // stay for all items of the block.  (On the vector unit, with the queries broadcast from LDS, this kernel took
-  // 23 us for 256 sequences x 8 kv heads.)
-  const int lane = tid & 63, wave = tid >> 6;
-  akv_half8 bh[2][4], bl[2][4];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const int idx = ((2 * wave + t) * 4 + ks) * 64 + lane;
-      bh[t][ks] = akv_as_half8(bop[idx]);
-      bl[t][ks] = akv_as_half8(bop[2048 + idx]);
-    }
-  for (int item = (int)blockIdx.x - 2; item < nq; item += nqb) {
-  const int s = item / KVH, h = item % KVH;
-  for (int i = tid; i < 8 * 128; i += 256) {
-    const int q = i >> 7, j = i & 127;
-    q_lds[q][j] = q < gqa ? akv_elem<QDT>::load(query, s * qs_seq + (h * gqa + q) * qs_head + j) : 0.f;
-  }
-  __syncthreads();
-  {
-    const int r = lane & 15, kg = lane >> 4;
-    float v[4][8];
-    float m = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const float4 x0 = *(const float4*)&q_lds[r & 7][32 * kg + 8 * ks];
-      const float4 x1 = *(const float4*)&q_lds[r & 7][32 * kg + 8 * ks + 4];
-      v[ks][0] = x0.x; v[ks][1] = x0.y; v[ks][2] = x0.z; v[ks][3] = x0.w;
-      v[ks][4] = x1.x; v[ks][5] = x1.y; v[ks][6] = x1.z; v[ks][7] = x1.w;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(v[ks][e]));
-    }
-    const uint32_t ex = akv_row_exponent(akv_rows_max(m));
-    const float sc = akv_row_scale(ex);
-    akv_float4v acc[2];
-    acc[0] = (akv_float4v){0.f, 0.f, 0.f, 0.f};
-    acc[1] = (akv_float4v){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      akv_half8 hi, lo;
-      akv_split8(v[ks], sc, hi, lo);
-      acc[0] = akv_mfma3(hi, lo, bh[0][ks], bl[0][ks], acc[0]);
-      acc[1] = akv_mfma3(hi, lo, bh[1][ks], bl[1][ks], acc[1]);
-    }
-    // lane (col, kg) holds query heads 4 kg + i (kg < 2) at output coordinates 8 col + 2 wave and + 1
-    const float usc = akv_row_unscale(ex) * (qscale / 64.f);     // lane q < 8: the factor of query head q
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float u0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(usc), i));
-      const float u1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(usc), 4 + i));
-      if (kg < 2) {
-        const float ui = kg == 0 ? u0 : u1;
-        qr_lds[4 * kg + i][8 * r + 2 * wave] = acc[0][i] * ui;
-        qr_lds[4 * kg + i][8 * r + 2 * wave + 1] = acc[1][i] * ui;
-      }
-    }
-  }
-  __syncthreads();
   // operand layout: [k-step n][lane (col, g)][e]: coordinate 32g + 4n + 2(e/4) + e%2 -- the four coordinates
   // of k-step n are the two code bytes (4-bit), the two 6-bit fields (3-bit) or the one code byte (2-bit) the
   // score wavefront looks up for that step; elements 2,3 and 6,7 repeat 0,1 and 4,5: they face the lo
-  // halves of the K table entries
-  for (int n = tid >> 6; n < 8; n += 4) {
-    const int lane = tid & 63;
-    const int col = lane & 15, g = lane >> 4;
-    unsigned short hbits[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int dim = 32 * g + 4 * n + 2 * (e >> 2) + (e & 1);
-      float v = 0.f;
-      if (col < 8) {
-        if (col < gqa) v = __half2float(__float2half_rn(qr_lds[col][dim]));
-      } else if (col - 8 < gqa) {
-        const float full = qr_lds[col - 8][dim];
-        v = full - __half2float(__float2half_rn(full));
-      }
-      hbits[e] = __half_as_ushort(__float2half_rn(v));
-    }
-    uint4 o;
-    o.x = hbits[0] | (hbits[1] << 16); o.y = hbits[2] | (hbits[3] << 16);
-    o.z = hbits[4] | (hbits[5] << 16); o.w = hbits[6] | (hbits[7] << 16);
-    qop[((size_t)(s * KVH + h) * 8 + n) * 64 + lane] = o;
-  }
-  __syncthreads();     // q_lds and qr_lds are rewritten by the next item
-  }
+  // halves of the K table entries.  (One (sequence, kv head) item a workgroup at a time, four rows of a tile of sixteen, this
+  // kernel took 17.0 us for 256 sequences of 8 kv heads, 9.5 now; for one sequence 5.5, now 4.6.)
+  ar_rotate_queries<128, QDT, true>(rows, (int)blockIdx.x - 2, nqb, query, qs_seq, qs_head, Pi, scale, S, QH, KVH, slots, qop, nullptr, qscale, bits);
 }
 
 // ----------------------------------------------------------------------------------
@@ -1100,12 +1014,13 @@ int akv_attn_mfma_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs
   x.wgdesc = ws.wgdesc;
   x.status = ws.status;
   const float qscale = a.scale * 1.4426950408889634f;   // scores come out in the log2 domain
-  // rotation blocks: one per (sequence, kv head) up to six per CU (what its registers admit at once), then they loop
-  const int cus = akv_cached_cu_count();
-  const int nqb = a.S * a.KVH < 6 * (cus > 0 ? cus : 256) ? a.S * a.KVH : 6 * (cus > 0 ? cus : 256);
+  // rotation blocks, up to three on a CU (then they loop)
+  const int cus = akv_cached_cu_count(), qslots = a.QH / a.KVH <= 4 ? 4 : 8;
+  const int nqb = ar_query_blocks(128, a.S, a.KVH, qslots, 3 * (cus > 0 ? cus : 256));
   const int pgrid = nqb + 2;
-  const uint4* bop = (const uint4*)(PiT + 128 * 128);    // the encode kernel's operand follows Pi and PiT in the prepared buffer
-#define MF_PRO(DT) akv_attn_mfma_prologue_kernel<DT><<<pgrid, 256, 0, stream>>>(query, qs_seq, qs_head, bop, a.centroids, a.S, a.QH, a.KVH, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, prefix, (uint4*)x.qop, (uint32_t*)x.lut, x.status, qscale, bits, nqb, ws.wgdesc, ws.seqw, grid)
+  const float* Pi = PiT - 128 * 128;
+  const akv_prep_scale* scale = (const akv_prep_scale*)((const char*)Pi + AKV_PREP_SCALE_OFFSET(128));
+#define MF_PRO(DT) akv_attn_mfma_prologue_kernel<DT><<<pgrid, 256, 0, stream>>>(query, qs_seq, qs_head, Pi, scale, a.centroids, a.S, a.QH, a.KVH, qslots, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, prefix, (uint4*)x.qop, (uint32_t*)x.lut, x.status, qscale, bits, nqb, ws.wgdesc, ws.seqw, grid)
   if (q_dtype == AKV_F16) MF_PRO(AKV_F16); else if (q_dtype == AKV_BF16) MF_PRO(AKV_BF16); else MF_PRO(AKV_F32);
 #undef MF_PRO
   AKV_LAUNCH_CHECK("akv_attn_mfma_prologue_kernel");

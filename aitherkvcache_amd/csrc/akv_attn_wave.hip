@@ -35,7 +35,7 @@
 // 49, 43 and 36 % at head_dim 64, 128 and 256, matrix cores 12 to 16, LDS 19 to 24.
 #include <type_traits>
 
-#include "akv_attn_common.h"
+#include "akv_attn_rows.h"
 #include "akv_device_once.h"
 
 typedef _Float16 aw_half8 __attribute__((ext_vector_type(8)));
@@ -81,171 +81,24 @@ struct aw_extra {
 };
 
 // ----------------------------------------------------------------------------------
-// prologue: block 0 cuts the block axis; the others take query heads blockIdx.x - 1, + gridDim.x - 1, ...: rotate, write
-// in operand order.  A thread holds AW_PRO_K entries of one column of Pi^T in registers, requested in one go before
-// anything else and kept for all heads of its workgroup (a trip to the L2 cache per entry, as in a plain loop over the
-// matrix, was 20 us at head_dim 256); D / AW_PRO_K threads share an output coordinate.
+// prologue: block 0 cuts the block axis, the others rotate query heads and write them in operand order (akv_attn_rows.h).
+// On the vector unit (a matrix column in registers, one row a workgroup at a time) it took 9.1 us for 384 rows of 256, 7.0 now;
+// 1,536 rows of 64 6.4, now 4.7.
 // ----------------------------------------------------------------------------------
-#define AW_PRO_K(D) ((D) == 64 ? 16 : 64)
-template <int D> constexpr int aw_pro_threads() { return D * (D / AW_PRO_K(D)); }      // 256, 256, 1024
 template <int D, int QDT>
-__global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_attn_wave_prologue_kernel(
-    const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const float* __restrict__ PiT, int S, int QH, int KVH,
-    const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix, uint2* __restrict__ qop,
-    float* __restrict__ fac, uint32_t* __restrict__ status, float qscale, int bits, int32_t* __restrict__ wgdesc,
+__global__ __launch_bounds__(256) void akv_attn_wave_prologue_kernel(
+    const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const float* __restrict__ Pi, const akv_prep_scale* __restrict__ scale,
+    int S, int QH, int KVH, int slots, const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix,
+    uint2* __restrict__ qop, float* __restrict__ fac, uint32_t* __restrict__ status, float qscale, int bits, int32_t* __restrict__ wgdesc,
     int32_t* __restrict__ seqw, int G, int shares) {
-  constexpr int K = AW_PRO_K(D), SHARES = D / K;
-  __shared__ __align__(16) float q_lds[2][D];          // [parity of the head]
-  __shared__ float sum_lds[SHARES][D];
-  __shared__ float max_lds[2][4];
+  __shared__ __align__(16) ar_rows<D> rows;
   __shared__ int32_t scratch[257];
-  const int tid = threadIdx.x;
   if (blockIdx.x == 0) {
-    if (tid == 0) status[0] = 0u;
+    if (threadIdx.x == 0) status[0] = 0u;
     akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares);
     return;
   }
-  const int t = tid % D, share = tid / D, gqa = QH / KVH;
-  float m[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) m[j] = PiT[(size_t)(share * K + j) * D + t];
-  int par = 0;
-  for (int item = (int)blockIdx.x - 1; item < S * QH; item += (int)gridDim.x - 1, par ^= 1) {
-    const int s = item / QH, hq = item % QH, h = hq / gqa, q = hq % gqa;
-    if (tid < D) q_lds[par][tid] = akv_elem<QDT>::load(query, s * qs_seq + hq * qs_head + tid);
-    __syncthreads();
-    float acc = 0.f;
-#pragma unroll
-    for (int j = 0; j < K; j += 4) {
-      const float4 x = *(const float4*)&q_lds[par][share * K + j];
-      acc = fmaf(m[j], x.x, acc);
-      acc = fmaf(m[j + 1], x.y, acc);
-      acc = fmaf(m[j + 2], x.z, acc);
-      acc = fmaf(m[j + 3], x.w, acc);
-    }
-    sum_lds[share][t] = acc;
-    __syncthreads();
-    float y = 0.f;
-    if (tid < D) {
-#pragma unroll
-      for (int i = 0; i < SHARES; ++i) y += sum_lds[i][tid];
-      const float mx = akv_wave_max(fabsf(y));
-      if ((tid & 63) == 0) max_lds[par][tid >> 6] = mx;
-    }
-    __syncthreads();
-    if (tid < D) {
-      float mx = 0.f;
-#pragma unroll
-      for (int i = 0; i < D / 64; ++i) mx = fmaxf(mx, max_lds[par][i]);
-      const uint32_t ex = akv_row_exponent(mx);
-      if (tid == 0) fac[(size_t)s * QH + hq] = akv_row_unscale(ex) * qscale;
-      // coordinate tid = quarter g, step n, place e of the step's four (2-bit codes are looked up as (0, 2) and (1, 3))
-      const float x = y * akv_row_scale(ex);
-      const __half hi = __float2half_rn(x);
-      const int g = tid / (D / 4), n = tid % (D / 4) / 4, c4 = tid & 3;
-      const int e = bits == 2 ? ((c4 & 1) << 1) + (c4 >> 1) : c4;
-      __half* dst = (__half*)(qop + (size_t)(s * KVH + h) * (D / 16 * 64) + n * 64 + 16 * g + q) + e;
-      dst[0] = hi;
-      dst[8 * 4] = __float2half_rn(x - __half2float(hi));
-      // (columns of no query head hold zeros)
-      if (q == 0)
-        for (int z = gqa; z < 8; ++z) { dst[z * 4] = __float2half_rn(0.f); dst[(8 + z) * 4] = __float2half_rn(0.f); }
-    }
-  }
-}
-
-// The same at head_dim 128, where the prepared rotation holds the matrix as an operand of the matrix cores (entries x 64: see
-// akv_attn_common.h): a workgroup takes 16 rows, the eight of two items (sequence, kv head) each, rows past the group's heads
-// zero.  200 sequences of eight query heads: 8.6 us with the kernel above, whose workgroups read the 64 KB matrix for one or two
-// rows each, 6.6 here; for few rows that one is shorter (16 sequences: 4.1 against 6.6).
-template <int QDT>
-__global__ __launch_bounds__(256) void akv_attn_wave_prologue128_kernel(
-    const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const uint4* __restrict__ bop, int S, int QH, int KVH,
-    const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix, uint2* __restrict__ qop,
-    float* __restrict__ fac, uint32_t* __restrict__ status, float qscale, int bits, int32_t* __restrict__ wgdesc,
-    int32_t* __restrict__ seqw, int G, int shares) {
-  __shared__ __align__(16) float q_lds[16][132];
-  __shared__ __align__(16) float y_lds[16][132];
-  __shared__ int32_t scratch[257];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (blockIdx.x == 0) {
-    if (tid == 0) status[0] = 0u;
-    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares);
-    return;
-  }
-  // wavefront w owns the operand's N-tiles 2 w and 2 w + 1: lane (col, g) = output coordinate 8 col + N-tile
-  const int col = lane & 15, g = lane >> 4, gqa = QH / KVH, nq = S * KVH;
-  akv_half8 bh[2][4], bl[2][4];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const int idx = ((2 * wave + t) * 4 + ks) * 64 + lane;
-      bh[t][ks] = akv_as_half8(bop[idx]);
-      bl[t][ks] = akv_as_half8(bop[2048 + idx]);
-    }
-  for (int pair = (int)blockIdx.x - 1; 2 * pair < nq; pair += (int)gridDim.x - 1) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int row = 2 * i + (tid >> 7), j = tid & 127, item = 2 * pair + (row >> 3), q = row & 7;
-      const int s = item / KVH, h = item % KVH;
-      q_lds[row][j] = item < nq && q < gqa ? akv_elem<QDT>::load(query, s * qs_seq + (h * gqa + q) * qs_head + j) : 0.f;
-    }
-    __syncthreads();
-    float v[4][8];
-    float m = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const float4 x0 = *(const float4*)&q_lds[col][32 * g + 8 * ks], x1 = *(const float4*)&q_lds[col][32 * g + 8 * ks + 4];
-      v[ks][0] = x0.x; v[ks][1] = x0.y; v[ks][2] = x0.z; v[ks][3] = x0.w;
-      v[ks][4] = x1.x; v[ks][5] = x1.y; v[ks][6] = x1.z; v[ks][7] = x1.w;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(v[ks][e]));
-    }
-    const uint32_t ex = akv_row_exponent(akv_rows_max(m));
-    const float sc = akv_row_scale(ex), usc = akv_row_unscale(ex) * (1.f / 64.f);      // of row `col`
-    akv_float4v acc[2];
-    acc[0] = (akv_float4v){0.f, 0.f, 0.f, 0.f};
-    acc[1] = (akv_float4v){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      akv_half8 hi, lo;
-      akv_split8(v[ks], sc, hi, lo);
-      acc[0] = akv_mfma3(hi, lo, bh[0][ks], bl[0][ks], acc[0]);
-      acc[1] = akv_mfma3(hi, lo, bh[1][ks], bl[1][ks], acc[1]);
-    }
-    // lane (col, g) holds rows 4 g + i at coordinates 8 col + 2 wave and + 1
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float u = __shfl(usc, 4 * g + i);
-      *(float2*)&y_lds[4 * g + i][8 * col + 2 * wave] = make_float2(acc[0][i] * u, acc[1][i] * u);
-    }
-    __syncthreads();
-    // wavefront w writes rows 4 w .. 4 w + 3: lane l % 32 = quarter and step, four coordinates; lanes 0..31 the rounding,
-    // 32..63 the remainder (2-bit codes are looked up as (0, 2) and (1, 3))
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 4 * wave + i, item = 2 * pair + (row >> 3), q = row & 7;
-      const float4 y = *(const float4*)&y_lds[row][4 * (lane & 31)];
-      const float mx = akv_wave_max(fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
-      const uint32_t ey = akv_row_exponent(mx);
-      const float s1 = akv_row_scale(ey);
-      float c[4] = {y.x * s1, y.y * s1, y.z * s1, y.w * s1};
-      if (bits == 2) { const float t = c[1]; c[1] = c[2]; c[2] = t; }
-      uint32_t w[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const __half hi = __float2half_rn(c[e]);
-        w[e] = __half_as_ushort(lane < 32 ? hi : __float2half_rn(c[e] - __half2float(hi)));
-      }
-      if (item < nq) {
-        qop[(size_t)item * (8 * 64) + (lane & 7) * 64 + 16 * ((lane >> 3) & 3) + (lane >> 5) * 8 + q] = make_uint2(w[0] | (w[1] << 16), w[2] | (w[3] << 16));
-        if (lane == 0 && q < gqa) fac[(size_t)(item / KVH) * QH + (item % KVH) * gqa + q] = akv_row_unscale(ey) * qscale;
-      }
-    }
-    // (the next rows are written behind this loop's first barrier's readers: q_lds is read before the second barrier, and
-    // y_lds is written behind the next first one)
-  }
+  ar_rotate_queries<D, QDT, false>(rows, (int)blockIdx.x - 1, (int)gridDim.x - 1, query, qs_seq, qs_head, Pi, scale, S, QH, KVH, slots, qop, fac, qscale, bits);
 }
 
 // ----------------------------------------------------------------------------------
@@ -868,27 +721,16 @@ int akv_attn_wave_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs
   x.hp = 0;
   const float qscale = a.scale * 1.4426950408889634f;   // scores come out in the log2 domain
   const int slots = aw_slots(a.KVH, d == 64 ? 16 : 8), shares = (d == 64 ? 16 : 8) / slots;
-  // rotation blocks: one per query head, up to what the CUs hold at once (then they loop: the matrix is read once per block)
-  const int cus = akv_cached_cu_count();
-  auto pgrid = [&](int dd) {
-    const int64_t most = (int64_t)(cus > 0 ? cus : 256) * (dd == 256 ? 1 : 4) / (dd == 256 ? 2 : 1), items = (int64_t)a.S * a.QH;
-    return (int)(items < most ? items : most) + 1;
-  };
-#define AW_PRO(DD, DT) akv_attn_wave_prologue_kernel<DD, DT><<<pgrid(DD), aw_pro_threads<DD>(), 0, stream>>>(query, qs_seq, qs_head, PiT, a.S, a.QH, a.KVH, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint2*)extra_ws, ws.qrot, ws.status, qscale, bits, ws.wgdesc, ws.seqw, grid, shares)
+  const int cus = akv_cached_cu_count(), qslots = a.QH / a.KVH <= 4 ? 4 : 8;
+  // rotation blocks, up to three on a CU (then they loop: a slice of the matrix is read once per block)
+  const int pgrid = ar_query_blocks(d, a.S, a.KVH, qslots, 3 * (cus > 0 ? cus : 256)) + 1;
+  const float* Pi = PiT - (size_t)d * d;
+  const akv_prep_scale* scale = (const akv_prep_scale*)((const char*)Pi + AKV_PREP_SCALE_OFFSET(d));
+#define AW_PRO(DD, DT) akv_attn_wave_prologue_kernel<DD, DT><<<pgrid, 256, 0, stream>>>(query, qs_seq, qs_head, Pi, scale, a.S, a.QH, a.KVH, qslots, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint2*)extra_ws, ws.qrot, ws.status, qscale, bits, ws.wgdesc, ws.seqw, grid, shares)
 #define AW_PRO_D(DD) do { if (q_dtype == AKV_F16) AW_PRO(DD, AKV_F16); else if (q_dtype == AKV_BF16) AW_PRO(DD, AKV_BF16); else AW_PRO(DD, AKV_F32); } while (0)
-  // (16 rows a workgroup; its registers admit three on a CU)
-  const int64_t pairs = ((int64_t)a.S * a.KVH + 1) / 2, most128 = (int64_t)(cus > 0 ? cus : 256) * 3;
-  const int grid128 = (int)(pairs < most128 ? pairs : most128) + 1;
-#define AW_PRO128(DT) akv_attn_wave_prologue128_kernel<DT><<<grid128, 256, 0, stream>>>(query, qs_seq, qs_head, (const uint4*)(PiT + 128 * 128), a.S, a.QH, a.KVH, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint2*)extra_ws, ws.qrot, ws.status, qscale, bits, ws.wgdesc, ws.seqw, grid, shares)
-  // (a row a workgroup while three on a CU hold them all: 512 rows 4.8 | 6.0 us, 1,024 rows 7.3 | 6.5)
-  const bool plain128 = (int64_t)a.S * a.QH <= most128;
   if (d == 64) AW_PRO_D(64);
-  else if (d == 256) AW_PRO_D(256);
-  else if (plain128) AW_PRO_D(128);
-  else if (q_dtype == AKV_F16) AW_PRO128(AKV_F16);
-  else if (q_dtype == AKV_BF16) AW_PRO128(AKV_BF16);
-  else AW_PRO128(AKV_F32);
-#undef AW_PRO128
+  else if (d == 128) AW_PRO_D(128);
+  else AW_PRO_D(256);
 #undef AW_PRO_D
 #undef AW_PRO
   AKV_LAUNCH_CHECK("akv_attn_wave_prologue_kernel");
