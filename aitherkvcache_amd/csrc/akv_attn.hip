@@ -5,7 +5,7 @@
 // This file holds the prologue, the reduce and the general main kernel (any of the three
 // bit widths, head_dim 64/128/256).  The MFMA main kernel for 4-bit / head_dim 128 is in
 // akv_attn_mfma.hip and plugs into the same prologue / reduce.
-#include "akv_attn_common.h"
+#include "akv_attn_rows.h"
 
 
 // ----------------------------------------------------------------------------------
@@ -473,6 +473,164 @@ static int akv_launch_attn_general_gq(const akv_attn_args& a, int grid, hipStrea
   return AKV_OK;
 }
 
+// ----------------------------------------------------------------------------------
+// reduce of head_dim 256 after the matrix-core kernel: 4 MR (sequence, query head) rows a workgroup at a time.  A wavefront
+// merges MR rows, RR_PF / MR slots of each requested ahead, and leaves them in LDS as two float16 terms; then it multiplies all
+// rows by its 64 outputs of Pi^T, which it holds in registers for all rows of the workgroup (the operand of the decode kernel in
+// the prepared buffer, requested behind the first partial results; one workgroup a CU).
+// On the vector unit, four heads a workgroup against all of the matrix, it took 13.5 us for 24 sequences of 16 heads, 8.8 now.
+// ----------------------------------------------------------------------------------
+#define RR_PF 16
+template <int ODT, int MR>
+__global__ __launch_bounds__(256, 1) void akv_attn_reduce_rows_kernel(
+    const float* __restrict__ part_acc, const float* __restrict__ part_ml, const uint4* __restrict__ slices, const akv_prep_scale* __restrict__ scale,
+    int S, int QH, void* __restrict__ out, int64_t os_seq, int64_t os_head, const uint32_t* __restrict__ status, const int32_t* __restrict__ seqw) {
+  constexpr int D = 256, PF = RR_PF / MR, ROWS = 4 * MR;
+  __shared__ __align__(16) ar_rows<D> rows;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int nrow = S * QH, items = (nrow + ROWS - 1) / ROWS;
+  constexpr int OB = ODT == AKV_F32 ? 4 : 2;
+  const bool wide = (((uintptr_t)out | (uintptr_t)(os_seq * OB) | (uintptr_t)(os_head * OB)) & 15) == 0;
+  float4 pre[MR][PF];
+  float2 ml[MR];                           // lane u: slot u
+  int n[MR];
+  size_t at[MR];                           // first slot of a row, in rows of partial results
+  auto request = [&](int item) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < MR; ++j) {
+      const int row = min(item * ROWS + MR * wave + j, nrow - 1), s = row / QH, h = row % QH;      // (past the end: the last row, not stored)
+      const int w_lo = seqw[2 * s];
+      n[j] = seqw[2 * s + 1] - w_lo + 1;
+      at[j] = (size_t)(w_lo + s) * QH + h;
+#pragma unroll
+      for (int u = 0; u < PF; ++u)
+        pre[j][u] = u < n[j] ? *(const float4*)(part_acc + (at[j] + (size_t)u * QH) * D + lane * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+      ml[j] = lane < n[j] ? *(const float2*)(part_ml + (at[j] + (size_t)lane * QH) * 2) : make_float2(-INFINITY, 0.f);
+    }
+  };
+  request(blockIdx.x);
+  __builtin_amdgcn_sched_barrier(0);
+  akv_half8 mh[4][8], mr[4][8];            // tile 4 wave + t, piece h: lane (m, g) coordinates 64 g + 8 h + e of output (t, m)
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int h = 0; h < 8; ++h) {
+      const int idx = ((4 * wave + t) * 8 + h) * 64 + lane;
+      mh[t][h] = akv_as_half8(slices[idx]);
+      mr[t][h] = akv_as_half8(slices[D * D / 8 + idx]);
+    }
+  const float up = scale->up * (AR_M_SCALE / 64.f);
+  // a main kernel whose bounded wait gave up has produced garbage: say so in every output
+  const float poison = status[0] != 0u ? __uint_as_float(0x7fc00000u) : 0.f;
+  __builtin_amdgcn_sched_barrier(0);
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+#pragma unroll
+    for (int j = 0; j < MR; ++j) {
+      float M = ml[j].x;
+      for (int u = 64 + lane; u < n[j]; u += 64) M = fmaxf(M, part_ml[(at[j] + (size_t)u * QH) * 2]);
+      M = akv_wave_max(M);
+      float l = 0.f;
+      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int u0 = 0; u0 < n[j]; u0 += 64) {
+        float2 x = ml[j];
+        if (u0 > 0) x = u0 + lane < n[j] ? *(const float2*)(part_ml + (at[j] + (size_t)(u0 + lane) * QH) * 2) : make_float2(-INFINITY, 0.f);
+        const float wgt = x.x > -INFINITY ? __expf(x.x - M) : 0.f;
+        l += wgt * x.y;
+        for (int v0 = u0; v0 < min(n[j], u0 + 64); v0 += PF) {
+          auto take = [&](int u) __attribute__((always_inline)) {
+            // (past the last slot: weight zero, what is held there is zeros or a slot again)
+            const float wu = v0 + u < n[j] ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), v0 - u0 + u)) : 0.f;
+            acc.x = fmaf(wu, pre[j][u].x, acc.x);
+            acc.y = fmaf(wu, pre[j][u].y, acc.y);
+            acc.z = fmaf(wu, pre[j][u].z, acc.z);
+            acc.w = fmaf(wu, pre[j][u].w, acc.w);
+          };
+          if (v0 + PF < n[j]) {
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+              take(u);
+              pre[j][u] = *(const float4*)(part_acc + (at[j] + (size_t)min(v0 + PF + u, n[j] - 1) * QH) * D + lane * 4);
+            }
+          } else {
+#pragma unroll
+            for (int u = 0; u < PF; ++u) take(u);
+          }
+        }
+      }
+      l = akv_wave_sum(l);
+      const float inv = l > 0.f ? 1.f / l : 1.f;
+      const float v[4] = {acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
+      float un;
+      const float sc = ar_scale(akv_wave_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])))), un);
+      ar_half4 hi, lo;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = v[i] * sc;
+        hi[i] = (_Float16)x;
+        lo[i] = (_Float16)(x - (float)hi[i]);
+      }
+      *(ar_half4*)&rows.term[0][MR * wave + j][lane * 4] = hi;
+      *(ar_half4*)&rows.term[1][MR * wave + j][lane * 4] = lo;
+      if (lane == 0) rows.unscale[MR * wave + j] = un * up;
+    }
+    if (item + (int)gridDim.x < items) request(item + gridDim.x);
+    __syncthreads();
+    akv_float4v y[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) y[t] = (akv_float4v){0.f, 0.f, 0.f, 0.f};
+    const int r = col & (ROWS - 1);
+#pragma unroll
+    for (int h = 0; h < 8; ++h) {
+      const akv_half8 x = *(const akv_half8*)&rows.term[0][r][64 * g + 8 * h], xl = *(const akv_half8*)&rows.term[1][r][64 * g + 8 * h];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        y[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(mh[t][h], x, y[t], 0, 0, 0);
+        y[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(mr[t][h], x, y[t], 0, 0, 0);
+        y[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(mh[t][h], xl, y[t], 0, 0, 0);
+      }
+    }
+    const int row = item * ROWS + col;
+    if (col < ROWS && row < nrow) {
+      const float u = rows.unscale[r];
+      const int64_t o = row / QH * os_seq + row % QH * os_head + 64 * wave + 8 * g;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {        // tiles 2 t and 2 t + 1: eight neighbouring outputs
+        union { typename akv_elem<ODT>::type e[8]; uint4 w[8 * OB / 16]; } x;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) akv_elem<ODT>::store(x.e, i, y[2 * t + (i >> 2)][i & 3] * u + poison);
+        if (wide) {
+#pragma unroll
+          for (int i = 0; i < 8 * OB / 16; ++i) ((uint4*)((char*)out + (o + 32 * t) * OB))[i] = x.w[i];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) akv_elem<ODT>::store(out, o + 32 * t + i, y[2 * t + (i >> 2)][i & 3] * u + poison);
+        }
+      }
+    }
+    __syncthreads();      // (the next rows go where these are)
+  }
+}
+
+static int akv_launch_reduce_rows(int odt, const akv_attn_args& a, const float* Pi, void* out, int64_t os_seq, int64_t os_head,
+                                  const uint32_t* status, const int32_t* seqw, hipStream_t stream) {
+  const int cus = akv_cached_cu_count() > 0 ? akv_cached_cu_count() : 256;
+  const int64_t nrow = (int64_t)a.S * a.QH;
+  // (sixteen rows at a time once four a CU are not all: 8,192 rows in one or two slots each, the step 115 us, 132 with four;
+  // 384 rows in ten slots each 62, 55 with four, 1,024 in three 57 and 53)
+  const bool many = nrow > (int64_t)4 * cus;
+  const int64_t items = many ? (nrow + 15) / 16 : (nrow + 3) / 4;
+  const int grid = (int)(items < cus ? items : cus);
+  const uint4* slices = (const uint4*)((const char*)Pi + AKV_PREP_SLICES_OFFSET(256));
+  const akv_prep_scale* scale = (const akv_prep_scale*)((const char*)Pi + AKV_PREP_SCALE_OFFSET(256));
+#define AKV_RR(DT) do { if (many) akv_attn_reduce_rows_kernel<DT, 4><<<grid, 256, 0, stream>>>(a.part_acc, a.part_ml, slices, scale, a.S, a.QH, out, os_seq, os_head, status, seqw); \
+                        else akv_attn_reduce_rows_kernel<DT, 1><<<grid, 256, 0, stream>>>(a.part_acc, a.part_ml, slices, scale, a.S, a.QH, out, os_seq, os_head, status, seqw); } while (0)
+  if (odt == AKV_F16) AKV_RR(AKV_F16); else if (odt == AKV_BF16) AKV_RR(AKV_BF16); else AKV_RR(AKV_F32);
+#undef AKV_RR
+  AKV_LAUNCH_CHECK("akv_attn_reduce_rows_kernel");
+  return AKV_OK;
+}
+
 template <int D, int BITS>
 static int akv_launch_attn_general(const akv_attn_args& a, int grid, hipStream_t stream) {
   const int gqa = a.QH / a.KVH;
@@ -577,6 +735,7 @@ static int akv_paged_attn_impl(
 #undef AKV_CASE
   }
   if (rc) return rc;
+  if (d == 256 && seqw != nullptr) return akv_launch_reduce_rows(out_dtype, a, Pi, out, os_seq, os_head, ws.status, seqw, stream);
   if (d == 64) return akv_launch_reduce<64>(out_dtype, a, Pi, nullptr, Gused, out, os_seq, os_head, ws.status, seqw, stream);
   if (d == 128) return akv_launch_reduce<128>(out_dtype, a, Pi, (const uint4*)((const char*)rot_prep + AKV_PREP_DECODE_OFFSET(128)), Gused, out, os_seq, os_head, ws.status, seqw, stream);
   if (d == 256) return akv_launch_reduce<256>(out_dtype, a, Pi, nullptr, Gused, out, os_seq, os_head, ws.status, seqw, stream);

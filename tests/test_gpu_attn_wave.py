@@ -83,6 +83,29 @@ def test_edges_of_3bit_rows_vs_float64(dev, d, qh, kvh, bs):
     test_edges_vs_float64(dev, d, 3, qh, kvh, bs)
 
 
+@pytest.mark.parametrize("seqs,qh,kvh", [(70, 15, 3), (64, 16, 4), (65, 16, 16), (2, 3, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_reduce_of_head_dim_256_at_its_row_counts(dev, seqs, qh, kvh, dtype):
+    """Around the number of rows from which sixteen are reduced at a time (four a CU), and row counts that no tile divides."""
+    rng, tq, rows, norms = make(dev, 256, 4, kvh, 12, 16, seqs)
+    ctx = rng.integers(0, 100, size=seqs).astype(np.int32)
+    tables = rng.integers(0, 12, size=(seqs, 7)).astype(np.int32)
+    q = torch.from_numpy(rng.standard_normal((seqs, qh, 256)).astype(np.float32)).to(dev).to(dtype)
+    P = tq._packed_dim
+    out = akv.TQPagedAttention(tq, qh).forward(q, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], torch.from_numpy(tables).to(dev),
+                                               torch.from_numpy(ctx).to(dev)).double().cpu()
+    K, V = (dequantised(tq, r, n, 256, 4) for r, n in zip(rows, norms))
+    R = tq.rotation.double().cpu()
+    for i, n in enumerate(ctx):
+        if n == 0:
+            assert not out[i].any()
+            continue
+        k, v = (x[torch.from_numpy(tables[i].astype(np.int64))].reshape(-1, kvh, 256)[:n] for x in (K, V))
+        ref = attend(q[i].double().cpu(), k, v, R)
+        # (bfloat16: the rounding of the output, 2^-9 of each)
+        assert (out[i] - ref).norm() <= (REL if dtype == torch.float32 else 2.0 ** -9) * ref.norm(), (i, n)
+
+
 @pytest.mark.parametrize("d,qh,kvh,bs,chunks", [(256, 16, 8, 16, 70), (256, 4, 1, 32, 70), (64, 16, 16, 32, 70),
                                                 (256, 8, 8, 16, 32), (256, 8, 8, 32, 64), (64, 16, 16, 16, 64), (64, 16, 16, 32, 32)])
 def test_more_chunks_than_a_window_of_block_ids(dev, d, qh, kvh, bs, chunks):
