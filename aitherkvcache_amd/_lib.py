@@ -108,6 +108,10 @@ SIGNATURES = {
 }
 
 _lib: Optional[C.CDLL] = None
+_calls = None          # the binding of the hot calls (csrc/akv_binding.cpp), once the library is loaded
+_BOUND = ("akv_paged_attn_workspace_bytes", "akv_paged_attn", "akv_encode_paged_kv", "akv_hybrid_paged_attn_workspace_bytes",
+          "akv_hybrid_paged_attn", "akv_hybrid25_paged_attn", "akv_hybrid_encode_paged_kv", "akv_hybrid25_encode_paged_kv",
+          "akv_decode_blocks_kv", "akv_tri_encode_paged", "akv_tri_decode_workspace_bytes", "akv_tri_decode_paged")
 
 
 def available() -> bool:
@@ -128,9 +132,26 @@ def lib() -> C.CDLL:
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
+        _bind(handle)
         handle.akv_last_error()       # the thread's thread-local block of the library, touched: see akv_touch_thread
         _lib = handle
     return _lib
+
+
+def _bind(handle: C.CDLL) -> None:
+    """Hand the functions of a loaded library to the binding of the hot calls."""
+    global _calls
+    from . import _binding
+    _binding.bind(torch._C._cuda_getCurrentRawStream, *(C.cast(getattr(handle, n), C.c_void_p).value for n in _BOUND))
+    _calls = _binding
+
+
+def calls():
+    """The binding: functions that take tensors and return a result, an akv_status, or None for a call that has to go the long
+    way (csrc/akv_binding.cpp says when)."""
+    if _calls is None:
+        lib()
+    return _calls
 
 
 class AkvError(RuntimeError):

@@ -70,11 +70,20 @@ class TQPagedAttention:
         k/v_packed [num_blocks, block_size, num_kv_heads, >= packed_dim] uint8 (may be strided
         views with 4-byte aligned rows), k/v_norms [num_blocks, block_size, num_kv_heads] float32,
         block_tables [num_seqs, max_blocks_per_seq] int32/int64, context_lens [num_seqs]."""
-        if num_kv_heads is None:
-            num_kv_heads = k_packed.shape[2]
         tq = self._tq
         if tq.rotation is not self.rotation:     # the quantizer's matrix was reassigned: follow it
             self.rotation = tq.rotation
+        if _static_out is None and self._block_selector is None and self._workspace is not None:
+            out = _lib.calls().uniform_attention(query, k_packed, k_norms, v_packed, v_norms, block_tables, context_lens, self.centroids,
+                                                 self._workspace, tq.prepared_rotation().ptr, num_kv_heads, self.num_query_heads,
+                                                 self.head_dim, self.packed_dim, self.bits, block_size, self.scale)
+            if out is not None:
+                if type(out) is int:
+                    _lib.check(out)
+                self._last_static = None
+                return out
+        if num_kv_heads is None:
+            num_kv_heads = k_packed.shape[2]
         if self._block_selector is not None:
             # as in the reference (:659-668): even / odd coordinates of the rotated query score the blocks,
             # the kernel then walks the filtered table

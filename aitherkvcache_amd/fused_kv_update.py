@@ -76,6 +76,11 @@ def fused_kv_update_pair(key, value, slot_mapping, k_packed, k_norms, v_packed, 
     kernel launch when the two tensors and the two caches have the same dtype, shapes and strides
     (key / value of a layer and the halves of a serving cache tensor do); two launches otherwise.
     Results equal two fused_kv_update calls."""
+    if prepared is not None:
+        rc = _lib.calls().uniform_encode(key, value, slot_mapping, k_packed, k_norms, v_packed, v_norms, rotation, boundaries,
+                                         prepared.ptr, bits, block_size, max_blocks)
+        if rc is not None:
+            return _lib.check(rc)
     same = (key.shape == value.shape and key.dtype == value.dtype and key.stride() == value.stride()
             and key.stride(-1) == 1 and key.dtype in (torch.float16, torch.bfloat16, torch.float32)
             and k_packed.shape == v_packed.shape and k_packed.stride() == v_packed.stride()
@@ -196,6 +201,12 @@ def fused_encode_and_store(tq_cache, layer_idx: int, key, value, slot_mapping) -
         plan = _StorePlan(tq_cache, layer_idx)
         plans[layer_idx] = plan
     f = plan.fixed
+    if f is not None and key.shape[1:] == plan.tail and key.shape[:1] == slot_mapping.shape:
+        kp, kn, vp, vn = plan.views
+        rc = _lib.calls().uniform_encode(key, value, slot_mapping, kp, kn, vp, vn, plan.rot, plan.bnd, f[0], f[2], plan.block_size,
+                                         plan.max_blocks)
+        if rc is not None:
+            return _lib.check(rc)
     if (f is not None and key.dtype in _DTYPE_OK and value.dtype is key.dtype and key.dim() == 3
             and key.shape[1:] == plan.tail and value.shape == key.shape and key.stride(2) == 1
             and key.stride() == value.stride() and key.device == plan.dev and value.device == plan.dev

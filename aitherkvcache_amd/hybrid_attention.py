@@ -14,6 +14,8 @@ import torch
 
 from . import _lib
 
+_FORMAT = {"akv_hybrid": 0, "akv_hybrid25": 1}
+
 
 def hybrid_encode_and_store(htq, x: torch.Tensor, slot_mapping: torch.Tensor, cache: torch.Tensor,
                             block_size: int = 16, max_blocks: int = 0) -> None:
@@ -49,6 +51,11 @@ def hybrid_encode_and_store_pair(htq, key: torch.Tensor, value: torch.Tensor, sl
     """K and V of a step (the two encodes of tq::hybrid_decode_step, reference vllm/hooks.py:271-284) in one call:
     one launch while the step is small.  Tensors or caches that differ in dtype, shape or strides go through
     hybrid_encode_and_store one after the other."""
+    if htq.group_order is None:
+        rc = _lib.calls().hybrid_encode(key, value, slot_mapping, k_cache, v_cache, htq.kernel_table, _FORMAT[htq._abi], htq.head_dim,
+                                        htq.packed_dim, block_size, max_blocks)
+        if rc is not None:
+            return _lib.check(rc)
     same = (key.shape == value.shape and key.dtype == value.dtype and key.stride() == value.stride()
             and key.dim() == 3 and key.stride(-1) == 1 and key.dtype in (torch.float16, torch.bfloat16, torch.float32)
             and k_cache.shape == v_cache.shape and k_cache.stride() == v_cache.stride()
@@ -85,11 +92,19 @@ class HybridPagedAttention:
 
     def forward(self, query, k_cache, v_cache, block_tables, context_lens, block_size: int = 16,
                 num_kv_heads: Optional[int] = None, scale: Optional[float] = None) -> torch.Tensor:
-        if num_kv_heads is None:
-            num_kv_heads = k_cache.shape[2]
         if scale is None:
             scale = 1.0 / (self.head_dim ** 0.5)
         table = self._htq.kernel_table
+        if self._workspace is not None and self._htq.group_order is None:
+            out = _lib.calls().hybrid_attention(query, k_cache, v_cache, block_tables, context_lens, table, self._workspace,
+                                                _FORMAT[self._htq._abi], num_kv_heads, self.num_query_heads, self.head_dim,
+                                                self._htq.packed_dim, block_size, scale)
+            if out is not None:
+                if type(out) is int:
+                    _lib.check(out)
+                return out
+        if num_kv_heads is None:
+            num_kv_heads = k_cache.shape[2]
         dev = _lib.require_gpu(query, k_cache, v_cache, block_tables, context_lens, table)
         num_seqs, num_q_heads, head_dim = query.shape
         if head_dim != self.head_dim or num_q_heads != self.num_query_heads:

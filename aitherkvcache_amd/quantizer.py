@@ -40,7 +40,7 @@ class TurboQuantConfig:
 def _rotation_key(rotation: torch.Tensor):
     """What tells one matrix from another without reading it: where it lies, how it is laid out there (a
     transposed view shares address and version with its base) and how often it has been written."""
-    return (rotation.data_ptr(), rotation._version, rotation.stride(), rotation.dtype, str(rotation.device))
+    return (rotation.data_ptr(), rotation._version, rotation.stride(), rotation.dtype, rotation.device)
 
 
 class PreparedRotation:

@@ -215,6 +215,14 @@ class TriAttention:
         with cache.fetch_sequence, cache.py:163-198, followed by decode_step).  query [B, QH, D];
         block_tables [B, max_blocks_per_seq] int32/int64; context_lens [B]; key positions are
         0..ctx-1 and query_pos defaults to ctx -> float32 [B, QH, D] (zeros where ctx == 0)."""
+        if query_pos is None and self._workspace is not None:
+            out = _lib.calls().spectral_attention(query, cache.k_indices, cache.k_packed, cache.k_scales, cache.v_indices, cache.v_packed,
+                                                  cache.v_scales, self._theta, block_tables, context_lens, self._workspace, self.head_dim,
+                                                  1 if self.config.pre_rope else 0)
+            if out is not None:
+                if type(out) is int:
+                    _lib.check(out)
+                return out
         dev = _lib.require_gpu(query, cache.k_indices, cache.k_packed, cache.k_scales, cache.v_indices,
                                cache.v_packed, cache.v_scales, block_tables, context_lens, query_pos)
         if self._theta.device != dev:

@@ -63,6 +63,10 @@ class SpectralKVCache:
         slot = block * block_size + position per token, one launch per tensor -- what the reference does with
         encode followed by store_token per token (cache.py:106-140).  Negative slots and slots past the cache are
         skipped.  No counterpart in the reference."""
+        rc = _lib.calls().spectral_encode(keys, values, slot_mapping, *self._arrays(), self.num_kv_heads, self.config.head_dim,
+                                          self.num_freqs, self.max_blocks * self.block_size)
+        if rc is not None:
+            return _lib.check(rc)
         T, KVH, D = keys.shape
         if KVH != self.num_kv_heads or D != self.config.head_dim or values.shape != keys.shape:
             raise ValueError(f"keys / values {tuple(keys.shape)} / {tuple(values.shape)} do not fit kv_heads="

@@ -68,6 +68,11 @@ def batch_decompress_active_blocks(key_cache, value_cache, k_buf, v_buf, tq, pac
     which the reference reads from class state (:1073-1075), are passed in."""
     if packed_dim != tq._packed_dim:
         raise ValueError(f"packed_dim {packed_dim} does not match the quantizer ({tq._packed_dim})")
+    if block_table.is_cuda and tq.rotation.is_cuda:
+        rc = _lib.calls().decode_blocks(key_cache, value_cache, k_buf, v_buf, block_table, k_norms, v_norms, tq.centroids,
+                                        tq.prepared_rotation().ptr, num_blocks, tq.head_dim, tq._packed_dim, tq.bits)
+        if rc is not None:
+            return _lib.check(rc)
     # one launch for both where the layouts agree and V's output does not lie within reach of K's
     if (key_cache.shape == value_cache.shape and key_cache.stride() == value_cache.stride()
             and k_norms.stride() == v_norms.stride() and k_buf.shape == v_buf.shape

@@ -1,0 +1,142 @@
+"""The binding of the hot calls takes plain well-formed calls and leaves every other one to the long way: both give the same bytes,
+and what the long way converts, allocates or refuses is converted, allocated or refused as before."""
+import contextlib
+
+import pytest
+import torch
+
+import aitherkvcache_amd as akv
+from aitherkvcache_amd import _lib
+from aitherkvcache_amd.hybrid_attention import hybrid_encode_and_store_pair
+from aitherkvcache_amd.triattention import TriAttention, TriAttentionConfig
+from aitherkvcache_amd.triattention.cache import SpectralKVCache
+from aitherkvcache_amd.vllm.decompress import batch_decompress_active_blocks
+
+pytestmark = pytest.mark.gpu
+S, QH, KVH, BS, NB = 3, 8, 2, 16, 20
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+class Counting:
+    """The binding with a count of the calls it took; taken=None: it takes none."""
+
+    def __init__(self, real, take):
+        self.real, self.take, self.taken = real, take, 0
+
+    def __getattr__(self, name):
+        def call(*args):
+            res = getattr(self.real, name)(*args) if self.take else None
+            self.taken += res is not None
+            return res
+        return call
+
+
+@contextlib.contextmanager
+def binding(monkeypatch, take):
+    c = Counting(_lib.calls(), take)
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "_calls", c)
+        yield c
+
+
+def uniform(dev, bits, d, dtype):
+    tq = akv.TurboQuant(head_dim=d, bits=bits, device=str(dev))
+    attn = akv.TQPagedAttention(tq, QH)
+
+    def run(x, slots, tables, lens, q):
+        rows = [torch.zeros(NB, BS, KVH, tq._packed_dim, dtype=torch.uint8, device=dev) for _ in range(2)]
+        norms = [torch.zeros(NB, BS, KVH, device=dev) for _ in range(2)]
+        akv.fused_kv_update_pair(x[0], x[1], slots, rows[0], norms[0], rows[1], norms[1], tq.rotation, tq.boundaries_inner, bits, BS, NB,
+                                 prepared=tq.prepared_rotation())
+        bufs = [torch.zeros(NB, BS, KVH, d, dtype=dtype, device=dev) for _ in range(2)]
+        batch_decompress_active_blocks(rows[0], rows[1], bufs[0], bufs[1], tq, tq._packed_dim, tables, NB, norms[0], norms[1])
+        return rows + norms + bufs + [attn.forward(q, rows[0], norms[0], rows[1], norms[1], tables, lens, block_size=BS)]
+    return run, 3
+
+
+def hybrid(dev, mode, d, dtype):
+    h = akv.HybridTurboQuant(head_dim=d, mode=mode, device=str(dev))
+    h.calibrate_uniform(KVH)
+    attn = akv.HybridPagedAttention(h, QH)
+
+    def run(x, slots, tables, lens, q):
+        rows = [torch.zeros(NB, BS, KVH, h.packed_dim, dtype=torch.uint8, device=dev) for _ in range(2)]
+        hybrid_encode_and_store_pair(h, x[0], x[1], slots, rows[0], rows[1], BS)
+        return rows + [attn.forward(q, rows[0], rows[1], tables, lens, block_size=BS)]
+    return run, 2
+
+
+def spectral(dev, _, d, dtype):
+    tri = TriAttention(TriAttentionConfig(head_dim=d, num_freqs=12, coeff_bits=4, num_kv_heads=KVH, num_query_heads=QH, block_size=BS), device=str(dev))
+
+    def run(x, slots, tables, lens, q):
+        cache = SpectralKVCache(tri.config, max_blocks=NB, device=str(dev))
+        cache.encode_and_store(x[0], x[1], slots)
+        return list(cache._arrays()) + [tri.decode_step_paged(q, cache, tables, lens)]
+    return run, 2
+
+
+CASES = [(uniform, 4, 128), (uniform, 3, 64), (uniform, 2, 256), (hybrid, "tq35", 128), (hybrid, "tq25", 128), (spectral, None, 128)]
+
+
+def inputs(dev, d, dtype, itype):
+    gen = torch.Generator(device=dev).manual_seed(d)
+    x = torch.randn(2, NB * BS, KVH, d, device=dev, generator=gen).to(dtype)
+    q = torch.randn(S, QH, d, device=dev, generator=gen).to(dtype)
+    tables = torch.randperm(NB, device=dev, generator=gen)[:S * 5].reshape(S, 5).to(itype)
+    lens = torch.tensor([80, 33, 1], device=dev, dtype=itype)
+    return x, torch.arange(NB * BS, device=dev, dtype=itype), tables, lens, q
+
+
+def check(got, want):
+    assert all(a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b) for a, b in zip(got, want, strict=True))
+
+
+@pytest.mark.parametrize("make,fmt,d", CASES)
+@pytest.mark.parametrize("dtype,itype", [(torch.float16, torch.int32), (torch.bfloat16, torch.int64), (torch.float32, torch.int64)])
+def test_binding_and_long_way_give_the_same(dev, monkeypatch, make, fmt, d, dtype, itype):
+    run, calls = make(dev, fmt, d, dtype)
+    args = inputs(dev, d, dtype, itype)
+    with binding(monkeypatch, False):
+        want = run(*args)
+    with binding(monkeypatch, True) as c:
+        check(run(*args), want)
+        assert c.taken == calls
+        x, slots, tables, lens, q = args
+        # every second token of a wider tensor, tables cut out of wider ones: as the strides say
+        wide, wt = torch.zeros(2, NB * BS, KVH + 1, d, dtype=dtype, device=dev), torch.full((S, 9), 10 ** 6, dtype=itype, device=dev)
+        wide[:, :, 1:], wt[:, 2:7] = x, tables
+        c.taken = 0
+        check(run(wide[:, :, 1:], slots, wt[:, 2:7], lens, q), want)
+        # the long way takes: transposed queries and tokens (copied), lengths of every second entry (copied), wrapped tensors
+        c.taken = 0
+        turned = q.transpose(1, 2).contiguous().transpose(1, 2)
+        check(run(x.transpose(2, 3).contiguous().transpose(2, 3), slots, tables, lens, turned), want)
+        check(run(x, slots, tables, lens.repeat_interleave(2)[::2], q), want)
+        before = c.taken
+        check(run([v.as_subclass(Sub) for v in x], slots, tables, lens, q), want)
+        assert c.taken > before                                     # (the calls without such a tensor)
+
+
+@pytest.mark.parametrize("make,fmt,d", CASES)
+def test_refusals_stay(dev, monkeypatch, make, fmt, d):
+    run, _ = make(dev, fmt, d, torch.float16)
+    x, slots, tables, lens, q = inputs(dev, d, torch.float16, torch.int32)
+    run(x, slots, tables, lens, q)                                  # the attention's workspace is there
+    refused = [(x, slots, tables, lens, q[:, :, :d // 2]), (x, slots, tables, lens, q[:, :5]), (x, slots, tables[0], lens, q), (x, slots, tables, lens, q.cpu())]
+    if make is not uniform:
+        refused.append((x[:, :, :, :d // 2], slots, tables, lens, q))
+    if make is spectral:
+        refused += [(x, slots[:5], tables, lens, q), (x, slots, tables, lens[:2], q)]
+    else:
+        refused.append((x, slots, tables.short(), lens, q))
+    for args in refused:
+        errors = []
+        for take in (False, True):
+            with binding(monkeypatch, take), pytest.raises(Exception) as e:
+                run(*args)
+            errors.append((e.type, str(e.value)))
+        assert errors[0] == errors[1]
