@@ -16,8 +16,6 @@
 #include "akv_attn_common.h"
 #include "akv_hybrid_layout.h"
 
-static bool hyb_lane_disabled();
-static bool hyb_lane_forced();
 static const float kHybKappa = (float)(1.2533141373155001 / 64.0);  // sqrt(pi/2) / 64
 
 __device__ __forceinline__ float hyb_half_bits_to_float(uint32_t b) {
@@ -107,147 +105,109 @@ __global__ __launch_bounds__(256) void hyb_encode_kernel(hyb_enc_args a) {
 }
 
 // ----------------------------------------------------------------------------------
-// encode, one LANE per vector (rows of 16-byte aligned input and output): the 64-point transforms run
+// encode, one LANE per group of a vector (rows of 16-byte aligned input and output): the 64-point transforms run
 // in the lane's registers, so no lane ever talks to another -- 384 additions per transform where the
 // wavefront-per-vector form above spends six shuffles per coordinate for one vector at a time.  Every
 // operation, the order of the butterflies and the order of the sums are those of the kernel above
 // (and of the reference); only the division is a reciprocal with one correction step.
+//
+// The two groups of a vector have nothing in common but the row they are written to: even wavefronts take group 0 of 64
+// vectors, odd ones group 1, and K and V are one launch.  What bounds it: vector instructions, some 45 a coordinate, as long as
+// there are several wavefronts per SIMD; below that, the chain of one lane.  K and V of 2,048 / 8,192 tokens of 8 heads:
+// 9.3 / 21.7 us; with both groups in one lane and a launch per tensor it was 42.9 (a wavefront per vector) / 47.1.
 // ----------------------------------------------------------------------------------
-// (The reference rounds every operation: the products come from akv_mul_rn, which the compiler may not
-// fuse into a multiply-add.  Where a product that is not exact feeds a tree of sums it also passes
-// through hyb_rounded(), an empty asm statement the optimiser cannot see through, so the tree is not
-// reassociated around it either.)
-__device__ __forceinline__ float hyb_rounded(float x) {
-  asm volatile("" : "+v"(x));
-  return x;
-}
-__device__ __forceinline__ void hyb_fwht64_regs(float (&v)[64]) {
-#pragma unroll
-  for (int h = 1; h < 64; h <<= 1)
-#pragma unroll
-    for (int i = 0; i < 64; ++i)
-      if ((i & h) == 0) {
-        const float lo = v[i], hi = v[i + h];
-        v[i] = akv_add_rn(lo, hi);
-        v[i + h] = akv_sub_rn(lo, hi);
-      }
-}
-// sum in the order of the wavefront reduction (partners 32, 16, ..., 1 apart)
-__device__ __forceinline__ float hyb_tree_sum64(float (&t)[64]) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1)
-#pragma unroll
-    for (int i = 0; i < m; ++i) t[i] = akv_add_rn(t[i], t[i + m]);
-  return t[0];
-}
-__device__ __forceinline__ void hyb_put_byte(uint32_t* words, int k, uint32_t byte) { words[k >> 2] |= byte << (8 * (k & 3)); }
-
-// one group of 64 coordinates of the lane's vector -> MB-bit codes, sign bits and the two norms as
-// dwords of the packed row (6 / 4 dwords of codes, 2 of signs, 1 of norms)
+// one group of 64 coordinates -> MB-bit codes, sign bits and the two norms as dwords of the packed row (6 / 4 dwords of codes,
+// 2 of signs, 1 of norms).  had, qjl, bnd: the same for all lanes (scalar loads); cen in LDS.
 template <int XDT, int MB>
-__device__ __forceinline__ void hyb_encode_group_lane(const void* x, int64_t off, const float* had,
-                                                       const float* qjl, const float* cen, const float* bnd,
-                                                       uint32_t* words) {
+__device__ __forceinline__ void hyb_encode_group_lane(const void* x, int64_t off, hyb_uniform had, hyb_uniform qjl, const float* cen,
+                                                      hyb_uniform bnd_, uint32_t* words) {
   constexpr int CW = 64 * MB / 32;       // dwords of codes
-  float u[64], v[64];
-  if constexpr (XDT == AKV_F32) {
-    const float4* p = (const float4*)((const float*)x + off);
+  float u[64], v[64], bnd[(1 << MB) - 1];
+  hyb_load_row<XDT, 64>(x, off, u);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) { const float4 q = p[i]; u[4 * i] = q.x; u[4 * i + 1] = q.y; u[4 * i + 2] = q.z; u[4 * i + 3] = q.w; }
-  } else {
-    const uint4* p = (const uint4*)((const unsigned short*)x + off);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint4 q = p[i];
-      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (XDT == AKV_F16) {
-          u[8 * i + 2 * j] = __half2float(__ushort_as_half((unsigned short)(w[j] & 0xffffu)));
-          u[8 * i + 2 * j + 1] = __half2float(__ushort_as_half((unsigned short)(w[j] >> 16)));
-        } else {
-          u[8 * i + 2 * j] = __uint_as_float(w[j] << 16);
-          u[8 * i + 2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-        }
-      }
-    }
-  }
+  for (int k = 0; k < (1 << MB) - 1; ++k) bnd[k] = bnd_[k];
 #pragma unroll
   for (int j = 0; j < 64; ++j) v[j] = hyb_rounded(akv_mul_rn(u[j], u[j]));
-  const float nrm = sqrtf(hyb_tree_sum64(v));
+  const float nrm = sqrtf(hyb_tree_sum<64>(v));
   const float den = akv_add_rn(nrm, 1e-10f);
   const float rcp = __frcp_rn(den);
-  const bool plain = !(den < INFINITY);
+  // x / den: reciprocal, then one correction step (the correctly rounded quotient but for rare ties).  An infinite or NaN norm:
+  // x * (1 / den) alone already is what the division gives; a divisor of 0 in the correction leaves it as it is.
+  // (The divisor is negated, not the quotient: a NaN keeps its sign.)
+  const float neg_den = den < INFINITY ? -den : 0.f;
 #pragma unroll
   for (int j = 0; j < 64; ++j) {
-    // x / den: reciprocal, then one correction step (the correctly rounded quotient but for rare ties)
     const float q0 = akv_mul_rn(u[j], rcp);
-    const float e = fmaf(-q0, den, u[j]);
-    // (an infinite or NaN norm: x * (1 / den) alone already is what the division gives)
-    const float q = plain ? q0 : fmaf(e, rcp, q0);
-    u[j] = q;
-    v[j] = akv_mul_rn(q, had[j]);
+    u[j] = fmaf(fmaf(q0, neg_den, u[j]), rcp, q0);
+    v[j] = akv_mul_rn(u[j], had[j]);
   }
-  hyb_fwht64_regs(v);
-#pragma unroll
-  for (int k = 0; k < CW + 3; ++k) words[k] = 0u;
+  hyb_fwht_regs<64>(v);
   // codes: MSB-first stream; the centroid of every code goes straight into the next transform
   if constexpr (MB == 3) {
 #pragma unroll
-    for (int g = 0; g < 8; ++g) {
-      uint32_t g24 = 0;
+    for (int h = 0; h < 2; ++h) {
+      uint32_t g24[4];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t c = akv_search<3>(akv_mul_rn(v[8 * g + i], 0.125f), bnd);
-        g24 |= c << (21 - 3 * i);
-        v[8 * g + i] = cen[c];
+      for (int g = 0; g < 4; ++g) {
+        g24[g] = 0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          float& r = v[32 * h + 8 * g + i];
+          hyb_append_code<3>(g24[g], akv_mul_rn(r, 0.125f), bnd);
+          r = cen[g24[g] & 7u];
+        }
       }
-      hyb_put_byte(words, 3 * g, g24 >> 16);
-      hyb_put_byte(words, 3 * g + 1, (g24 >> 8) & 0xffu);
-      hyb_put_byte(words, 3 * g + 2, g24 & 0xffu);
+      words[3 * h] = __builtin_bswap32((g24[0] << 8) | (g24[1] >> 16));
+      words[3 * h + 1] = __builtin_bswap32((g24[1] << 16) | (g24[2] >> 8));
+      words[3 * h + 2] = __builtin_bswap32((g24[2] << 24) | g24[3]);
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      uint32_t b = 0;
+    for (int k = 0; k < 4; ++k) {
+      uint32_t w = 0u;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t c = akv_search<2>(akv_mul_rn(v[4 * k + i], 0.125f), bnd);
-        b |= c << (6 - 2 * i);
-        v[4 * k + i] = cen[c];
+      for (int i = 0; i < 16; ++i) {
+        hyb_append_code<2>(w, akv_mul_rn(v[16 * k + i], 0.125f), bnd);
+        v[16 * k + i] = cen[w & 3u];
       }
-      hyb_put_byte(words, k, b);
+      words[k] = __builtin_bswap32(w);
     }
   }
-  hyb_fwht64_regs(v);
+  hyb_fwht_regs<64>(v);
 #pragma unroll
   for (int j = 0; j < 64; ++j) {
     const float mse_hat = akv_mul_rn(akv_mul_rn(v[j], had[j]), 0.125f);
     u[j] = akv_sub_rn(u[j], mse_hat);              // residual
     v[j] = hyb_rounded(akv_mul_rn(u[j], u[j]));
   }
-  const float rn = sqrtf(hyb_tree_sum64(v));
+  const float rn = sqrtf(hyb_tree_sum<64>(v));
 #pragma unroll
   for (int j = 0; j < 64; ++j) v[j] = akv_mul_rn(u[j], qjl[j]);
-  hyb_fwht64_regs(v);
+  hyb_fwht_regs<64>(v);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    uint32_t b = 0;
+  for (int k = 0; k < 2; ++k) {
+    uint32_t w = 0u;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) b |= (akv_mul_rn(v[8 * k + i], 0.125f) >= 0.f ? 1u : 0u) << (7 - i);
-    hyb_put_byte(words + CW, k, b);
+    for (int i = 0; i < 32; ++i) hyb_append_sign(w, akv_mul_rn(v[32 * k + i], 0.125f));
+    words[CW + k] = __builtin_bswap32(w);
   }
   words[CW + 2] = (uint32_t)__half_as_ushort(__float2half_rn(nrm)) | ((uint32_t)__half_as_ushort(__float2half_rn(rn)) << 16);
 }
 
 template <int XDT, bool PAGED>
 __global__ __launch_bounds__(256) void hyb_encode_lane_kernel(hyb_enc_args a) {
-  __shared__ float tab[AKV_HYB_TABLE_FLOATS];
-  for (int i = threadIdx.x; i < AKV_HYB_TABLE_FLOATS; i += 256) tab[i] = a.table[i];
+  __shared__ float cen[12];              // 8 centroids of group 0, 4 of group 1
+  if (threadIdx.x < 12) cen[threadIdx.x] = a.table[HYB_CEN0 + threadIdx.x];
+  static_assert(HYB_CEN1 == HYB_CEN0 + 8, "the two codebooks lie together");
   __syncthreads();
-  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (n >= a.n) return;
-  uint8_t* dst;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int64_t n = (int64_t)blockIdx.x * 128 + (wave >> 1) * 64 + (threadIdx.x & 63);
+  const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n;
+  if (n >= n_total) return;
+  const bool second = PAGED && n >= a.n;
+  if (second) n -= a.n;
+  const void* x = second ? a.x2 : a.x;
+  uint8_t* dst = second ? a.out2 : a.out;
   int64_t off;
   if (PAGED) {
     const int64_t tok = n / a.heads, head = n - tok * a.heads;
@@ -256,17 +216,24 @@ __global__ __launch_bounds__(256) void hyb_encode_lane_kernel(hyb_enc_args a) {
     if (slot < 0) return;
     const int64_t blk = slot / a.block_size, pos = slot - blk * a.block_size;
     if (blk >= a.max_blocks) return;
-    dst = a.out + blk * a.ps0 + pos * a.ps1 + head * a.ps2;
+    dst += blk * a.ps0 + pos * a.ps1 + head * a.ps2;
   } else {
     off = n * a.xs0;
-    dst = a.out + n * a.ps0;
+    dst += n * a.ps0;
   }
-  uint32_t row[16];
-  hyb_encode_group_lane<XDT, 3>(a.x, off, tab + HYB_HAD0, tab + HYB_QJL0, tab + HYB_CEN0, tab + HYB_BND0, row);
-  hyb_encode_group_lane<XDT, 2>(a.x, off + 64, tab + HYB_HAD1, tab + HYB_QJL1, tab + HYB_CEN1, tab + HYB_BND1, row + 9);
-  uint4* d4 = (uint4*)dst;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) d4[i] = make_uint4(row[4 * i], row[4 * i + 1], row[4 * i + 2], row[4 * i + 3]);
+  hyb_uniform tab = (hyb_uniform)a.table;
+  uint32_t row[9];
+  if ((wave & 1) == 0) {                 // dwords 0 .. 8 of the row
+    hyb_encode_group_lane<XDT, 3>(x, off, tab + HYB_HAD0, tab + HYB_QJL0, cen, tab + HYB_BND0, row);
+    ((uint4*)dst)[0] = make_uint4(row[0], row[1], row[2], row[3]);
+    ((uint4*)dst)[1] = make_uint4(row[4], row[5], row[6], row[7]);
+    ((uint32_t*)dst)[8] = row[8];
+  } else {                               // dwords 9 .. 15
+    hyb_encode_group_lane<XDT, 2>(x, off + 64, tab + HYB_HAD1, tab + HYB_QJL1, cen + 8, tab + HYB_BND1, row);
+    ((uint32_t*)dst)[9] = row[0];
+    ((uint2*)dst)[5] = make_uint2(row[1], row[2]);
+    ((uint4*)dst)[3] = make_uint4(row[3], row[4], row[5], row[6]);
+  }
 }
 
 // ----------------------------------------------------------------------------------
@@ -308,21 +275,30 @@ __global__ __launch_bounds__(256) void hyb_decode_kernel(const uint8_t* __restri
   }
 }
 
-// decode, one lane per vector (16-byte aligned rows): the same operations as above, transforms in registers
+// decode, one lane per group of a vector (16-byte aligned rows): the same operations as above, transforms in registers; even
+// wavefronts take group 0 of 64 vectors, odd ones group 1.  The values go out through LDS, eight lanes a row.  What bounds it:
+// memory, and a chain of 8 us whatever the size.  Four sequences of
+// 2,000 to 8,000 tokens of 8 heads: 19.5 us; a lane per vector that wrote its row itself took 33.
 template <int MB>
-__device__ __forceinline__ void hyb_decode_group_lane(const uint32_t* words, const float* had, const float* qjl,
-                                                       const float* cen, float kappa, float* out) {
+__device__ __forceinline__ void hyb_decode_group_lane(const uint32_t* words, hyb_uniform had, hyb_uniform qjl, const float* cen, float kappa, float* v) {
   constexpr int CW = 64 * MB / 32;
-  auto byte_of = [&](int k) { return (words[k >> 2] >> (8 * (k & 3))) & 0xffu; };
-  float v[64], w[64];
+  float w[64];
+  uint32_t c[CW + 1], sign[2];
+#pragma unroll
+  for (int k = 0; k < CW; ++k) c[k] = __builtin_bswap32(words[k]);
+  c[CW] = 0u;
+  sign[0] = ~__builtin_bswap32(words[CW]);
+  sign[1] = ~__builtin_bswap32(words[CW + 1]);
 #pragma unroll
   for (int j = 0; j < 64; ++j) {
-    v[j] = cen[akv_stream_code<MB>(j, byte_of)];
-    const uint32_t bit = (byte_of(4 * CW + (j >> 3)) >> (7 - (j & 7))) & 1u;
-    w[j] = bit ? kappa : -kappa;
+    constexpr uint32_t MASK = (1u << MB) - 1u;
+    const int at = j * MB, in = at & 31;           // MB bits of the MSB-first stream from bit `at` on
+    const uint32_t code = in + MB <= 32 ? c[at >> 5] >> (32 - MB - in) : __builtin_amdgcn_alignbit(c[at >> 5], c[(at >> 5) + 1], 64 - MB - in);
+    v[j] = cen[code & MASK];
+    w[j] = __uint_as_float(__float_as_uint(kappa) | ((sign[j >> 5] << (j & 31)) & 0x80000000u));
   }
-  hyb_fwht64_regs(v);
-  hyb_fwht64_regs(w);
+  hyb_fwht_regs<64>(v);
+  hyb_fwht_regs<64>(w);
   const float n = hyb_half_bits_to_float(words[CW + 2]);
   const float rn = hyb_half_bits_to_float(words[CW + 2] >> 16);
 #pragma unroll
@@ -331,25 +307,41 @@ __device__ __forceinline__ void hyb_decode_group_lane(const uint32_t* words, con
     const float qjl_hat = akv_mul_rn(akv_mul_rn(w[j], qjl[j]), 0.125f);
     v[j] = akv_mul_rn(akv_add_rn(mse_hat, hyb_rounded(akv_mul_rn(qjl_hat, rn))), n);
   }
-  float4* o4 = (float4*)out;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) o4[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
 }
 
 __global__ __launch_bounds__(256) void hyb_decode_lane_kernel(const uint8_t* __restrict__ packed, int64_t ps,
                                                               int64_t n_vec, const float* __restrict__ table,
                                                               float kappa, float* __restrict__ out, int64_t os) {
-  __shared__ float tab[AKV_HYB_TABLE_FLOATS];
-  for (int i = threadIdx.x; i < AKV_HYB_TABLE_FLOATS; i += 256) tab[i] = table[i];
+  __shared__ float cen[12];              // 8 centroids of group 0, 4 of group 1
+  __shared__ __align__(16) float turn[4][HYB_TURN_FLOATS];
+  if (threadIdx.x < 12) cen[threadIdx.x] = table[HYB_CEN0 + threadIdx.x];
   __syncthreads();
-  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (n >= n_vec) return;
-  uint32_t row[16];
-  const uint4* p = (const uint4*)(packed + n * ps);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) { const uint4 q = p[i]; row[4 * i] = q.x; row[4 * i + 1] = q.y; row[4 * i + 2] = q.z; row[4 * i + 3] = q.w; }
-  hyb_decode_group_lane<3>(row, tab + HYB_HAD0, tab + HYB_QJL0, tab + HYB_CEN0, kappa, out + n * os);
-  hyb_decode_group_lane<2>(row + 9, tab + HYB_HAD1, tab + HYB_QJL1, tab + HYB_CEN1, kappa, out + n * os + 64);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t n0 = (int64_t)blockIdx.x * 128 + (wave >> 1) * 64;
+  if (n0 >= n_vec) return;
+  const int64_t n = n0 + lane < n_vec ? n0 + lane : n_vec - 1;       // past the end: read, not stored
+  const uint8_t* p = packed + n * ps;
+  hyb_uniform tab = (hyb_uniform)table;
+  float v[64];
+  uint32_t row[9];
+  if ((wave & 1) == 0) {                 // dwords 0 .. 8 of the row
+    const uint4 a = ((const uint4*)p)[0], b = ((const uint4*)p)[1];
+    row[0] = a.x; row[1] = a.y; row[2] = a.z; row[3] = a.w;
+    row[4] = b.x; row[5] = b.y; row[6] = b.z; row[7] = b.w;
+    row[8] = ((const uint32_t*)p)[8];
+    hyb_decode_group_lane<3>(row, tab + HYB_HAD0, tab + HYB_QJL0, cen, kappa, v);
+  } else {                               // dwords 9 .. 15
+    const uint2 a = ((const uint2*)p)[5];
+    const uint4 b = ((const uint4*)p)[3];
+    row[0] = ((const uint32_t*)p)[9];
+    row[1] = a.x; row[2] = a.y;
+    row[3] = b.x; row[4] = b.y; row[5] = b.z; row[6] = b.w;
+    hyb_decode_group_lane<2>(row, tab + HYB_HAD1, tab + HYB_QJL1, cen + 8, kappa, v);
+  }
+  float* o = out + n0 * os + 64 * (wave & 1);
+  const int rows = (int)(n_vec - n0 < 64 ? n_vec - n0 : 64);
+  hyb_store_turned(v, turn[wave], o, os, rows, lane);
+  hyb_store_turned(v + 32, turn[wave], o + 32, os, rows, lane);
 }
 
 // ----------------------------------------------------------------------------------
@@ -595,32 +587,15 @@ static int hyb_grid(int64_t n) {
   return (int)(g < 1 ? 1 : (g > cap ? cap : g));
 }
 
-static bool hyb_lane_forced() {
-  const char* e = getenv("AKV_HYBRID_LANE_ENCODE");        // (read per call: tests switch it)
-  return e && e[0] == '1';
-}
-
-static bool hyb_lane_disabled() {
-  static int v = -1;
-  if (v < 0) {
-    const char* e = getenv("AKV_HYBRID_WAVE_ENCODE");
-    v = (e && e[0] == '1') ? 1 : 0;
-  }
-  return v == 1;
-}
-
+// From here on a lane per group: 8.6 us up to 16 K vectors, then rising with the wavefronts per SIMD; a wavefront per vector takes
+// 4.6 us for 2,048 vectors, 8.8 for 8,192 and 15.4 for 16,384 (8 heads, bfloat16, K and V together).
+#define HYB_LANE_MIN 8192
 template <bool PAGED>
 static int hyb_launch_encode(int dt, const hyb_enc_args& a, hipStream_t stream) {
-  // 16-byte aligned input rows and packed rows: one lane per vector
-  const int64_t xal = dt == AKV_F32 ? 3 : 7;      // elements per 16 bytes, minus one
-  // ... and enough of them: a lane walks its vector's six transforms alone (20 us however few vectors there are),
-  // a wavefront per vector takes 7 us for a serving step of 2,048 vectors and 0.8 ns more per vector; they meet
-  // near 16 K vectors
-  const bool lane_form = (((uintptr_t)a.x | (uintptr_t)a.out | (uintptr_t)a.ps0 | (uintptr_t)(PAGED ? a.ps1 | a.ps2 : 0)) & 15) == 0 &&
-                         ((a.xs0 | (PAGED ? a.xs1 : 0)) & xal) == 0 && !hyb_lane_disabled() &&
-                         (a.n >= 16384 || hyb_lane_forced()) && a.x2 == nullptr;
-  if (lane_form) {
-    const int lgrid = (int)((a.n + 255) / 256);
+  const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n;
+  if (hyb_lane_aligned(a.x, a.x2, a.xs0, PAGED ? a.xs1 : 0, dt, a.out, a.out2, a.ps0 | (PAGED ? a.ps1 | a.ps2 : 0), 16) &&
+      hyb_lane_form(n_total >= HYB_LANE_MIN)) {
+    const int lgrid = (int)((n_total + 127) / 128);
     switch (dt) {
       case AKV_F16: hyb_encode_lane_kernel<AKV_F16, PAGED><<<lgrid, 256, 0, stream>>>(a); break;
       case AKV_BF16: hyb_encode_lane_kernel<AKV_BF16, PAGED><<<lgrid, 256, 0, stream>>>(a); break;
@@ -629,7 +604,7 @@ static int hyb_launch_encode(int dt, const hyb_enc_args& a, hipStream_t stream) 
     AKV_LAUNCH_CHECK("hyb_encode_lane_kernel");
     return AKV_OK;
   }
-  const int grid = hyb_grid((PAGED && a.x2) ? 2 * a.n : a.n);
+  const int grid = hyb_grid(n_total);
   switch (dt) {
     case AKV_F16: hyb_encode_kernel<AKV_F16, PAGED><<<grid, 256, 0, stream>>>(a); break;
     case AKV_BF16: hyb_encode_kernel<AKV_BF16, PAGED><<<grid, 256, 0, stream>>>(a); break;
@@ -670,8 +645,7 @@ extern "C" int akv_hybrid_encode_paged(const void* x, int x_dtype, int64_t num_t
   return hyb_launch_encode<true>(x_dtype, a, (hipStream_t)stream);
 }
 
-// K and V of a step in one launch while the call is small (a wavefront per vector); two launches of the form
-// for large calls otherwise.  Both tensors and both caches have the strides given.
+// K and V of a step in one launch.  Both tensors and both caches have the strides given.
 extern "C" int akv_hybrid_encode_paged_kv(const void* x_k, const void* x_v, int x_dtype, int64_t num_tokens,
                                           int num_kv_heads, int64_t xs_token, int64_t xs_head,
                                           const void* slot_mapping, int slot_itype,
@@ -681,13 +655,6 @@ extern "C" int akv_hybrid_encode_paged_kv(const void* x_k, const void* x_v, int 
   AKV_REQUIRE(num_tokens >= 0 && num_kv_heads > 0, "akv_hybrid_encode_paged_kv: bad sizes");
   if (num_tokens == 0 || max_blocks == 0) return AKV_OK;
   AKV_REQUIRE(x_k && x_v && out_k && out_v, "akv_hybrid_encode_paged_kv: null pointer");
-  if (num_tokens * num_kv_heads >= 16384) {
-    const int rc = akv_hybrid_encode_paged(x_k, x_dtype, num_tokens, num_kv_heads, xs_token, xs_head, slot_mapping,
-                                           slot_itype, hyb_table, out_k, ps_blk, ps_pos, ps_head, block_size, max_blocks, stream);
-    if (rc) return rc;
-    return akv_hybrid_encode_paged(x_v, x_dtype, num_tokens, num_kv_heads, xs_token, xs_head, slot_mapping,
-                                   slot_itype, hyb_table, out_v, ps_blk, ps_pos, ps_head, block_size, max_blocks, stream);
-  }
   AKV_REQUIRE(akv_valid_dtype(x_dtype) && akv_valid_itype(slot_itype), "akv_hybrid_encode_paged_kv: bad dtype");
   AKV_REQUIRE(block_size > 0 && max_blocks >= 0, "akv_hybrid_encode_paged_kv: bad block_size/max_blocks");
   AKV_REQUIRE(slot_mapping && hyb_table, "akv_hybrid_encode_paged_kv: null pointer");
@@ -705,10 +672,9 @@ extern "C" int akv_hybrid_decode(const uint8_t* packed, int64_t packed_stride_by
   if (n == 0) return AKV_OK;
   AKV_REQUIRE(packed && hyb_table && out, "akv_hybrid_decode: null pointer");
   AKV_REQUIRE(packed_stride_bytes >= 64 && out_stride >= 128, "akv_hybrid_decode: stride smaller than row");
-  // (a lane per vector from 64 K vectors on; below that a wavefront per vector ends two to three microseconds earlier)
-  if (!hyb_lane_disabled() && (((uintptr_t)packed | (uintptr_t)packed_stride_bytes | (uintptr_t)out) & 15) == 0 &&
-      (out_stride & 3) == 0 && (n >= 65536 || hyb_lane_forced())) {
-    hyb_decode_lane_kernel<<<(int)((n + 255) / 256), 256, 0, (hipStream_t)stream>>>(packed, packed_stride_bytes, n,
+  // (16 K / 24 K / 32 K vectors: 7.8 / 8.1 / 9.2 us in the lanes' registers, 6.4 / 8.7 / 10.8 with a wavefront per vector)
+  if ((((uintptr_t)packed | (uintptr_t)packed_stride_bytes | (uintptr_t)out) & 15) == 0 && (out_stride & 3) == 0 && hyb_lane_form(n >= 22528)) {
+    hyb_decode_lane_kernel<<<(int)((n + 127) / 128), 256, 0, (hipStream_t)stream>>>(packed, packed_stride_bytes, n,
                                                                                   hyb_table, kHybKappa, out, out_stride);
     AKV_LAUNCH_CHECK("hyb_decode_lane_kernel");
     return AKV_OK;

@@ -130,6 +130,125 @@ __global__ __launch_bounds__(256) void h25_encode_kernel(h25_enc_args a) {
 }
 
 // ----------------------------------------------------------------------------------
+// encode, one LANE per vector (rows of 16-byte aligned input, 4-byte aligned output): as in the tq35 encoder the transforms,
+// sums and bit streams stay in the lane's registers, and every operation and the order of the sums are those of the kernel
+// above.  One wavefront takes both groups of its 64 vectors, the small one first: as wavefronts of their own they would be a
+// third and two thirds of the work, and the SIMDs that got the large ones would end last.
+//
+// Divisions.  By the two roots: reciprocal, product, one correction; for these two divisors that is the correctly rounded quotient
+// of every significand (all 2^23 of them tried).  By a norm: two corrections, the first of which leaves less than one
+// unit in the last place, from where the second rounds correctly (Markstein, 1990).  Both for quotients and remainders above 2^-126.
+//
+// What bounds it: the chain of one lane up to one wavefront per SIMD, then vector instructions, some 45 a coordinate.  K and V of
+// 2,048 / 8,192 tokens of 8 heads: 14.2 / 20.2 us, with a wavefront per vector 30.1 / 113.
+// ----------------------------------------------------------------------------------
+__device__ __forceinline__ float h25_by_root(float x, float root, float rcp) {
+  const float q = akv_mul_rn(x, rcp);
+  return fmaf(fmaf(q, root, -x), -rcp, q);                 // (in this form a zero keeps its sign)
+}
+// x[0 .. N) /= norm + 1e-10
+template <int N>
+__device__ __forceinline__ void h25_normalise(float* u, float nrm) {
+  const float den = akv_add_rn(nrm, 1e-10f), rcp = __frcp_rn(den);
+  const float neg_den = den < INFINITY ? -den : 0.f;       // (an infinite or NaN norm: x * (1 / den) already is the quotient)
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    float q = akv_mul_rn(u[j], rcp);
+    q = fmaf(fmaf(q, neg_den, u[j]), rcp, q);              // (the divisor is negated, not the quotient: a NaN keeps its sign)
+    u[j] = fmaf(fmaf(q, neg_den, u[j]), rcp, q);
+  }
+}
+// a group of N coordinates (32, or 96 as blocks of 64 and 32) from coordinate `at` on
+template <int XDT, int N, int MB>
+__device__ __forceinline__ void h25_encode_group_lane(const void* x, int64_t off, hyb_uniform had, hyb_uniform qjl, const float* cen,
+                                                      hyb_uniform bnd_, uint32_t* words) {
+  constexpr int CW = N * MB / 32;
+  constexpr float root = N == 32 ? kH25Root0 : kH25Root1, rcp_root = 1.f / root;
+  float u[N], v[N], bnd[(1 << MB) - 1];
+  hyb_load_row<XDT, N>(x, off, u);
+#pragma unroll
+  for (int k = 0; k < (1 << MB) - 1; ++k) bnd[k] = bnd_[k];
+  auto norm = [&]() {
+    if constexpr (N == 32) return sqrtf(hyb_tree_sum<32>(v));
+    else return sqrtf(akv_add_rn(hyb_tree_sum<64>(v), hyb_tree_sum<32>(v + 64)));
+  };
+  auto transform = [&]() {
+    hyb_fwht_regs<N == 32 ? 32 : 64>(v);
+    if constexpr (N == 96) hyb_fwht_regs<32>(v + 64);
+  };
+#pragma unroll
+  for (int j = 0; j < N; ++j) v[j] = hyb_rounded(akv_mul_rn(u[j], u[j]));
+  const float nrm = norm();
+  h25_normalise<N>(u, nrm);
+#pragma unroll
+  for (int j = 0; j < N; ++j) v[j] = akv_mul_rn(u[j], had[j]);
+  transform();
+#pragma unroll
+  for (int k = 0; k < CW; ++k) {
+    uint32_t w = 0u;
+#pragma unroll
+    for (int i = 0; i < 32 / MB; ++i) {
+      float& r = v[32 / MB * k + i];
+      hyb_append_code<MB>(w, h25_by_root(r, root, rcp_root), bnd);
+      r = cen[w & ((1u << MB) - 1u)];
+    }
+    words[k] = __builtin_bswap32(w);
+  }
+  transform();
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    u[j] = akv_sub_rn(u[j], h25_by_root(akv_mul_rn(v[j], had[j]), root, rcp_root));      // residual
+    v[j] = hyb_rounded(akv_mul_rn(u[j], u[j]));
+  }
+  const float rn = norm();
+#pragma unroll
+  for (int j = 0; j < N; ++j) v[j] = akv_mul_rn(u[j], qjl[j]);
+  transform();
+#pragma unroll
+  for (int k = 0; k < N / 32; ++k) {
+    uint32_t w = 0u;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) hyb_append_sign(w, akv_mul_rn(v[32 * k + i], rcp_root));      // (the quotient has this sign)
+    words[CW + k] = __builtin_bswap32(w);
+  }
+  words[CW + N / 32] = (uint32_t)__half_as_ushort(__float2half_rn(nrm)) | ((uint32_t)__half_as_ushort(__float2half_rn(rn)) << 16);
+}
+
+template <int XDT, bool PAGED>
+__global__ __launch_bounds__(256) void h25_encode_lane_kernel(h25_enc_args a) {
+  __shared__ float cen[6];               // 4 centroids of group 0, 2 of group 1
+  if (threadIdx.x < 6) cen[threadIdx.x] = a.table[H25_CEN0 + threadIdx.x];
+  static_assert(H25_CEN1 == H25_CEN0 + 4, "the two codebooks lie together");
+  __syncthreads();
+  int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n;
+  if (n >= n_total) return;
+  const bool second = PAGED && n >= a.n;
+  if (second) n -= a.n;
+  const void* x = second ? a.x2 : a.x;
+  uint8_t* dst = second ? a.out2 : a.out;
+  int64_t off;
+  if (PAGED) {
+    const int64_t tok = n / a.heads, head = n - tok * a.heads;
+    off = tok * a.xs0 + head * a.xs1;
+    const int64_t slot = akv_load_index(a.slots, a.slot_itype, tok);
+    if (slot < 0) return;
+    const int64_t blk = slot / a.block_size, pos = slot - blk * a.block_size;
+    if (blk >= a.max_blocks) return;
+    dst += blk * a.ps0 + pos * a.ps1 + head * a.ps2;
+  } else {
+    off = n * a.xs0;
+    dst += n * a.ps0;
+  }
+  hyb_uniform tab = (hyb_uniform)a.table;
+  uint32_t row[H25_ROW / 4];
+  h25_encode_group_lane<XDT, 32, 2>(x, off, tab + H25_HAD, tab + H25_QJL, cen, tab + H25_BND0, row);
+  h25_encode_group_lane<XDT, 96, 1>(x, off + 32, tab + H25_HAD + 32, tab + H25_QJL + 32, cen + 4, tab + H25_BND1, row + 4);
+#pragma unroll
+  for (int i = 0; i < H25_ROW / 4; ++i) ((uint32_t*)dst)[i] = row[i];
+}
+
+// ----------------------------------------------------------------------------------
 // decode: one wavefront per vector
 // ----------------------------------------------------------------------------------
 // code, centroid and sign of the lane's two coordinates from a row in LDS or registers (byte accessor)
@@ -177,6 +296,62 @@ __global__ __launch_bounds__(256) void h25_decode_kernel(const uint8_t* __restri
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
+// decode in the lanes' registers (rows of 4-byte aligned input, 16-byte aligned output): the same operations as above; even
+// wavefronts take the block of 64 coordinates of 64 vectors, odd ones the two blocks of 32.  The values go out through LDS, eight
+// lanes a row.  What bounds it: memory, and a chain of 8 us
+// whatever the size.  64 K vectors 11.7 us, four sequences of 2,000 to 8,000 tokens of 8 heads 24.8 (a wavefront per vector: 21.7, 39.5).
+template <int GROUP, int N>       // N coordinates that are transformed together
+__device__ __forceinline__ void h25_decode_block_lane(const uint32_t* codes, const uint32_t* signs, uint32_t norms, hyb_uniform had, hyb_uniform qjl,
+                                                      const float* cen, float* v) {
+  constexpr int MB = GROUP == 0 ? 2 : 1;
+  constexpr float root = GROUP == 0 ? kH25Root0 : kH25Root1, rcp_root = 1.f / root, kappa = GROUP == 0 ? kH25Kappa0 : kH25Kappa1;
+  float w[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const uint32_t c = __builtin_bswap32(codes[j * MB >> 5]), s = ~__builtin_bswap32(signs[j >> 5]);
+    v[j] = cen[(c >> (32 - MB - (j * MB & 31))) & ((1u << MB) - 1u)];
+    w[j] = __uint_as_float(__float_as_uint(kappa) | ((s << (j & 31)) & 0x80000000u));
+  }
+  hyb_fwht_regs<N>(v);
+  hyb_fwht_regs<N>(w);
+  const float n = h25_half_bits_to_float(norms), rn = h25_half_bits_to_float(norms >> 16);
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float mse = h25_by_root(akv_mul_rn(v[j], had[j]), root, rcp_root);
+    const float sk = h25_by_root(akv_mul_rn(w[j], qjl[j]), root, rcp_root);
+    v[j] = akv_mul_rn(akv_add_rn(mse, hyb_rounded(akv_mul_rn(sk, rn))), n);
+  }
+}
+
+__global__ __launch_bounds__(256) void h25_decode_lane_kernel(const uint8_t* __restrict__ packed, int64_t ps, int64_t n_vec,
+                                                              const float* __restrict__ table, float* __restrict__ out, int64_t os) {
+  __shared__ float cen[6];               // 4 centroids of group 0, 2 of group 1
+  __shared__ __align__(16) float turn[4][HYB_TURN_FLOATS];
+  if (threadIdx.x < 6) cen[threadIdx.x] = table[H25_CEN0 + threadIdx.x];
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t n0 = (int64_t)blockIdx.x * 128 + (wave >> 1) * 64;
+  if (n0 >= n_vec) return;
+  const int64_t n = n0 + lane < n_vec ? n0 + lane : n_vec - 1;       // past the end: read, not stored
+  const uint32_t* p = (const uint32_t*)(packed + n * ps);
+  hyb_uniform tab = (hyb_uniform)table;
+  float* o = out + n0 * os;
+  const int rows = (int)(n_vec - n0 < 64 ? n_vec - n0 : 64);
+  float v[64];
+  if ((wave & 1) == 0) {
+    const uint32_t codes[2] = {p[4], p[5]}, signs[2] = {p[7], p[8]};
+    h25_decode_block_lane<1, 64>(codes, signs, p[10], tab + H25_HAD + 32, tab + H25_QJL + 32, cen + 4, v);
+    hyb_store_turned(v, turn[wave], o + 32, os, rows, lane);
+    hyb_store_turned(v + 32, turn[wave], o + 64, os, rows, lane);
+  } else {
+    const uint32_t codes[3] = {p[0], p[1], p[6]}, signs[2] = {p[2], p[9]}, norms[2] = {p[3], p[10]};
+    h25_decode_block_lane<0, 32>(codes, signs, norms[0], tab + H25_HAD, tab + H25_QJL, cen, v);
+    h25_decode_block_lane<1, 32>(codes + 2, signs + 1, norms[1], tab + H25_HAD + 96, tab + H25_QJL + 96, cen + 4, v + 32);
+    hyb_store_turned(v, turn[wave], o, os, rows, lane);
+    hyb_store_turned(v + 32, turn[wave], o + 96, os, rows, lane);
   }
 }
 
@@ -505,9 +680,27 @@ static int h25_grid(int64_t n) {
   return (int)(g < 1 ? 1 : (g > cap ? cap : g));
 }
 
+// Decode in the lanes' registers from here on: 8.1 / 8.6 / 9.5 us for 16 K / 24 K / 32 K vectors, a wavefront per vector
+// 7.0 / 9.6 / 12.2.
+#define H25_DECODE_LANE_MIN 22528
+// Encode likewise from here on: 14.1 us up to 32 K vectors; a wavefront per vector takes 4.6 us for 2,048 vectors, 9.0 for 8,192
+// and 15.8 for 16,384 (8 heads, bfloat16, K and V together).
+#define H25_LANE_MIN 14336
 template <bool PAGED>
 static int h25_launch_encode(int dt, const h25_enc_args& a, hipStream_t stream) {
-  const int grid = h25_grid((PAGED && a.x2) ? 2 * a.n : a.n);
+  const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n;
+  if (hyb_lane_aligned(a.x, a.x2, a.xs0, PAGED ? a.xs1 : 0, dt, a.out, a.out2, a.ps0 | (PAGED ? a.ps1 | a.ps2 : 0), 4) &&
+      hyb_lane_form(n_total >= H25_LANE_MIN)) {
+    const int lgrid = (int)((n_total + 255) / 256);
+    switch (dt) {
+      case AKV_F16: h25_encode_lane_kernel<AKV_F16, PAGED><<<lgrid, 256, 0, stream>>>(a); break;
+      case AKV_BF16: h25_encode_lane_kernel<AKV_BF16, PAGED><<<lgrid, 256, 0, stream>>>(a); break;
+      default: h25_encode_lane_kernel<AKV_F32, PAGED><<<lgrid, 256, 0, stream>>>(a); break;
+    }
+    AKV_LAUNCH_CHECK("h25_encode_lane_kernel");
+    return AKV_OK;
+  }
+  const int grid = h25_grid(n_total);
   switch (dt) {
     case AKV_F16: h25_encode_kernel<AKV_F16, PAGED><<<grid, 256, 0, stream>>>(a); break;
     case AKV_BF16: h25_encode_kernel<AKV_BF16, PAGED><<<grid, 256, 0, stream>>>(a); break;
@@ -573,6 +766,12 @@ extern "C" int akv_hybrid25_decode(const uint8_t* packed, int64_t packed_stride_
   if (n == 0) return AKV_OK;
   AKV_REQUIRE(packed && hyb_table && out, "akv_hybrid25_decode: null pointer");
   AKV_REQUIRE(packed_stride_bytes >= H25_ROW && out_stride >= 128, "akv_hybrid25_decode: stride smaller than row");
+  if ((((uintptr_t)packed | (uintptr_t)packed_stride_bytes) & 3) == 0 && ((uintptr_t)out & 15) == 0 && (out_stride & 3) == 0 &&
+      hyb_lane_form(n >= H25_DECODE_LANE_MIN)) {
+    h25_decode_lane_kernel<<<(int)((n + 127) / 128), 256, 0, (hipStream_t)stream>>>(packed, packed_stride_bytes, n, hyb_table, out, out_stride);
+    AKV_LAUNCH_CHECK("h25_decode_lane_kernel");
+    return AKV_OK;
+  }
   h25_decode_kernel<<<h25_grid(n), 256, 0, (hipStream_t)stream>>>(packed, packed_stride_bytes, n, hyb_table, out, out_stride);
   AKV_LAUNCH_CHECK("h25_decode_kernel");
   return AKV_OK;

@@ -36,6 +36,121 @@ __device__ __forceinline__ float hyb_fwht64(float v, int lane) {
   return v;
 }
 
+// ---- a lane per vector or group: transforms, sums and bit streams in the lane's registers.
+// (The reference rounds every operation: the products come from akv_mul_rn, which the compiler may not fuse into a
+// multiply-add.  Where a product that is not exact feeds a tree of sums it also passes through hyb_rounded(), an empty asm
+// statement the optimiser cannot see through, so the tree is not reassociated around it either.)
+typedef const __attribute__((address_space(4))) float* hyb_uniform;       // a table read at the same place by all lanes: scalar loads
+__device__ __forceinline__ float hyb_rounded(float x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+// N-point Walsh-Hadamard transform of v[0 .. N)
+template <int N>
+__device__ __forceinline__ void hyb_fwht_regs(float* v) {
+#pragma unroll
+  for (int h = 1; h < N; h <<= 1)
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if ((i & h) == 0) {
+        const float lo = v[i], hi = v[i + h];
+        v[i] = akv_add_rn(lo, hi);
+        v[i + h] = akv_sub_rn(lo, hi);
+      }
+}
+// sum in the order of the reduction over lanes (partners N/2, ..., 1 apart); t is used up
+template <int N>
+__device__ __forceinline__ float hyb_tree_sum(float* t) {
+#pragma unroll
+  for (int m = N / 2; m >= 1; m >>= 1)
+#pragma unroll
+    for (int i = 0; i < m; ++i) t[i] = akv_add_rn(t[i], t[i + m]);
+  return t[0];
+}
+// N coordinates of a row (16-byte aligned) as floats
+template <int XDT, int N>
+__device__ __forceinline__ void hyb_load_row(const void* x, int64_t off, float* u) {
+  if constexpr (XDT == AKV_F32) {
+    const float4* p = (const float4*)((const float*)x + off);
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) { const float4 q = p[i]; u[4 * i] = q.x; u[4 * i + 1] = q.y; u[4 * i + 2] = q.z; u[4 * i + 3] = q.w; }
+  } else {
+    const uint4* p = (const uint4*)((const unsigned short*)x + off);
+#pragma unroll
+    for (int i = 0; i < N / 8; ++i) {
+      const uint4 q = p[i];
+      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (XDT == AKV_F16) {
+          u[8 * i + 2 * j] = __half2float(__ushort_as_half((unsigned short)(w[j] & 0xffffu)));
+          u[8 * i + 2 * j + 1] = __half2float(__ushort_as_half((unsigned short)(w[j] >> 16)));
+        } else {
+          u[8 * i + 2 * j] = __uint_as_float(w[j] << 16);
+          u[8 * i + 2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+        }
+      }
+    }
+  }
+}
+// w = 2 w + bit per level: the code of y (how many boundaries lie below it; a NaN lies past all of them) by halving, its bits
+// shifted into a stream as the carry of an addition -- 10 (3 bits) and 5 (2 bits) instructions with the append, where counting
+// takes two a boundary.
+template <int MB>
+__device__ __forceinline__ void hyb_append_code(uint32_t& w, float y, const float (&b)[(1 << MB) - 1]) {
+  if constexpr (MB == 3) {
+    float t0, t1, t2;
+    asm("v_cmp_nle_f32 vcc, %4, %8\n\t"
+        "v_cndmask_b32 %2, %6, %10, vcc\n\t"
+        "v_cndmask_b32 %1, %5, %9, vcc\n\t"
+        "v_cndmask_b32 %3, %7, %11, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %4, %2\n\t"
+        "v_cndmask_b32 %1, %1, %3, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %4, %1\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
+        : "+v"(w), "=&v"(t0), "=&v"(t1), "=&v"(t2)
+        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6])
+        : "vcc");
+  } else if constexpr (MB == 2) {
+    float t;
+    asm("v_cmp_nle_f32 vcc, %2, %4\n\t"
+        "v_cndmask_b32 %1, %3, %5, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %2, %1\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
+        : "+v"(w), "=&v"(t)
+        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2])
+        : "vcc");
+  } else {
+    asm("v_cmp_nle_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(y), "v"(b[0]) : "vcc");
+  }
+}
+// w = 2 w + (y >= 0)
+__device__ __forceinline__ void hyb_append_sign(uint32_t& w, float y) {
+  asm("v_cmp_le_f32 vcc, 0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(y) : "vcc");
+}
+
+// 32 values of every lane's row to memory: through LDS (64 rows of 36 floats, a wavefront's own), so that eight lanes write 128
+// bytes of a row at a time.  out: the first row's 32 values, 16-byte aligned; rows from `rows` on are not stored.
+#define HYB_TURN_FLOATS (64 * 36)
+__device__ __forceinline__ void hyb_store_turned(const float* v, float* turn, float* out, int64_t os, int rows, int lane) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < 8; ++i) *(float4*)&turn[36 * lane + 4 * i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 8 * i + (lane >> 3), c = 4 * (lane & 7);
+    const float4 q = *(const float4*)&turn[36 * r + c];
+    if (r < rows) *(float4*)(out + (int64_t)r * os + c) = q;
+  }
+}
+
 // ---- tq25 (the row: akv_hybrid25.hip): tables, transforms
 #define H25_HAD 0          // [128] Hadamard signs in coordinate order (group 0's 32, then group 1's 96)
 #define H25_QJL 128        // [128] QJL signs likewise
@@ -67,6 +182,20 @@ struct h25_roles {
   __device__ __forceinline__ explicit h25_roles(int lane)
       : ca(32 + lane), cb(lane < 32 ? lane : 64 + lane), b0(lane < 32), ja(lane), jb(lane < 32 ? lane : 32 + lane) {}
 };
+
+// the lane forms of the codecs: rows they can read and write wide, and calls that are large enough (`large`) unless an
+// environment variable asks for one of the forms
+static inline bool hyb_lane_aligned(const void* x, const void* x2, int64_t xs0, int64_t xs1, int dt, const void* out, const void* out2,
+                                    int64_t out_strides, int out_align) {
+  const int64_t xal = dt == AKV_F32 ? 3 : 7;      // elements per 16 bytes, minus one
+  return (((uintptr_t)x | (uintptr_t)x2) & 15) == 0 && ((xs0 | xs1) & xal) == 0 &&
+         (((uintptr_t)out | (uintptr_t)out2 | (uintptr_t)out_strides) & (uintptr_t)(out_align - 1)) == 0;
+}
+static inline bool hyb_lane_form(bool large) {
+  static const bool never = [] { const char* e = getenv("AKV_HYBRID_WAVE_ENCODE"); return e && e[0] == '1'; }();
+  const char* e = getenv("AKV_HYBRID_LANE_ENCODE");        // (read per call: tests switch it)
+  return !never && (large || (e && e[0] == '1'));
+}
 
 // matrix-core attention on hybrid rows (akv_attn_hyb.hip)
 struct akv_attn_ws;

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import aitherkvcache_amd as akv
+from aitherkvcache_amd.hybrid_attention import hybrid_encode_and_store_pair
 from oracle import tq_oracle as O
 from tests.util import kv_like, MAX_ULPS
 
@@ -250,3 +251,40 @@ def test_key_and_value_of_a_step_in_one_call(golden, tq25, dev, mode, row):
     sl = torch.arange(37, device=dev)
     akv.hybrid_encode_and_store_pair(h, k37, wide[..., :128], sl, a, b, BS)
     assert torch.equal(a.reshape(-1, KVH, row)[:37], h.encode(k37)) and torch.equal(b.reshape(-1, KVH, row)[:37], h.encode(v37))
+
+
+@pytest.mark.parametrize("mode", ["tq35", "tq25"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 300])
+def test_lane_forms_of_the_codec_at_the_edges_of_a_workgroup(dev, monkeypatch, mode, dtype, n):
+    """A lane per vector or group against a wavefront per vector (which takes the same vectors from rows that are not 16-byte
+    aligned): the same bytes, and nothing is written past the last vector."""
+    h = akv.HybridTurboQuant(head_dim=128, mode=mode, device=str(dev))
+    h.calibrate_uniform(1)
+    gen = torch.Generator(device=dev).manual_seed(n)
+    x = torch.randn(2, n, 1, 128, device=dev, generator=gen)
+    x *= torch.logspace(-6, 3, n, device=dev).reshape(1, n, 1, 1)
+    x[0, n // 2] = 0.0
+    x[1, n // 3, 0, 5], x[1, n // 3, 0, 100] = 3e4, float("inf")      # an infinite norm: the other coordinates become zeros, that one NaN
+    x = x.to(dtype)
+    odd = torch.empty(2, n, 1, 129, dtype=dtype, device=dev)
+    odd[..., 1:] = x
+    slots = torch.arange(n, device=dev)
+    slots[n // 4] = -1
+    caches = []
+    for src in (odd[..., 1:], x):
+        monkeypatch.setenv("AKV_HYBRID_LANE_ENCODE", "1")
+        rows = torch.full((2, n + 2, 1, 1, 64), 0x5A, dtype=torch.uint8, device=dev)
+        hybrid_encode_and_store_pair(h, src[0], src[1], slots, rows[0][..., :h.packed_dim], rows[1][..., :h.packed_dim], 1)
+        caches.append(rows)
+    assert torch.equal(caches[0], caches[1])
+    assert bool((caches[1][:, n:] == 0x5A).all()) and bool((caches[1][:, n // 4] == 0x5A).all())
+    assert bool((caches[1][..., h.packed_dim:] == 0x5A).all())
+    flat = h.encode(x.reshape(-1, 128)).reshape(2, n, -1)
+    keep = torch.arange(n, device=dev) != n // 4
+    assert torch.equal(flat[:, keep], caches[1][:, :n, 0, 0, :h.packed_dim][:, keep])
+    # decode: rows at an odd byte pitch and output as it comes against aligned ones
+    pitched = torch.zeros(2 * n, h.packed_dim + 1, dtype=torch.uint8, device=dev)
+    pitched[:, 1:] = flat.reshape(2 * n, -1)
+    a, b = h.decode(pitched[:, 1:]), h.decode(flat.reshape(2 * n, -1))
+    assert torch.equal(a.view(torch.int32), b.view(torch.int32))
