@@ -322,3 +322,83 @@ __device__ __forceinline__ uint32_t akv_search(float y, const float* bnd) {
   if (y != y) c = (1u << BITS) - 1u;  // searchsorted places NaN after every boundary
   return c;
 }
+// ---- codes by halving
+// The boundaries in the order that halving needs; a NaN lies below no value, like infinity.  (Codebooks are sorted: the branch is
+// not taken.  What is counted does not depend on the order.)
+template <int N>
+__device__ __forceinline__ void akv_sort_boundaries(float (&b)[N]) {
+  bool sorted = b[N - 1] == b[N - 1];
+#pragma unroll
+  for (int k = 0; k + 1 < N; ++k) sorted = sorted && b[k] <= b[k + 1];
+  if (__builtin_expect(!sorted, 0)) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) b[k] = b[k] == b[k] ? b[k] : INFINITY;
+#pragma unroll
+    for (int r = 0; r < N; ++r)
+#pragma unroll
+      for (int k = r & 1; k + 1 < N; k += 2) {
+        const float lo = fminf(b[k], b[k + 1]), hi = fmaxf(b[k], b[k + 1]);
+        b[k] = lo;
+        b[k + 1] = hi;
+      }
+  }
+}
+// w = 2 w + bit per level: the code of y (how many of the sorted boundaries lie below it; a NaN lies past all of them), its bits
+// shifted into a stream as the carry of an addition -- 19 (4 bits), 10 (3) and 5 (2) instructions with the append, where counting
+// takes two a boundary.
+template <int MB>
+__device__ __forceinline__ void akv_append_code(uint32_t& w, float y, const float (&b)[(1 << MB) - 1]) {
+  if constexpr (MB == 4) {
+    float s0, s2, s4, s6, t1, t3, t5;
+    asm("v_cmp_nle_f32 vcc, %8, %16\n\t"
+        "v_cndmask_b32 %6, %12, %20, vcc\n\t"
+        "v_cndmask_b32 %5, %10, %18, vcc\n\t"
+        "v_cndmask_b32 %7, %14, %22, vcc\n\t"
+        "v_cndmask_b32 %1, %9, %17, vcc\n\t"
+        "v_cndmask_b32 %2, %11, %19, vcc\n\t"
+        "v_cndmask_b32 %3, %13, %21, vcc\n\t"
+        "v_cndmask_b32 %4, %15, %23, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %8, %6\n\t"
+        "v_cndmask_b32 %5, %5, %7, vcc\n\t"
+        "v_cndmask_b32 %1, %1, %3, vcc\n\t"
+        "v_cndmask_b32 %2, %2, %4, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %8, %5\n\t"
+        "v_cndmask_b32 %1, %1, %2, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %8, %1\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
+        : "+v"(w), "=&v"(s0), "=&v"(s2), "=&v"(s4), "=&v"(s6), "=&v"(t1), "=&v"(t3), "=&v"(t5)
+        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]), "v"(b[8]), "v"(b[9]), "v"(b[10]), "v"(b[11]),
+          "v"(b[12]), "v"(b[13]), "v"(b[14])
+        : "vcc");
+  } else if constexpr (MB == 3) {
+    float t0, t1, t2;
+    asm("v_cmp_nle_f32 vcc, %4, %8\n\t"
+        "v_cndmask_b32 %2, %6, %10, vcc\n\t"
+        "v_cndmask_b32 %1, %5, %9, vcc\n\t"
+        "v_cndmask_b32 %3, %7, %11, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %4, %2\n\t"
+        "v_cndmask_b32 %1, %1, %3, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %4, %1\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
+        : "+v"(w), "=&v"(t0), "=&v"(t1), "=&v"(t2)
+        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6])
+        : "vcc");
+  } else if constexpr (MB == 2) {
+    float t;
+    asm("v_cmp_nle_f32 vcc, %2, %4\n\t"
+        "v_cndmask_b32 %1, %3, %5, vcc\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
+        "v_cmp_nle_f32 vcc, %2, %1\n\t"
+        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
+        : "+v"(w), "=&v"(t)
+        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2])
+        : "vcc");
+  } else {
+    asm("v_cmp_nle_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(y), "v"(b[0]) : "vcc");
+  }
+}

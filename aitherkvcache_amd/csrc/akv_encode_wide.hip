@@ -1,13 +1,15 @@
 // MFMA encode (norm -> rotate -> codebook search -> pack -> store) at head_dim 64 and 256 for float16, bfloat16 and float32
 // input, flat rows or scattered through a slot mapping (K and V of a step in one launch).
 //
-//   Y[row, j] = sum_i X[row, i] Pi[j, i]              v_mfma_f32_16x16x32_f16
+//   Y[row, j] = sum_i X[row, i] Pi[j, i]              v_mfma_f32_16x16x32_f16, Pi the first operand
 //
-// Wavefront w of a workgroup owns output coordinates 16 w .. 16 w + 15 and keeps its 16 x D slice of Pi in registers,
-// split into two float16 terms from the float32 matrix at its start.  A workgroup takes 16 MT rows at a time: its threads
+// Wavefront w of a workgroup owns NT times 16 output coordinates and keeps these rows of Pi in registers, split into two float16
+// terms from the float32 matrix at its start.  A workgroup takes 16 MT rows at a time: its threads
 // load them (four neighbouring elements each), reduce the squared norms over the lanes of a row and leave the rows in LDS;
-// every wavefront multiplies all of them by its slice and searches the codebook; the codes meet in LDS and are packed by
-// the byte.  Two barriers a step, the next rows requested before the first.
+// every wavefront multiplies all of them by its slice.  A lane then holds four neighbouring coordinates of one row: their
+// codes, found by halving, are one halfword for LDS, and pairs of halfwords are stored.  Two barriers a step, the next rows
+// requested before the first.  PARTS workgroups share the coordinates of a row where there are few rows: each loads and splits
+// only its part of the matrix (and all of the rows).
 //
 // Precision: float16 rows are exact in the operand.  bfloat16 and float32 rows are scaled by the power of two that
 // brings the largest element to [2^10, 2^11): bfloat16 is then exact (down to 2^-27 of the largest element), float32 is
@@ -15,7 +17,9 @@
 // kernel's chain of float32 sums is no closer to 64 bits.
 //
 // What bounds it: a decode step (192 to 768 rows) is one step per workgroup, a chain of trips to memory: matrix and rows,
-// slots, stores.  Large calls are bound by the search, two vector instructions per boundary and value.
+// slots, stores: 11.4 us before the coordinates were shared out, 6.4 now (head_dim 256, up to 1,024 rows).  Large calls are bound
+// by the search, 22 vector instructions a value in 4 bits.  K and V of 8,192 tokens of 8 heads in 4 bits: 80.5 us at
+// head_dim 256 and 16.5 at 64, where counting with two instructions a boundary and a byte per code through LDS took 98.2 and 21.4.
 #include "akv_common.h"
 
 typedef _Float16 ew_half8 __attribute__((ext_vector_type(8)));
@@ -25,9 +29,12 @@ typedef float ew_float4 __attribute__((ext_vector_type(4)));
 #define EW_PI_SCALE 1024.f
 #define EW_PI_EXP 10
 
-template <int D, int MT, int XDT> struct ew_cfg {
-  static constexpr int WAVES = D / 16, THREADS = WAVES * 64, ROWS = 16 * MT;
+template <int D, int MT, int XDT, int PARTS, int NT> struct ew_cfg {
+  static constexpr int DP = D / PARTS;                     // output coordinates of a workgroup
+  static constexpr int WAVES = DP / (16 * NT), THREADS = WAVES * 64, ROWS = 16 * MT;
   static constexpr int TPR = D / 4;                        // threads of a row while loading
+  static constexpr int PIECES = ROWS * TPR / THREADS;      // pieces of four elements a thread loads
+  static constexpr int CPITCH = DP / 4 + 2;                // halfwords of codes per row in LDS
   static constexpr int KS = D / 32;
   static constexpr int PITCH = D + 8;                      // float16 per row in LDS (16 bytes more: eight rows meet all banks)
   static constexpr int NA = XDT == AKV_F32 ? 2 : 1;        // float16 terms of a row
@@ -50,27 +57,28 @@ template <int XDT> __device__ __forceinline__ void ew_floats(const typename ew_p
   }
 }
 
-template <int D, int BITS, int XDT, bool PAGED, int MT>
-__global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kernel(akv_gen_args a, const float* __restrict__ Pi, const akv_prep_scale* __restrict__ scale) {
-  typedef ew_cfg<D, MT, XDT> cfg;
+template <int D, int BITS, int XDT, bool PAGED, int MT, int PARTS, int NT>
+__global__ __launch_bounds__((ew_cfg<D, MT, XDT, PARTS, NT>::THREADS)) void akv_encode_wide_kernel(akv_gen_args a, const float* __restrict__ Pi, const akv_prep_scale* __restrict__ scale) {
+  typedef ew_cfg<D, MT, XDT, PARTS, NT> cfg;
   typedef typename ew_piece<XDT>::type piece_t;
-  constexpr int ROWS = cfg::ROWS, TPR = cfg::TPR, KS = cfg::KS, PITCH = cfg::PITCH, NA = cfg::NA, THREADS = cfg::THREADS;
+  constexpr int ROWS = cfg::ROWS, TPR = cfg::TPR, KS = cfg::KS, PITCH = cfg::PITCH, NA = cfg::NA, THREADS = cfg::THREADS, PIECES = cfg::PIECES, DP = cfg::DP;
   constexpr int NB = (1 << BITS) - 1;
   constexpr int XB = XDT == AKV_F32 ? 4 : 2;
   __shared__ __align__(16) _Float16 rows[NA][ROWS][PITCH];
-  __shared__ __align__(16) uint8_t codes[ROWS][D + 16];
-  __shared__ float4 info[ROWS];                            // reciprocal of the norm, exponent to put back, norm, not finite
+  __shared__ __align__(16) unsigned short codes[ROWS][cfg::CPITCH];
+  __shared__ float4 info[ROWS];                            // reciprocal of the norm (NaN: not finite), exponent to put back, norm
   __shared__ int64_t dst[2][ROWS];                         // [parity of the step] address of the packed row, 0 = skip
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, g = lane >> 4;
   const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n;
-  const int64_t steps = (n_total + ROWS - 1) / ROWS;
+  const int64_t steps = (n_total + ROWS - 1) / ROWS, first = blockIdx.x / PARTS, stride = gridDim.x / PARTS;
+  const int part = PARTS > 1 ? (int)(blockIdx.x % PARTS) : 0;
 
   // ---- rows: thread (row, part) of piece i
-  piece_t R[MT];
+  piece_t R[PIECES];
   auto fetch = [&](int64_t step) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
+    for (int i = 0; i < PIECES; ++i) {
       const int u = tid + i * THREADS;
       int64_t n = step * ROWS + u / TPR;
       if (n >= n_total) n = n_total - 1;                   // past the end: loaded, not stored
@@ -86,35 +94,37 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kerne
       R[i] = *(const piece_t*)((const char*)(second ? a.x2 : a.x) + XB * (off + 4 * (u % TPR)));
     }
   };
-  fetch(blockIdx.x);
+  fetch(first);
 
   const float pi_scale = EW_PI_SCALE * scale->down;
   const int pi_exp = scale->k - EW_PI_EXP;
-  // ---- the wavefront's slice of Pi: lane (col, g) holds row 16 wave + col, elements 32 ks + 8 g + e
-  ew_half8 Bh[KS], Bl[KS];
+  // ---- the wavefront's NT slices of Pi: lane (col, g) holds row DP part + 16 (NT wave + nt) + col, elements 32 ks + 8 g + e
+  ew_half8 Bh[NT][KS], Bl[NT][KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const float4* p = (const float4*)(Pi + (size_t)(16 * wave + col) * D + 32 * ks + 8 * g);
+  for (int k = 0; k < NT * KS; ++k) {
+    const int nt = k / KS, ks = k % KS;
+    const float4* p = (const float4*)(Pi + (size_t)(DP * part + 16 * (NT * wave + nt) + col) * D + 32 * ks + 8 * g);
     const float4 p0 = p[0], p1 = p[1];
     const float v[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float s = v[e] * pi_scale;
       const _Float16 h = (_Float16)s;
-      Bh[ks][e] = h;
-      Bl[ks][e] = (_Float16)(s - (float)h);
+      Bh[nt][ks][e] = h;
+      Bl[nt][ks][e] = (_Float16)(s - (float)h);
     }
   }
   float bnd[NB];
 #pragma unroll
   for (int k = 0; k < NB; ++k) bnd[k] = a.table[k];
+  akv_sort_boundaries(bnd);
 
   int par = 0;
-  for (int64_t step = blockIdx.x; step < steps; step += gridDim.x, par ^= 1) {
+  for (int64_t step = first; step < steps; step += stride, par ^= 1) {
     // ---- norm, conversion, rows into LDS
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int u = tid + i * THREADS, row = u / TPR, part = u % TPR;
+    for (int i = 0; i < PIECES; ++i) {
+      const int u = tid + i * THREADS, row = u / TPR, at = u % TPR;
       float x[4];
       ew_floats<XDT>(R[i], x);
       float ss = 0.f, mx = 0.f;
@@ -149,11 +159,11 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kerne
           lo.h[e] = (_Float16)(s - (float)hi.h[e]);
         }
       }
-      *(uint2*)&rows[0][row][4 * part] = hi.u;
-      if constexpr (NA == 2) *(uint2*)&rows[NA - 1][row][4 * part] = lo.u;
-      if (part == 0) {
+      *(uint2*)&rows[0][row][4 * at] = hi.u;
+      if constexpr (NA == 2) *(uint2*)&rows[NA - 1][row][4 * at] = lo.u;
+      if (at == 0) {
         const float nrm = sqrtf(ss);
-        info[row] = make_float4(1.f / (nrm + 1e-10f), __int_as_float(put_back), nrm, bad ? 1.f : 0.f);
+        info[row] = make_float4(bad ? NAN : 1.f / (nrm + 1e-10f), __int_as_float(put_back), nrm, 0.f);
       }
     }
     // ---- thread r resolves row r of the step
@@ -182,47 +192,49 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kerne
       }
       dst[par][tid] = dp;
     }
-    if (step + gridDim.x < steps) fetch(step + gridDim.x);
+    if (step + stride < steps) fetch(step + stride);
     __syncthreads();
-    if (norm_at != nullptr) *norm_at = info[tid].z;
+    if (norm_at != nullptr && part == 0) *norm_at = info[tid].z;
 
-    // ---- rotate and search: lane (col, g) ends up with rows 16 mt + 4 g + i of coordinate 16 wave + col
+    // ---- rotate and search: lane (col, g) ends up with coordinates 16 (NT wave + nt) + 4 g + i of row 16 mt + col
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      ew_float4 acc = {0.f, 0.f, 0.f, 0.f};
+      ew_float4 acc[NT];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = ew_float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         const ew_half8 x = *(const ew_half8*)&rows[0][16 * mt + col][32 * ks + 8 * g];
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, Bh[ks], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(x, Bl[ks], acc, 0, 0, 0);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bh[nt][ks], x, acc[nt], 0, 0, 0);
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bl[nt][ks], x, acc[nt], 0, 0, 0);
+        }
         if constexpr (NA == 2) {
           const ew_half8 xl = *(const ew_half8*)&rows[NA - 1][16 * mt + col][32 * ks + 8 * g];
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, Bh[ks], acc, 0, 0, 0);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bh[nt][ks], xl, acc[nt], 0, 0, 0);
         }
       }
+      const float2 f = *(const float2*)&info[16 * mt + col];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 f = info[16 * mt + 4 * g + i];
-        const float y = ldexpf(acc[i] * f.x, __float_as_int(f.y));
-        uint32_t c = 0;
+      for (int nt = 0; nt < NT; ++nt) {
+        uint32_t c = 0;                                    // first code in the top bits; NaN lies past every boundary
 #pragma unroll
-        for (int k = 0; k < NB; ++k) c += bnd[k] < y ? 1u : 0u;
-        if (f.w != 0.f || y != y) c = NB;                  // NaN lies past every boundary
-        codes[16 * mt + 4 * g + i][16 * wave + col] = (uint8_t)c;
+        for (int i = 0; i < 4; ++i) akv_append_code<BITS>(c, ldexpf(acc[nt][i] * f.x, __float_as_int(f.y)), bnd);
+        codes[16 * mt + col][4 * (NT * wave + nt) + g] = (unsigned short)c;
       }
     }
     __syncthreads();
 
-    // ---- pack and store: eight codes are BITS bytes
-    for (int u = tid; u < ROWS * (D / 8); u += THREADS) {
-      const int row = u / (D / 8), part = u % (D / 8);
+    // ---- store: eight codes are BITS bytes
+    for (int u = tid; u < ROWS * (DP / 8); u += THREADS) {
+      const int row = u / (DP / 8), at = u % (DP / 8);
       const int64_t dp = dst[par][row];
       if (dp == 0) continue;
-      const uint2 c = *(const uint2*)&codes[row][8 * part];
-      uint8_t* p = (uint8_t*)(uintptr_t)dp + BITS * part;
-      // first code in the top bits
-      auto four = [](uint32_t v) { return ((v & 0xffu) << (3 * BITS)) | (((v >> 8) & 0xffu) << (2 * BITS)) | (((v >> 16) & 0xffu) << BITS) | (v >> 24); };
-      const uint32_t w = (four(c.x) << (4 * BITS)) | four(c.y);
+      const uint32_t c = *(const uint32_t*)&codes[row][2 * at];
+      uint8_t* p = (uint8_t*)(uintptr_t)dp + BITS * (DP / 8 * part + at);
+      const uint32_t w = ((c & 0xffffu) << (4 * BITS)) | (c >> 16);
       if constexpr (BITS == 4) {
         *(uint32_t*)p = __builtin_bswap32(w);
       } else if constexpr (BITS == 2) {
@@ -238,22 +250,30 @@ __global__ __launch_bounds__((D == 256 ? 1024 : 256)) void akv_encode_wide_kerne
   }
 }
 
-template <int D, int BITS, int XDT, bool PAGED, int MT>
+template <int D, int BITS, int XDT, bool PAGED, int MT, int PARTS, int NT>
 static int ew_launch(const akv_gen_args& a, const float* Pi, hipStream_t stream) {
   const akv_prep_scale* scale = (const akv_prep_scale*)((const char*)Pi + AKV_PREP_SCALE_OFFSET(D));
-  typedef ew_cfg<D, MT, XDT> cfg;
+  typedef ew_cfg<D, MT, XDT, PARTS, NT> cfg;
   const int cus = akv_cached_cu_count();
   const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n, steps = (n_total + cfg::ROWS - 1) / cfg::ROWS;
-  const int64_t most = (int64_t)(cus > 0 ? cus : 256) * (D == 256 ? 1 : 4);
-  AKV_LAUNCH_TIMED((akv_encode_wide_kernel<D, BITS, XDT, PAGED, MT>), (int)(steps < most ? steps : most), cfg::THREADS, 0, stream, a, Pi, scale);
+  const int64_t most = (int64_t)(cus > 0 ? cus : 256) * (D == 256 && PARTS == 1 ? 1 : 4) / PARTS;
+  AKV_LAUNCH_TIMED((akv_encode_wide_kernel<D, BITS, XDT, PAGED, MT, PARTS, NT>), (int)(steps < most ? steps : most) * PARTS, cfg::THREADS, 0, stream, a, Pi, scale);
   AKV_LAUNCH_CHECK("akv_encode_wide_kernel");
   return AKV_OK;
 }
-// More rows a step once every workgroup has several steps: a barrier is then shared by more products
+// head_dim 256: a quarter of the coordinates per workgroup while all of these fit the chip at once (three a CU): 6.4 us up to
+// 1,024 rows, 8.5 for 2,048 and 10.5 for 3,072, where one workgroup for all coordinates takes 11.2; at 4,096 rows it is
+// 15.1 against 11.4.  More rows a step once every workgroup has several steps: a barrier is then shared by more products.
 template <int D, int BITS, int XDT, bool PAGED>
 static int ew_launch_rows(const akv_gen_args& a, const float* Pi, hipStream_t stream) {
   const int64_t n_total = (PAGED && a.x2) ? 2 * a.n : a.n;
-  return n_total > 16384 ? ew_launch<D, BITS, XDT, PAGED, D == 256 ? 2 : 4>(a, Pi, stream) : ew_launch<D, BITS, XDT, PAGED, 1>(a, Pi, stream);
+  if constexpr (D == 256) {
+    const int cus = akv_cached_cu_count();
+    if (n_total <= 12 * (cus > 0 ? cus : 256)) return ew_launch<D, BITS, XDT, PAGED, 1, 4, 1>(a, Pi, stream);
+    return n_total > 16384 ? ew_launch<D, BITS, XDT, PAGED, 2, 1, 2>(a, Pi, stream) : ew_launch<D, BITS, XDT, PAGED, 1, 1, 2>(a, Pi, stream);
+  } else {
+    return n_total > 16384 ? ew_launch<D, BITS, XDT, PAGED, 4, 1, 1>(a, Pi, stream) : ew_launch<D, BITS, XDT, PAGED, 1, 1, 1>(a, Pi, stream);
+  }
 }
 template <int D, int BITS>
 static int ew_launch_dt(int x_dtype, bool paged, const akv_gen_args& a, const float* Pi, hipStream_t stream) {

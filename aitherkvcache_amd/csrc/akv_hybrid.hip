@@ -126,6 +126,7 @@ __device__ __forceinline__ void hyb_encode_group_lane(const void* x, int64_t off
   hyb_load_row<XDT, 64>(x, off, u);
 #pragma unroll
   for (int k = 0; k < (1 << MB) - 1; ++k) bnd[k] = bnd_[k];
+  akv_sort_boundaries(bnd);
 #pragma unroll
   for (int j = 0; j < 64; ++j) v[j] = hyb_rounded(akv_mul_rn(u[j], u[j]));
   const float nrm = sqrtf(hyb_tree_sum<64>(v));
@@ -153,7 +154,7 @@ __device__ __forceinline__ void hyb_encode_group_lane(const void* x, int64_t off
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           float& r = v[32 * h + 8 * g + i];
-          hyb_append_code<3>(g24[g], akv_mul_rn(r, 0.125f), bnd);
+          akv_append_code<3>(g24[g], akv_mul_rn(r, 0.125f), bnd);
           r = cen[g24[g] & 7u];
         }
       }
@@ -167,7 +168,7 @@ __device__ __forceinline__ void hyb_encode_group_lane(const void* x, int64_t off
       uint32_t w = 0u;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        hyb_append_code<2>(w, akv_mul_rn(v[16 * k + i], 0.125f), bnd);
+        akv_append_code<2>(w, akv_mul_rn(v[16 * k + i], 0.125f), bnd);
         v[16 * k + i] = cen[w & 3u];
       }
       words[k] = __builtin_bswap32(w);

@@ -168,6 +168,7 @@ __device__ __forceinline__ void h25_encode_group_lane(const void* x, int64_t off
   hyb_load_row<XDT, N>(x, off, u);
 #pragma unroll
   for (int k = 0; k < (1 << MB) - 1; ++k) bnd[k] = bnd_[k];
+  akv_sort_boundaries(bnd);
   auto norm = [&]() {
     if constexpr (N == 32) return sqrtf(hyb_tree_sum<32>(v));
     else return sqrtf(akv_add_rn(hyb_tree_sum<64>(v), hyb_tree_sum<32>(v + 64)));
@@ -189,7 +190,7 @@ __device__ __forceinline__ void h25_encode_group_lane(const void* x, int64_t off
 #pragma unroll
     for (int i = 0; i < 32 / MB; ++i) {
       float& r = v[32 / MB * k + i];
-      hyb_append_code<MB>(w, h25_by_root(r, root, rcp_root), bnd);
+      akv_append_code<MB>(w, h25_by_root(r, root, rcp_root), bnd);
       r = cen[w & ((1u << MB) - 1u)];
     }
     words[k] = __builtin_bswap32(w);

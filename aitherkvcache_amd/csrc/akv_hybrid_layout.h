@@ -93,40 +93,6 @@ __device__ __forceinline__ void hyb_load_row(const void* x, int64_t off, float* 
     }
   }
 }
-// w = 2 w + bit per level: the code of y (how many boundaries lie below it; a NaN lies past all of them) by halving, its bits
-// shifted into a stream as the carry of an addition -- 10 (3 bits) and 5 (2 bits) instructions with the append, where counting
-// takes two a boundary.
-template <int MB>
-__device__ __forceinline__ void hyb_append_code(uint32_t& w, float y, const float (&b)[(1 << MB) - 1]) {
-  if constexpr (MB == 3) {
-    float t0, t1, t2;
-    asm("v_cmp_nle_f32 vcc, %4, %8\n\t"
-        "v_cndmask_b32 %2, %6, %10, vcc\n\t"
-        "v_cndmask_b32 %1, %5, %9, vcc\n\t"
-        "v_cndmask_b32 %3, %7, %11, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %4, %2\n\t"
-        "v_cndmask_b32 %1, %1, %3, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %4, %1\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
-        : "+v"(w), "=&v"(t0), "=&v"(t1), "=&v"(t2)
-        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6])
-        : "vcc");
-  } else if constexpr (MB == 2) {
-    float t;
-    asm("v_cmp_nle_f32 vcc, %2, %4\n\t"
-        "v_cndmask_b32 %1, %3, %5, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %2, %1\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
-        : "+v"(w), "=&v"(t)
-        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2])
-        : "vcc");
-  } else {
-    asm("v_cmp_nle_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(y), "v"(b[0]) : "vcc");
-  }
-}
 // w = 2 w + (y >= 0)
 __device__ __forceinline__ void hyb_append_sign(uint32_t& w, float y) {
   asm("v_cmp_le_f32 vcc, 0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(y) : "vcc");

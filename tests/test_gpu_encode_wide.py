@@ -118,3 +118,32 @@ def test_matrices_that_are_no_rotation(dev, d, bits, dtype, factor):
     got = O._UNPACK[bits](packed.cpu().numpy().reshape(-1, tq._packed_dim)[:1000], d)
     assert np.count_nonzero(got != ref) <= max(3, ref.size * 2e-5)      # (values that lie on a boundary to within float32)
     assert np.allclose(norms.cpu().numpy().reshape(-1)[:1000], np.linalg.norm(x64, axis=-1), rtol=1e-6)
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_shared_coordinates_and_boundaries_in_any_order(dev, bits, dtype):
+    """head_dim 256: calls of few rows share a row's coordinates out over workgroups, others do not -- the same bytes and norms.
+    The boundaries are counted, whatever their order; one that is NaN counts for no value."""
+    tq = akv.TurboQuant(head_dim=256, bits=bits, device=str(dev))
+    gen = torch.Generator(device=dev).manual_seed(bits)
+    x = torch.randn(5000, 256, device=dev, generator=gen)
+    x[7], x[8, 100], x[9, 3] = 0.0, float("nan"), float("inf")
+    x = x.to(dtype)
+    p, n = tq.encode(x)
+    for rows in (1, 15, 16, 17, 1025, 3071, 3072, 3073):
+        ps, ns = tq.encode(x[:rows])
+        assert torch.equal(ps, p[:rows]) and torch.equal(ns.view(torch.int32), n[:rows].view(torch.int32)), rows
+    slots = torch.arange(3000, device=dev)
+
+    def paged(boundaries, m):
+        packed, norms = torch.zeros(3000, 1, 1, tq._packed_dim, dtype=torch.uint8, device=dev), torch.zeros(3000, 1, 1, device=dev)
+        akv.fused_kv_update(x[:m, None], slots[:m], packed, norms, tq.rotation, boundaries, bits, block_size=1)
+        return packed[:m, 0, 0]
+    b = tq.boundaries_inner
+    for m in (20, 3000):
+        assert torch.equal(paged(b.flip(0).contiguous(), m), p[:m])
+        hole, top = b.clone(), b.clone()
+        hole[b.numel() // 2], top[b.numel() // 2] = float("nan"), float("inf")
+        finite = torch.isfinite(x[:m].float()).all(-1)              # (a NaN value lies past every boundary, infinite or not)
+        assert torch.equal(paged(hole, m)[finite], paged(top.sort().values, m)[finite])
