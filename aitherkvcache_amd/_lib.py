@@ -99,6 +99,7 @@ SIGNATURES = {
     "akv_block_select": (_i, [_p, _p, _i, _i64, _p, _i, _i, _i64, _i, _i, _i, _i, _p, _p, _p]),
     "akv_tri_encode": (_i, [_p, _i, _i64, _i, _i64, _i, _i, _p, _p, _p, _p]),
     "akv_tri_encode_paged": (_i, [_p, _i, _i64, _i, _i, _i64, _i64, _i, _p, _i, _i64, _p, _p, _p, _p]),
+    "akv_tri_encode_paged_kv": (_i, [_p, _p, _i, _i64, _i, _i, _i64, _i64, _i, _p, _i, _i64, _p, _p, _p, _p, _p, _p, _p]),
     "akv_tri_decode_workspace_bytes": (_sz, [_i, _i, _i]),
     "akv_tri_scores": (_i, [_p, _i, _p, _p, _p, _p, _p, _i, _p, _i, _p, _i, _i64, _i, _i, _i, _i, _i, _i, _p]),
     "akv_tri_decode_step": (_i, [_p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i,
@@ -111,7 +112,7 @@ _lib: Optional[C.CDLL] = None
 _calls = None          # the binding of the hot calls (csrc/akv_binding.cpp), once the library is loaded
 _BOUND = ("akv_paged_attn_workspace_bytes", "akv_paged_attn", "akv_encode_paged_kv", "akv_hybrid_paged_attn_workspace_bytes",
           "akv_hybrid_paged_attn", "akv_hybrid25_paged_attn", "akv_hybrid_encode_paged_kv", "akv_hybrid25_encode_paged_kv",
-          "akv_decode_blocks_kv", "akv_tri_encode_paged", "akv_tri_decode_workspace_bytes", "akv_tri_decode_paged")
+          "akv_decode_blocks_kv", "akv_tri_encode_paged_kv", "akv_tri_decode_workspace_bytes", "akv_tri_decode_paged")
 
 
 def available() -> bool:

@@ -26,7 +26,7 @@ struct Library {
   decltype(&akv_hybrid_paged_attn) hybrid_attn[2];                  // tq35, tq25
   decltype(&akv_hybrid_encode_paged_kv) hybrid_encode[2];
   decltype(&akv_decode_blocks_kv) decode_blocks;
-  decltype(&akv_tri_encode_paged) tri_encode;
+  decltype(&akv_tri_encode_paged_kv) tri_encode;
   decltype(&akv_tri_decode_workspace_bytes) tri_bytes;
   decltype(&akv_tri_decode_paged) tri_decode;
 } g_lib;
@@ -287,19 +287,16 @@ PyObject* spectral_encode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const at::Tensor* c[6];
   for (int i = 0; i < 6; ++i) c[i] = &ts.take(a[3 + i]);
   if (!ts.ok() || keys.dim() != 3 || keys.size(0) == 0 || keys.size(1) != v[0] || keys.size(2) != v[1] || values.sizes() != keys.sizes() ||
-      keys.stride(2) != 1 || values.stride(2) != 1 || float_code(keys) < 0 || float_code(values) < 0 || index_code(slots) < 0 || !slots.is_contiguous() ||
+      values.strides() != keys.strides() || keys.stride(2) != 1 || float_code(keys) < 0 || values.scalar_type() != keys.scalar_type() || index_code(slots) < 0 || !slots.is_contiguous() ||
       slots.numel() != keys.size(0))
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
-  int rc = 0;
+  int rc;
   Py_BEGIN_ALLOW_THREADS;
-  for (int i = 0; i < 2 && rc == 0; ++i) {
-    const at::Tensor& x = i ? values : keys;
-    rc = g_lib.tri_encode(x.const_data_ptr(), float_code(x), x.size(0), (int)v[0], (int)v[1], x.stride(0), x.stride(1), (int)v[2], slots.const_data_ptr(),
-                          index_code(slots), v[3], (uint8_t*)c[3 * i]->mutable_data_ptr(), (uint8_t*)c[3 * i + 1]->mutable_data_ptr(),
-                          c[3 * i + 2]->mutable_data_ptr(), stream);
-  }
+  rc = g_lib.tri_encode(keys.const_data_ptr(), values.const_data_ptr(), float_code(keys), keys.size(0), (int)v[0], (int)v[1], keys.stride(0), keys.stride(1),
+                        (int)v[2], slots.const_data_ptr(), index_code(slots), v[3], (uint8_t*)c[0]->mutable_data_ptr(), (uint8_t*)c[1]->mutable_data_ptr(),
+                        c[2]->mutable_data_ptr(), (uint8_t*)c[3]->mutable_data_ptr(), (uint8_t*)c[4]->mutable_data_ptr(), c[5]->mutable_data_ptr(), stream);
   Py_END_ALLOW_THREADS;
   return status(rc);
 }

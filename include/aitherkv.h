@@ -432,6 +432,13 @@ int akv_tri_encode_paged(const void* x, int x_dtype, int64_t num_tokens, int num
                          const void* slot_mapping, int slot_itype, int64_t num_slots,
                          uint8_t* indices, uint8_t* coeffs, void* scales, void* stream);
 
+/* K and V of a step in one launch: x_k and x_v have the dtype, shape and strides given. */
+int akv_tri_encode_paged_kv(const void* x_k, const void* x_v, int x_dtype, int64_t num_tokens, int num_kv_heads, int d,
+                            int64_t xs_token, int64_t xs_head, int num_freqs,
+                            const void* slot_mapping, int slot_itype, int64_t num_slots,
+                            uint8_t* k_indices, uint8_t* k_coeffs, void* k_scales,
+                            uint8_t* v_indices, uint8_t* v_coeffs, void* v_scales, void* stream);
+
 /* ---------------------------------------------------------------------------------
  * Block selection for sparse decode attention -- aither_kvcache/block_selector.py.
  * The attention entry points take the filtered table and context lengths as they are.
