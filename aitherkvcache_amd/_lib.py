@@ -128,6 +128,7 @@ def lib() -> C.CDLL:
             raise RuntimeError(
                 f"{LIB_PATH} not found: the HIP extension is not built and there is no CPU "
                 "fallback. Run `make -C aitherkvcache_amd/csrc`.")
+        from . import _binding  # noqa: F401 -- first: the library's thread-local block is to be the newest of the process
         handle = C.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(handle, name)

@@ -585,3 +585,17 @@ def test_tri_pair_series_and_dct_helpers():
     assert np.max(np.abs(dct(x).numpy() - scipy.fft.dct(x.numpy(), type=2, norm="ortho", axis=-1))) < 1e-13
     assert float((idct(dct(x, Dm), Dm) - x).abs().max()) < 1e-13
 
+
+
+def test_the_binding_has_no_thread_local_storage():
+    """Loaded beside the library it would leave every thread's table of such blocks out of date, 1 us a launch."""
+    import struct
+    from aitherkvcache_amd import _lib
+    path = os.path.join(os.path.dirname(_lib.__file__), "_binding.so")
+    if not os.path.exists(path):
+        pytest.skip("not built")
+    with open(path, "rb") as f:
+        elf = f.read()
+    at, size, count = struct.unpack_from("<Q", elf, 32)[0], *struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, at + i * size)[0] for i in range(count)]
+    assert 1 in kinds and 7 not in kinds          # PT_LOAD, PT_TLS
