@@ -32,7 +32,7 @@
 //
 // What bounds it: the chain of trips to LDS and memory a wavefront walks, at two to four wavefronts a SIMD.  No unit is full
 // (profiles/attn_wave_sq_counters.txt, share of the kernel's cycles): vector unit
-// 49, 43 and 36 % at head_dim 64, 128 and 256, matrix cores 12 to 16, LDS 19 to 24.
+// 44, 41 and 34 % at head_dim 64, 128 and 256, matrix cores 13 to 17, LDS 18 to 24.
 #include <type_traits>
 
 #include "akv_attn_rows.h"

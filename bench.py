@@ -414,6 +414,7 @@ def encode_sweep(torch, akv, L, tq, dev, gen):
 
 
 DECODE_DTYPE = "fp16 hi+lo MFMA operands (keys and queries carry 22 bits, values 11), f32 accumulate and softmax"
+HYBRID_DTYPE = "int8-digit MFMA operands for scores (levels 16 bits, queries 24), fp16 levels and hi+lo weights for values, f32 softmax and sums"
 
 
 def traffic_fields(workload):
@@ -472,7 +473,7 @@ def run_decode(torch, akv, L, dev, workload, tq4, steps, warmup, cpu, cpu_second
     kms = kernel_ms(torch, L, step, max(20, steps))
     res = dict(metric="tq-t4nc paged-decode attn GB/s" if workload == "decode4" else f"{workload} paged-decode attn GB/s",
                value=algo_bytes / ms / 1e6, ms_per_step=ms,
-               dtype="f32 (vector kernels, no matrix cores)" if bits == "tq25" else DECODE_DTYPE,
+               dtype=HYBRID_DTYPE if bits in ("tq25", "tq35") else DECODE_DTYPE,
                config={"workload": name, "context_tokens": tokens, "algorithmic_bytes_per_step": algo_bytes,
                        "cache_copies_alternated": 2, "preconditioning_s": PRECONDITION_S})
     achieved = tokens * per_tok / kms / 1e6
