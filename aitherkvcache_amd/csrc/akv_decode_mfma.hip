@@ -286,7 +286,9 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
     const uint32_t lo = (uint32_t)__half_as_ushort(l0) | ((uint32_t)__half_as_ushort(l1) << 16);
     // (the dynamic LDS block is the kernel's only LDS object: its offsets are LDS addresses)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) *(dm_lds_u128*)(uintptr_t)(uint32_t)(e * 256 + half * 128 + i * 16) = (dm_u32x4){hi, lo, hi, lo};
+    for (int i = 0; i < 8; ++i)      // (each entry starts with another of its pieces: sixteen lanes then write to all banks, not to two
+      // groups: K and V of 4 x 500 tokens of 8 heads 10.5 -> 9.2 us)
+      *(dm_lds_u128*)(uintptr_t)(uint32_t)(e * 256 + half * 128 + ((i + e) & 7) * 16) = (dm_u32x4){hi, lo, hi, lo};
   }
 
   __syncthreads();
