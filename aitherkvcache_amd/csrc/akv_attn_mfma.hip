@@ -327,7 +327,8 @@ __device__ __forceinline__ void mf_load_table_words(const uint32_t* __restrict__
   }
 }
 // Entries lie 256 bytes apart, so the four entries that sixteen lanes write at a time would meet on the same banks: each starts
-// with another of its pieces (decode steps up to 0.7 us shorter: 24 contexts of 200 in 2 bits 23.2 -> 22.5, a large one no longer).  Not so at 3 bits: a quarter of the threads write, and the main loop came out slower (126.0 -> 127.7).
+// with another of its pieces (decode steps up to 0.7 us shorter: 24 contexts of 200 in 2 bits 23.2 -> 22.5, a large one no
+// longer).  Not so at 3 bits: a quarter of the threads write, and the main loop came out slower (126.0 -> 127.7).
 template <int BITS>
 __device__ __forceinline__ void mf_fill_tables(const uint32_t (&w)[6]) {
   if constexpr (BITS == 3) {
