@@ -344,61 +344,114 @@ __device__ __forceinline__ void akv_sort_boundaries(float (&b)[N]) {
   }
 }
 // w = 2 w + bit per level: the code of y (how many of the sorted boundaries lie below it; a NaN lies past all of them), its bits
-// shifted into a stream as the carry of an addition -- 19 (4 bits), 10 (3) and 5 (2) instructions with the append, where counting
-// takes two a boundary.
+// shifted into a stream as the carry of an addition, for two values at a time -- 20 (4 bits), 11 (3) and 6 (2) instructions a value
+// with the append, where counting takes two a boundary.
+//
+// A carry or mask that a vector compare writes may be read two wait states later at the earliest (gfx940 and up; the compiler puts
+// them between, but it does not look inside inline assembly).  Hence two values: between a compare of one and its use stand the
+// selections of the other, and an s_nop at both ends, where they are too few.
 template <int MB>
-__device__ __forceinline__ void akv_append_code(uint32_t& w, float y, const float (&b)[(1 << MB) - 1]) {
+__device__ __forceinline__ void akv_append_codes(uint32_t& wa, float ya, uint32_t& wb, float yb, const float (&b)[(1 << MB) - 1]) {
+  uint64_t m;      // the second value's masks
   if constexpr (MB == 4) {
-    float s0, s2, s4, s6, t1, t3, t5;
-    asm("v_cmp_nle_f32 vcc, %8, %16\n\t"
-        "v_cndmask_b32 %6, %12, %20, vcc\n\t"
-        "v_cndmask_b32 %5, %10, %18, vcc\n\t"
-        "v_cndmask_b32 %7, %14, %22, vcc\n\t"
-        "v_cndmask_b32 %1, %9, %17, vcc\n\t"
-        "v_cndmask_b32 %2, %11, %19, vcc\n\t"
-        "v_cndmask_b32 %3, %13, %21, vcc\n\t"
-        "v_cndmask_b32 %4, %15, %23, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %8, %6\n\t"
-        "v_cndmask_b32 %5, %5, %7, vcc\n\t"
-        "v_cndmask_b32 %1, %1, %3, vcc\n\t"
-        "v_cndmask_b32 %2, %2, %4, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %8, %5\n\t"
-        "v_cndmask_b32 %1, %1, %2, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %8, %1\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
-        : "+v"(w), "=&v"(s0), "=&v"(s2), "=&v"(s4), "=&v"(s6), "=&v"(t1), "=&v"(t3), "=&v"(t5)
-        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]), "v"(b[8]), "v"(b[9]), "v"(b[10]), "v"(b[11]),
-          "v"(b[12]), "v"(b[13]), "v"(b[14])
+    float a1, a2, a3, a4, a5, a6, a7, b1, b2, b3, b4, b5, b6, b7;
+    asm("v_cmp_nle_f32 vcc, %[ya], %[c7]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[c7]\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32 %[a6], %[c3], %[c11], vcc\n\t"
+        "v_cndmask_b32 %[a5], %[c1], %[c9], vcc\n\t"
+        "v_cndmask_b32 %[a7], %[c5], %[c13], vcc\n\t"
+        "v_cndmask_b32 %[a1], %[c0], %[c8], vcc\n\t"
+        "v_cndmask_b32 %[a2], %[c2], %[c10], vcc\n\t"
+        "v_cndmask_b32 %[a3], %[c4], %[c12], vcc\n\t"
+        "v_cndmask_b32 %[a4], %[c6], %[c14], vcc\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "v_cmp_nle_f32 vcc, %[ya], %[a6]\n\t"
+        "v_cndmask_b32 %[b6], %[c3], %[c11], %[m]\n\t"
+        "v_cndmask_b32 %[b5], %[c1], %[c9], %[m]\n\t"
+        "v_cndmask_b32 %[b7], %[c5], %[c13], %[m]\n\t"
+        "v_cndmask_b32 %[b1], %[c0], %[c8], %[m]\n\t"
+        "v_cndmask_b32 %[b2], %[c2], %[c10], %[m]\n\t"
+        "v_cndmask_b32 %[b3], %[c4], %[c12], %[m]\n\t"
+        "v_cndmask_b32 %[b4], %[c6], %[c14], %[m]\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[b6]\n\t"
+        "v_cndmask_b32 %[a5], %[a5], %[a7], vcc\n\t"
+        "v_cndmask_b32 %[a1], %[a1], %[a3], vcc\n\t"
+        "v_cndmask_b32 %[a2], %[a2], %[a4], vcc\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "v_cmp_nle_f32 vcc, %[ya], %[a5]\n\t"
+        "v_cndmask_b32 %[b5], %[b5], %[b7], %[m]\n\t"
+        "v_cndmask_b32 %[b1], %[b1], %[b3], %[m]\n\t"
+        "v_cndmask_b32 %[b2], %[b2], %[b4], %[m]\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[b5]\n\t"
+        "v_cndmask_b32 %[a1], %[a1], %[a2], vcc\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "v_cmp_nle_f32 vcc, %[ya], %[a1]\n\t"
+        "v_cndmask_b32 %[b1], %[b1], %[b2], %[m]\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[b1]\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]"
+        : [wa] "+v"(wa), [wb] "+v"(wb), [m] "=&s"(m), [a1] "=&v"(a1), [a2] "=&v"(a2), [a3] "=&v"(a3), [a4] "=&v"(a4), [a5] "=&v"(a5), [a6] "=&v"(a6),
+          [a7] "=&v"(a7), [b1] "=&v"(b1), [b2] "=&v"(b2), [b3] "=&v"(b3), [b4] "=&v"(b4), [b5] "=&v"(b5), [b6] "=&v"(b6), [b7] "=&v"(b7)
+        : [ya] "v"(ya), [yb] "v"(yb), [c0] "v"(b[0]), [c1] "v"(b[1]), [c2] "v"(b[2]), [c3] "v"(b[3]), [c4] "v"(b[4]), [c5] "v"(b[5]), [c6] "v"(b[6]),
+          [c7] "v"(b[7]), [c8] "v"(b[8]), [c9] "v"(b[9]), [c10] "v"(b[10]), [c11] "v"(b[11]), [c12] "v"(b[12]), [c13] "v"(b[13]), [c14] "v"(b[14])
         : "vcc");
   } else if constexpr (MB == 3) {
-    float t0, t1, t2;
-    asm("v_cmp_nle_f32 vcc, %4, %8\n\t"
-        "v_cndmask_b32 %2, %6, %10, vcc\n\t"
-        "v_cndmask_b32 %1, %5, %9, vcc\n\t"
-        "v_cndmask_b32 %3, %7, %11, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %4, %2\n\t"
-        "v_cndmask_b32 %1, %1, %3, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %4, %1\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
-        : "+v"(w), "=&v"(t0), "=&v"(t1), "=&v"(t2)
-        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6])
+    float a1, a2, a3, b1, b2, b3;
+    asm("v_cmp_nle_f32 vcc, %[ya], %[c3]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[c3]\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32 %[a2], %[c1], %[c5], vcc\n\t"
+        "v_cndmask_b32 %[a1], %[c0], %[c4], vcc\n\t"
+        "v_cndmask_b32 %[a3], %[c2], %[c6], vcc\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "v_cmp_nle_f32 vcc, %[ya], %[a2]\n\t"
+        "v_cndmask_b32 %[b2], %[c1], %[c5], %[m]\n\t"
+        "v_cndmask_b32 %[b1], %[c0], %[c4], %[m]\n\t"
+        "v_cndmask_b32 %[b3], %[c2], %[c6], %[m]\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[b2]\n\t"
+        "v_cndmask_b32 %[a1], %[a1], %[a3], vcc\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "v_cmp_nle_f32 vcc, %[ya], %[a1]\n\t"
+        "v_cndmask_b32 %[b1], %[b1], %[b3], %[m]\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[b1]\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]"
+        : [wa] "+v"(wa), [wb] "+v"(wb), [m] "=&s"(m), [a1] "=&v"(a1), [a2] "=&v"(a2), [a3] "=&v"(a3), [b1] "=&v"(b1), [b2] "=&v"(b2), [b3] "=&v"(b3)
+        : [ya] "v"(ya), [yb] "v"(yb), [c0] "v"(b[0]), [c1] "v"(b[1]), [c2] "v"(b[2]), [c3] "v"(b[3]), [c4] "v"(b[4]), [c5] "v"(b[5]), [c6] "v"(b[6])
         : "vcc");
   } else if constexpr (MB == 2) {
-    float t;
-    asm("v_cmp_nle_f32 vcc, %2, %4\n\t"
-        "v_cndmask_b32 %1, %3, %5, vcc\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"
-        "v_cmp_nle_f32 vcc, %2, %1\n\t"
-        "v_addc_co_u32 %0, vcc, %0, %0, vcc"
-        : "+v"(w), "=&v"(t)
-        : "v"(y), "v"(b[0]), "v"(b[1]), "v"(b[2])
+    float a1, b1;
+    asm("v_cmp_nle_f32 vcc, %[ya], %[c1]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[c1]\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32 %[a1], %[c0], %[c2], vcc\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "v_cmp_nle_f32 vcc, %[ya], %[a1]\n\t"
+        "v_cndmask_b32 %[b1], %[c0], %[c2], %[m]\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[b1]\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]"
+        : [wa] "+v"(wa), [wb] "+v"(wb), [m] "=&s"(m), [a1] "=&v"(a1), [b1] "=&v"(b1)
+        : [ya] "v"(ya), [yb] "v"(yb), [c0] "v"(b[0]), [c1] "v"(b[1]), [c2] "v"(b[2])
         : "vcc");
   } else {
-    asm("v_cmp_nle_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(y), "v"(b[0]) : "vcc");
+    asm("v_cmp_nle_f32 vcc, %[ya], %[c0]\n\t"
+        "v_cmp_nle_f32 %[m], %[yb], %[c0]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]"
+        : [wa] "+v"(wa), [wb] "+v"(wb), [m] "=&s"(m)
+        : [ya] "v"(ya), [yb] "v"(yb), [c0] "v"(b[0])
+        : "vcc");
   }
 }

@@ -18,8 +18,8 @@
 //
 // What bounds it: a decode step (192 to 768 rows) is one step per workgroup, a chain of trips to memory: matrix and rows,
 // slots, stores: 11.4 us before the coordinates were shared out, 6.4 now (head_dim 256, up to 1,024 rows).  Large calls are bound
-// by the search, 22 vector instructions a value in 4 bits.  K and V of 8,192 tokens of 8 heads in 4 bits: 80.5 us at
-// head_dim 256 and 16.5 at 64, where counting with two instructions a boundary and a byte per code through LDS took 98.2 and 21.4.
+// by the search, 23 instructions a value in 4 bits.  K and V of 8,192 tokens of 8 heads in 4 bits: 82.0 us at
+// head_dim 256 and 17.6 at 64, where counting with two instructions a boundary and a byte per code through LDS took 98.0 and 22.5.
 #include "akv_common.h"
 
 typedef _Float16 ew_half8 __attribute__((ext_vector_type(8)));
@@ -219,10 +219,13 @@ __global__ __launch_bounds__((ew_cfg<D, MT, XDT, PARTS, NT>::THREADS)) void akv_
       const float2 f = *(const float2*)&info[16 * mt + col];
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        uint32_t c = 0;                                    // first code in the top bits; NaN lies past every boundary
+        uint32_t c[2] = {0, 0};                            // first code in the top bits; NaN lies past every boundary
+        float y[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) akv_append_code<BITS>(c, ldexpf(acc[nt][i] * f.x, __float_as_int(f.y)), bnd);
-        codes[16 * mt + col][4 * (NT * wave + nt) + g] = (unsigned short)c;
+        for (int i = 0; i < 4; ++i) y[i] = ldexpf(acc[nt][i] * f.x, __float_as_int(f.y));
+        akv_append_codes<BITS>(c[0], y[0], c[1], y[2], bnd);
+        akv_append_codes<BITS>(c[0], y[1], c[1], y[3], bnd);
+        codes[16 * mt + col][4 * (NT * wave + nt) + g] = (unsigned short)((c[0] << (2 * BITS)) | c[1]);
       }
     }
     __syncthreads();

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void hyb_encode_kernel(hyb_enc_args a) {
 // The two groups of a vector have nothing in common but the row they are written to: even wavefronts take group 0 of 64
 // vectors, odd ones group 1, and K and V are one launch.  What bounds it: vector instructions, some 45 a coordinate, as long as
 // there are several wavefronts per SIMD; below that, the chain of one lane.  K and V of 2,048 / 8,192 tokens of 8 heads:
-// 9.3 / 21.7 us; with both groups in one lane and a launch per tensor it was 42.9 (a wavefront per vector) / 47.1.
+// 9.2 / 22.3 us; with both groups in one lane and a launch per tensor it was 42.9 (a wavefront per vector) / 47.1.
 // ----------------------------------------------------------------------------------
 // one group of 64 coordinates -> MB-bit codes, sign bits and the two norms as dwords of the packed row (6 / 4 dwords of codes,
 // 2 of signs, 1 of norms).  had, qjl, bnd: the same for all lanes (scalar loads); cen in LDS.
@@ -149,13 +149,15 @@ __device__ __forceinline__ void hyb_encode_group_lane(const void* x, int64_t off
     for (int h = 0; h < 2; ++h) {
       uint32_t g24[4];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+      for (int g = 0; g < 4; g += 2) {
         g24[g] = 0u;
+        g24[g + 1] = 0u;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          float& r = v[32 * h + 8 * g + i];
-          akv_append_code<3>(g24[g], akv_mul_rn(r, 0.125f), bnd);
+          float &r = v[32 * h + 8 * g + i], &s = v[32 * h + 8 * g + 8 + i];
+          akv_append_codes<3>(g24[g], akv_mul_rn(r, 0.125f), g24[g + 1], akv_mul_rn(s, 0.125f), bnd);
           r = cen[g24[g] & 7u];
+          s = cen[g24[g + 1] & 7u];
         }
       }
       words[3 * h] = __builtin_bswap32((g24[0] << 8) | (g24[1] >> 16));
@@ -165,13 +167,15 @@ __device__ __forceinline__ void hyb_encode_group_lane(const void* x, int64_t off
   } else {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      uint32_t w = 0u;
+      uint32_t w = 0u, x = 0u;           // upper and lower half of the word
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        akv_append_code<2>(w, akv_mul_rn(v[16 * k + i], 0.125f), bnd);
-        v[16 * k + i] = cen[w & 3u];
+      for (int i = 0; i < 8; ++i) {
+        float &r = v[16 * k + i], &s = v[16 * k + 8 + i];
+        akv_append_codes<2>(w, akv_mul_rn(r, 0.125f), x, akv_mul_rn(s, 0.125f), bnd);
+        r = cen[w & 3u];
+        s = cen[x & 3u];
       }
-      words[k] = __builtin_bswap32(w);
+      words[k] = __builtin_bswap32((w << 16) | x);
     }
   }
   hyb_fwht_regs<64>(v);
@@ -186,17 +190,13 @@ __device__ __forceinline__ void hyb_encode_group_lane(const void* x, int64_t off
   for (int j = 0; j < 64; ++j) v[j] = akv_mul_rn(u[j], qjl[j]);
   hyb_fwht_regs<64>(v);
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    uint32_t w = 0u;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) hyb_append_sign(w, akv_mul_rn(v[32 * k + i], 0.125f));
-    words[CW + k] = __builtin_bswap32(w);
-  }
+  for (int k = 0; k < 2; ++k) words[CW + k] = __builtin_bswap32(hyb_sign_word(v + 32 * k, 0.125f));
   words[CW + 2] = (uint32_t)__half_as_ushort(__float2half_rn(nrm)) | ((uint32_t)__half_as_ushort(__float2half_rn(rn)) << 16);
 }
 
+// (three wavefronts a SIMD: float16 needs the limit for that, the other types stay below it, and float32 spills under it)
 template <int XDT, bool PAGED>
-__global__ __launch_bounds__(256) void hyb_encode_lane_kernel(hyb_enc_args a) {
+__global__ __launch_bounds__(256, XDT == AKV_F16 ? 3 : 1) void hyb_encode_lane_kernel(hyb_enc_args a) {
   __shared__ float cen[12];              // 8 centroids of group 0, 4 of group 1
   if (threadIdx.x < 12) cen[threadIdx.x] = a.table[HYB_CEN0 + threadIdx.x];
   static_assert(HYB_CEN1 == HYB_CEN0 + 8, "the two codebooks lie together");

@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void h25_encode_kernel(h25_enc_args a) {
 // unit in the last place, from where the second rounds correctly (Markstein, 1990).  Both for quotients and remainders above 2^-126.
 //
 // What bounds it: the chain of one lane up to one wavefront per SIMD, then vector instructions, some 45 a coordinate.  K and V of
-// 2,048 / 8,192 tokens of 8 heads: 14.2 / 20.2 us, with a wavefront per vector 30.1 / 113.
+// 2,048 / 8,192 tokens of 8 heads: 14.5 / 20.8 us, with a wavefront per vector 30.1 / 113.
 // ----------------------------------------------------------------------------------
 __device__ __forceinline__ float h25_by_root(float x, float root, float rcp) {
   const float q = akv_mul_rn(x, rcp);
@@ -186,14 +186,15 @@ __device__ __forceinline__ void h25_encode_group_lane(const void* x, int64_t off
   transform();
 #pragma unroll
   for (int k = 0; k < CW; ++k) {
-    uint32_t w = 0u;
+    uint32_t w = 0u, x = 0u;             // upper and lower half of the word
 #pragma unroll
-    for (int i = 0; i < 32 / MB; ++i) {
-      float& r = v[32 / MB * k + i];
-      akv_append_code<MB>(w, h25_by_root(r, root, rcp_root), bnd);
+    for (int i = 0; i < 16 / MB; ++i) {
+      float &r = v[32 / MB * k + i], &s = v[32 / MB * k + 16 / MB + i];
+      akv_append_codes<MB>(w, h25_by_root(r, root, rcp_root), x, h25_by_root(s, root, rcp_root), bnd);
       r = cen[w & ((1u << MB) - 1u)];
+      s = cen[x & ((1u << MB) - 1u)];
     }
-    words[k] = __builtin_bswap32(w);
+    words[k] = __builtin_bswap32((w << 16) | x);
   }
   transform();
 #pragma unroll
@@ -206,17 +207,12 @@ __device__ __forceinline__ void h25_encode_group_lane(const void* x, int64_t off
   for (int j = 0; j < N; ++j) v[j] = akv_mul_rn(u[j], qjl[j]);
   transform();
 #pragma unroll
-  for (int k = 0; k < N / 32; ++k) {
-    uint32_t w = 0u;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) hyb_append_sign(w, akv_mul_rn(v[32 * k + i], rcp_root));      // (the quotient has this sign)
-    words[CW + k] = __builtin_bswap32(w);
-  }
+  for (int k = 0; k < N / 32; ++k) words[CW + k] = __builtin_bswap32(hyb_sign_word(v + 32 * k, rcp_root));      // (the quotient has this sign)
   words[CW + N / 32] = (uint32_t)__half_as_ushort(__float2half_rn(nrm)) | ((uint32_t)__half_as_ushort(__float2half_rn(rn)) << 16);
 }
 
 template <int XDT, bool PAGED>
-__global__ __launch_bounds__(256) void h25_encode_lane_kernel(h25_enc_args a) {
+__global__ __launch_bounds__(256, 2) void h25_encode_lane_kernel(h25_enc_args a) {
   __shared__ float cen[6];               // 4 centroids of group 0, 2 of group 1
   if (threadIdx.x < 6) cen[threadIdx.x] = a.table[H25_CEN0 + threadIdx.x];
   static_assert(H25_CEN1 == H25_CEN0 + 4, "the two codebooks lie together");

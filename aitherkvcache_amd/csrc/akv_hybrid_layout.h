@@ -93,9 +93,23 @@ __device__ __forceinline__ void hyb_load_row(const void* x, int64_t off, float* 
     }
   }
 }
-// w = 2 w + (y >= 0)
-__device__ __forceinline__ void hyb_append_sign(uint32_t& w, float y) {
-  asm("v_cmp_le_f32 vcc, 0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(w) : "v"(y) : "vcc");
+// the signs of v[0 .. 32) (a bit set where v scale >= 0), first value in the top bit: both halves of the word side by side, so that
+// two wait states lie between a compare and its use (akv_append_codes)
+__device__ __forceinline__ uint32_t hyb_sign_word(const float* v, float scale) {
+  uint32_t a = 0u, b = 0u;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    uint64_t m;
+    asm("v_cmp_le_f32 vcc, 0, %[ya]\n\t"
+        "v_cmp_le_f32 %[m], 0, %[yb]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[wa], vcc, %[wa], %[wa], vcc\n\t"
+        "v_addc_co_u32 %[wb], %[m], %[wb], %[wb], %[m]"
+        : [wa] "+v"(a), [wb] "+v"(b), [m] "=&s"(m)
+        : [ya] "v"(akv_mul_rn(v[i], scale)), [yb] "v"(akv_mul_rn(v[16 + i], scale))
+        : "vcc");
+  }
+  return (a << 16) | b;
 }
 
 // 32 values of every lane's row to memory: through LDS (64 rows of 36 floats, a wavefront's own), so that eight lanes write 128
