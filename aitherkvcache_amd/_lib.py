@@ -203,6 +203,25 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
+def check_caches(block_size: int, num_kv_heads: int, *caches: torch.Tensor) -> None:
+    """The positions and heads a call addresses exist in its cache tensors [blocks, positions, heads, ...]."""
+    for t in caches:
+        if t.shape[1] < block_size or t.shape[2] < num_kv_heads:
+            raise ValueError(f"block_size {block_size} and {num_kv_heads} kv heads do not fit a cache of shape {tuple(t.shape)}")
+
+
+def check_batch(num_seqs: int, block_tables: torch.Tensor, context_lens: torch.Tensor) -> None:
+    """Every sequence has a row of the block tables and a length."""
+    if block_tables.shape[0] < num_seqs or context_lens.numel() < num_seqs:
+        raise ValueError(f"{num_seqs} sequences, but block_tables {tuple(block_tables.shape)} and context_lens {tuple(context_lens.shape)}")
+
+
+def check_slots(num_tokens: int, slot_mapping: torch.Tensor) -> None:
+    """Every token has a slot."""
+    if slot_mapping.numel() < num_tokens:
+        raise ValueError(f"{num_tokens} tokens, but slot_mapping {tuple(slot_mapping.shape)}")
+
+
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 

@@ -97,14 +97,22 @@ bool stream_of(int device, void*& stream) {
 }
 PyObject* status(int rc) { return PyLong_FromLong(rc); }
 
-// rows of a cache: [blocks, positions, heads, bytes]
-bool packed_rows(const at::Tensor& t, int64_t bytes) { return t.dim() == 4 && t.scalar_type() == at::kByte && t.stride(3) == 1 && t.size(3) >= bytes; }
-bool norm_rows(const at::Tensor& t) { return t.dim() == 3 && t.scalar_type() == at::kFloat; }
+// rows of a cache: [blocks, positions, heads, bytes], and their norms; a call addresses `block` positions and `heads` heads
+bool packed_rows(const at::Tensor& t, int64_t bytes, int64_t block, int64_t heads) {
+  return t.dim() == 4 && t.scalar_type() == at::kByte && t.stride(3) == 1 && t.size(3) >= bytes && t.size(1) >= block && t.size(2) >= heads;
+}
+bool norm_rows(const at::Tensor& t, int64_t block, int64_t heads) {
+  return t.dim() == 3 && t.scalar_type() == at::kFloat && t.size(1) >= block && t.size(2) >= heads;
+}
+// a table of at least n floats
+bool floats(const at::Tensor& t, int64_t n) { return t.scalar_type() == at::kFloat && t.is_contiguous() && t.numel() >= n; }
+// the blocks a write may go to: those the caller names (0: all), as far as they exist
+int64_t blocks_of(int64_t named, int64_t held) { return named != 0 ? std::min(named, held) : held; }
 
 // what every attention call checks of its queries, tables and lengths
 bool attn_inputs(const at::Tensor& q, const at::Tensor& tables, const at::Tensor& lens, int64_t heads, int64_t d) {
   return q.dim() == 3 && q.size(0) > 0 && q.size(1) == heads && q.size(2) == d && q.stride(2) == 1 && float_code(q) >= 0 && tables.dim() == 2 &&
-         tables.stride(1) == 1 && index_code(tables) >= 0 && lens.dim() == 1 && lens.is_contiguous() && index_code(lens) >= 0;
+         tables.size(0) >= q.size(0) && lens.numel() >= q.size(0) && tables.stride(1) == 1 && index_code(tables) >= 0 && lens.dim() == 1 && lens.is_contiguous() && index_code(lens) >= 0;
 }
 
 // (query, k_packed, k_norms, v_packed, v_norms, block_tables, context_lens, centroids, workspace or None, prepared rotation,
@@ -118,8 +126,9 @@ PyObject* uniform_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const at::Tensor &q = ts.take(a[0]), &kp = ts.take(a[1]), &kn = ts.take(a[2]), &vp = ts.take(a[3]), &vn = ts.take(a[4]);
   const at::Tensor &bt = ts.take(a[5]), &cl = ts.take(a[6]), &cen = ts.take(a[7]), &ws = ts.take(a[8]);
   const int64_t heads = v[2], d = v[3], row = v[4], bits = v[5], block = v[6];
-  if (!ts.ok() || !attn_inputs(q, bt, cl, heads, d) || !packed_rows(kp, row) || !packed_rows(vp, row) || !norm_rows(kn) || !norm_rows(vn)) Py_RETURN_NONE;
+  if (!ts.ok() || !attn_inputs(q, bt, cl, heads, d) || kp.dim() != 4 || bits < 2 || bits > 4 || !floats(cen, 1 << bits)) Py_RETURN_NONE;
   const int64_t seqs = q.size(0), kv_heads = a[10] == Py_None ? kp.size(2) : v[1];
+  if (!packed_rows(kp, row, block, kv_heads) || !packed_rows(vp, row, block, kv_heads) || !norm_rows(kn, block, kv_heads) || !norm_rows(vn, block, kv_heads)) Py_RETURN_NONE;
   if (ws.numel() < (int64_t)g_lib.attn_bytes((int)seqs, (int)heads, (int)d)) Py_RETURN_NONE;
   const int64_t blocks = std::min(std::min(kp.size(0), kn.size(0)), std::min(vp.size(0), vn.size(0)));
   void* stream;
@@ -154,8 +163,9 @@ PyObject* hybrid_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const at::Tensor &q = ts.take(a[0]), &kc = ts.take(a[1]), &vc = ts.take(a[2]), &bt = ts.take(a[3]), &cl = ts.take(a[4]);
   const at::Tensor &table = ts.take(a[5]), &ws = ts.take(a[6]);
   const int64_t heads = v[2], d = v[3], row = v[4], block = v[5];
-  if (!ts.ok() || v[0] < 0 || v[0] > 1 || !attn_inputs(q, bt, cl, heads, d) || !packed_rows(kc, row) || !packed_rows(vc, row)) Py_RETURN_NONE;
+  if (!ts.ok() || v[0] < 0 || v[0] > 1 || !attn_inputs(q, bt, cl, heads, d) || kc.dim() != 4 || !floats(table, AKV_HYB_TABLE_FLOATS)) Py_RETURN_NONE;
   const int64_t seqs = q.size(0), kv_heads = a[8] == Py_None ? kc.size(2) : v[1];
+  if (!packed_rows(kc, row, block, kv_heads) || !packed_rows(vc, row, block, kv_heads)) Py_RETURN_NONE;
   if (ws.numel() < (int64_t)g_lib.hybrid_bytes((int)seqs, (int)heads)) Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
@@ -193,11 +203,11 @@ PyObject* uniform_encode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensors ts;
   const at::Tensor &key = ts.take(a[0]), &value = ts.take(a[1]), &slots = ts.take(a[2]), &kp = ts.take(a[3]), &kn = ts.take(a[4]);
   const at::Tensor &vp = ts.take(a[5]), &vn = ts.take(a[6]), &rot = ts.take(a[7]), &bnd = ts.take(a[8]);
-  (void)rot;
   if (!ts.ok() || !pair_inputs(key, value, slots) || v[1] < 2 || v[1] > 4 || key.size(2) % 8 != 0) Py_RETURN_NONE;
-  const int64_t row = key.size(2) * v[1] / 8;
-  if (!packed_rows(kp, row) || !packed_rows(vp, row) || !norm_rows(kn) || !norm_rows(vn) || kp.sizes() != vp.sizes() || kp.strides() != vp.strides() || kn.sizes() != vn.sizes() || kn.strides() != vn.strides() ||
-      bnd.scalar_type() != at::kFloat || !bnd.is_contiguous() || (key.size(2) & (key.size(2) - 1)) != 0)
+  const int64_t heads = key.size(1), d = key.size(2), row = d * v[1] / 8, block = v[2];
+  if (!packed_rows(kp, row, block, heads) || !norm_rows(kn, block, heads) || vp.scalar_type() != at::kByte || vn.scalar_type() != at::kFloat ||
+      kp.sizes() != vp.sizes() || kp.strides() != vp.strides() || kn.sizes() != vn.sizes() || kn.strides() != vn.strides() || rot.dim() != 2 ||
+      rot.size(0) != d || rot.size(1) != d || !floats(bnd, (1 << v[1]) - 1) || (d & (d - 1)) != 0)
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
@@ -207,7 +217,7 @@ PyObject* uniform_encode(PyObject*, PyObject* const* a, Py_ssize_t n) {
                     slots.const_data_ptr(), index_code(slots), (const void*)(uintptr_t)v[0], (const float*)bnd.const_data_ptr(), (int)v[1],
                     (uint8_t*)kp.mutable_data_ptr(), (uint8_t*)vp.mutable_data_ptr(), kp.stride(0), kp.stride(1), kp.stride(2),
                     (float*)kn.mutable_data_ptr(), (float*)vn.mutable_data_ptr(), kn.stride(0), kn.stride(1), kn.stride(2), (int)v[2],
-                    v[3] != 0 ? v[3] : kp.size(0), stream);
+                    blocks_of(v[3], std::min(kp.size(0), kn.size(0))), stream);
   Py_END_ALLOW_THREADS;
   return status(rc);
 }
@@ -221,8 +231,8 @@ PyObject* hybrid_encode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!integer(a[6 + i], v[i])) Py_RETURN_NONE;
   Tensors ts;
   const at::Tensor &key = ts.take(a[0]), &value = ts.take(a[1]), &slots = ts.take(a[2]), &kc = ts.take(a[3]), &vc = ts.take(a[4]), &table = ts.take(a[5]);
-  if (!ts.ok() || v[0] < 0 || v[0] > 1 || !pair_inputs(key, value, slots) || key.size(2) != v[1] || !packed_rows(kc, v[2]) || !packed_rows(vc, v[2]) ||
-      kc.sizes() != vc.sizes() || kc.strides() != vc.strides())
+  if (!ts.ok() || v[0] < 0 || v[0] > 1 || !floats(table, AKV_HYB_TABLE_FLOATS) || !pair_inputs(key, value, slots) || key.size(2) != v[1] || !packed_rows(kc, v[2], v[3], key.size(1)) ||
+      vc.scalar_type() != at::kByte || kc.sizes() != vc.sizes() || kc.strides() != vc.strides())
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
@@ -230,7 +240,7 @@ PyObject* hybrid_encode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Py_BEGIN_ALLOW_THREADS;
   rc = g_lib.hybrid_encode[v[0]](key.const_data_ptr(), value.const_data_ptr(), float_code(key), key.size(0), (int)key.size(1), key.stride(0), key.stride(1),
                                  slots.const_data_ptr(), index_code(slots), (const float*)table.const_data_ptr(), (uint8_t*)kc.mutable_data_ptr(),
-                                 (uint8_t*)vc.mutable_data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2), (int)v[3], v[4] != 0 ? v[4] : kc.size(0), stream);
+                                 (uint8_t*)vc.mutable_data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2), (int)v[3], blocks_of(v[4], kc.size(0)), stream);
   Py_END_ALLOW_THREADS;
   return status(rc);
 }
@@ -254,11 +264,11 @@ PyObject* decode_blocks(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const at::Tensor &kc = ts.take(a[0]), &vc = ts.take(a[1]), &kb = ts.take(a[2]), &vb = ts.take(a[3]), &ids = ts.take(a[4]);
   const at::Tensor &kn = ts.take(a[5]), &vn = ts.take(a[6]), &cen = ts.take(a[7]);
   const int64_t blocks = v[1], d = v[2];
-  if (!ts.ok() || !packed_rows(kc, v[3]) || !packed_rows(vc, v[3]) || !norm_rows(kn) || !norm_rows(vn) || kb.dim() != 4 || kb.stride(3) != 1 ||
+  if (!ts.ok() || !packed_rows(kc, v[3], 0, 0) || !packed_rows(vc, v[3], 0, 0) || !norm_rows(kn, 0, 0) || !norm_rows(vn, 0, 0) || kb.dim() != 4 || kb.stride(3) != 1 ||
       float_code(kb) < 0 || kb.size(3) != d || kb.numel() == 0 || vb.scalar_type() != kb.scalar_type() || kb.sizes() != vb.sizes() ||
       kb.strides() != vb.strides() || kc.sizes() != vc.sizes() || kc.strides() != vc.strides() || kn.sizes() != vn.sizes() || kn.strides() != vn.strides() ||
       kc.sizes().slice(0, 3) != kn.sizes() || kc.sizes().slice(0, 3) != kb.sizes().slice(0, 3) || blocks <= 0 || blocks > kc.size(0) ||
-      index_code(ids) < 0 || !ids.is_contiguous() || ids.numel() == 0)
+      v[4] < 2 || v[4] > 4 || !floats(cen, 1 << v[4]) || index_code(ids) < 0 || !ids.is_contiguous() || ids.numel() == 0)
     Py_RETURN_NONE;
   const auto k = span(kb), w = span(vb);
   if (!(k.second <= w.first || w.second <= k.first)) Py_RETURN_NONE;

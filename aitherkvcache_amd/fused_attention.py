@@ -112,6 +112,8 @@ class TQPagedAttention:
         for name, t in (("k_packed", k_packed), ("v_packed", v_packed)):
             if t.dtype != torch.uint8 or t.stride(-1) != 1 or t.shape[-1] < self.packed_dim:
                 raise ValueError(f"{name} must be uint8 with contiguous rows of >= {self.packed_dim} bytes")
+        _lib.check_caches(block_size, num_kv_heads, k_packed, k_norms, v_packed, v_norms)
+        _lib.check_batch(num_seqs, block_tables, context_lens)
         if _static_out is not None and (k_norms.dtype != torch.float32 or v_norms.dtype != torch.float32):
             raise ValueError("forward_no_alloc needs float32 norms (a conversion would allocate)")
         k_norms = k_norms if k_norms.dtype == torch.float32 else k_norms.float()

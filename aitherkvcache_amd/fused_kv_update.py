@@ -25,6 +25,19 @@ _DTYPE_OK = (torch.float16, torch.bfloat16, torch.float32)
 __all__ = ["fused_tq4_kv_update", "fused_kv_update", "fused_encode_and_store", "HAS_TRITON", "HAS_HIP"]
 
 
+def _check_write(num_tokens, num_kv_heads, head_dim, slot_mapping, packed, norms, rotation, boundaries, bits, block_size,
+                 max_blocks, prepared) -> int:
+    """Everything a write reads and writes by these sizes exists; returns how many blocks it may write to."""
+    _lib.check_caches(block_size, num_kv_heads, packed, norms)
+    _lib.check_slots(num_tokens, slot_mapping)
+    rotated = rotation.shape[0] if prepared is None else getattr(prepared, "head_dim", head_dim)
+    if rotated != head_dim:
+        raise ValueError(f"head_dim {head_dim}, but a rotation of {rotated} coordinates")
+    if boundaries.numel() < (1 << bits) - 1:
+        raise ValueError(f"{bits} bits, but {boundaries.numel()} boundaries")
+    return min(max_blocks, packed.shape[0], norms.shape[0])
+
+
 def fused_kv_update(x, slot_mapping, out_packed, out_norms, rotation, boundaries, bits,
                     block_size=16, max_blocks=0, prepared=None) -> None:
     """Quantize-and-store for one cache tensor (K or V) at `bits` in {2, 3, 4}.
@@ -47,6 +60,8 @@ def fused_kv_update(x, slot_mapping, out_packed, out_norms, rotation, boundaries
         raise ValueError("out_packed must be uint8 and out_norms float32")
     if out_packed.shape[-1] < packed_size(head_dim, bits) or out_packed.stride(-1) != 1:
         raise ValueError("out_packed rows are too short or not contiguous in the last dim")
+    max_blocks = _check_write(num_tokens, num_kv_heads, head_dim, slot_mapping, out_packed, out_norms, rotation, boundaries,
+                              bits, block_size, max_blocks, prepared)
     if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         x = x.float()
     if x.stride(-1) != 1:
@@ -103,6 +118,8 @@ def fused_kv_update_pair(key, value, slot_mapping, k_packed, k_norms, v_packed, 
         raise ValueError("packed caches must be uint8 and norms float32")
     if k_packed.shape[-1] < packed_size(head_dim, bits) or k_packed.stride(-1) != 1:
         raise ValueError("packed rows are too short or not contiguous in the last dim")
+    max_blocks = _check_write(num_tokens, num_kv_heads, head_dim, slot_mapping, k_packed, k_norms, rotation, boundaries,
+                              bits, block_size, max_blocks, prepared)
     slots = slot_mapping if slot_mapping.is_contiguous() else slot_mapping.contiguous()
     prep = prepared if prepared is not None else prepared_rotation_for(rotation)
     bnd = boundaries if (boundaries.dtype == torch.float32 and boundaries.is_contiguous()) \
@@ -143,6 +160,8 @@ class _StorePlan:
                 and kn.stride() == vn.stride() and kp.dtype == torch.uint8 and vp.dtype == torch.uint8
                 and kn.dtype == torch.float32 and vn.dtype == torch.float32 and kp.stride(-1) == 1
                 and kp.shape[-1] >= packed_size(head_dim, tq.bits) and hasattr(tq, "prepared_rotation")
+                and min(kp.shape[1], kn.shape[1]) >= tq_cache.block_size and kn.shape[2] >= kp.shape[2]
+                and tq.rotation.shape[0] == head_dim and tq.boundaries_inner.numel() >= (1 << tq.bits) - 1
                 and head_dim > 0 and (head_dim & (head_dim - 1)) == 0)
         self.fixed = None
         if not same:
@@ -155,7 +174,7 @@ class _StorePlan:
         self.tail = (kp.shape[2], head_dim)
         self.fixed = (self.prep.ptr, self.bnd.data_ptr(), tq.bits, kp.data_ptr(), vp.data_ptr(), kp.stride(0),
                       kp.stride(1), kp.stride(2), kn.data_ptr(), vn.data_ptr(), kn.stride(0), kn.stride(1),
-                      kn.stride(2), self.block_size, self.max_blocks)
+                      kn.stride(2), self.block_size, min(self.max_blocks, kp.shape[0], kn.shape[0]))
 
     def _storage(self):
         """Where the layer's four tensors lie now, or None when one of them has been replaced.  A container that is

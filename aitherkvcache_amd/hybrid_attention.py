@@ -32,6 +32,9 @@ def hybrid_encode_and_store(htq, x: torch.Tensor, slot_mapping: torch.Tensor, ca
         raise ValueError(f"cache must be uint8 with contiguous rows of >= {htq.packed_dim} bytes")
     if head_dim != htq.head_dim:
         raise ValueError(f"head_dim {head_dim} != {htq.head_dim}")
+    _lib.check_caches(block_size, num_kv_heads, cache)
+    _lib.check_slots(num_tokens, slot_mapping)
+    max_blocks = min(max_blocks, cache.shape[0])
     if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         x = x.float()
     x = htq.to_group_order(x, head_axis=1)        # (a variance-ranked split: coordinates into group order first)
@@ -73,6 +76,9 @@ def hybrid_encode_and_store_pair(htq, key: torch.Tensor, value: torch.Tensor, sl
         max_blocks = k_cache.shape[0]
     table = htq.kernel_table
     dev = _lib.require_gpu(key, value, slot_mapping, k_cache, v_cache, table)
+    _lib.check_caches(block_size, num_kv_heads, k_cache)
+    _lib.check_slots(num_tokens, slot_mapping)
+    max_blocks = min(max_blocks, k_cache.shape[0])
     _lib.check(getattr(_lib.lib(), htq._abi + "_encode_paged_kv")(
         key.data_ptr(), value.data_ptr(), _lib.dtype_code(key), num_tokens, num_kv_heads, key.stride(0), key.stride(1),
         slot_mapping.data_ptr(), _lib.itype_code(slot_mapping), table.data_ptr(),
@@ -127,6 +133,8 @@ class HybridPagedAttention:
         for name, t in (("k_cache", k_cache), ("v_cache", v_cache)):
             if t.dtype != torch.uint8 or t.stride(-1) != 1 or t.shape[-1] < self._htq.packed_dim:
                 raise ValueError(f"{name} must be uint8 with contiguous rows of >= {self._htq.packed_dim} bytes")
+        _lib.check_caches(block_size, num_kv_heads, k_cache, v_cache)
+        _lib.check_batch(num_seqs, block_tables, context_lens)
         bt = block_tables if block_tables.stride(-1) == 1 else block_tables.contiguous()
         cl = context_lens if context_lens.is_contiguous() else context_lens.contiguous()
         L = _lib.lib()

@@ -140,3 +140,60 @@ def test_refusals_stay(dev, monkeypatch, make, fmt, d):
                 run(*args)
             errors.append((e.type, str(e.value)))
         assert errors[0] == errors[1]
+
+
+@pytest.mark.parametrize("take", [False, True])
+@pytest.mark.parametrize("fmt", ["uniform", "tq35"])
+def test_sizes_that_do_not_fit_are_refused(dev, monkeypatch, fmt, take):
+    """Nothing is launched that would read past a table, a list of lengths or slots, or a cache; neither way.  (Larger ones are fine.)"""
+    d, uni = 128, fmt == "uniform"
+    x, slots, tables, lens, q = inputs(dev, d, torch.float16, torch.int32)
+    t = akv.TurboQuant(head_dim=d, bits=4, device=str(dev)) if uni else akv.HybridTurboQuant(head_dim=d, mode=fmt, device=str(dev))
+    if not uni:
+        t.calibrate_uniform(KVH)
+    attn = (akv.TQPagedAttention if uni else akv.HybridPagedAttention)(t, QH)
+    prep = t.prepared_rotation() if uni else None
+
+    def caches(positions=BS, heads=KVH, norm_blocks=NB, norm_positions=BS, norm_heads=KVH):
+        rows = [torch.zeros(NB, positions, heads, t._packed_dim if uni else t.packed_dim, dtype=torch.uint8, device=dev) for _ in range(2)]
+        norms = [torch.zeros(norm_blocks, norm_positions, norm_heads, device=dev) for _ in range(2)]
+        return (rows[0], norms[0], rows[1], norms[1]) if uni else tuple(rows)
+
+    def write(c, x=x, slots=slots, block=BS, blocks=NB, prep=prep):
+        if uni:
+            akv.fused_kv_update_pair(x[0], x[1], slots, *c, t.rotation, t.boundaries_inner, 4, block, blocks, prepared=prep)
+        else:
+            hybrid_encode_and_store_pair(t, x[0], x[1], slots, *c, block, blocks)
+        return c
+
+    def read(c, tables=tables, lens=lens, block=BS, kv_heads=None):
+        return attn.forward(q, *c, tables, lens, block_size=block, num_kv_heads=kv_heads)
+
+    good = write(caches())
+    want = read(good)                                               # the attention's workspace is there
+    with binding(monkeypatch, take) as c:
+        for args in [dict(tables=tables[:2]), dict(lens=lens[:2]), dict(block=2 * BS), dict(kv_heads=2 * KVH)]:
+            with pytest.raises(ValueError):
+                read(good, **args)
+        bad = [(caches(), dict(slots=slots[:5])), (caches(), dict(block=2 * BS)), (caches(heads=KVH - 1), {}), (caches(positions=BS // 2), {})]
+        if uni:
+            bad += [(caches(norm_positions=BS // 2), {}), (caches(norm_heads=KVH - 1), {}), (caches(), dict(x=x[..., :64], prep=prep))]
+            for shape in (dict(norm_positions=BS // 2), dict(norm_heads=KVH - 1)):
+                with pytest.raises(ValueError):
+                    read(caches(**shape))
+        for cache, args in bad:
+            with pytest.raises(ValueError):
+                write(cache, **args)
+        assert c.taken == 0
+        # accepted as ever: more rows and lengths than sequences, fewer heads and positions than the cache has
+        assert torch.equal(read(good, tables=torch.cat([tables, tables]), lens=torch.cat([lens, lens])), want)
+        assert torch.equal(read(write(caches(positions=2 * BS, heads=KVH + 1, norm_positions=2 * BS, norm_heads=KVH + 1)), kv_heads=KVH), want)
+        # blocks past the end of the cache or of its norms are skipped, whatever number of blocks is named
+        far = slots + (slots >= NB * BS // 2) * NB * BS
+        half = write(caches(), slots=far, blocks=10 ** 6)
+        for a, b in zip(half, good):
+            assert torch.equal(a[:NB // 2], b[:NB // 2]) and not a[NB // 2:].any()
+        if uni:
+            short = write(caches(norm_blocks=NB // 2))
+            assert torch.equal(short[0][:NB // 2], good[0][:NB // 2]) and torch.equal(short[3], good[3][:NB // 2]) and not short[2][NB // 2:].any()
+        assert (c.taken > 0) == take
