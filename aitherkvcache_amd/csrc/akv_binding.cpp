@@ -136,9 +136,8 @@ PyObject* uniform_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::Tensor out;
   try {
     out = at::empty({seqs, heads, d}, q.options());
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (const std::exception&) {      // (no memory: the long way tries again and raises torch's own error)
+    Py_RETURN_NONE;
   }
   int rc;
   Py_BEGIN_ALLOW_THREADS;
@@ -172,9 +171,8 @@ PyObject* hybrid_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::Tensor out;
   try {
     out = at::empty({seqs, heads, d}, q.options());
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (const std::exception&) {      // (no memory: the long way tries again and raises torch's own error)
+    Py_RETURN_NONE;
   }
   int rc;
   Py_BEGIN_ALLOW_THREADS;
@@ -333,9 +331,8 @@ PyObject* spectral_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::Tensor out;
   try {
     out = at::empty({b, qh, d}, q.options().dtype(at::kFloat));
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (const std::exception&) {      // (no memory: the long way tries again and raises torch's own error)
+    Py_RETURN_NONE;
   }
   int rc;
   Py_BEGIN_ALLOW_THREADS;

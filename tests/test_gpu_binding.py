@@ -197,3 +197,26 @@ def test_sizes_that_do_not_fit_are_refused(dev, monkeypatch, fmt, take):
             short = write(caches(norm_blocks=NB // 2))
             assert torch.equal(short[0][:NB // 2], good[0][:NB // 2]) and torch.equal(short[3], good[3][:NB // 2]) and not short[2][NB // 2:].any()
         assert (c.taken > 0) == take
+
+
+@pytest.mark.parametrize("take", [False, True])
+@pytest.mark.parametrize("make,fmt,d", [(uniform, 4, 128), (hybrid, "tq35", 128), (spectral, None, 128)])
+def test_out_of_memory_is_the_error_of_torch(dev, monkeypatch, make, fmt, d, take):
+    """What an engine catches to shrink its batch: the output of a call does not fit the memory that is left."""
+    run, _ = make(dev, fmt, d, torch.float32)
+    x, slots, _, _, _ = inputs(dev, d, torch.float32, torch.int32)
+    many = 20000                                                    # 82 MB of output
+    torch.cuda.empty_cache()                                        # (no segment is held of which that could be a part)
+    q = torch.zeros(many, QH, d, device=dev)
+    tables, lens = torch.zeros(many, 1, dtype=torch.int32, device=dev), torch.zeros(many, dtype=torch.int32, device=dev)
+    run(x[:, :BS], slots[:BS], tables, lens, q)                     # the attention's workspace is there
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (16 << 20)) / total, dev)
+    try:
+        with binding(monkeypatch, take), pytest.raises(torch.OutOfMemoryError):
+            run(x[:, :BS], slots[:BS], tables, lens, q)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert not run(x[:, :BS], slots[:BS], tables, lens, q)[-1].any()
