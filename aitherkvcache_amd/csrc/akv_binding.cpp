@@ -95,6 +95,16 @@ bool stream_of(int device, void*& stream) {
   Py_DECREF(handle);
   return !PyErr_Occurred();
 }
+// f(args...) with the interpreter's lock given up.  What is read of tensors is in `args`, read while it is held: another thread may
+// give a tensor other storage or sizes once it is not.
+template <class F, class... Args>
+int without_gil(F f, Args... args) noexcept {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS;
+  rc = f(args...);
+  Py_END_ALLOW_THREADS;
+  return rc;
+}
 PyObject* status(int rc) { return PyLong_FromLong(rc); }
 
 // rows of a cache: [blocks, positions, heads, bytes], and their norms; a call addresses `block` positions and `heads` heads
@@ -133,21 +143,13 @@ PyObject* uniform_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t blocks = std::min(std::min(kp.size(0), kn.size(0)), std::min(vp.size(0), vn.size(0)));
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
-  at::Tensor out;
-  try {
-    out = at::empty({seqs, heads, d}, q.options());
-  } catch (const std::exception&) {      // (no memory: the long way tries again and raises torch's own error)
-    Py_RETURN_NONE;
-  }
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = g_lib.attn(q.const_data_ptr(), float_code(q), q.stride(0), q.stride(1), (const uint8_t*)kp.const_data_ptr(), kp.stride(0), kp.stride(1), kp.stride(2),
-                  (const float*)kn.const_data_ptr(), kn.stride(0), kn.stride(1), kn.stride(2), (const uint8_t*)vp.const_data_ptr(), vp.stride(0), vp.stride(1),
-                  vp.stride(2), (const float*)vn.const_data_ptr(), vn.stride(0), vn.stride(1), vn.stride(2), bt.const_data_ptr(), index_code(bt), bt.stride(0),
-                  cl.const_data_ptr(), index_code(cl), (const void*)(uintptr_t)v[0], (const float*)cen.const_data_ptr(), (int)bits, out.mutable_data_ptr(),
-                  float_code(out), out.stride(0), out.stride(1), (int)seqs, (int)heads, (int)kv_heads, (int)d, (int)block, blocks, bt.size(1),
-                  (float)PyFloat_AS_DOUBLE(a[16]), ws.mutable_data_ptr(), (size_t)ws.numel(), stream);
-  Py_END_ALLOW_THREADS;
+  at::Tensor out = at::empty({seqs, heads, d}, q.options());
+  const int rc = without_gil(g_lib.attn, q.const_data_ptr(), float_code(q), q.stride(0), q.stride(1), (const uint8_t*)kp.const_data_ptr(), kp.stride(0), kp.stride(1), kp.stride(2),
+                             (const float*)kn.const_data_ptr(), kn.stride(0), kn.stride(1), kn.stride(2), (const uint8_t*)vp.const_data_ptr(), vp.stride(0), vp.stride(1),
+                             vp.stride(2), (const float*)vn.const_data_ptr(), vn.stride(0), vn.stride(1), vn.stride(2), bt.const_data_ptr(), index_code(bt), bt.stride(0),
+                             cl.const_data_ptr(), index_code(cl), (const void*)(uintptr_t)v[0], (const float*)cen.const_data_ptr(), (int)bits, out.mutable_data_ptr(),
+                             float_code(out), out.stride(0), out.stride(1), (int)seqs, (int)heads, (int)kv_heads, (int)d, (int)block, blocks, bt.size(1),
+                             (float)PyFloat_AS_DOUBLE(a[16]), ws.mutable_data_ptr(), (size_t)ws.numel(), stream);
   return rc ? status(rc) : THPVariable_Wrap(std::move(out));
 }
 
@@ -168,20 +170,12 @@ PyObject* hybrid_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (ws.numel() < (int64_t)g_lib.hybrid_bytes((int)seqs, (int)heads)) Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
-  at::Tensor out;
-  try {
-    out = at::empty({seqs, heads, d}, q.options());
-  } catch (const std::exception&) {      // (no memory: the long way tries again and raises torch's own error)
-    Py_RETURN_NONE;
-  }
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = g_lib.hybrid_attn[v[0]](q.const_data_ptr(), float_code(q), q.stride(0), q.stride(1), (const uint8_t*)kc.const_data_ptr(), kc.stride(0), kc.stride(1),
-                               kc.stride(2), (const uint8_t*)vc.const_data_ptr(), vc.stride(0), vc.stride(1), vc.stride(2), bt.const_data_ptr(), index_code(bt),
-                               bt.stride(0), cl.const_data_ptr(), index_code(cl), (const float*)table.const_data_ptr(), out.mutable_data_ptr(), float_code(out),
-                               out.stride(0), out.stride(1), (int)seqs, (int)heads, (int)kv_heads, (int)block, std::min(kc.size(0), vc.size(0)), bt.size(1),
-                               (float)PyFloat_AS_DOUBLE(a[13]), ws.mutable_data_ptr(), (size_t)ws.numel(), stream);
-  Py_END_ALLOW_THREADS;
+  at::Tensor out = at::empty({seqs, heads, d}, q.options());
+  const int rc = without_gil(g_lib.hybrid_attn[v[0]], q.const_data_ptr(), float_code(q), q.stride(0), q.stride(1), (const uint8_t*)kc.const_data_ptr(), kc.stride(0), kc.stride(1),
+                             kc.stride(2), (const uint8_t*)vc.const_data_ptr(), vc.stride(0), vc.stride(1), vc.stride(2), bt.const_data_ptr(), index_code(bt),
+                             bt.stride(0), cl.const_data_ptr(), index_code(cl), (const float*)table.const_data_ptr(), out.mutable_data_ptr(), float_code(out),
+                             out.stride(0), out.stride(1), (int)seqs, (int)heads, (int)kv_heads, (int)block, std::min(kc.size(0), vc.size(0)), bt.size(1),
+                             (float)PyFloat_AS_DOUBLE(a[13]), ws.mutable_data_ptr(), (size_t)ws.numel(), stream);
   return rc ? status(rc) : THPVariable_Wrap(std::move(out));
 }
 
@@ -209,14 +203,11 @@ PyObject* uniform_encode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = g_lib.encode(key.const_data_ptr(), value.const_data_ptr(), float_code(key), key.size(0), (int)key.size(1), (int)key.size(2), key.stride(0), key.stride(1),
-                    slots.const_data_ptr(), index_code(slots), (const void*)(uintptr_t)v[0], (const float*)bnd.const_data_ptr(), (int)v[1],
-                    (uint8_t*)kp.mutable_data_ptr(), (uint8_t*)vp.mutable_data_ptr(), kp.stride(0), kp.stride(1), kp.stride(2),
-                    (float*)kn.mutable_data_ptr(), (float*)vn.mutable_data_ptr(), kn.stride(0), kn.stride(1), kn.stride(2), (int)v[2],
-                    blocks_of(v[3], std::min(kp.size(0), kn.size(0))), stream);
-  Py_END_ALLOW_THREADS;
+  const int rc = without_gil(g_lib.encode, key.const_data_ptr(), value.const_data_ptr(), float_code(key), key.size(0), (int)key.size(1), (int)key.size(2), key.stride(0), key.stride(1),
+                             slots.const_data_ptr(), index_code(slots), (const void*)(uintptr_t)v[0], (const float*)bnd.const_data_ptr(), (int)v[1],
+                             (uint8_t*)kp.mutable_data_ptr(), (uint8_t*)vp.mutable_data_ptr(), kp.stride(0), kp.stride(1), kp.stride(2),
+                             (float*)kn.mutable_data_ptr(), (float*)vn.mutable_data_ptr(), kn.stride(0), kn.stride(1), kn.stride(2), (int)v[2],
+                             blocks_of(v[3], std::min(kp.size(0), kn.size(0))), stream);
   return status(rc);
 }
 
@@ -234,12 +225,9 @@ PyObject* hybrid_encode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = g_lib.hybrid_encode[v[0]](key.const_data_ptr(), value.const_data_ptr(), float_code(key), key.size(0), (int)key.size(1), key.stride(0), key.stride(1),
-                                 slots.const_data_ptr(), index_code(slots), (const float*)table.const_data_ptr(), (uint8_t*)kc.mutable_data_ptr(),
-                                 (uint8_t*)vc.mutable_data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2), (int)v[3], blocks_of(v[4], kc.size(0)), stream);
-  Py_END_ALLOW_THREADS;
+  const int rc = without_gil(g_lib.hybrid_encode[v[0]], key.const_data_ptr(), value.const_data_ptr(), float_code(key), key.size(0), (int)key.size(1), key.stride(0), key.stride(1),
+                             slots.const_data_ptr(), index_code(slots), (const float*)table.const_data_ptr(), (uint8_t*)kc.mutable_data_ptr(),
+                             (uint8_t*)vc.mutable_data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2), (int)v[3], blocks_of(v[4], kc.size(0)), stream);
   return status(rc);
 }
 
@@ -272,14 +260,11 @@ PyObject* decode_blocks(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!(k.second <= w.first || w.second <= k.first)) Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = g_lib.decode_blocks((const uint8_t*)kc.const_data_ptr(), (const uint8_t*)vc.const_data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2),
-                           (const float*)kn.const_data_ptr(), (const float*)vn.const_data_ptr(), kn.stride(0), kn.stride(1), kn.stride(2), ids.const_data_ptr(),
-                           index_code(ids), ids.numel(), blocks, (int)kc.size(1), (int)kc.size(2), (int)d, (const void*)(uintptr_t)v[0],
-                           (const float*)cen.const_data_ptr(), (int)v[4], kb.mutable_data_ptr(), vb.mutable_data_ptr(), float_code(kb), kb.stride(0), kb.stride(1),
-                           kb.stride(2), stream);
-  Py_END_ALLOW_THREADS;
+  const int rc = without_gil(g_lib.decode_blocks, (const uint8_t*)kc.const_data_ptr(), (const uint8_t*)vc.const_data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2),
+                             (const float*)kn.const_data_ptr(), (const float*)vn.const_data_ptr(), kn.stride(0), kn.stride(1), kn.stride(2), ids.const_data_ptr(),
+                             index_code(ids), ids.numel(), blocks, (int)kc.size(1), (int)kc.size(2), (int)d, (const void*)(uintptr_t)v[0],
+                             (const float*)cen.const_data_ptr(), (int)v[4], kb.mutable_data_ptr(), vb.mutable_data_ptr(), float_code(kb), kb.stride(0), kb.stride(1),
+                             kb.stride(2), stream);
   return status(rc);
 }
 
@@ -300,12 +285,9 @@ PyObject* spectral_encode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = g_lib.tri_encode(keys.const_data_ptr(), values.const_data_ptr(), float_code(keys), keys.size(0), (int)v[0], (int)v[1], keys.stride(0), keys.stride(1),
-                        (int)v[2], slots.const_data_ptr(), index_code(slots), v[3], (uint8_t*)c[0]->mutable_data_ptr(), (uint8_t*)c[1]->mutable_data_ptr(),
-                        c[2]->mutable_data_ptr(), (uint8_t*)c[3]->mutable_data_ptr(), (uint8_t*)c[4]->mutable_data_ptr(), c[5]->mutable_data_ptr(), stream);
-  Py_END_ALLOW_THREADS;
+  const int rc = without_gil(g_lib.tri_encode, keys.const_data_ptr(), values.const_data_ptr(), float_code(keys), keys.size(0), (int)v[0], (int)v[1], keys.stride(0), keys.stride(1),
+                             (int)v[2], slots.const_data_ptr(), index_code(slots), v[3], (uint8_t*)c[0]->mutable_data_ptr(), (uint8_t*)c[1]->mutable_data_ptr(),
+                             c[2]->mutable_data_ptr(), (uint8_t*)c[3]->mutable_data_ptr(), (uint8_t*)c[4]->mutable_data_ptr(), c[5]->mutable_data_ptr(), stream);
   return status(rc);
 }
 
@@ -328,20 +310,12 @@ PyObject* spectral_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   void* stream;
   if (!stream_of(ts.device(), stream)) return nullptr;
-  at::Tensor out;
-  try {
-    out = at::empty({b, qh, d}, q.options().dtype(at::kFloat));
-  } catch (const std::exception&) {      // (no memory: the long way tries again and raises torch's own error)
-    Py_RETURN_NONE;
-  }
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = g_lib.tri_decode(q.const_data_ptr(), float_code(q), (const uint8_t*)c[0]->const_data_ptr(), (const uint8_t*)c[1]->const_data_ptr(),
-                        c[2]->const_data_ptr(), (const uint8_t*)c[3]->const_data_ptr(), (const uint8_t*)c[4]->const_data_ptr(), c[5]->const_data_ptr(),
-                        (const float*)theta.const_data_ptr(), nullptr, 0, bt.const_data_ptr(), index_code(bt), bt.stride(0), cl.const_data_ptr(), index_code(cl),
-                        (float*)out.mutable_data_ptr(), (int)b, c[0]->size(0), (int)c[0]->size(1), bt.size(1), (int)qh, (int)kvh, (int)d, (int)c[0]->size(3),
-                        (int)v[1], ws.mutable_data_ptr(), (size_t)ws.numel(), stream);
-  Py_END_ALLOW_THREADS;
+  at::Tensor out = at::empty({b, qh, d}, q.options().dtype(at::kFloat));
+  const int rc = without_gil(g_lib.tri_decode, q.const_data_ptr(), float_code(q), (const uint8_t*)c[0]->const_data_ptr(), (const uint8_t*)c[1]->const_data_ptr(),
+                             c[2]->const_data_ptr(), (const uint8_t*)c[3]->const_data_ptr(), (const uint8_t*)c[4]->const_data_ptr(), c[5]->const_data_ptr(),
+                             (const float*)theta.const_data_ptr(), nullptr, 0, bt.const_data_ptr(), index_code(bt), bt.stride(0), cl.const_data_ptr(), index_code(cl),
+                             (float*)out.mutable_data_ptr(), (int)b, c[0]->size(0), (int)c[0]->size(1), bt.size(1), (int)qh, (int)kvh, (int)d, (int)c[0]->size(3),
+                             (int)v[1], ws.mutable_data_ptr(), (size_t)ws.numel(), stream);
   if (rc == AKV_ERR_UNSUPPORTED) Py_RETURN_NONE;
   return rc ? status(rc) : THPVariable_Wrap(std::move(out));
 }
@@ -364,15 +338,26 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
+// an exception of torch (no memory for an output, a tensor without storage): the long way tries again and raises torch's own error
+template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
+PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) noexcept {
+  try {
+    return F(self, a, n);
+  } catch (const std::exception&) {
+    if (PyErr_Occurred()) return nullptr;
+    Py_RETURN_NONE;
+  }
+}
+
 PyMethodDef kMethods[] = {
     {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
-    {"uniform_attention", (PyCFunction)(void (*)(void))uniform_attention, METH_FASTCALL, nullptr},
-    {"hybrid_attention", (PyCFunction)(void (*)(void))hybrid_attention, METH_FASTCALL, nullptr},
-    {"uniform_encode", (PyCFunction)(void (*)(void))uniform_encode, METH_FASTCALL, nullptr},
-    {"hybrid_encode", (PyCFunction)(void (*)(void))hybrid_encode, METH_FASTCALL, nullptr},
-    {"decode_blocks", (PyCFunction)(void (*)(void))decode_blocks, METH_FASTCALL, nullptr},
-    {"spectral_encode", (PyCFunction)(void (*)(void))spectral_encode, METH_FASTCALL, nullptr},
-    {"spectral_attention", (PyCFunction)(void (*)(void))spectral_attention, METH_FASTCALL, nullptr},
+    {"uniform_attention", (PyCFunction)(void (*)(void))guarded<uniform_attention>, METH_FASTCALL, nullptr},
+    {"hybrid_attention", (PyCFunction)(void (*)(void))guarded<hybrid_attention>, METH_FASTCALL, nullptr},
+    {"uniform_encode", (PyCFunction)(void (*)(void))guarded<uniform_encode>, METH_FASTCALL, nullptr},
+    {"hybrid_encode", (PyCFunction)(void (*)(void))guarded<hybrid_encode>, METH_FASTCALL, nullptr},
+    {"decode_blocks", (PyCFunction)(void (*)(void))guarded<decode_blocks>, METH_FASTCALL, nullptr},
+    {"spectral_encode", (PyCFunction)(void (*)(void))guarded<spectral_encode>, METH_FASTCALL, nullptr},
+    {"spectral_attention", (PyCFunction)(void (*)(void))guarded<spectral_attention>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 
