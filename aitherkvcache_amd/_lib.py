@@ -8,6 +8,9 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import re
+import sys
+import warnings
 from typing import Optional
 
 import torch
@@ -128,30 +131,62 @@ def lib() -> C.CDLL:
             raise RuntimeError(
                 f"{LIB_PATH} not found: the HIP extension is not built and there is no CPU "
                 "fallback. Run `make -C aitherkvcache_amd/csrc`.")
-        from . import _binding  # noqa: F401 -- first: the library's thread-local block is to be the newest of the process
+        binding = _load_binding()     # first: the library's thread-local block is to be the newest of the process
         handle = C.CDLL(LIB_PATH)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-        _bind(handle)
+        _bind(handle, binding)
         handle.akv_last_error()       # the thread's thread-local block of the library, touched: see akv_touch_thread
         _lib = handle
     return _lib
 
 
-def _bind(handle: C.CDLL) -> None:
+class _NoBinding:
+    """In the binding's place where there is none: every call goes the long way."""
+
+    def __getattr__(self, name):
+        return _take_nothing
+
+
+def _take_nothing(*args):
+    return None
+
+
+def _load_binding():
+    """The extension module, or None (and a warning) where it is missing or was built for another Python or torch."""
+    here = (re.match(r"[\d.]*\d", torch.__version__).group(), "%d.%d" % sys.version_info[:2])
+    try:
+        from . import _binding
+        built = getattr(_binding, "BUILT_FOR", None)
+        if built != here:
+            raise ImportError(f"built for torch and Python {built}, not {here}")
+        return _binding
+    except ImportError as e:
+        warnings.warn(f"the binding of the hot calls cannot be loaded ({e}): they take longer on the host. "
+                      "Run `make -C aitherkvcache_amd/csrc`.", RuntimeWarning, stacklevel=3)
+        return None
+
+
+def _bind(handle: C.CDLL, binding) -> None:
     """Hand the functions of a loaded library to the binding of the hot calls."""
     global _calls
-    from . import _binding
-    _binding.bind(torch._C._cuda_getCurrentRawStream, *(C.cast(getattr(handle, n), C.c_void_p).value for n in _BOUND))
-    _calls = _binding
+    raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if binding is None or raw_stream is None:
+        _calls = _NoBinding()
+        return
+    binding.bind(raw_stream, *(C.cast(getattr(handle, n), C.c_void_p).value for n in _BOUND))
+    _calls = binding
 
 
 def calls():
     """The binding: functions that take tensors and return a result, an akv_status, or None for a call that has to go the long
-    way (csrc/akv_binding.cpp says when)."""
+    way (csrc/akv_binding.cpp says when).  Without a built library that is every call: the long way checks the call first and
+    then says what is missing."""
     if _calls is None:
+        if not available():
+            return _NoBinding()
         lib()
     return _calls
 

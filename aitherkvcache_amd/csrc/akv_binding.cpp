@@ -13,6 +13,7 @@
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "../../include/aitherkv.h"
 
@@ -363,4 +364,14 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_binding", nullptr, -1, kMethods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__binding(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__binding(void) {
+  PyObject* m = PyModule_Create(&kModule);
+  // (what it was compiled against: _lib.py loads no other)
+  PyObject* built = Py_BuildValue("(ss)", TORCH_VERSION, Py_STRINGIFY(PY_MAJOR_VERSION) "." Py_STRINGIFY(PY_MINOR_VERSION));
+  if (!m || !built || PyModule_AddObject(m, "BUILT_FOR", built) < 0) {
+    Py_XDECREF(built);
+    Py_XDECREF(m);
+    return nullptr;
+  }
+  return m;
+}
