@@ -11,7 +11,7 @@
 //   rows     requested a chunk ahead straight into LDS (16 rows an instruction); nothing passes through registers, and an
 //            instruction touches every row once.  The 16-byte pieces of rows are permuted so that the sixteen lanes that read
 //            the same place of sixteen rows meet different banks.
-//   scores   v_mfma_i32_16x16x64_i8, 16 tokens a tile.  A level is an integer of two signed bytes, looked up four codes at
+//   scores   v_mfma_i32_16x16x64_i8, 16 tokens a tile.  A level is an integer of three signed bytes (the query's form), looked up four codes at
 //            a time by byte permutes from registers; signs are +-64, their bits as they lie (no look-up).  The query is three
 //            signed bytes (23 bits and a sign, one scale a head), in the columns 4 d + head of digit d.  Sums are exact.
 //   softmax  on packed scores: the lanes of a row add the digits up so that lane 4 k + c ends up with two of the eight
@@ -23,7 +23,8 @@
 // What bounds it: the issue of vector instructions, 610 a chunk and kv head (vector unit 78 % of the cycles, matrix cores 15 %,
 // LDS 41 %).  The kernel before this one (four score and four value wavefronts that handed chunks over through polled counters,
 // codes spread to nibbles and looked up in LDS) issued some 1,300 at two wavefronts a SIMD.  A decode step, this | that, bfloat16:
-// 64 sequences of 4,000 to 8,192 tokens, 32 heads on 8: 160 | 211 us; 256 of 64 to 512: 82 | 111; 64 of 300: 45 | 54; 4 of 300:
+// 64 sequences of 4,000 to 8,192 tokens, 32 heads on 8: 167 | 211 us (160 with levels of keys in two bytes, off by 1e-6 of the
+// largest: float32 outputs whose scores reach some hundreds had twice the error); 256 of 64 to 512: 82 | 111; 64 of 300: 45 | 54; 4 of 300:
 // 29 | 38; 32 of 1,000 to 9,000 with 64 heads on 8: 130 | 188, 8 on 1: 42 | 61.  Head counts that are no multiple of four a kv
 // head (levels of float32's accuracy, see hw35) | the vector kernel: 28 on 4: 107 | 570; 16 on 16: 166 | 238.
 // tq25 rows | the vector kernel (tables of partial products in LDS): 64 of 4,000 to 8,192, 32 heads on 8: 160 | 335; 256 of 64 to
@@ -57,8 +58,7 @@ typedef __attribute__((address_space(3))) hw_int4 hw_lds_i128;
 #define HW_TINY 90             // value factors count as at least 2^-HW_TINY in the running maximum
 #define HW_WIN 32              // chunks served by one window of 64 block ids
 #define HW_QMAX 8290000.f      // largest query integer: 126.5 * 2^16, its top byte stays in range
-#define HW_LEVELS 32639        // largest level integer: 127 * 2^8 + 127
-#define HW_SEARCH 65536        // candidates for the unit of the levels
+#define HW_SEARCH 65536        // candidates for the factor of the value levels
 // LDS: per wavefront two chunk buffers | per wavefront factors of 32 keys (16 bytes each), of 32 values and their exponents (32) |
 // per wavefront (max, sum) of four heads | per wavefront its query operand (in registers it would make the loop spill)
 #define HW_BUF 8192u
@@ -71,22 +71,18 @@ typedef __attribute__((address_space(3))) hw_int4 hw_lds_i128;
 static_assert(HW_LDS <= 52 * 1024, "three workgroups a CU, whatever the granularity");
 // words of the table block kept in the workspace.  Tag and mark lie where the other kernels' table blocks have them, so that
 // whichever kernel used the workspace last is known.
-#define HW_W_KA0 0             // bytes of the 3-bit levels: high 0..3, 4..7, low 0..3, 4..7
-#define HW_W_KA1 4             // of the 2-bit levels: high, low
-#define HW_W_VA0 6             // bytes of float16(alpha c): low 0..3, 4..7, high 0..3, 4..7
-#define HW_W_VA1 10            // low, high
-#define HW_W_UNIT 12           // units of the two level sets
-#define HW_W_ALPHA 14          // alpha of the two value sets
-// the same for calls of float32's accuracy: three digits, float16 remainders of the value levels
-#define HW_W_KP0 16            // top, middle, low digit of the 3-bit levels, two words each
-#define HW_W_KP1 22            // of the 2-bit levels
-#define HW_W_VP0 25            // remainders, as HW_W_VA0
-#define HW_W_VP1 29
-#define HW_W_UNITP 31
+#define HW_W_KA0 0             // bytes of the 3-bit levels, three digits, top first: levels 0..3, 4..7 of each
+#define HW_W_KA1 6             // of the 2-bit levels
+#define HW_W_VA0 9             // bytes of float16(alpha c): low 0..3, 4..7, high 0..3, 4..7
+#define HW_W_VA1 13            // low, high
+#define HW_W_VP0 15            // their remainders, likewise
+#define HW_W_VP1 19
+#define HW_W_UNIT 21           // units of the two level sets
+#define HW_W_ALPHA 23          // alpha of the two value sets
+#define HW_W_DELTA 25          // tq25: half the distance of the two levels of a 1-bit code, and their middle
+#define HW_W_MIDDLE 26
 #define HW_W_TAG 768
 #define HW_W_MARK 784
-#define HW_W_DELTA 33          // tq25: half the distance of the two levels of a 1-bit code, and their middle
-#define HW_W_MIDDLE 34
 #define HW_MARK 0x48570000u    // plus the format
 #define HW_VALUES 2048u        // of a chunk buffer: the value rows
 
@@ -155,11 +151,12 @@ __device__ __forceinline__ int hw35_kcoord(int part, int g, int r, int b) {
   return 8 * (2 * g + (b & 1)) + r + 4 * (b >> 1);
 }
 
-// P: for float32's accuracy -- levels of keys in three digits, of values in two float16 terms
+// P: for float32's accuracy -- levels of values in two float16 terms, not one
 template <bool P> struct hw35 {
   static constexpr uint32_t MARK = HW_MARK + 35;
+  static constexpr int PER_SIMD = P ? 2 : 3; // wavefronts that the registers admit
   static constexpr float KAPPA = (float)(1.2533141373155001 / 64.0);         // sqrt(pi/2) / 64
-  static constexpr int KD = P ? 3 : 2;       // digits of a level
+  static constexpr int KD = 3;               // digits of a level of keys
   static constexpr int TILE = 1024;          // bytes of sixteen rows in LDS
   static constexpr int NT = 18;              // value tiles: A0 of bytes 0..15 (3), of 16..23 (3), A1 (4), B0 (4), B1 (4)
   // lane (n, g) of a score tile, row n: addresses of its pieces
@@ -185,9 +182,9 @@ template <bool P> struct hw35 {
     const uint32_t r = col >> 1, row = 4u * g + (r & 3u);
     tr = buf + HW_VALUES + (r >> 2) * TILE + row * 64u + (col & 1u) * 8u + (g << 4);
 #pragma unroll
-    for (int i = 0; i < 2 * KD; ++i) ka0[i] = lut[(P ? HW_W_KP0 : HW_W_KA0) + i];
+    for (int i = 0; i < 2 * KD; ++i) ka0[i] = lut[HW_W_KA0 + i];
 #pragma unroll
-    for (int i = 0; i < KD; ++i) ka1[i] = lut[(P ? HW_W_KP1 : HW_W_KA1) + i];
+    for (int i = 0; i < KD; ++i) ka1[i] = lut[HW_W_KA1 + i];
 #pragma unroll
     for (int i = 0; i < (P ? 8 : 4); ++i) va0[i] = lut[i < 4 ? HW_W_VA0 + i : HW_W_VP0 + i - 4];
 #pragma unroll
@@ -294,8 +291,7 @@ template <bool P> struct hw35 {
         sg[x] = __builtin_amdgcn_mfma_i32_16x16x64_i8(v, q(1 + 2 * x), zero, 0, 0, 0);
       }
       auto whole = [&](const hw_int4 (&d)[KD], int i) __attribute__((always_inline)) {
-        if constexpr (P) return fmaf((float)d[0][i], 65536.f, (float)((d[1][i] << 8) + d[2][i]));
-        else return (float)((d[0][i] << 8) + d[1][i]);
+        return fmaf((float)d[0][i], 65536.f, (float)((d[1][i] << 8) + d[2][i]));
       };
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -417,8 +413,7 @@ template <bool P> struct hw35 {
   // constants of the factors: (n0, n0 r0, n1, n1 r1) times these on the score side
   static __device__ __forceinline__ hw_float4 kscale(const uint32_t* lut) {
     const float sign = -KAPPA / 64.f;
-    const int u = P ? HW_W_UNITP : HW_W_UNIT;
-    return (hw_float4){__uint_as_float(lut[u]), sign, __uint_as_float(lut[u + 1]), sign};
+    return (hw_float4){__uint_as_float(lut[HW_W_UNIT]), sign, __uint_as_float(lut[HW_W_UNIT + 1]), sign};
   }
   // row i of the lane's rows of the finished tiles
   static __device__ __forceinline__ void finish(const uint32_t* lut, hw_float4 (&o)[NT], int i, float (&v)[NT]) {
@@ -453,7 +448,7 @@ template <bool P> struct hw35 {
 // middle is a constant of the head, and the sum of the weights comes out of the value product in a row nobody else has.
 struct hw25 {
   static constexpr uint32_t MARK = HW_MARK + 25;
-  static constexpr int KD = 2;               // (only says how many wavefronts the registers admit)
+  static constexpr int PER_SIMD = 3;
   static constexpr int TILE = 768;
   static constexpr int NT = 20;              // value tiles: A0 (2), B0 (2), A1 (8), B1 (8)
   static constexpr int SUM_B = 128;          // sums: A0 0..31, A1 32..127, B0 and B1 from 128 on in the same order
@@ -471,7 +466,7 @@ struct hw25 {
     const uint32_t r = col >> 1, row = 4u * g + (r & 3u);
     tr = buf + HW_VALUES + (r >> 2) * TILE + row * 48u + (col & 1u) * 8u;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) ka[i] = lut[HW_W_KP1 + i];
+    for (int i = 0; i < 3; ++i) ka[i] = lut[HW_W_KA1 + i];
 #pragma unroll
     for (int i = 0; i < 4; ++i) va[i] = lut[i < 2 ? HW_W_VA1 + i : HW_W_VP1 + i - 2];
     delta = __uint_as_float(lut[HW_W_DELTA]);
@@ -630,7 +625,7 @@ struct hw25 {
     }
   }
   static __device__ __forceinline__ hw_float4 kscale(const uint32_t* lut) {
-    return (hw_float4){__uint_as_float(lut[HW_W_UNITP + 1]), -kH25Kappa0 / 64.f, -1.f / 64.f, -kH25Kappa1 / 64.f};
+    return (hw_float4){__uint_as_float(lut[HW_W_UNIT + 1]), -kH25Kappa0 / 64.f, -1.f / 64.f, -kH25Kappa1 / 64.f};
   }
   static __device__ __forceinline__ void finish(const uint32_t* lut, hw_float4 (&o)[NT], int i, float (&v)[NT]) {
     const float ia = 1.f / __uint_as_float(lut[HW_W_ALPHA + 1]), dl = __uint_as_float(lut[HW_W_DELTA]), md = __uint_as_float(lut[HW_W_MIDDLE]);
@@ -675,7 +670,7 @@ struct hw25 {
 // ----------------------------------------------------------------------------------
 // N: bytes of a request, 16 where rows allow it, else 4
 template <class F, int N>
-__global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_kernel(hw_args a) {
+__global__ __launch_bounds__(HW_W * 64, F::PER_SIMD) void akv_attn_hyb_kernel(hw_args a) {
   // The dynamic LDS block is the kernel's only LDS object: its offsets are LDS addresses.
   constexpr int NT = F::NT;
   const int lane = threadIdx.x & 63;
@@ -929,14 +924,13 @@ __global__ __launch_bounds__(HW_W * 64, F::KD == 2 ? 3 : 2) void akv_attn_hyb_ke
 // ----------------------------------------------------------------------------------
 // tables, built by a workgroup of 256 threads
 // ----------------------------------------------------------------------------------
-// byte `byte_of` of four levels, table[0..3], a word: of their integers in units of `unit` (kd digits, top first), or of the
+// byte `byte_of` of four levels, table[0..3], a word: of their integers in units of `unit` (three digits, top first), or of the
 // float16 form of alpha times a level (low byte first), rounding or remainder
-__device__ __forceinline__ uint32_t hw_key_bytes(const float* table, float unit, int kd, int byte_of) {
+__device__ __forceinline__ uint32_t hw_key_bytes(const float* table, float unit, int byte_of) {
   uint32_t word = 0;
   for (int v = 0; v < 4; ++v) {
-    const int n = (int)rintf(table[v] / unit), d0 = ((n + 128) & 255) - 128, n1 = (n - d0) >> 8;
-    const int d1 = kd == 3 ? ((n1 + 128) & 255) - 128 : n1, d2 = (n1 - d1) >> 8;
-    word |= ((uint32_t)(byte_of == kd - 1 ? d0 : byte_of == kd - 2 ? d1 : d2) & 255u) << (8 * v);
+    const int n = (int)rintf(table[v] / unit), d0 = ((n + 128) & 255) - 128, n1 = (n - d0) >> 8, d1 = ((n1 + 128) & 255) - 128;
+    word |= ((uint32_t)(byte_of == 2 ? d0 : byte_of == 1 ? d1 : (n1 - d1) >> 8) & 255u) << (8 * v);
   }
   return word;
 }
@@ -962,28 +956,24 @@ __device__ __forceinline__ float hw_base(float top) {
 
 template <bool P> __device__ void hw35<P>::tables(const float* table, uint32_t* lut) {
   __shared__ float best_err[256], best[256];
-  __shared__ float chosen[4], fine[2];
+  __shared__ float unit[2], alpha[2];
   const int tid = threadIdx.x;
-  // A free factor per set of levels makes them nearly exact: sets 0, 1 the unit of the 3- and 2-bit integers of two digits,
-  // sets 2, 3 alpha of fp16(alpha c), from HW_SEARCH candidates within a factor of two the one with the smallest largest error
-  // (relative to the largest level, and to each level).  16-bit integers then carry the levels to 1e-6, not 1.5e-5.  The
-  // largest alpha c lies in [2^9, 2^11), so that no remainder is a subnormal.
+  // alpha of float16(alpha c): a free factor makes the levels nearly exact, of HW_SEARCH candidates within a factor of two the one
+  // with the smallest largest error (relative to each level).  The largest alpha c lies in [2^9, 2^11), so that no remainder is a
+  // subnormal.
 #pragma unroll 1
-  for (int set = 0; set < 4; ++set) {
-    const int v0 = set & 1 ? 8 : 0, v1 = set & 1 ? 12 : 8;
-    float top = 0.f;
-    for (int v = v0; v < v1; ++v) top = fmaxf(top, fabsf(table[HYB_CEN0 + v]));
-    const float base = top > 0.f ? __uint_as_float((min(max(254u + 9u - ((__float_as_uint(top) >> 23) & 0xffu), 1u), 253u)) << 23) : 1.f;
+  for (int set = 0; set < 2; ++set) {
+    const float* lv = table + HYB_CEN0 + 8 * set;
+    const int n = set ? 4 : 8;
+    const float top = hw_top(lv, n), base = hw_base(top);
     float berr = INFINITY, bval = 1.f;
 #pragma unroll 1
     for (int k = 0; k < HW_SEARCH / 256; ++k) {
       const float al = 1.f + (float)(tid * (HW_SEARCH / 256) + k) / (float)HW_SEARCH;
-      const float inv = (float)HW_LEVELS * 0.5f * al / top;        // levels an integer, at most HW_LEVELS
       float worst = 0.f;
-      for (int v = v0; v < v1; ++v) {
-        const float x = table[HYB_CEN0 + v] * (set < 2 ? inv : al * base);
-        const float e = set < 2 ? fabsf(rintf(x) - x) / al : x != 0.f ? fabsf(__half2float(__float2half_rn(x)) - x) / fabsf(x) : 0.f;
-        worst = fmaxf(worst, e);
+      for (int v = 0; v < n; ++v) {
+        const float x = lv[v] * (al * base);
+        worst = fmaxf(worst, x != 0.f ? fabsf(__half2float(__float2half_rn(x)) - x) / fabsf(x) : 0.f);
       }
       if (worst < berr) { berr = worst; bval = al; }
     }
@@ -992,39 +982,25 @@ template <bool P> __device__ void hw35<P>::tables(const float* table, uint32_t* 
     best[tid] = bval;
     __syncthreads();
     if (tid == 0) {
-      int at = 0;
       for (int t = 1; t < 256; ++t)
-        if (best_err[t] < best_err[at]) at = t;
-      chosen[set] = set < 2 ? (top > 0.f ? top / ((float)HW_LEVELS * 0.5f * best[at]) : 1.f) : best[at] * base;
-      if (set < 2) fine[set] = top > 0.f ? top * (1.f / HW_QMAX) : 1.f;
+        if (best_err[t] < berr) { berr = best_err[t]; bval = best[t]; }
+      alpha[set] = bval * base;
+      unit[set] = top > 0.f ? top * (1.f / HW_QMAX) : 1.f;
     }
-    __syncthreads();
   }
-  if (tid < 4) lut[HW_W_UNIT + tid] = __float_as_uint(chosen[tid]);      // (units, then alphas)
-  if (tid < 2) lut[HW_W_UNITP + tid] = __float_as_uint(fine[tid]);
-  if (tid < HW_W_UNITP && (tid < HW_W_UNIT || tid >= HW_W_KP0)) {
-    // thread = a word of the bytes of four levels: which set, which levels, which byte of what
-    const bool p = tid >= HW_W_KP0, vals = p ? tid >= HW_W_VP0 : tid >= HW_W_VA0;
-    const int i = tid - (p ? (vals ? HW_W_VP0 : HW_W_KP0) : (vals ? HW_W_VA0 : HW_W_KA0));
-    const int kd = vals ? 2 : p ? 3 : 2, set = i < 2 * kd ? 0 : 1;
-    const int v0 = set ? 8 : 4 * (i & 1), byte_of = set ? i - 2 * kd : i >> 1;       // keys: top digit first, values: low byte first
-    uint32_t word = 0;
-    for (int v = 0; v < 4; ++v) {
-      const float level = table[HYB_CEN0 + v0 + v];
-      uint32_t byte;
-      if (!vals) {
-        const int n = (int)rintf(level / (p ? fine[set] : chosen[set])), d0 = ((n + 128) & 255) - 128, n1 = (n - d0) >> 8;
-        const int d1 = p ? ((n1 + 128) & 255) - 128 : n1, d2 = (n1 - d1) >> 8;
-        byte = (uint32_t)(byte_of == kd - 1 ? d0 : byte_of == kd - 2 ? d1 : d2) & 255u;
-      } else {
-        const float x = chosen[2 + set] * level;
-        const __half hi = __float2half_rn(x);
-        const uint32_t bits = __half_as_ushort(p ? __float2half_rn(x - __half2float(hi)) : hi);
-        byte = byte_of == 0 ? bits & 255u : bits >> 8;
-      }
-      word |= byte << (8 * v);
-    }
-    lut[tid] = word;
+  __syncthreads();
+  if (tid < 2) {
+    lut[HW_W_UNIT + tid] = __float_as_uint(unit[tid]);
+    lut[HW_W_ALPHA + tid] = __float_as_uint(alpha[tid]);
+  }
+  // thread = a word of the bytes of four levels
+  const float *c0 = table + HYB_CEN0, *c1 = c0 + 8;
+  if (tid < HW_W_KA1) lut[tid] = hw_key_bytes(c0 + 4 * (tid & 1), unit[0], tid >> 1);
+  else if (tid < HW_W_VA0) lut[tid] = hw_key_bytes(c1, unit[1], tid - HW_W_KA1);
+  else if (tid < HW_W_UNIT) {
+    const bool remainder = tid >= HW_W_VP0;
+    const int i = tid - (remainder ? HW_W_VP0 : HW_W_VA0);
+    lut[tid] = i < 4 ? hw_value_bytes(c0 + 4 * (i & 1), alpha[0], remainder, i >> 1) : hw_value_bytes(c1, alpha[1], remainder, i - 4);
   }
 }
 
@@ -1033,11 +1009,11 @@ __device__ void hw25::tables(const float* table, uint32_t* lut) {
   const float* lv = table + H25_CEN0;
   const float top = hw_top(lv, 4), alpha = hw_base(top), unit = top > 0.f ? top * (1.f / HW_QMAX) : 1.f;
   const float c0 = table[H25_CEN1], c1 = table[H25_CEN1 + 1];
-  if (tid < 3) lut[HW_W_KP1 + tid] = hw_key_bytes(lv, unit, 3, tid);
+  if (tid < 3) lut[HW_W_KA1 + tid] = hw_key_bytes(lv, unit, tid);
   if (tid < 2) lut[HW_W_VA1 + tid] = hw_value_bytes(lv, alpha, false, tid);
   if (tid < 2) lut[HW_W_VP1 + tid] = hw_value_bytes(lv, alpha, true, tid);
   if (tid == 0) {
-    lut[HW_W_UNITP + 1] = __float_as_uint(unit);
+    lut[HW_W_UNIT + 1] = __float_as_uint(unit);
     lut[HW_W_ALPHA + 1] = __float_as_uint(alpha);
     lut[HW_W_DELTA] = __float_as_uint(0.5f * (c1 - c0));
     lut[HW_W_MIDDLE] = __float_as_uint(0.5f * (c1 + c0));
@@ -1254,7 +1230,7 @@ int akv_attn_hyb_run(int format, const void* query, int q_dtype, int64_t qs_seq,
     return hw_run<hw25>(query, q_dtype, qs_seq, qs_head, table, scale, a, ws, out, out_dtype, os_seq, os_head, stream,
                         [&](int grid) { return hw_launch<hw25, 4>(a, grid, stream); });
   const uint64_t all = (uint64_t)(uintptr_t)a.kc | (uint64_t)(uintptr_t)a.vc | a.kps_blk | a.kps_pos | a.kps_head | a.vps_blk | a.vps_pos | a.vps_head;
-  // groups of four query heads: the accuracy that the float16 levels of values leave; other counts: float32's, which they always had
+  // groups of four query heads: the accuracy that one float16 a level of values leaves; other counts: float32's, which they always had
   const bool wide = (all & 15) == 0, exact = a.gqa % 4 != 0;
   return hw_run<hw35<false>>(query, q_dtype, qs_seq, qs_head, table, scale, a, ws, out, out_dtype, os_seq, os_head, stream, [&](int grid) {
     return exact ? (wide ? hw_launch<hw35<true>, 16>(a, grid, stream) : hw_launch<hw35<true>, 4>(a, grid, stream))

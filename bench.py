@@ -414,7 +414,7 @@ def encode_sweep(torch, akv, L, tq, dev, gen):
 
 
 DECODE_DTYPE = "fp16 hi+lo MFMA operands (keys and queries carry 22 bits, values 11), f32 accumulate and softmax"
-HYBRID_DTYPE = "int8-digit MFMA operands for scores (levels 16 bits, queries 24), fp16 levels and hi+lo weights for values, f32 softmax and sums"
+HYBRID_DTYPE = "int8-digit MFMA operands for scores (levels and queries 24 bits), fp16 levels and hi+lo weights for values, f32 softmax and sums"
 
 
 def traffic_fields(workload):

@@ -138,3 +138,19 @@ def test_one_bit_levels_that_are_not_symmetric(dev, qh, kvh):
     K, V = (h.decode(r.contiguous()).double().cpu().reshape(-1, kvh, 128)[:120] for r in rows)
     ref = attend(q[0].double().cpu(), K, V)
     assert (out[0] - ref).norm() <= EXACT * ref.norm()
+
+
+@pytest.mark.parametrize("qh,kvh", [(8, 2), (8, 1), (6, 2)])
+def test_key_levels_have_more_than_sixteen_bits(dev, qh, kvh):
+    """tq35 with levels that one float16 holds, so that values are exact, seven of them far below the eighth: as multiples of 2^-15
+    of the largest they were off by up to 1e-4 of themselves, and outputs by 1.5e-5."""
+    rng, h, rows = make(dev, "tq35", kvh, 8, 16, 64, 11)
+    levels = [-0.25, -0.151, -0.0717, -0.0213, 0.0127, 0.0611, 0.1423, 4.2, -1.41, -0.4527, 0.4318, 1.623]
+    h.kernel_table[256:268] = (0.1 * torch.tensor(levels, device=dev)).half().float()
+    q = torch.from_numpy((2 * rng.standard_normal((1, qh, 128))).astype(np.float32)).to(dev)
+    out = akv.HybridPagedAttention(h, qh).forward(q, rows[0], rows[1], torch.arange(8, dtype=torch.int32, device=dev)[None],
+                                                  torch.tensor([128], dtype=torch.int32, device=dev)).double().cpu()
+    K, V = (h.decode(r.contiguous()).double().cpu().reshape(-1, kvh, 128) for r in rows)
+    ref = attend(q[0].double().cpu(), K, V)
+    print(f"[key levels] {qh} on {kvh}: {float((out[0] - ref).norm() / ref.norm()):.2e}", flush=True)
+    assert (out[0] - ref).norm() <= EXACT * ref.norm(), float((out[0] - ref).norm() / ref.norm())
