@@ -153,7 +153,7 @@ __device__ __forceinline__ int hw35_kcoord(int part, int g, int r, int b) {
 
 // P: for float32's accuracy -- levels of values in two float16 terms, not one
 template <bool P> struct hw35 {
-  static constexpr uint32_t MARK = HW_MARK + 35;
+  static constexpr uint32_t MARK = HW_MARK + (P ? 36 : 35);      // (the value levels of the two have factors of their own)
   static constexpr int PER_SIMD = P ? 2 : 3; // wavefronts that the registers admit
   static constexpr float KAPPA = (float)(1.2533141373155001 / 64.0);         // sqrt(pi/2) / 64
   static constexpr int KD = 3;               // digits of a level of keys
@@ -954,39 +954,81 @@ __device__ __forceinline__ float hw_base(float top) {
   return top > 0.f ? __uint_as_float((min(max(254u + 9u - ((__float_as_uint(top) >> 23) & 0xffu), 1u), 253u)) << 23) : 1.f;
 }
 
+// Factor of N value levels whose float16 forms are used without remainders: a free factor makes them nearly exact.  Of HW_SEARCH
+// candidates within a factor of two, a quarter here for each wavefront of the workgroup, the one with the smallest largest error
+// relative to each level, and that error.  Four candidates a lane side by side; levels beyond the fourth only where one of the
+// wavefront's 256 still is better than its best so far.  (The first call with a new workspace waits for this: 34 us more
+// than a later one.  658 with a division a level, one candidate at a time, and units of two sets of key levels searched for
+// too; 187 on the kernel before this one.)
+template <int N> __device__ __forceinline__ float hw_search(const float* table, float base, float& factor) {
+  float c[N], rel[N];
+#pragma unroll
+  for (int v = 0; v < N; ++v) {
+    c[v] = table[v] * base;
+    rel[v] = c[v] != 0.f ? 1.f / fabsf(c[v]) : 0.f;
+  }
+  float least = INFINITY, mine = INFINITY, at = 1.f;      // of the wavefront, of the lane and where
+#pragma unroll 1
+  for (int k = 0; k < HW_SEARCH / 256; k += 4) {
+    float al[4], worst[4] = {0.f, 0.f, 0.f, 0.f};         // (errors times al)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) al[i] = 1.f + (float)((int)threadIdx.x * (HW_SEARCH / 256) + k + i) * (1.f / HW_SEARCH);
+    auto levels = [&](int v0, int v1) __attribute__((always_inline)) {
+#pragma unroll
+      for (int v = v0; v < v1; ++v)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float x = c[v] * al[i];
+          worst[i] = fmaxf(worst[i], fabsf(__half2float(__float2half_rn(x)) - x) * rel[v]);
+        }
+    };
+    auto better = [&]() __attribute__((always_inline)) {
+      bool any = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) any = any || worst[i] < least * al[i];
+      return __builtin_amdgcn_ballot_w64(any) != 0;
+    };
+    levels(0, 4);
+    if (!better()) continue;
+    if constexpr (N > 4) {
+      levels(4, N);
+      if (!better()) continue;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (worst[i] < mine * al[i]) { mine = worst[i] / al[i]; at = al[i]; }
+    least = -akv_wave_max(-mine);
+  }
+  const uint64_t who = __builtin_amdgcn_ballot_w64(mine == least);
+  factor = who ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(at), __builtin_ctzll(who))) : 1.f;
+  return least;
+}
+
 template <bool P> __device__ void hw35<P>::tables(const float* table, uint32_t* lut) {
-  __shared__ float best_err[256], best[256];
+  __shared__ float err[2][4], at[2][4];
   __shared__ float unit[2], alpha[2];
   const int tid = threadIdx.x;
-  // alpha of float16(alpha c): a free factor makes the levels nearly exact, of HW_SEARCH candidates within a factor of two the one
-  // with the smallest largest error (relative to each level).  The largest alpha c lies in [2^9, 2^11), so that no remainder is a
-  // subnormal.
-#pragma unroll 1
-  for (int set = 0; set < 2; ++set) {
-    const float* lv = table + HYB_CEN0 + 8 * set;
-    const int n = set ? 4 : 8;
-    const float top = hw_top(lv, n), base = hw_base(top);
-    float berr = INFINITY, bval = 1.f;
-#pragma unroll 1
-    for (int k = 0; k < HW_SEARCH / 256; ++k) {
-      const float al = 1.f + (float)(tid * (HW_SEARCH / 256) + k) / (float)HW_SEARCH;
-      float worst = 0.f;
-      for (int v = 0; v < n; ++v) {
-        const float x = lv[v] * (al * base);
-        worst = fmaxf(worst, x != 0.f ? fabsf(__half2float(__float2half_rn(x)) - x) / fabsf(x) : 0.f);
-      }
-      if (worst < berr) { berr = worst; bval = al; }
+  const float *c0 = table + HYB_CEN0, *c1 = c0 + 8;
+  const float top[2] = {hw_top(c0, 8), hw_top(c1, 4)};
+  // alpha of float16(alpha c): the largest alpha c lies in [2^9, 2^11), so that no remainder is a subnormal
+  if constexpr (!P) {
+    float a0, a1;
+    const float e0 = hw_search<8>(c0, hw_base(top[0]), a0), e1 = hw_search<4>(c1, hw_base(top[1]), a1);
+    if ((tid & 63) == 0) {
+      err[0][tid >> 6] = e0;
+      at[0][tid >> 6] = a0;
+      err[1][tid >> 6] = e1;
+      at[1][tid >> 6] = a1;
     }
     __syncthreads();
-    best_err[tid] = berr;
-    best[tid] = bval;
-    __syncthreads();
-    if (tid == 0) {
-      for (int t = 1; t < 256; ++t)
-        if (best_err[t] < berr) { berr = best_err[t]; bval = best[t]; }
-      alpha[set] = bval * base;
-      unit[set] = top > 0.f ? top * (1.f / HW_QMAX) : 1.f;
-    }
+  }
+  if (tid < 2) {
+    float al = 1.f, least = INFINITY;
+    if constexpr (!P)
+      for (int w = 0; w < 4; ++w)
+        if (err[tid][w] < least) { least = err[tid][w]; al = at[tid][w]; }
+    alpha[tid] = al * hw_base(top[tid]);
+    unit[tid] = top[tid] > 0.f ? top[tid] * (1.f / HW_QMAX) : 1.f;
   }
   __syncthreads();
   if (tid < 2) {
@@ -994,7 +1036,6 @@ template <bool P> __device__ void hw35<P>::tables(const float* table, uint32_t* 
     lut[HW_W_ALPHA + tid] = __float_as_uint(alpha[tid]);
   }
   // thread = a word of the bytes of four levels
-  const float *c0 = table + HYB_CEN0, *c1 = c0 + 8;
   if (tid < HW_W_KA1) lut[tid] = hw_key_bytes(c0 + 4 * (tid & 1), unit[0], tid >> 1);
   else if (tid < HW_W_VA0) lut[tid] = hw_key_bytes(c1, unit[1], tid - HW_W_KA1);
   else if (tid < HW_W_UNIT) {
@@ -1191,6 +1232,7 @@ static int hw_launch(const hw_args& a, int grid, hipStream_t stream) {
   return AKV_OK;
 }
 
+template <class F> struct hw_type { typedef F type; };
 // the three kernels of a call; `main` launches the middle one
 template <class F, class M>
 static int hw_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float scale, const hw_args& a,
@@ -1232,8 +1274,10 @@ int akv_attn_hyb_run(int format, const void* query, int q_dtype, int64_t qs_seq,
   const uint64_t all = (uint64_t)(uintptr_t)a.kc | (uint64_t)(uintptr_t)a.vc | a.kps_blk | a.kps_pos | a.kps_head | a.vps_blk | a.vps_pos | a.vps_head;
   // groups of four query heads: the accuracy that one float16 a level of values leaves; other counts: float32's, which they always had
   const bool wide = (all & 15) == 0, exact = a.gqa % 4 != 0;
-  return hw_run<hw35<false>>(query, q_dtype, qs_seq, qs_head, table, scale, a, ws, out, out_dtype, os_seq, os_head, stream, [&](int grid) {
-    return exact ? (wide ? hw_launch<hw35<true>, 16>(a, grid, stream) : hw_launch<hw35<true>, 4>(a, grid, stream))
-                 : (wide ? hw_launch<hw35<false>, 16>(a, grid, stream) : hw_launch<hw35<false>, 4>(a, grid, stream));
-  });
+  auto run = [&](auto f) {
+    typedef typename decltype(f)::type F;
+    return hw_run<F>(query, q_dtype, qs_seq, qs_head, table, scale, a, ws, out, out_dtype, os_seq, os_head, stream,
+                     [&](int grid) { return wide ? hw_launch<F, 16>(a, grid, stream) : hw_launch<F, 4>(a, grid, stream); });
+  };
+  return exact ? run(hw_type<hw35<true>>()) : run(hw_type<hw35<false>>());
 }
