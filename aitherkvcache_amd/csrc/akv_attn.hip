@@ -486,7 +486,7 @@ __global__ __launch_bounds__(256, 1) void akv_attn_reduce_rows_kernel(
     const float* __restrict__ part_acc, const float* __restrict__ part_ml, const uint4* __restrict__ slices, const akv_prep_scale* __restrict__ scale,
     int S, int QH, void* __restrict__ out, int64_t os_seq, int64_t os_head, const uint32_t* __restrict__ status, const int32_t* __restrict__ seqw) {
   constexpr int D = 256, PF = RR_PF / MR, ROWS = 4 * MR;
-  __shared__ __align__(16) ar_rows<D> rows;
+  __shared__ __align__(16) ar_rows<D, 2> rows;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
   const int nrow = S * QH, items = (nrow + ROWS - 1) / ROWS;

@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void akv_attn_mfma_prologue_kernel(
     int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix,
     uint4* __restrict__ qop, uint32_t* __restrict__ lut, uint32_t* __restrict__ status, float qscale, int bits, int nqb,
     int32_t* __restrict__ wgdesc, int32_t* __restrict__ seqw, int G) {
-  __shared__ __align__(16) ar_rows<128> rows;
+  __shared__ __align__(16) ar_rows<128, ar_terms<QDT>()> rows;
   __shared__ int32_t scratch[257];
   __shared__ float best_err[256];
   __shared__ float best_alpha[256];

@@ -2,12 +2,16 @@
 //
 //   Y[n, row] = sum_k M[n, k] X[row, k]           v_mfma_f32_16x16x32_f16
 //
-// A wavefront keeps sixteen rows of the matrix (outputs) in registers, split into two float16 terms from the float32 matrix
-// at its start, and multiplies sixteen rows of X at a time, which lie in LDS as two float16 terms each.  Lane (row, g) ends
-// up with four neighbouring outputs 4 g .. 4 g + 3 of its row: what is stored next is eight or sixteen bytes.
+// A wavefront keeps sixteen rows of the matrix (outputs) in registers, split into float16 terms at its start, and multiplies
+// sixteen rows of X at a time, which lie in LDS as float16 terms.  Lane (row, g) ends up with four neighbouring outputs
+// 4 g .. 4 g + 3 of its row: what is stored next is eight or sixteen bytes.
 //
-// Precision: a row is scaled by a power of two (the largest element to [2^5, 2^6)), the matrix by its prepared one; both terms
-// are rounded to nearest, the product of two remainders is left out: 2^-22 of a product, sums in float32.
+// Precision: a row is scaled by a power of two (the largest element to [2^5, 2^6)), the matrix by its prepared one, all terms are
+// rounded to nearest, sums are float32.  Queries: three terms of the float32 matrix against one of float16 and bfloat16 queries, which
+// hold them exactly (down to 2^-30 of the largest), or three of float32 ones, products down to 2^-24: at head_dim 64, 128 and 256
+// the mean error of a float32 attention output of 300 tokens is 3.7, 4.4 and 5.4e-7; float32 multiply-adds gave 3.8, 4.8 and 5.7,
+// three products of two terms each 4.2, 5.0 and 6.2.  (A step of 24 sequences, 16 heads on 4 of 256, takes 0.6 us longer than with
+// those.)  The reduce at head_dim 256 keeps to two terms: outputs of a single token are at 2.1e-7, 2.2 with multiply-adds.
 #pragma once
 #include "akv_attn_common.h"
 
@@ -17,15 +21,16 @@ typedef _Float16 ar_half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 ar_half4 __attribute__((ext_vector_type(4)));
 typedef float ar_float4 __attribute__((ext_vector_type(4)));
 
-template <int D> struct ar_rows {
+template <int D, int TERMS> struct ar_rows {
   static constexpr int KS = D / 32, PITCH = D + 8;      // (sixteen bytes more: eight rows meet all banks)
-  _Float16 term[2][16][PITCH];
+  _Float16 term[TERMS][16][PITCH];
   float unscale[16];                                    // of a row
 };
 
+#define AR_THIRD 4096.f        // third terms are kept this much larger: they are no subnormals then
 // sixteen rows of a matrix: lane (m, g) holds row m, elements 32 ks + 8 g + e
 template <int D> struct ar_matrix {
-  ar_half8 hi[D / 32], lo[D / 32];
+  ar_half8 term[3][D / 32];
   __device__ __forceinline__ void load(const float* __restrict__ m, float scale) {
     const int lane = threadIdx.x & 63;
     const float4* p = (const float4*)(m + (size_t)(lane & 15) * D + 8 * (lane >> 4));
@@ -41,22 +46,31 @@ template <int D> struct ar_matrix {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float s = x[e] * scale;
-        hi[ks][e] = (_Float16)s;
-        lo[ks][e] = (_Float16)(s - (float)hi[ks][e]);
+        term[0][ks][e] = (_Float16)s;
+        const float r = s - (float)term[0][ks][e];
+        term[1][ks][e] = (_Float16)r;
+        term[2][ks][e] = (_Float16)((r - (float)term[1][ks][e]) * AR_THIRD);
       }
     }
   }
-  __device__ __forceinline__ ar_float4 times(const ar_rows<D>& rows) const {
+  template <int TERMS> __device__ __forceinline__ ar_float4 times(const ar_rows<D, TERMS>& rows) const {
     const int lane = threadIdx.x & 63, row = lane & 15, g = lane >> 4;
-    ar_float4 acc = {0.f, 0.f, 0.f, 0.f};
+    ar_float4 first = {0.f, 0.f, 0.f, 0.f}, second = first, third = first;
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) {
-      const ar_half8 x = *(const ar_half8*)&rows.term[0][row][32 * ks + 8 * g], xl = *(const ar_half8*)&rows.term[1][row][32 * ks + 8 * g];
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[ks], x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[ks], x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[ks], xl, acc, 0, 0, 0);
+      ar_half8 x[TERMS];
+#pragma unroll
+      for (int i = 0; i < TERMS; ++i) x[i] = *(const ar_half8*)&rows.term[i][row][32 * ks + 8 * g];
+      first = __builtin_amdgcn_mfma_f32_16x16x32_f16(term[0][ks], x[0], first, 0, 0, 0);
+      second = __builtin_amdgcn_mfma_f32_16x16x32_f16(term[1][ks], x[0], second, 0, 0, 0);
+      third = __builtin_amdgcn_mfma_f32_16x16x32_f16(term[2][ks], x[0], third, 0, 0, 0);
+      if constexpr (TERMS == 3) {
+        second = __builtin_amdgcn_mfma_f32_16x16x32_f16(term[0][ks], x[1], second, 0, 0, 0);
+        second = __builtin_amdgcn_mfma_f32_16x16x32_f16(term[1][ks], x[1], second, 0, 0, 0);
+        third = __builtin_amdgcn_mfma_f32_16x16x32_f16(term[0][ks], x[2], third, 0, 0, 0);
+      }
     }
-    return acc;
+    return first + (second + third * (1.f / AR_THIRD));
   }
 };
 // scale of a row whose largest magnitude is m, and what undoes it (and AR_M_SCALE)
@@ -67,6 +81,8 @@ __device__ __forceinline__ float ar_scale(float m, float& unscale) {
 }
 
 // ----------------------------------------------------------------------------------
+// terms of a query: float16 and bfloat16 fit one
+template <int QDT> constexpr int ar_terms() { return QDT == AKV_F32 ? 3 : 1; }
 // Query rows into the operand of a main kernel, by workgroup b of nb (a multiple of D / 64) of 256 threads: b % (D / 64) is its
 // slice of 64 outputs, b / (D / 64) its first tile of sixteen rows.  A tile holds 16 / `slots` (sequence, kv head) items of up to
 // `slots` query heads (4 or 8; the rest of a tile's rows are zero: columns of the operand that no head has but a main kernel
@@ -76,7 +92,7 @@ __device__ __forceinline__ float ar_scale(float m, float& unscale) {
 // Lane (column, quarter) of a step: column q the rounding of query head q's coordinates, 8 + q their remainder.
 // ----------------------------------------------------------------------------------
 template <int D, int QDT, bool FULL>
-__device__ __forceinline__ void ar_rotate_queries(ar_rows<D>& rows, int b, int nb, const void* __restrict__ query, int64_t qs_seq, int64_t qs_head,
+__device__ __forceinline__ void ar_rotate_queries(ar_rows<D, ar_terms<QDT>()>& rows, int b, int nb, const void* __restrict__ query, int64_t qs_seq, int64_t qs_head,
                                                   const float* __restrict__ Pi, const akv_prep_scale* __restrict__ scale, int S, int QH, int KVH,
                                                   int slots, void* __restrict__ qop, float* __restrict__ fac, float qscale, int bits) {
   constexpr int NS = D / 64, EPT = D / 16;
@@ -109,15 +125,19 @@ __device__ __forceinline__ void ar_rotate_queries(ar_rows<D>& rows, int b, int n
     un *= up;
 #pragma unroll
     for (int i = 0; i < EPT; i += 4) {
-      ar_half4 hi, lo;
+      constexpr int TERMS = ar_terms<QDT>();
+      ar_half4 t[TERMS];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float s = x[i + e] * sc;
-        hi[e] = (_Float16)s;
-        lo[e] = (_Float16)(s - (float)hi[e]);
+        float s = x[i + e] * sc;
+#pragma unroll
+        for (int j = 0; j < TERMS; ++j) {
+          t[j][e] = (_Float16)(j == 2 ? s * AR_THIRD : s);
+          s -= (float)t[j][e];
+        }
       }
-      *(ar_half4*)&rows.term[0][row][16 * i + 4 * part] = hi;
-      *(ar_half4*)&rows.term[1][row][16 * i + 4 * part] = lo;
+#pragma unroll
+      for (int j = 0; j < TERMS; ++j) *(ar_half4*)&rows.term[j][row][16 * i + 4 * part] = t[j];
     }
     const int item = tile * per + row / slots, q = row % slots;
     if (part == 0) {

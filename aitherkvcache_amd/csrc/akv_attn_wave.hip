@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void akv_attn_wave_prologue_kernel(
     int S, int QH, int KVH, int slots, const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix,
     uint2* __restrict__ qop, float* __restrict__ fac, uint32_t* __restrict__ status, float qscale, int bits, int32_t* __restrict__ wgdesc,
     int32_t* __restrict__ seqw, int G, int shares) {
-  __shared__ __align__(16) ar_rows<D> rows;
+  __shared__ __align__(16) ar_rows<D, ar_terms<QDT>()> rows;
   __shared__ int32_t scratch[257];
   if (blockIdx.x == 0) {
     if (threadIdx.x == 0) status[0] = 0u;
