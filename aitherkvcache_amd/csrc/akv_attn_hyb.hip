@@ -116,12 +116,14 @@ __device__ __forceinline__ hw_int4 hw_as_int4(uint4 u) {
 // (x & mask) | rest in one instruction
 __device__ __forceinline__ uint32_t hw_and_or(uint32_t x, uint32_t mask, uint32_t rest) { return __builtin_amdgcn_bitop3_b32(x, mask, rest, 0xEA); }
 // N bytes per lane from base + voff into LDS at lds + N lane.  (The compiler does not see the request: whoever reads waits by
-// hw_landed(); a wavefront's buffers are its own.  No earlier LDS read of the wavefront is in flight any more.)
+// hw_landed(); a wavefront's buffers are its own.  No earlier LDS read of the wavefront is in flight any more.  Five wait states
+// before the request: its base may come from a lane read, a restored register for one, and the compiler counts none of them here;
+// nor the one behind m0.)
 template <int N> __device__ __forceinline__ void hw_request(const uint8_t* base, uint32_t voff, uint32_t lds) {
   if constexpr (N == 16)
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "{m0}"(lds) : "memory");
   else
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 3\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(base), "{m0}"(lds) : "memory");
 }
 __device__ __forceinline__ void hw_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 

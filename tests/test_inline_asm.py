@@ -42,3 +42,25 @@ def test_masks_are_read_two_wait_states_after_they_were_written():
     found = [(name, lines) for name, lines, _ in statements()]
     assert sum(any(x.startswith("v_cmp") for x in lines) for _, lines in found) >= 4, "the statements with compares were not found"
     assert not [(name, early_reads(lines)) for name, lines in found if early_reads(lines)]
+
+
+def wait_states(lines, op):
+    """Wait states between the start of a statement and its first instruction `op`."""
+    gone = 0
+    for line in lines:
+        if line.startswith(op):
+            return gone
+        gone += int(line.split()[1]) + 1 if line.startswith("s_nop") else 1
+    return None
+
+
+def test_requests_into_lds_take_m0_and_wait_for_their_base():
+    """A memory instruction reads a scalar register five wait states after a vector instruction wrote it at the earliest, and one
+    after m0 was written; the compiler counts neither into a statement."""
+    found = [(lines, rest) for _, lines, rest in statements() if any("global_load" in x for x in lines)]
+    assert found
+    for lines, rest in found:
+        assert wait_states(lines, "global_load") >= 5, lines
+        assert '"{m0}"(' in rest
+    for _, lines, rest in statements():
+        assert not any(re.match(r"s_\w+ m0,", x) for x in lines), "m0 written behind the compiler's back"
