@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
         bl[t][ks] = akv_as_half8(bop[2048 + idx]);
       }
   }
-  // a main kernel whose bounded wait gave up has produced garbage: say so in every output
+  // a call marked as failed says so in every output
   const float poison = status[0] != 0u ? __uint_as_float(0x7fc00000u) : 0.f;
   for (int item = blockIdx.x; item < S * groups; item += gridDim.x) {
   const int s = item / groups, hg = item % groups;
@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256, 1) void akv_attn_reduce_rows_kernel(
       mr[t][h] = akv_as_half8(slices[D * D / 8 + idx]);
     }
   const float up = scale->up * (AR_M_SCALE / 64.f);
-  // a main kernel whose bounded wait gave up has produced garbage: say so in every output
+  // a call marked as failed says so in every output
   const float poison = status[0] != 0u ? __uint_as_float(0x7fc00000u) : 0.f;
   __builtin_amdgcn_sched_barrier(0);
   for (int item = blockIdx.x; item < items; item += gridDim.x) {

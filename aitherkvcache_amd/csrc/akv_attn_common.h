@@ -52,8 +52,8 @@ static inline size_t akv_align256(size_t v) { return (v + 255) & ~(size_t)255; }
 #define AKV_WS_LUT_BYTES 4096
 #define AKV_WS_STATUS_BYTES 256
 #define AKV_WS_HEADER_BYTES (AKV_WS_LUT_BYTES + AKV_WS_STATUS_BYTES)
-// status word 0: nonzero when a bounded wait inside the main kernel of the most recent call gave up
-// (cleared by the prologue, set with a plain vector store, turned into NaN outputs by the reduce)
+// status word 0: nonzero when the most recent call failed (cleared by the prologue, turned into NaN outputs by the reduce).  No
+// kernel has a wait that could give up; the prologue of hybrid calls sets it when akv_debug_set_handoff_spin_limit(0) says so.
 #define AKV_STATUS_HANDOFF_TIMEOUT 1u
 // record of a workgroup (int32 words): its range [g0, g1) of the global block axis; then its first segment: the
 // sequence (-1: not recorded, the kernel searches the prefix), the sequence's first and one-past-last global

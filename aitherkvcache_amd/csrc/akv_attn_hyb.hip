@@ -1145,7 +1145,7 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_reduce_kernel(const float* _
   const int s = item / QH, h = item % QH;
   const int w_lo = seqw[2 * s], w_hi = seqw[2 * s + 1];
   const int64_t obase = s * os_seq + h * os_head;
-  // (a call whose kernels reported a failure has produced garbage: every output says so)
+  // (a call marked as failed says so in every output)
   const float poison = status[0] != 0u ? __uint_as_float(0x7fc00000u) : 0.f;
   int at[4];
 #pragma unroll
@@ -1200,8 +1200,8 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_reduce_kernel(const float* _
 // ----------------------------------------------------------------------------------
 bool akv_attn_mfma_disabled();
 
-// polls of a bounded wait inside a kernel (akv_debug_set_handoff_spin_limit).  No kernel has such a wait any more; a limit of
-// none still marks a call as failed, so that callers can see what a failed call looks like.
+// akv_debug_set_handoff_spin_limit: 0 marks calls as failed, so that callers can see what a failed call looks like.  (No kernel has
+// a wait that could give up.)
 static int g_spin_limit = -1;
 extern "C" int akv_debug_set_handoff_spin_limit(int polls) {
   g_spin_limit = polls;

@@ -551,7 +551,7 @@ __global__ __launch_bounds__(64) void hyb_attn_reduce_kernel(
   const int lane = threadIdx.x;
   const int b0 = prefix[s], b1 = prefix[s + 1];
   const int64_t obase = s * os_seq + h * os_head;
-  // a main kernel whose bounded wait gave up has produced garbage: say so in every output
+  // a call marked as failed says so in every output
   const float poison = status[0] != 0u ? __uint_as_float(0x7fc00000u) : 0.f;
   if (b1 <= b0) {
     akv_elem<ODT>::store(out, obase + lane, poison);

@@ -153,8 +153,8 @@ class TQPagedAttention:
         return out if out.dtype == query.dtype else out.to(query.dtype)
 
     def last_call_status(self) -> int:
-        """0 when the most recent forward() / forward_no_alloc() ran clean; bit 0 set when a bounded hand-off
-        wait inside its main kernel gave up (the outputs of that call are NaN).  Synchronises the stream."""
+        """0 when the most recent forward() / forward_no_alloc() ran clean; bit 0 set when it failed on the device (its
+        outputs are NaN).  Synchronises the stream."""
         if getattr(self, "_last_static", None) is not None:
             return _lib.attn_status_static(self._last_static)       # the library's built-in scratch array
         return _lib.attn_status(self._workspace)

@@ -158,6 +158,6 @@ class HybridPagedAttention:
         return out if out.dtype == query.dtype else out.to(query.dtype)
 
     def last_call_status(self) -> int:
-        """0 when the most recent forward() ran clean; bit 0 set when a bounded hand-off wait inside
-        its main kernel gave up (the outputs of that call are NaN).  Synchronises the stream."""
+        """0 when the most recent forward() ran clean; bit 0 set when it failed on the device (its outputs are NaN).
+        Synchronises the stream."""
         return _lib.attn_status(self._workspace)

@@ -230,14 +230,15 @@ int akv_paged_attn_static(const void* query, int q_dtype, int64_t qs_seq, int64_
                           void* stream);
 
 /* Status of the most recent akv_paged_attn / akv_hybrid_paged_attn call that used `workspace`
- * (no counterpart in the reference): 0 in *flags (host pointer) = clean, bit 0 = a bounded wait inside a kernel gave
- * up; the outputs of such a call are all NaN.  This waits for `stream`.  (No kernel of this library waits inside any more.)
+ * (no counterpart in the reference): 0 in *flags (host pointer) = clean, bit 0 = failed on the device; the outputs of such a
+ * call are all NaN.  This waits for `stream`.  (Kernels whose bounded waits could give up set the bit; none of this library
+ * waits inside any more, so only the switch below does.)
  * workspace == NULL asks about the most recent akv_paged_attn_static call on the current device
  * (0 when there has been none).
- * akv_debug_set_handoff_spin_limit sets the number of polls such a wait makes (negative = the default).  It exists so that
- * a test can exercise the failure path from the host: with 0 an akv_hybrid_paged_attn call on tq35 rows reports a failure,
- * every kernel runs to its end.  The akv_debug_* and
- * akv_profile_* switches are process-global words read at each launch and are not synchronised: set them
+ * akv_debug_set_handoff_spin_limit(0) marks calls as failed, any other value ends that (0 was the number of polls at which every
+ * wait gave up; the name has stayed).  It is there so that a caller can see what a failed call looks like: akv_hybrid_paged_attn
+ * and akv_hybrid25_paged_attn on blocks of 16 or 32 tokens then report a failure, every kernel runs as ever.  The akv_debug_*
+ * and akv_profile_* switches are process-global words read at each launch and are not synchronised: set them
  * from one thread while no call of another thread is being issued. */
 int akv_paged_attn_status(const void* workspace, int* flags, void* stream);
 int akv_debug_set_handoff_spin_limit(int polls);

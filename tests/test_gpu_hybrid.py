@@ -381,9 +381,8 @@ def test_one_object_across_batch_sizes(golden, dev):
 
 
 def test_handoff_timeout_is_reported(golden, dev):
-    """The tq35 kernel hands chunks from its score to its value wavefronts through polled counters with a
-    bounded wait.  With a limit of zero polls every wait gives up at once (the kernels still run to their
-    end): outputs are NaN and the status query says so; with the default limit the next call is clean."""
+    """A call marked as failed from the host (no kernel waits inside, so none can fail by itself): outputs are NaN and the
+    status query says so; with the default limit the next call is clean."""
     from aitherkvcache_amd import _lib
     h = akv.HybridTurboQuant(device=str(dev))
     h.calibrate_uniform(num_kv_heads=8)
