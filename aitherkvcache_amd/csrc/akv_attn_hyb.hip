@@ -11,24 +11,26 @@
 //   rows     requested a chunk ahead straight into LDS (16 rows an instruction); nothing passes through registers, and an
 //            instruction touches every row once.  The 16-byte pieces of rows are permuted so that the sixteen lanes that read
 //            the same place of sixteen rows meet different banks.
-//   scores   v_mfma_i32_16x16x64_i8, 16 tokens a tile.  A level is an integer of three signed bytes (the query's form), looked up four codes at
+//   scores   v_mfma_i32_16x16x64_i8, 16 tokens a tile.  A level is an integer of three signed bytes, looked up four codes at
 //            a time by byte permutes from registers; signs are +-64, their bits as they lie (no look-up).  The query is three
-//            signed bytes (23 bits and a sign, one scale a head), in the columns 4 d + head of digit d.  Sums are exact.
+//            signed bytes too (23 bits and a sign, one scale a head), in the columns 4 d + head of digit d.  Sums are exact.
 //   softmax  on packed scores: the lanes of a row add the digits up so that lane 4 k + c ends up with two of the eight
 //            tokens of head c, as in akv_attn_wave_kernel.
 //   values   v_mfma_f32_16x16x32_f16, all 32 tokens of a chunk in one product.  The transposing LDS read hands a lane one byte
 //            position of eight tokens; codes are looked up four tokens at a time (two byte permutes, two to interleave), signs
 //            are the sign bit of 1.0.  A weight is two float16 terms, columns 0..3 and 4..7.
 //
-// What bounds it: the issue of vector instructions, 610 a chunk and kv head (vector unit 78 % of the cycles, matrix cores 15 %,
-// LDS 41 %).  The kernel before this one (four score and four value wavefronts that handed chunks over through polled counters,
-// codes spread to nibbles and looked up in LDS) issued some 1,300 at two wavefronts a SIMD.  A decode step, this | that, bfloat16:
-// 64 sequences of 4,000 to 8,192 tokens, 32 heads on 8: 167 | 211 us (160 with levels of keys in two bytes, off by 1e-6 of the
-// largest: float32 outputs whose scores reach some hundreds had twice the error); 256 of 64 to 512: 82 | 111; 64 of 300: 45 | 54; 4 of 300:
-// 29 | 38; 32 of 1,000 to 9,000 with 64 heads on 8: 130 | 188, 8 on 1: 42 | 61.  Head counts that are no multiple of four a kv
-// head (levels of float32's accuracy, see hw35) | the vector kernel: 28 on 4: 107 | 570; 16 on 16: 166 | 238.
-// tq25 rows | the vector kernel (tables of partial products in LDS): 64 of 4,000 to 8,192, 32 heads on 8: 160 | 335; 256 of 64 to
-// 512: 88 | 114; 32 of 1,000 to 9,000 with 8 heads on 1: 43 | 246, 28 on 4: 78 | 278, 16 on 16: 130 | 144; 4 of 300: the same.
+// What bounds it: the issue of vector instructions, 660 a chunk and kv head (64 sequences of 8,192 tokens: vector unit 73 % of the
+// cycles, matrix cores 15 %, LDS 36 %).  The kernel before this one (four score and four value wavefronts that handed chunks over
+// through polled counters, codes spread to nibbles and looked up in LDS) issued some 1,300 at two wavefronts a SIMD.  A decode
+// step, its write included, this | that, bfloat16:
+// 64 sequences of 4,000 to 8,192 tokens, 32 heads on 8: 166 | 211 us; 256 of 64 to 512: 84 | 111; 64 of 300: 45 | 54; 4 of 300:
+// 24 | 38; 32 of 1,000 to 9,000 with 64 heads on 8: 134 | 188, 8 on 1: 42 | 61.  (With levels of keys in two bytes the first was 159
+// and the last but one 127, but they are off by 1e-6 of the largest: float32 outputs whose scores reach some hundreds had
+// twice the error.)  Head counts that are no multiple of four a kv head (values of float32's accuracy, see hw35) | the vector
+// kernel: 28 on 4: 106 | 570; 16 on 16: 165 | 238.
+// tq25 rows | the vector kernel (tables of partial products in LDS): 64 of 4,000 to 8,192, 32 heads on 8: 156 | 335; 256 of 64 to
+// 512: 88 | 114; 32 of 1,000 to 9,000 with 8 heads on 1: 43 | 246, 28 on 4: 78 | 278, 16 on 16: 126 | 144; 4 of 300: the same.
 #include <type_traits>
 
 #include "akv_attn_common.h"
@@ -518,8 +520,8 @@ struct hw25 {
         x = x | (x << 18);
         return hw_as_long(hw_and_or(x, 0x80808080u, 0x40404040u), hw_and_or(x << 4, 0x80808080u, 0x40404040u));
       };
-      // (the two products of a part are added up here: the second one started from the first one's sums, which the compiler let
-      // overlap its own in part, and wrong sums came out)
+      // (the two products of a part are added up here: wrong sums came out when the second one, of another shape, started from the
+      // first one's.  Why was not found.)
       hw_int4 c[3], sg[3], sh[2];
       {
         const uint32_t x = a0[j] | (a0[j] << 18), s0 = (x >> 6) & 0x03030303u, s1 = (x >> 2) & 0x03030303u;
@@ -1220,7 +1222,9 @@ bool akv_attn_hyb_applicable(int block_size, const int64_t* strides6) {
   return true;
 }
 
-// ranges the block axis is cut into: three workgroups a CU, as many as its registers admit
+// ranges the block axis is cut into: three workgroups a CU over all head slots, what the registers of hw35<false> and hw25 admit
+// (hw35<true> runs two of them at a time), but no more than akv_attn_grid(), two a CU: the workspace holds records and partial
+// results for so many, and calls of up to four groups of query heads get no more.  (The other choices have not been measured.)
 static int hw_ranges(int kv_groups, int hp) {
   const int cus = akv_cached_cu_count(), most = akv_attn_grid();
   const int per = (kv_groups + hp - 1) / hp, want = (cus > 0 ? cus : 256) * 3 / per;

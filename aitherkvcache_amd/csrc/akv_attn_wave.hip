@@ -26,7 +26,7 @@
 // 2-bit codes are looked up as nibbles: two masks and a shift spread a byte of four codes, no second table.  3-bit codes are
 // looked up in pairs, six bits as they lie: a group of eight codes is 24 bits, big-endian, spread to a byte a field by six
 // instructions (one permute among them, which also takes the group out of unaligned bytes); the table then has 64 entries.
-// 3 bits, decode step, this | the vector kernel that served 64 and 256 and the eight-slot kernel at 128: 32 heads on 8 of 64,
+// 3 bits, an attention call (no write), this | the vector kernel that served 64 and 256 and the eight-slot kernel at 128: 32 heads on 8 of 64,
 // 48 sequences of 512 to 8,192 tokens 56.3 | 113.2 us; 16 on 4 of 256, 24 sequences 66.7 | 141.5; 8 on 1 of 128, 48 of 1,024
 // to 16,384 39.3 | 62.2; 8 on 2 of 128 52.6 | 62.3.
 //
@@ -408,7 +408,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           // in 8..15.  PACK = 4 (at most four query heads): lane 4 k + c of a row takes the token pair k of head c, the first
           // term from lane c, the second from lane 8 + c; PACK = 2: lane c takes tile 0, lane 8 + c tile 1 of head c.  Every lane
           // on all eight tokens of its column, as the accumulator lies, were 16 exponentials a lane (a quarter of the rate of
-          // other vector instructions) in place of 4 or 8.  A decode step, 32 query heads on 8 of 64, 48 sequences of 512 to 8,192
+          // other vector instructions) in place of 4 or 8.  An attention call, 32 query heads on 8 of 64, 48 sequences of 512 to 8,192
           // tokens: 64.9 -> 60.1 us; 16 on 4 of 256, 24 sequences: 64.4 -> 63.0; 8 on 1 of 128, 48 of 1,024 to 16,384: 36.9 -> 35.9.
           float sv[NV], vn[NV], tv[NV];
           if constexpr (PACK == 4) {

@@ -736,7 +736,7 @@ extern "C" int akv_hybrid_paged_attn(
   if (workspace_bytes < need)
     return akv_fail(AKV_ERR_WORKSPACE, "akv_hybrid_paged_attn: workspace %zu < %zu bytes", workspace_bytes, need);
 
-  // groups of four query heads over blocks of 16 or 32 tokens: the matrix-core kernel
+  // blocks of 16 or 32 tokens: the matrix-core kernel, whatever the grouping of the heads
   const int64_t strides6[6] = {kps_blk, kps_pos, kps_head, vps_blk, vps_pos, vps_head};
   if (max_blocks_per_seq > 0 && num_blocks < ((int64_t)1 << 31) && akv_attn_hyb_applicable(block_size, strides6)) {
     akv_hyb_attn_args m;

@@ -51,8 +51,8 @@ def hybrid_encode_and_store(htq, x: torch.Tensor, slot_mapping: torch.Tensor, ca
 def hybrid_encode_and_store_pair(htq, key: torch.Tensor, value: torch.Tensor, slot_mapping: torch.Tensor,
                                  k_cache: torch.Tensor, v_cache: torch.Tensor, block_size: int = 16,
                                  max_blocks: int = 0) -> None:
-    """K and V of a step (the two encodes of tq::hybrid_decode_step, reference vllm/hooks.py:271-284) in one call:
-    one launch while the step is small.  Tensors or caches that differ in dtype, shape or strides go through
+    """K and V of a step (the two encodes of tq::hybrid_decode_step, reference vllm/hooks.py:271-284) in one call
+    and one launch.  Tensors or caches that differ in dtype, shape or strides go through
     hybrid_encode_and_store one after the other."""
     if htq.group_order is None:
         rc = _lib.calls().hybrid_encode(key, value, slot_mapping, k_cache, v_cache, htq.kernel_table, _FORMAT[htq._abi], htq.head_dim,

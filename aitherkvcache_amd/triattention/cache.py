@@ -60,9 +60,9 @@ class SpectralKVCache:
     def encode_and_store(self, keys: torch.Tensor, values: torch.Tensor, slot_mapping: torch.Tensor) -> None:
         """Encode-on-write of a step: keys / values [num_tokens, kv_heads, head_dim] (keys before RoPE) are encoded
         (SpectralKVEncoder.encode, reference encoder.py:73-149) and written into the block pool at
-        slot = block * block_size + position per token, one launch per tensor -- what the reference does with
-        encode followed by store_token per token (cache.py:106-140).  Negative slots and slots past the cache are
-        skipped.  No counterpart in the reference."""
+        slot = block * block_size + position per token, K and V in one launch where both have one type
+        and layout -- what the reference does with encode followed by store_token per token (cache.py:106-140).
+        Negative slots and slots past the cache are skipped.  No counterpart in the reference."""
         rc = _lib.calls().spectral_encode(keys, values, slot_mapping, *self._arrays(), self.num_kv_heads, self.config.head_dim,
                                           self.num_freqs, self.max_blocks * self.block_size)
         if rc is not None:
