@@ -445,7 +445,9 @@ def _make_impl_class():
             cache = cls._tq_gpu_cache
             if cache is not None and key is not None and value is not None:
                 try:
-                    fused_encode_and_store(cache, self._tq_layer_idx, key, value, attn_metadata.slot_mapping)
+                    slots = attn_metadata.slot_mapping
+                    n = min(key.shape[0], slots.shape[0])      # vLLM may pad key and value, not the slots
+                    fused_encode_and_store(cache, self._tq_layer_idx, key[:n], value[:n], slots[:n])
                 except Exception as e:      # the copy is an optimisation: serving goes on without it
                     print(f"[TQ] encode error L{self._tq_layer_idx}: {e}", file=sys.stderr, flush=True)
             if (cls._fused_enabled and cache is not None

@@ -279,6 +279,29 @@ def test_shadow_copy_serves_decode(golden, dev, impl_cls, monkeypatch):
     assert float(cache.k_norms[1][3, 4, 0]) > 0 and float(cache.k_norms[0][3, 4, 0]) == 0     # token 20 -> block 3, row 4
 
 
+def test_shadow_copy_takes_padded_keys(dev, impl_cls, monkeypatch, capsys):
+    """Keys and values padded beyond the step's tokens, slots that are not: the tokens go into the copy."""
+    monkeypatch.delenv("AITHER_TQ_MODE", raising=False)
+    monkeypatch.delenv("AITHER_TQ_PRIMARY", raising=False)
+    impl_cls.reset_class_state()
+    impl_cls._INIT_AFTER_FORWARDS = 1
+    layers = [impl_cls(QH, 128, 1 / math.sqrt(128), num_kv_heads=KVH) for _ in range(LAYERS)]
+    kv_cache = torch.zeros(NB, 2, BS, KVH, 128, dtype=torch.float16, device=dev)
+    tables = np.array([[2, 3]], dtype=np.int32)
+    rng = np.random.default_rng(80)
+    for step in range(2):
+        k, v = t(kv_like(rng, (8, KVH, 128)), dev), t(kv_like(rng, (8, KVH, 128)), dev)
+        md = meta(dev, slots_of(tables, 0, 5 * step, 5 * step + 5), tables, [5 * step + 5], 5, 5, query_lens=[5])
+        out = torch.zeros(8, QH * 128, dtype=torch.float16, device=dev)
+        for impl in layers:
+            with pytest.raises(RuntimeError, match="vLLM"):                                  # prefill is the parent's
+                impl.forward(None, out.clone(), k, v, kv_cache, md, output=out)
+    cache = impl_cls._tq_gpu_cache
+    assert "encode error" not in capsys.readouterr().err
+    for norms, x in ((cache.k_norms, k), (cache.v_norms, v)):
+        assert torch.allclose(norms[1][2, 5:10], x[:5].float().norm(dim=-1), rtol=1e-5) and torch.all(norms[1][2, 10:] == 0) and torch.all(norms[1][3] == 0)
+
+
 def test_profiling_run_and_draft_layers(dev, impl_cls):
     target = impl_cls(QH, 128, 0.1, num_kv_heads=KVH, kv_cache_dtype="tq-t4nc")
     draft = impl_cls(4, 64, 0.1, num_kv_heads=1, kv_cache_dtype="tq-t4nc")
