@@ -58,9 +58,9 @@ def decode_step(query, key, value, kv_cache, output, k_norms, v_norms, slot_mapp
     tq = _tq_quantizers[head_size]
     key_cache, value_cache = kv_cache[:, 0], kv_cache[:, 1]
     block_size = key_cache.shape[1]
-    n = key.shape[0]
+    n = min(key.shape[0], slot_mapping.shape[0])      # vLLM may pad key and value, not the slots
     prep = tq.prepared_rotation()
-    fused_kv_update_pair(key, value, slot_mapping[:n], key_cache, k_norms[layer_idx], value_cache,
+    fused_kv_update_pair(key[:n], value[:n], slot_mapping[:n], key_cache, k_norms[layer_idx], value_cache,
                          v_norms[layer_idx], tq.rotation, tq.boundaries_inner, tq.bits,
                          block_size=block_size, prepared=prep)
     attn = _tq_fused_attn.get((layer_idx, head_size))
@@ -81,8 +81,8 @@ def hybrid_decode_step(query, key, value, kv_cache, output, slot_mapping, block_
     htq = _tq_quantizers[head_size]
     key_cache, value_cache = kv_cache[:, 0], kv_cache[:, 1]
     block_size = key_cache.shape[1]
-    n = key.shape[0]
-    hybrid_encode_and_store_pair(htq, key, value, slot_mapping[:n], key_cache, value_cache, block_size=block_size)
+    n = min(key.shape[0], slot_mapping.shape[0])      # vLLM may pad key and value, not the slots
+    hybrid_encode_and_store_pair(htq, key[:n], value[:n], slot_mapping[:n], key_cache, value_cache, block_size=block_size)
     attn = _tq_fused_attn.get((layer_idx, head_size))
     if attn is None:
         attn = HybridPagedAttention(htq, num_heads)

@@ -302,6 +302,31 @@ def test_shadow_copy_takes_padded_keys(dev, impl_cls, monkeypatch, capsys):
         assert torch.allclose(norms[1][2, 5:10], x[:5].float().norm(dim=-1), rtol=1e-5) and torch.all(norms[1][2, 10:] == 0) and torch.all(norms[1][3] == 0)
 
 
+@pytest.mark.parametrize("mode,row", [(None, 68), ("tq35", 64), ("tq25", 44)])
+def test_decode_steps_take_padded_keys(dev, mode, row):
+    """The custom ops' bodies: keys and values of more rows than there are slots write those that have one."""
+    from aitherkvcache_amd.vllm import hooks
+    hooks.reset_state()
+    hooks.init_quantizer(128, mode=mode, device=str(dev), num_kv_heads=KVH) if mode else hooks.init_quantizer(128, bits=4, device=str(dev))
+    rng = np.random.default_rng(81)
+    key, value = (t(kv_like(rng, (5, KVH, 128)), dev) for _ in range(2))
+    q = t(rng.standard_normal((5, QH, 128)).astype(np.float16), dev)
+    slots, lens = t(np.array([0, BS, 2 * BS]), dev), t(np.ones(3, dtype=np.int32), dev)
+    tables = t(np.arange(3, dtype=np.int32)[:, None].copy(), dev)
+    results = []
+    for rows in (3, 5):
+        kv, norms = torch.zeros(4, 2, BS, KVH, row, dtype=torch.uint8, device=dev), torch.zeros(2, 1, 4, BS, KVH, device=dev)
+        out = torch.zeros(5, QH, 128, dtype=torch.float16, device=dev)
+        fixed = (slots, tables, lens, 0, QH, KVH, 128, 0.09, 3)
+        if mode:
+            hooks.hybrid_decode_step(q, key[:rows], value[:rows], kv, out, *fixed)
+        else:
+            hooks.decode_step(q, key[:rows], value[:rows], kv, out, norms[0], norms[1], *fixed)
+        results.append((kv, norms, out))
+    hooks.reset_state()
+    assert all(torch.equal(*x) for x in zip(*results)) and bool(results[0][0][2].any()) and not bool(results[0][0][3].any())
+
+
 def test_profiling_run_and_draft_layers(dev, impl_cls):
     target = impl_cls(QH, 128, 0.1, num_kv_heads=KVH, kv_cache_dtype="tq-t4nc")
     draft = impl_cls(4, 64, 0.1, num_kv_heads=1, kv_cache_dtype="tq-t4nc")
