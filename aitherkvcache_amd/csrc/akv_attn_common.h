@@ -56,8 +56,8 @@ static inline size_t akv_align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // kernel has a wait that could give up; the prologue of hybrid calls sets it when akv_debug_set_handoff_spin_limit(0) says so.
 #define AKV_STATUS_HANDOFF_TIMEOUT 1u
 // record of a workgroup (int32 words): its range [g0, g1) of the global block axis; then its first segment: the
-// sequence (-1: not recorded, the kernel searches the prefix), the sequence's first and one-past-last global
-// block, its context length in tokens (clamped to the table width)
+// sequence (-1: the range is empty), the sequence's first and one-past-last global block, its context length in
+// tokens (clamped to the table width)
 #define AKV_WGREC 8
 #define AKV_WGREC_G0 0
 #define AKV_WGREC_G1 1
@@ -181,7 +181,7 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
   int32_t* p_ctx = lds + 130;           // [64] context length in tokens (clamped to the table width)
   int32_t* p_mode = lds + 194;          // [0] 1 = whole workgroups per sequence, [1] = total blocks
   if (S > 64) {
-    // many sequences: the general scan, equal ranges, first segments found by the main kernel itself
+    // many sequences: the general scan, equal ranges
     akv_block_prefix_scan(context_lens, cl_itype, S, block_size, max_blocks_per_seq, prefix, lds);
     __threadfence_block();
     __syncthreads();                    // the prefix written by this workgroup is readable by all of it
@@ -192,13 +192,24 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
       const int g0 = min(total, w * per);
       rec[AKV_WGREC_G0] = g0;
       rec[AKV_WGREC_G1] = min(total, g0 + per);
-      rec[AKV_WGREC_SEQ] = -1;
+      if (g0 >= total) rec[AKV_WGREC_SEQ] = -1;
     }
     for (int s = tid; s < S; s += blockDim.x) {
       const int b0 = prefix[s], b1 = prefix[s + 1];
       const int w_lo = per > 0 ? b0 / per : 0;
       seqw[2 * s] = w_lo;
       seqw[2 * s + 1] = (per > 0 && b1 > b0) ? (b1 - 1) / per : w_lo - 1;
+      // the ranges that start in the sequence: each start lies in one
+      if (b1 > b0) {
+        const int ctx = (int)akv_seq_tokens(context_lens, cl_itype, s, block_size, max_blocks_per_seq);
+        for (int w = (b0 + per - 1) / per; w < G && w * per < b1; ++w) {
+          int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
+          rec[AKV_WGREC_SEQ] = s;
+          rec[AKV_WGREC_SB0] = b0;
+          rec[AKV_WGREC_SB1] = b1;
+          rec[AKV_WGREC_CTX] = ctx;
+        }
+      }
     }
     return;
   }
@@ -303,26 +314,23 @@ __device__ __forceinline__ int akv_find_seq(const int32_t* __restrict__ prefix, 
   return lo;
 }
 
-// The same search for a whole wavefront with up to 63 sequences: lane i holds prefix[i] (one vector load at the
-// start of the kernel, `held`), the sequence is the number of entries 1..S that do not exceed g, and the bounds
-// of the sequence come out of the register -- no chain of dependent loads per segment.  More sequences than
-// that take the scalar search.
-__device__ __forceinline__ int akv_prefix_hold(const int32_t* __restrict__ prefix, int S) {
-  const int lane = threadIdx.x & 63;
-  return prefix[min(lane, S)];
-}
-__device__ __forceinline__ int akv_find_seq_held(const int32_t* __restrict__ prefix, int S, int held, int g,
-                                                 int& sb0, int& sb1) {
-  if (S <= 63) {
-    const int lane = threadIdx.x & 63;
-    const int s = __popcll(__ballot(lane >= 1 && lane <= S && held <= g));
-    sb0 = __builtin_amdgcn_readlane(held, s);
-    sb1 = __builtin_amdgcn_readlane(held, s + 1);
-    return s;
+// The sequence of a workgroup's next segment, for a whole wavefront: `s` held the segment before, the range goes on at global block
+// `g` = that sequence's end < prefix[S].  Mostly the next one, its end one load away; empty sequences are passed over 64 at a time.
+// (A binary search was a chain of dependent loads, eight for 256 sequences, in every segment, the first
+// included: a step of 200 contexts of 300 took 57.2 us, now 54.5; 100 of 600 46.4, now 43.7.)
+__device__ __forceinline__ int akv_next_seq(const int32_t* __restrict__ prefix, int S, int s, int g, int& sb0, int& sb1) {
+  ++s;
+  sb0 = g;
+  sb1 = __builtin_amdgcn_readfirstlane(prefix[s + 1]);
+  if (sb1 <= g) {
+    int below;
+    do {
+      const int end = prefix[min(s + 1 + (int)(threadIdx.x & 63), S)];
+      below = __popcll(__ballot(end <= g));
+      if (below < 64) sb1 = __builtin_amdgcn_readlane(end, below);
+      s += below;
+    } while (below == 64);
   }
-  const int s = akv_find_seq(prefix, S, g);
-  sb0 = prefix[s];
-  sb1 = prefix[s + 1];
   return s;
 }
 

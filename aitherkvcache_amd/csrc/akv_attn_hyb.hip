@@ -717,24 +717,15 @@ __global__ __launch_bounds__(HW_W * 64, F::PER_SIMD) void akv_attn_hyb_kernel(hw
   const uint8_t* kbase = a.kc + (int64_t)hd * a.kps_head;
   const uint8_t* vbase = a.vc + (int64_t)hd * a.vps_head;
 
-  int gcur = g0;
+  int gcur = g0, s = s_first, sb0 = sb0_first, sb1 = sb1_first, ctx = ctx_first;
   while (gcur < g1) {
-    int s, sb0, sb1;
-    int64_t ctx;
-    if (gcur == g0 && s_first >= 0) {
-      s = s_first;
-      sb0 = sb0_first;
-      sb1 = sb1_first;
-      ctx = ctx_first;
-    } else {
-      s = __builtin_amdgcn_readfirstlane(akv_find_seq(a.prefix, a.S, gcur));
-      sb0 = a.prefix[s];
-      sb1 = a.prefix[s + 1];
-      ctx = akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq);
+    if (gcur != g0) {
+      s = akv_next_seq(a.prefix, a.S, s, gcur, sb0, sb1);
+      ctx = __builtin_amdgcn_readfirstlane((int)akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq));
     }
     const int blk_lo = gcur - sb0;
     const int blk_hi = min(g1, sb1) - sb0;
-    const int t_end = (int)min((int64_t)blk_hi * bs, ctx);
+    const int t_end = (int)min((int64_t)blk_hi * bs, (int64_t)ctx);
     gcur = sb0 + blk_hi;
     const int nblk = blk_hi - blk_lo;
     const int nchunks = bs32 ? nblk : (nblk + 1) >> 1;

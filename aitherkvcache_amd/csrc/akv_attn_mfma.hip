@@ -296,7 +296,7 @@ struct mf_vraw {       // value wavefront
 // (lane i: block blk_lo + i of the segment, clamped to the segment's last), fetched at the kernel's entry
 struct mf_start {
   int g0, g1;              // the workgroup's range of the global block axis
-  int s, sb0, sb1, ctx;    // first segment: sequence (-1: search the prefix), its first and one-past-last global block, its tokens
+  int s, sb0, sb1, ctx;    // first segment: sequence, its first and one-past-last global block, its tokens
   int pbwin;
   uint32_t lutw[6];        // the words of the workspace's table block this thread turns into table entries (mf_fill_tables)
 };
@@ -397,16 +397,13 @@ __device__ __forceinline__ void mf_role_main(const akv_attn_args& a, const akv_m
   // block, its second tile 16 positions further in.  bs32 is the same in every wavefront.
   const bool bs32 = a.block_size == 32;
   const int bs = bs32 ? 32 : 16;
-  // (the block prefix of the batch in a register, one entry per lane: finding a segment's sequence and its
-  // bounds costs no chain of dependent loads)
-  const int held = akv_prefix_hold(a.prefix, a.S);
   // the workgroup's range of the global block axis, as the prologue cut it (whole workgroups per sequence
   // when the batch has few sequences, equal ranges otherwise)
   const int g0 = st.g0, g1 = st.g1;
   // the window of block ids: lane i of pbwin holds the physical id of block (2 * win_c0 + i) of the segment
   // (win_c0 + i for blocks of 32).  `fresh`: it holds window 0 of the first segment, from the kernel's entry.
   int pbwin = st.pbwin, win_c0 = 0;
-  bool fresh = st.s >= 0;
+  bool fresh = true;
   const int gqa = a.QH / a.KVH;
   // The tables are written by all wavefronts of the workgroup once, AFTER each has requested what its first chunks
   // need: the fill (LDS stores from registers and the barrier that publishes them) then runs beside those round
@@ -420,24 +417,17 @@ __device__ __forceinline__ void mf_role_main(const akv_attn_args& a, const akv_m
     }
   };
 
-  int gcur = g0;
+  int gcur = g0, s = st.s, sb0 = st.sb0, sb1 = st.sb1, ctx = st.ctx;
   while (gcur < g1) {
     // the first segment starts from the workgroup's record (scalar loads that the kernel's entry has already
-    // brought in), later ones -- a range that crosses into the next sequence -- search the held prefix
-    int s, sb0, sb1;
-    int64_t ctx;
-    if (gcur == g0 && st.s >= 0) {
-      s = st.s;
-      sb0 = st.sb0;
-      sb1 = st.sb1;
-      ctx = st.ctx;
-    } else {
-      s = akv_find_seq_held(a.prefix, a.S, held, gcur, sb0, sb1);
-      ctx = akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq);
+    // brought in)
+    if (gcur != g0) {
+      s = akv_next_seq(a.prefix, a.S, s, gcur, sb0, sb1);
+      ctx = __builtin_amdgcn_readfirstlane((int)akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq));
     }
     const int blk_lo = gcur - sb0;
     const int blk_hi = min(g1, sb1) - sb0;
-    const int t_end = (int)min((int64_t)blk_hi * bs, ctx);
+    const int t_end = (int)min((int64_t)blk_hi * bs, (int64_t)ctx);
     gcur = sb0 + blk_hi;
     const int nblk = blk_hi - blk_lo;
     const int nchunks = bs32 ? nblk : (nblk + 1) >> 1;
@@ -962,7 +952,7 @@ __global__ __launch_bounds__(MF_THREADS) void akv_attn_mfma_kernel(akv_attn_args
     st.sb1 = rec[AKV_WGREC_SB1];
     st.ctx = rec[AKV_WGREC_CTX];
     st.pbwin = 0;
-    if (st.g0 < st.g1 && st.s >= 0) {
+    if (st.g0 < st.g1) {
       const int blk_lo = st.g0 - st.sb0, blk_hi = min(st.g1, st.sb1) - st.sb0;
       const int bi = min(blk_lo + (int)(threadIdx.x & 63), blk_hi - 1);
       st.pbwin = (int)akv_clamp_block(akv_load_index(a.block_tables, a.bt_itype, st.s * a.bt_stride + bi), a.num_blocks);

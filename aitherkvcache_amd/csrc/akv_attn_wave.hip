@@ -171,9 +171,6 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
   // memory; at 64 and 256 there are no registers left to hold its words until then (they would be spilled).
   constexpr int TPE = W * 64 / 256;                        // threads of an entry
   const float r0 = a.centroids[(threadIdx.x / TPE >> (BITS == 3 ? 3 : 4)) & ((1 << BITS) - 1)], r1 = a.centroids[threadIdx.x / TPE & ((1 << BITS) - 1)];
-  // block prefix of the batch, lane i: entry i * pstep, the first step of the search for a segment's sequence
-  const int pstep = a.S <= 63 ? 1 : (a.S + 64) / 64;
-  int pwin = a.prefix[min(lane * pstep, a.S)], pwin0 = pstep == 1 ? 0 : -1;
   float mx_c = 0.f;
   for (int v = 0; v < (1 << BITS); ++v) mx_c = fmaxf(mx_c, fabsf(a.centroids[v]));
   asm volatile("" : "+v"(mx_c) : "s"(g0), "s"(sb0_first));      // (the record and the codebook in one wait)
@@ -207,39 +204,15 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
   const int kb = PACK == 4 ? (lane >> 2) & 3 : (lane >> 3) & 1;     // which NV of a head's eight tokens
   const uint32_t nread = nbase + (uint32_t)g * 16u + (PACK == 4 ? 64u * (uint32_t)(kb >> 1) + 8u * (uint32_t)(kb & 1) : 64u * (uint32_t)kb);
 
-  int gcur = g0;
+  int gcur = g0, s = s_first, sb0 = sb0_first, sb1 = sb1_first, ctx = ctx_first;
   while (gcur < g1) {
-    int s, sb0, sb1;
-    int64_t ctx;
-    if (gcur == g0 && s_first >= 0) {
-      s = s_first;
-      sb0 = sb0_first;
-      sb1 = sb1_first;
-      ctx = ctx_first;
-    } else {
-      // the last s with prefix[s] <= gcur (below prefix[S]).  From 64 sequences on pwin first says in which stretch, then holds
-      // the 64 entries from pwin0 on, which mostly serve the next segments too.  (A binary search was eight dependent loads for
-      // 200 sequences, again in every segment.)
-      int below = __popcll(__ballot(pwin <= gcur));
-      if (pwin0 < 0) {
-        pwin0 = (below - 1) * pstep;
-        below = 64;
-      } else if (below == 64) {
-        pwin0 += 63;
-      }
-      while (below == 64) {
-        pwin = a.prefix[min(pwin0 + lane, a.S)];
-        below = __popcll(__ballot(pwin <= gcur));
-        if (below == 64) pwin0 += 63;
-      }
-      s = pwin0 + below - 1;
-      sb0 = __builtin_amdgcn_readlane(pwin, below - 1);
-      sb1 = __builtin_amdgcn_readlane(pwin, below);
-      ctx = akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq);
+    if (gcur != g0) {
+      s = akv_next_seq(a.prefix, a.S, s, gcur, sb0, sb1);
+      ctx = __builtin_amdgcn_readfirstlane((int)akv_seq_tokens(a.context_lens, a.cl_itype, s, bs, a.max_blocks_per_seq));
     }
     const int blk_lo = gcur - sb0;
     const int blk_hi = min(g1, sb1) - sb0;
-    const int t_end = (int)min((int64_t)blk_hi * bs, ctx);
+    const int t_end = (int)min((int64_t)blk_hi * bs, (int64_t)ctx);
     gcur = sb0 + blk_hi;
     const int nblk = blk_hi - blk_lo;
     const int nchunks = bs32 ? nblk : (nblk + 1) >> 1;

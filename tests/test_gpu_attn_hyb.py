@@ -195,3 +195,20 @@ def test_a_new_workspace_costs_little(dev, qh, kvh):
     later, first = least(False), least(True)
     print(f"[new workspace] {qh} on {kvh}: {first:.1f} us, later {later:.1f} us", flush=True)
     assert first < later + 120
+
+
+@pytest.mark.parametrize("mode,qh,kvh", [("tq35", 32, 8), ("tq25", 12, 2)])
+def test_many_sequences_and_empty_ones_vs_float64(dev, mode, qh, kvh):
+    """Runs of empty sequences longer than a wavefront's lanes, one sequence in most of the workgroups, many that share one."""
+    rng, h, rows = make(dev, mode, kvh, 40, 16, 64 if mode == "tq35" else 44, qh)
+    ctx = np.concatenate([np.zeros(100), [30000], np.zeros(130), rng.integers(1, 130, size=150), np.zeros(70), rng.integers(1, 40, size=5)]).astype(np.int32)
+    tables = rng.integers(0, 40, size=(len(ctx), 30000 // 16)).astype(np.int32)
+    K, V = (h.decode(r.contiguous()).double().cpu() for r in rows)
+    q = torch.from_numpy(rng.standard_normal((len(ctx), qh, 128)).astype(np.float32)).to(dev)
+    out = akv.HybridPagedAttention(h, qh).forward(q, rows[0], rows[1], torch.from_numpy(tables).to(dev), torch.from_numpy(ctx).to(dev)).double().cpu()
+    assert not out[torch.from_numpy(ctx == 0)].any()
+    for i in np.flatnonzero(ctx):
+        t = torch.from_numpy(tables[i, :-(-int(ctx[i]) // 16)].astype(np.int64))
+        k, v = (x[t].reshape(-1, kvh, 128)[:ctx[i]] for x in (K, V))
+        ref = attend(q[i].double().cpu(), k, v)
+        assert (out[i] - ref).norm() <= limit(mode, qh, kvh) * ref.norm(), (i, ctx[i])
