@@ -51,7 +51,12 @@ __global__ __launch_bounds__(256) void akv_attn_prologue_kernel(
 // Pi in registers across its items: with one workgroup per item a batch of 256 sequences x 32 heads
 // read the 64 KB matrix 4096 times (43 us for the kernel; 2048 items on 512 workgroups: see the host side).
 // ----------------------------------------------------------------------------------
-template <int D, int ODT>
+// AHEAD (head_dim 128, more items than workgroups: many sequences, each in a few slots): the partial results of a workgroup's next
+// item are requested before it rotates this one, and their places one item earlier still (256 sequences of 64 to 512 tokens, 32 heads:
+// the step 66.5 -> 63.8 us; stores of single outputs by sixteen lanes of a wavefront instead of pairs by all had their share in it).
+template <int ODT> struct red_pair { typedef uint32_t type; };
+template <> struct red_pair<AKV_F32> { typedef uint2 type; };
+template <int D, int ODT, bool AHEAD>
 __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
     const int32_t* __restrict__ prefix, const float* __restrict__ part_acc,
     const float* __restrict__ part_ml, const float* __restrict__ Pi, const uint4* __restrict__ bop, int S, int QH, int G,
@@ -79,39 +84,33 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
   }
   // a call marked as failed says so in every output
   const float poison = status[0] != 0u ? __uint_as_float(0x7fc00000u) : 0.f;
-  for (int item = blockIdx.x; item < S * groups; item += gridDim.x) {
-  const int s = item / groups, hg = item % groups;
-  const int h = hg * 4 + wave;
-  // workgroups of the main kernel whose ranges meet the sequence: from the record of the matrix-core
+  const bool pairs = (((uintptr_t)out / sizeof(typename akv_elem<ODT>::type) | (uintptr_t)os_seq | (uintptr_t)os_head) & 1) == 0;
+  // the first RED_PF partial accumulators are requested before anything is known about their
+  // weights, so that their round trip overlaps the one of the (max, sum) pairs
+  // (only slots that exist are read: a batch of many short sequences has one or two per head)
+  constexpr int RED_PF = AHEAD ? 8 : D == 128 ? 32 : 16;
+  float pre[RED_PF][DPL];
+  float2 ml0 = make_float2(-INFINITY, 0.f);      // lane u: slot w_lo + u
+  // workgroups of the main kernel whose ranges meet the item's sequence: from the record of the matrix-core
   // kernel's prologue (seqw), else from the equal cut of the block axis
-  int b0 = 0, b1 = 0, w_lo, w_hi;
-  if (seqw != nullptr) {
-    w_lo = seqw[2 * s];
-    w_hi = seqw[2 * s + 1];
-  } else {
-    b0 = prefix[s];
-    b1 = prefix[s + 1];
-    const int per = (prefix[S] + G - 1) / G;
-    w_lo = per > 0 ? b0 / per : 0;
-    w_hi = b1 > b0 ? (b1 - 1) / per : w_lo - 1;
-  }
-  if (w_hi < w_lo) {        // an empty sequence (the same for the whole workgroup)
-    if (h < QH) {
-#pragma unroll
-      for (int i = 0; i < DPL; ++i) akv_elem<ODT>::store(out, s * os_seq + h * os_head + lane * DPL + i, poison);
+  auto range = [&](int item, int& lo, int& hi) __attribute__((always_inline)) {
+    const int s = item / groups;
+    if (seqw != nullptr) {
+      lo = seqw[2 * s];
+      hi = seqw[2 * s + 1];
+    } else {
+      const int b0 = prefix[s], b1 = prefix[s + 1];
+      const int per = (prefix[S] + G - 1) / G;
+      lo = per > 0 ? b0 / per : 0;
+      hi = b1 > b0 ? (b1 - 1) / per : lo - 1;
     }
-    continue;
-  }
-  if (h < QH) {
-    // the first RED_PF partial accumulators are requested before anything is known about their
-    // weights, so that their round trip overlaps the one of the (max, sum) pairs
-    // (only slots that exist are read: a batch of many short sequences has one or two per head)
-    constexpr int RED_PF = D == 128 ? 32 : 16;
-    float pre[RED_PF][DPL];
+  };
+  auto request = [&](int item, int lo, int hi) __attribute__((always_inline)) {
+    const int s = item / groups, h = min(item % groups * 4 + wave, QH - 1);
 #pragma unroll
     for (int u = 0; u < RED_PF; ++u) {
-      if (w_lo + u <= w_hi) {
-        const size_t slot = (size_t)(w_lo + u + s) * QH + h;
+      if (lo + u <= hi) {
+        const size_t slot = (size_t)(lo + u + s) * QH + h;
 #pragma unroll
         for (int i = 0; i < DPL; ++i) pre[u][i] = part_acc[slot * D + lane * DPL + i];
       } else {
@@ -119,21 +118,38 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
         for (int i = 0; i < DPL; ++i) pre[u][i] = 0.f;
       }
     }
+    ml0 = make_float2(-INFINITY, 0.f);
+    if (lo + lane <= hi) ml0 = *(const float2*)(part_ml + ((size_t)(lo + lane + s) * QH + h) * 2);
+  };
+  const int items = S * groups;
+  int w_lo = 0, w_hi = -1;
+  if constexpr (AHEAD) {
+    range(blockIdx.x, w_lo, w_hi);
+    request(blockIdx.x, w_lo, w_hi);
+  }
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+  const int s = item / groups, hg = item % groups;
+  const int h = hg * 4 + wave;
+  int next_lo = 0, next_hi = -1;
+  if constexpr (AHEAD) {
+    range(min(item + (int)gridDim.x, items - 1), next_lo, next_hi);
+  } else {
+    range(item, w_lo, w_hi);
+    request(item, w_lo, w_hi);
+  }
+  {
     // lanes over slots: global max and sum; with at most 64 slots (the usual case) lane u keeps the
     // weight of slot w_lo + u and the second pass takes it from there
     const bool few = w_hi - w_lo < 64;
-    float M = -INFINITY, ms0 = -INFINITY, ls0 = 0.f;
-    for (int w = w_lo + lane; w <= w_hi; w += 64) {
-      const size_t slot = (size_t)(w + s) * QH + h;
-      const float2 ml = *(const float2*)(part_ml + slot * 2);
-      if (w < w_lo + 64) { ms0 = ml.x; ls0 = ml.y; }
-      M = fmaxf(M, ml.x);
-    }
+    const float ms0 = ml0.x, ls0 = ml0.y;
+    float M = ms0;
+    const int hc = min(h, QH - 1);       // (a group's heads past the last: that one again, not stored)
+    for (int w = w_lo + 64 + lane; w <= w_hi; w += 64) M = fmaxf(M, part_ml[((size_t)(w + s) * QH + hc) * 2]);
     M = akv_wave_max(M);
     const float wgt0 = ms0 > -INFINITY ? __expf(ms0 - M) : 0.f;
     float l = wgt0 * ls0;
     for (int w = w_lo + 64 + lane; w <= w_hi; w += 64) {
-      const size_t slot = (size_t)(w + s) * QH + h;
+      const size_t slot = (size_t)(w + s) * QH + hc;
       const float ms = part_ml[slot * 2];
       if (ms > -INFINITY) l += __expf(ms - M) * part_ml[slot * 2 + 1];
     }
@@ -154,7 +170,7 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
           const int w = min(w0 + u, w_hi);
-          const size_t slot = (size_t)(w + s) * QH + h;
+          const size_t slot = (size_t)(w + s) * QH + hc;
           const float wl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt0), w - w_lo));
           const float wgt = (w0 + u <= w_hi) ? wl : 0.f;
 #pragma unroll
@@ -164,7 +180,7 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
     } else {
 #pragma unroll 8
       for (int w = w_lo + RED_PF; w <= w_hi; ++w) {
-        const size_t slot = (size_t)(w + s) * QH + h;
+        const size_t slot = (size_t)(w + s) * QH + hc;
         const float ms = part_ml[slot * 2];
         const float wgt = ms > -INFINITY ? __expf(ms - M) : 0.f;
 #pragma unroll
@@ -174,11 +190,13 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
     const float inv = l > 0.f ? 1.f / l : 1.f;
 #pragma unroll
     for (int i = 0; i < DPL; ++i) a_lds[wave][lane * DPL + i] = acc[i] * inv;
-  } else {
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) a_lds[wave][lane * DPL + i] = 0.f;
   }
-  __syncthreads();
+  if constexpr (AHEAD) {
+    w_lo = next_lo;
+    w_hi = next_hi;
+    if (item + (int)gridDim.x < items) request(item + gridDim.x, w_lo, w_hi);
+  }
+  akv_lds_barrier();      // (the requests keep flying)
   if constexpr (D == 128) {
     // A operand: row r = head r % 4 of the item (rows 4..15 repeat them and are not used), contracted coordinates
     // 32 kg + 8 ks + e of the merged vector; result: lane (col, 0) holds heads 0..3 for output coordinates
@@ -207,14 +225,28 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
       acc[0] = akv_mfma3(hi, lo, bh[0][ks], bl[0][ks], acc[0]);
       acc[1] = akv_mfma3(hi, lo, bh[1][ks], bl[1][ks], acc[1]);
     }
+    // lane (col, kg) stores head kg (every fourth row of the tile is the same), two neighbouring coordinates at a time: one store
+    // of a wavefront in place of eight
     const float usc = akv_row_unscale(ex) * (1.f / 64.f);     // lane i < 4: the factor of head i
+    float y0 = acc[0][0], y1 = acc[1][0], uh = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(usc), 0));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 1; i < 4; ++i) {
       const float ui = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(usc), i));
-      const int hq = hg * 4 + i;
-      if (kg == 0 && hq < QH) {
-        akv_elem<ODT>::store(out, s * os_seq + hq * os_head + 8 * r + 2 * wave, acc[0][i] * ui + poison);
-        akv_elem<ODT>::store(out, s * os_seq + hq * os_head + 8 * r + 2 * wave + 1, acc[1][i] * ui + poison);
+      y0 = kg == i ? acc[0][i] : y0;
+      y1 = kg == i ? acc[1][i] : y1;
+      uh = kg == i ? ui : uh;
+    }
+    const int hq = hg * 4 + kg;
+    if (hq < QH) {
+      const int64_t o = s * os_seq + hq * os_head + 8 * r + 2 * wave;
+      union { typename akv_elem<ODT>::type e[2]; typename red_pair<ODT>::type w; } x;
+      akv_elem<ODT>::store(x.e, 0, y0 * uh + poison);
+      akv_elem<ODT>::store(x.e, 1, y1 * uh + poison);
+      if (pairs) {
+        *(typename red_pair<ODT>::type*)((char*)out + o * (int64_t)sizeof(x.e[0])) = x.w;
+      } else {
+        akv_elem<ODT>::store(out, o, y0 * uh + poison);
+        akv_elem<ODT>::store(out, o + 1, y1 * uh + poison);
       }
     }
   } else {
@@ -263,7 +295,7 @@ __global__ __launch_bounds__(256, 3) void akv_attn_reduce_kernel(
     if (hg * 4 + q < QH) akv_elem<ODT>::store(out, s * os_seq + (hg * 4 + q) * os_head + j, v + poison);
   }
   }
-  __syncthreads();       // the merged vectors are read until here; the next item overwrites them
+  akv_lds_barrier();     // the merged vectors are read until here; the next item overwrites them
   }
 }
 
@@ -645,11 +677,15 @@ static int akv_launch_reduce(int odt, const akv_attn_args& a, const float* Pi, c
   const int items = a.S * ((a.QH + 3) / 4);
   const int cus = akv_cached_cu_count();
   const int grid = items < 3 * (cus > 0 ? cus : 256) ? items : 3 * (cus > 0 ? cus : 256);
-  switch (odt) {
-    case AKV_F16: akv_attn_reduce_kernel<D, AKV_F16><<<grid, 256, 0, stream>>>(a.prefix, a.part_acc, a.part_ml, Pi, bop, a.S, a.QH, G, out, os_seq, os_head, status, seqw); break;
-    case AKV_BF16: akv_attn_reduce_kernel<D, AKV_BF16><<<grid, 256, 0, stream>>>(a.prefix, a.part_acc, a.part_ml, Pi, bop, a.S, a.QH, G, out, os_seq, os_head, status, seqw); break;
-    default: akv_attn_reduce_kernel<D, AKV_F32><<<grid, 256, 0, stream>>>(a.prefix, a.part_acc, a.part_ml, Pi, bop, a.S, a.QH, G, out, os_seq, os_head, status, seqw); break;
+#define AKV_RED(DT, A) akv_attn_reduce_kernel<D, DT, A><<<grid, 256, 0, stream>>>(a.prefix, a.part_acc, a.part_ml, Pi, bop, a.S, a.QH, G, out, os_seq, os_head, status, seqw)
+#define AKV_RED_T(A) do { if (odt == AKV_F16) AKV_RED(AKV_F16, A); else if (odt == AKV_BF16) AKV_RED(AKV_BF16, A); else AKV_RED(AKV_F32, A); } while (0)
+  if constexpr (D == 128) {
+    if (items > grid) AKV_RED_T(true); else AKV_RED_T(false);
+  } else {
+    AKV_RED_T(false);
   }
+#undef AKV_RED_T
+#undef AKV_RED
   AKV_LAUNCH_CHECK("akv_attn_reduce_kernel");
   return AKV_OK;
 }
