@@ -43,6 +43,7 @@ typedef _Float16 aw_half2 __attribute__((ext_vector_type(2)));
 typedef float aw_float2 __attribute__((ext_vector_type(2)));
 typedef float aw_float4 __attribute__((ext_vector_type(4)));
 typedef uint32_t aw_u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t aw_u32x3 __attribute__((ext_vector_type(3), aligned(4)));
 typedef uint32_t aw_u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const aw_u32x2 aw_lds_cu64;
 typedef __attribute__((address_space(3))) aw_u32x4 aw_lds_u128;
@@ -62,9 +63,14 @@ template <int D, int BITS> struct aw_cfg {
   static constexpr int W = D == 64 ? 16 : 8;            // wavefronts: what their registers admit on a CU
   static constexpr int CPL = D / 16;                    // coordinates per lane of a value tile = M-tiles
   static constexpr int KS = D / 16;                     // MFMA steps of a score tile (four coordinates a lane each)
-  static constexpr int KDW = BITS == 3 && D == 64 ? 2 : D * BITS / 128;   // dwords read for a quarter of a code row
-  static constexpr int VB = CPL * (BITS == 3 ? 4 : BITS) / 8;             // bytes of a lane's codes of one token (3 bits: spread to nibbles' room)
-  static constexpr int VDW = BITS == 3 ? 2 : VB >= 4 ? VB / 4 : 1;        // dwords (3 bits: the eight bytes around them)
+  // keys: a lane reads a quarter of a code row from both tiles of a chunk, or half of one from one tile (KHALF) where that is at
+  // most sixteen bytes, and half of it is handed on
+  static constexpr bool KHALF = D * BITS / 128 <= 2;
+  static constexpr int KDW = KHALF ? D * BITS / 64 : D * BITS / 128;      // dwords of a request
+  // values: VB bytes of codes of one token a lane (3 bits: spread to nibbles' room); a request takes twice that of one token, for
+  // the lane and the one eight lanes away
+  static constexpr int VB = CPL * (BITS == 3 ? 4 : BITS) / 8;
+  static constexpr int VRD = BITS == 3 ? (D == 256 ? 3 : 2) : VB >= 2 ? VB / 2 : 1;      // dwords of a request
 };
 // LDS: table | per wavefront: 32 key norms, 32 value norms, 32 exponents of those | per wavefront: (max, sum) of eight
 // heads | per wavefront: accumulators of its heads (merging only)
@@ -122,6 +128,36 @@ __device__ __forceinline__ uint32_t aw_here(uint32_t v) {
   asm volatile("" : "+v"(v));
   return v;
 }
+// N dwords that are aligned to four bytes
+template <int N, int M> __device__ __forceinline__ void aw_request(uint32_t (&r)[M], const unsigned char* p) {
+  static_assert(N <= M, "registers");
+  if constexpr (N >= 4) {
+    const uint4 t = *(const uint4*)p;
+    r[0] = t.x; r[1] = t.y; r[2] = t.z; r[3] = t.w;
+    if constexpr (N == 6) {
+      const uint2 u = *(const uint2*)(p + 16);
+      r[4] = u.x; r[5] = u.y;
+    }
+    if constexpr (N == 8) {
+      const uint4 u = *(const uint4*)(p + 16);
+      r[4] = u.x; r[5] = u.y; r[6] = u.z; r[7] = u.w;
+    }
+  } else if constexpr (N == 3) {
+    const aw_u32x3 t = *(const aw_u32x3*)p;
+    r[0] = t.x; r[1] = t.y; r[2] = t.z;
+  } else if constexpr (N == 2) {
+    const uint2 t = *(const uint2*)p;
+    r[0] = t.x; r[1] = t.y;
+  } else {
+    r[0] = *(const uint32_t*)p;
+  }
+}
+// What lanes 8 p + c of a row hold of one piece each, first and second half x and y of it, the piece of token p: the half p of both
+// tokens
+__device__ __forceinline__ void aw_trade(uint32_t x, uint32_t y, uint32_t& first, uint32_t& second) {
+  first = akv_dpp_banks_u<0x128 /*row_ror:8*/, 0xc>(x, y);
+  second = akv_dpp_banks_u<0x128 /*row_ror:8*/, 0x3>(y, x);
+}
 // 3-bit codes: a group of eight is a big-endian word of 24 bits.  Its four fields of two codes each, one per byte (the first
 // field in byte 3); and the same for two half groups of twelve bits in the halves of a word (first field in byte 1 and 3).
 __device__ __forceinline__ uint32_t aw_spread12(uint32_t x) { return ((x << 2) & 0x3F003F00u) | (x & 0x003F003Fu); }
@@ -150,7 +186,8 @@ __device__ __forceinline__ void aw_pair(aw_pairs<BITS, N>& p, uint32_t wa, uint3
 template <int D, int BITS, int PACK>
 __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(akv_attn_args a, aw_extra x) {
   typedef aw_cfg<D, BITS> cfg;
-  constexpr int W = cfg::W, CPL = cfg::CPL, KS = cfg::KS, KDW = cfg::KDW, VB = cfg::VB, VDW = cfg::VDW;
+  constexpr int W = cfg::W, CPL = cfg::CPL, KS = cfg::KS, KDW = cfg::KDW, VB = cfg::VB, VRD = cfg::VRD;
+  constexpr bool KHALF = cfg::KHALF;
   constexpr int CPB = BITS == 2 ? 4 : 2;                   // codes of a byte
   constexpr int NV = 8 / PACK;                             // tokens of a lane in the softmax
   // The dynamic LDS block is the kernel's only LDS object: its offsets are LDS addresses.
@@ -237,15 +274,18 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           pbwin = (int)akv_clamp_block(akv_load_index(a.block_tables, a.bt_itype, s * a.bt_stride + bi), a.num_blocks);
           win_k = k0;
         };
-        // 3 bits: a lane reads whole dwords around its codes; the selectors gather a group's three bytes, first byte on top
-        // (at head_dim 64 a lane of values has half a group: the two bytes with its twelve bits)
-        constexpr int GB = D == 64 ? 3 : 3 * D / 128;                   // bytes from one (pair of) lane's groups to the next's
-        const int vfirst = GB * (D == 64 ? col >> 1 : col), vdw = BITS != 3 ? 0 : min(vfirst >> 2, 3 * D / 32 - 2);
-        const uint32_t o3k = D == 64 ? 2u * (g & 1) : 0u, o3v = (uint32_t)(vfirst - 4 * vdw) + (D == 64 ? (uint32_t)(col & 1) : 0u);
-        const uint32_t ksel3 = 0x0c000102u + 0x010101u * o3k;
-        const uint32_t vsel3 = D == 64 ? 0x0c0c0001u + 0x0101u * o3v : 0x0c000102u + 0x010101u * o3v;
-        const uint32_t koff = (uint32_t)(hd * a.kps_head + col * a.kps_pos + (BITS == 3 ? (3 * D / 32 * g) & ~3 : KDW * 4 * g));
-        const uint32_t voff = (uint32_t)(hd * a.vps_head + 4 * g * a.vps_pos + (BITS == 3 ? 4 * vdw : VB * col));
+        // Few requests: with two of a quarter row a lane for keys and eight of the lane's own codes for values the address unit was
+        // busy for 80,000 of 99,000 cycles at head_dim 64, 43,000 of 64,000 at 256.  Decode steps: 48 sequences, one kv head of 128
+        // 35.1 -> 33.8 us, heads of 64 66.4 -> 65.2, of 256 in 2 bits 42.0 -> 40.2.
+        // Lane (8 p + c, g) reads piece c, of 2 VB bytes, of the first (p = 0) or second token of a pair and hands half of it on.
+        // 3 bits: whole dwords around the piece; the selectors gather a group's three bytes, first byte on top.
+        const int vp = col >> 3, vc = col & 7;
+        constexpr int GB = 3 * D / 64;                                  // bytes from one piece to the next (3 bits)
+        const int vdw = BITS != 3 ? 0 : min(GB * vc >> 2, 3 * D / 32 - VRD);
+        const uint32_t vsel3 = 0x0c000102u + 0x010101u * (uint32_t)(GB * vc - 4 * vdw);
+        const uint32_t koff = KHALF ? (uint32_t)(hd * a.kps_head + col * a.kps_pos + KDW * 4 * (g & 1))
+                                    : (uint32_t)(hd * a.kps_head + col * a.kps_pos + KDW * 4 * g);
+        const uint32_t voff = (uint32_t)(hd * a.vps_head + (4 * g + (VB >= 4 ? vp : 2 * vp)) * a.vps_pos + (BITS == 3 ? 4 * vdw : 2 * VB * vc));
         const uint32_t ktile1 = bs32 ? 16u * (uint32_t)a.kps_pos : 0u, vtile1 = bs32 ? 16u * (uint32_t)a.vps_pos : 0u;
         const int ntok = lane & 31, npos = bs32 ? ntok : ntok & 15;
         const float* nptr = lane >= 32 ? a.vn : a.kn;
@@ -255,7 +295,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
         // Codes and norms sit in one set of registers: the next chunk's keys are requested when this one's are scored, its
         // values when these are weighed (a second set made the compiler spill in the loop at head_dim 256 and move registers
         // elsewhere).
-        uint32_t kr[2][KDW], vr[8][VDW];
+        uint32_t kr[KHALF ? 1 : 2][KDW], vr[2][2][VRD];
         float nrm;
         auto blocks = [&](int k, uint32_t& pb0, uint32_t& pb1) {
           const int w = bs32 ? k - win_k : 2 * (k - win_k);
@@ -267,25 +307,14 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           blocks(k, pb[0], pb[1]);
           nrm = nptr[(uint64_t)(ntok >= 16 ? pb[1] : pb[0]) * nblk_stride + noff];
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const unsigned char* p = a.kp + (uint64_t)pb[j] * (uint32_t)a.kps_blk + (j ? ktile1 : 0u) + aw_here(koff);
-            if constexpr (KDW == 1) {
-              kr[j][0] = *(const uint32_t*)p;
-            } else if constexpr (KDW == 2 || KDW == 3 || KDW == 6) {
-              const uint2 t = *(const uint2*)(p + (KDW - 2) * 4);
-              kr[j][KDW - 2] = t.x; kr[j][KDW - 1] = t.y;
-              if constexpr (KDW == 3) kr[j][0] = *(const uint32_t*)p;
-              if constexpr (KDW == 6) {
-                const uint4 f = *(const uint4*)p;
-                kr[j][0] = f.x; kr[j][1] = f.y; kr[j][2] = f.z; kr[j][3] = f.w;
-              }
-            } else {
-#pragma unroll
-              for (int i = 0; i < KDW / 4; ++i) {
-                const uint4 t = *(const uint4*)(p + 16 * i);
-                kr[j][4 * i] = t.x; kr[j][4 * i + 1] = t.y; kr[j][4 * i + 2] = t.z; kr[j][4 * i + 3] = t.w;
-              }
+          for (int j = 0; j < (KHALF ? 1 : 2); ++j) {
+            const unsigned char* p = a.kp + (uint64_t)pb[j] * (uint32_t)a.kps_blk + (j ? ktile1 : 0u);
+            if constexpr (KHALF) {
+              const unsigned char* p1 = a.kp + (uint64_t)pb[1] * (uint32_t)a.kps_blk + ktile1;
+              p = g >= 2 ? p1 : p;
             }
+            p += aw_here(koff);
+            aw_request<KDW>(kr[j], p);
           }
         };
         auto load_values = [&](int k) {
@@ -295,18 +324,10 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           for (int j = 0; j < 2; ++j) {
             const unsigned char* vb = a.vp + (uint64_t)pb[j] * (uint32_t)a.vps_blk + (j ? vtile1 : 0u);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const unsigned char* p = vb + (uint32_t)(i * (int)a.vps_pos) + aw_here(voff);
-              if constexpr (BITS == 3) {
-                const uint2 t = *(const uint2*)p;
-                vr[4 * j + i][0] = t.x; vr[4 * j + i][VDW - 1] = t.y;
-              } else if constexpr (VB == 1) vr[4 * j + i][0] = *p;
-              else if constexpr (VB == 2) vr[4 * j + i][0] = *(const uint16_t*)p;
-              else if constexpr (VB == 4) vr[4 * j + i][0] = *(const uint32_t*)p;
-              else {
-                const uint2 t = *(const uint2*)p;
-                vr[4 * j + i][0] = t.x; vr[4 * j + i][VDW - 1] = t.y;
-              }
+            for (int q = 0; q < 2; ++q) {
+              const unsigned char* p = vb + (uint32_t)((VB >= 4 ? 2 * q : q) * (int)a.vps_pos) + aw_here(voff);
+              if constexpr (VB == 1 && BITS != 3) vr[j][q][0] = *(const uint16_t*)p;
+              else aw_request<VRD>(vr[j][q], p);
             }
           }
         };
@@ -316,7 +337,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
         load_values(0);
         uint2 qd[KS];
         {
-          const uint2* qp = x.qop + (size_t)(s * a.KVH + h) * (KS * 64) + lane;
+          const uint2* qp = x.qop + (size_t)(s * a.KVH + h) * (KS * 64) + (KHALF ? 16 * (g < 2 ? 2 * g : 2 * g - 3) + col : lane);      // the quarter the lane ends up with
 #pragma unroll
           for (int st = 0; st < KS; ++st) qd[st] = qp[st * 64];
         }
@@ -335,6 +356,35 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           akv_wave_sync();
 
           // ---- scores
+          // the words of both tiles: bytes (3 bits: groups of eight codes) of the lane's quarter of a row.  KHALF: lanes g < 2 hold half g of
+          // a row of tile 0, the others half g - 2 of one of tile 1; two pairs of rows of lanes trade a quarter.
+          constexpr int KW = BITS == 3 ? D / 32 : D * BITS / 128;
+          uint32_t kw[2][KW];
+#pragma unroll
+          for (int j = 0; j < (KHALF ? 1 : 2); ++j) {
+            constexpr int N = KHALF ? 2 * KW : KW;
+            uint32_t w[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+              // (3 bits: four groups in three dwords)
+              if constexpr (BITS == 3) {
+                const int b = 3 * (i & 3), at = 3 * (i >> 2) + b / 4;
+                w[i] = __builtin_amdgcn_perm(kr[j][min(at + 1, KDW - 1)], kr[j][at], 0x0c000102u + 0x010101u * (b % 4));
+              } else {
+                w[i] = kr[j][i];
+              }
+            }
+#pragma unroll
+            for (int i = 0; i < KW; ++i) {
+              if constexpr (KHALF) {
+                auto t = __builtin_amdgcn_permlane32_swap(w[i], w[KW + i], false, false);
+                kw[0][i] = t[0];
+                kw[1][i] = t[1];
+              } else {
+                kw[j][i] = w[i];
+              }
+            }
+          }
           aw_float4 acc[2];
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
@@ -343,25 +393,18 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
               const aw_u32x2 q0 = {qd[st].x, qd[st].x}, q1 = {qd[st].y, qd[st].y};
               acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(lo, hi), aw_operand(q0, q1), acc[j], 0, 0, 0);
             };
-            if constexpr (BITS == 3) {
 #pragma unroll
-              for (int i = 0; i < D / 32; ++i) {
-                // (four groups in three dwords; at head_dim 64 two in eight bytes)
-                const int b = D == 64 ? 3 * i : 3 * (i & 3), at = D == 64 ? 0 : 3 * (i >> 2) + b / 4;
-                const uint32_t up = kr[j][min(at + 1, KDW - 1)], sel = D == 64 ? ksel3 + 0x030303u * i : 0x0c000102u + 0x010101u * (b % 4);
-                const uint32_t w = aw_spread24(__builtin_amdgcn_perm(up, kr[j][at], sel));
+            for (int i = 0; i < KW; ++i) {
+              if constexpr (BITS == 3) {
+                const uint32_t w = aw_spread24(kw[j][i]);
                 step(2 * i, aw_look<3>(copy, w), aw_look<2>(copy, w));
                 step(2 * i + 1, aw_look<1>(copy, w), aw_look<0>(copy, w));
-              }
-            } else
-#pragma unroll
-            for (int i = 0; i < KDW; ++i) {
-              const uint32_t w = kr[j][i];
-              if constexpr (BITS == 4) {
+              } else if constexpr (BITS == 4) {
+                const uint32_t w = kw[j][i];
                 step(2 * i, aw_look<0>(copy, w), aw_look<1>(copy, w));
                 step(2 * i + 1, aw_look<2>(copy, w), aw_look<3>(copy, w));
               } else {
-                const uint32_t even = (w >> 2) & 0x33333333u, odd = w & 0x33333333u;
+                const uint32_t even = (kw[j][i] >> 2) & 0x33333333u, odd = kw[j][i] & 0x33333333u;
                 step(4 * i, aw_look<0>(copy, even), aw_look<0>(copy, odd));
                 step(4 * i + 1, aw_look<1>(copy, even), aw_look<1>(copy, odd));
                 step(4 * i + 2, aw_look<2>(copy, even), aw_look<2>(copy, odd));
@@ -482,15 +525,36 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           // ---- values
           if constexpr (VB >= 4) {
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < 2; ++j) {
+              constexpr int VW = VB / 4;
+              uint32_t word[4][VW];                  // of a tile's four tokens: words of codes (3 bits: of fields)
 #pragma unroll
-              for (int d = 0; d < VB / 4; ++d) {
+              for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int d = 0; d < VW; ++d) {
+                  const uint32_t(&r)[VRD] = vr[j][q];
+                  if constexpr (BITS != 3) {
+                    aw_trade(r[d], r[VW + d], word[2 * q][d], word[2 * q + 1][d]);
+                  } else {
+                    uint32_t x, y;
+                    if constexpr (D == 256) {        // four groups in three dwords
+                      auto group = [&](int i) { return __builtin_amdgcn_perm(r[min(3 * i / 4 + 1, 2)], r[3 * i / 4], 0x0c000102u + 0x010101u * (3 * i % 4)); };
+                      x = group(d);
+                      y = group(2 + d);
+                    } else {
+                      x = __builtin_amdgcn_perm(r[1], r[0], vsel3);
+                      y = __builtin_amdgcn_perm(r[1], r[0], vsel3 + 0x030303u);
+                    }
+                    aw_trade(x, y, word[2 * q][d], word[2 * q + 1][d]);
+                    word[2 * q][d] = aw_spread24(word[2 * q][d]);
+                    word[2 * q + 1][d] = aw_spread24(word[2 * q + 1][d]);
+                  }
+                }
+#pragma unroll
+              for (int d = 0; d < VW; ++d) {
                 aw_pairs<BITS, 0> p01, p23;
-                auto word = [&](int i) __attribute__((always_inline)) {
-                  return BITS == 3 ? aw_spread24(__builtin_amdgcn_perm(vr[4 * j + i][VDW - 1], vr[4 * j + i][0], vsel3 + 0x030303u * d)) : vr[4 * j + i][d];
-                };
-                aw_pair(p01, word(0), word(1));
-                aw_pair(p23, word(2), word(3));
+                aw_pair(p01, word[0][d], word[1][d]);
+                aw_pair(p23, word[2][d], word[3][d]);
                 auto byte = [&](auto kc) __attribute__((always_inline)) {
                   constexpr int K = decltype(kc)::value;
 #pragma unroll
@@ -502,16 +566,23 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
                 byte(std::integral_constant<int, 0>{}); byte(std::integral_constant<int, 1>{});
                 byte(std::integral_constant<int, 2>{}); byte(std::integral_constant<int, 3>{});
               }
+            }
           } else if constexpr (VB == 2) {
-            // two bytes per token: both token pairs of a tile side by side in one word
+            // two bytes per token: both token pairs of a tile side by side in one word (a request's pair: tokens two apart)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
               aw_pairs<BITS, 0> p;
-              auto word = [&](int i) __attribute__((always_inline)) {
-                if constexpr (BITS != 3) return vr[4 * j + i][0] | (vr[4 * j + i + 2][0] << 16);
-                const uint32_t x = __builtin_amdgcn_perm(vr[4 * j + i][VDW - 1], vr[4 * j + i][0], vsel3) |
-                                   __builtin_amdgcn_perm(vr[4 * j + i + 2][VDW - 1], vr[4 * j + i + 2][0], (vsel3 << 16) | 0x0c0cu);
-                return aw_spread12(x >> (col & 1 ? 0 : 4));
+              auto word = [&](int q) __attribute__((always_inline)) {
+                if constexpr (BITS != 3) {
+                  const uint32_t x = vr[j][q][0];
+                  const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128 /*row_ror:8*/, 0xf, 0xf, false);
+                  return __builtin_amdgcn_perm(y, x, vp ? 0x03020706u : 0x05040100u);
+                }
+                // the group of eight codes of both tokens, then twelve bits of each
+                const uint32_t x = __builtin_amdgcn_perm(vr[j][q][VRD - 1], vr[j][q][0], vsel3);
+                uint32_t t0, t1;
+                aw_trade(x, x, t0, t1);
+                return aw_spread12((t0 >> (vp ? 0 : 12) & 0xFFFu) | (t1 << (vp ? 16 : 4) & 0x0FFF0000u));
               };
               aw_pair(p, word(0), word(1));
               if constexpr (BITS == 3) {         // (the first field is the upper byte of a half)
@@ -530,7 +601,11 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           } else {
             // one byte per token: the pairs of both tiles side by side
             aw_pairs<BITS, 0> p;
-            auto join = [&](int t) { return vr[t][0] | (vr[t + 2][0] << 8) | (vr[t + 4][0] << 16) | (vr[t + 6][0] << 24); };
+            auto join = [&](int q) {
+              const uint32_t x = vr[0][q][0] | (vr[1][q][0] << 16);
+              const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128 /*row_ror:8*/, 0xf, 0xf, false);
+              return __builtin_amdgcn_perm(y, x, vp ? 0x03070105u : 0x06020400u);
+            };
             aw_pair(p, join(0), join(1));
 #pragma unroll
             for (int q = 0; q < CPB; ++q) {
@@ -549,7 +624,9 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
         fill_once();
       }
 
-      // ---- partial result: lane (col < gqa, g) holds coordinates CPL (4 g + i) + n of query head col
+      // ---- partial result: lane (col < gqa, g) holds rows 4 g + i of value tile n for query head col: coordinates o_at + 2 CPL i + n
+      // (row 8 p + c is half p of piece c)
+      const int o_at = CPL * (8 * (g & 1) + (g >> 1));
       const size_t slot = (size_t)(blockIdx.x + s) * a.QH + h * gqa;
       float M = m_run, wgt = inv_cs, L = l_run;
       const int shares = min(R, nchunks);      // wavefronts of the head that hold a result
@@ -590,17 +667,17 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int n = 0; n < CPL; n += 4)
-              *(float4*)(a.part_acc + (slot + col) * D + CPL * (4 * g + i) + n) = make_float4(o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]);
+              *(float4*)(a.part_acc + (slot + col) * D + o_at + 2 * CPL * i + n) = make_float4(o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]);
         }
       } else {
         const uint32_t wave_bytes = (uint32_t)gqa * D * 4u;
         if (active && r < shares && col < gqa) {
-          const uint32_t at = aw_acc_off<W>() + (uint32_t)wave * wave_bytes + (uint32_t)(col * D + CPL * 4 * g) * 4u;
+          const uint32_t at = aw_acc_off<W>() + (uint32_t)wave * wave_bytes + (uint32_t)(col * D + o_at) * 4u;
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int n = 0; n < CPL; n += 4)
-              *(aw_lds_f128*)(uintptr_t)(at + (uint32_t)(CPL * i + n) * 4u) = (aw_float4){o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]};
+              *(aw_lds_f128*)(uintptr_t)(at + (uint32_t)(2 * CPL * i + n) * 4u) = (aw_float4){o[n][i], o[n + 1][i], o[n + 2][i], o[n + 3][i]};
         }
         akv_lds_barrier();
         if (active) {
