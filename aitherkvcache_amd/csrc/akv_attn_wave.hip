@@ -152,6 +152,30 @@ template <int N, int M> __device__ __forceinline__ void aw_request(uint32_t (&r)
     r[0] = *(const uint32_t*)p;
   }
 }
+template <int I, int N, class F> __device__ __forceinline__ void aw_each_from(F& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    aw_each_from<I + 1, N>(f);
+  }
+}
+template <int N, class F> __device__ __forceinline__ void aw_each(F f) { aw_each_from<0, N>(f); }
+// N products of two look-ups each, the look-ups A products ahead.  Left to itself the compiler makes every product wait for
+// look-ups requested right before it, a trip to LDS each time (decode steps: 100 contexts of 200 to 1,000 with heads of 256 59.1 -> 55.5 us;
+// 2 bits 40.2 -> 38.5; one kv head of 128 33.8 -> 33.3; heads of 64 65.2 -> 64.6).
+template <int A, int N, class L, class M> __device__ __forceinline__ void aw_products(L look, M product) {
+  static_assert(A <= N, "look-ups ahead");
+  aw_u32x2 w[A][2];
+  auto first = [&](auto i) __attribute__((always_inline)) { look(i, w[i][0], w[i][1]); };
+  aw_each<A>(first);
+  __builtin_amdgcn_sched_barrier(0x6 /*vector and scalar arithmetic may pass*/);
+  auto one = [&](auto i) __attribute__((always_inline)) {
+    constexpr int I = decltype(i)::value;
+    product(i, aw_operand(w[I % A][0], w[I % A][1]));
+    if constexpr (I + A < N) look(std::integral_constant<int, I + A>{}, w[I % A][0], w[I % A][1]);
+    __builtin_amdgcn_sched_barrier(0x6);
+  };
+  aw_each<N>(one);
+}
 // What lanes 8 p + c of a row hold of one piece each, first and second half x and y of it, the piece of token p: the half p of both
 // tokens
 __device__ __forceinline__ void aw_trade(uint32_t x, uint32_t y, uint32_t& first, uint32_t& second) {
@@ -188,6 +212,7 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
   typedef aw_cfg<D, BITS> cfg;
   constexpr int W = cfg::W, CPL = cfg::CPL, KS = cfg::KS, KDW = cfg::KDW, VB = cfg::VB, VRD = cfg::VRD;
   constexpr bool KHALF = cfg::KHALF;
+  constexpr int AHEAD = D == 64 ? 3 : 4;                   // products whose look-ups are under way (at head_dim 64 there are no registers for four)
   constexpr int CPB = BITS == 2 ? 4 : 2;                   // codes of a byte
   constexpr int NV = 8 / PACK;                             // tokens of a lane in the softmax
   // The dynamic LDS block is the kernel's only LDS object: its offsets are LDS addresses.
@@ -385,33 +410,34 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
               }
             }
           }
-          aw_float4 acc[2];
+          if constexpr (BITS == 3) {
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            acc[j] = (aw_float4){0.f, 0.f, 0.f, 0.f};
-            auto step = [&](int st, aw_u32x2 lo, aw_u32x2 hi) {
-              const aw_u32x2 q0 = {qd[st].x, qd[st].x}, q1 = {qd[st].y, qd[st].y};
-              acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(lo, hi), aw_operand(q0, q1), acc[j], 0, 0, 0);
-            };
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int i = 0; i < KW; ++i) {
-              if constexpr (BITS == 3) {
-                const uint32_t w = aw_spread24(kw[j][i]);
-                step(2 * i, aw_look<3>(copy, w), aw_look<2>(copy, w));
-                step(2 * i + 1, aw_look<1>(copy, w), aw_look<0>(copy, w));
-              } else if constexpr (BITS == 4) {
-                const uint32_t w = kw[j][i];
-                step(2 * i, aw_look<0>(copy, w), aw_look<1>(copy, w));
-                step(2 * i + 1, aw_look<2>(copy, w), aw_look<3>(copy, w));
-              } else {
-                const uint32_t even = (kw[j][i] >> 2) & 0x33333333u, odd = kw[j][i] & 0x33333333u;
-                step(4 * i, aw_look<0>(copy, even), aw_look<0>(copy, odd));
-                step(4 * i + 1, aw_look<1>(copy, even), aw_look<1>(copy, odd));
-                step(4 * i + 2, aw_look<2>(copy, even), aw_look<2>(copy, odd));
-                step(4 * i + 3, aw_look<3>(copy, even), aw_look<3>(copy, odd));
-              }
-            }
+              for (int i = 0; i < KW; ++i) kw[j][i] = aw_spread24(kw[j][i]);
           }
+          aw_float4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+          // (the tiles take turns: two chains of sums)
+          aw_products<AHEAD, 2 * KS>(
+              [&](auto i, aw_u32x2& x, aw_u32x2& y) __attribute__((always_inline)) {
+                constexpr int I = decltype(i)::value, st = I / 2;
+                const uint32_t w = kw[I % 2][st / (KS / KW)];
+                if constexpr (BITS == 4) {
+                  x = aw_look<2 * (st & 1)>(copy, w);
+                  y = aw_look<2 * (st & 1) + 1>(copy, w);
+                } else if constexpr (BITS == 3) {
+                  x = aw_look<3 - 2 * (st & 1)>(copy, w);
+                  y = aw_look<2 - 2 * (st & 1)>(copy, w);
+                } else {
+                  x = aw_look<(st & 3)>(copy, (w >> 2) & 0x33333333u);
+                  y = aw_look<(st & 3)>(copy, w & 0x33333333u);
+                }
+              },
+              [&](auto i, aw_half8 op) __attribute__((always_inline)) {
+                constexpr int I = decltype(i)::value, st = I / 2;
+                const aw_u32x2 q0 = {qd[st].x, qd[st].x}, q1 = {qd[st].y, qd[st].y};
+                acc[I % 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op, aw_operand(q0, q1), acc[I % 2], 0, 0, 0);
+              });
 
           __builtin_amdgcn_sched_barrier(0);
           // (past the end: the last chunk once more, out of the window it is in)
@@ -550,28 +576,28 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
                     word[2 * q + 1][d] = aw_spread24(word[2 * q + 1][d]);
                   }
                 }
+              aw_pairs<BITS, 0> p01[VW], p23[VW];
 #pragma unroll
               for (int d = 0; d < VW; ++d) {
-                aw_pairs<BITS, 0> p01, p23;
-                aw_pair(p01, word[0][d], word[1][d]);
-                aw_pair(p23, word[2][d], word[3][d]);
-                auto byte = [&](auto kc) __attribute__((always_inline)) {
-                  constexpr int K = decltype(kc)::value;
-#pragma unroll
-                  for (int q = 0; q < CPB; ++q) {
-                    const int n = (4 * d + (BITS == 3 ? 3 - K : K)) * CPB + q;
-                    o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<K>(copy, p01.w[q]), aw_look<K>(copy, p23.w[q])), wop[j], o[n], 0, 0, 0);
-                  }
-                };
-                byte(std::integral_constant<int, 0>{}); byte(std::integral_constant<int, 1>{});
-                byte(std::integral_constant<int, 2>{}); byte(std::integral_constant<int, 3>{});
+                aw_pair(p01[d], word[0][d], word[1][d]);
+                aw_pair(p23[d], word[2][d], word[3][d]);
               }
+              aw_products<AHEAD, CPL>(
+                  [&](auto i, aw_u32x2& x, aw_u32x2& y) __attribute__((always_inline)) {
+                    constexpr int I = decltype(i)::value, q = I % CPB, K = I / CPB % 4, d = I / CPB / 4;
+                    x = aw_look<K>(copy, p01[d].w[q]);
+                    y = aw_look<K>(copy, p23[d].w[q]);
+                  },
+                  [&](auto i, aw_half8 op) __attribute__((always_inline)) {
+                    constexpr int I = decltype(i)::value, q = I % CPB, K = I / CPB % 4, d = I / CPB / 4, n = (4 * d + (BITS == 3 ? 3 - K : K)) * CPB + q;
+                    o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op, wop[j], o[n], 0, 0, 0);
+                  });
             }
           } else if constexpr (VB == 2) {
             // two bytes per token: both token pairs of a tile side by side in one word (a request's pair: tokens two apart)
+            aw_pairs<BITS, 0> p[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-              aw_pairs<BITS, 0> p;
               auto word = [&](int q) __attribute__((always_inline)) {
                 if constexpr (BITS != 3) {
                   const uint32_t x = vr[j][q][0];
@@ -584,20 +610,19 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
                 aw_trade(x, x, t0, t1);
                 return aw_spread12((t0 >> (vp ? 0 : 12) & 0xFFFu) | (t1 << (vp ? 16 : 4) & 0x0FFF0000u));
               };
-              aw_pair(p, word(0), word(1));
-              if constexpr (BITS == 3) {         // (the first field is the upper byte of a half)
-#pragma unroll
-                for (int q = 0; q < CPB; ++q) {
-                  o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<1>(copy, p.w[q]), aw_look<3>(copy, p.w[q])), wop[j], o[q], 0, 0, 0);
-                  o[CPB + q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<0>(copy, p.w[q]), aw_look<2>(copy, p.w[q])), wop[j], o[CPB + q], 0, 0, 0);
-                }
-              } else
-#pragma unroll
-              for (int q = 0; q < CPB; ++q) {
-                o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<0>(copy, p.w[q]), aw_look<2>(copy, p.w[q])), wop[j], o[q], 0, 0, 0);
-                o[CPB + q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<1>(copy, p.w[q]), aw_look<3>(copy, p.w[q])), wop[j], o[CPB + q], 0, 0, 0);
-              }
+              aw_pair(p[j], word(0), word(1));
             }
+            // (3 bits: the first field is the upper byte of a half)
+            aw_products<AHEAD, 2 * CPL>(
+                [&](auto i, aw_u32x2& x, aw_u32x2& y) __attribute__((always_inline)) {
+                  constexpr int I = decltype(i)::value, j = I / CPL, half = I / CPB % 2, K = BITS == 3 ? 1 - half : half;
+                  x = aw_look<K>(copy, p[j].w[I % CPB]);
+                  y = aw_look<K + 2>(copy, p[j].w[I % CPB]);
+                },
+                [&](auto i, aw_half8 op) __attribute__((always_inline)) {
+                  constexpr int I = decltype(i)::value;
+                  o[I % CPL] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op, wop[I / CPL], o[I % CPL], 0, 0, 0);
+                });
           } else {
             // one byte per token: the pairs of both tiles side by side
             aw_pairs<BITS, 0> p;
@@ -607,11 +632,16 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
               return __builtin_amdgcn_perm(y, x, vp ? 0x03070105u : 0x06020400u);
             };
             aw_pair(p, join(0), join(1));
-#pragma unroll
-            for (int q = 0; q < CPB; ++q) {
-              o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<0>(copy, p.w[q]), aw_look<1>(copy, p.w[q])), wop[0], o[q], 0, 0, 0);
-              o[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aw_operand(aw_look<2>(copy, p.w[q]), aw_look<3>(copy, p.w[q])), wop[1], o[q], 0, 0, 0);
-            }
+            aw_products<AHEAD, 2 * CPL>(
+                [&](auto i, aw_u32x2& x, aw_u32x2& y) __attribute__((always_inline)) {
+                  constexpr int I = decltype(i)::value, j = I / CPL;
+                  x = aw_look<2 * j>(copy, p.w[I % CPL]);
+                  y = aw_look<2 * j + 1>(copy, p.w[I % CPL]);
+                },
+                [&](auto i, aw_half8 op) __attribute__((always_inline)) {
+                  constexpr int I = decltype(i)::value;
+                  o[I % CPL] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op, wop[I / CPL], o[I % CPL], 0, 0, 0);
+                });
           }
           __builtin_amdgcn_sched_barrier(0);
           load_values(min(k + 1, mine - 1));
