@@ -827,13 +827,21 @@ __global__ __launch_bounds__(HW_W * 64, F::PER_SIMD) void akv_attn_hyb_kernel(hw
             }
         }
         // ---- running softmax in the log2 domain over t = score + exponent of the value factors
-        const float mx = akv_rows_max(akv_banks_max(fmaxf(tv[0], tv[1])));
-        // (the frame moves only when the maximum has outgrown it: moving the sums costs more than all of the softmax)
-        const float m_new = mx - HW_FRAME > m_run + HW_SLACK ? mx - HW_FRAME : m_run;
-        const float resc = __builtin_amdgcn_exp2f(m_run - m_new);      // 0 on the first chunk
-        m_run = m_new;
-        const float p0 = __builtin_amdgcn_exp2f(sv[0] - m_new), p1 = __builtin_amdgcn_exp2f(sv[1] - m_new);
-        l_run = l_run * resc + (p0 + p1);
+        // (the frame moves only when the maximum has outgrown it: moving the sums costs more than all of the softmax, and looking
+        // for the maximum over the lanes some 25 instructions: a step of 64 contexts of 4,000 to 8,192 168.1 -> 165.7 us)
+        if (__builtin_amdgcn_ballot_w64(tv[0] > m_run + (HW_FRAME + HW_SLACK) || tv[1] > m_run + (HW_FRAME + HW_SLACK)) != 0) {
+          const float mx = akv_rows_max(akv_banks_max(fmaxf(tv[0], tv[1])));
+          const float m_new = mx - HW_FRAME > m_run + HW_SLACK ? mx - HW_FRAME : m_run;
+          const float resc = __builtin_amdgcn_exp2f(m_run - m_new);      // 0 on the first chunk
+          m_run = m_new;
+          l_run *= resc;
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[n][i] *= resc;
+        }
+        const float p0 = __builtin_amdgcn_exp2f(sv[0] - m_run), p1 = __builtin_amdgcn_exp2f(sv[1] - m_run);
+        l_run += p0 + p1;
         // ---- weights of the four parts, two float16 terms each, in the same place: part, term, lane group, head, token pair.
         // Columns 0..3 read term 0, 4..7 term 1 (8..15 the same again, for nobody).
 #pragma unroll
@@ -852,12 +860,6 @@ __global__ __launch_bounds__(HW_W * 64, F::PER_SIMD) void akv_attn_hyb_kernel(hw
           const hw_int4 w = *(hw_lds_i128*)(uintptr_t)(wread + keys + 512u * x);
           return hw_operand((uint32_t)w[0], (uint32_t)w[1], (uint32_t)w[2], (uint32_t)w[3]);
         };
-        if (__builtin_amdgcn_ballot_w64(resc != 1.f) != 0) {
-#pragma unroll
-          for (int n = 0; n < NT; ++n)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[n][i] *= resc;
-        }
         __builtin_amdgcn_sched_barrier(0);
         f.values(keys, weights, o);
       }
