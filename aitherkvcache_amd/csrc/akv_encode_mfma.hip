@@ -31,6 +31,8 @@
 // row is short enough; if not, or if two boundaries share a cell or lie outside (-1, 1) (no such
 // codebook is produced by the library), the kernel counts all boundaries instead.
 //
+// (Above: the kernel of the largest calls.  Calls of up to some hundred vectors a CU keep the matrix in registers: akv_encode_rows_kernel.)
+//
 // A wavefront encodes EM_ROWS vectors per step (its M-tiles share every B operand read from LDS);
 // a workgroup is EM_WAVES independent wavefronts plus the B operand (64 KB) and the cell table.
 // Vector-unit and matrix-core time add up on a SIMD here (measured), so the search is kept to six
@@ -133,7 +135,7 @@ __device__ __forceinline__ uint32_t em_cell(float y) {
 }
 
 // MT: M-tiles (16 vectors each) per wavefront step -- MT, or 1 for float32 input
-// SPLIT (calls of a few thousand vectors, e.g. one serving step): a workgroup is eight wavefronts that share ONE
+// SPLIT (calls of up to two thousand vectors, e.g. one serving step): a workgroup is eight wavefronts that share ONE
 // step of 16 vectors, wavefront w computes N-tile w with its eighth of the B operand straight from memory in
 // registers -- no 64 KB fill, no cell table, one barrier; the codes meet in LDS and 256 threads pack and store
 // them.  Same products, same reciprocal, same comparison against the boundaries: the same codes.
@@ -681,6 +683,354 @@ __global__ __launch_bounds__(EM_THREADS) void akv_encode_mfma_kernel(akv_gen_arg
   }
 }
 
+#define ER_PER_CU 3               // workgroups: what their registers admit with four tiles of rows
+// workgroup barrier that orders LDS traffic only (what has been requested from memory keeps flying)
+__device__ __forceinline__ void er_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// ----------------------------------------------------------------------------------
+// encode with the matrix in registers: a workgroup is four wavefronts that share rows, wavefront w owns output coordinates
+// 32 w .. 32 w + 31 (two tiles of 16, both terms, 64 registers) and multiplies them into all rows of a step of 16 MT.  The threads
+// load the rows (128 / EPT lanes a row), take their norms and leave them in LDS as float16 terms, once for all wavefronts:
+//
+//   Y[j, v] = sum_i Pi[j, i] X[v, i]              v_mfma_f32_16x16x32_f16, Pi the first operand
+//
+// Row m of tile t is coordinate 32 w + 8 (m / 4) + 4 t + m % 4, so lane (v, g) ends up with coordinates 32 w + 8 g .. + 7 of row v:
+// one group of the packed row, stored from where it is.  One barrier a step: the rows of the next step go to the other half
+// of the buffer while this one's are multiplied, and those of the one after that are on their way.  The terms, their products and the
+// order of the sums are those of the kernel above.
+// ----------------------------------------------------------------------------------
+template <int XDT, int MT> struct er_cfg {
+  static constexpr int ROWS = 16 * MT, LPR = 16 / MT;             // rows of a step, lanes of a row while loading
+  static constexpr int NA = XDT == AKV_F32 ? 2 : 1, NP = MT * NA; // float16 terms of a row, 16-byte pieces of a thread
+  static constexpr int PITCH = 128 * 2 + 16;                      // bytes of a row in LDS (sixteen rows meet all banks)
+  static constexpr int BND = EM_CELLS * 8, DST = BND + 64, INFO = DST + 2 * ROWS * 8, DATA = INFO + 2 * ROWS * 4;
+  static constexpr int LDS = DATA + 2 * NA * ROWS * PITCH;
+};
+// floor((2^32 - 1) / heads) and / block size; slots of the cache.  (Products in 32 and 24 bits: er_fits.  In 64 bits they were a quarter
+// of a step's vector cycles.)
+struct er_div { uint32_t heads_r, block_r, slots; };
+
+template <int BITS, bool PAGED, int XDT, int MT>
+__global__ __launch_bounds__(256, ER_PER_CU) void akv_encode_rows_kernel(akv_gen_args a, const uint4* __restrict__ bop, er_div dv) {
+  extern __shared__ __align__(16) unsigned char lds[];            // the kernel's only LDS object: the cell table lies at address 0
+  typedef er_cfg<XDT, MT> cfg;
+  constexpr int ROWS = cfg::ROWS, LPR = cfg::LPR, NA = cfg::NA, NP = cfg::NP, PITCH = cfg::PITCH;
+  constexpr int XB = XDT == AKV_F32 ? 4 : 2, NB = (1 << BITS) - 1;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int row = tid / LPR, part = tid % LPR;
+  const uint32_t n_one = (uint32_t)a.n, n_total = PAGED && a.x2 ? 2u * n_one : n_one;
+  const uint32_t steps = (n_total + ROWS - 1) / ROWS, stride = gridDim.x;
+
+  // ---- rows of a step: thread (row, part) takes elements 8 MT part .. + 8 MT - 1
+  uint4 R[NP];
+  uint32_t tok = 0, head = 0;
+  bool second = false, held = false;
+  int64_t slot = 0;
+  auto fetch = [&](uint32_t step) {
+    uint32_t n = step * ROWS + row;
+    held = n < n_total;                                          // (past the end: the last row, not stored)
+    n = min(n, n_total - 1);
+    second = PAGED && n >= n_one;
+    if (second) n -= n_one;
+    tok = n;
+    if constexpr (PAGED) tok = akv_div32(n, (uint32_t)a.heads, dv.heads_r, head);
+    const uint64_t off = (uint64_t)tok * (uint32_t)a.xs0 + (PAGED ? __umul24(head, (uint32_t)a.xs1) : 0u);
+    const char* p = (const char*)(second ? a.x2 : a.x) + XB * off;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int h = 0; h < NA; ++h) R[i * NA + h] = *(const uint4*)(p + (part * MT + i) * 8 * XB + 16 * h);
+    if constexpr (PAGED) slot = akv_load_index(a.slots, a.slot_itype, tok);
+  };
+  uint32_t step = blockIdx.x;
+  fetch(step);
+
+  // ---- the wavefront's tiles of the matrix
+  em_half8 Ph[2][4], Pl[2][4];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      union { uint4 u; em_half8 h; } ch, cl;
+      const int at = ((4 * t + (col & 3)) * 4 + ks) * 64 + 16 * g + 4 * wave + (col >> 2);
+      ch.u = bop[at];
+      cl.u = bop[2048 + at];
+      Ph[t][ks] = ch.h;
+      Pl[t][ks] = cl.h;
+    }
+
+  // ---- cell table (as above; every thread judges the boundaries for itself)
+  bool linear;
+  {
+    float b[NB];
+    uint32_t cell[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) b[k] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(a.table[k])));
+    bool ok = fabsf(b[0]) < 1.f && fabsf(b[NB - 1]) < 1.f;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      cell[k] = __builtin_amdgcn_readfirstlane(em_cell(b[k]) >> 3);
+      if (k > 0) ok = ok && b[k] > b[k - 1] && cell[k] != cell[k - 1];
+    }
+    linear = !ok || ((const uint32_t*)(bop + EM_B_BYTES / 16))[0] != 0u;
+    if (tid == 0) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k) ((float*)(lds + cfg::BND))[k] = b[k];
+    }
+#pragma unroll
+    for (int c = tid; c < EM_CELLS; c += 256) {
+      uint32_t base = 0;
+      float inside = INFINITY;
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        base += cell[k] < (uint32_t)c ? 1u : 0u;
+        inside = cell[k] == (uint32_t)c ? b[k] : inside;
+      }
+      *(uint2*)(lds + 8 * c) = make_uint2(base, __float_as_uint(inside));
+    }
+  }
+
+  // ---- the rows held: norm, float16 terms into half `buf` of the buffer, where the packed row goes
+  auto convert = [&](int buf) {
+    // squared norm: a quarter of the row is one chain of sums, as above, which its 4 / MT lanes walk one after another
+    float ss = 0.f;
+#pragma unroll
+    for (int stage = 0; stage < 4 / MT; ++stage) {
+      if (stage > 0) ss = __uint_as_float(akv_dpp_u32<(MT == 1 ? 0x90 : 0xA0) /*the lane before: quad_perm 0,0,1,2 or 0,0,2,2*/>(__float_as_uint(ss)));
+      if (stage > 0 && part % (4 / MT) == 0) ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const uint32_t w[4] = {R[i].x, R[i].y, R[i].z, R[i].w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if constexpr (XDT == AKV_F16) {
+            union { uint32_t u; em_half2 h; } cv;
+            cv.u = w[q];
+            ss = __builtin_amdgcn_fdot2(cv.h, cv.h, ss, false);
+          } else if constexpr (XDT == AKV_BF16) {
+            const float e0 = __uint_as_float(w[q] << 16), e1 = __uint_as_float(w[q] & 0xffff0000u);
+            ss = fmaf(e0, e0, ss);
+            ss = fmaf(e1, e1, ss);
+          } else {
+            ss = fmaf(__uint_as_float(w[q]), __uint_as_float(w[q]), ss);
+          }
+        }
+      }
+    }
+    constexpr int LAST = 4 / MT - 1;                 // lanes part % (4 / MT) == LAST hold the sum of their quarter
+    ss += akv_lane_xor<4 / MT>(ss);
+    ss += akv_lane_xor<8 / MT>(ss);
+    uint32_t unscale = 0x3f800000u;
+    bool nonfinite = false;
+    uint4 hi[MT], lo[MT];
+    if constexpr (XDT == AKV_F16) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) hi[i] = R[i];
+    } else {
+      // scaled by the power of two of the largest element, as above
+      uint32_t ef;
+      if constexpr (XDT == AKV_BF16) {
+        em_us2 mx2 = {0, 0};
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const uint32_t w[4] = {R[i].x, R[i].y, R[i].z, R[i].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            union { uint32_t u; em_us2 v; } mm;
+            mm.u = w[q] & 0x7fff7fffu;
+            mx2 = __builtin_elementwise_max(mx2, mm.v);
+          }
+        }
+        ef = max((uint32_t)mx2[0], (uint32_t)mx2[1]) >> 7;
+      } else {
+        uint32_t mx = 0u;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+          const uint32_t w[4] = {R[i].x, R[i].y, R[i].z, R[i].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) mx = max(mx, w[q] & 0x7fffffffu);
+        }
+        ef = mx >> 23;
+      }
+      ef = max(ef, akv_lane_xor_u32<1>(ef));
+      ef = max(ef, akv_lane_xor_u32<2>(ef));
+      if constexpr (LPR >= 8) ef = max(ef, akv_lane_xor_u32<4>(ef));
+      if constexpr (LPR >= 16) ef = max(ef, akv_lane_xor_u32<8>(ef));
+      nonfinite = ef == 255u;
+      if (ef == 0u || ef == 255u) ef = 127u;       // all (sub)zero, or not finite (flagged)
+      if (ef == 254u) ef = 253u;                   // keep the scale a normal number
+      const float sc = __uint_as_float((254u - ef) << 23);
+      unscale = ef << 23;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        union { uint4 u; uint32_t w[4]; em_half2 h2[4]; } ph, pl;
+        if constexpr (XDT == AKV_BF16) {
+          const uint32_t w[4] = {R[i].x, R[i].y, R[i].z, R[i].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            auto pk = __builtin_amdgcn_cvt_pkrtz(__uint_as_float(w[q] << 16) * sc, __uint_as_float(w[q] & 0xffff0000u) * sc);
+            ph.h2[q] = (em_half2){(_Float16)pk[0], (_Float16)pk[1]};
+          }
+        } else {
+          const uint32_t w[8] = {R[2 * i].x, R[2 * i].y, R[2 * i].z, R[2 * i].w, R[2 * i + NA - 1].x, R[2 * i + NA - 1].y, R[2 * i + NA - 1].z, R[2 * i + NA - 1].w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float x0 = __uint_as_float(w[2 * q]) * sc, x1 = __uint_as_float(w[2 * q + 1]) * sc;
+            const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
+            ph.h2[q] = (em_half2){h0, h1};
+            pl.h2[q] = (em_half2){(_Float16)(x0 - (float)h0), (_Float16)(x1 - (float)h1)};
+          }
+          lo[i] = pl.u;
+        }
+        hi[i] = ph.u;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      unsigned char* p = lds + cfg::DATA + (buf * NA * ROWS + row) * PITCH + (part * MT + i) * 16;
+      *(uint4*)p = hi[i];
+      if constexpr (NA == 2) *(uint4*)(p + ROWS * PITCH) = lo[i];
+    }
+    const float nrm = sqrtf(ss);
+    const float r = (1.f / (nrm + 1e-10f)) * (1.f / EM_PSCALE) * __uint_as_float(unscale);
+    const bool nan_row = XDT == AKV_F16 ? !(nrm < INFINITY) : (nonfinite || nrm != nrm);
+    // ---- where the row goes
+    uint8_t* pb = second ? a.packed2 : a.packed;
+    float* nb = second ? a.norms2 : a.norms;
+    bool stored = held;
+    if constexpr (PAGED) {
+      stored = held && (uint64_t)slot < dv.slots;
+      uint32_t pos;
+      const uint32_t blk = akv_div32((uint32_t)slot, (uint32_t)a.block_size, dv.block_r, pos);
+      pb += (uint64_t)blk * (uint32_t)a.ps0 + (__umul24(pos, (uint32_t)a.ps1) + __umul24(head, (uint32_t)a.ps2));
+      nb += (uint64_t)blk * (uint32_t)a.ns0 + (__umul24(pos, (uint32_t)a.ns1) + __umul24(head, (uint32_t)a.ns2));
+    } else {
+      pb += (uint64_t)tok * (uint32_t)a.ps0;
+      nb += tok;
+    }
+    if (part == LAST) {
+      ((uint64_t*)(lds + cfg::DST))[buf * ROWS + row] = stored ? (uint64_t)(uintptr_t)pb : 0u;
+      ((float*)(lds + cfg::INFO))[buf * ROWS + row] = nan_row ? __uint_as_float(0x7fc00000u) : r;
+      if (stored) *nb = nrm;
+    }
+  };
+
+  // ---- rotate, search, pack, store
+  auto encode = [&](auto linear_tag, int buf) {
+    constexpr bool LINEAR = decltype(linear_tag)::value;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const int v = buf * ROWS + 16 * mt + col;
+      em_float4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      const unsigned char* p = lds + cfg::DATA + (buf * NA * ROWS + 16 * mt + col) * PITCH + 64 * g;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const em_half8 x = *(const em_half8*)(p + 16 * ks);
+        em_half8 xl;
+        if constexpr (NA == 2) xl = *(const em_half8*)(p + ROWS * PITCH + 16 * ks);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ph[t][ks], x, acc[t], 0, 0, 0);
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Pl[t][ks], x, acc[t], 0, 0, 0);
+          if constexpr (NA == 2) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ph[t][ks], xl, acc[t], 0, 0, 0);
+        }
+      }
+      const float r = ((const float*)(lds + cfg::INFO))[v];
+      const uint64_t dp = ((const uint64_t*)(lds + cfg::DST))[v];
+      float y[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) y[k] = acc[k >> 2][k & 3] * r;
+      uint32_t code[8];
+      if constexpr (!LINEAR) {
+        em_u32x2 e[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) e[k] = *(em_lds_u64*)(uintptr_t)em_cell(y[k]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) code[k] = e[k].x + (__uint_as_float(e[k].y) < y[k] ? 1u : 0u);
+      } else {
+        const float* bnd = (const float*)(lds + cfg::BND);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          code[k] = 0;
+#pragma unroll 1
+          for (int b = 0; b < NB; ++b) code[k] += bnd[b] < y[k] ? 1u : 0u;
+        }
+      }
+      // the group by shift and add, its codes in the order in which they enter it from the top
+      uint32_t w = 0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) w = (w << BITS) + code[BITS == 4 ? 6 - (k & ~1) + (k & 1) : BITS == 3 ? k : ((k + 4) & 7)];
+      if (!(r == r)) w = 0xffffffffu;                // NaN vector: last level everywhere
+      if (dp != 0) {
+        uint8_t* q = (uint8_t*)(uintptr_t)dp + BITS * (4 * wave + g);
+        if constexpr (BITS == 4) {
+          *(uint32_t*)q = w;
+        } else if constexpr (BITS == 3) {
+          q[0] = (uint8_t)(w >> 16);
+          q[1] = (uint8_t)(w >> 8);
+          q[2] = (uint8_t)w;
+        } else {
+          *(uint16_t*)q = (uint16_t)w;
+        }
+      }
+    }
+  };
+
+  convert(0);
+  if (step + stride < steps) fetch(step + stride);
+  __syncthreads();
+  auto all = [&](auto linear_tag) __attribute__((always_inline)) {
+    for (int buf = 0; step < steps; step += stride, buf ^= 1) {
+      if (step + stride < steps) {
+        convert(buf ^ 1);                            // (that half was read before the barrier)
+        if (step + 2 * stride < steps) fetch(step + 2 * stride);
+      }
+      encode(linear_tag, buf);
+      er_barrier();
+    }
+  };
+  if (__builtin_expect(!linear, 1)) all(std::false_type{});
+  else all(std::true_type{});
+}
+
+// what the kernel's 32- and 24-bit products take
+static bool er_fits(const akv_gen_args& a, bool paged, int64_t n_total) {
+  auto below = [](int64_t v, int bits) { return v >= 0 && v < ((int64_t)1 << bits); };
+  if (!below(n_total, 31) || !below(a.xs0, 32) || !below(a.ps0, 32)) return false;
+  if (!paged) return true;
+  return below(a.max_blocks, 31) && below(a.block_size, 24) && a.max_blocks * a.block_size < ((int64_t)1 << 31) && below(a.heads, 24) && below(a.ns0, 32) &&
+         below(a.xs1, 24) && below(a.ps1, 24) && below(a.ps2, 24) && below(a.ns1, 24) && below(a.ns2, 24) && below(a.heads * a.xs1, 32) &&
+         below(a.block_size * a.ps1 + a.heads * a.ps2, 32) && below(a.block_size * a.ns1 + a.heads * a.ns2, 32);
+}
+
+template <int BITS, bool PAGED, int XDT, int MT>
+static int er_launch(const akv_gen_args& a, const uint4* bop, const er_div& dv, int grid, hipStream_t stream) {
+  AKV_LAUNCH_TIMED((akv_encode_rows_kernel<BITS, PAGED, XDT, MT>), grid, 256, (er_cfg<XDT, MT>::LDS), stream, a, bop, dv);
+  AKV_LAUNCH_CHECK("akv_encode_rows_kernel");
+  return AKV_OK;
+}
+template <int BITS, bool PAGED, int XDT>
+static int er_run_rows(const akv_gen_args& a, const uint4* bop, int64_t n, int cus, hipStream_t stream) {
+  er_div dv = {0u, 0u, 0u};
+  if constexpr (PAGED) dv = {0xffffffffu / (uint32_t)a.heads, 0xffffffffu / (uint32_t)a.block_size, (uint32_t)(a.max_blocks * a.block_size)};
+  const int tiles = n <= 16 * (int64_t)cus ? 1 : XDT == AKV_F32 || n <= 32 * (int64_t)cus ? 2 : 4;
+  const int64_t steps = (n + 16 * tiles - 1) / (16 * tiles), most = ER_PER_CU * (int64_t)cus;
+  const int grid = (int)(steps < most ? steps : most);
+  if (tiles == 1) return er_launch<BITS, PAGED, XDT, 1>(a, bop, dv, grid, stream);
+  if constexpr (XDT != AKV_F32)
+    if (tiles == 4) return er_launch<BITS, PAGED, XDT, 4>(a, bop, dv, grid, stream);
+  return er_launch<BITS, PAGED, XDT, 2>(a, bop, dv, grid, stream);
+}
+static int er_run(const akv_gen_args& a, bool paged, int x_dtype, int bits, const uint4* bop, int64_t n, int cus, hipStream_t stream) {
+#define ER_DT(BB, PG) (x_dtype == AKV_F16 ? er_run_rows<BB, PG, AKV_F16>(a, bop, n, cus, stream) : x_dtype == AKV_BF16 ? er_run_rows<BB, PG, AKV_BF16>(a, bop, n, cus, stream) \
+                                                                                                : er_run_rows<BB, PG, AKV_F32>(a, bop, n, cus, stream))
+  if (bits == 4) return paged ? ER_DT(4, true) : ER_DT(4, false);
+  if (bits == 3) return paged ? ER_DT(3, true) : ER_DT(3, false);
+  return paged ? ER_DT(2, true) : ER_DT(2, false);
+#undef ER_DT
+}
+
 // the split form exists for 16-bit rows addressed row by row; returns false where it does not
 template <int BB, bool PG, int DT, bool DR>
 static bool em_launch_split(int grid, hipStream_t stream, const akv_gen_args& a, const uint4* bop) {
@@ -713,14 +1063,20 @@ int akv_encode_mfma_try(const akv_gen_args& a, bool paged, int x_dtype, int d, i
   const uint4* bop = (const uint4*)((const float*)rot_prep + (size_t)2 * d * d);
   const int64_t n_total = (paged && a.x2) ? 2 * a.n : a.n;
   const int cus = akv_cached_cu_count();
-  // A call too small to give every CU a step of 32 vectors (one serving step: 4,096 vectors) runs the form with 16
-  // vectors per wavefront step: twice the workgroups, half the chain of products and searches that its one busy
-  // wavefront per workgroup walks through alone.
-  const bool narrow = paged && x_dtype != AKV_F32 && (n_total + EM_ROWS - 1) / EM_ROWS < cus;
-  // ... and one (paged or flat) that leaves a workgroup at most two steps of 16 vectors shares each step among
-  // eight wavefronts
-  const bool split = x_dtype != AKV_F32 && (n_total + 15) / 16 <= 2 * (int64_t)cus && !getenv("AKV_ENCODE_NO_SPLIT");
-  const int rows_per_step = (x_dtype == AKV_F32 || narrow || split) ? 16 : EM_ROWS;
+  // Calls of up to some hundred vectors a CU take the kernel with the matrix in registers: no 64 KB fill, and a wavefront's chain
+  // is a quarter of a row's tiles.  Steps of 16, 32 or 64 rows, so that the calls that give a CU one step have it on every CU.
+  // Keys and values in bfloat16 and 4 bits, us, the kernel above | that one: 8,192 vectors 8.5 | 5.8, 16,384 9.3 | 6.9, 32,768
+  // 10.1 | 8.9, 65,536 13.4 | 12.7, 131,072 20.8 | 19.1; but 192,000 24.8 | 25.6, and rows that fill its workgroups with two steps
+  // each, 88,000 to 98,304, 16.3 to 17.0 | 16.8 to 17.2.  Float16, no conversion to share: 32,768 9.4 | 8.6, but 48,000 11.6 | 11.7,
+  // 80,000 14.2 | 14.7; flat rows, of which that kernel checks none, 65,536 11.4 | 12.2.  3 bits, three stores of a byte: 32,768 8.9 | 8.4, 48,000 11.3 | 11.3, 65,536 12.6 | 12.8.  Float32: 1,600
+  // 7.8 | 5.2, 16,384 8.9 | 8.0, 20,320 10.5 | 10.4, 32,768 11.9 | 12.2.
+  // The fewest share each step of 16 vectors among eight wavefronts: 2,048 vectors 5.0 | 5.2, 4,096 5.4 | 5.2.
+  const int64_t per_cu = n_total / cus;
+  const bool plain = getenv("AKV_ENCODE_NO_SPLIT") != nullptr;
+  const bool split = x_dtype != AKV_F32 && n_total <= 8 * (int64_t)cus && !plain;
+  const bool rows = x_dtype == AKV_F32 ? per_cu <= 80 : bits == 3 ? per_cu <= 128 : x_dtype == AKV_F16 || !paged ? per_cu <= 160 : per_cu < 340 || (per_cu > 384 && per_cu <= 512);
+  if (rows && !split && !plain && er_fits(a, paged, n_total)) return er_run(a, paged, x_dtype, bits, bop, n_total, cus, stream);
+  const int rows_per_step = (x_dtype == AKV_F32 || split) ? 16 : EM_ROWS;
   const int64_t steps = (n_total + rows_per_step - 1) / rows_per_step;
   // steps are dealt round-robin over workgroups first, so a small call (one serving step) spreads
   // over as many CUs as it has steps instead of filling the wavefronts of a few
@@ -738,8 +1094,7 @@ int akv_encode_mfma_try(const akv_gen_args& a, bool paged, int x_dtype, int d, i
 #define EM_LAUNCH(BB, PG, DT, DR)                                                                     \
   do {                                                                                               \
     if (split && em_launch_split<BB, PG, DT, DR>(grid, stream, a, bop)) break;                       \
-    if (DT == AKV_F32 || (PG && narrow)) EM_LAUNCH_MT(BB, PG, DT, DR, 1);                             \
-    else EM_LAUNCH_MT(BB, PG, DT, DR, (DT == AKV_F32 ? 1 : EM_MT));                                   \
+    EM_LAUNCH_MT(BB, PG, DT, DR, (DT == AKV_F32 ? 1 : EM_MT));                                        \
   } while (0)
 #define EM_LAUNCH_DT(BB, PG, DR) do { if (x_dtype == AKV_F16) EM_LAUNCH(BB, PG, AKV_F16, DR); else if (x_dtype == AKV_BF16) EM_LAUNCH(BB, PG, AKV_BF16, DR); else EM_LAUNCH(BB, PG, AKV_F32, DR); } while (0)
   // flat rows whose byte offsets stay below 2^31 take the variant with 32-bit lane offsets

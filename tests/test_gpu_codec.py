@@ -684,3 +684,54 @@ def test_read_probe_sums_what_it_reads(dev):
     with pytest.raises(ValueError):
         _lib.check(L.akv_debug_read_probe(0, 16, sink.data_ptr(), _lib.stream_ptr(dev)))
 
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,H,BS", [(257, 8, 16), (585, 7, 24), (293, 28, 32), (7100, 7, 16)])
+def test_calls_of_some_hundred_rows_a_cu_write_the_bytes_of_the_large_ones(golden, dev, bits, dtype, T, H, BS, monkeypatch):
+    """Keys and values through the kernel with the matrix in registers -- steps of 16, 32 and 64 rows, a last step of a few, one step
+    a workgroup and several, heads and block sizes that are no powers of two -- and through the one with the matrix in LDS:
+    codes, norms and untouched rows byte for byte, with NaN, infinite and zero rows and slots outside the cache."""
+    tq = make_tq(golden, dev, bits)
+    P = tq._packed_dim
+    NB = -(-T // BS) + 1
+    rng = np.random.default_rng(900 + bits + T)
+    xs = []
+    for _ in range(2):
+        x = kv_like(rng, (T, H, 128)).astype(np.float32)
+        x[3, 1, 5], x[4, 2, 7], x[5, 0] = np.nan, np.inf, 0
+        xs.append(torch.from_numpy(x).to(dev).to(dtype))
+    slots = rng.permutation(NB * BS)[:T].astype(np.int64)
+    slots[::9], slots[1::11] = -1, NB * BS + 5
+    sd = torch.from_numpy(slots).to(dev)
+    outs = []
+    for off in ("", "1"):
+        monkeypatch.delenv("AKV_ENCODE_NO_SPLIT", raising=False)
+        if off:
+            monkeypatch.setenv("AKV_ENCODE_NO_SPLIT", "1")
+        rows = [torch.full((NB, BS, H, P + 4), 0xAB, dtype=torch.uint8, device=dev) for _ in range(2)]
+        norms = [torch.full((NB, BS, H), -5.0, device=dev) for _ in range(2)]
+        akv.fused_kv_update_pair(xs[0], xs[1], sd, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], tq.rotation, tq.boundaries_inner, bits, block_size=BS)
+        flat = tq.encode(xs[0].reshape(-1, 128))
+        outs.append([t.cpu().numpy() for t in (*rows, *norms, *flat)])
+    monkeypatch.delenv("AKV_ENCODE_NO_SPLIT", raising=False)
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b, equal_nan=a.dtype != np.uint8)
+    ok = (slots >= 0) & (slots < NB * BS)
+    assert int(np.sum(outs[0][2] != -5.0)) == int(ok.sum()) * H
+
+
+def test_encode_rows_far_apart(golden, dev, monkeypatch):
+    """Positions of a block further apart than 24 bits hold: the call keeps to 64-bit offsets and writes the same bytes."""
+    tq = make_tq(golden, dev, 4)
+    P, H, T = tq._packed_dim, 2, 1100
+    x = torch.from_numpy(kv_like(np.random.default_rng(41), (T, H, 128))).to(dev)
+    slots = torch.full((T,), -1, dtype=torch.int64, device=dev)
+    slots[:16] = torch.arange(16, device=dev).flip(0)
+    far = torch.zeros(4 * 4 * ((1 << 24) + 64), dtype=torch.uint8, device=dev).as_strided((4, 4, H, P), (4 * ((1 << 24) + 64), (1 << 24) + 64, P, 1))
+    near = torch.zeros(4, 4, H, P, dtype=torch.uint8, device=dev)
+    norms = [torch.zeros(4, 4, H, device=dev) for _ in range(2)]
+    for rows, n in zip((far, near), norms):
+        akv.fused_kv_update(x, slots, rows, n, tq.rotation, tq.boundaries_inner, 4, 4)
+    assert torch.equal(far.contiguous(), near) and torch.equal(*norms) and bool(near.any())
