@@ -6,9 +6,11 @@
 //         scaled by 64), in the order its lanes take them from the prepared-rotation buffer (akv_dm_slices_kernel).  D / C
 //         wavefronts share a row.
 //     B = centroids of the codes: lane (v = l % 16, g = l / 16) loads quarter g of the packed row of vector v.  A code
-//         BYTE (two codes) indexes a table in LDS whose 8-byte entry is the float16 pair (c[a], c[b]) and the pair of
-//         remainders (c = hi + lo to ~22 bits); every entry is replicated 32 times (address = byte * 256 + (lane & 31) * 8,
-//         built by one byte permute), so look-ups do not conflict on a bank.
+//         BYTE (two codes) indexes a table in LDS whose entry is the float16 pair (c[a], c[b]), 32 times, and the pair of
+//         remainders (c = hi + lo to ~22 bits), 32 times (address = byte * 256 + (lane & 31) * 4, built by one byte permute, and
+//         128 bytes on), so look-ups do not conflict on a bank.  Both by one request of eight bytes, they landed side by side and were
+//         moved to their operands, 64 of some 360 vector instructions of a step (K and V of 20k tokens x 8 heads at head_dim 128:
+//         37.8 -> 36.7 us, 3 bits 38.9 -> 37.5, head_dim 256 68.2 -> 66.3; look-ups a piece ahead of the products 37.0, 38.4, 67.0).
 //     Three products per tile: Pi_hi c_hi + Pi_hi c_lo + Pi_lo c_hi.
 //   The rows of an A tile are permuted so that a lane ends up with eight neighbouring coordinates of ONE row from two tiles:
 //   it needs one norm and one address per vector, and the four lanes of a vector write 64 neighbouring bytes per store.
@@ -16,7 +18,7 @@
 // 3-bit and 2-bit rows are spread to one code per nibble in registers (akv_nibble.h) and take the same table; the
 // coordinate order that the spreading leaves is matched when the matrix is loaded.
 //
-// What bounds it: the loop, 48 products of 16 cycles and some 430 vector instructions of four per 16 rows of head_dim 128
+// What bounds it: the loop, 48 products of 16 cycles and some 150 vector instructions of four per 16 rows of head_dim 128
 // and wavefront at two wavefronts a SIMD, and the trips to memory around it.
 // Flat rows at head_dim 128 (us; the matrix in LDS, 64 KB read per 32 rows | split from the float32 matrix in every launch |
 // as it is now): 4-bit to float16, 4,096 rows 10.2 | 9.5 | 5.9, 65,536 rows 14.6 | 16.9 | 13.1, 2^20 rows 110 | 110 | 105; 3-bit
@@ -35,7 +37,7 @@ typedef _Float16 dm_half2 __attribute__((ext_vector_type(2)));
 typedef __bf16 dm_bf162 __attribute__((ext_vector_type(2)));
 typedef uint32_t dm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t dm_u32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) const dm_u32x2 dm_lds_cu64;
+typedef __attribute__((address_space(3))) const uint32_t dm_lds_cu32;
 typedef __attribute__((address_space(3))) dm_u32x4 dm_lds_u128;
 
 #define DM_WAVES 8
@@ -288,11 +290,11 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
 #pragma unroll
     for (int i = 0; i < 8; ++i)      // (each entry starts with another of its pieces: sixteen lanes then write to all banks, not to two
       // groups: K and V of 4 x 500 tokens of 8 heads 10.5 -> 9.2 us)
-      *(dm_lds_u128*)(uintptr_t)(uint32_t)(e * 256 + half * 128 + ((i + e) & 7) * 16) = (dm_u32x4){hi, lo, hi, lo};
+      *(dm_lds_u128*)(uintptr_t)(uint32_t)(e * 256 + half * 128 + ((i + e) & 7) * 16) = half ? (dm_u32x4){lo, lo, lo, lo} : (dm_u32x4){hi, hi, hi, hi};
   }
 
   __syncthreads();
-  const uint32_t copy = (uint32_t)(lane & 31) * 8u;
+  const uint32_t copy = (uint32_t)(lane & 31) * 4u;
 
   if (step >= steps) return;
   uint32_t kw[DM_MT][KS];
@@ -331,9 +333,10 @@ __global__ __launch_bounds__(DM_THREADS) void akv_decode_mfma_kernel(akv_gen_arg
         for (int mt = 0; mt < DM_MT; ++mt)
 #pragma unroll
           for (int b = 0; b < 4; ++b) {
-            const dm_u32x2 t = *(dm_lds_cu64*)(uintptr_t)__builtin_amdgcn_perm(kw[mt][ks], copy, 0x0c020400u + ((uint32_t)b << 8));
-            ch[mt].u[b] = t.x;
-            cl[mt].u[b] = t.y;
+            uint32_t at = __builtin_amdgcn_perm(kw[mt][ks], copy, 0x0c020400u + ((uint32_t)b << 8));
+            ch[mt].u[b] = *(dm_lds_cu32*)(uintptr_t)at;
+            asm("" : "+v"(at));       // (seen as one place and another, the two would be read by one request into neighbouring registers)
+            cl[mt].u[b] = *(dm_lds_cu32*)(uintptr_t)(at + 128u);
           }
         // (term by term: products in a row do not wait for each other's sum)
 #pragma unroll
