@@ -153,6 +153,11 @@ __device__ __forceinline__ void akv_block_prefix_scan(const void* context_lens, 
   if (tid == 255) prefix[S] = base + inc;
 }
 
+// longest range of whole workgroups against an equal cut, in chunks
+__device__ __forceinline__ bool akv_attn_aligned_pays(int aligned, int equal, int shares) {
+  return shares > 1 ? (aligned + shares - 1) / shares <= (equal + shares - 1) / shares + 1 : aligned <= equal + 3;
+}
+
 // ----------------------------------------------------------------------------------
 // Block prefix of the batch and partition of the global block axis among the G workgroups of the matrix-core
 // kernel, written by one workgroup of 256 threads or more.
@@ -163,14 +168,17 @@ __device__ __forceinline__ void akv_block_prefix_scan(const void* context_lens, 
 // sequence gets whole workgroups: the smallest lambda (chunks per workgroup) with sum_s ceil(c_s / lambda) <= G
 // is found by bisection (the sum is non-increasing in lambda), sequence s takes k_s = ceil(c_s / lambda)
 // consecutive workgroups and splits its c_s chunks evenly among them; left-over workgroups get an empty range.
-// Otherwise the axis is cut into G equal ranges as before.  Either way workgroups and sequences both advance
+// Otherwise the axis is cut into G equal ranges.  Either way workgroups and sequences both advance
 // monotonically along the axis, so slot = workgroup + sequence stays unique, and seqw[s] = (first, last
 // workgroup that meets sequence s), which the reduce kernel reads instead of dividing by the range length.
 // `cb` = blocks per chunk of the main kernel (2 for blocks of 16 tokens, 1 for blocks of 32).  `shares` > 1: so many wavefronts
-// of a workgroup go through its chunks side by side and merge their results at the end of every segment.  Whole workgroups then
-// pay for more sequences too (a second segment costs what one more round of chunks does): up to half the workgroups, while the
-// longest range is at most a round longer than an equal one (one kv head, 48 sequences: of 700 tokens 21.3 -> 17.7 us, of 1k to
-// 16k the step 41.2 -> 36.6).
+// of a workgroup go through its chunks side by side and merge their results at the end of every segment.
+//
+// A second segment costs a workgroup as much as three chunks or one more round of chunks of its shares, so whole workgroups also
+// pay for more sequences, up to half the workgroups, while the longest range is no more than that longer than an equal one.  One
+// kv head, 48 sequences: of 700 tokens 21.3 -> 17.7 us, of 1k to 16k the step 41.2 -> 36.6.  Eight kv heads: the step of 40
+// sequences of 300 to 3,000 39.3 -> 35.0 us, of 64 of 100 to 1,500 40.6 -> 33.7, of 100 of 200 to 1,000 42.0 -> 37.6, of 128 of 300 33.1, 41.9 before;
+// heads of 256 55.5 -> 49.5, tq35 65.2 -> 56.1.  Up to 256 sequences are judged, a thread each.
 // ----------------------------------------------------------------------------------
 __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G, int cb, int32_t* wgdesc, int32_t* seqw,
                                                    int32_t* lds /*[>= 257]*/, const void* context_lens, int cl_itype,
@@ -186,6 +194,65 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
     __threadfence_block();
     __syncthreads();                    // the prefix written by this workgroup is readable by all of it
     const int total = prefix[S];
+    if (S <= 256) {
+      int32_t* p_part = lds + 4;          // [2][4] of the wavefronts (lds[0..3] may still be read by the scan above)
+      const int b0 = tid < S ? prefix[tid] : 0, b1 = tid < S ? prefix[tid + 1] : 0;
+      const int c = (b1 - b0 + cb - 1) / cb;
+      int turn = 0;
+      auto sum_all = [&](int v) {
+        const int mine = akv_wave_sum(v);
+        if (lane == 0 && tid < 256) p_part[4 * turn + (tid >> 6)] = mine;
+        __syncthreads();
+        const int all = p_part[4 * turn] + p_part[4 * turn + 1] + p_part[4 * turn + 2] + p_part[4 * turn + 3];
+        turn ^= 1;                        // (the other half is written next: nobody reads that one any more)
+        return all;
+      };
+      const int sumc = sum_all(c), nz = sum_all(c > 0 ? 1 : 0);
+      const int equal = max(1, (sumc + G - 1) / G);
+      int lo = equal;
+      bool aligned = false;
+      if (nz >= 1 && 2 * nz <= G) {
+        int hi = (sumc + (G - nz) - 1) / (G - nz);
+        while (lo < hi) {
+          const int mid = (lo + hi) >> 1;
+          if (sum_all((c + mid - 1) / mid) <= G) hi = mid; else lo = mid + 1;
+        }
+        aligned = akv_attn_aligned_pays(lo, equal, shares);
+      }
+      if (aligned) {
+        const int k = (c + lo - 1) / lo;
+        const int inc = akv_wave_inclusive_scan(k);
+        if (lane == 63 && tid < 256) p_part[4 * turn + (tid >> 6)] = inc;
+        __syncthreads();
+        int first = inc - k, used = 0;
+        for (int w = 0; w < 4; ++w) {
+          if (w < (tid >> 6)) first += p_part[4 * turn + w];
+          used += p_part[4 * turn + w];
+        }
+        if (tid < S) {
+          seqw[2 * tid] = first;
+          seqw[2 * tid + 1] = first + k - 1;
+          if (k > 0) {
+            const int ctx = (int)akv_seq_tokens(context_lens, cl_itype, tid, block_size, max_blocks_per_seq), pc = (c + k - 1) / k * cb;
+            for (int j = 0; j < k; ++j) {
+              int32_t* rec = wgdesc + (size_t)(first + j) * AKV_WGREC;
+              rec[AKV_WGREC_G0] = b0 + j * pc;            // (below b1: k - 1 ranges of at most lo chunks do not hold c)
+              rec[AKV_WGREC_G1] = min(b1, b0 + (j + 1) * pc);
+              rec[AKV_WGREC_SEQ] = tid;
+              rec[AKV_WGREC_SB0] = b0;
+              rec[AKV_WGREC_SB1] = b1;
+              rec[AKV_WGREC_CTX] = ctx;
+            }
+          }
+        }
+        for (int w = used + tid; w < G; w += blockDim.x) {
+          int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
+          rec[AKV_WGREC_G0] = rec[AKV_WGREC_G1] = 0;
+          rec[AKV_WGREC_SEQ] = -1;
+        }
+        return;
+      }
+    }
     const int per = (total + G - 1) / G;
     for (int w = tid; w < G; w += blockDim.x) {
       int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
@@ -233,7 +300,7 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
     int aligned = (nz >= 1 && nz * 8 <= G) ? 1 : 0;
     int lo = (sumc + G - 1) / G;
     if (lo < 1) lo = 1;
-    if (aligned || (shares > 1 && nz >= 1 && 2 * nz <= G)) {
+    if (aligned || (nz >= 1 && 2 * nz <= G)) {
       const int equal = lo;
       int hi = (sumc + (G - nz) - 1) / (G - nz);      // always feasible
       while (lo < hi) {
@@ -241,7 +308,7 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
         const int tot = akv_wave_sum((c + mid - 1) / mid);
         if (tot <= G) hi = mid; else lo = mid + 1;
       }
-      if ((lo + shares - 1) / shares <= (equal + shares - 1) / shares + 1) aligned = 1;
+      if (akv_attn_aligned_pays(lo, equal, shares)) aligned = 1;
     }
     if (aligned) {
       const int k = (c + lo - 1) / lo;
