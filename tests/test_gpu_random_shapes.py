@@ -15,6 +15,7 @@ from oracle import tq_oracle as O
 from tests.test_gpu_attention import within_tol
 from tests.test_gpu_hybrid import build_cache as hybrid_cache, params as hybrid_params
 from tests.util import kv_like
+from tests import test_gpu_attention
 
 pytestmark = pytest.mark.gpu
 
@@ -256,3 +257,10 @@ def test_paged_update_random_shapes(golden, dev, seed):
         assert int(np.max(np.abs(ca.astype(int) - cb.astype(int)), initial=0)) <= 1
         if T:
             assert np.max(np.abs(gn - ref_n) / np.maximum(np.abs(ref_n), 1e-30)) <= 1e-6
+
+
+@pytest.mark.parametrize("bits,S,empty_every", [(4, 100, 0), (3, 127, 2), (4, 128, 0), (2, 129, 0), (4, 256, 3), (4, 257, 2)])
+def test_partition_of_batches_beyond_a_wavefront(golden, dev, bits, S, empty_every):
+    """Whole workgroups for up to half as many non-empty sequences as there are workgroups, judged by a thread per sequence of up
+    to 256; equal ranges beyond."""
+    test_gpu_attention.test_partition_of_the_block_axis_by_batch_shape(golden, dev, bits, S, empty_every)
