@@ -1062,7 +1062,7 @@ int akv_encode_mfma_try(const akv_gen_args& a, bool paged, int x_dtype, int d, i
   if (((uintptr_t)a.packed | (uintptr_t)a.packed2 | (uintptr_t)a.ps0 | (uintptr_t)a.ps1 | (uintptr_t)a.ps2) & amask) return AKV_ERR_UNSUPPORTED;
   const uint4* bop = (const uint4*)((const float*)rot_prep + (size_t)2 * d * d);
   const int64_t n_total = (paged && a.x2) ? 2 * a.n : a.n;
-  const int cus = akv_cached_cu_count();
+  const int cus = akv_cached_cu_count() > 0 ? akv_cached_cu_count() : 256;
   // Calls of up to some hundred vectors a CU take the kernel with the matrix in registers: no 64 KB fill, and a wavefront's chain
   // is a quarter of a row's tiles.  Steps of 16, 32 or 64 rows, so that the calls that give a CU one step have it on every CU.
   // Keys and values in bfloat16 and 4 bits, us, the kernel above | that one: 8,192 vectors 8.5 | 5.8, 16,384 9.3 | 6.9, 32,768

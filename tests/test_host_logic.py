@@ -599,3 +599,28 @@ def test_the_binding_has_no_thread_local_storage():
     at, size, count = struct.unpack_from("<Q", elf, 32)[0], *struct.unpack_from("<HH", elf, 54)
     kinds = [struct.unpack_from("<I", elf, at + i * size)[0] for i in range(count)]
     assert 1 in kinds and 7 not in kinds          # PT_LOAD, PT_TLS
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="says what happens where no device answers")
+def test_encode_without_a_device_is_an_error():
+    """The choice of a kernel goes by the number of compute units, which is 0 where no device answers: an error code, in a process
+    of its own because it was a division by zero."""
+    code = """
+import ctypes, sys
+import torch
+from aitherkvcache_amd import _lib
+L = _lib.lib()
+count = ctypes.c_int()
+if L.akv_device_cu_count(ctypes.byref(count)) == 0:
+    sys.exit(0)                                   # (a device after all: these are host addresses)
+prep, table, packed = torch.zeros(1 << 18), torch.zeros(16), torch.zeros(64 * 64, dtype=torch.uint8)
+norms, slots = torch.zeros(64), torch.zeros(64, dtype=torch.int64)
+for dtype, code in _lib._DTYPE.items():
+    x = torch.zeros(64, 128, dtype=dtype)
+    rc = L.akv_encode(x.data_ptr(), code, 64, 128, 128, prep.data_ptr(), table.data_ptr(), 4, packed.data_ptr(), 64, norms.data_ptr(), None)
+    assert rc == _lib.AKV_ERR_HIP, (dtype, rc)
+    rc = L.akv_encode_paged_kv(x.data_ptr(), x.data_ptr(), code, 64, 1, 128, 128, 128, slots.data_ptr(), _lib.AKV_I64, prep.data_ptr(), table.data_ptr(), 4,
+                               packed.data_ptr(), packed.data_ptr(), 1024, 64, 64, norms.data_ptr(), norms.data_ptr(), 16, 1, 1, 16, 4, None)
+    assert rc == _lib.AKV_ERR_HIP, (dtype, rc)
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
