@@ -686,3 +686,33 @@ def test_partition_of_the_block_axis_by_batch_shape(golden, dev, bits, S, empty_
     for s_, r_ in refs.items():
         assert within_tol(out[s_], r_), f"sequence {s_} of {S} (ctx {ctx[s_]})"
     assert attn.last_call_status() == 0
+
+
+@pytest.mark.parametrize("S", [100, 200])
+def test_a_long_context_among_short_ones_costs_no_more_than_both_apart(golden, dev, S):
+    """One context over most of the workgroups among many in one or two each: the reduce merges its hundred and more partial results
+    with as many requests under way as for the others (one at a time they took longer than all of the attention)."""
+    tq = make_tq(golden, dev, 4)
+    rng = np.random.default_rng(77)
+    NB, KVH, QH, long = 4000, 8, 32, 30000
+    kp, kn, vp, vn = build_cache(rng, tq, dev, NB, KVH, 4)
+    attn = akv.TQPagedAttention(tq, QH)
+
+    def least(ctx):
+        ctx = np.asarray(ctx, dtype=np.int64)
+        tables = t(rng.integers(0, NB, size=(len(ctx), -(-long // 16))).astype(np.int32), dev)
+        q, ctx = t(rng.standard_normal((len(ctx), QH, 128)).astype(np.float16), dev), t(ctx, dev)
+        times = []
+        for _ in range(6):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(50):
+                attn.forward(q, kp, kn, vp, vn, tables, ctx)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end) * 20)
+        return min(times)
+
+    both, one, many = least([200] * (S // 3) + [long] + [200] * (S - S // 3 - 1)), least([long]), least([200] * (S - 1))
+    print(f"[long among {S}] {both:.1f} us, apart {one:.1f} and {many:.1f}", flush=True)
+    assert both < one + many
