@@ -124,10 +124,11 @@ __device__ __forceinline__ int64_t akv_seq_tokens(const void* context_lens, int 
   return ctx < cap ? ctx : cap;
 }
 
-// One workgroup (256 threads or more: those past 255 hold nothing) writes prefix[0..S].
-__device__ __forceinline__ void akv_block_prefix_scan(const void* context_lens, int cl_itype, int S,
-                                                      int block_size, int64_t max_blocks_per_seq,
-                                                      int32_t* prefix, int32_t* scratch /*[>= 4] LDS*/) {
+// One workgroup (256 threads or more: those past 255 hold nothing) writes prefix[0..S].  Returns the entry of the thread's first
+// sequence, min(S, tid * ceil(S / 256)), and in `end` that of the next thread's.
+__device__ __forceinline__ int akv_block_prefix_scan(const void* context_lens, int cl_itype, int S,
+                                                     int block_size, int64_t max_blocks_per_seq,
+                                                     int32_t* prefix, int32_t* scratch /*[>= 4] LDS*/, int* end = nullptr) {
   const int tid = threadIdx.x;
   const int chunk = (S + 255) / 256;
   const int lo = min(S, tid * chunk), hi = min(S, lo + chunk);
@@ -151,11 +152,21 @@ __device__ __forceinline__ void akv_block_prefix_scan(const void* context_lens, 
     run += akv_seq_blocks(context_lens, cl_itype, s, block_size, max_blocks_per_seq);
   }
   if (tid == 255) prefix[S] = base + inc;
+  if (end) *end = base + inc;
+  return base + inc - sum;
 }
 
 // longest range of whole workgroups against an equal cut, in chunks
 __device__ __forceinline__ bool akv_attn_aligned_pays(int aligned, int equal, int shares) {
   return shares > 1 ? (aligned + shares - 1) / shares <= (equal + shares - 1) / shares + 1 : aligned <= equal + 3;
+}
+
+// the last i < n (a power of two) with entry[i] <= v: entries non-decreasing, entry[0] <= v
+__device__ __forceinline__ int akv_last_at_most(const int32_t* entry, int n, int v) {
+  int at = 0;
+  for (int step = n >> 1; step > 0; step >>= 1)
+    if (entry[at + step] <= v) at += step;
+  return at;
 }
 
 // ----------------------------------------------------------------------------------
@@ -164,40 +175,49 @@ __device__ __forceinline__ bool akv_attn_aligned_pays(int aligned, int equal, in
 //
 // A workgroup whose range crosses a sequence boundary starts twice (query operand, block ids, first rows, a
 // partial chunk at both ends): measured, such workgroups finish 5 us after the others and ARE the tail of
-// the launch.  So when the batch has few sequences (at most 64 in all, the non-empty ones at most G / 8) every
-// sequence gets whole workgroups: the smallest lambda (chunks per workgroup) with sum_s ceil(c_s / lambda) <= G
-// is found by bisection (the sum is non-increasing in lambda), sequence s takes k_s = ceil(c_s / lambda)
-// consecutive workgroups and splits its c_s chunks evenly among them; left-over workgroups get an empty range.
-// Otherwise the axis is cut into G equal ranges.  Either way workgroups and sequences both advance
+// the launch.  So sequences get whole workgroups where that pays: the smallest lambda (chunks per workgroup) with
+// sum_s ceil(c_s / lambda) <= G is found by bisection (the sum is non-increasing in lambda), sequence s takes
+// k_s = ceil(c_s / lambda) consecutive workgroups and splits its c_s chunks evenly among them; left-over workgroups get an
+// empty range.  Otherwise the axis is cut into G equal ranges.  Either way workgroups and sequences both advance
 // monotonically along the axis, so slot = workgroup + sequence stays unique, and seqw[s] = (first, last
 // workgroup that meets sequence s), which the reduce kernel reads instead of dividing by the range length.
 // `cb` = blocks per chunk of the main kernel (2 for blocks of 16 tokens, 1 for blocks of 32).  `shares` > 1: so many wavefronts
 // of a workgroup go through its chunks side by side and merge their results at the end of every segment.
 //
-// A second segment costs a workgroup as much as three chunks or one more round of chunks of its shares, so whole workgroups also
-// pay for more sequences, up to half the workgroups, while the longest range is no more than that longer than an equal one.  One
+// Whole workgroups: with at most 64 sequences always where the non-empty ones are at most G / 8.  A second segment costs a
+// workgroup as much as three chunks or one more round of chunks of its shares, so also with up to 256 sequences, the non-empty
+// ones at most half the workgroups, while the longest range is no more than that longer than an equal one.  One
 // kv head, 48 sequences: of 700 tokens 21.3 -> 17.7 us, of 1k to 16k the step 41.2 -> 36.6.  Eight kv heads: the step of 40
 // sequences of 300 to 3,000 39.3 -> 35.0 us, of 64 of 100 to 1,500 40.6 -> 33.7, of 100 of 200 to 1,000 42.0 -> 37.6, of 128 of 300 33.1, 41.9 before;
-// heads of 256 55.5 -> 49.5, tq35 65.2 -> 56.1.  Up to 256 sequences are judged, a thread each.
+// heads of 256 55.5 -> 49.5, tq35 65.2 -> 56.1.
+//
+// At most 64 sequences are held by one wavefront, more by a thread each (or several each); records are written by a thread per
+// workgroup, which finds its sequence among the starts in LDS.  (By a thread per sequence, one of 30,000 tokens among 99 of
+// 200 had 150 records to write alone: the kernel 10.9 us, now 6.3.)
 // ----------------------------------------------------------------------------------
+#define AKV_PART_WORDS 592              // LDS of akv_attn_partition (int32 words)
 __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G, int cb, int32_t* wgdesc, int32_t* seqw,
-                                                   int32_t* lds /*[>= 257]*/, const void* context_lens, int cl_itype,
+                                                   int32_t* lds /*[AKV_PART_WORDS]*/, const void* context_lens, int cl_itype,
                                                    int block_size, int64_t max_blocks_per_seq, int shares = 1) {
   const int tid = threadIdx.x, lane = tid & 63;
-  int32_t* p_wfirst = lds;              // [65] first workgroup of each sequence; [64] = workgroups in use
-  int32_t* p_pref = lds + 65;           // [65] block prefix; [64] = total
-  int32_t* p_ctx = lds + 130;           // [64] context length in tokens (clamped to the table width)
-  int32_t* p_mode = lds + 194;          // [0] 1 = whole workgroups per sequence, [1] = total blocks
+  const int n = S > 64 ? 256 : 64;      // starts in LDS: of every sequence, beyond 256 of every `chunk`-th
+  const int chunk = (S + 255) / 256;
+  int32_t* p_wfirst = lds;              // [n + 1] first workgroup of each sequence; [n] = workgroups in use
+  int32_t* p_pref = lds + 257;          // [n + 1] block prefix; [n] = total
+  int32_t* p_ctx = lds + 514;           // [64] context length in tokens, clamped to the table width (at most 64 sequences)
+  int32_t* p_mode = lds + 578;          // [0] 1 = whole workgroups per sequence (at most 64 sequences)
+  int32_t* p_part = lds + 580;          // [2][4] sums of the wavefronts (more)
+  int32_t* p_scan = lds + 588;          // [4]
+  bool aligned = false;
   if (S > 64) {
-    // many sequences: the general scan, equal ranges
-    akv_block_prefix_scan(context_lens, cl_itype, S, block_size, max_blocks_per_seq, prefix, lds);
+    int b1;
+    const int b0 = akv_block_prefix_scan(context_lens, cl_itype, S, block_size, max_blocks_per_seq, prefix, p_scan, &b1);
+    if (tid < 256) p_pref[tid] = b0;
+    if (tid == 255) p_pref[256] = b1;
     __threadfence_block();
     __syncthreads();                    // the prefix written by this workgroup is readable by all of it
-    const int total = prefix[S];
     if (S <= 256) {
-      int32_t* p_part = lds + 4;          // [2][4] of the wavefronts (lds[0..3] may still be read by the scan above)
-      const int b0 = tid < S ? prefix[tid] : 0, b1 = tid < S ? prefix[tid + 1] : 0;
-      const int c = (b1 - b0 + cb - 1) / cb;
+      const int c = (b1 - b0 + cb - 1) / cb;                     // chunks of the thread's sequence (0: none, or an empty one)
       int turn = 0;
       auto sum_all = [&](int v) {
         const int mine = akv_wave_sum(v);
@@ -210,9 +230,8 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
       const int sumc = sum_all(c), nz = sum_all(c > 0 ? 1 : 0);
       const int equal = max(1, (sumc + G - 1) / G);
       int lo = equal;
-      bool aligned = false;
       if (nz >= 1 && 2 * nz <= G) {
-        int hi = (sumc + (G - nz) - 1) / (G - nz);
+        int hi = (sumc + (G - nz) - 1) / (G - nz);      // always feasible
         while (lo < hi) {
           const int mid = (lo + hi) >> 1;
           if (sum_all((c + mid - 1) / mid) <= G) hi = mid; else lo = mid + 1;
@@ -224,80 +243,43 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
         const int inc = akv_wave_inclusive_scan(k);
         if (lane == 63 && tid < 256) p_part[4 * turn + (tid >> 6)] = inc;
         __syncthreads();
-        int first = inc - k, used = 0;
-        for (int w = 0; w < 4; ++w) {
+        int first = inc - k;
+        for (int w = 0; w < 3; ++w)
           if (w < (tid >> 6)) first += p_part[4 * turn + w];
-          used += p_part[4 * turn + w];
-        }
+        if (tid < 256) p_wfirst[tid] = first;
+        if (tid == 255) p_wfirst[256] = first + k;
         if (tid < S) {
           seqw[2 * tid] = first;
           seqw[2 * tid + 1] = first + k - 1;
-          if (k > 0) {
-            const int ctx = (int)akv_seq_tokens(context_lens, cl_itype, tid, block_size, max_blocks_per_seq), pc = (c + k - 1) / k * cb;
-            for (int j = 0; j < k; ++j) {
-              int32_t* rec = wgdesc + (size_t)(first + j) * AKV_WGREC;
-              rec[AKV_WGREC_G0] = b0 + j * pc;            // (below b1: k - 1 ranges of at most lo chunks do not hold c)
-              rec[AKV_WGREC_G1] = min(b1, b0 + (j + 1) * pc);
-              rec[AKV_WGREC_SEQ] = tid;
-              rec[AKV_WGREC_SB0] = b0;
-              rec[AKV_WGREC_SB1] = b1;
-              rec[AKV_WGREC_CTX] = ctx;
-            }
-          }
-        }
-        for (int w = used + tid; w < G; w += blockDim.x) {
-          int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
-          rec[AKV_WGREC_G0] = rec[AKV_WGREC_G1] = 0;
-          rec[AKV_WGREC_SEQ] = -1;
-        }
-        return;
-      }
-    }
-    const int per = (total + G - 1) / G;
-    for (int w = tid; w < G; w += blockDim.x) {
-      int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
-      const int g0 = min(total, w * per);
-      rec[AKV_WGREC_G0] = g0;
-      rec[AKV_WGREC_G1] = min(total, g0 + per);
-      if (g0 >= total) rec[AKV_WGREC_SEQ] = -1;
-    }
-    for (int s = tid; s < S; s += blockDim.x) {
-      const int b0 = prefix[s], b1 = prefix[s + 1];
-      const int w_lo = per > 0 ? b0 / per : 0;
-      seqw[2 * s] = w_lo;
-      seqw[2 * s + 1] = (per > 0 && b1 > b0) ? (b1 - 1) / per : w_lo - 1;
-      // the ranges that start in the sequence: each start lies in one
-      if (b1 > b0) {
-        const int ctx = (int)akv_seq_tokens(context_lens, cl_itype, s, block_size, max_blocks_per_seq);
-        for (int w = (b0 + per - 1) / per; w < G && w * per < b1; ++w) {
-          int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
-          rec[AKV_WGREC_SEQ] = s;
-          rec[AKV_WGREC_SB0] = b0;
-          rec[AKV_WGREC_SB1] = b1;
-          rec[AKV_WGREC_CTX] = ctx;
         }
       }
     }
-    return;
-  }
-  // at most 64 sequences: one wavefront holds the batch, lane = sequence
-  if (tid < 64) {
-    int n = 0, ctx = 0;
+    if (!aligned) {
+      const int per = (p_pref[256] + G - 1) / G;
+      for (int s = tid; s < S; s += blockDim.x) {
+        const int first = prefix[s], last = prefix[s + 1];
+        const int w_lo = per > 0 ? first / per : 0;
+        seqw[2 * s] = w_lo;
+        seqw[2 * s + 1] = (per > 0 && last > first) ? (last - 1) / per : w_lo - 1;
+      }
+    }
+  } else if (tid < 64) {
+    int blocks = 0, ctx = 0;
     if (lane < S) {
       ctx = (int)akv_seq_tokens(context_lens, cl_itype, lane, block_size, max_blocks_per_seq);
-      n = (ctx + block_size - 1) / block_size;
+      blocks = (ctx + block_size - 1) / block_size;
     }
-    const int inc = akv_wave_inclusive_scan(n);
+    const int inc = akv_wave_inclusive_scan(blocks);
     const int total = __builtin_amdgcn_readlane(inc, 63);
-    const int b0 = inc - n;
+    const int b0 = inc - blocks;
     if (lane < S) prefix[lane] = b0;
     if (lane == 0) prefix[S] = total;
     p_pref[lane] = b0;
     p_ctx[lane] = ctx;
-    const int c = (n + cb - 1) / cb;                             // chunks of the lane's sequence
+    const int c = (blocks + cb - 1) / cb;                        // chunks of the lane's sequence
     const int sumc = akv_wave_sum(c);
     const int nz = __popcll(__ballot(c > 0));
-    int aligned = (nz >= 1 && nz * 8 <= G) ? 1 : 0;
+    aligned = nz >= 1 && nz * 8 <= G;
     int lo = (sumc + G - 1) / G;
     if (lo < 1) lo = 1;
     if (aligned || (nz >= 1 && 2 * nz <= G)) {
@@ -308,7 +290,7 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
         const int tot = akv_wave_sum((c + mid - 1) / mid);
         if (tot <= G) hi = mid; else lo = mid + 1;
       }
-      if (akv_attn_aligned_pays(lo, equal, shares)) aligned = 1;
+      if (akv_attn_aligned_pays(lo, equal, shares)) aligned = true;
     }
     if (aligned) {
       const int k = (c + lo - 1) / lo;
@@ -323,27 +305,25 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
       const int per = (total + G - 1) / G;
       const int w_lo = per > 0 ? b0 / per : 0;
       seqw[2 * lane] = w_lo;
-      seqw[2 * lane + 1] = (per > 0 && n > 0) ? (b0 + n - 1) / per : w_lo - 1;
+      seqw[2 * lane + 1] = (per > 0 && blocks > 0) ? (b0 + blocks - 1) / per : w_lo - 1;
     }
     if (lane == 0) {
       p_pref[64] = total;
-      p_mode[0] = aligned;
-      p_mode[1] = total;
+      p_mode[0] = aligned ? 1 : 0;
     }
   }
   __syncthreads();
-  const int aligned = p_mode[0], total = p_mode[1];
-  const int per = (total + G - 1) / G;
+  if (S <= 64) aligned = p_mode[0] != 0;
+  const int total = p_pref[n], per = (total + G - 1) / G;
   for (int w = tid; w < G; w += blockDim.x) {
-    int g0 = 0, g1 = 0, s = -1;
+    int g0 = 0, g1 = 0, s = -1, b0 = 0, b1 = 0;
     if (aligned) {
-      if (w < p_wfirst[64]) {
-        // the last s with p_wfirst[s] <= w (entries are non-decreasing; a sequence without workgroups shares the
-        // next one's entry and is passed over; entries of lanes past the batch equal the number in use)
-        int cnt = 0;
-        for (int i = 0; i < 64; ++i) cnt += (p_wfirst[i] <= w) ? 1 : 0;
-        s = cnt - 1;
-        const int b0 = p_pref[s], b1 = p_pref[s + 1];
+      if (w < p_wfirst[n]) {
+        // (a sequence without workgroups shares the next one's entry and is passed over; entries past the batch equal the
+        // number in use)
+        s = akv_last_at_most(p_wfirst, n, w);
+        b0 = p_pref[s];
+        b1 = p_pref[s + 1];
         const int k = p_wfirst[s + 1] - p_wfirst[s];
         const int c = (b1 - b0 + cb - 1) / cb;
         const int pc = (c + k - 1) / k;
@@ -354,9 +334,19 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
       g0 = min(total, w * per);
       g1 = min(total, g0 + per);
       if (g0 < g1) {
-        int cnt = 0;
-        for (int i = 0; i < 64; ++i) cnt += (i < S && p_pref[i] <= g0) ? 1 : 0;
-        s = cnt - 1;      // the last sequence that starts at or before g0 (an empty one shares its successor's start)
+        s = akv_last_at_most(p_pref, n, g0);    // the last sequence that starts at or before g0 (an empty one shares its successor's start)
+        b0 = p_pref[s];
+        b1 = p_pref[s + 1];
+        if (chunk > 1) {
+          int hi = min(S, (s + 1) * chunk);     // prefix[s] <= g0 < prefix[hi]
+          s *= chunk;
+          while (hi - s > 1) {
+            const int mid = (s + hi) >> 1;
+            if (prefix[mid] <= g0) s = mid; else hi = mid;
+          }
+          b0 = prefix[s];
+          b1 = prefix[s + 1];
+        }
       }
     }
     int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
@@ -364,9 +354,9 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
     rec[AKV_WGREC_G1] = g1;
     rec[AKV_WGREC_SEQ] = g0 < g1 ? s : -1;
     if (g0 < g1) {
-      rec[AKV_WGREC_SB0] = p_pref[s];
-      rec[AKV_WGREC_SB1] = p_pref[s + 1];
-      rec[AKV_WGREC_CTX] = p_ctx[s];
+      rec[AKV_WGREC_SB0] = b0;
+      rec[AKV_WGREC_SB1] = b1;
+      rec[AKV_WGREC_CTX] = S > 64 ? (int)akv_seq_tokens(context_lens, cl_itype, s, block_size, max_blocks_per_seq) : p_ctx[s];
     }
   }
 }

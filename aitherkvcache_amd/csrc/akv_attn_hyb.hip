@@ -1069,7 +1069,7 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_prologue_kernel(
     uint4* __restrict__ qop, float* __restrict__ fac, uint32_t* __restrict__ lut, uint32_t* __restrict__ status, uint32_t start_status,
     int32_t* __restrict__ wgdesc, int32_t* __restrict__ seqw, int G, int shares) {
   __shared__ int8_t dig[3][4][256];       // [digit][query head][sum]
-  __shared__ int32_t scratch[257];
+  __shared__ int32_t scratch[AKV_PART_WORDS];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (blockIdx.x == 0) {
     if (tid == 0) status[0] = start_status;

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void akv_attn_mfma_prologue_kernel(
     uint4* __restrict__ qop, uint32_t* __restrict__ lut, uint32_t* __restrict__ status, float qscale, int bits, int nqb,
     int32_t* __restrict__ wgdesc, int32_t* __restrict__ seqw, int G) {
   __shared__ __align__(16) ar_rows<128, ar_terms<QDT>()> rows;
-  __shared__ int32_t scratch[257];
+  __shared__ int32_t scratch[AKV_PART_WORDS];
   __shared__ float best_err[256];
   __shared__ float best_alpha[256];
   const int tid = threadIdx.x;

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void akv_attn_wave_prologue_kernel(
     uint2* __restrict__ qop, float* __restrict__ fac, uint32_t* __restrict__ status, float qscale, int bits, int32_t* __restrict__ wgdesc,
     int32_t* __restrict__ seqw, int G, int shares) {
   __shared__ __align__(16) ar_rows<D, ar_terms<QDT>()> rows;
-  __shared__ int32_t scratch[257];
+  __shared__ int32_t scratch[AKV_PART_WORDS];
   if (blockIdx.x == 0) {
     if (threadIdx.x == 0) status[0] = 0u;
     akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares);

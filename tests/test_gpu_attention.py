@@ -661,10 +661,9 @@ def test_value_norms_far_outside_the_float16_range(golden, dev, bits, case):
 @pytest.mark.parametrize("bits", [4, 2])
 @pytest.mark.parametrize("S,empty_every", [(40, 0), (33, 2), (64, 0), (64, 3), (65, 0), (20, 0), (32, 0), (1, 0)])
 def test_partition_of_the_block_axis_by_batch_shape(golden, dev, bits, S, empty_every):
-    """The three ways the prologue cuts the block axis among the workgroups -- whole workgroups per sequence (few
-    non-empty sequences), equal ranges with the sequences held by one wavefront (up to 64 sequences), equal
-    ranges through the general scan (more) -- with empty sequences in between, sequences of one token and
-    lengths that leave the last workgroup of a sequence a single block: every sequence against the oracle."""
+    """Whole workgroups per sequence, the sequences held by one wavefront (up to 64) or by a thread each (more), with
+    empty sequences in between, sequences of one token and lengths that leave the last workgroup of a sequence a
+    single block: every sequence against the oracle.  (Equal ranges: test_ranges_of_workgroups_vs_float64.)"""
     tq = make_tq(golden, dev, bits)
     rng = np.random.default_rng(8800 + 7 * S + bits + empty_every)
     NB, KVH, QH = 400, 8, 32

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import aitherkvcache_amd as akv
-from tests.util import kv_like
+from tests.util import batch_of_ranges, kv_like, whole_workgroups
 
 pytestmark = pytest.mark.gpu
 
@@ -208,6 +208,29 @@ def test_many_sequences_and_empty_ones_vs_float64(dev, mode, qh, kvh):
     out = akv.HybridPagedAttention(h, qh).forward(q, rows[0], rows[1], torch.from_numpy(tables).to(dev), torch.from_numpy(ctx).to(dev)).double().cpu()
     assert not out[torch.from_numpy(ctx == 0)].any()
     for i in np.flatnonzero(ctx):
+        t = torch.from_numpy(tables[i, :-(-int(ctx[i]) // 16)].astype(np.int64))
+        k, v = (x[t].reshape(-1, kvh, 128)[:ctx[i]] for x in (K, V))
+        ref = attend(q[i].double().cpu(), k, v)
+        assert (out[i] - ref).norm() <= limit(mode, qh, kvh) * ref.norm(), (i, ctx[i])
+
+
+@pytest.mark.parametrize("kind", ["whole, one long", "whole, half", "equal, one long", "equal, few (55)"])
+# (workgroups a compute unit: three for two groups of four kv head slots at a time, or two; wavefronts of a kv head)
+@pytest.mark.parametrize("mode,qh,kvh,per_cu,shares", [("tq35", 32, 8, 1.5, 1), ("tq25", 12, 2, 2, 2)])
+def test_ranges_of_workgroups_vs_float64(dev, mode, qh, kvh, per_cu, shares, kind):
+    rng, h, rows = make(dev, mode, kvh, 40, 16, 64 if mode == "tq35" else 44, qh)
+    ctx, look = batch_of_ranges(rng, kind)
+    whole = whole_workgroups(ctx, int(per_cu * torch.cuda.get_device_properties(dev).multi_processor_count), shares)
+    if mode == "tq25" and kind.startswith("equal"):
+        assert whole
+        pytest.skip("512 workgroups: whole ones")
+    assert whole == kind.startswith("whole")
+    tables = rng.integers(0, 40, size=(len(ctx), int(ctx.max() + 15) // 16)).astype(np.int32)
+    K, V = (h.decode(r.contiguous()).double().cpu() for r in rows)
+    q = torch.from_numpy(rng.standard_normal((len(ctx), qh, 128)).astype(np.float32)).to(dev)
+    out = akv.HybridPagedAttention(h, qh).forward(q, rows[0], rows[1], torch.from_numpy(tables).to(dev), torch.from_numpy(ctx).to(dev)).double().cpu()
+    assert not out[torch.from_numpy(ctx == 0)].any()
+    for i in look:
         t = torch.from_numpy(tables[i, :-(-int(ctx[i]) // 16)].astype(np.int64))
         k, v = (x[t].reshape(-1, kvh, 128)[:ctx[i]] for x in (K, V))
         ref = attend(q[i].double().cpu(), k, v)

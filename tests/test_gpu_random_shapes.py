@@ -261,6 +261,5 @@ def test_paged_update_random_shapes(golden, dev, seed):
 
 @pytest.mark.parametrize("bits,S,empty_every", [(4, 100, 0), (3, 127, 2), (4, 128, 0), (2, 129, 0), (4, 256, 3), (4, 257, 2)])
 def test_partition_of_batches_beyond_a_wavefront(golden, dev, bits, S, empty_every):
-    """Whole workgroups for up to half as many non-empty sequences as there are workgroups, judged by a thread per sequence of up
-    to 256; equal ranges beyond."""
+    """More sequences than a wavefront has lanes: whole workgroups for 100 and 127, equal ranges for the others."""
     test_gpu_attention.test_partition_of_the_block_axis_by_batch_shape(golden, dev, bits, S, empty_every)

@@ -42,3 +42,34 @@ def check_codes(packed, norms, x, R, bits, ref_packed=None, ref_norms=None, d=12
     assert np.max(np.abs(ng[nz] - nr[nz]) / nr[nz]) < 1e-6
     assert np.all(ng[~nz] == 0)
     return n
+
+
+def whole_workgroups(ctx, ranges, shares, block_size=16):
+    """Whether the attention kernels give every sequence whole ones of `ranges` workgroups (akv_attn_partition), rather than cut the
+    blocks of the batch into equal ranges."""
+    chunks = [-(-(-(-int(c) // block_size)) // (32 // block_size)) for c in ctx]
+    some = sum(c > 0 for c in chunks)
+    if len(ctx) <= 64 and 0 < 8 * some <= ranges:
+        return True
+    if len(ctx) > 256 or some == 0 or 2 * some > ranges:
+        return False
+    equal = longest = max(1, -(-sum(chunks) // ranges))
+    while sum(-(-c // longest) for c in chunks) > ranges:
+        longest += 1
+    return -(-longest // shares) <= -(-equal // shares) + 1 if shares > 1 else longest <= equal + 3
+
+
+def batch_of_ranges(rng, kind):
+    """Contexts of a batch for each way its blocks are cut, with 65 to 256 sequences and at most 64, and the sequences to look at."""
+    if kind == "whole, one long":            # runs of empty sequences longer than a wavefront, one sequence in most of the workgroups
+        ctx = np.concatenate([np.zeros(70), [30000], rng.integers(1, 130, size=60), np.zeros(66), rng.integers(1, 40, size=5)])
+    elif kind == "whole, half":              # as many sequences as half the workgroups
+        ctx = rng.integers(290, 310, size=128)
+    elif kind == "equal, one long":
+        ctx = np.concatenate([rng.integers(1, 130, size=110), np.zeros(25), [30000], rng.integers(1, 130, size=110), np.zeros(10)])
+    else:                                    # "equal, few": 60 sequences do not divide the workgroups
+        ctx = rng.integers(7969, 8001, size=55 if kind == "equal, few (55)" else 60)
+    ctx = ctx.astype(np.int32)
+    some = np.flatnonzero(ctx)
+    look = some if len(some) < 100 else np.concatenate([some[:3], some[30:80:5], [int(ctx.argmax())], some[100::9], some[-2:]])
+    return ctx, look if "few" not in kind else some[[0, 1, 2, 14, 30, 53, 54]]
