@@ -737,14 +737,15 @@ int akv_attn_mfma_head_groups(int gqa);
 // At head_dim 128 the kernel of akv_attn_mfma.hip has eight head slots, most of them idle where a rank keeps one or two (groups
 // of) kv heads.  The rule takes nothing that the width of the tables changes: a serving engine's are as wide as its longest
 // context may become, whatever the contexts are.  Measured, prologue, main kernel and reduce in a graph (us, this | that), eight
-// query heads a group:
-//   one group     1 context of 700 14.7 | 14.7, of 2,700 19.7 | 20.0; 16 of 170 14.9 | 15.4; 48 of 700 17.7 | 20.1,
-//                 of 8,192 30.1 | 48.9; 64 of 100 15.9 | 18.6; 200 of 300 25.6 | 25.8; 256 of 1,000 29.5 | 39.3
-//                 (slower only near 100 of 300: 23.0 | 21.8)
-//   two groups    1 of 700 15.0 | 15.5; 32 of 700 18.5 | 18.4; 48 of 8,192 43.1 | 51.7; 64 of 100 18.0 | 20.4, of 700
-//                 21.8 | 20.8, of 3,000 32.2 | 33.0; but 200 of 300 33.0 | 31.6
-// Two groups lose once sequences no longer get whole workgroups (more than 64: akv_attn_partition): four wavefronts then merge
-// a few chunks at every change of the sequence.
+// query heads a group, 4 bits:
+//   one group     32 of 700 15.3 | 14.9; 64 of 100 14.2 | 13.8, of 700 16.5 | 17.0, of 3,000 21.3 | 29.2; 128 of 100 15.9 | 15.0, of
+//                 1,000 20.8 | 25.0, of 1,000 to 4,000 32.4 | 44.4; 200 of 300 21.5 | 21.4, of 1,000 27.8 | 33.6; 256 of 1,000 24.5 | 35.7
+//   two groups    32 of 700 17.1 | 16.1; 64 of 100 15.1 | 15.0, of 700 18.6 | 18.3, of 3,000 27.0 | 30.7;
+//                 100 of 100 17.0 | 16.3, of 300 19.7 | 18.2, of 1,000 24.6 | 26.2, of 1,000 to 8,000 50.7 | 58.3; 128 of 300
+//                 19.9 | 18.9, of 1,000 25.6 | 27.3; 200 of 300 28.0 | 26.3, of 1,000 35.8 | 37.5
+// Short contexts are up to 1.5 us faster there (it starts sooner), long ones faster here.  One group loses at most 6 % and gains up to
+// 46.  Two lose up to 8 % below 1,000 tokens and gain up to 16 above, with few sequences as with many; the host cannot see the contexts,
+// and batches of more than 64 sequences, where neither choice is the better one throughout, are left to that kernel.
 bool akv_attn_wave_applicable(const akv_attn_args& a, int d, int bits) {
   if (!(d == 64 || d == 128 || d == 256) || bits < 2 || bits > 4 || !akv_attn_mfma_takes(a, bits)) return false;
   if (d != 128) return true;
