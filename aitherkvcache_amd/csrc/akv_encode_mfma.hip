@@ -31,7 +31,7 @@
 // row is short enough; if not, or if two boundaries share a cell or lie outside (-1, 1) (no such
 // codebook is produced by the library), the kernel counts all boundaries instead.
 //
-// (Above: the kernel of the largest calls.  Calls of up to some hundred vectors a CU keep the matrix in registers: akv_encode_rows_kernel.)
+// (Above: the kernel of the larger calls.  Calls of one or two steps a CU keep the matrix in registers: akv_encode_rows_kernel.)
 //
 // A wavefront encodes EM_ROWS vectors per step (its M-tiles share every B operand read from LDS);
 // a workgroup is EM_WAVES independent wavefronts plus the B operand (64 KB) and the cell table.
@@ -135,7 +135,7 @@ __device__ __forceinline__ uint32_t em_cell(float y) {
 }
 
 // MT: M-tiles (16 vectors each) per wavefront step -- MT, or 1 for float32 input
-// SPLIT (calls of up to two thousand vectors, e.g. one serving step): a workgroup is eight wavefronts that share ONE
+// SPLIT (calls of some thousand vectors, e.g. one serving step): a workgroup is eight wavefronts that share ONE
 // step of 16 vectors, wavefront w computes N-tile w with its eighth of the B operand straight from memory in
 // registers -- no 64 KB fill, no cell table, one barrier; the codes meet in LDS and 256 threads pack and store
 // them.  Same products, same reciprocal, same comparison against the boundaries: the same codes.
@@ -683,35 +683,30 @@ __global__ __launch_bounds__(EM_THREADS) void akv_encode_mfma_kernel(akv_gen_arg
   }
 }
 
-#define ER_PER_CU 3               // workgroups: what their registers admit with four tiles of rows
-// workgroup barrier that orders LDS traffic only (what has been requested from memory keeps flying)
-__device__ __forceinline__ void er_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // ----------------------------------------------------------------------------------
-// encode with the matrix in registers: a workgroup is four wavefronts that share rows, wavefront w owns output coordinates
-// 32 w .. 32 w + 31 (two tiles of 16, both terms, 64 registers) and multiplies them into all rows of a step of 16 MT.  The threads
-// load the rows (128 / EPT lanes a row), take their norms and leave them in LDS as float16 terms, once for all wavefronts:
+// encode with the matrix in registers: a workgroup is four wavefronts that share a step of 16 MT rows, wavefront w owns output
+// coordinates 32 w .. 32 w + 31 (two tiles of 16, both terms, 64 registers) and multiplies them into all rows.  The threads
+// load the rows (16 / MT lanes a row), take their norms and leave them in LDS as float16 terms, once for all wavefronts:
 //
 //   Y[j, v] = sum_i Pi[j, i] X[v, i]              v_mfma_f32_16x16x32_f16, Pi the first operand
 //
 // Row m of tile t is coordinate 32 w + 8 (m / 4) + 4 t + m % 4, so lane (v, g) ends up with coordinates 32 w + 8 g .. + 7 of row v:
-// one group of the packed row, stored from where it is.  One barrier a step: the rows of the next step go to the other half
-// of the buffer while this one's are multiplied, and those of the one after that are on their way.  The terms, their products and the
-// order of the sums are those of the kernel above.
+// one group of the packed row, stored from where it is.  The terms, their products and the order of the sums are those of the
+// kernel above.
 // ----------------------------------------------------------------------------------
 template <int XDT, int MT> struct er_cfg {
   static constexpr int ROWS = 16 * MT, LPR = 16 / MT;             // rows of a step, lanes of a row while loading
   static constexpr int NA = XDT == AKV_F32 ? 2 : 1, NP = MT * NA; // float16 terms of a row, 16-byte pieces of a thread
   static constexpr int PITCH = 128 * 2 + 16;                      // bytes of a row in LDS (sixteen rows meet all banks)
-  static constexpr int BND = EM_CELLS * 8, DST = BND + 64, INFO = DST + 2 * ROWS * 8, DATA = INFO + 2 * ROWS * 4;
-  static constexpr int LDS = DATA + 2 * NA * ROWS * PITCH;
+  static constexpr int BND = EM_CELLS * 8, DST = BND + 64, INFO = DST + ROWS * 8, DATA = INFO + ROWS * 4;
+  static constexpr int LDS = DATA + NA * ROWS * PITCH;
 };
 // floor((2^32 - 1) / heads) and / block size; slots of the cache.  (Products in 32 and 24 bits: er_fits.  In 64 bits they were a quarter
 // of a step's vector cycles.)
 struct er_div { uint32_t heads_r, block_r, slots; };
 
 template <int BITS, bool PAGED, int XDT, int MT>
-__global__ __launch_bounds__(256, ER_PER_CU) void akv_encode_rows_kernel(akv_gen_args a, const uint4* __restrict__ bop, er_div dv) {
+__global__ __launch_bounds__(256, 3) void akv_encode_rows_kernel(akv_gen_args a, const uint4* __restrict__ bop, er_div dv) {
   extern __shared__ __align__(16) unsigned char lds[];            // the kernel's only LDS object: the cell table lies at address 0
   typedef er_cfg<XDT, MT> cfg;
   constexpr int ROWS = cfg::ROWS, LPR = cfg::LPR, NA = cfg::NA, NP = cfg::NP, PITCH = cfg::PITCH;
@@ -720,15 +715,14 @@ __global__ __launch_bounds__(256, ER_PER_CU) void akv_encode_rows_kernel(akv_gen
   const int col = lane & 15, g = lane >> 4;
   const int row = tid / LPR, part = tid % LPR;
   const uint32_t n_one = (uint32_t)a.n, n_total = PAGED && a.x2 ? 2u * n_one : n_one;
-  const uint32_t steps = (n_total + ROWS - 1) / ROWS, stride = gridDim.x;
 
-  // ---- rows of a step: thread (row, part) takes elements 8 MT part .. + 8 MT - 1
+  // ---- the rows: thread (row, part) takes elements 8 MT part .. + 8 MT - 1
   uint4 R[NP];
   uint32_t tok = 0, head = 0;
   bool second = false, held = false;
   int64_t slot = 0;
-  auto fetch = [&](uint32_t step) {
-    uint32_t n = step * ROWS + row;
+  {
+    uint32_t n = blockIdx.x * ROWS + row;
     held = n < n_total;                                          // (past the end: the last row, not stored)
     n = min(n, n_total - 1);
     second = PAGED && n >= n_one;
@@ -742,9 +736,7 @@ __global__ __launch_bounds__(256, ER_PER_CU) void akv_encode_rows_kernel(akv_gen
 #pragma unroll
       for (int h = 0; h < NA; ++h) R[i * NA + h] = *(const uint4*)(p + (part * MT + i) * 8 * XB + 16 * h);
     if constexpr (PAGED) slot = akv_load_index(a.slots, a.slot_itype, tok);
-  };
-  uint32_t step = blockIdx.x;
-  fetch(step);
+  }
 
   // ---- the wavefront's tiles of the matrix
   em_half8 Ph[2][4], Pl[2][4];
@@ -791,8 +783,8 @@ __global__ __launch_bounds__(256, ER_PER_CU) void akv_encode_rows_kernel(akv_gen
     }
   }
 
-  // ---- the rows held: norm, float16 terms into half `buf` of the buffer, where the packed row goes
-  auto convert = [&](int buf) {
+  // ---- norms, float16 terms into LDS, where the packed rows go
+  {
     // squared norm: a quarter of the row is one chain of sums, as above, which its 4 / MT lanes walk one after another
     float ss = 0.f;
 #pragma unroll
@@ -888,7 +880,7 @@ __global__ __launch_bounds__(256, ER_PER_CU) void akv_encode_rows_kernel(akv_gen
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      unsigned char* p = lds + cfg::DATA + (buf * NA * ROWS + row) * PITCH + (part * MT + i) * 16;
+      unsigned char* p = lds + cfg::DATA + row * PITCH + (part * MT + i) * 16;
       *(uint4*)p = hi[i];
       if constexpr (NA == 2) *(uint4*)(p + ROWS * PITCH) = lo[i];
     }
@@ -910,20 +902,21 @@ __global__ __launch_bounds__(256, ER_PER_CU) void akv_encode_rows_kernel(akv_gen
       nb += tok;
     }
     if (part == LAST) {
-      ((uint64_t*)(lds + cfg::DST))[buf * ROWS + row] = stored ? (uint64_t)(uintptr_t)pb : 0u;
-      ((float*)(lds + cfg::INFO))[buf * ROWS + row] = nan_row ? __uint_as_float(0x7fc00000u) : r;
+      ((uint64_t*)(lds + cfg::DST))[row] = stored ? (uint64_t)(uintptr_t)pb : 0u;
+      ((float*)(lds + cfg::INFO))[row] = nan_row ? __uint_as_float(0x7fc00000u) : r;
       if (stored) *nb = nrm;
     }
-  };
+  }
+  __syncthreads();
 
   // ---- rotate, search, pack, store
-  auto encode = [&](auto linear_tag, int buf) {
+  auto encode = [&](auto linear_tag) __attribute__((always_inline)) {
     constexpr bool LINEAR = decltype(linear_tag)::value;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      const int v = buf * ROWS + 16 * mt + col;
+      const int v = 16 * mt + col;
       em_float4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-      const unsigned char* p = lds + cfg::DATA + (buf * NA * ROWS + 16 * mt + col) * PITCH + 64 * g;
+      const unsigned char* p = lds + cfg::DATA + v * PITCH + 64 * g;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         const em_half8 x = *(const em_half8*)(p + 16 * ks);
@@ -977,22 +970,12 @@ __global__ __launch_bounds__(256, ER_PER_CU) void akv_encode_rows_kernel(akv_gen
     }
   };
 
-  convert(0);
-  if (step + stride < steps) fetch(step + stride);
-  __syncthreads();
-  auto all = [&](auto linear_tag) __attribute__((always_inline)) {
-    for (int buf = 0; step < steps; step += stride, buf ^= 1) {
-      if (step + stride < steps) {
-        convert(buf ^ 1);                            // (that half was read before the barrier)
-        if (step + 2 * stride < steps) fetch(step + 2 * stride);
-      }
-      encode(linear_tag, buf);
-      er_barrier();
-    }
-  };
-  if (__builtin_expect(!linear, 1)) all(std::false_type{});
-  else all(std::true_type{});
+  if (__builtin_expect(!linear, 1)) encode(std::false_type{});
+  else encode(std::true_type{});
 }
+
+// rows a CU up to which a call of 16-bit rows shares each step of 16 among eight wavefronts (akv_encode_mfma_try)
+static constexpr int em_split_rows(int bits, bool paged) { return paged && bits != 4 ? 8 : 16; }
 
 // what the kernel's 32- and 24-bit products take
 static bool er_fits(const akv_gen_args& a, bool paged, int64_t n_total) {
@@ -1005,22 +988,21 @@ static bool er_fits(const akv_gen_args& a, bool paged, int64_t n_total) {
 }
 
 template <int BITS, bool PAGED, int XDT, int MT>
-static int er_launch(const akv_gen_args& a, const uint4* bop, const er_div& dv, int grid, hipStream_t stream) {
-  AKV_LAUNCH_TIMED((akv_encode_rows_kernel<BITS, PAGED, XDT, MT>), grid, 256, (er_cfg<XDT, MT>::LDS), stream, a, bop, dv);
+static int er_launch(const akv_gen_args& a, const uint4* bop, const er_div& dv, int64_t n, hipStream_t stream) {
+  AKV_LAUNCH_TIMED((akv_encode_rows_kernel<BITS, PAGED, XDT, MT>), (int)((n + 16 * MT - 1) / (16 * MT)), 256, (er_cfg<XDT, MT>::LDS), stream, a, bop, dv);
   AKV_LAUNCH_CHECK("akv_encode_rows_kernel");
   return AKV_OK;
 }
+// steps of 16, 32 or 64 rows (float32: of 32 at most), so that a call that gives a CU one step has it on every CU
 template <int BITS, bool PAGED, int XDT>
 static int er_run_rows(const akv_gen_args& a, const uint4* bop, int64_t n, int cus, hipStream_t stream) {
   er_div dv = {0u, 0u, 0u};
   if constexpr (PAGED) dv = {0xffffffffu / (uint32_t)a.heads, 0xffffffffu / (uint32_t)a.block_size, (uint32_t)(a.max_blocks * a.block_size)};
-  const int tiles = n <= 16 * (int64_t)cus ? 1 : XDT == AKV_F32 || n <= 32 * (int64_t)cus ? 2 : 4;
-  const int64_t steps = (n + 16 * tiles - 1) / (16 * tiles), most = ER_PER_CU * (int64_t)cus;
-  const int grid = (int)(steps < most ? steps : most);
-  if (tiles == 1) return er_launch<BITS, PAGED, XDT, 1>(a, bop, dv, grid, stream);
+  if constexpr (XDT == AKV_F32 || em_split_rows(BITS, PAGED) < 16)
+    if (n <= 16 * (int64_t)cus) return er_launch<BITS, PAGED, XDT, 1>(a, bop, dv, n, stream);
   if constexpr (XDT != AKV_F32)
-    if (tiles == 4) return er_launch<BITS, PAGED, XDT, 4>(a, bop, dv, grid, stream);
-  return er_launch<BITS, PAGED, XDT, 2>(a, bop, dv, grid, stream);
+    if (n > 32 * (int64_t)cus) return er_launch<BITS, PAGED, XDT, 4>(a, bop, dv, n, stream);
+  return er_launch<BITS, PAGED, XDT, 2>(a, bop, dv, n, stream);
 }
 static int er_run(const akv_gen_args& a, bool paged, int x_dtype, int bits, const uint4* bop, int64_t n, int cus, hipStream_t stream) {
 #define ER_DT(BB, PG) (x_dtype == AKV_F16 ? er_run_rows<BB, PG, AKV_F16>(a, bop, n, cus, stream) : x_dtype == AKV_BF16 ? er_run_rows<BB, PG, AKV_BF16>(a, bop, n, cus, stream) \
@@ -1063,19 +1045,26 @@ int akv_encode_mfma_try(const akv_gen_args& a, bool paged, int x_dtype, int d, i
   const uint4* bop = (const uint4*)((const float*)rot_prep + (size_t)2 * d * d);
   const int64_t n_total = (paged && a.x2) ? 2 * a.n : a.n;
   const int cus = akv_cached_cu_count() > 0 ? akv_cached_cu_count() : 256;
-  // Calls of up to some hundred vectors a CU take the kernel with the matrix in registers: no 64 KB fill, and a wavefront's chain
-  // is a quarter of a row's tiles.  Steps of 16, 32 or 64 rows, so that the calls that give a CU one step have it on every CU.
-  // Keys and values in bfloat16 and 4 bits, us, the kernel above | that one: 8,192 vectors 8.5 | 5.8, 16,384 9.3 | 6.9, 32,768
-  // 10.1 | 8.9, 65,536 13.4 | 12.7, 131,072 20.8 | 19.1; but 192,000 24.8 | 25.6, and rows that fill its workgroups with two steps
-  // each, 88,000 to 98,304, 16.3 to 17.0 | 16.8 to 17.2.  Float16, no conversion to share: 32,768 9.4 | 8.6, but 48,000 11.6 | 11.7,
-  // 80,000 14.2 | 14.7; flat rows, of which that kernel checks none, 65,536 11.4 | 12.2.  3 bits, three stores of a byte: 32,768 8.9 | 8.4, 48,000 11.3 | 11.3, 65,536 12.6 | 12.8.  Float32: 1,600
-  // 7.8 | 5.2, 16,384 8.9 | 8.0, 20,320 10.5 | 10.4, 32,768 11.9 | 12.2.
-  // The fewest share each step of 16 vectors among eight wavefronts: 2,048 vectors 5.0 | 5.2, 4,096 5.4 | 5.2.
-  const int64_t per_cu = n_total / cus;
+  // Calls that give a CU at most one step of 64 rows (float32: 32), or two where the rows are checked slot by slot or have 3 bits,
+  // take the kernel with the matrix in registers: no 64 KB fill, and a wavefront's chain is a quarter of a row's tiles.  A second
+  // or third step a CU brings the matrix in again, so the kernel above takes over at once.  A call among others, inputs in
+  // turn, us, the kernel above | that one, at the last size of the rule and the next above it:
+  //   paged bf16 4 bits 64 rows a CU 9.4 | 6.8, 128 10.6 | 9.7, 136 11.8 | 11.8, 192 12.3 | 12.4, 352 16.0 | 16.9
+  //               3 bits 128 10.2 | 9.7, 136 11.3 | 12.0; 2 bits 128 9.7 | 9.3, 136 10.8 | 11.3
+  //         f16  4 bits 128 10.1 | 9.6, 160 11.2 | 12.0; 3 bits 9.6 | 9.4, 10.7 | 11.9; 2 bits 9.3 | 9.0, 10.3 | 11.3
+  //         f32  4 bits 64 9.6 | 9.0, 80 10.7 | 11.1; 3 bits 9.1 | 8.6, 10.1 | 10.8; 2 bits 8.7 | 8.2, 9.6 | 10.3
+  //   flat  f16  4 bits 64 7.7 | 6.3, 68 7.7 | 8.3; 2 bits 6.9 | 5.7, 6.9 | 7.5; 3 bits 128 9.2 | 8.8, 160 10.2 | 11.2
+  //         bf16 4 bits 64 8.1 | 6.5, 80 8.5 | 8.9; 2 bits 7.2 | 5.8, 7.7 | 7.9; 3 bits 128 9.7 | 9.1, 160 11.1 | 11.4
+  //         f32  4 bits 32 7.3 | 5.8, 48 8.1 | 8.5; 3 bits 6.8 | 5.4, 7.7 | 8.1; 2 bits 6.3 | 5.2, 7.1 | 7.8
+  // (Beyond, several steps a workgroup with rows of the next on their way were faster here and there, paged bf16 4 bits 512 rows a CU 20.2 | 19.0,
+  // and slower as often, 384 16.5 | 17.0, 2 bits 15.3 | 16.5, 768 26.6 | 28.1: nothing to go by.)
+  // The fewest share each step of 16 rows among eight wavefronts, that | this form: 16 rows a CU paged f16 4 bits 4.9 | 4.7, bf16
+  // 5.1 | 5.1 (12 rows 5.1 | 5.0), but 3 bits 4.4 | 4.5, 4.5 | 4.9, 2 bits 4.1 | 4.3, 4.2 | 4.7; flat f16 4.8 | 4.2, bf16 4.9 | 4.5, 3 bits
+  // 4.2 | 4.0, 2 bits 4.1 | 3.9; 24 rows flat f16 4 bits 7.9 | 8.8.
   const bool plain = getenv("AKV_ENCODE_NO_SPLIT") != nullptr;
-  const bool split = x_dtype != AKV_F32 && n_total <= 8 * (int64_t)cus && !plain;
-  const bool rows = x_dtype == AKV_F32 ? per_cu <= 80 : bits == 3 ? per_cu <= 128 : x_dtype == AKV_F16 || !paged ? per_cu <= 160 : per_cu < 340 || (per_cu > 384 && per_cu <= 512);
-  if (rows && !split && !plain && er_fits(a, paged, n_total)) return er_run(a, paged, x_dtype, bits, bop, n_total, cus, stream);
+  const bool split = x_dtype != AKV_F32 && n_total <= em_split_rows(bits, paged) * (int64_t)cus && !plain;
+  const int64_t most = (x_dtype == AKV_F32 ? 32 : 64) * (int64_t)cus * (paged || (bits == 3 && x_dtype != AKV_F32) ? 2 : 1);
+  if (n_total <= most && !split && !plain && er_fits(a, paged, n_total)) return er_run(a, paged, x_dtype, bits, bop, n_total, cus, stream);
   const int rows_per_step = (x_dtype == AKV_F32 || split) ? 16 : EM_ROWS;
   const int64_t steps = (n_total + rows_per_step - 1) / rows_per_step;
   // steps are dealt round-robin over workgroups first, so a small call (one serving step) spreads

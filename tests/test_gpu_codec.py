@@ -275,7 +275,7 @@ def test_small_paged_calls_share_a_step_among_wavefronts(golden, dev, bits, dtyp
     P = tq._packed_dim
     NB, BS, H = 40, 16, 8
     rng = np.random.default_rng(500 + bits)
-    for T in (1, 37, 256, 600):                       # 8 .. 4,800 vectors: one step, ragged, a serving step, two steps per workgroup
+    for T in (1, 37, 256, 600):                       # 8 .. 4,800 vectors: one step, ragged, a serving step, more than are shared
         x = kv_like(rng, (T, H, 128)).astype(np.float32)
         if T > 30:
             x[3, 1, 5] = np.nan
@@ -688,21 +688,28 @@ def test_read_probe_sums_what_it_reads(dev):
 
 @pytest.mark.parametrize("bits", [2, 3, 4])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T,H,BS", [(257, 8, 16), (585, 7, 24), (293, 28, 32), (7100, 7, 16)])
-def test_calls_of_some_hundred_rows_a_cu_write_the_bytes_of_the_large_ones(golden, dev, bits, dtype, T, H, BS, monkeypatch):
-    """Keys and values through the kernel with the matrix in registers -- steps of 16, 32 and 64 rows, a last step of a few, one step
-    a workgroup and several, heads and block sizes that are no powers of two -- and through the one with the matrix in LDS:
-    codes, norms and untouched rows byte for byte, with NaN, infinite and zero rows and slots outside the cache."""
+@pytest.mark.parametrize("form,T,H,BS", [("paged", 203, 8, 16), ("paged", 257, 8, 16), ("paged", 585, 7, 24), ("paged", 292, 28, 32), ("paged", 2340, 7, 16),
+                                         ("flat", 4095, 1, 0), ("flat", 4097, 1, 0), ("flat", 8191, 1, 0), ("flat", 8193, 1, 0), ("flat", 16381, 1, 0), ("flat", 32767, 1, 0)])
+def test_calls_of_a_step_or_two_a_cu_write_the_bytes_of_the_large_ones(golden, dev, bits, dtype, form, T, H, BS, monkeypatch):
+    """Keys and values, or flat rows, through the kernel with the matrix in registers -- steps of 16, 32 and 64 rows, a last step of a
+    few, one and two steps a CU, heads and block sizes that are no powers of two -- and through the one with the matrix in LDS:
+    codes, norms and untouched rows byte for byte, with NaN, infinite and zero rows and slots outside the cache.  (What the rule
+    leaves to other kernels is not run: a kernel would be held against itself.)"""
+    cus, n = torch.cuda.get_device_properties(dev).multi_processor_count, (2 if form == "paged" else 1) * T * H
+    wide = 32 if dtype == torch.float32 else 64
+    fewest = -1 if dtype == torch.float32 else 8 if form == "paged" and bits != 4 else 16
+    if not fewest * cus < n <= wide * cus * (2 if form == "paged" or (bits == 3 and wide == 64) else 1):
+        pytest.skip("another kernel's")
     tq = make_tq(golden, dev, bits)
     P = tq._packed_dim
-    NB = -(-T // BS) + 1
+    NB = -(-T // BS) + 1 if form == "paged" else 1
     rng = np.random.default_rng(900 + bits + T)
     xs = []
     for _ in range(2):
         x = kv_like(rng, (T, H, 128)).astype(np.float32)
-        x[3, 1, 5], x[4, 2, 7], x[5, 0] = np.nan, np.inf, 0
+        x[3, -1, 5], x[4, -1, 7], x[5, 0] = np.nan, np.inf, 0
         xs.append(torch.from_numpy(x).to(dev).to(dtype))
-    slots = rng.permutation(NB * BS)[:T].astype(np.int64)
+    slots = rng.permutation(max(T, NB * BS))[:T].astype(np.int64)
     slots[::9], slots[1::11] = -1, NB * BS + 5
     sd = torch.from_numpy(slots).to(dev)
     outs = []
@@ -710,22 +717,24 @@ def test_calls_of_some_hundred_rows_a_cu_write_the_bytes_of_the_large_ones(golde
         monkeypatch.delenv("AKV_ENCODE_NO_SPLIT", raising=False)
         if off:
             monkeypatch.setenv("AKV_ENCODE_NO_SPLIT", "1")
+        if form == "flat":
+            outs.append([t.cpu().numpy() for t in tq.encode(xs[0].reshape(-1, 128))])
+            continue
         rows = [torch.full((NB, BS, H, P + 4), 0xAB, dtype=torch.uint8, device=dev) for _ in range(2)]
         norms = [torch.full((NB, BS, H), -5.0, device=dev) for _ in range(2)]
         akv.fused_kv_update_pair(xs[0], xs[1], sd, rows[0][..., :P], norms[0], rows[1][..., :P], norms[1], tq.rotation, tq.boundaries_inner, bits, block_size=BS)
-        flat = tq.encode(xs[0].reshape(-1, 128))
-        outs.append([t.cpu().numpy() for t in (*rows, *norms, *flat)])
+        outs.append([t.cpu().numpy() for t in (*rows, *norms)])
     monkeypatch.delenv("AKV_ENCODE_NO_SPLIT", raising=False)
     for a, b in zip(*outs):
         assert np.array_equal(a, b, equal_nan=a.dtype != np.uint8)
-    ok = (slots >= 0) & (slots < NB * BS)
-    assert int(np.sum(outs[0][2] != -5.0)) == int(ok.sum()) * H
+    if form == "paged":
+        assert int(np.sum(outs[0][2] != -5.0)) == int(np.sum((slots >= 0) & (slots < NB * BS))) * H
 
 
 def test_encode_rows_far_apart(golden, dev, monkeypatch):
     """Positions of a block further apart than 24 bits hold: the call keeps to 64-bit offsets and writes the same bytes."""
     tq = make_tq(golden, dev, 4)
-    P, H, T = tq._packed_dim, 2, 1100
+    P, H, T = tq._packed_dim, 2, 2100
     x = torch.from_numpy(kv_like(np.random.default_rng(41), (T, H, 128))).to(dev)
     slots = torch.full((T,), -1, dtype=torch.int64, device=dev)
     slots[:16] = torch.arange(16, device=dev).flip(0)
