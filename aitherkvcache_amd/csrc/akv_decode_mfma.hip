@@ -35,7 +35,6 @@ typedef float dm_float4 __attribute__((ext_vector_type(4)));
 typedef float dm_float2 __attribute__((ext_vector_type(2)));
 typedef _Float16 dm_half2 __attribute__((ext_vector_type(2)));
 typedef __bf16 dm_bf162 __attribute__((ext_vector_type(2)));
-typedef uint32_t dm_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t dm_u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const uint32_t dm_lds_cu32;
 typedef __attribute__((address_space(3))) dm_u32x4 dm_lds_u128;

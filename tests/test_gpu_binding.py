@@ -212,11 +212,20 @@ def test_out_of_memory_is_the_error_of_torch(dev, monkeypatch, make, fmt, d, tak
     run(x[:, :BS], slots[:BS], tables, lens, q)                     # the attention's workspace is there
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    # a segment of torch's that is held for a part of it, as other tests may leave them: there is room in it for the output
+    whole = torch.empty(600 << 20, dtype=torch.uint8, device=dev)
+    del whole
+    held = [torch.empty(20 << 20, dtype=torch.uint8, device=dev)]
+    torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(dev).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (16 << 20)) / total, dev)
     try:
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:                                             # (what such segments have left)
+                held.append(torch.empty(16 << 20, dtype=torch.uint8, device=dev))
         with binding(monkeypatch, take), pytest.raises(torch.OutOfMemoryError):
             run(x[:, :BS], slots[:BS], tables, lens, q)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0, dev)
+        del held
     assert not run(x[:, :BS], slots[:BS], tables, lens, q)[-1].any()
