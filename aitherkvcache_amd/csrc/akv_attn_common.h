@@ -156,9 +156,9 @@ __device__ __forceinline__ int akv_block_prefix_scan(const void* context_lens, i
   return base + inc - sum;
 }
 
-// longest range of whole workgroups against an equal cut, in chunks
-__device__ __forceinline__ bool akv_attn_aligned_pays(int aligned, int equal, int shares) {
-  return shares > 1 ? (aligned + shares - 1) / shares <= (equal + shares - 1) / shares + 1 : aligned <= equal + 3;
+// longest range of whole workgroups against an equal cut, in chunks (akv_attn_partition)
+__device__ __forceinline__ bool akv_attn_aligned_pays(int aligned, int equal, int shares, int longer) {
+  return shares > 1 ? (aligned + shares - 1) / shares <= (equal + shares - 1) / shares + 1 : aligned <= equal + max(longer, equal <= 8 ? 1 : 0);
 }
 
 // the last i < n (a power of two) with entry[i] <= v: entries non-decreasing, entry[0] <= v
@@ -185,11 +185,18 @@ __device__ __forceinline__ int akv_last_at_most(const int32_t* entry, int n, int
 // of a workgroup go through its chunks side by side and merge their results at the end of every segment.
 //
 // Whole workgroups: with at most 64 sequences always where the non-empty ones are at most G / 8.  A second segment costs a
-// workgroup as much as three chunks or one more round of chunks of its shares, so also with up to 256 sequences, the non-empty
-// ones at most half the workgroups, while the longest range is no more than that longer than an equal one.  One
+// workgroup as much as some chunks or one more round of chunks of its shares, so also with up to 256 sequences, the non-empty
+// ones at most half the workgroups, while the longest range is no more than that longer than an equal one (`longer`, from eight
+// chunks down at least one).  One
 // kv head, 48 sequences: of 700 tokens 21.3 -> 17.7 us, of 1k to 16k the step 41.2 -> 36.6.  Eight kv heads: the step of 40
 // sequences of 300 to 3,000 39.3 -> 35.0 us, of 64 of 100 to 1,500 40.6 -> 33.7, of 100 of 200 to 1,000 42.0 -> 37.6, of 128 of 300 33.1, 41.9 before;
 // heads of 256 55.5 -> 49.5, tq35 65.2 -> 56.1.
+// Attention of batches of G / 8 to G / 2 sequences of 250 to 6,000 tokens, equal ranges over whole workgroups, by what these are longer:
+//   kernel of akv_attn_mfma.hip        none 1.00 to 1.33, 1 chunk 1.04 to 1.33, 2 1.04 to 1.15, 3 1.03 to 1.06, 12 0.95 to 0.99
+//   independent wavefronts, one share  none 0.99 to 1.35, 1 1.00 to 1.26, 2 0.99 to 1.15, 3 0.96 to 1.08 (heads of 64 0.98 to 1.00), 4 0.97 to 1.06
+//   as many workgroups as half again the chip holds (tq35, groups of other than four heads, from three groups or heads on): the ranges of a CU
+//     take turns, a second segment hides behind another's products and a longer range does not: none 0.97 to 1.58, 1 chunk up to
+//     ranges of eight 1.00 to 1.17, beyond 0.91 to 1.02, 2 0.90 to 1.03, 3 0.91 to 0.99
 //
 // At most 64 sequences are held by one wavefront, more by a thread each (or several each); records are written by a thread per
 // workgroup, which finds its sequence among the starts in LDS.  (By a thread per sequence, one of 30,000 tokens among 99 of
@@ -198,7 +205,7 @@ __device__ __forceinline__ int akv_last_at_most(const int32_t* entry, int n, int
 #define AKV_PART_WORDS 592              // LDS of akv_attn_partition (int32 words)
 __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G, int cb, int32_t* wgdesc, int32_t* seqw,
                                                    int32_t* lds /*[AKV_PART_WORDS]*/, const void* context_lens, int cl_itype,
-                                                   int block_size, int64_t max_blocks_per_seq, int shares = 1) {
+                                                   int block_size, int64_t max_blocks_per_seq, int shares, int longer) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int n = S > 64 ? 256 : 64;      // starts in LDS: of every sequence, beyond 256 of every `chunk`-th
   const int chunk = (S + 255) / 256;
@@ -236,7 +243,7 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
           const int mid = (lo + hi) >> 1;
           if (sum_all((c + mid - 1) / mid) <= G) hi = mid; else lo = mid + 1;
         }
-        aligned = akv_attn_aligned_pays(lo, equal, shares);
+        aligned = akv_attn_aligned_pays(lo, equal, shares, longer);
       }
       if (aligned) {
         const int k = (c + lo - 1) / lo;
@@ -290,7 +297,7 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
         const int tot = akv_wave_sum((c + mid - 1) / mid);
         if (tot <= G) hi = mid; else lo = mid + 1;
       }
-      if (akv_attn_aligned_pays(lo, equal, shares)) aligned = true;
+      if (akv_attn_aligned_pays(lo, equal, shares, longer)) aligned = true;
     }
     if (aligned) {
       const int k = (c + lo - 1) / lo;

@@ -1067,13 +1067,13 @@ __global__ __launch_bounds__(256) void akv_attn_hyb_prologue_kernel(
     const void* __restrict__ query, int64_t qs_seq, int64_t qs_head, const float* __restrict__ table, float qscale, int S, int QH,
     int KVH, int hgroup, int gqa, const void* context_lens, int cl_itype, int block_size, int64_t max_blocks_per_seq, int32_t* prefix,
     uint4* __restrict__ qop, float* __restrict__ fac, uint32_t* __restrict__ lut, uint32_t* __restrict__ status, uint32_t start_status,
-    int32_t* __restrict__ wgdesc, int32_t* __restrict__ seqw, int G, int shares) {
+    int32_t* __restrict__ wgdesc, int32_t* __restrict__ seqw, int G, int shares, int longer) {
   __shared__ int8_t dig[3][4][256];       // [digit][query head][sum]
   __shared__ int32_t scratch[AKV_PART_WORDS];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   if (blockIdx.x == 0) {
     if (tid == 0) status[0] = start_status;
-    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares);
+    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares, longer);
     return;
   }
   if (blockIdx.x == 1) {
@@ -1236,10 +1236,12 @@ template <class F> struct hw_type { typedef F type; };
 template <class F, class M>
 static int hw_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_head, const float* table, float scale, const hw_args& a,
                   const akv_attn_ws& ws, void* out, int out_dtype, int64_t os_seq, int64_t os_head, hipStream_t stream, M main) {
-  const int G = hw_ranges(a.KVH, a.hp), shares = HW_W / a.hp;
+  const int G = hw_ranges(a.KVH, a.hp), shares = HW_W / a.hp, cus = akv_cached_cu_count();
+  // (akv_attn_partition: a second segment in chunks; nothing where more workgroups take turns than the chip holds)
+  const int longer = G * a.hgroups > F::PER_SIMD * (cus > 0 ? cus : 256) ? 0 : 2;
   const float qscale = scale * 1.4426950408889634f;      // scores come out in the log2 domain
   const uint32_t start_status = g_spin_limit == 0 ? AKV_STATUS_HANDOFF_TIMEOUT : 0u;
-#define HW_PRO(DT) akv_attn_hyb_prologue_kernel<F, DT><<<a.S * a.KVH + 2, 256, 0, stream>>>(query, qs_seq, qs_head, table, qscale, a.S, a.QH, a.KVH, a.hgroup, a.gqa, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint4*)a.qop, ws.qrot, ws.lut, ws.status, start_status, ws.wgdesc, ws.seqw, G, shares)
+#define HW_PRO(DT) akv_attn_hyb_prologue_kernel<F, DT><<<a.S * a.KVH + 2, 256, 0, stream>>>(query, qs_seq, qs_head, table, qscale, a.S, a.QH, a.KVH, a.hgroup, a.gqa, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint4*)a.qop, ws.qrot, ws.lut, ws.status, start_status, ws.wgdesc, ws.seqw, G, shares, longer)
   if (q_dtype == AKV_F16) HW_PRO(AKV_F16); else if (q_dtype == AKV_BF16) HW_PRO(AKV_BF16); else HW_PRO(AKV_F32);
 #undef HW_PRO
   AKV_LAUNCH_CHECK("akv_attn_hyb_prologue_kernel");

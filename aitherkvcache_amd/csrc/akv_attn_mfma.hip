@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void akv_attn_mfma_prologue_kernel(
   if ((int)blockIdx.x == 0) {
     if (tid == 0) status[0] = 0u;
     akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size,
-                       max_blocks_per_seq);
+                       max_blocks_per_seq, 1, 3);
     return;
   }
   if ((int)blockIdx.x == 1) {

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void akv_attn_wave_prologue_kernel(
   __shared__ int32_t scratch[AKV_PART_WORDS];
   if (blockIdx.x == 0) {
     if (threadIdx.x == 0) status[0] = 0u;
-    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares);
+    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares, 2);
     return;
   }
   ar_rotate_queries<D, QDT, false>(rows, (int)blockIdx.x - 1, (int)gridDim.x - 1, query, qs_seq, qs_head, Pi, scale, S, QH, KVH, slots, qop, fac, qscale, bits);

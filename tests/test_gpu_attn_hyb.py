@@ -214,21 +214,23 @@ def test_many_sequences_and_empty_ones_vs_float64(dev, mode, qh, kvh):
         assert (out[i] - ref).norm() <= limit(mode, qh, kvh) * ref.norm(), (i, ctx[i])
 
 
-@pytest.mark.parametrize("kind", ["whole, one long", "whole, half", "equal, one long", "equal, few (55)"])
-# (workgroups a compute unit: three for two groups of four kv head slots at a time, or two; wavefronts of a kv head)
-@pytest.mark.parametrize("mode,qh,kvh,per_cu,shares", [("tq35", 32, 8, 1.5, 1), ("tq25", 12, 2, 2, 2)])
-def test_ranges_of_workgroups_vs_float64(dev, mode, qh, kvh, per_cu, shares, kind):
+@pytest.mark.parametrize("mode,qh,kvh,per_cu,kind", [
+    # two groups of four kv head slots: three workgroups a compute unit
+    ("tq35", 32, 8, 1.5, "whole, one long"), ("tq35", 32, 8, 1.5, "whole, half"), ("tq35", 32, 8, 1.5, "equal, one long"), ("tq35", 32, 8, 1.5, "equal, most"),
+    ("tq35", 32, 8, 1.5, "equal, few (55)"),
+    # four of them, and a kernel of which two workgroups fit a compute unit: longer ranges do not pay
+    ("tq35", 40, 8, 0.75, "equal, ragged"), ("tq35", 40, 8, 0.75, "whole, short"),
+    # one, in pairs of wavefronts
+    ("tq25", 12, 2, 2, "whole, one long"), ("tq25", 12, 2, 2, "whole, half"), ("tq25", 12, 2, 2, "equal, most")])
+def test_ranges_of_workgroups_vs_float64(dev, mode, qh, kvh, per_cu, kind):
     rng, h, rows = make(dev, mode, kvh, 40, 16, 64 if mode == "tq35" else 44, qh)
     ctx, look = batch_of_ranges(rng, kind)
-    whole = whole_workgroups(ctx, int(per_cu * torch.cuda.get_device_properties(dev).multi_processor_count), shares)
-    if mode == "tq25" and kind.startswith("equal"):
-        assert whole
-        pytest.skip("512 workgroups: whole ones")
-    assert whole == kind.startswith("whole")
     tables = rng.integers(0, 40, size=(len(ctx), int(ctx.max() + 15) // 16)).astype(np.int32)
     K, V = (h.decode(r.contiguous()).double().cpu() for r in rows)
     q = torch.from_numpy(rng.standard_normal((len(ctx), qh, 128)).astype(np.float32)).to(dev)
-    out = akv.HybridPagedAttention(h, qh).forward(q, rows[0], rows[1], torch.from_numpy(tables).to(dev), torch.from_numpy(ctx).to(dev)).double().cpu()
+    attn = akv.HybridPagedAttention(h, qh)
+    out = attn.forward(q, rows[0], rows[1], torch.from_numpy(tables).to(dev), torch.from_numpy(ctx).to(dev)).double().cpu()
+    assert whole_workgroups(attn, int(per_cu * torch.cuda.get_device_properties(dev).multi_processor_count), ctx) == kind.startswith("whole")
     assert not out[torch.from_numpy(ctx == 0)].any()
     for i in look:
         t = torch.from_numpy(tables[i, :-(-int(ctx[i]) // 16)].astype(np.int64))

@@ -44,19 +44,23 @@ def check_codes(packed, norms, x, R, bits, ref_packed=None, ref_norms=None, d=12
     return n
 
 
-def whole_workgroups(ctx, ranges, shares, block_size=16):
-    """Whether the attention kernels give every sequence whole ones of `ranges` workgroups (akv_attn_partition), rather than cut the
-    blocks of the batch into equal ranges."""
-    chunks = [-(-(-(-int(c) // block_size)) // (32 // block_size)) for c in ctx]
-    some = sum(c > 0 for c in chunks)
-    if len(ctx) <= 64 and 0 < 8 * some <= ranges:
-        return True
-    if len(ctx) > 256 or some == 0 or 2 * some > ranges:
-        return False
-    equal = longest = max(1, -(-sum(chunks) // ranges))
-    while sum(-(-c // longest) for c in chunks) > ranges:
-        longest += 1
-    return -(-longest // shares) <= -(-equal // shares) + 1 if shares > 1 else longest <= equal + 3
+def whole_workgroups(attn, ranges, ctx, block_size=16):
+    """How the last call of an attention object cut the blocks of its batch among `ranges` workgroups, from the records in its
+    workspace (behind 4,352 bytes: range, sequence, the sequence's blocks, its tokens): whole ones for every sequence, or ranges that cross
+    sequences.  The records are checked on the way."""
+    records = attn._workspace[4352:4352 + 32 * ranges].cpu().numpy().view(np.int32).reshape(ranges, 8)
+    ends = np.cumsum(-(-np.asarray(ctx, dtype=np.int64) // block_size))
+    at, whole = 0, True
+    for g0, g1, seq, sb0, sb1, tokens in records[:, :6]:
+        if g0 >= g1:
+            assert seq == -1
+            continue
+        assert g0 == at and seq == np.searchsorted(ends, g0, side="right"), (g0, g1, seq)
+        assert (sb0, sb1, tokens) == (ends[seq - 1] if seq else 0, ends[seq], ctx[seq]), (g0, seq)
+        whole &= bool(g1 <= sb1)
+        at = g1
+    assert at == ends[-1]
+    return whole
 
 
 def batch_of_ranges(rng, kind):
@@ -65,11 +69,17 @@ def batch_of_ranges(rng, kind):
         ctx = np.concatenate([np.zeros(70), [30000], rng.integers(1, 130, size=60), np.zeros(66), rng.integers(1, 40, size=5)])
     elif kind == "whole, half":              # as many sequences as half the workgroups
         ctx = rng.integers(290, 310, size=128)
+    elif kind == "whole, short":
+        ctx = rng.integers(230, 256, size=60)
     elif kind == "equal, one long":
         ctx = np.concatenate([rng.integers(1, 130, size=110), np.zeros(25), [30000], rng.integers(1, 130, size=110), np.zeros(10)])
-    else:                                    # "equal, few": 60 sequences do not divide the workgroups
+    elif kind == "equal, most":              # more than are held by a thread each: two or three starts a thread
+        ctx = np.concatenate([rng.integers(1, 130, size=300), np.zeros(100), [30000], rng.integers(1, 130, size=200), np.zeros(60)])
+    elif kind == "equal, ragged":            # a decode batch of mixed lengths
+        ctx = rng.integers(532, 10112, size=33)
+    else:                                    # "equal, few": sequences that do not divide the workgroups
         ctx = rng.integers(7969, 8001, size=55 if kind == "equal, few (55)" else 60)
     ctx = ctx.astype(np.int32)
     some = np.flatnonzero(ctx)
     look = some if len(some) < 100 else np.concatenate([some[:3], some[30:80:5], [int(ctx.argmax())], some[100::9], some[-2:]])
-    return ctx, look if "few" not in kind else some[[0, 1, 2, 14, 30, 53, 54]]
+    return ctx, look if "few" not in kind and "ragged" not in kind else some[[0, 1, 2, 14, 30, -2, -1]]
