@@ -161,12 +161,14 @@ __device__ __forceinline__ bool akv_attn_aligned_pays(int aligned, int equal, in
   return shares > 1 ? (aligned + shares - 1) / shares <= (equal + shares - 1) / shares + 1 : aligned <= equal + max(longer, equal <= 8 ? 1 : 0);
 }
 
-// the last i < n (a power of two) with entry[i] <= v: entries non-decreasing, entry[0] <= v
-__device__ __forceinline__ int akv_last_at_most(const int32_t* entry, int n, int v) {
-  int at = 0;
-  for (int step = n >> 1; step > 0; step >>= 1)
-    if (entry[at + step] <= v) at += step;
-  return at;
+// the last i < n (a power of two) with entry[i] <= v, for two v side by side: entries non-decreasing, entry[0] <= v
+__device__ __forceinline__ void akv_last_at_most(const int32_t* entry, int n, int v0, int v1, int& i0, int& i1) {
+  i0 = i1 = 0;
+  for (int step = n >> 1; step > 0; step >>= 1) {
+    const int e0 = entry[i0 + step], e1 = entry[i1 + step];
+    i0 += e0 <= v0 ? step : 0;
+    i1 += e1 <= v1 ? step : 0;
+  }
 }
 
 // ----------------------------------------------------------------------------------
@@ -202,7 +204,7 @@ __device__ __forceinline__ int akv_last_at_most(const int32_t* entry, int n, int
 // workgroup, which finds its sequence among the starts in LDS.  (By a thread per sequence, one of 30,000 tokens among 99 of
 // 200 had 150 records to write alone: the kernel 10.9 us, now 6.3.)
 // ----------------------------------------------------------------------------------
-#define AKV_PART_WORDS 592              // LDS of akv_attn_partition (int32 words)
+#define AKV_PART_WORDS 784              // LDS of akv_attn_partition (int32 words)
 __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G, int cb, int32_t* wgdesc, int32_t* seqw,
                                                    int32_t* lds /*[AKV_PART_WORDS]*/, const void* context_lens, int cl_itype,
                                                    int block_size, int64_t max_blocks_per_seq, int shares, int longer) {
@@ -211,12 +213,13 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
   const int chunk = (S + 255) / 256;
   int32_t* p_wfirst = lds;              // [n + 1] first workgroup of each sequence; [n] = workgroups in use
   int32_t* p_pref = lds + 257;          // [n + 1] block prefix; [n] = total
-  int32_t* p_ctx = lds + 514;           // [64] context length in tokens, clamped to the table width (at most 64 sequences)
-  int32_t* p_mode = lds + 578;          // [0] 1 = whole workgroups per sequence (at most 64 sequences)
-  int32_t* p_part = lds + 580;          // [2][4] sums of the wavefronts (more)
-  int32_t* p_scan = lds + 588;          // [4]
+  int32_t* p_ctx = lds + 514;           // [256] context length in tokens, clamped to the table width (at most 256 sequences)
+  int32_t* p_mode = lds + 770;          // [0] 1 = whole workgroups per sequence (at most 64 sequences)
+  int32_t* p_part = lds + 771;          // [2][4] sums of the wavefronts (more)
+  int32_t* p_scan = lds + 779;          // [4]
   bool aligned = false;
   if (S > 64) {
+    if (S <= 256 && tid < S) p_ctx[tid] = (int)akv_seq_tokens(context_lens, cl_itype, tid, block_size, max_blocks_per_seq);
     int b1;
     const int b0 = akv_block_prefix_scan(context_lens, cl_itype, S, block_size, max_blocks_per_seq, prefix, p_scan, &b1);
     if (tid < 256) p_pref[tid] = b0;
@@ -258,6 +261,26 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
         if (tid < S) {
           seqw[2 * tid] = first;
           seqw[2 * tid + 1] = first + k - 1;
+        }
+        // a few records a sequence: by its thread (100 contexts of 100 to 1,000, tq35, 16 heads on 4: the step 37.7 us; looked up
+        // below, 38.4)
+        if (!__syncthreads_or(k > 8)) {
+          const int pc = k > 0 ? (c + k - 1) / k * cb : 0;
+          for (int j = 0; j < k; ++j) {
+            int32_t* rec = wgdesc + (size_t)(first + j) * AKV_WGREC;
+            rec[AKV_WGREC_G0] = b0 + j * pc;              // (below b1: k - 1 ranges of at most lo chunks do not hold c)
+            rec[AKV_WGREC_G1] = min(b1, b0 + (j + 1) * pc);
+            rec[AKV_WGREC_SEQ] = tid;
+            rec[AKV_WGREC_SB0] = b0;
+            rec[AKV_WGREC_SB1] = b1;
+            rec[AKV_WGREC_CTX] = p_ctx[tid];
+          }
+          for (int w = p_wfirst[256] + tid; w < G; w += blockDim.x) {
+            int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
+            rec[AKV_WGREC_G0] = rec[AKV_WGREC_G1] = 0;
+            rec[AKV_WGREC_SEQ] = -1;
+          }
+          return;
         }
       }
     }
@@ -322,15 +345,10 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
   __syncthreads();
   if (S <= 64) aligned = p_mode[0] != 0;
   const int total = p_pref[n], per = (total + G - 1) / G;
-  for (int w = tid; w < G; w += blockDim.x) {
-    int g0 = 0, g1 = 0, s = -1, b0 = 0, b1 = 0;
+  auto record = [&](int w, int s) {
+    int g0 = 0, g1 = 0, b0 = p_pref[s], b1 = p_pref[s + 1];
     if (aligned) {
       if (w < p_wfirst[n]) {
-        // (a sequence without workgroups shares the next one's entry and is passed over; entries past the batch equal the
-        // number in use)
-        s = akv_last_at_most(p_wfirst, n, w);
-        b0 = p_pref[s];
-        b1 = p_pref[s + 1];
         const int k = p_wfirst[s + 1] - p_wfirst[s];
         const int c = (b1 - b0 + cb - 1) / cb;
         const int pc = (c + k - 1) / k;
@@ -340,20 +358,15 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
     } else {
       g0 = min(total, w * per);
       g1 = min(total, g0 + per);
-      if (g0 < g1) {
-        s = akv_last_at_most(p_pref, n, g0);    // the last sequence that starts at or before g0 (an empty one shares its successor's start)
-        b0 = p_pref[s];
-        b1 = p_pref[s + 1];
-        if (chunk > 1) {
-          int hi = min(S, (s + 1) * chunk);     // prefix[s] <= g0 < prefix[hi]
-          s *= chunk;
-          while (hi - s > 1) {
-            const int mid = (s + hi) >> 1;
-            if (prefix[mid] <= g0) s = mid; else hi = mid;
-          }
-          b0 = prefix[s];
-          b1 = prefix[s + 1];
+      if (g0 < g1 && chunk > 1) {
+        int hi = min(S, (s + 1) * chunk);     // prefix[s] <= g0 < prefix[hi]
+        s *= chunk;
+        while (hi - s > 1) {
+          const int mid = (s + hi) >> 1;
+          if (prefix[mid] <= g0) s = mid; else hi = mid;
         }
+        b0 = prefix[s];
+        b1 = prefix[s + 1];
       }
     }
     int32_t* rec = wgdesc + (size_t)w * AKV_WGREC;
@@ -363,8 +376,19 @@ __device__ __forceinline__ void akv_attn_partition(int32_t* prefix, int S, int G
     if (g0 < g1) {
       rec[AKV_WGREC_SB0] = b0;
       rec[AKV_WGREC_SB1] = b1;
-      rec[AKV_WGREC_CTX] = S > 64 ? (int)akv_seq_tokens(context_lens, cl_itype, s, block_size, max_blocks_per_seq) : p_ctx[s];
+      rec[AKV_WGREC_CTX] = S > 256 ? (int)akv_seq_tokens(context_lens, cl_itype, s, block_size, max_blocks_per_seq) : p_ctx[s];
     }
+  };
+  for (int w = tid; w < G; w += 2 * blockDim.x) {
+    // The sequence of a workgroup: the last whose first workgroup, or whose start, does not lie behind it.  (One without
+    // workgroups or blocks shares the next one's entry and is passed over; entries past the batch equal the number of workgroups in use,
+    // or of blocks.  Workgroups that get nothing: any.)
+    const int w1 = w + (int)blockDim.x;
+    int s0, s1;
+    if (aligned) akv_last_at_most(p_wfirst, n, min(w, p_wfirst[n] - 1), min(w1, p_wfirst[n] - 1), s0, s1);
+    else akv_last_at_most(p_pref, n, min(w * per, total - 1), min(w1 * per, total - 1), s0, s1);
+    record(w, s0);
+    if (w1 < G) record(w1, s1);
   }
 }
 
