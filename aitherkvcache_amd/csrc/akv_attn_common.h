@@ -195,7 +195,8 @@ __device__ __forceinline__ void akv_last_at_most(const int32_t* entry, int n, in
 // heads of 256 55.5 -> 49.5, tq35 65.2 -> 56.1.
 // Attention of batches of G / 8 to G / 2 sequences of 250 to 6,000 tokens, equal ranges over whole workgroups, by what these are longer:
 //   kernel of akv_attn_mfma.hip        none 1.00 to 1.33, 1 chunk 1.04 to 1.33, 2 1.04 to 1.15, 3 1.03 to 1.06, 12 0.95 to 0.99
-//   independent wavefronts, one share  none 0.99 to 1.35, 1 1.00 to 1.26, 2 0.99 to 1.15, 3 0.96 to 1.08 (heads of 64 0.98 to 1.00), 4 0.97 to 1.06
+//   independent wavefronts, one share  none 0.97 to 1.35, 1 1.00 to 1.26, 2 0.99 to 1.15; 3 heads of 256 0.98 to 1.03, hybrid rows 0.98
+//     to 1.12 (64 contexts of 4,000 to 8,192 1.01), but heads of 64 0.98 to 1.00, and tq35 with two workgroups a CU 0.96 to 1.01; 4 0.97 to 1.06
 //   as many workgroups as half again the chip holds (tq35, groups of other than four heads, from three groups or heads on): the ranges of a CU
 //     take turns, a second segment hides behind another's products and a longer range does not: none 0.97 to 1.58, 1 chunk up to
 //     ranges of eight 1.00 to 1.17, beyond 0.91 to 1.02, 2 0.90 to 1.03, 3 0.91 to 0.99

@@ -1238,7 +1238,7 @@ static int hw_run(const void* query, int q_dtype, int64_t qs_seq, int64_t qs_hea
                   const akv_attn_ws& ws, void* out, int out_dtype, int64_t os_seq, int64_t os_head, hipStream_t stream, M main) {
   const int G = hw_ranges(a.KVH, a.hp), shares = HW_W / a.hp, cus = akv_cached_cu_count();
   // (akv_attn_partition: a second segment in chunks; nothing where more workgroups take turns than the chip holds)
-  const int longer = G * a.hgroups > F::PER_SIMD * (cus > 0 ? cus : 256) ? 0 : 2;
+  const int longer = G * a.hgroups > F::PER_SIMD * (cus > 0 ? cus : 256) ? 0 : F::PER_SIMD == 3 ? 3 : 2;
   const float qscale = scale * 1.4426950408889634f;      // scores come out in the log2 domain
   const uint32_t start_status = g_spin_limit == 0 ? AKV_STATUS_HANDOFF_TIMEOUT : 0u;
 #define HW_PRO(DT) akv_attn_hyb_prologue_kernel<F, DT><<<a.S * a.KVH + 2, 256, 0, stream>>>(query, qs_seq, qs_head, table, qscale, a.S, a.QH, a.KVH, a.hgroup, a.gqa, a.context_lens, a.cl_itype, a.block_size, a.max_blocks_per_seq, ws.prefix, (uint4*)a.qop, ws.qrot, ws.lut, ws.status, start_status, ws.wgdesc, ws.seqw, G, shares, longer)

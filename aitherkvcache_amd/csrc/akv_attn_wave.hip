@@ -30,9 +30,9 @@
 // 48 sequences of 512 to 8,192 tokens 56.3 | 113.2 us; 16 on 4 of 256, 24 sequences 66.7 | 141.5; 8 on 1 of 128, 48 of 1,024
 // to 16,384 39.3 | 62.2; 8 on 2 of 128 52.6 | 62.3.
 //
-// What bounds it: the chain of trips to LDS and memory a wavefront walks, at two to four wavefronts a SIMD.  No unit is full
-// (profiles/attn_wave_sq_counters.txt, share of the kernel's cycles): vector unit
-// 44, 41 and 34 % at head_dim 64, 128 and 256, matrix cores 13 to 17, LDS 18 to 24.
+// What bounds it: the chain of trips to LDS and memory a wavefront walks, at two to four wavefronts a SIMD.  Share of the kernel's
+// cycles (profiles/attn_wave_sq_counters.txt), head_dim 64, 128 and 256: address unit 71, 30 and 59 %, vector unit 49, 46 and 36,
+// matrix cores 13, 16 and 18, LDS 19, 27 and 24.
 #include <type_traits>
 
 #include "akv_attn_rows.h"
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void akv_attn_wave_prologue_kernel(
   __shared__ int32_t scratch[AKV_PART_WORDS];
   if (blockIdx.x == 0) {
     if (threadIdx.x == 0) status[0] = 0u;
-    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares, 2);
+    akv_attn_partition(prefix, S, G, block_size == 32 ? 1 : 2, wgdesc, seqw, scratch, context_lens, cl_itype, block_size, max_blocks_per_seq, shares, D == 64 ? 2 : 3);
     return;
   }
   ar_rotate_queries<D, QDT, false>(rows, (int)blockIdx.x - 1, (int)gridDim.x - 1, query, qs_seq, qs_head, Pi, scale, S, QH, KVH, slots, qop, fac, qscale, bits);
@@ -299,8 +299,9 @@ __global__ __launch_bounds__((D == 64 ? 16 : 8) * 64) void akv_attn_wave_kernel(
           pbwin = (int)akv_clamp_block(akv_load_index(a.block_tables, a.bt_itype, s * a.bt_stride + bi), a.num_blocks);
           win_k = k0;
         };
-        // Few requests: with two of a quarter row a lane for keys and eight of the lane's own codes for values the address unit was
-        // busy for 80,000 of 99,000 cycles at head_dim 64, 43,000 of 64,000 at 256.  Decode steps: 48 sequences, one kv head of 128
+        // Few requests: with two of a quarter row a lane for keys and eight of the lane's own codes for values there were 704,000 a launch
+        // at head_dim 64 (48 sequences of 512 to 8,192, 8 kv heads), now 407,000; 234,000 and 176,000 at 256.  (The address unit is busy
+        // about as long as before.)  Decode steps: 48 sequences, one kv head of 128
         // 35.1 -> 33.8 us, heads of 64 66.4 -> 65.2, of 256 in 2 bits 42.0 -> 40.2.
         // Lane (8 p + c, g) reads piece c, of 2 VB bytes, of the first (p = 0) or second token of a pair and hands half of it on.
         // 3 bits: whole dwords around the piece; the selectors gather a group's three bytes, first byte on top.

@@ -9,8 +9,9 @@
 //         BYTE (two codes) indexes a table in LDS whose entry is the float16 pair (c[a], c[b]), 32 times, and the pair of
 //         remainders (c = hi + lo to ~22 bits), 32 times (address = byte * 256 + (lane & 31) * 4, built by one byte permute, and
 //         128 bytes on), so look-ups do not conflict on a bank.  Both by one request of eight bytes, they landed side by side and were
-//         moved to their operands, 64 of some 360 vector instructions of a step (K and V of 20k tokens x 8 heads at head_dim 128:
-//         37.8 -> 36.7 us, 3 bits 38.9 -> 37.5, head_dim 256 68.2 -> 66.3; look-ups a piece ahead of the products 37.0, 38.4, 67.0).
+//         moved to their operands, some 50 of 510 vector instructions of a step of 32 rows (K and V of 20k tokens x 8 heads to
+//         bfloat16 blocks at head_dim 128: 41.2 -> 40.4 us, 3 bits 43.1 -> 42.1, head_dim 256 145.8 -> 142.0; look-ups a piece ahead of the
+//         products were no faster).
 //     Three products per tile: Pi_hi c_hi + Pi_hi c_lo + Pi_lo c_hi.
 //   The rows of an A tile are permuted so that a lane ends up with eight neighbouring coordinates of ONE row from two tiles:
 //   it needs one norm and one address per vector, and the four lanes of a vector write 64 neighbouring bytes per store.
@@ -18,7 +19,7 @@
 // 3-bit and 2-bit rows are spread to one code per nibble in registers (akv_nibble.h) and take the same table; the
 // coordinate order that the spreading leaves is matched when the matrix is loaded.
 //
-// What bounds it: the loop, 48 products of 16 cycles and some 150 vector instructions of four per 16 rows of head_dim 128
+// What bounds it: the loop, 48 products of 16 cycles and some 210 vector instructions of four per 16 rows of head_dim 128
 // and wavefront at two wavefronts a SIMD, and the trips to memory around it.
 // Flat rows at head_dim 128 (us; the matrix in LDS, 64 KB read per 32 rows | split from the float32 matrix in every launch |
 // as it is now): 4-bit to float16, 4,096 rows 10.2 | 9.5 | 5.9, 65,536 rows 14.6 | 16.9 | 13.1, 2^20 rows 110 | 110 | 105; 3-bit
