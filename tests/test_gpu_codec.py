@@ -686,20 +686,28 @@ def test_read_probe_sums_what_it_reads(dev):
 
 
 
-@pytest.mark.parametrize("bits", [2, 3, 4])
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("form,T,H,BS", [("paged", 203, 8, 16), ("paged", 257, 8, 16), ("paged", 585, 7, 24), ("paged", 292, 28, 32), ("paged", 2340, 7, 16),
-                                         ("flat", 4095, 1, 0), ("flat", 4097, 1, 0), ("flat", 8191, 1, 0), ("flat", 8193, 1, 0), ("flat", 16381, 1, 0), ("flat", 32767, 1, 0)])
-def test_calls_of_a_step_or_two_a_cu_write_the_bytes_of_the_large_ones(golden, dev, bits, dtype, form, T, H, BS, monkeypatch):
+def register_form_rows(form, dtype, bits):
+    """Rows a CU, (more than, up to), that the kernel with the matrix in registers takes."""
+    wide = 32 if dtype == torch.float32 else 64
+    fewest = 0 if dtype == torch.float32 else 8 if form == "paged" and bits != 4 else 16
+    return fewest, wide * (2 if form == "paged" or (bits == 3 and wide == 64) else 1)
+
+
+REGISTER_FORM = [(form, T, H, BS, dtype, bits)
+                 for form, T, H, BS in [("paged", 203, 8, 16), ("paged", 257, 8, 16), ("paged", 585, 7, 24), ("paged", 292, 28, 32), ("paged", 2340, 7, 16), ("flat", 4095, 1, 0),
+                                        ("flat", 4097, 1, 0), ("flat", 8191, 1, 0), ("flat", 8193, 1, 0), ("flat", 16381, 1, 0), ("flat", 32767, 1, 0)]
+                 for dtype in (torch.float16, torch.bfloat16, torch.float32) for bits in (2, 3, 4)
+                 if (lambda least, most: least * 256 < (2 if form == "paged" else 1) * T * H <= most * 256)(*register_form_rows(form, dtype, bits))]
+
+
+@pytest.mark.parametrize("form,T,H,BS,dtype,bits", REGISTER_FORM)
+def test_calls_of_a_step_or_two_a_cu_write_the_bytes_of_the_large_ones(golden, dev, form, T, H, BS, dtype, bits, monkeypatch):
     """Keys and values, or flat rows, through the kernel with the matrix in registers -- steps of 16, 32 and 64 rows, a last step of a
     few, one and two steps a CU, heads and block sizes that are no powers of two -- and through the one with the matrix in LDS:
     codes, norms and untouched rows byte for byte, with NaN, infinite and zero rows and slots outside the cache.  (What the rule
-    leaves to other kernels is not run: a kernel would be held against itself.)"""
-    cus, n = torch.cuda.get_device_properties(dev).multi_processor_count, (2 if form == "paged" else 1) * T * H
-    wide = 32 if dtype == torch.float32 else 64
-    fewest = -1 if dtype == torch.float32 else 8 if form == "paged" and bits != 4 else 16
-    if not fewest * cus < n <= wide * cus * (2 if form == "paged" or (bits == 3 and wide == 64) else 1):
-        pytest.skip("another kernel's")
+    leaves to other kernels is not in the list: a kernel would be held against itself.)"""
+    least, most = register_form_rows(form, dtype, bits)
+    assert least < (2 if form == "paged" else 1) * T * H / torch.cuda.get_device_properties(dev).multi_processor_count <= most
     tq = make_tq(golden, dev, bits)
     P = tq._packed_dim
     NB = -(-T // BS) + 1 if form == "paged" else 1
